@@ -295,6 +295,84 @@ def work(case):
     return {"bytes": B * L * case["V"] * size + 4 * pairs + 8 * B * L, "flops": 3 * B * L * case["V"] + sweep}
 
 
+# ---- the same in 64 bits ---------------------------------------------------------------------------------------
+
+def _square(links):
+    """[B, L, L]: links[b, i, d] at (i, i + d + 1), -inf elsewhere."""
+    B, L, W = links.shape
+    d = torch.arange(L, device=links.device).view(1, L) - torch.arange(L, device=links.device).view(L, 1) - 1
+    inside = (d >= 0) & (d < W)
+    full = links.gather(2, d.clamp(0, W - 1).expand(B, L, L))
+    return full.masked_fill_(~inside, NEG_INF)
+
+
+def _exact_loss(case, s):
+    match, edges = s["match"].detach().double(), _square(s["links"].detach().double())
+    B, T, L = match.shape
+    last, end = s["tgt_len"] - 1, s["out_len"] - 1
+    rows = torch.arange(B, device=match.device)
+    alpha = torch.full_like(match, NEG_INF)
+    alpha[:, 0, 0] = match[:, 0, 0]
+    for t in range(1, T):
+        alpha[:, t] = torch.logsumexp(alpha[:, t - 1].unsqueeze(2) + edges, 1) + match[:, t]
+    z = alpha[rows, last, end]
+    if s["grad"] is None:
+        return z
+    scale = s["grad"].double().view(B, 1)
+    grad_match, grad_edges = torch.zeros_like(match), torch.zeros_like(edges)
+    stop = torch.where(torch.arange(L, device=match.device) == end.view(B, 1), 0.0, NEG_INF).double()
+    beta = torch.full_like(stop, NEG_INF)       # log-probability of what follows node and step
+    for t in reversed(range(T)):
+        if t + 1 < T:
+            ahead = edges + (match[:, t + 1] + beta).unsqueeze(1)
+            share = (alpha[:, t] - z.view(B, 1)).unsqueeze(2) + ahead
+            grad_edges += torch.exp(share) * scale.unsqueeze(2)
+            beta = torch.logsumexp(ahead, 2)
+        beta = torch.where((last == t).view(B, 1), stop, beta)
+        grad_match[:, t] = torch.exp(alpha[:, t] + beta - z.view(B, 1)) * scale
+    W = s["links"].shape[2]
+    j = torch.arange(L, device=match.device).view(L, 1) + torch.arange(1, W + 1, device=match.device).view(1, W)
+    grad_links = grad_edges.gather(2, j.clamp(max=L - 1).expand(B, L, W)).masked_fill_(j >= L, 0.0)
+    return z, grad_match, grad_links
+
+
+def _exact_gather(case, s):
+    logits = s["logits"].detach().double()
+    ids = s["targets"].unsqueeze(1).expand(-1, logits.shape[1], -1)
+    lse = torch.logsumexp(logits, -1, keepdim=True)
+    selected, grad = logits.gather(-1, ids) - lse, s["grad"].double()
+    out = (logits - lse).exp_().mul_(-grad.sum(-1, keepdim=True))
+    return selected, out.scatter_add_(-1, ids, grad)
+
+
+def _exact_links(case, s):
+    B, L, W = case["B"], case["L"], case["window"]
+    i, j = torch.arange(L, device="cuda").view(L, 1), torch.arange(L, device="cuda").view(1, L)
+    shifted = (i + torch.arange(1, W + 1, device="cuda").view(1, W))
+    links, grad_scores, grad_gates = [], [], []
+    for b in range(B):
+        scores = s["scores"][b].detach().double().requires_grad_()
+        gates = s["gates"][b].detach().double().requires_grad_()
+        allowed = (j > i) & (j <= i + W) & (j < s["valid_end"][b].view(L, 1))
+        some = allowed.any(1)
+        logp = torch.log_softmax(scores.masked_fill(~allowed.unsqueeze(2), -1e30), 1) + gates.unsqueeze(1)
+        mixed = torch.logsumexp(logp, 2)
+        keep = (allowed & some.view(L, 1)).gather(1, shifted.clamp(max=L - 1)) & (shifted < L)
+        mine = mixed.gather(1, shifted.clamp(max=L - 1))
+        grads = torch.autograd.grad(mine, (scores, gates), s["grad"][b].double().masked_fill(~keep, 0.0))
+        links.append(mine.detach().masked_fill(~keep, NEG_INF))
+        grad_scores.append(grads[0])
+        grad_gates.append(grads[1])
+    return torch.stack(links), torch.stack(grad_scores), torch.stack(grad_gates)
+
+
+def exact(case, seed):
+    """What run() returns for these inputs in float64 by plain torch.  None where the outputs are whole numbers, and for
+    the criterion, whose gradients hang on a path and on targets forced along it (its parts are cases of their own)."""
+    made = {"loss": _exact_loss, "gather": _exact_gather, "links": _exact_links}.get(case["kind"])
+    return None if made is None else made(case, prepare(case, seed))
+
+
 def tolerance(case):
     kind, dtype = case["kind"], case["dtype"]
     if kind in ("align", "decode"):
