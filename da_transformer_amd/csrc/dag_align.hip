@@ -514,17 +514,126 @@ __global__ __launch_bounds__(kTileWaves * kWave) void dag_align_tiles_kernel(Ali
 #undef DAGX_STAMP
 }
 
-// One wave per sample walks the path backwards through the score table.  The sweep has recorded, for
-// every cell, the lowest block of 64 nodes that holds a best predecessor, so a step scans 64
-// candidates (lanes <-> nodes of that block): it re-evaluates fl32(A[t-1][i] + E[i][j]) -- the very
-// operation of the sweep, hence bit-identical -- takes the maximum and, among the lanes that hold it,
-// the lowest node: the first-index rule of torch.max (fs_plugins/custom_ops/dag_loss.py:253-257, :350).
-// The row of source blocks of step t-1 is fetched together with the candidates of step t (it does
-// not depend on where the path goes), so a step costs one memory round trip.
+// Walking the path backwards through the score table.  The sweep has recorded, for every cell, the lowest block of 64
+// nodes that holds a best predecessor, so a step scans 64 candidates (lanes <-> nodes of that block): it re-evaluates
+// fl32(A[t-1][i] + E[i][j]) -- the very operation of the sweep, hence bit-identical -- takes the maximum and, among the
+// lanes that hold it, the lowest node: the first-index rule of torch.max (fs_plugins/custom_ops/dag_loss.py:253-257, :350).
 //
-// The workgroup has kOneGroupThreads threads all the same: a sample that the pipeline gave up on (flags[b] set) is
-// done again here, from scratch, by the one-workgroup method; for every other sample all waves but the first leave
-// at once.  (A launch of its own for the flagged samples, which are rare, would cost every call its latency.)
+// The steps are a serial chain, one wave per sample, so what bounds the walk is the latency of a step.  Read from memory a
+// step's scores and transitions cost a round trip to HBM (0.61 us a step).  A path moves on by a few nodes a step, so it
+// stays in a block of 64 nodes for several steps and nearly always finds its predecessor in that block or the one below:
+// while wave 0 walks through block J out of LDS, the other waves bring in what a walk through block J - 1 reads (the
+// transitions from its two predecessor blocks, and kWalkRows rows of their scores and of the source blocks, whichever
+// step the walk enters with).  A predecessor further away is read from memory, a walk that leaves the staged rows or jumps
+// over a block stages again in front of the next step.  Measured: see launch_align.
+constexpr int kWalkRows = 48;             // two buffers and the decoder's own 25 KB fit the 160 KB of a CU
+constexpr int kWalkPitch = kBlk + 1;      // the lanes read a column of the transitions: no two in one bank
+struct WalkStage {
+    float e[2 * kBlk * kWalkPitch];       // E[(J-1)*64 + r][J*64 + c] at r * kWalkPitch + c, -inf where there is none
+    float a[kWalkRows * 2 * kBlk];        // row r: A[hi - 1 - r] of blocks J - 1 and J
+    unsigned src[kWalkRows * kBlk / 4];   // row r: source blocks of (hi - r, block J), a byte each
+};
+constexpr size_t kWalkLds = 2 * sizeof(WalkStage);
+
+template <typename TL, int NT>
+__device__ __forceinline__ void stage_walk(WalkStage &w, const float *A, const unsigned char *srcblk, int spitch, const TL *links,
+                                           int L, int translen, int J, int hi) {
+    constexpr int kHelpers = NT - kWave;
+    const int q = (int)threadIdx.x - kWave;
+    constexpr int kE = (2 * kBlk * kBlk + kHelpers - 1) / kHelpers, kA = (kWalkRows * 2 * kBlk + kHelpers - 1) / kHelpers;
+    constexpr int kS = (kWalkRows * kBlk / 4 + kHelpers - 1) / kHelpers;
+    TL ve[kE];
+    float va[kA];
+    unsigned vs[kS];
+    bool in[kE];
+#pragma unroll
+    for (int u = 0; u < kE; ++u) {   // everything is requested before anything is stored
+        const int x = q + u * kHelpers, i = (J - 1) * kBlk + x / kBlk, j = J * kBlk + x % kBlk, d = j - i - 1;
+        in[u] = x < 2 * kBlk * kBlk && i >= 0 && j < L && d >= 0 && d < translen;
+        ve[u] = links[in[u] ? (int64_t)i * translen + d : 0];
+    }
+#pragma unroll
+    for (int u = 0; u < kA; ++u) {
+        const int x = q + u * kHelpers, row = hi - 1 - x / (2 * kBlk), i = (J - 1) * kBlk + x % (2 * kBlk);
+        va[u] = A[row >= 0 && i >= 0 && i < L && x < kWalkRows * 2 * kBlk ? (int64_t)row * L + i : 0];
+    }
+#pragma unroll
+    for (int u = 0; u < kS; ++u) {
+        const int x = q + u * kHelpers, row = hi - x / (kBlk / 4), at = J * kBlk + (x % (kBlk / 4)) * 4;
+        vs[u] = *reinterpret_cast<const unsigned *>(srcblk + (row >= 1 && at < spitch && x < kWalkRows * kBlk / 4 ? (int64_t)row * spitch + at : 0));
+    }
+#pragma unroll
+    for (int u = 0; u < kE; ++u) {
+        const int x = q + u * kHelpers;
+        if (x < 2 * kBlk * kBlk) w.e[(x / kBlk) * kWalkPitch + x % kBlk] = in[u] ? to_float(ve[u]) : DAGX_NEG_INF;
+    }
+#pragma unroll
+    for (int u = 0; u < kA; ++u) { const int x = q + u * kHelpers; if (x < kWalkRows * 2 * kBlk) w.a[x] = va[u]; }
+#pragma unroll
+    for (int u = 0; u < kS; ++u) { const int x = q + u * kHelpers; if (x < kWalkRows * kBlk / 4) w.src[x] = vs[u]; }
+}
+
+// From cell (s, j) down to row `stop` by the whole workgroup: visit(row, node) for the predecessor found in every row,
+// called by all lanes of wave 0; it returns the node to go on from, or -1 to end the walk (node: -1 where no candidate
+// has a finite score).  lds: kWalkLds bytes.  s, j are uniform over the workgroup.
+template <typename TL, int NT, typename VISIT>
+__device__ __forceinline__ void walk_back(const float *A, const unsigned char *srcblk, int spitch, const TL *links, int L,
+                                          int translen, int s, int j, int stop, WalkStage *lds, VISIT visit) {
+    __shared__ int at[2][2];
+    if (s <= stop) return;
+    const bool walker = threadIdx.x < kWave;
+    const int lane = threadIdx.x & (kWave - 1);
+    int cur = 0, J = j / kBlk, hi = s;
+    if (!walker) stage_walk<TL, NT>(lds[0], A, srcblk, spitch, links, L, translen, J, hi);
+    __syncthreads();
+    for (int round = 0;; ++round) {
+        const int next_hi = s - 1;
+        if (!walker) {
+            if (J > 0 && next_hi > stop) stage_walk<TL, NT>(lds[cur ^ 1], A, srcblk, spitch, links, L, translen, J - 1, next_hi);
+        } else {
+            const WalkStage &w = lds[cur];
+            const unsigned char *src = reinterpret_cast<const unsigned char *>(w.src);
+            while (s > stop && j >= 0 && j / kBlk == J && hi - s < kWalkRows) {
+                const int r = hi - s, c = j & (kBlk - 1);
+                // both predecessor blocks are read along with the byte that says which of them it is
+                const float e0 = w.e[lane * kWalkPitch + c], e1 = w.e[(kBlk + lane) * kWalkPitch + c];
+                const float a0 = w.a[r * 2 * kBlk + lane], a1 = w.a[r * 2 * kBlk + kBlk + lane];
+                const int I = __builtin_amdgcn_readfirstlane((int)src[r * kBlk + c]);
+                float x;
+                if (I == J) x = a1 + e1;
+                else if (I == J - 1) x = a0 + e0;
+                else {
+                    const int i = I * kBlk + lane, d = j - i - 1;
+                    const bool valid = d >= 0 && d < translen && i < L;
+                    const float e = to_float(links[valid ? (int64_t)i * translen + d : 0]);
+                    const float av = A[(int64_t)(s - 1) * L + (i < L ? i : L - 1)];
+                    x = valid ? av + e : DAGX_NEG_INF;
+                }
+                const float top = wave64_max(x);
+                // lowest lane among those that hold the maximum
+                const int to = top > DAGX_NEG_INF ? I * kBlk + (int)__builtin_ctzll(__builtin_amdgcn_ballot_w64(x == top)) : -1;
+                --s;
+                j = __builtin_amdgcn_readfirstlane(visit(s, to));
+            }
+            if (lane == 0) { at[round & 1][0] = s; at[round & 1][1] = j; }
+        }
+        __syncthreads();
+        s = __builtin_amdgcn_readfirstlane(at[round & 1][0]);
+        j = __builtin_amdgcn_readfirstlane(at[round & 1][1]);
+        if (s <= stop || j < 0) return;
+        cur ^= 1;
+        if (j / kBlk == J - 1 && next_hi > stop && next_hi >= s && next_hi - s < kWalkRows) {
+            J -= 1; hi = next_hi;
+        } else {
+            J = j / kBlk; hi = s;
+            if (!walker) stage_walk<TL, NT>(lds[cur], A, srcblk, spitch, links, L, translen, J, hi);
+            __syncthreads();
+        }
+    }
+}
+
+// The backtrack of the alignment, one workgroup per sample.  A sample that the pipeline gave up on (flags[b] set) is
+// done again here, from scratch, by the one-workgroup method.  (A launch of its own for the flagged samples, which are rare, would cost every call its latency.)
 constexpr int kOneGroupThreads = 1024;
 template <typename TM, typename TL, bool TRACE_LDS>
 __global__ __launch_bounds__(kOneGroupThreads) void dag_backtrack_kernel(
@@ -535,49 +644,24 @@ __global__ __launch_bounds__(kOneGroupThreads) void dag_backtrack_kernel(
         align_one_sample<TM, TL, kOneGroupThreads, TRACE_LDS>(a, b, lds_a);
         return;
     }
-    if (threadIdx.x >= kWave) return;
-    const int lane = threadIdx.x;
+    const int lane = threadIdx.x & (kWave - 1);
+    const bool walker = threadIdx.x < kWave;
     const int T = a.T, L = a.L, translen = a.translen;
-    const int64_t *out_len = a.out_len, *tgt_len = a.tgt_len;
-    const TL *links_all = static_cast<const TL *>(a.links);
     int64_t *path = a.path + (int64_t)b * L;
-    for (int j = lane; j < L; j += kWave) path[j] = -1;
-    const int Lb = (int)out_len[b], Tb = (int)tgt_len[b];
+    if (walker)
+        for (int j = lane; j < L; j += kWave) path[j] = -1;
+    const int Lb = (int)a.out_len[b], Tb = (int)a.tgt_len[b];
     if (!(Tb >= 1 && Lb >= 1 && Tb <= T && Lb <= L && Tb <= Lb)) return;
     const float *A = table + (int64_t)b * T * L;
     const int spitch = srcblk_pitch(L);
-    const unsigned char *srcblk = srcblk_all + (int64_t)b * T * spitch;
-    const TL *links = links_all + (int64_t)b * L * translen;
-    if (!(A[(Tb - 1) * L + Lb - 1] > DAGX_NEG_INF)) return;   // no finite path
+    if (!(A[(int64_t)(Tb - 1) * L + Lb - 1] > DAGX_NEG_INF)) return;   // no finite path
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");     // the -1 fill precedes the path entries (same wave)
-    // a row of source blocks: L <= 1024 bytes, 16 per lane (lane l holds bytes 16 l .. 16 l + 15)
-    typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
-    auto load_row = [&](int t, unsigned (&r)[4]) {   // rows are 16-byte aligned and padded to 16 bytes
-        const u32x4 v = *reinterpret_cast<const u32x4 *>(srcblk + t * spitch + (16 * lane < spitch ? 16 * lane : 0));
-        r[0] = v.x; r[1] = v.y; r[2] = v.z; r[3] = v.w;
-    };
-    unsigned row[4];
-    if (Tb > 1) load_row(Tb - 1, row);
-    int j = Lb - 1;
-    for (int t = Tb - 1; t >= 1; --t) {
-        if (lane == 0) path[j] = t;
-        // source block of (t, j): byte j of the row
-        const int q = (j >> 2) & 3, src_lane = j >> 4;
-        const unsigned w = q == 0 ? row[0] : q == 1 ? row[1] : q == 2 ? row[2] : row[3];
-        const int I = (int)((unsigned)__builtin_amdgcn_readlane((int)w, src_lane) >> (8 * (j & 3))) & 0xff;
-        const int i = I * kBlk + lane;
-        const int d = j - i - 1;
-        const bool valid = d >= 0 && d < translen;
-        const float e = to_float(links[valid ? i * translen + d : 0]);
-        const float av = A[(t - 1) * L + (i < L ? i : L - 1)];
-        if (t > 1) load_row(t - 1, row);                 // for the next step, in the same round trip
-        const float x = valid ? av + e : DAGX_NEG_INF;
-        const float top = wave64_max(x);
-        if (!(top > DAGX_NEG_INF)) return;               // cannot happen on a finite path
-        // lowest lane among those that hold the maximum
-        j = I * kBlk + (int)__builtin_ctzll(__builtin_amdgcn_ballot_w64(x == top));
-    }
-    if (lane == 0) path[j] = 0;
+    if (threadIdx.x == 0) path[Lb - 1] = Tb - 1;
+    walk_back<TL, kOneGroupThreads>(A, srcblk_all + (int64_t)b * T * spitch, spitch, static_cast<const TL *>(a.links) + (int64_t)b * L * translen,
+                                    L, translen, Tb - 1, Lb - 1, 0, reinterpret_cast<WalkStage *>(lds_a), [&](int t, int j) {
+        if (lane == 0 && j >= 0) path[j] = t;
+        return j;   // (-1, the end of the walk, cannot happen on a finite path)
+    });
 }
 
 constexpr size_t kAlignLdsBudget = 144 * 1024;
@@ -636,9 +720,12 @@ static int launch_align(AlignArgs a, void *workspace, hipStream_t st) {
         const int B8 = (a.B + 7) & ~7;
         hipLaunchKernelGGL((dag_align_tiles_kernel<TM, TL>), dim3(B8 * C), dim3(kTileWaves * kWave), 0, st, ta);
         if ((rc = check_launch("dag_align_tiles"))) return rc;
-        // the backtrack, and the samples that the pipeline gave up on
+        // the backtrack, and the samples that the pipeline gave up on.  (float32, kernel time: with every step read from
+        // memory by one wave 38.7 us at B=64 L=512 T=64 and 174 us at B=16 L=1024 T=256, with the steps staged in LDS
+        // 26.0 and 76.5 us.)
         const bool in_lds = trace_fits_lds(a.T, a.L);
-        const size_t lds = (size_t)a.L * 8 + (in_lds ? (size_t)a.T * a.L * 2 : (size_t)0);
+        const size_t redo_lds = (size_t)a.L * 8 + (in_lds ? (size_t)a.T * a.L * 2 : (size_t)0);
+        const size_t lds = redo_lds > kWalkLds ? redo_lds : kWalkLds;
         auto kern = in_lds ? dag_backtrack_kernel<TM, TL, true> : dag_backtrack_kernel<TM, TL, false>;
         if (lds > 48 * 1024) {
             hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
@@ -789,8 +876,11 @@ struct DecodeArgs {
     int64_t *out_tokens, *out_count, *pred_length, *nodes;
 };
 
+// One workgroup per sample: the best node of every step, the best length, the walk back (walk_back) and the tokens.
 template <typename TL>
 __global__ __launch_bounds__(kDecodeThreads) void viterbi_select_kernel(DecodeArgs a) {
+    extern __shared__ float lds_walk[];
+    __shared__ int s_star;
     __shared__ float sbest[kDecodeMaxSteps];
     __shared__ int sidx[kDecodeMaxSteps];
     __shared__ int walk[kDecodeMaxSteps];
@@ -848,43 +938,28 @@ __global__ __launch_bounds__(kDecodeThreads) void viterbi_select_kernel(DecodeAr
         }
     }
     __syncthreads();
-    if (wave != 0) return;
     // best length: score / (t+1)^beta, first index among equals
-    float best = DAGX_NEG_INF;
-    int arg = lane;
-    for (int t = lane; t < n_max; t += kWave) {
-        const float q = sbest[t] / a.penalty[t];
-        if (q > best) { best = q; arg = t; }
+    if (wave == 0) {
+        float best = DAGX_NEG_INF;
+        int arg = lane;
+        for (int t = lane; t < n_max; t += kWave) {
+            const float q = sbest[t] / a.penalty[t];
+            if (q > best) { best = q; arg = t; }
+        }
+        float top;
+        const int t_star = wave_first_argmax(best, arg, top);
+        if (lane == 0) { a.pred_length[b] = t_star + 1; walk[t_star] = sidx[t_star]; s_star = t_star; }
     }
-    float top;
-    const int t_star = wave_first_argmax(best, arg, top);
-    const int n = t_star + 1;
-    int j = sidx[t_star];
-    if (lane == 0) { a.pred_length[b] = n; walk[n - 1] = j; }
-    // walk back: table row s = t + 1 holds reach_t; the predecessor of (s, j) lies in block srcblk[s][j]
-    typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
-    auto load_row = [&](int s, unsigned (&r)[4]) {
-        const u32x4 v = *reinterpret_cast<const u32x4 *>(srcblk + s * spitch + (16 * lane < spitch ? 16 * lane : 0));
-        r[0] = v.x; r[1] = v.y; r[2] = v.z; r[3] = v.w;
-    };
-    unsigned rowb[4];
-    if (n > 1) load_row(n, rowb);
-    for (int s = n; s >= 2; --s) {
-        const int q = (j >> 2) & 3, src_lane = j >> 4;
-        const unsigned w = q == 0 ? rowb[0] : q == 1 ? rowb[1] : q == 2 ? rowb[2] : rowb[3];
-        const int I = (int)((unsigned)__builtin_amdgcn_readlane((int)w, src_lane) >> (8 * (j & 3))) & 0xff;
-        const int i = I * kBlk + lane;
-        const int d = j - i - 1;
-        const bool valid = d >= 0 && d < translen && i < L;
-        const float e = to_float(links[valid ? (int64_t)i * translen + d : 0]);
-        const float av = A[(int64_t)(s - 1) * L + (i < L ? i : L - 1)];
-        if (s > 2) load_row(s - 1, rowb);
-        const float x = valid ? av + e : DAGX_NEG_INF;
-        float tp;
-        const int lo = wave_first_argmax(x, lane, tp);
-        j = tp > DAGX_NEG_INF ? I * kBlk + lo : 0;       // (a path of finite score never meets the other case)
-        if (lane == 0) walk[s - 2] = j;
-    }
+    __syncthreads();
+    const int n = __builtin_amdgcn_readfirstlane(s_star) + 1;
+    // table row s = t + 1 holds reach_t
+    walk_back<TL, kDecodeThreads>(A, srcblk, spitch, links, L, translen, n, __builtin_amdgcn_readfirstlane(sidx[n - 1]), 1,
+                                  reinterpret_cast<WalkStage *>(lds_walk), [&](int s, int to) {
+        const int j = to >= 0 ? to : 0;       // (a path of finite score never meets the other case)
+        if (lane == 0) walk[s - 1] = j;
+        return j;
+    });
+    if (wave != 0) return;
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
     __builtin_amdgcn_wave_barrier();
     // tokens: the last one always stays, an earlier one when it is not the pad and differs from its successor
@@ -956,7 +1031,10 @@ static int launch_decode(const void *links, const float *node_logp, const int64_
     if ((rc = check_launch("viterbi_table"))) return rc;
     DecodeArgs d{table, srcblk, links, out_len, node_tokens, penalty, T, L, translen, max_length, pad,
                  out_tokens, out_count, pred_length, nodes};
-    hipLaunchKernelGGL((viterbi_select_kernel<TL>), dim3(B), dim3(kDecodeThreads), 0, st, d);
+    auto select = viterbi_select_kernel<TL>;
+    const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(select), hipFuncAttributeMaxDynamicSharedMemorySize, (int)kWalkLds);
+    if (e != hipSuccess) { set_error("dag_viterbi_decode: cannot reserve %zu bytes of LDS: %s", kWalkLds, hipGetErrorString(e)); return DAGX_ERR_LAUNCH; }
+    hipLaunchKernelGGL(select, dim3(B), dim3(kDecodeThreads), kWalkLds, st, d);
     return check_launch("viterbi_select");
 }
 

@@ -281,6 +281,29 @@ def test_alignment_of_samples_the_pipeline_gave_up_on(shape):
     assert torch.equal(paths[0], rpath)
 
 
+@pytest.mark.parametrize("L,T,translen,hop", [
+    (64, 60, None, 1),        # more steps inside one block than rows are staged for
+    (128, 120, None, 1),      # the same with a block below
+    (1024, 8, None, 140),     # every step jumps over a block
+    (1024, 11, 129, 100),     # predecessors one and two blocks away
+    (300, 299, 3, 1), (65, 2, None, 64), (449, 100, 70, 5)])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16])
+def test_alignment_paths_that_dwell_and_jump(L, T, translen, hop, dtype):
+    """The backtrack stages a block of nodes and the one below it, a fixed number of steps at a time: paths that stay in
+    a block for longer, that skip blocks and that end in the first ones.  Scores are whole numbers: every sum is exact."""
+    B = 3
+    match, links_sq, ol, tl = random_problem(L + T, B, L, T, dtype=torch.float32, translen=translen)
+    if translen is not None:
+        ol = torch.minimum(ol, (tl - 1) * translen + 1)
+    links = tn.extract_valid_links(links_sq, translen)
+    links[:, :, :] = (links * 2).round().masked_fill(torch.isinf(links), NEG_INF)
+    if links.shape[2] >= hop:
+        links[:, :, hop - 1] += 20.0
+    match, links = match.round().to(dtype), links.to(dtype)
+    path = dagx.dag_best_alignment(match.to(DEV), links.to(DEV), ol.to(DEV), tl.to(DEV))
+    assert torch.equal(path.cpu(), _torch_path(match, links, ol, tl))
+
+
 def test_alignment_calls_in_a_row_and_on_a_second_stream():
     """Calls of different shapes in a row on one stream (each clears its pipeline words itself, whatever the last call
     left in the reused workspace), then the same on a second stream and again on the first: all must give the

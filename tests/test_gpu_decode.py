@@ -55,6 +55,13 @@ def test_viterbi_decode_matches_the_oracle(B, L, translen, scale, beta, joint):
     _run_and_compare(links, u, tok, out_len, translen, scale, beta, joint)
 
 
+@pytest.mark.parametrize("L,hop", [(200, 1), (500, 90), (1024, 150), (130, 64)])
+def test_viterbi_walk_that_dwells_and_jumps(L, hop):
+    """Long stays in one block of nodes and jumps over blocks: what the walk back stages does not cover them."""
+    links, u, tok, out_len = peaked_case(L, 3, L, hop=hop, min_len=L // 2)
+    _run_and_compare(links, u, tok, out_len, L - 1, 2.0, 1.0, True)
+
+
 @pytest.mark.parametrize("joint", [False, True])
 def test_viterbi_decode_full_size(joint):
     """B=64, L=512 (64 source tokens upsampled 8 times), 128 steps."""
