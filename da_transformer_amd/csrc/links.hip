@@ -6,11 +6,16 @@
 // This is what fs_plugins/models/glat_decomposed_with_link.py:380-404 computes with a masked_fill, a
 // gather into the shifted layout (:319-335), a log_softmax over the transitions, an add and a
 // logsumexp over the heads -- each a pass over a [B,L,translen,H] float tensor.  Here a row (b, i) is
-// read once: its window is H * n contiguous floats of `content`, held in registers by one wave (no
-// LDS, no barrier: the per-head reductions run on the DPP network).
-// HBM-bound: the forward reads the windows and writes [B,L,translen]; the backward reads the windows
-// again and writes the gradient over the whole [B,L,L,H] tensor in place (zeros outside the windows),
-// as the dense batched-GEMM backward that follows it expects.
+// read once: its window is H * n contiguous elements of `content`, held in registers by one, two or four
+// waves (four window positions a lane, so that a row leaves room for enough other rows on a SIMD to cover its loads).
+// HBM-bound once the waves in flight suffice: the forward reads the windows and writes [B,L,translen]; the backward reads
+// the windows again and writes the gradient over the whole [B,L,L,H] tensor in place (zeros outside the windows), as the
+// dense batched-GEMM backward that follows it expects.
+// Measured, forward and backward one after the other, against one wave per row with the whole window in registers (2 waves
+// a SIMD), three exponentials per score in the backward and cached zeros: B=64 L=512 H=8 float32 94 + 167 -> 58 + 168 us
+// (1.2 GB: 5.3 TB/s); B=16 L=1024 H=8 float16 88 + 171 -> 46 + 61 us (4.1 TB/s); B=8 L=512 H=16 float32 29 + 52 -> 16 + 36 us.
+// Non-temporal zeros alone took 164 -> 168, 83 -> 61 and 48 -> 36 us off the backwards and 78 -> 58 us off the first
+// forward, which finds less to write back; the gradient inside the window, stored the same way, was slower again.
 #include <type_traits>
 
 #include "dagx_common.h"
@@ -20,71 +25,56 @@ namespace dagx {
 constexpr int kLinkThreads = 256;                 // four waves, one row each
 constexpr int kLinkWaves = kLinkThreads / kWave;
 
-// ---- 64-lane reductions on the DPP network (no LDS traffic); the result is wave-uniform ------------
-template <int CTRL, int ROW_MASK>
-__device__ __forceinline__ float dpp_take(float v) {   // lanes outside ROW_MASK get 0
-    return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL, ROW_MASK, 0xf, false));
+// ---- reductions of one value per head over the 64 lanes --------------------------------------------
+// The heads are shared out while they are reduced: in every step a lane keeps half of its heads, hands the other half to
+// its partner and takes the partner's half of its own (7 operations for 8 heads where reducing every head by itself takes 48).
+// The partners are lane ^ 15, ^ 7, ^ 3, ^ 1 (DPP row_mirror, row_half_mirror, quad_perm): each differs from the lane in the
+// step's bit and agrees in the ones before it.  Afterwards lane l holds the total of head head_of<H>(l).
+template <int CTRL>
+__device__ __forceinline__ float dpp_lane(float v) {
+    return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL, 0xf, 0xf, true));
 }
-__device__ __forceinline__ float lanes_sum(float v) {
-    v += dpp_take<0xB1, 0xf>(v);    // quad_perm [1,0,3,2]
-    v += dpp_take<0x4E, 0xf>(v);    // quad_perm [2,3,0,1]
-    v += dpp_take<0x141, 0xf>(v);   // row_half_mirror
-    v += dpp_take<0x140, 0xf>(v);   // row_mirror: every lane holds the sum of its row of 16
-    v += dpp_take<0x142, 0xa>(v);   // row_bcast:15 into rows 1 and 3
-    v += dpp_take<0x143, 0xc>(v);   // row_bcast:31 into rows 2 and 3: lane 63 holds the total
-    return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), 63));
+template <int H> __device__ __forceinline__ int head_of(int lane) { return (lane & 15) / (16 / H); }
+template <int H> __device__ __forceinline__ constexpr int lane_of(int head) { return head * (16 / H); }
+struct OpMax { static __device__ __forceinline__ float apply(float a, float b) { return fmaxf(a, b); } };
+struct OpSum { static __device__ __forceinline__ float apply(float a, float b) { return a + b; } };
+template <typename OP, int CTRL, int N>
+__device__ __forceinline__ void share_step(float (&v)[N], bool upper) {   // v[0 .. N/2) <- the lane's half, with the partner's values
+    if constexpr (N > 1) {
+#pragma unroll
+        for (int c = 0; c < N / 2; ++c) {
+            const float mine = upper ? v[c + N / 2] : v[c], other = upper ? v[c] : v[c + N / 2];
+            v[c] = OP::apply(mine, dpp_lane<CTRL>(other));
+        }
+    } else {
+        v[0] = OP::apply(v[0], dpp_lane<CTRL>(v[0]));
+    }
 }
-__device__ __forceinline__ float lanes_max(float v) {
-    // (-inf is the neutral element here, so lanes a step does not reach must not contribute 0)
-    auto step = [&](float t, float keep) { return fmaxf(keep, t); };
-    v = step(__builtin_bit_cast(float, __builtin_amdgcn_update_dpp(__builtin_bit_cast(int, v), __builtin_bit_cast(int, v), 0xB1, 0xf, 0xf, false)), v);
-    v = step(__builtin_bit_cast(float, __builtin_amdgcn_update_dpp(__builtin_bit_cast(int, v), __builtin_bit_cast(int, v), 0x4E, 0xf, 0xf, false)), v);
-    v = step(__builtin_bit_cast(float, __builtin_amdgcn_update_dpp(__builtin_bit_cast(int, v), __builtin_bit_cast(int, v), 0x141, 0xf, 0xf, false)), v);
-    v = step(__builtin_bit_cast(float, __builtin_amdgcn_update_dpp(__builtin_bit_cast(int, v), __builtin_bit_cast(int, v), 0x140, 0xf, 0xf, false)), v);
-    v = step(__builtin_bit_cast(float, __builtin_amdgcn_update_dpp(__builtin_bit_cast(int, v), __builtin_bit_cast(int, v), 0x142, 0xa, 0xf, false)), v);
-    v = step(__builtin_bit_cast(float, __builtin_amdgcn_update_dpp(__builtin_bit_cast(int, v), __builtin_bit_cast(int, v), 0x143, 0xc, 0xf, false)), v);
-    return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), 63));
+template <typename OP, int H>
+__device__ __forceinline__ float lanes_share(const float (&v)[H], int lane) {
+    float a[H], b[H > 2 ? H / 2 : 1], c[H > 4 ? H / 4 : 1], d[H > 8 ? H / 8 : 1];
+#pragma unroll
+    for (int k = 0; k < H; ++k) a[k] = v[k];
+    share_step<OP, 0x140, H>(a, lane & 8);
+#pragma unroll
+    for (int k = 0; k < (int)(sizeof(b) / 4); ++k) b[k] = a[k];
+    share_step<OP, 0x141>(b, lane & 4);
+#pragma unroll
+    for (int k = 0; k < (int)(sizeof(c) / 4); ++k) c[k] = b[k];
+    share_step<OP, 0x1B>(c, lane & 2);
+#pragma unroll
+    for (int k = 0; k < (int)(sizeof(d) / 4); ++k) d[k] = c[k];
+    share_step<OP, 0xB1>(d, lane & 1);
+    float t = d[0];
+    t = OP::apply(t, __shfl_xor(t, 16, kWave));
+    t = OP::apply(t, __shfl_xor(t, 32, kWave));
+    return t;
 }
-
-// The same for H values at once, step by step across the heads: the independent chains fill each
-// other's DPP wait states.
+// the value that the lanes of head c hold, wave-uniform
 template <int H>
-__device__ __forceinline__ void lanes_sum_all(float (&v)[H]) {
+__device__ __forceinline__ void lanes_spread(float t, float (&v)[H]) {
 #pragma unroll
-    for (int c = 0; c < H; ++c) v[c] += dpp_take<0xB1, 0xf>(v[c]);
-#pragma unroll
-    for (int c = 0; c < H; ++c) v[c] += dpp_take<0x4E, 0xf>(v[c]);
-#pragma unroll
-    for (int c = 0; c < H; ++c) v[c] += dpp_take<0x141, 0xf>(v[c]);
-#pragma unroll
-    for (int c = 0; c < H; ++c) v[c] += dpp_take<0x140, 0xf>(v[c]);
-#pragma unroll
-    for (int c = 0; c < H; ++c) v[c] += dpp_take<0x142, 0xa>(v[c]);
-#pragma unroll
-    for (int c = 0; c < H; ++c) v[c] += dpp_take<0x143, 0xc>(v[c]);
-#pragma unroll
-    for (int c = 0; c < H; ++c) v[c] = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v[c]), 63));
-}
-template <int CTRL, int ROW_MASK>
-__device__ __forceinline__ float dpp_keep(float v) {   // lanes outside ROW_MASK keep their own value
-    return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(__builtin_bit_cast(int, v), __builtin_bit_cast(int, v), CTRL, ROW_MASK, 0xf, false));
-}
-template <int H>
-__device__ __forceinline__ void lanes_max_all(float (&v)[H]) {
-#pragma unroll
-    for (int c = 0; c < H; ++c) v[c] = fmaxf(v[c], dpp_keep<0xB1, 0xf>(v[c]));
-#pragma unroll
-    for (int c = 0; c < H; ++c) v[c] = fmaxf(v[c], dpp_keep<0x4E, 0xf>(v[c]));
-#pragma unroll
-    for (int c = 0; c < H; ++c) v[c] = fmaxf(v[c], dpp_keep<0x141, 0xf>(v[c]));
-#pragma unroll
-    for (int c = 0; c < H; ++c) v[c] = fmaxf(v[c], dpp_keep<0x140, 0xf>(v[c]));
-#pragma unroll
-    for (int c = 0; c < H; ++c) v[c] = fmaxf(v[c], dpp_keep<0x142, 0xa>(v[c]));
-#pragma unroll
-    for (int c = 0; c < H; ++c) v[c] = fmaxf(v[c], dpp_keep<0x143, 0xc>(v[c]));
-#pragma unroll
-    for (int c = 0; c < H; ++c) v[c] = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v[c]), 63));
+    for (int c = 0; c < H; ++c) v[c] = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, t), lane_of<H>(c)));
 }
 
 // The H scores of one window position, as floats (one or two 16-byte loads for the usual H).
@@ -116,90 +106,108 @@ __device__ __forceinline__ LinkRow link_row(const int64_t *valid_end, int64_t ro
     return r;
 }
 
-// links and lse (the per-head log normalisers, [B][L][H], kept for the backward).  PER window
-// positions per lane: L <= 64 * PER.
-template <typename TC, int H, int PER>
+constexpr int kLinkPer = 4;                       // window positions per lane
+// Sums of products of probabilities are taken as they are down to 2^-100, where terms that left the float32 range (below
+// 2^-126) still do not count; below, and where something overflowed, a position takes the route through its largest term.
+constexpr float kLinkTiny = 7.8886091e-31f, kLinkHuge = 1.2676506e+30f;
+
+// links and lse (the per-head log normalisers, [B][L][H], kept for the backward).  WPR waves share a row: wave `sub` has
+// the chunks sub, sub + WPR, ... of 64 window positions; min(translen, L - 1) <= 64 * kLinkPer * WPR.
+template <typename TC, int H, int WPR>
 __global__ __launch_bounds__(kLinkThreads) void links_fwd_kernel(
     const TC *__restrict__ content, const float *__restrict__ log_gates, const int64_t *__restrict__ valid_end,
     int64_t rows, int L, int translen, TC *__restrict__ links, float *__restrict__ lse_out) {
-    const int lane = threadIdx.x & (kWave - 1);
-    const int64_t row = (int64_t)blockIdx.x * kLinkWaves + threadIdx.x / kWave;
-    if (row >= rows) return;
+    __shared__ float2 part[kLinkWaves][H];
+    const int lane = threadIdx.x & (kWave - 1), wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+    const int sub = wave % WPR, head = head_of<H>(lane);
+    // The last rows first, eight workgroups at a time (a row stays on the XCD that the backward takes it to): they are what
+    // the producer of the scores wrote last, and the first rows, which the backward starts with, are the last that passed
+    // the memory-side cache.
+    const unsigned octet = gridDim.x & ~7u, blk = blockIdx.x < octet ? (octet - 8 - (blockIdx.x & ~7u)) + (blockIdx.x & 7u) : blockIdx.x;
+    const int64_t row = (int64_t)blk * (kLinkWaves / WPR) + wave / WPR;
+    if (row >= rows) { if (WPR > 1) __syncthreads(); return; }   // the one barrier of the others
     // The window is loaded before valid_end is known (up to the end of the row, which always exists), so
     // that a wave waits for one memory round trip, not two; what lies past valid_end is masked afterwards.
     const int i = (int)(row % L);
     const int nmax = L - 1 - i < translen ? L - 1 - i : translen;
     const TC *win = content + (row * L + i + 1) * H;
-    float x[PER][H];
+    float x[kLinkPer][H];
 #pragma unroll
-    for (int k = 0; k < PER; ++k) {
-        const int d = lane + k * kWave;
+    for (int k = 0; k < kLinkPer; ++k) {
+        const int d = lane + (k * WPR + sub) * kWave;
         if (d < nmax) load_heads<TC, H>(win + (int64_t)d * H, x[k]);
     }
+    const float gate2 = log_gates[row * H + head] * kLog2e;
     const LinkRow r = link_row(valid_end, row, L, translen);
     TC *out = links + row * translen;
-    if (r.n == 0) {   // no transition leaves this node
-        for (int d = lane; d < translen; d += kWave) out[d] = from_float<TC>(DAGX_NEG_INF);
-        if (lse_out && lane < H) lse_out[row * H + lane] = DAGX_NEG_INF;
-        return;
-    }
-    // Chunk by chunk (64 positions), only the chunks that reach into the window are worked on (one
-    // wave-uniform test per chunk and pass: rows near the end of a graph are short), and only the chunk
-    // that holds the end of the window needs masking.
-    // per head: maximum, then the sum of exp(x - max) = 2^(x * log2e - max * log2e), over the window
+    // Only the chunks that reach into the window are worked on (one wave-uniform test per chunk and pass: rows near the
+    // end of a graph are short), and only the chunk that holds the end of the window needs masking.
+    // per head: maximum, then the sum of exp(x - max) = 2^(x * log2e - max * log2e), over this wave's part of the window
     float m[H], sum[H];
 #pragma unroll
     for (int c = 0; c < H; ++c) { m[c] = DAGX_NEG_INF; sum[c] = 0.f; }
 #pragma unroll
-    for (int k = 0; k < PER; ++k)
-        if (k * kWave < r.n) {
-            if ((k + 1) * kWave > r.n) {   // the last chunk of the window
-                const bool in = lane + k * kWave < r.n;
+    for (int k = 0; k < kLinkPer; ++k) {
+        const int d0 = (k * WPR + sub) * kWave;
+        if (d0 < r.n) {
+            if (d0 + kWave > r.n) {
+                const bool in = lane + d0 < r.n;
 #pragma unroll
                 for (int c = 0; c < H; ++c) x[k][c] = in ? x[k][c] : DAGX_NEG_INF;
             }
 #pragma unroll
             for (int c = 0; c < H; ++c) m[c] = fmaxf(m[c], x[k][c]);
         }
-    lanes_max_all<H>(m);
-    float shift[H];   // -max * log2e; 0 for a head without any finite score: 2^(-inf) = 0, no NaN
-#pragma unroll
-    for (int c = 0; c < H; ++c) shift[c] = m[c] > DAGX_NEG_INF ? -m[c] * kLog2e : 0.f;
-#pragma unroll
-    for (int k = 0; k < PER; ++k)
-        if (k * kWave < r.n)
-#pragma unroll
-            for (int c = 0; c < H; ++c) sum[c] += fast_exp2(__builtin_fmaf(x[k][c], kLog2e, shift[c]));
-    lanes_sum_all<H>(sum);
-    // bias = (log_gate - lse) in base 2 is what is added to a score of head c (a head without any
-    // finite score drops out)
-    float bias[H];
-    bool any_head = false;
-#pragma unroll
-    for (int c = 0; c < H; ++c) {
-        const float lse2 = m[c] > DAGX_NEG_INF ? fast_log2(sum[c]) - shift[c] : DAGX_NEG_INF;
-        if (lse_out && lane == 0) lse_out[row * H + c] = lse2 * kLn2;
-        bias[c] = lse2 > DAGX_NEG_INF ? __builtin_fmaf(log_gates[row * H + c], kLog2e, -lse2) : DAGX_NEG_INF;
-        any_head = any_head || lse2 > DAGX_NEG_INF;
     }
-    // mix the heads: log2 sum_c 2^(x * log2e + bias_c), lane-local.  Every term is at most 1 (a score
-    // never exceeds its head's normaliser, a gate log-probability is at most 0), so no maximum is needed
-    // unless all terms underflow -- a transition less likely than 2^-126 -- which takes the exact route.
+    const float m_own = lanes_share<OpMax, H>(m, lane);
+    lanes_spread<H>(m_own > DAGX_NEG_INF ? -m_own * kLog2e : 0.f, m);   // 0 for a head without any finite score: 2^(-inf) = 0, no NaN
+    // the scores become e = 2^(x * log2e - max * log2e): their only exponential
 #pragma unroll
-    for (int k = 0; k < PER; ++k) {
-        const int d = lane + k * kWave;
-        if (k * kWave >= translen) break;
+    for (int k = 0; k < kLinkPer; ++k)
+        if ((k * WPR + sub) * kWave < r.n)
+#pragma unroll
+            for (int c = 0; c < H; ++c) { x[k][c] = fast_exp2(__builtin_fmaf(x[k][c], kLog2e, m[c])); sum[c] += x[k][c]; }
+    float top = m_own, tot = lanes_share<OpSum, H>(sum, lane);
+    if (WPR > 1) {
+        if (lane < 16) part[wave][head] = make_float2(top, tot);
+        __syncthreads();
+        const int w0 = wave - sub;
+        float2 q[WPR];
+#pragma unroll
+        for (int w = 0; w < WPR; ++w) { q[w] = part[w0 + w][head]; top = fmaxf(top, q[w].x); }
+        tot = 0.f;
+#pragma unroll
+        for (int w = 0; w < WPR; ++w) tot += q[w].x > DAGX_NEG_INF ? q[w].y * fast_exp2((q[w].x - top) * kLog2e) : q[w].y;
+    }
+    // (a head without any finite score drops out; from here on every lane has the values of its head)
+    const float log_tot = fast_log2(tot);
+    const float lse2 = top > DAGX_NEG_INF ? __builtin_fmaf(top, kLog2e, log_tot) : DAGX_NEG_INF;
+    const bool alive = lse2 > DAGX_NEG_INF;
+    if (lse_out && sub == 0 && lane < 16) lse_out[row * H + head] = lse2 * kLn2;
+    // mix the heads: log2 sum_c e_c * f_c with f = 2^(max - lse + gate), lane-local
+    float f[H];
+    lanes_spread<H>(alive && m_own > DAGX_NEG_INF ? fast_exp2(__builtin_fmaf(m_own - top, kLog2e, gate2 - log_tot)) : 0.f, f);
+    const float bias_own = alive ? gate2 - lse2 : DAGX_NEG_INF;
+#pragma unroll
+    for (int k = 0; k < kLinkPer; ++k) {
+        const int d0 = (k * WPR + sub) * kWave, d = lane + d0;
+        if (d0 >= translen) break;
         float v = DAGX_NEG_INF;
-        if (k * kWave < r.n) {
-            float y[H], acc = 0.f;
+        if (d0 < r.n) {
+            float acc = 0.f;
 #pragma unroll
-            for (int c = 0; c < H; ++c) { y[c] = __builtin_fmaf(x[k][c], kLog2e, bias[c]); acc += fast_exp2(y[c]); }
-            if (d < r.n) {
-                if (__builtin_expect(acc >= 1.17549435e-38f, 1)) v = fast_log2(acc) * kLn2;
-                else if (any_head) {
-                    float ym = DAGX_NEG_INF;
+            for (int c = 0; c < H; ++c) acc = __builtin_fmaf(x[k][c], f[c], acc);
+            const bool slow = d < r.n && !(acc >= kLinkTiny && acc <= kLinkHuge);
+            if (d < r.n) v = fast_log2(acc) * kLn2;
+            if (__builtin_expect(__builtin_amdgcn_ballot_w64(slow) != 0, 0)) {   // from the scores again, against the largest term
+                float bias[H];
+                lanes_spread<H>(bias_own, bias);
+                if (slow) {
+                    float y[H], ym = DAGX_NEG_INF;
+                    load_heads<TC, H>(win + (int64_t)d * H, y);
 #pragma unroll
-                    for (int c = 0; c < H; ++c) ym = fmaxf(ym, y[c]);
+                    for (int c = 0; c < H; ++c) { y[c] = __builtin_fmaf(y[c], kLog2e, bias[c]); ym = fmaxf(ym, y[c]); }
+                    v = DAGX_NEG_INF;
                     if (ym > DAGX_NEG_INF) {
                         float acc2 = 0.f;
 #pragma unroll
@@ -214,112 +222,140 @@ __global__ __launch_bounds__(kLinkThreads) void links_fwd_kernel(
 }
 
 // In place: content[b][i][j][c] <- d loss / d content, 0 outside the window; grad_gates[b][i][c] =
-// d loss / d log_gates.  With y = x - lse_c + g_c and w = grad_links[d] * exp(y - log sum_c' exp(y_c')):
-//   d/dg_c = W_c = sum_d w[d][c],      d/dx[d][c] = w[d][c] - W_c * exp(x[d][c] - lse_c).
-// The normaliser over the heads is formed again from the scores, in float32, and not taken from the stored
-// `links` (which the kernel does not read): rounded to bfloat16 a link value of -6 is 0.03 off, and every weight
-// of its position with it by 3 %.
-template <typename TC, int H, int PER>
+// d loss / d log_gates.  With p = exp(x - lse_c), G_c = exp(g_c) and q_c = grad_links[d] * G_c / sum_c' p_c' G_c':
+//   d/dg_c = W_c = sum_d q[d][c] p[d][c],      d/dx[d][c] = p[d][c] * (q[d][c] - W_c):
+// one exponential per score.  The normaliser over the heads is formed again from the scores, in float32, and not taken
+// from the stored `links` (which the kernel does not read): rounded to bfloat16 a link value of -6 is 0.03 off, and every
+// weight of its position with it by 3 %.
+template <typename TC, int H, int WPR>
 __global__ __launch_bounds__(kLinkThreads) void links_bwd_kernel(
     TC *__restrict__ content, const float *__restrict__ log_gates, const int64_t *__restrict__ valid_end,
-    int64_t rows, int L, int translen, const TC *__restrict__ links, const float *__restrict__ lse_in,
+    int64_t rows, int L, int translen, const float *__restrict__ lse_in,
     const TC *__restrict__ grad_links, float *__restrict__ grad_gates) {
-    const int lane = threadIdx.x & (kWave - 1);
-    const int64_t row = (int64_t)blockIdx.x * kLinkWaves + threadIdx.x / kWave;
-    if (row >= rows) return;
-    const LinkRow r = link_row(valid_end, row, L, translen);
+    __shared__ float part[kLinkWaves][H];
+    const int lane = threadIdx.x & (kWave - 1), wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+    const int sub = wave % WPR, head = head_of<H>(lane);
+    const int64_t row = (int64_t)blockIdx.x * (kLinkWaves / WPR) + wave / WPR;
+    if (row >= rows) { if (WPR > 1) __syncthreads(); return; }   // the one barrier of the others
+    const int i = (int)(row % L);
+    const int nmax = L - 1 - i < translen ? L - 1 - i : translen;
     TC *full = content + row * L * H;
-    float zeros[H];
+    TC *win = full + (int64_t)(i + 1) * H;
+    float x[kLinkPer][H], go[kLinkPer];   // scores, then p; incoming gradient, then grad / sum_c p_c G_c
 #pragma unroll
-    for (int c = 0; c < H; ++c) zeros[c] = 0.f;
-    // outside the window: zeros (nothing of it was read)
-    for (int j = lane; j < L; j += kWave)
-        if (j < r.jlo || j >= r.jlo + r.n) store_heads<TC, H>(full + (int64_t)j * H, zeros);
-    if (r.n == 0) {
-        if (lane < H) grad_gates[row * H + lane] = 0.f;
-        return;
-    }
-    TC *win = full + (int64_t)r.jlo * H;
-    float lse[H], bias[H];
-#pragma unroll
-    for (int c = 0; c < H; ++c) {
-        lse[c] = lse_in[row * H + c];
-        bias[c] = lse[c] > DAGX_NEG_INF ? log_gates[row * H + c] - lse[c] : DAGX_NEG_INF;
-    }
-    // scores, incoming gradient and the link value of every window position of this lane.  When the scores of
-    // a lane do not fit the register file (16 heads x 16 positions) they are not kept: the second pass reads
-    // them again (from L2, the row was just read) instead of spilling them.
-    constexpr bool KEEP = H * PER <= 128;
-    float x[KEEP ? PER : 1][H], go[PER], lo[PER];   // lo: the link value of the position (natural log), formed in the first pass
-#pragma unroll
-    for (int k = 0; k < PER; ++k) {
-        const int d = lane + k * kWave;
-        go[k] = 0.f; lo[k] = DAGX_NEG_INF;
-        if (d < r.n) {
-            if (KEEP) load_heads<TC, H>(win + (int64_t)d * H, x[KEEP ? k : 0]);
+    for (int k = 0; k < kLinkPer; ++k) {
+        const int d = lane + (k * WPR + sub) * kWave;
+        if (d < nmax) {
+            load_heads<TC, H>(win + (int64_t)d * H, x[k]);
             go[k] = to_float(grad_links[row * translen + d]);
-        } else if (KEEP) {
-#pragma unroll
-            for (int c = 0; c < H; ++c) x[KEEP ? k : 0][c] = DAGX_NEG_INF;
         }
     }
-    auto weight = [&](const float (&xk)[H], int k, int c) -> float {   // w[d][c]
-        const float y = xk[c] + bias[c];
-        return (lo[k] > DAGX_NEG_INF && y > DAGX_NEG_INF) ? go[k] * fast_exp2((y - lo[k]) * kLog2e) : 0.f;
-    };
-    // first pass over a position: log sum_c exp(y_c) against the largest y_c (kept in lo[k]), and with the terms
-    // already at hand the position's share of W_c
-    auto first_pass = [&](const float (&xk)[H], int k, float (&wsum)[H]) {
-        float y[H], ym = DAGX_NEG_INF;
-#pragma unroll
-        for (int c = 0; c < H; ++c) { y[c] = (xk[c] + bias[c]) * kLog2e; ym = fmaxf(ym, y[c]); }
-        if (!(ym > DAGX_NEG_INF)) return;   // no head reaches this position (or a NaN score: the weights stay 0, as before)
-        float e[H], acc = 0.f;
-#pragma unroll
-        for (int c = 0; c < H; ++c) { e[c] = fast_exp2(y[c] - ym); acc += e[c]; }
-        lo[k] = (ym + fast_log2(acc)) * kLn2;
-        const float f = go[k] / acc;
-#pragma unroll
-        for (int c = 0; c < H; ++c) wsum[c] += f * e[c];
-    };
-    float wsum[H];
-#pragma unroll
-    for (int c = 0; c < H; ++c) wsum[c] = 0.f;
-#pragma unroll
-    for (int k = 0; k < PER; ++k) {
-        const int d = lane + k * kWave;
-        if (KEEP) {
-            if (d < r.n) first_pass(x[KEEP ? k : 0], k, wsum);
-        } else if (d < r.n) {
-            float xk[H];
-            load_heads<TC, H>(win + (int64_t)d * H, xk);
-            first_pass(xk, k, wsum);
-        }
+    const float lse_own = lse_in[row * H + head], gate_own = log_gates[row * H + head];
+    const LinkRow r = link_row(valid_end, row, L, translen);
+    // outside the window: zeros (nothing of it is used), in contiguous pieces that pass the caches by
+    {
+        typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
+        typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
+        using Piece = std::conditional_t<(sizeof(TC) * H >= 16), u32x4, u32x2>;
+        constexpr int kEach = (int)(sizeof(TC) * H / sizeof(Piece));   // pieces per node
+        Piece *p = reinterpret_cast<Piece *>(full);
+        const int before = r.jlo * kEach, behind = (r.jlo + r.n) * kEach, end = L * kEach;
+        const Piece zero = {};
+        for (int q = lane + sub * kWave; q < before && q < end; q += WPR * kWave) __builtin_nontemporal_store(zero, p + q);
+        for (int q = behind + lane + sub * kWave; q < end; q += WPR * kWave) __builtin_nontemporal_store(zero, p + q);
     }
-    lanes_sum_all<H>(wsum);
-    if (lane < H) {
-        float gsel = 0.f;
-#pragma unroll
-        for (int c = 0; c < H; ++c) gsel = lane == c ? wsum[c] : gsel;
-        grad_gates[row * H + lane] = gsel;
-    }
-#pragma unroll
-    for (int k = 0; k < PER; ++k) {
-        const int d = lane + k * kWave;
-        if (d >= r.n) break;
-        float xk[H], dx[H];
-        if (KEEP) {
-#pragma unroll
-            for (int c = 0; c < H; ++c) xk[c] = x[KEEP ? k : 0][c];
-        } else {
-            load_heads<TC, H>(win + (int64_t)d * H, xk);
-        }
+    const bool alive = lse_own > DAGX_NEG_INF;
+    const bool every_head = __builtin_amdgcn_ballot_w64(alive) == ~0ull;
+    float nlse[H], G[H], wsum[H];
+    lanes_spread<H>(-lse_own * kLog2e, nlse);
+    lanes_spread<H>(fast_exp2(gate_own * kLog2e), G);
+    // The route of the positions whose sum leaves the range, and of rows with a head that reaches no position (or holds a
+    // NaN: it takes no part): from the scores, against the largest term.  w: the position's d/dg_c, pr: exp(x - lse).
+    auto general = [&](int d, float grad, float (&w)[H], float (&pr)[H]) __attribute__((always_inline)) {
+        float lse[H], gate[H], ym = DAGX_NEG_INF, acc = 0.f;
+        lanes_spread<H>(lse_own, lse);
+        lanes_spread<H>(gate_own, gate);
+        load_heads<TC, H>(win + (int64_t)d * H, pr);
 #pragma unroll
         for (int c = 0; c < H; ++c) {
-            const float p = (lse[c] > DAGX_NEG_INF && xk[c] > DAGX_NEG_INF) ? fast_exp2((xk[c] - lse[c]) * kLog2e) : 0.f;
-            dx[c] = weight(xk, k, c) - wsum[c] * p;
+            const float bias = lse[c] > DAGX_NEG_INF ? gate[c] - lse[c] : DAGX_NEG_INF;
+            w[c] = (pr[c] + bias) * kLog2e;
+            ym = fmaxf(ym, w[c]);
+            pr[c] = (lse[c] > DAGX_NEG_INF && pr[c] > DAGX_NEG_INF) ? fast_exp2((pr[c] - lse[c]) * kLog2e) : 0.f;
         }
-        store_heads<TC, H>(win + (int64_t)d * H, dx);
+        const bool some = ym > DAGX_NEG_INF;   // else no head reaches this position (or a NaN score: the weights stay 0)
+#pragma unroll
+        for (int c = 0; c < H; ++c) {
+            w[c] = some && w[c] > DAGX_NEG_INF ? fast_exp2(w[c] - ym) : 0.f;
+            acc += w[c];
+        }
+        const float t = some ? grad / acc : 0.f;
+#pragma unroll
+        for (int c = 0; c < H; ++c) w[c] = some ? w[c] * t : 0.f;
+    };
+#pragma unroll
+    for (int c = 0; c < H; ++c) wsum[c] = 0.f;
+    unsigned slow = 0;   // bit k: position k takes the general route
+#pragma unroll
+    for (int k = 0; k < kLinkPer; ++k) {
+        const int d0 = (k * WPR + sub) * kWave, d = lane + d0;
+        if (d0 < r.n) {
+            const bool in = d < r.n;
+            float acc = 0.f;
+#pragma unroll
+            for (int c = 0; c < H; ++c) {
+                x[k][c] = fast_exp2(__builtin_fmaf(x[k][c], kLog2e, nlse[c]));
+                acc = __builtin_fmaf(x[k][c], G[c], acc);
+            }
+            const bool fine = every_head && acc >= kLinkTiny && acc <= kLinkHuge;
+            const float grad = go[k];
+            go[k] = in && fine ? grad / acc : 0.f;
+            if (in && fine) {
+#pragma unroll
+                for (int c = 0; c < H; ++c) wsum[c] = __builtin_fmaf(go[k] * G[c], x[k][c], wsum[c]);   // (0 + q p: rounded once)
+            }
+            if (__builtin_expect(__builtin_amdgcn_ballot_w64(in && !fine) != 0, 0)) {
+                float w[H], pr[H];
+                const bool mine = in && !fine;
+                general(mine ? d : 0, grad, w, pr);
+                if (mine) {
+                    slow |= 1u << k;
+#pragma unroll
+                    for (int c = 0; c < H; ++c) wsum[c] += w[c];
+                }
+            }
+        }
+    }
+    float W_own = lanes_share<OpSum, H>(wsum, lane);
+    if (WPR > 1) {
+        if (lane < 16) part[wave][head] = W_own;
+        __syncthreads();
+        const int w0 = wave - sub;
+        W_own = 0.f;
+#pragma unroll
+        for (int w = 0; w < WPR; ++w) W_own += part[w0 + w][head];
+    }
+    if (sub == 0 && lane < 16) grad_gates[row * H + head] = W_own;
+    float W[H];
+    lanes_spread<H>(W_own, W);
+#pragma unroll
+    for (int k = 0; k < kLinkPer; ++k) {
+        const int d0 = (k * WPR + sub) * kWave, d = lane + d0;
+        if (d0 >= r.n) break;
+        float dx[H];
+#pragma unroll
+        for (int c = 0; c < H; ++c) dx[c] = x[k][c] * (go[k] * G[c] - W[c]);   // (the product as in W: a window of one position gives 0)
+        if (__builtin_expect(__builtin_amdgcn_ballot_w64((slow >> k) & 1u) != 0, 0)) {
+            const bool mine = (slow >> k) & 1u;
+            const float grad = d < r.n ? to_float(grad_links[row * translen + d]) : 0.f;
+            float w[H], pr[H];
+            general(mine ? d : 0, grad, w, pr);
+            if (mine) {
+#pragma unroll
+                for (int c = 0; c < H; ++c) dx[c] = w[c] - W[c] * pr[c];
+            }
+        }
+        if (d < r.n) store_heads<TC, H>(win + (int64_t)d * H, dx);
     }
 }
 
@@ -334,27 +370,27 @@ static int check_links(const void *content, int dtype, const void *log_gates, co
     return DAGX_OK;
 }
 
-// window positions per lane: the smallest of 4, 8, 16 that covers the row
+// Waves per row: the fewest that hold the longest window at kLinkPer positions a lane.
 template <typename TC, int H>
 static int launch_links_fwd(const void *content, const float *log_gates, const int64_t *valid_end, int B, int L, int translen,
                             void *links, float *lse, hipStream_t st) {
     const int64_t rows = (int64_t)B * L;
-    const dim3 grid((unsigned)((rows + kLinkWaves - 1) / kLinkWaves)), block(kLinkThreads);
-#define DAGX_GO(PER) hipLaunchKernelGGL((links_fwd_kernel<TC, H, PER>), grid, block, 0, st, static_cast<const TC *>(content), \
-                                        log_gates, valid_end, rows, L, translen, static_cast<TC *>(links), lse)
-    if (L <= 4 * kWave) DAGX_GO(4); else if (L <= 8 * kWave) DAGX_GO(8); else DAGX_GO(16);
+    const int n = translen < L - 1 ? translen : L - 1;
+#define DAGX_GO(WPR) hipLaunchKernelGGL((links_fwd_kernel<TC, H, WPR>), dim3((unsigned)((rows * WPR + kLinkWaves - 1) / kLinkWaves)), dim3(kLinkThreads), 0, st, \
+                                        static_cast<const TC *>(content), log_gates, valid_end, rows, L, translen, static_cast<TC *>(links), lse)
+    if (n <= kLinkPer * kWave) DAGX_GO(1); else if (n <= 2 * kLinkPer * kWave) DAGX_GO(2); else DAGX_GO(4);
 #undef DAGX_GO
     return check_launch("links_fwd");
 }
 template <typename TC, int H>
 static int launch_links_bwd(void *content, const float *log_gates, const int64_t *valid_end, int B, int L, int translen,
-                            const void *links, const float *lse, const void *grad_links, float *grad_gates, hipStream_t st) {
+                            const float *lse, const void *grad_links, float *grad_gates, hipStream_t st) {
     const int64_t rows = (int64_t)B * L;
-    const dim3 grid((unsigned)((rows + kLinkWaves - 1) / kLinkWaves)), block(kLinkThreads);
-#define DAGX_GO(PER) hipLaunchKernelGGL((links_bwd_kernel<TC, H, PER>), grid, block, 0, st, static_cast<TC *>(content), log_gates, \
-                                        valid_end, rows, L, translen, static_cast<const TC *>(links), lse,                         \
+    const int n = translen < L - 1 ? translen : L - 1;
+#define DAGX_GO(WPR) hipLaunchKernelGGL((links_bwd_kernel<TC, H, WPR>), dim3((unsigned)((rows * WPR + kLinkWaves - 1) / kLinkWaves)), dim3(kLinkThreads), 0, st, \
+                                        static_cast<TC *>(content), log_gates, valid_end, rows, L, translen, lse,                                               \
                                         static_cast<const TC *>(grad_links), grad_gates)
-    if (L <= 4 * kWave) DAGX_GO(4); else if (L <= 8 * kWave) DAGX_GO(8); else DAGX_GO(16);
+    if (n <= kLinkPer * kWave) DAGX_GO(1); else if (n <= 2 * kLinkPer * kWave) DAGX_GO(2); else DAGX_GO(4);
 #undef DAGX_GO
     return check_launch("links_bwd");
 }
@@ -390,7 +426,7 @@ extern "C" int dagx_links_bwd(void *content_inout, int dtype, const float *log_g
     if (B == 0) return DAGX_OK;
     if (!lse || !grad_links || !grad_gates) { set_error("dag_links_bwd: a saved-state or output pointer is null"); return DAGX_ERR_ARGUMENT; }
     hipStream_t st = static_cast<hipStream_t>(stream);
-#define CALL(T, HH) launch_links_bwd<T, HH>(content_inout, log_gates, valid_end, B, L, translen, links, lse, grad_links, grad_gates, st)
+#define CALL(T, HH) launch_links_bwd<T, HH>(content_inout, log_gates, valid_end, B, L, translen, lse, grad_links, grad_gates, st)
     DAGX_LINKS_DISPATCH(CALL)
 #undef CALL
 }

@@ -38,7 +38,8 @@ def _compare(got, want, rtol, atol):
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("B,L,H,translen", [(3, 17, 8, 5), (2, 70, 4, 100), (2, 300, 16, 64), (1, 1024, 8, 1023),
-                                            (1, 600, 16, 599), (1, 1024, 16, 1023), (1, 498, 4, 497), (1, 786, 4, 785)])
+                                            (1, 600, 16, 599), (1, 1024, 16, 1023), (1, 498, 4, 497), (1, 786, 4, 785),
+                                            (1, 257, 8, 256), (3, 259, 16, 257), (1, 513, 8, 512), (1, 515, 4, 513), (5, 3, 8, 2)])
 def test_forward_and_backward_match_oracle(dtype, B, L, H, translen):
     content, gates, lens = _case(B, L, H, dtype)
     mask = _mask(lens, L)
@@ -107,6 +108,29 @@ def test_feeds_dag_loss_and_extreme_scores():
     loss = dagx.dag_loss(match, links, ol, tl)
     loss.sum().backward()
     assert torch.isfinite(loss).all() and torch.isfinite(c.grad).all() and c.grad.abs().sum() > 0
+
+
+@pytest.mark.parametrize("B,L,H", [(2, 120, 4), (1, 300, 8), (1, 700, 16)])
+def test_scores_that_leave_the_float32_range(B, L, H):
+    """Score ranges of several hundred: most positions are less likely than 2^-100, where the kernels turn from plain
+    sums of probabilities to sums against the largest term -- with and without a head that reaches no position.  The
+    tolerances: scores of 300 are rounded to 2^-16 relative to 1, and every probability with them."""
+    content, gates, lens = _case(B, L, H, torch.float32, seed=L, scale=60.0)
+    gates[:, ::3] = gates[:, ::3] * 30
+    gates[0, 5, 1] = NEG_INF
+    mask = _mask(lens, L)
+    vend = lens[:, None].expand(-1, L).contiguous()
+    c64 = content.double().requires_grad_(); g64 = gates.double().requires_grad_()
+    want = tn.multihead_links(c64, g64, mask, L - 1)
+    weight = torch.randn(want.shape, generator=torch.Generator().manual_seed(5))
+    (want.masked_fill(want == NEG_INF, 0.0) * weight.double()).sum().backward()
+    c = content.to(DEV).requires_grad_(); g = gates.to(DEV).requires_grad_()
+    got = dagx.dag_multihead_links(c * 1, g, vend.to(DEV), L - 1)
+    _compare(got.detach().cpu().double(), want.detach(), 1e-5, 2e-4)
+    (got.masked_fill(got == NEG_INF, 0.0) * weight.to(DEV)).sum().backward()
+    for mine, ref in ((c.grad, c64.grad), (g.grad, g64.grad)):
+        ref = ref.nan_to_num(0.0)                          # (the oracle's gate of -inf)
+        assert torch.allclose(mine.cpu().double(), ref, rtol=2e-4, atol=2e-4 * ref.abs().max().item())
 
 
 def test_full_size_properties():
