@@ -5,6 +5,7 @@ import pytest
 import torch
 
 import da_transformer_amd as dagx
+from da_transformer_amd.custom_ops.glat import _force_emit
 from oracle import torch_native as tn
 from helpers import random_problem
 from test_oracle_glat import random_case
@@ -37,7 +38,7 @@ def _force_case(seed, B, T, L, dup=False):
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
-@pytest.mark.parametrize("B,T,L", [(3, 7, 20), (4, 16, 64), (2, 9, 300), (1, 1, 1)])
+@pytest.mark.parametrize("B,T,L", [(3, 7, 20), (4, 16, 64), (2, 9, 300), (1, 1, 1), (2, 65, 129), (3, 128, 128), (2, 63, 1024)])
 @pytest.mark.parametrize("transposed", [False, True])
 def test_force_alignment_forward_is_bit_exact(dtype, B, T, L, transposed):
     gen = torch.Generator().manual_seed(B * 100 + T)
@@ -53,6 +54,8 @@ def test_force_alignment_forward_is_bit_exact(dtype, B, T, L, transposed):
     got = dagx.dag_force_alignment(dev, force.to(DEV))
     assert got.is_contiguous()
     _same(got, want)
+    forced = (force.unsqueeze(1) == torch.arange(T).view(1, T, 1)).any(2)        # the rule of the gradient, on the same values
+    _same(_force_emit(dev, force.to(DEV), True), torch.where(forced.unsqueeze(2), torch.zeros_like(match), match))
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.float16])
