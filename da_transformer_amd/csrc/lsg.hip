@@ -125,7 +125,12 @@ __global__ __launch_bounds__(BLOCK) void lsg_fwd_kernel(
     float *__restrict__ sel, int64_t ss0, int64_t ss1, int64_t ss2,
     float *__restrict__ lse_out, int64_t *__restrict__ argmax_out = nullptr, float *__restrict__ maxlogp_out = nullptr) {
     constexpr int N = Pack<T>::N;
-    const int64_t row = blockIdx.x;
+    // Last rows first, eight at a time (a row stays on the XCD that the backward takes it to): what the producer of the
+    // logits, or a backward in the same storage, wrote last is still in the memory-side cache or on its way out of it, and
+    // so are the first rows when the backward begins with them.  [64,512,40000] float16, 64 ids: forward behind a backward
+    // 468.7 -> 444.3 us, backward 890.2 -> 883.1 us; [16,512,16000] 58.1 -> 55.6 us forward; smaller ones the same.
+    const unsigned octet = gridDim.x & ~7u;
+    const int64_t row = blockIdx.x < octet ? (octet - 8 - (blockIdx.x & ~7u)) + (blockIdx.x & 7u) : blockIdx.x;
     const int tid = threadIdx.x;
     const T *xr = x + row * V;
     int head; int64_t nvec, tail0;
