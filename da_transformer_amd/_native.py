@@ -2,7 +2,9 @@
 
 There is no fallback: if the library is missing or a call fails, a RuntimeError is raised.
 """
+import contextlib
 import ctypes
+import functools
 import os
 
 import torch
@@ -89,8 +91,21 @@ def ptr(t):
     return None if t is None else t.data_ptr()
 
 
+def raw_stream(index):
+    """Handle of the current stream of device `index` (without the Stream object around it: 0.2 us instead of 3)."""
+    return torch._C._cuda_getCurrentRawStream(index)
+
+
 def stream_of(t):
-    return torch.cuda.current_stream(t.device).cuda_stream
+    return raw_stream(t.device.index)
+
+
+_SAME_DEVICE = contextlib.nullcontext()
+
+
+def on_device(dev):
+    """`with on_device(t.device)`: the tensor's device made the current one -- nothing to do, and nothing done, where it is."""
+    return _SAME_DEVICE if torch.cuda.current_device() == dev.index else torch.cuda.device(dev)
 
 
 def check(rc):
@@ -98,5 +113,7 @@ def check(rc):
         raise RuntimeError("dagx: " + lib().dagx_last_error().decode())
 
 
+@functools.lru_cache(maxsize=1024)
 def workspace_bytes(op, B, T, L, translen):
+    """A function of its arguments alone; a training run meets the same few shapes again and again."""
     return int(lib().dagx_workspace_bytes(op, B, T, L, translen))

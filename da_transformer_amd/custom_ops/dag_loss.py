@@ -22,11 +22,17 @@ __all__ = ["dag_loss", "dag_best_alignment", "dag_logsoftmax_gather_inplace",
            "DagLossFunc", "DagBestAlignmentFunc", "DagLogsoftmaxGatherFunc", "get_dag_kernel"]
 
 
+_gpu_found = False
+
+
 def get_dag_kernel():
     """Handle of the native library (fs_plugins/custom_ops/dag_loss.py:36-63 compiles its
     extension here; this one is built ahead of time).  Raises RuntimeError without a GPU."""
-    if not torch.cuda.is_available():
-        raise RuntimeError("You need GPU to use the custom DAG operations")
+    global _gpu_found
+    if not _gpu_found:
+        if not torch.cuda.is_available():
+            raise RuntimeError("You need GPU to use the custom DAG operations")
+        _gpu_found = True   # (asking the runtime again on every call would cost it a few microseconds)
     return nat.lib()
 
 
@@ -36,7 +42,7 @@ _clean_workspaces = {}
 def _clean_workspace(dev, nbytes):
     """Zero-filled scratch for dagx_loss_fwd.  The library needs it zero on entry and leaves it zero,
     so one buffer per (device, stream) is allocated once and handed to every call on that stream."""
-    key = (dev.index, torch.cuda.current_stream(dev).cuda_stream)
+    key = (dev.index, nat.raw_stream(dev.index))
     ws = _clean_workspaces.get(key)
     if ws is None or ws.numel() < nbytes:
         ws = torch.zeros(max(nbytes, 8), dtype=torch.uint8, device=dev)
@@ -46,7 +52,7 @@ def _clean_workspace(dev, nbytes):
 
 def _forget_workspace(dev):
     """After a failed call the buffer may hold words of an unfinished launch: the next call allocates a new one."""
-    _clean_workspaces.pop((dev.index, torch.cuda.current_stream(dev).cuda_stream), None)
+    _clean_workspaces.pop((dev.index, nat.raw_stream(dev.index)), None)
 
 
 def _check_dag_inputs(match_all, links, output_length, target_length, who):
@@ -65,6 +71,19 @@ def _check_dag_inputs(match_all, links, output_length, target_length, who):
         raise RuntimeError(f"{who}: inputs live on different devices")
     if match_all.dtype != torch.float64 or links.dtype != torch.float64:   # (float64: kernels of their own, both tensors)
         nat.dtype_code(match_all), nat.dtype_code(links)
+
+
+def _sweep_tables(bsz, tarlen, prelen):
+    """How the forward's tables share one allocation: its size in bytes, and the byte offsets of the residuals of
+    both sweeps and of their block offsets; the read-outs logz [2, bsz] lie at its start.  float64 first, every table on a
+    multiple of 256 bytes."""
+    def room(nbytes):
+        return (nbytes + 255) & ~255
+    offs = room(16 * bsz)
+    each_off = room(8 * bsz * tarlen * ((prelen + 63) // 64))
+    hats = offs + 2 * each_off
+    each_hat = room(4 * bsz * tarlen * prelen)
+    return hats + 2 * each_hat, (hats, hats + each_hat, offs, offs + each_off)
 
 
 class DagLossFunc(Function):
@@ -88,12 +107,11 @@ class DagLossFunc(Function):
         bsz, tarlen, prelen = match_all.shape
         translen = links.shape[2]
         dev = match_all.device
-        nblk = (prelen + 63) // 64
-        with torch.cuda.device(dev):
-            # sweep results: fp32 residuals + fp64 block offsets (see include/dagx.h)
-            hats = torch.empty(2, bsz, tarlen, prelen, dtype=torch.float32, device=dev)
-            offs = torch.empty(2, bsz, tarlen, nblk, dtype=torch.float64, device=dev)
-            logz = torch.empty(2, bsz, dtype=torch.float64, device=dev)
+        with nat.on_device(dev):
+            # sweep results: fp64 block offsets and read-outs, fp32 residuals (see include/dagx.h), in one allocation
+            tables, at = _sweep_tables(bsz, tarlen, prelen)
+            state = torch.empty(tables, dtype=torch.uint8, device=dev)
+            base = state.data_ptr()
             # a tensor of its own, not a view of anything made here: the criterion overwrites entries of
             # the returned loss in place (fs_plugins/criterions/nat_dag_loss.py:190-191)
             loss = torch.empty(bsz, dtype=torch.float32, device=dev)
@@ -104,32 +122,34 @@ class DagLossFunc(Function):
                 nat.check(nat.lib().dagx_loss_fwd(
                     nat.ptr(match_all), nat.dtype_code(match_all), nat.strides3(match_all),
                     nat.ptr(links), nat.dtype_code(links), nat.ptr(output_length), nat.ptr(target_length),
-                    bsz, tarlen, prelen, translen, nat.ptr(hats[0]), nat.ptr(hats[1]), nat.ptr(offs[0]), nat.ptr(offs[1]),
-                    nat.ptr(logz), nat.ptr(loss), nat.ptr(flags), int(need_grad), nat.ptr(ws), nbytes, nat.stream_of(match_all)))
+                    bsz, tarlen, prelen, translen, base + at[0], base + at[1], base + at[2], base + at[3],
+                    base, nat.ptr(loss), nat.ptr(flags), int(need_grad), nat.ptr(ws), nbytes, nat.stream_of(match_all)))
             except RuntimeError:
                 _forget_workspace(dev)
                 raise
         DagLossFunc.last_sample_flags = flags
-        ctx.save_for_backward(hats, offs, logz, flags, match_all, links, output_length, target_length)
+        ctx.save_for_backward(state, flags, match_all, links, output_length, target_length)
         # with gradients this is the beta read-out (the partition function the backward uses), else alpha's
         return loss
 
     @staticmethod
     def backward(ctx, grad_output):
-        hats, offs, logz, flags, match_all, links, output_length, target_length = ctx.saved_tensors
+        state, flags, match_all, links, output_length, target_length = ctx.saved_tensors
         want_match, want_links = ctx.needs_input_grad[0], ctx.needs_input_grad[1]
         if not (want_match or want_links):
             return None, None, None, None
         bsz, tarlen, prelen = match_all.shape
         translen = links.shape[2]
-        grad_output = grad_output.to(torch.float32)
-        with torch.cuda.device(match_all.device):
+        base, at = state.data_ptr(), _sweep_tables(bsz, tarlen, prelen)[1]
+        if grad_output.dtype != torch.float32:
+            grad_output = grad_output.to(torch.float32)
+        with nat.on_device(match_all.device):
             grad_match = torch.empty(bsz, tarlen, prelen, dtype=match_all.dtype, device=match_all.device) \
                 if want_match else None
             grad_links = torch.empty_like(links) if want_links else None
             nat.check(nat.lib().dagx_loss_bwd(
-                nat.ptr(grad_output), grad_output.stride(0), nat.ptr(hats[0]), nat.ptr(hats[1]),
-                nat.ptr(offs[0]), nat.ptr(offs[1]), nat.ptr(logz), nat.ptr(flags),
+                nat.ptr(grad_output), grad_output.stride(0), base + at[0], base + at[1],
+                base + at[2], base + at[3], base, nat.ptr(flags),
                 nat.ptr(match_all), nat.dtype_code(match_all), nat.strides3(match_all),
                 nat.ptr(links), nat.dtype_code(links), nat.ptr(output_length), nat.ptr(target_length),
                 bsz, tarlen, prelen, translen, nat.ptr(grad_match), nat.ptr(grad_links),
@@ -165,7 +185,7 @@ class DagBestAlignmentFunc(Function):
         target_length = target_length.contiguous()
         bsz, tarlen, prelen = match_all.shape
         translen = links.shape[2]
-        with torch.cuda.device(match_all.device):
+        with nat.on_device(match_all.device):
             path = torch.empty(bsz, prelen, dtype=torch.int64, device=match_all.device)
             nbytes = nat.workspace_bytes(nat.OP_BEST_ALIGNMENT, bsz, tarlen, prelen, translen)
             ws = torch.empty(nbytes, dtype=torch.uint8, device=match_all.device) if nbytes else None
@@ -226,7 +246,7 @@ class DagLogsoftmaxGatherFunc(Function):
         bsz, prelen, vocab = word_ins_out.shape
         slen = select_idx.shape[2]
         require_gradient = ctx.needs_input_grad[0]
-        with torch.cuda.device(word_ins_out.device):
+        with nat.on_device(word_ins_out.device):
             if transposed_storage:
                 selected = torch.empty(bsz, slen, prelen, dtype=torch.float32, device=word_ins_out.device).transpose(1, 2)
             else:
@@ -259,7 +279,7 @@ class DagLogsoftmaxGatherFunc(Function):
         slen = select_idx.shape[2]
         if grad_output.dtype != torch.float32:
             grad_output = grad_output.float()
-        with torch.cuda.device(grad_input.device):
+        with nat.on_device(grad_input.device):
             nat.check(nat.lib().dagx_lsg_bwd(
                 nat.ptr(grad_input), nat.dtype_code(grad_input), bsz, prelen, vocab, slen,
                 nat.ptr(select_idx), nat.strides3(select_idx), nat.ptr(grad_output), nat.strides3(grad_output),
@@ -308,7 +328,7 @@ def dag_logsoftmax_gather_argmax(word_ins_out, select_idx, transposed_storage=Fa
     bsz, prelen, vocab = word_ins_out.shape
     slen = select_idx.shape[2]
     dev = word_ins_out.device
-    with torch.cuda.device(dev):
+    with nat.on_device(dev):
         if transposed_storage:
             selected = torch.empty(bsz, slen, prelen, dtype=torch.float32, device=dev).transpose(1, 2)
         else:
@@ -333,7 +353,7 @@ def dag_logsoftmax_max(output_logits):
         raise RuntimeError("dag_logsoftmax_max: output_logits must be a contiguous 3-d GPU tensor")
     bsz, prelen, vocab = output_logits.shape
     dev = output_logits.device
-    with torch.cuda.device(dev):
+    with nat.on_device(dev):
         tokens = torch.empty(bsz, prelen, dtype=torch.int64, device=dev)
         values = torch.empty(bsz, prelen, dtype=torch.float32, device=dev)
         nat.check(nat.lib().dagx_lsg_fwd_argmax(

@@ -13,6 +13,29 @@ ViterbiResult = namedtuple("ViterbiResult", "output_tokens output_scores pred_le
 LookaheadResult = namedtuple("LookaheadResult", "output_tokens output_scores nodes")
 
 
+def _outputs(bsz, width, dev):
+    """nodes and tokens [bsz, width] and token counts [bsz], the last two next to each other."""
+    flat = torch.empty(bsz * (2 * width + 1), dtype=torch.int64, device=dev)
+    nodes, tokens = flat[:2 * bsz * width].view(2, bsz, width).unbind(0)
+    return flat[bsz * width:], nodes, tokens, flat[2 * bsz * width:]
+
+
+# Up to this much is copied to the host in one go with the counts, unused columns included, for one synchronisation
+# instead of two and no kernels to find the longest output and to cut the columns off.
+_COPY_WHOLE_BYTES = 128 * 1024
+
+
+def _tokens_on_host(both, tokens, counts):
+    """tokens[:, :longest] as a CPU tensor; both: the tokens with the counts behind them."""
+    bsz, width = tokens.shape
+    if bsz == 0:
+        return tokens[:, :0].cpu()
+    if both.numel() * 8 > _COPY_WHOLE_BYTES:
+        return tokens[:, :max(counts.tolist())].cpu()
+    host = both.cpu()
+    return host[:bsz * width].view(bsz, width)[:, :max(host[bsz * width:].tolist())].clone(memory_format=torch.contiguous_format)
+
+
 def _node_scores(name, links, output_logits_normalized, output_length):
     get_dag_kernel()
     if isinstance(output_logits_normalized, (tuple, list)):
@@ -40,15 +63,13 @@ def dag_lookahead_decode(links, output_logits_normalized, output_length, decode_
     bsz, prelen, translen = links.shape
     links = links.contiguous()
     output_length = output_length.contiguous()
-    with torch.cuda.device(links.device):
-        out_tokens, nodes = torch.empty((2, bsz, prelen), dtype=torch.int64, device=links.device).unbind(0)
-        out_count = torch.empty(bsz, dtype=torch.int64, device=links.device)
+    with nat.on_device(links.device):
+        both, nodes, out_tokens, out_count = _outputs(bsz, prelen, links.device)
         nat.check(nat.lib().dagx_lookahead_decode(
             nat.ptr(links), nat.dtype_code(links), nat.ptr(node_logp), nat.ptr(node_tokens), nat.ptr(output_length),
             bsz, prelen, translen, float(decode_beta), int(bool(greedy)), int(pad_index),
             nat.ptr(out_tokens), nat.ptr(out_count), nat.ptr(nodes), nat.stream_of(links)))
-    longest = int(out_count.max()) if bsz else 0
-    output_tokens = out_tokens[:, :longest].cpu()
+    output_tokens = _tokens_on_host(both, out_tokens, out_count)
     return LookaheadResult(output_tokens, torch.full(output_tokens.size(), 1.0), nodes)
 
 
@@ -73,9 +94,9 @@ def dag_viterbi_decode(links, output_logits_normalized, output_length, decode_up
     output_length = output_length.contiguous()
     # the reference's penalty tensor, computed the same way on the host
     penalty = ((torch.arange(max_length) + 1) ** decode_viterbibeta).to(torch.float32).to(links.device)
-    with torch.cuda.device(links.device):
-        out_tokens, nodes = torch.empty((2, bsz, max_length), dtype=torch.int64, device=links.device).unbind(0)
-        out_count, pred_length = torch.empty((2, bsz), dtype=torch.int64, device=links.device).unbind(0)
+    with nat.on_device(links.device):
+        both, nodes, out_tokens, out_count = _outputs(bsz, max_length, links.device)
+        pred_length = torch.empty(bsz, dtype=torch.int64, device=links.device)
         nbytes = nat.workspace_bytes(nat.OP_VITERBI_DECODE, bsz, max_length, prelen, translen)
         ws = torch.empty(nbytes, dtype=torch.uint8, device=links.device) if nbytes else None
         nat.check(nat.lib().dagx_viterbi_decode(
@@ -83,6 +104,5 @@ def dag_viterbi_decode(links, output_logits_normalized, output_length, decode_up
             bsz, prelen, translen, max_length, nat.ptr(penalty), int(bool(joint)), int(pad_index),
             nat.ptr(out_tokens), nat.ptr(out_count), nat.ptr(pred_length), nat.ptr(nodes),
             nat.ptr(ws), nbytes, nat.stream_of(links)))
-    longest = int(out_count.max()) if bsz else 0
-    output_tokens = out_tokens[:, :longest].cpu()
+    output_tokens = _tokens_on_host(both, out_tokens, out_count)
     return ViterbiResult(output_tokens, torch.full(output_tokens.size(), 1.0), pred_length, nodes)

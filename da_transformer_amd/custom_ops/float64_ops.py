@@ -24,7 +24,7 @@ class DagLossFunc64(Function):
         bsz, tarlen, prelen = match_all.shape
         translen = links.shape[2]
         dev = match_all.device
-        with torch.cuda.device(dev):
+        with nat.on_device(dev):
             alpha = torch.empty(bsz, tarlen, prelen, dtype=torch.float64, device=dev)
             beta = torch.empty_like(alpha) if need_grad else None
             loss = torch.empty(bsz, dtype=torch.float64, device=dev)
@@ -48,7 +48,7 @@ class DagLossFunc64(Function):
         bsz, tarlen, prelen = match_all.shape
         translen = links.shape[2]
         grad_output = grad_output.to(torch.float64)
-        with torch.cuda.device(match_all.device):
+        with nat.on_device(match_all.device):
             grad_match = torch.empty(bsz, tarlen, prelen, dtype=torch.float64, device=match_all.device) if want_match else None
             grad_links = torch.empty_like(links) if want_links else None
             nat.check(nat.lib().dagx_loss_f64_bwd(
@@ -67,7 +67,7 @@ def best_alignment_f64(match_all, links, output_length, target_length):
     bsz, tarlen, prelen = match_all.shape
     translen = links.shape[2]
     dev = match_all.device
-    with torch.cuda.device(dev):
+    with nat.on_device(dev):
         path = torch.empty(bsz, prelen, dtype=torch.int64, device=dev)
         nbytes = nat.workspace_bytes(nat.OP_BEST_ALIGNMENT_F64, bsz, tarlen, prelen, translen)
         ws = torch.empty(max(nbytes, 8) // 8, dtype=torch.float64, device=dev)
@@ -88,7 +88,7 @@ class DagLogsoftmaxGatherFunc64(Function):
         slen = select_idx.shape[2]
         dev = word_ins_out.device
         require_gradient = ctx.needs_input_grad[0]
-        with torch.cuda.device(dev):
+        with nat.on_device(dev):
             if transposed_storage:
                 selected = torch.empty(bsz, slen, prelen, dtype=torch.float64, device=dev).transpose(1, 2)
             else:
@@ -117,7 +117,7 @@ class DagLogsoftmaxGatherFunc64(Function):
         bsz, prelen, vocab = grad_input.shape
         slen = select_idx.shape[2]
         grad_output = grad_output.to(torch.float64)
-        with torch.cuda.device(grad_input.device):
+        with nat.on_device(grad_input.device):
             nat.check(nat.lib().dagx_lsg_f64_bwd(
                 nat.ptr(grad_input), bsz, prelen, vocab, slen, nat.ptr(select_idx), nat.strides3(select_idx),
                 nat.ptr(grad_output), nat.strides3(grad_output), nat.ptr(lse), nat.stream_of(grad_input)))

@@ -13,7 +13,7 @@ from .dag_loss import get_dag_kernel
 def _force_emit(match, force_emit, gradient):
     bsz, tarlen, prelen = match.shape
     out = torch.empty(bsz, tarlen, prelen, dtype=match.dtype, device=match.device)
-    with torch.cuda.device(match.device):
+    with nat.on_device(match.device):
         nat.check(nat.lib().dagx_force_emit(
             nat.ptr(match), nat.dtype_code(match), nat.strides3(match), nat.ptr(force_emit),
             bsz, tarlen, prelen, int(gradient), nat.ptr(out), nat.stream_of(match)))
@@ -74,7 +74,7 @@ def dag_glat_oracle(path, tgt_tokens, pred_tokens, glat_prev_mask=None):
         raise RuntimeError("dag_glat_oracle: tgt_tokens must be [batch, tarlen]")
     path, tgt_tokens, pred_tokens = path.contiguous(), tgt_tokens.contiguous(), pred_tokens.contiguous()
     mask = None if glat_prev_mask is None else glat_prev_mask.contiguous()
-    with torch.cuda.device(path.device):
+    with nat.on_device(path.device):
         oracle = torch.empty_like(path)
         same_num = torch.empty(bsz, dtype=torch.int64, device=path.device)
         nat.check(nat.lib().dagx_glat_glance(
@@ -96,7 +96,7 @@ def dag_glat_mix(path, oracle, prev_output_tokens, keep_prob, rand, glat_prev_ma
     path, oracle, prev = path.contiguous(), oracle.contiguous(), prev_output_tokens.contiguous()
     keep_prob, rand = keep_prob.contiguous(), rand.contiguous()
     mask = None if glat_prev_mask is None else glat_prev_mask.contiguous()
-    with torch.cuda.device(path.device):
+    with nat.on_device(path.device):
         keep = torch.empty(shape, dtype=torch.bool, device=path.device)
         tokens = torch.empty_like(path)
         force = torch.empty_like(path)
@@ -128,7 +128,7 @@ def dag_glat_glance(path, tgt_tokens, pred_tokens, prev_output_tokens, target_le
     path, tgt_tokens, pred_tokens = path.contiguous(), tgt_tokens.contiguous(), pred_tokens.contiguous()
     prev, target_length, rand = prev_output_tokens.contiguous(), target_length.contiguous(), rand.contiguous()
     mask = None if glat_prev_mask is None else glat_prev_mask.contiguous()
-    with torch.cuda.device(path.device):
+    with nat.on_device(path.device):
         oracle, tokens, force = torch.empty((3,) + shape, dtype=torch.int64, device=path.device).unbind(0)
         same_num = torch.empty(bsz, dtype=torch.int64, device=path.device)
         keep_prob = torch.empty(shape, dtype=torch.float32, device=path.device)

@@ -49,7 +49,7 @@ class DagMultiheadLinksFunc(Function):
         gates = log_gates.detach().to(torch.float32).contiguous()
         vend = valid_end.contiguous()
         need_grad = ctx.needs_input_grad[0] or ctx.needs_input_grad[1]
-        with torch.cuda.device(content.device):
+        with nat.on_device(content.device):
             links = torch.empty(bsz, prelen, translen, dtype=content.dtype, device=content.device)
             lse = torch.empty(bsz, prelen, heads, dtype=torch.float32, device=content.device) if need_grad else None
             nat.check(nat.lib().dagx_links_fwd(
@@ -69,7 +69,7 @@ class DagMultiheadLinksFunc(Function):
         bsz, prelen, _, heads = content.shape
         translen = links.shape[2]
         grad_links = grad_links.to(content.dtype).contiguous()
-        with torch.cuda.device(content.device):
+        with nat.on_device(content.device):
             grad_gates = torch.empty(bsz, prelen, heads, dtype=torch.float32, device=content.device)
             # the scores' storage becomes their gradient (they are not needed by anything else:
             # the batched product that made them differentiates through its factors)
