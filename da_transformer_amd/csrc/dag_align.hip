@@ -17,6 +17,8 @@
 // bit-identical to the torch-native rule.
 #include "dag_tiles.h"
 
+#include <atomic>
+
 namespace dagx {
 
 struct AlignArgs {
@@ -688,6 +690,25 @@ __global__ void dag_align_fill_kernel(int *p, int n, int nflags, int flag) {
     if (i < n) p[i] = i >= n - nflags ? flag : 0;
 }
 
+// Dynamic LDS beyond the default limit: raised once per device and instantiation (bit d of `done`: device d), to the most
+// any launch asks for.
+static int raise_lds_limit(const void *kern, size_t bytes, std::atomic<unsigned long long> &done, const char *who) {
+    int device = 0;
+    (void)hipGetDevice(&device);
+    const unsigned long long bit = 1ull << (device & 63);
+    if (done.load(std::memory_order_acquire) & bit) return DAGX_OK;
+    const hipError_t e = hipFuncSetAttribute(kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
+    if (e != hipSuccess) { set_error("%s: cannot reserve %zu bytes of LDS: %s", who, bytes, hipGetErrorString(e)); return DAGX_ERR_LAUNCH; }
+    done.fetch_or(bit, std::memory_order_release);
+    return DAGX_OK;
+}
+constexpr size_t kBacktrackMostLds = kAlignLdsBudget > kWalkLds ? kAlignLdsBudget : kWalkLds;   // (the redo alone asks for at most the former)
+template <typename TM, typename TL, bool TRACE_LDS>
+static int prepare_backtrack() {
+    static std::atomic<unsigned long long> done{0};
+    return raise_lds_limit(reinterpret_cast<const void *>(dag_backtrack_kernel<TM, TL, TRACE_LDS>), kBacktrackMostLds, done, "dag_best_alignment");
+}
+
 template <typename TM, typename TL>
 static int launch_align(AlignArgs a, void *workspace, hipStream_t st) {
     constexpr int NT = 1024;
@@ -727,10 +748,7 @@ static int launch_align(AlignArgs a, void *workspace, hipStream_t st) {
         const size_t redo_lds = (size_t)a.L * 8 + (in_lds ? (size_t)a.T * a.L * 2 : (size_t)0);
         const size_t lds = redo_lds > kWalkLds ? redo_lds : kWalkLds;
         auto kern = in_lds ? dag_backtrack_kernel<TM, TL, true> : dag_backtrack_kernel<TM, TL, false>;
-        if (lds > 48 * 1024) {
-            hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-            if (e != hipSuccess) { set_error("dag_best_alignment: cannot reserve %zu bytes of LDS: %s", lds, hipGetErrorString(e)); return DAGX_ERR_LAUNCH; }
-        }
+        if ((rc = in_lds ? prepare_backtrack<TM, TL, true>() : prepare_backtrack<TM, TL, false>())) return rc;
         hipLaunchKernelGGL(kern, dim3(a.B), dim3(kOneGroupThreads), lds, st, ta.table, ta.srcblk, ta.flags, a);
         return check_launch("dag_backtrack");
     }
@@ -981,6 +999,31 @@ __global__ __launch_bounds__(kDecodeThreads) void viterbi_select_kernel(DecodeAr
     for (int k = count + lane; k < n_max; k += kWave) out_tokens[k] = a.pad;
 }
 
+template <typename TL>
+static int prepare_select() {
+    static std::atomic<unsigned long long> done{0};
+    return raise_lds_limit(reinterpret_cast<const void *>(viterbi_select_kernel<TL>), kWalkLds, done, "dag_viterbi_decode");
+}
+
+// What dagx_prepare_device does for the kernels of this file.
+template <typename TM, typename TL>
+static int prepare_backtracks() {
+    const int rc = prepare_backtrack<TM, TL, true>();
+    return rc ? rc : prepare_backtrack<TM, TL, false>();
+}
+template <typename TL>
+static int prepare_walks() {
+    int rc = prepare_backtracks<float, TL>();
+    if (!rc) rc = prepare_backtracks<__half, TL>();
+    if (!rc) rc = prepare_backtracks<bf16_t, TL>();
+    return rc ? rc : prepare_select<TL>();
+}
+int prepare_align_kernels() {
+    int rc = prepare_walks<float>();
+    if (!rc) rc = prepare_walks<__half>();
+    return rc ? rc : prepare_walks<bf16_t>();
+}
+
 // workspace: [table B*T*L f32 | sync 16 + B*C | flags B | pad to 16 bytes | srcblk B*T*pitch bytes | match rows B*3*L f32]
 static size_t decode_words(int B, int T, int L, int translen, int C) {
     return (size_t)B * T * L + 16 + (size_t)B * (C > 0 ? C : 1) + (size_t)B + 4 + (size_t)B * T * srcblk_pitch(L) / 4 + (size_t)B * 3 * L;
@@ -1032,8 +1075,7 @@ static int launch_decode(const void *links, const float *node_logp, const int64_
     DecodeArgs d{table, srcblk, links, out_len, node_tokens, penalty, T, L, translen, max_length, pad,
                  out_tokens, out_count, pred_length, nodes};
     auto select = viterbi_select_kernel<TL>;
-    const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(select), hipFuncAttributeMaxDynamicSharedMemorySize, (int)kWalkLds);
-    if (e != hipSuccess) { set_error("dag_viterbi_decode: cannot reserve %zu bytes of LDS: %s", kWalkLds, hipGetErrorString(e)); return DAGX_ERR_LAUNCH; }
+    if ((rc = prepare_select<TL>())) return rc;
     hipLaunchKernelGGL(select, dim3(B), dim3(kDecodeThreads), kWalkLds, st, d);
     return check_launch("viterbi_select");
 }

@@ -1956,6 +1956,7 @@ extern "C" int dagx_prepare_device(void) {
     int rc = prepare_tiles_kernels_of<float>();
     if (!rc) rc = prepare_tiles_kernels_of<__half>();
     if (!rc) rc = prepare_tiles_kernels_of<bf16_t>();
+    if (!rc) rc = prepare_align_kernels();
     void *ptr = nullptr;
     if (!rc) rc = scratch_of_current_device(&ptr);
     return rc;

@@ -166,7 +166,8 @@ int dagx_loss_fwd(const void *match, int match_dtype, const int64_t match_stride
 int dagx_loss_fwd_init_workspace(void *workspace, size_t workspace_bytes, void *stream);
 
 /* What dagx_loss_fwd and dagx_loss_fwd_noalloc otherwise do on their first call on a device, for the current
- * device: the LDS limit of the tile kernels (hipFuncSetAttribute) and the address of the built-in scratch array
+ * device (and dagx_best_alignment and dagx_viterbi_decode on theirs): the LDS limit of the kernels
+ * (hipFuncSetAttribute) and the address of the built-in scratch array
  * (hipGetSymbolAddress).  Neither may be part of a stream capture: a caller that captures these entry points into a
  * HIP graph calls this once per device beforehand (or makes one ordinary call first).  No reference counterpart. */
 int dagx_prepare_device(void);
