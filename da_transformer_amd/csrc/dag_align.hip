@@ -575,17 +575,21 @@ __device__ __forceinline__ void stage_walk(WalkStage &w, const float *A, const u
     for (int u = 0; u < kS; ++u) { const int x = q + u * kHelpers; if (x < kWalkRows * kBlk / 4) w.src[x] = vs[u]; }
 }
 
-// From cell (s, j) down to row `stop` by the whole workgroup: visit(row, node) for the predecessor found in every row,
-// called by all lanes of wave 0; it returns the node to go on from, or -1 to end the walk (node: -1 where no candidate
-// has a finite score).  lds: kWalkLds bytes.  s, j are uniform over the workgroup.
-template <typename TL, int NT, typename VISIT>
+// From cell (s, j) down to row `stop` by the whole workgroup: put(row, node), called by single lanes of wave 0, takes the
+// predecessors found.  Where no candidate has a finite score the walk ends, or with ZERO_FOR_DEAD goes on from node 0.
+// lds: kWalkLds bytes.  s, j are uniform over the workgroup.
+// A step is a chain of dependent instructions of one wave, so its length is what counts: the byte that names the block and
+// the scores and transitions of both blocks are read in one LDS round trip, and the nodes found are kept in a register, one
+// a lane, and put 64 rows at a time.
+template <typename TL, int NT, bool ZERO_FOR_DEAD, typename PUT>
 __device__ __forceinline__ void walk_back(const float *A, const unsigned char *srcblk, int spitch, const TL *links, int L,
-                                          int translen, int s, int j, int stop, WalkStage *lds, VISIT visit) {
+                                          int translen, int s, int j, int stop, WalkStage *lds, PUT put) {
     __shared__ int at[2][2];
     if (s <= stop) return;
     const bool walker = threadIdx.x < kWave;
     const int lane = threadIdx.x & (kWave - 1);
     int cur = 0, J = j / kBlk, hi = s;
+    int mine = -1;   // the node found for the row whose number ends in `lane`
     if (!walker) stage_walk<TL, NT>(lds[0], A, srcblk, spitch, links, L, translen, J, hi);
     __syncthreads();
     for (int round = 0;; ++round) {
@@ -594,17 +598,16 @@ __device__ __forceinline__ void walk_back(const float *A, const unsigned char *s
             if (J > 0 && next_hi > stop) stage_walk<TL, NT>(lds[cur ^ 1], A, srcblk, spitch, links, L, translen, J - 1, next_hi);
         } else {
             const WalkStage &w = lds[cur];
-            const unsigned char *src = reinterpret_cast<const unsigned char *>(w.src);
-            while (s > stop && j >= 0 && j / kBlk == J && hi - s < kWalkRows) {
-                const int r = hi - s, c = j & (kBlk - 1);
-                // both predecessor blocks are read along with the byte that says which of them it is
-                const float e0 = w.e[lane * kWalkPitch + c], e1 = w.e[(kBlk + lane) * kWalkPitch + c];
-                const float a0 = w.a[r * 2 * kBlk + lane], a1 = w.a[r * 2 * kBlk + kBlk + lane];
-                const int I = __builtin_amdgcn_readfirstlane((int)src[r * kBlk + c]);
-                float x;
-                if (I == J) x = a1 + e1;
-                else if (I == J - 1) x = a0 + e0;
-                else {
+            const unsigned char *src = reinterpret_cast<const unsigned char *>(w.src) + (hi - s) * kBlk;
+            const float *arow = w.a + (hi - s) * 2 * kBlk + lane, *ecol = w.e + lane * kWalkPitch;
+            for (int left = min(s - stop, kWalkRows - (hi - s)); left > 0 && j >> 6 == J; --left) {   // (-1: no block)
+                const int c = j & (kBlk - 1);
+                int byte = src[c];
+                float e0 = ecol[c], e1 = ecol[kBlk * kWalkPitch + c], a0 = arow[0], a1 = arow[kBlk];
+                asm volatile("" : "+v"(byte), "+v"(e0), "+v"(e1), "+v"(a0), "+v"(a1));   // (else read one after the other)
+                const int I = __builtin_amdgcn_readfirstlane(byte);
+                float x = I == J ? a1 + e1 : a0 + e0;
+                if (__builtin_expect((unsigned)(J - I) > 1u, 0)) {
                     const int i = I * kBlk + lane, d = j - i - 1;
                     const bool valid = d >= 0 && d < translen && i < L;
                     const float e = to_float(links[valid ? (int64_t)i * translen + d : 0]);
@@ -613,16 +616,26 @@ __device__ __forceinline__ void walk_back(const float *A, const unsigned char *s
                 }
                 const float top = wave64_max(x);
                 // lowest lane among those that hold the maximum
-                const int to = top > DAGX_NEG_INF ? I * kBlk + (int)__builtin_ctzll(__builtin_amdgcn_ballot_w64(x == top)) : -1;
+                j = I * kBlk + (int)__builtin_ctzll(__builtin_amdgcn_ballot_w64(x == top));
+                if (__builtin_expect(!(top > DAGX_NEG_INF), 0)) j = ZERO_FOR_DEAD ? 0 : -1;
                 --s;
-                j = __builtin_amdgcn_readfirstlane(visit(s, to));
+                src += kBlk; arow += 2 * kBlk;
+                const int slot = s & (kWave - 1);
+                mine = lane == slot ? j : mine;
+                if (slot == 0) {
+                    if (mine >= 0) put(s + lane, mine);
+                    mine = -1;
+                }
             }
             if (lane == 0) { at[round & 1][0] = s; at[round & 1][1] = j; }
         }
         __syncthreads();
         s = __builtin_amdgcn_readfirstlane(at[round & 1][0]);
         j = __builtin_amdgcn_readfirstlane(at[round & 1][1]);
-        if (s <= stop || j < 0) return;
+        if (s <= stop || j < 0) {
+            if (walker && mine >= 0) put((s & ~(kWave - 1)) + lane, mine);
+            return;
+        }
         cur ^= 1;
         if (j / kBlk == J - 1 && next_hi > stop && next_hi >= s && next_hi - s < kWalkRows) {
             J -= 1; hi = next_hi;
@@ -646,12 +659,10 @@ __global__ __launch_bounds__(kOneGroupThreads) void dag_backtrack_kernel(
         align_one_sample<TM, TL, kOneGroupThreads, TRACE_LDS>(a, b, lds_a);
         return;
     }
-    const int lane = threadIdx.x & (kWave - 1);
-    const bool walker = threadIdx.x < kWave;
     const int T = a.T, L = a.L, translen = a.translen;
     int64_t *path = a.path + (int64_t)b * L;
-    if (walker)
-        for (int j = lane; j < L; j += kWave) path[j] = -1;
+    if (threadIdx.x < kWave)
+        for (int j = threadIdx.x; j < L; j += kWave) path[j] = -1;
     const int Lb = (int)a.out_len[b], Tb = (int)a.tgt_len[b];
     if (!(Tb >= 1 && Lb >= 1 && Tb <= T && Lb <= L && Tb <= Lb)) return;
     const float *A = table + (int64_t)b * T * L;
@@ -659,11 +670,9 @@ __global__ __launch_bounds__(kOneGroupThreads) void dag_backtrack_kernel(
     if (!(A[(int64_t)(Tb - 1) * L + Lb - 1] > DAGX_NEG_INF)) return;   // no finite path
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");     // the -1 fill precedes the path entries (same wave)
     if (threadIdx.x == 0) path[Lb - 1] = Tb - 1;
-    walk_back<TL, kOneGroupThreads>(A, srcblk_all + (int64_t)b * T * spitch, spitch, static_cast<const TL *>(a.links) + (int64_t)b * L * translen,
-                                    L, translen, Tb - 1, Lb - 1, 0, reinterpret_cast<WalkStage *>(lds_a), [&](int t, int j) {
-        if (lane == 0 && j >= 0) path[j] = t;
-        return j;   // (-1, the end of the walk, cannot happen on a finite path)
-    });
+    walk_back<TL, kOneGroupThreads, false>(A, srcblk_all + (int64_t)b * T * spitch, spitch, static_cast<const TL *>(a.links) + (int64_t)b * L * translen,
+                                           L, translen, Tb - 1, Lb - 1, 0, reinterpret_cast<WalkStage *>(lds_a),
+                                           [&](int t, int j) { path[j] = t; });   // (the walk does not end early on a finite path)
 }
 
 constexpr size_t kAlignLdsBudget = 144 * 1024;
@@ -743,7 +752,7 @@ static int launch_align(AlignArgs a, void *workspace, hipStream_t st) {
         if ((rc = check_launch("dag_align_tiles"))) return rc;
         // the backtrack, and the samples that the pipeline gave up on.  (float32, kernel time: with every step read from
         // memory by one wave 38.7 us at B=64 L=512 T=64 and 174 us at B=16 L=1024 T=256, with the steps staged in LDS
-        // 26.0 and 76.5 us.)
+        // 24.1 and 65.0 us.)
         const bool in_lds = trace_fits_lds(a.T, a.L);
         const size_t redo_lds = (size_t)a.L * 8 + (in_lds ? (size_t)a.T * a.L * 2 : (size_t)0);
         const size_t lds = redo_lds > kWalkLds ? redo_lds : kWalkLds;
@@ -923,8 +932,8 @@ __global__ __launch_bounds__(kDecodeThreads) void viterbi_select_kernel(DecodeAr
         to_end[c] = ok ? to_float(links[(int64_t)j * translen + d]) : DAGX_NEG_INF;
     }
     // best node of every step (first index among equals, over all L nodes as the tensor formulation);
-    // a wave takes kRows steps at a time so that their rows are in flight together
-    constexpr int kRows = 4, kWaves = kDecodeThreads / kWave;
+    // a wave takes kRows steps at a time, kCols blocks of 64 nodes of each, so that it waits for sixteen loads at once
+    constexpr int kRows = 4, kCols = 4, kWaves = kDecodeThreads / kWave;
     const int nblk = (L + kWave - 1) / kWave;
     for (int t0 = wave * kRows; t0 < n_max; t0 += kWaves * kRows) {
         float best[kRows];
@@ -932,21 +941,24 @@ __global__ __launch_bounds__(kDecodeThreads) void viterbi_select_kernel(DecodeAr
 #pragma unroll
         for (int r = 0; r < kRows; ++r) { best[r] = DAGX_NEG_INF; arg[r] = lane; }
 #pragma unroll
-        for (int c = 0; c < kMaxBlocksFast; ++c) {
-            if (c < nblk) {
-                const int j = c * kWave + lane;
-                float x[kRows];
+        for (int c0 = 0; c0 < kMaxBlocksFast; c0 += kCols) {
+            if (c0 >= nblk) break;
+            float x[kCols][kRows];   // all requested before any is looked at
+#pragma unroll
+            for (int c = 0; c < kCols; ++c)
 #pragma unroll
                 for (int r = 0; r < kRows; ++r) {
-                    const int t = t0 + r < n_max ? t0 + r : n_max - 1;
-                    x[r] = (sane && j < Lb) ? A[(int64_t)(t + 1) * L + j] : DAGX_NEG_INF;   // (j < Lb <= L)
+                    const int t = t0 + r < n_max ? t0 + r : n_max - 1, j = (c0 + c) * kWave + lane;
+                    x[c][r] = A[(int64_t)(t + 1) * L + (j < L ? j : L - 1)];
                 }
 #pragma unroll
+            for (int c = 0; c < kCols; ++c)
+#pragma unroll
                 for (int r = 0; r < kRows; ++r) {
-                    const float v = x[r] + to_end[c];
+                    const int j = (c0 + c) * kWave + lane;
+                    const float v = sane && j < Lb ? x[c][r] + to_end[c0 + c] : DAGX_NEG_INF;   // (j < Lb <= L; cells behind are not written)
                     if (v > best[r]) { best[r] = v; arg[r] = j; }
                 }
-            }
         }
 #pragma unroll
         for (int r = 0; r < kRows; ++r) {
@@ -971,12 +983,9 @@ __global__ __launch_bounds__(kDecodeThreads) void viterbi_select_kernel(DecodeAr
     __syncthreads();
     const int n = __builtin_amdgcn_readfirstlane(s_star) + 1;
     // table row s = t + 1 holds reach_t
-    walk_back<TL, kDecodeThreads>(A, srcblk, spitch, links, L, translen, n, __builtin_amdgcn_readfirstlane(sidx[n - 1]), 1,
-                                  reinterpret_cast<WalkStage *>(lds_walk), [&](int s, int to) {
-        const int j = to >= 0 ? to : 0;       // (a path of finite score never meets the other case)
-        if (lane == 0) walk[s - 1] = j;
-        return j;
-    });
+    // (a path of finite score never meets a cell without a finite candidate)
+    walk_back<TL, kDecodeThreads, true>(A, srcblk, spitch, links, L, translen, n, __builtin_amdgcn_readfirstlane(sidx[n - 1]), 1,
+                                        reinterpret_cast<WalkStage *>(lds_walk), [&](int s, int j) { walk[s - 1] = j; });
     if (wave != 0) return;
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
     __builtin_amdgcn_wave_barrier();
