@@ -73,17 +73,9 @@ def _check_dag_inputs(match_all, links, output_length, target_length, who):
         nat.dtype_code(match_all), nat.dtype_code(links)
 
 
-def _sweep_tables(bsz, tarlen, prelen):
-    """How the forward's tables share one allocation: its size in bytes, and the byte offsets of the residuals of
-    both sweeps and of their block offsets; the read-outs logz [2, bsz] lie at its start.  float64 first, every table on a
-    multiple of 256 bytes."""
-    def room(nbytes):
-        return (nbytes + 255) & ~255
-    offs = room(16 * bsz)
-    each_off = room(8 * bsz * tarlen * ((prelen + 63) // 64))
-    hats = offs + 2 * each_off
-    each_hat = room(4 * bsz * tarlen * prelen)
-    return hats + 2 * each_hat, (hats, hats + each_hat, offs, offs + each_off)
+def _sweep_offsets(bsz, tarlen, prelen):
+    """Elements of one sweep's residuals and of one sweep's block offsets."""
+    return bsz * tarlen * prelen, bsz * tarlen * ((prelen + 63) // 64)
 
 
 class DagLossFunc(Function):
@@ -108,10 +100,12 @@ class DagLossFunc(Function):
         translen = links.shape[2]
         dev = match_all.device
         with nat.on_device(dev):
-            # sweep results: fp64 block offsets and read-outs, fp32 residuals (see include/dagx.h), in one allocation
-            tables, at = _sweep_tables(bsz, tarlen, prelen)
-            state = torch.empty(tables, dtype=torch.uint8, device=dev)
-            base = state.data_ptr()
+            # sweep results: fp32 residuals of both sweeps; fp64 block offsets of both and, behind them, the read-outs
+            # logz [2, bsz] (see include/dagx.h)
+            nhat, noff = _sweep_offsets(bsz, tarlen, prelen)
+            hats = torch.empty(2 * nhat, dtype=torch.float32, device=dev)
+            offs = torch.empty(2 * (noff + bsz), dtype=torch.float64, device=dev)
+            hat, off = hats.data_ptr(), offs.data_ptr()
             # a tensor of its own, not a view of anything made here: the criterion overwrites entries of
             # the returned loss in place (fs_plugins/criterions/nat_dag_loss.py:190-191)
             loss = torch.empty(bsz, dtype=torch.float32, device=dev)
@@ -122,25 +116,26 @@ class DagLossFunc(Function):
                 nat.check(nat.lib().dagx_loss_fwd(
                     nat.ptr(match_all), nat.dtype_code(match_all), nat.strides3(match_all),
                     nat.ptr(links), nat.dtype_code(links), nat.ptr(output_length), nat.ptr(target_length),
-                    bsz, tarlen, prelen, translen, base + at[0], base + at[1], base + at[2], base + at[3],
-                    base, nat.ptr(loss), nat.ptr(flags), int(need_grad), nat.ptr(ws), nbytes, nat.stream_of(match_all)))
+                    bsz, tarlen, prelen, translen, hat, hat + 4 * nhat, off, off + 8 * noff,
+                    off + 16 * noff, nat.ptr(loss), nat.ptr(flags), int(need_grad), nat.ptr(ws), nbytes, nat.stream_of(match_all)))
             except RuntimeError:
                 _forget_workspace(dev)
                 raise
         DagLossFunc.last_sample_flags = flags
-        ctx.save_for_backward(state, flags, match_all, links, output_length, target_length)
+        ctx.save_for_backward(hats, offs, flags, match_all, links, output_length, target_length)
         # with gradients this is the beta read-out (the partition function the backward uses), else alpha's
         return loss
 
     @staticmethod
     def backward(ctx, grad_output):
-        state, flags, match_all, links, output_length, target_length = ctx.saved_tensors
+        hats, offs, flags, match_all, links, output_length, target_length = ctx.saved_tensors
         want_match, want_links = ctx.needs_input_grad[0], ctx.needs_input_grad[1]
         if not (want_match or want_links):
             return None, None, None, None
         bsz, tarlen, prelen = match_all.shape
         translen = links.shape[2]
-        base, at = state.data_ptr(), _sweep_tables(bsz, tarlen, prelen)[1]
+        nhat, noff = _sweep_offsets(bsz, tarlen, prelen)
+        hat, off = hats.data_ptr(), offs.data_ptr()
         if grad_output.dtype != torch.float32:
             grad_output = grad_output.to(torch.float32)
         with nat.on_device(match_all.device):
@@ -148,8 +143,8 @@ class DagLossFunc(Function):
                 if want_match else None
             grad_links = torch.empty_like(links) if want_links else None
             nat.check(nat.lib().dagx_loss_bwd(
-                nat.ptr(grad_output), grad_output.stride(0), base + at[0], base + at[1],
-                base + at[2], base + at[3], base, nat.ptr(flags),
+                nat.ptr(grad_output), grad_output.stride(0), hat, hat + 4 * nhat,
+                off, off + 8 * noff, off + 16 * noff, nat.ptr(flags),
                 nat.ptr(match_all), nat.dtype_code(match_all), nat.strides3(match_all),
                 nat.ptr(links), nat.dtype_code(links), nat.ptr(output_length), nat.ptr(target_length),
                 bsz, tarlen, prelen, translen, nat.ptr(grad_match), nat.ptr(grad_links),
