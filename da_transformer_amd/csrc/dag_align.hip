@@ -7,7 +7,7 @@
 //  * dag_align_tiles_kernel + dag_backtrack_kernel (L <= 1024): the sweep keeps E as 64x64 register
 //    tiles and evaluates a step with one DPP-broadcast add and one max per (i, j) pair, spread over
 //    the same pipeline of workgroups as the loss sweeps; it stores only the score table.  The
-//    backtrack (one wave per sample) then re-derives, for the T_b cells on the path only, the
+//    backtrack (a wave per sample walks, others stage for it) then re-derives, for the T_b cells on the path only, the
 //    lowest predecessor index attaining the stored maximum.
 //  * dag_align_kernel: one workgroup per sample, thread <-> node j scanning its predecessors in
 //    ascending order with a strict '>' (back-pointers in LDS when T*L fits, else in the caller's
