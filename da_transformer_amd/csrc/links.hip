@@ -107,9 +107,19 @@ __device__ __forceinline__ LinkRow link_row(const int64_t *valid_end, int64_t ro
 }
 
 constexpr int kLinkPer = 4;                       // window positions per lane
-// Sums of products of probabilities are taken as they are down to 2^-100, where terms that left the float32 range (below
-// 2^-126) still do not count; below, and where something overflowed, a position takes the route through its largest term.
-constexpr float kLinkTiny = 7.8886091e-31f, kLinkHuge = 1.2676506e+30f;
+// Sums of products of probabilities are taken as they are down to 2^-100 times the largest factor that a gate puts before a
+// probability (1 at least): a probability that left the float32 range (below 2^-126) still does not count there, whatever
+// its gate.  Below that, and above kLinkHuge, which gates of at most 0 never reach, a position takes the route through its
+// largest term.
+constexpr float kLinkTiny = 7.8886091e-31f, kLinkHuge = 64.0f;
+template <int H>
+__device__ __forceinline__ float least_sum(float own, const float (&factor)[H]) {   // own: the factor of the lane's head
+    float most = 1.0f;
+    if (__builtin_expect(__builtin_amdgcn_ballot_w64(own > 1.0f) != 0, 0))
+#pragma unroll
+        for (int c = 0; c < H; ++c) most = fmaxf(most, factor[c]);
+    return kLinkTiny * most;
+}
 
 // links and lse (the per-head log normalisers, [B][L][H], kept for the backward).  WPR waves share a row: wave `sub` has
 // the chunks sub, sub + WPR, ... of 64 window positions; min(translen, L - 1) <= 64 * kLinkPer * WPR.
@@ -186,8 +196,9 @@ __global__ __launch_bounds__(kLinkThreads) void links_fwd_kernel(
     if (lse_out && sub == 0 && lane < 16) lse_out[row * H + head] = lse2 * kLn2;
     // mix the heads: log2 sum_c e_c * f_c with f = 2^(max - lse + gate), lane-local
     float f[H];
-    lanes_spread<H>(alive && m_own > DAGX_NEG_INF ? fast_exp2(__builtin_fmaf(m_own - top, kLog2e, gate2 - log_tot)) : 0.f, f);
-    const float bias_own = alive ? gate2 - lse2 : DAGX_NEG_INF;
+    const float f_own = alive && m_own > DAGX_NEG_INF ? fast_exp2(__builtin_fmaf(m_own - top, kLog2e, gate2 - log_tot)) : 0.f;
+    lanes_spread<H>(f_own, f);
+    const float bias_own = alive ? gate2 - lse2 : DAGX_NEG_INF, least = least_sum<H>(f_own, f);
 #pragma unroll
     for (int k = 0; k < kLinkPer; ++k) {
         const int d0 = (k * WPR + sub) * kWave, d = lane + d0;
@@ -197,7 +208,7 @@ __global__ __launch_bounds__(kLinkThreads) void links_fwd_kernel(
             float acc = 0.f;
 #pragma unroll
             for (int c = 0; c < H; ++c) acc = __builtin_fmaf(x[k][c], f[c], acc);
-            const bool slow = d < r.n && !(acc >= kLinkTiny && acc <= kLinkHuge);
+            const bool slow = d < r.n && !(acc >= least && acc <= kLinkHuge);
             if (d < r.n) v = fast_log2(acc) * kLn2;
             if (__builtin_expect(__builtin_amdgcn_ballot_w64(slow) != 0, 0)) {   // from the scores again, against the largest term
                 float bias[H];
@@ -268,7 +279,9 @@ __global__ __launch_bounds__(kLinkThreads) void links_bwd_kernel(
     const bool every_head = __builtin_amdgcn_ballot_w64(alive) == ~0ull;
     float nlse[H], G[H], wsum[H];
     lanes_spread<H>(-lse_own * kLog2e, nlse);
-    lanes_spread<H>(fast_exp2(gate_own * kLog2e), G);
+    const float G_own = fast_exp2(gate_own * kLog2e);
+    lanes_spread<H>(G_own, G);
+    const float least = least_sum<H>(G_own, G);
     // The route of the positions whose sum leaves the range, and of rows with a head that reaches no position (or holds a
     // NaN: it takes no part): from the scores, against the largest term.  w: the position's d/dg_c, pr: exp(x - lse).
     auto general = [&](int d, float grad, float (&w)[H], float (&pr)[H]) __attribute__((always_inline)) {
@@ -307,7 +320,7 @@ __global__ __launch_bounds__(kLinkThreads) void links_bwd_kernel(
                 x[k][c] = fast_exp2(__builtin_fmaf(x[k][c], kLog2e, nlse[c]));
                 acc = __builtin_fmaf(x[k][c], G[c], acc);
             }
-            const bool fine = every_head && acc >= kLinkTiny && acc <= kLinkHuge;
+            const bool fine = every_head && acc >= least && acc <= kLinkHuge;
             const float grad = go[k];
             go[k] = in && fine ? grad / acc : 0.f;
             if (in && fine) {

@@ -182,3 +182,37 @@ def test_scores_reused_after_backward_fail_loudly():
     total = links.masked_fill(links == NEG_INF, 0.0).sum() + other_use
     with pytest.raises(RuntimeError, match="modified by an inplace operation"):
         total.backward()
+
+
+def _run_backward(content, gates, vend, translen, weight):
+    """links, and the gradients of (links * weight).sum() over the allowed transitions, all on the CPU."""
+    c = content.to(DEV).requires_grad_(); g = gates.to(DEV).requires_grad_()
+    got = dagx.dag_multihead_links(c * 1, g, vend.to(DEV), translen)
+    got.backward(weight.to(DEV))
+    return got.detach().cpu(), c.grad.cpu(), g.grad.cpu()
+
+
+@pytest.mark.parametrize("gate", [3.0, 25.0, 80.0])
+@pytest.mark.parametrize("B,L,H", [(2, 120, 4), (1, 300, 8), (1, 700, 16)])
+def test_gates_above_zero(B, L, H, gate):
+    """Gates need not be log-probabilities.  In every third row a probability that is below the smallest float32 number
+    (gate 25, 80) carries its position once its gate has been added, while the other heads keep the position's sum above
+    2^-100: head 0 stands at -63.5 there, the others at -68 each.  The other rows: random scores, one gate above 0.
+    Scores of 150 times log2(e), added to a normaliser of that size, are rounded to 2^-17 each: a few 1e-5 in a link."""
+    content, gates, lens = _case(B, L, H, torch.float32, seed=L, scale=25.0, ragged=False)
+    gates[:, 1::3, H - 1] = gate
+    content[:, ::3] = -68.0
+    content[:, ::3, :, 0] = -63.5 - gate
+    for i in range(0, L - 1, 3):
+        content[:, i, i + 1] = 0.0
+    gates[:, ::3] = 0.0
+    gates[:, ::3, 0] = gate
+    vend = lens[:, None].expand(-1, L).contiguous()
+    c64 = content.double().requires_grad_(); g64 = gates.double().requires_grad_()
+    want = tn.multihead_links(c64, g64, _mask(lens, L), L - 1)
+    weight = torch.randn(want.shape, generator=torch.Generator().manual_seed(5))
+    (want.masked_fill(want == NEG_INF, 0.0) * weight.double()).sum().backward()
+    got, dc, dg = _run_backward(content, gates, vend, L - 1, weight)
+    _compare(got.double(), want.detach(), 1e-5, 5e-5)
+    for mine, ref in ((dc, c64.grad), (dg, g64.grad)):
+        assert torch.allclose(mine.double(), ref, rtol=2e-4, atol=2e-4 * ref.abs().max().item())
