@@ -220,10 +220,11 @@ __global__ __launch_bounds__(kLinkThreads) void links_fwd_kernel(
                     for (int c = 0; c < H; ++c) { y[c] = __builtin_fmaf(y[c], kLog2e, bias[c]); ym = fmaxf(ym, y[c]); }
                     v = DAGX_NEG_INF;
                     if (ym > DAGX_NEG_INF) {
+                        const float shift = ym < -DAGX_NEG_INF ? ym : 0.f;   // (a gate of +inf: the link is +inf, not inf - inf)
                         float acc2 = 0.f;
 #pragma unroll
-                        for (int c = 0; c < H; ++c) acc2 += fast_exp2(y[c] - ym);
-                        v = (ym + fast_log2(acc2)) * kLn2;
+                        for (int c = 0; c < H; ++c) acc2 += fast_exp2(y[c] - shift);
+                        v = (shift + fast_log2(acc2)) * kLn2;
                     }
                 }
             }
@@ -283,7 +284,8 @@ __global__ __launch_bounds__(kLinkThreads) void links_bwd_kernel(
     lanes_spread<H>(G_own, G);
     const float least = least_sum<H>(G_own, G);
     // The route of the positions whose sum leaves the range, and of rows with a head that reaches no position (or holds a
-    // NaN: it takes no part): from the scores, against the largest term.  w: the position's d/dg_c, pr: exp(x - lse).
+    // NaN, which reaches every gradient of the row): from the scores, against the largest term.  w: the position's d/dg_c,
+    // pr: exp(x - lse).
     auto general = [&](int d, float grad, float (&w)[H], float (&pr)[H]) __attribute__((always_inline)) {
         float lse[H], gate[H], ym = DAGX_NEG_INF, acc = 0.f;
         lanes_spread<H>(lse_own, lse);
@@ -296,10 +298,10 @@ __global__ __launch_bounds__(kLinkThreads) void links_bwd_kernel(
             ym = fmaxf(ym, w[c]);
             pr[c] = (lse[c] > DAGX_NEG_INF && pr[c] > DAGX_NEG_INF) ? fast_exp2((pr[c] - lse[c]) * kLog2e) : 0.f;
         }
-        const bool some = ym > DAGX_NEG_INF;   // else no head reaches this position (or a NaN score: the weights stay 0)
+        const bool some = ym > DAGX_NEG_INF;   // else no head reaches this position: the weights stay 0
 #pragma unroll
         for (int c = 0; c < H; ++c) {
-            w[c] = some && w[c] > DAGX_NEG_INF ? fast_exp2(w[c] - ym) : 0.f;
+            w[c] = some ? fast_exp2(w[c] - ym) : 0.f;   // (0 for a head that does not reach it, NaN for a NaN)
             acc += w[c];
         }
         const float t = some ? grad / acc : 0.f;

@@ -216,3 +216,24 @@ def test_gates_above_zero(B, L, H, gate):
     _compare(got.double(), want.detach(), 1e-5, 5e-5)
     for mine, ref in ((dc, c64.grad), (dg, g64.grad)):
         assert torch.allclose(mine.double(), ref, rtol=2e-4, atol=2e-4 * ref.abs().max().item())
+
+
+@pytest.mark.parametrize("L,H", [(40, 4), (300, 8), (700, 16)])
+def test_not_a_number_and_infinity_are_not_hidden(L, H):
+    """A NaN or an infinity among the scores or gates of a node reaches all gradients of that node and no other's, so that
+    a loss scaler sees it; in the forward a NaN score stays at its position, a NaN gate takes the row and a gate of +inf
+    makes its links +inf."""
+    content, gates, lens = _case(1, L, H, torch.float32, seed=L, ragged=False)
+    vend = lens[:, None].expand(-1, L).contiguous()
+    weight = torch.randn(1, L, L - 1, generator=torch.Generator().manual_seed(5))
+    clean = _run_backward(content, gates, vend, L - 1, weight)
+    content[0, 2, L - 5, 1] = float("nan"); gates[0, 5, 1] = float("nan")
+    content[0, 7, 20, 2] = float("inf"); gates[0, 9, 3] = float("inf")
+    got, dc, dg = _run_backward(content, gates, vend, L - 1, weight)
+    assert torch.equal(torch.isnan(got[0, 2]), torch.arange(L - 1) == L - 5 - 3)
+    assert torch.isnan(got[0, 5, :L - 6]).all() and (got[0, 9, :L - 10] == float("inf")).all()
+    for i in (2, 5, 7, 9):
+        assert torch.isnan(dc[0, i, i + 1:]).all() and (dc[0, i, :i + 1] == 0).all() and torch.isnan(dg[0, i]).all()
+    rest = torch.tensor([i not in (2, 5, 7, 9) for i in range(L)])
+    for mine, ref in zip((got, dc, dg), clean):
+        assert torch.equal(mine[0, rest], ref[0, rest])
