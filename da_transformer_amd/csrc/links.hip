@@ -111,7 +111,8 @@ constexpr int kLinkPer = 4;                       // window positions per lane
 // probability (1 at least): a probability that left the float32 range (below 2^-126) still does not count there, whatever
 // its gate.  Below that, and above kLinkHuge, which gates of at most 0 never reach, a position takes the route through its
 // largest term.
-constexpr float kLinkTiny = 7.8886091e-31f, kLinkHuge = 64.0f;
+// kLinkMostGrad: 2^26; over a sum of at least 2^-100 times the largest factor, and times that factor, it is still finite.
+constexpr float kLinkTiny = 7.8886091e-31f, kLinkHuge = 64.0f, kLinkMostGrad = 67108864.0f;
 template <int H>
 __device__ __forceinline__ float least_sum(float own, const float (&factor)[H]) {   // own: the factor of the lane's head
     float most = 1.0f;
@@ -283,7 +284,7 @@ __global__ __launch_bounds__(kLinkThreads) void links_bwd_kernel(
     const float G_own = fast_exp2(gate_own * kLog2e);
     lanes_spread<H>(G_own, G);
     const float least = least_sum<H>(G_own, G);
-    // The route of the positions whose sum leaves the range, and of rows with a head that reaches no position (or holds a
+    // The route of the positions whose sum or gradient leaves the range, and of rows with a head that reaches no position (or holds a
     // NaN, which reaches every gradient of the row): from the scores, against the largest term.  w: the position's d/dg_c,
     // pr: exp(x - lse).
     auto general = [&](int d, float grad, float (&w)[H], float (&pr)[H]) __attribute__((always_inline)) {
@@ -322,8 +323,8 @@ __global__ __launch_bounds__(kLinkThreads) void links_bwd_kernel(
                 x[k][c] = fast_exp2(__builtin_fmaf(x[k][c], kLog2e, nlse[c]));
                 acc = __builtin_fmaf(x[k][c], G[c], acc);
             }
-            const bool fine = every_head && acc >= least && acc <= kLinkHuge;
             const float grad = go[k];
+            const bool fine = every_head && acc >= least && acc <= kLinkHuge && fabsf(grad) <= kLinkMostGrad;
             go[k] = in && fine ? grad / acc : 0.f;
             if (in && fine) {
 #pragma unroll

@@ -237,3 +237,17 @@ def test_not_a_number_and_infinity_are_not_hidden(L, H):
     rest = torch.tensor([i not in (2, 5, 7, 9) for i in range(L)])
     for mine, ref in zip((got, dc, dg), clean):
         assert torch.equal(mine[0, rest], ref[0, rest])
+
+
+@pytest.mark.parametrize("L,H", [(40, 4), (300, 8), (700, 16)])
+def test_large_gradients_of_unlikely_transitions(L, H):
+    """An incoming gradient of 1e30 at transitions down to e^-69: the gradient over the probability leaves the float32
+    range, its product with a head's probability does not.  (Scores of 100: probabilities to a few 1e-5, as above.)"""
+    content, gates, lens = _case(1, L, H, torch.float32, seed=L, scale=18.0, ragged=False)
+    c64 = content.double().requires_grad_(); g64 = gates.double().requires_grad_()
+    want = tn.multihead_links(c64, g64, _mask(lens, L), L - 1)
+    weight = torch.randn(want.shape, generator=torch.Generator().manual_seed(5)) * 1e30
+    (want.masked_fill(want == NEG_INF, 0.0) * weight.double()).sum().backward()
+    _, dc, dg = _run_backward(content, gates, lens[:, None].expand(-1, L).contiguous(), L - 1, weight)
+    for mine, ref in ((dc, c64.grad), (dg, g64.grad)):
+        assert torch.allclose(mine.double(), ref, rtol=2e-4, atol=2e-4 * ref.abs().max().item())
