@@ -11,11 +11,11 @@
 // HBM-bound once the waves in flight suffice: the forward reads the windows and writes [B,L,translen]; the backward reads
 // the windows again and writes the gradient over the whole [B,L,L,H] tensor in place (zeros outside the windows), as the
 // dense batched-GEMM backward that follows it expects.
-// Measured, forward and backward one after the other, against one wave per row with the whole window in registers (2 waves
-// a SIMD), three exponentials per score in the backward and cached zeros: B=64 L=512 H=8 float32 94 + 167 -> 58 + 168 us
-// (1.2 GB: 5.3 TB/s); B=16 L=1024 H=8 float16 88 + 171 -> 46 + 61 us (4.1 TB/s); B=8 L=512 H=16 float32 29 + 52 -> 16 + 36 us.
-// Non-temporal zeros alone took 164 -> 168, 83 -> 61 and 48 -> 36 us off the backwards and 78 -> 58 us off the first
-// forward, which finds less to write back; the gradient inside the window, stored the same way, was slower again.
+// Measured, forward behind backward in the same storage, lengths between 3/4 L and L, against one wave per row with the
+// whole window in registers (2 waves a SIMD), three exponentials per score in the backward and cached zeros: B=64 L=512
+// H=8 float32 254 -> 218 us, B=32 118 -> 80, float16 B=64 215 -> 118; B=16 L=1024 H=8 float16 229 -> 98; B=8 L=512 H=16
+// float32 76 -> 47.  Between the copy that lays the scores out and the one that takes the gradient, those included: 803 ->
+// 780, 408 -> 381, 586 -> 475, 602 -> 474, 228 -> 203.  Non-temporal stores of the gradient inside the window were slower.
 #include <type_traits>
 
 #include "dagx_common.h"
@@ -244,7 +244,7 @@ template <typename TC, int H, int WPR>
 __global__ __launch_bounds__(kLinkThreads) void links_bwd_kernel(
     TC *__restrict__ content, const float *__restrict__ log_gates, const int64_t *__restrict__ valid_end,
     int64_t rows, int L, int translen, const float *__restrict__ lse_in,
-    const TC *__restrict__ grad_links, float *__restrict__ grad_gates) {
+    const TC *__restrict__ grad_links, float *__restrict__ grad_gates, bool past_caches) {
     __shared__ float part[kLinkWaves][H];
     const int lane = threadIdx.x & (kWave - 1), wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
     const int sub = wave % WPR, head = head_of<H>(lane);
@@ -265,7 +265,7 @@ __global__ __launch_bounds__(kLinkThreads) void links_bwd_kernel(
     }
     const float lse_own = lse_in[row * H + head], gate_own = log_gates[row * H + head];
     const LinkRow r = link_row(valid_end, row, L, translen);
-    // outside the window: zeros (nothing of it is used), in contiguous pieces that pass the caches by
+    // outside the window: zeros (nothing of it is used), in contiguous pieces that pass the caches by if told to
     {
         typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
         typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
@@ -274,8 +274,13 @@ __global__ __launch_bounds__(kLinkThreads) void links_bwd_kernel(
         Piece *p = reinterpret_cast<Piece *>(full);
         const int before = r.jlo * kEach, behind = (r.jlo + r.n) * kEach, end = L * kEach;
         const Piece zero = {};
-        for (int q = lane + sub * kWave; q < before && q < end; q += WPR * kWave) __builtin_nontemporal_store(zero, p + q);
-        for (int q = behind + lane + sub * kWave; q < end; q += WPR * kWave) __builtin_nontemporal_store(zero, p + q);
+        if (past_caches) {
+            for (int q = lane + sub * kWave; q < before && q < end; q += WPR * kWave) __builtin_nontemporal_store(zero, p + q);
+            for (int q = behind + lane + sub * kWave; q < end; q += WPR * kWave) __builtin_nontemporal_store(zero, p + q);
+        } else {
+            for (int q = lane + sub * kWave; q < before && q < end; q += WPR * kWave) p[q] = zero;
+            for (int q = behind + lane + sub * kWave; q < end; q += WPR * kWave) p[q] = zero;
+        }
     }
     const bool alive = lse_own > DAGX_NEG_INF;
     const bool every_head = __builtin_amdgcn_ballot_w64(alive) == ~0ull;
@@ -403,9 +408,17 @@ static int launch_links_bwd(void *content, const float *log_gates, const int64_t
                             const float *lse, const void *grad_links, float *grad_gates, hipStream_t st) {
     const int64_t rows = (int64_t)B * L;
     const int n = translen < L - 1 ? translen : L - 1;
+    // The zeros pass the caches by where the tensor and what else is in use leave them no room in the 256 MB memory-side
+    // cache; where they do, the transposition or batched product that reads the gradient next finds them there.  Forward and
+    // backward between the copy that lays the scores out and the one that takes the gradient, B = 16 ... 64, L=512 H=8
+    // float32 (us, past the caches / through them): transitions of any length 128 MB 190 / 181, 160 MB 237 / 226,
+    // 192 MB 284 / 285, 224 MB 334 / 343, 512 MB 780 / 791; at most 32: 128 MB 167 / 152, 192 MB 247 / 239, 256 MB 327 /
+    // 342, 512 MB 645 / 682.  float16 and bfloat16 cross near 192 MB too.  (Forward behind backward in one storage: equal up to
+    // 160 MB, 25 / 32 in favour of the caches at 128 MB and transitions of at most 32, 75 / 78 against them at 192 MB.)
+    const bool past_caches = rows * L * H * (int64_t)sizeof(TC) > (176 << 20);
 #define DAGX_GO(WPR) hipLaunchKernelGGL((links_bwd_kernel<TC, H, WPR>), dim3((unsigned)((rows * WPR + kLinkWaves - 1) / kLinkWaves)), dim3(kLinkThreads), 0, st, \
                                         static_cast<TC *>(content), log_gates, valid_end, rows, L, translen, lse,                                               \
-                                        static_cast<const TC *>(grad_links), grad_gates)
+                                        static_cast<const TC *>(grad_links), grad_gates, past_caches)
     if (n <= kLinkPer * kWave) DAGX_GO(1); else if (n <= 2 * kLinkPer * kWave) DAGX_GO(2); else DAGX_GO(4);
 #undef DAGX_GO
     return check_launch("links_bwd");
