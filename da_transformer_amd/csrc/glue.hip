@@ -54,11 +54,13 @@ __global__ __launch_bounds__(kGlueThreads) void force_emit_kernel(
 }
 
 // The same for an input whose targets lie next to each other ([B,L,T] storage: the criterion's transposed view of the
-// gather's output).  Bound by memory; row by row such an input is read in pieces of 32 bytes.  Here a workgroup takes a
-// tile of 64 targets x 128 nodes through LDS, so both sides move whole cache lines.  B=16 T=256 L=1024 float32: 51.9 us row by row, 13.4 us
-// here (33.5 MB; an input with its nodes next to each other: 12.7 us); B=32 T=128 L=700 float16 21.2 and 12.1 us; B=64
-// T=64 L=512 float32 11.7 and 11.0 us.
+// gather's output).  Bound by memory, small ones by latency; row by row such an input is read in pieces of 32 bytes.  Here a
+// workgroup takes a tile of 64 targets x 128 nodes through LDS, so both sides move whole cache lines.  float32, us, row by
+// row / here: B=16 T=256 L=1024 24.0 / 8.5 when the input is still in the caches and 27.8 / 13.9 behind 600 MB of other
+// writes (33.5 MB); B=64 T=128 L=512 28.7 / 8.3 and 31.0 / 13.0.  An element at a time out of
+// LDS instead of eight, the store of a tile of 64 targets alone took 3 us more: B=1 T=64 L=512 7.0 -> 4.8.
 constexpr int kCrossT = 64, kCrossL = 128;
+static_assert(kCrossT == kWave && kCrossT % (8 * kGlueThreads / kWave) == 0, "");
 template <typename TM, bool kGrad>
 __global__ __launch_bounds__(kGlueThreads) void force_emit_cross_kernel(
     const TM *__restrict__ in, int64_t s0, int64_t s1, int64_t s2,
@@ -68,7 +70,7 @@ __global__ __launch_bounds__(kGlueThreads) void force_emit_cross_kernel(
     __shared__ TM tile[kCrossL * kPitch];
     __shared__ int forced[kCrossT];
     const int b = blockIdx.z, t0 = blockIdx.x * kCrossT, j0 = blockIdx.y * kCrossL;
-    const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
+    const int lane = threadIdx.x & (kWave - 1), wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
     const int64_t *fe = force_emit + (int64_t)b * L;
     const TM *src = in + b * s0;
     TM v[kCrossL / kWaves];   // all of a thread's elements are on their way while the targets are looked through
@@ -86,18 +88,26 @@ __global__ __launch_bounds__(kGlueThreads) void force_emit_cross_kernel(
 #pragma unroll
     for (int u = 0; u < kCrossL / kWaves; ++u) tile[(wave + u * kWaves) * kPitch + lane] = v[u];
     __syncthreads();
+    const unsigned long long pinned = __builtin_amdgcn_ballot_w64(forced[lane] != 0);
+    constexpr int kTurn = 8;   // elements that a thread reads before it stores them: one LDS wait for all
 #pragma unroll
     for (int c = 0; c < kCrossL / kWave; ++c) {
         const int jl = c * kWave + lane, j = j0 + jl;
         if (j >= L) break;
         const int64_t pin = fe[j];
-        for (int r = wave; r < kCrossT && t0 + r < T; r += kWaves) {
-            const int t = t0 + r;
-            const bool f = forced[r] != 0;
-            const TM x = tile[jl * kPitch + r];
-            TM *dst = out + ((int64_t)b * T + t) * L + j;
-            if (kGrad) *dst = f ? from_float<TM>(0.0f) : x;
-            else *dst = from_float<TM>(f ? (pin == t ? 0.0f : DAGX_NEG_INF) : to_float(x) + 0.0f);
+        for (int r0 = wave; r0 < kCrossT && t0 + r0 < T; r0 += kTurn * kWaves) {
+            TM x[kTurn];
+#pragma unroll
+            for (int u = 0; u < kTurn; ++u) x[u] = tile[jl * kPitch + r0 + u * kWaves];
+#pragma unroll
+            for (int u = 0; u < kTurn; ++u) {
+                const int r = r0 + u * kWaves, t = t0 + r;
+                if (t >= T) break;
+                const bool f = (pinned >> r) & 1;
+                TM *dst = out + ((int64_t)b * T + t) * L + j;
+                if (kGrad) *dst = f ? from_float<TM>(0.0f) : x[u];
+                else *dst = from_float<TM>(f ? (pin == t ? 0.0f : DAGX_NEG_INF) : to_float(x[u]) + 0.0f);
+            }
         }
     }
 }
@@ -171,8 +181,13 @@ __global__ __launch_bounds__(kGlueThreads) void glat_glance_kernel(GlatArgs a) {
 
 template <typename TM>
 static int launch_force_emit(const void *in, const int64_t *s, const int64_t *fe, int B, int T, int L, bool grad, void *out, hipStream_t st) {
-    // across: targets next to each other, and more of them than a row-by-row workgroup reads together
-    if (s[1] == 1 && s[2] != 1 && T > kForceRows) {
+    // Across: targets next to each other, and more of them than a row-by-row workgroup reads together.  Graphs of up to 256
+    // nodes with more than 32 targets stay with the rows until these make 512 workgroups: their few tiles leave most of the
+    // chip idle.  float32, us, rows / tiles: B=16 L=1024 T=16 8.2 / 4.3, T=64 8.4 / 5.6; B=64 L=512 T=64 6.7 / 5.9; B=1
+    // L=512 T=64 5.1 / 4.8; B=16 L=184 T=24 4.1 / 4.1, T=64 4.2 / 4.8, T=128 4.3 / 4.9; B=64 L=184 T=48 4.5 / 4.6, T=64
+    // 5.2 / 5.1, T=128 8.3 / 5.7; B=128 L=256 T=64 13.2 / 5.7.  (Past the rule: B=64 L=1024 T=96 11.4 / 12.9, T=128 11.8 /
+    // 15.0, T=192 84.7 / 21.6.)
+    if (s[1] == 1 && s[2] != 1 && T > kForceRows && (L > 256 || T <= 32 || (int64_t)B * ((T + kForceRows - 1) / kForceRows) >= 512)) {
         const dim3 cross((unsigned)((T + kCrossT - 1) / kCrossT), (unsigned)((L + kCrossL - 1) / kCrossL), (unsigned)B);
         if (grad)
             hipLaunchKernelGGL((force_emit_cross_kernel<TM, true>), cross, dim3(kGlueThreads), 0, st, static_cast<const TM *>(in), s[0], s[1], s[2], fe, T, L, static_cast<TM *>(out));

@@ -38,7 +38,8 @@ def _force_case(seed, B, T, L, dup=False):
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
-@pytest.mark.parametrize("B,T,L", [(3, 7, 20), (4, 16, 64), (2, 9, 300), (1, 1, 1), (2, 65, 129), (3, 128, 128), (2, 63, 1024)])
+@pytest.mark.parametrize("B,T,L", [(3, 7, 20), (4, 16, 64), (2, 9, 300), (1, 1, 1), (2, 65, 129), (3, 128, 128), (2, 63, 1024),
+                                   (2, 65, 257), (3, 128, 384), (2, 33, 300), (3, 32, 65), (64, 64, 70), (57, 66, 200)])
 @pytest.mark.parametrize("transposed", [False, True])
 def test_force_alignment_forward_is_bit_exact(dtype, B, T, L, transposed):
     gen = torch.Generator().manual_seed(B * 100 + T)
