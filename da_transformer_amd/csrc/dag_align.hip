@@ -911,7 +911,7 @@ __global__ __launch_bounds__(kDecodeThreads) void viterbi_select_kernel(DecodeAr
     __shared__ float sbest[kDecodeMaxSteps];
     __shared__ int sidx[kDecodeMaxSteps];
     __shared__ int walk[kDecodeMaxSteps];
-    const int b = blockIdx.x, tid = threadIdx.x, lane = tid & (kWave - 1), wave = tid / kWave;
+    const int b = blockIdx.x, tid = threadIdx.x, lane = tid & (kWave - 1), wave = __builtin_amdgcn_readfirstlane(tid / kWave);
     const int L = a.L, T = a.T, translen = a.translen, n_max = a.max_length;
     const int Lb = (int)a.out_len[b];
     const float *A = a.table + (int64_t)b * T * L;
@@ -935,7 +935,13 @@ __global__ __launch_bounds__(kDecodeThreads) void viterbi_select_kernel(DecodeAr
     // a wave takes kRows steps at a time, kCols blocks of 64 nodes of each, so that it waits for sixteen loads at once
     constexpr int kRows = 4, kCols = 4, kWaves = kDecodeThreads / kWave;
     const int nblk = (L + kWave - 1) / kWave;
+    const unsigned in_last = min(lane, L - 1 - (nblk - 1) * kWave);
     for (int t0 = wave * kRows; t0 < n_max; t0 += kWaves * kRows) {
+        // An address is a scalar part and one of two offsets a lane, formed when it is needed: kept from one turn to the next,
+        // sixteen of them a lane took the kernel to 128 registers and scratch, and so to one workgroup a CU.
+        unsigned off = lane, off_last = in_last;
+        int last = nblk - 1;
+        asm volatile("" : "+v"(off), "+v"(off_last), "+s"(last));
         float best[kRows];
         int arg[kRows];
 #pragma unroll
@@ -948,15 +954,16 @@ __global__ __launch_bounds__(kDecodeThreads) void viterbi_select_kernel(DecodeAr
             for (int c = 0; c < kCols; ++c)
 #pragma unroll
                 for (int r = 0; r < kRows; ++r) {
-                    const int t = t0 + r < n_max ? t0 + r : n_max - 1, j = (c0 + c) * kWave + lane;
-                    x[c][r] = A[(int64_t)(t + 1) * L + (j < L ? j : L - 1)];
+                    const int t = t0 + r < n_max ? t0 + r : n_max - 1, blk = min(c0 + c, last);
+                    const float *from = A + (int64_t)(t + 1) * L + blk * kWave;
+                    x[c][r] = from[blk < last ? off : off_last];
                 }
 #pragma unroll
             for (int c = 0; c < kCols; ++c)
 #pragma unroll
                 for (int r = 0; r < kRows; ++r) {
                     const int j = (c0 + c) * kWave + lane;
-                    const float v = sane && j < Lb ? x[c][r] + to_end[c0 + c] : DAGX_NEG_INF;   // (j < Lb <= L; cells behind are not written)
+                    const float v = x[c][r] + to_end[c0 + c];   // (from node Lb on -inf or, where a cell was not written, NaN: never taken)
                     if (v > best[r]) { best[r] = v; arg[r] = j; }
                 }
         }
