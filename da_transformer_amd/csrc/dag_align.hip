@@ -7,7 +7,7 @@
 //  * dag_align_tiles_kernel + dag_backtrack_kernel (L <= 1024): the sweep keeps E as 64x64 register
 //    tiles and evaluates a step with one DPP-broadcast add and one max per (i, j) pair, spread over
 //    the same pipeline of workgroups as the loss sweeps; it stores only the score table.  The
-//    backtrack (a wave per sample walks, others stage for it) then re-derives, for the T_b cells on the path only, the
+//    backtrack (a wave per sample walks, others may stage for it) then re-derives, for the T_b cells on the path only, the
 //    lowest predecessor index attaining the stored maximum.
 //  * dag_align_kernel: one workgroup per sample, thread <-> node j scanning its predecessors in
 //    ascending order with a strict '>' (back-pointers in LDS when T*L fits, else in the caller's
@@ -527,7 +527,7 @@ __global__ __launch_bounds__(kTileWaves * kWave) void dag_align_tiles_kernel(Ali
 // while wave 0 walks through block J out of LDS, the other waves bring in what a walk through block J - 1 reads (the
 // transitions from its two predecessor blocks, and kWalkRows rows of their scores and of the source blocks, whichever
 // step the walk enters with).  A predecessor further away is read from memory, a walk that leaves the staged rows or jumps
-// over a block stages again in front of the next step.  Measured: see launch_align.
+// over a block stages again in front of the next step.  Measured: see launch_align; when it does not pay: see walk_back.
 constexpr int kWalkRows = 48;             // two buffers and the decoder's own 25 KB fit the 160 KB of a CU
 constexpr int kWalkPitch = kBlk + 1;      // the lanes read a column of the transitions: no two in one bank
 struct WalkStage {
@@ -575,6 +575,39 @@ __device__ __forceinline__ void stage_walk(WalkStage &w, const float *A, const u
     for (int u = 0; u < kS; ++u) { const int x = q + u * kHelpers; if (x < kWalkRows * kBlk / 4) w.src[x] = vs[u]; }
 }
 
+// The walk with every step read from memory, by one wave, without LDS: the row of source blocks of the next step is fetched
+// together with the candidates of this one (it does not depend on where the path goes), so a step costs one round trip.
+// Arguments as walk_back_staged's.
+template <typename TL, bool ZERO_FOR_DEAD, typename PUT>
+__device__ __forceinline__ void walk_back_in_memory(const float *A, const unsigned char *srcblk, int spitch, const TL *links, int L,
+                                                    int translen, int s, int j, int stop, PUT put) {
+    typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
+    const int lane = threadIdx.x & (kWave - 1);
+    auto load_row = [&](int t) {   // L <= 1024 bytes: lane l holds bytes 16 l .. 16 l + 15 (rows are padded to 16 bytes)
+        return *reinterpret_cast<const u32x4 *>(srcblk + (int64_t)t * spitch + (16 * lane < spitch ? 16 * lane : 0));
+    };
+    u32x4 row = {};
+    if (s > stop) row = load_row(s);
+    for (; s > stop; --s) {
+        const int q = (j >> 2) & 3;
+        const unsigned w = q == 0 ? row.x : q == 1 ? row.y : q == 2 ? row.z : row.w;
+        const int I = (int)((unsigned)__builtin_amdgcn_readlane((int)w, j >> 4) >> (8 * (j & 3))) & 0xff;
+        const int i = I * kBlk + lane, d = j - i - 1;
+        const bool valid = d >= 0 && d < translen && i < L;
+        const float e = to_float(links[valid ? (int64_t)i * translen + d : 0]);
+        const float av = A[(int64_t)(s - 1) * L + (i < L ? i : L - 1)];
+        if (s - 1 > stop) row = load_row(s - 1);
+        const float x = valid ? av + e : DAGX_NEG_INF;
+        const float top = wave64_max(x);
+        j = I * kBlk + (int)__builtin_ctzll(__builtin_amdgcn_ballot_w64(x == top));   // the lowest lane among those that hold the maximum
+        if (__builtin_expect(!(top > DAGX_NEG_INF), 0)) {
+            if (!ZERO_FOR_DEAD) return;
+            j = 0;
+        }
+        if (lane == 0) put(s - 1, j);
+    }
+}
+
 // From cell (s, j) down to row `stop` by the whole workgroup: put(row, node), called by single lanes of wave 0, takes the
 // predecessors found.  Where no candidate has a finite score the walk ends, or with ZERO_FOR_DEAD goes on from node 0.
 // lds: kWalkLds bytes.  s, j are uniform over the workgroup.
@@ -582,7 +615,7 @@ __device__ __forceinline__ void stage_walk(WalkStage &w, const float *A, const u
 // the scores and transitions of both blocks are read in one LDS round trip, and the nodes found are kept in a register, one
 // a lane, and put 64 rows at a time.
 template <typename TL, int NT, bool ZERO_FOR_DEAD, typename PUT>
-__device__ __forceinline__ void walk_back(const float *A, const unsigned char *srcblk, int spitch, const TL *links, int L,
+__device__ __forceinline__ void walk_back_staged(const float *A, const unsigned char *srcblk, int spitch, const TL *links, int L,
                                           int translen, int s, int j, int stop, WalkStage *lds, PUT put) {
     __shared__ int at[2][2];
     if (s <= stop) return;
@@ -647,10 +680,23 @@ __device__ __forceinline__ void walk_back(const float *A, const unsigned char *s
     }
 }
 
+// STAGED: lds holds kWalkLds bytes.  A path with few steps a block, as Viterbi decoding finds where no transition stands out,
+// walks in memory all the same: a block staged costs as much as about four steps from memory (2.3 and 0.6 us; Viterbi decoding
+// at B=64, paths of 13 nodes: L=512 staged 229 us, in memory 221; L=1024 982 and 967).
+constexpr int kWalkStepsPerBlock = 4;
+template <typename TL, int NT, bool ZERO_FOR_DEAD, bool STAGED, typename PUT>
+__device__ __forceinline__ void walk_back(const float *A, const unsigned char *srcblk, int spitch, const TL *links, int L,
+                                          int translen, int s, int j, int stop, WalkStage *lds, PUT put) {
+    if (STAGED && s - stop >= kWalkStepsPerBlock * (j / kBlk + 1))
+        walk_back_staged<TL, NT, ZERO_FOR_DEAD>(A, srcblk, spitch, links, L, translen, s, j, stop, lds, put);
+    else if (threadIdx.x < kWave)
+        walk_back_in_memory<TL, ZERO_FOR_DEAD>(A, srcblk, spitch, links, L, translen, s, j, stop, put);
+}
+
 // The backtrack of the alignment, one workgroup per sample.  A sample that the pipeline gave up on (flags[b] set) is
 // done again here, from scratch, by the one-workgroup method.  (A launch of its own for the flagged samples, which are rare, would cost every call its latency.)
 constexpr int kOneGroupThreads = 1024;
-template <typename TM, typename TL, bool TRACE_LDS>
+template <typename TM, typename TL, bool TRACE_LDS, bool STAGED>
 __global__ __launch_bounds__(kOneGroupThreads) void dag_backtrack_kernel(
     const float *__restrict__ table, const unsigned char *__restrict__ srcblk_all, const int *__restrict__ flags, AlignArgs a) {
     extern __shared__ float lds_a[];
@@ -670,13 +716,19 @@ __global__ __launch_bounds__(kOneGroupThreads) void dag_backtrack_kernel(
     if (!(A[(int64_t)(Tb - 1) * L + Lb - 1] > DAGX_NEG_INF)) return;   // no finite path
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");     // the -1 fill precedes the path entries (same wave)
     if (threadIdx.x == 0) path[Lb - 1] = Tb - 1;
-    walk_back<TL, kOneGroupThreads, false>(A, srcblk_all + (int64_t)b * T * spitch, spitch, static_cast<const TL *>(a.links) + (int64_t)b * L * translen,
+    walk_back<TL, kOneGroupThreads, false, STAGED>(A, srcblk_all + (int64_t)b * T * spitch, spitch, static_cast<const TL *>(a.links) + (int64_t)b * L * translen,
                                            L, translen, Tb - 1, Lb - 1, 0, reinterpret_cast<WalkStage *>(lds_a),
                                            [&](int t, int j) { path[j] = t; });   // (the walk does not end early on a finite path)
 }
 
 constexpr size_t kAlignLdsBudget = 144 * 1024;
-
+// A walk that stages takes the LDS of a CU, so batches beyond the 256 CUs go in turns; walks in memory share a CU.  The
+// alignment's staged walk is short enough for two turns of graphs of more than two blocks (backtrack, us, in memory / staged:
+// B=300 L=64 T=16 12.9 / 14.2, L=184 T=32 25.6 / 23.2, L=512 T=64 50 / 43; B=512 L=184 25.5 / 24.5, L=328 T=41 32.9 / 34.9;
+// B=1024 L=64 15.4 / 28.0, L=100 T=24 21.6 / 37.8); the decoder's select kernel is not (B=300 L=184, 46 steps, paths of 27
+// nodes: 23.7 / 26.7; L=64, 16 steps, paths of 7: 12.0 / 15.4).
+static bool staged_alignment(int B, int L) { return B <= 256 || (B <= 512 && L > 2 * kBlk); }
+static bool staged_decode(int B) { return B <= 256; }
 
 static bool trace_fits_lds(int T, int L) {
     return L <= 65535 && (size_t)L * 8 + (size_t)T * L * 2 <= kAlignLdsBudget;
@@ -712,10 +764,18 @@ static int raise_lds_limit(const void *kern, size_t bytes, std::atomic<unsigned 
     return DAGX_OK;
 }
 constexpr size_t kBacktrackMostLds = kAlignLdsBudget > kWalkLds ? kAlignLdsBudget : kWalkLds;   // (the redo alone asks for at most the former)
-template <typename TM, typename TL, bool TRACE_LDS>
+template <typename TM, typename TL, bool TRACE_LDS, bool STAGED>
 static int prepare_backtrack() {
     static std::atomic<unsigned long long> done{0};
-    return raise_lds_limit(reinterpret_cast<const void *>(dag_backtrack_kernel<TM, TL, TRACE_LDS>), kBacktrackMostLds, done, "dag_best_alignment");
+    return raise_lds_limit(reinterpret_cast<const void *>(dag_backtrack_kernel<TM, TL, TRACE_LDS, STAGED>), kBacktrackMostLds, done, "dag_best_alignment");
+}
+
+template <typename TM, typename TL>
+static int prepare_backtracks() {
+    int rc = prepare_backtrack<TM, TL, true, true>();
+    if (!rc) rc = prepare_backtrack<TM, TL, true, false>();
+    if (!rc) rc = prepare_backtrack<TM, TL, false, true>();
+    return rc ? rc : prepare_backtrack<TM, TL, false, false>();
 }
 
 template <typename TM, typename TL>
@@ -755,9 +815,11 @@ static int launch_align(AlignArgs a, void *workspace, hipStream_t st) {
         // 24.1 and 65.0 us.)
         const bool in_lds = trace_fits_lds(a.T, a.L);
         const size_t redo_lds = (size_t)a.L * 8 + (in_lds ? (size_t)a.T * a.L * 2 : (size_t)0);
-        const size_t lds = redo_lds > kWalkLds ? redo_lds : kWalkLds;
-        auto kern = in_lds ? dag_backtrack_kernel<TM, TL, true> : dag_backtrack_kernel<TM, TL, false>;
-        if ((rc = in_lds ? prepare_backtrack<TM, TL, true>() : prepare_backtrack<TM, TL, false>())) return rc;
+        const bool staged = staged_alignment(a.B, a.L);
+        const size_t lds = staged && redo_lds < kWalkLds ? kWalkLds : redo_lds;
+        auto kern = in_lds ? (staged ? dag_backtrack_kernel<TM, TL, true, true> : dag_backtrack_kernel<TM, TL, true, false>)
+                           : (staged ? dag_backtrack_kernel<TM, TL, false, true> : dag_backtrack_kernel<TM, TL, false, false>);
+        if ((rc = prepare_backtracks<TM, TL>())) return rc;
         hipLaunchKernelGGL(kern, dim3(a.B), dim3(kOneGroupThreads), lds, st, ta.table, ta.srcblk, ta.flags, a);
         return check_launch("dag_backtrack");
     }
@@ -904,7 +966,7 @@ struct DecodeArgs {
 };
 
 // One workgroup per sample: the best node of every step, the best length, the walk back (walk_back) and the tokens.
-template <typename TL>
+template <typename TL, bool STAGED>
 __global__ __launch_bounds__(kDecodeThreads) void viterbi_select_kernel(DecodeArgs a) {
     extern __shared__ float lds_walk[];
     __shared__ int s_star;
@@ -991,7 +1053,7 @@ __global__ __launch_bounds__(kDecodeThreads) void viterbi_select_kernel(DecodeAr
     const int n = __builtin_amdgcn_readfirstlane(s_star) + 1;
     // table row s = t + 1 holds reach_t
     // (a path of finite score never meets a cell without a finite candidate)
-    walk_back<TL, kDecodeThreads, true>(A, srcblk, spitch, links, L, translen, n, __builtin_amdgcn_readfirstlane(sidx[n - 1]), 1,
+    walk_back<TL, kDecodeThreads, true, STAGED>(A, srcblk, spitch, links, L, translen, n, __builtin_amdgcn_readfirstlane(sidx[n - 1]), 1,
                                         reinterpret_cast<WalkStage *>(lds_walk), [&](int s, int j) { walk[s - 1] = j; });
     if (wave != 0) return;
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
@@ -1018,15 +1080,10 @@ __global__ __launch_bounds__(kDecodeThreads) void viterbi_select_kernel(DecodeAr
 template <typename TL>
 static int prepare_select() {
     static std::atomic<unsigned long long> done{0};
-    return raise_lds_limit(reinterpret_cast<const void *>(viterbi_select_kernel<TL>), kWalkLds, done, "dag_viterbi_decode");
+    return raise_lds_limit(reinterpret_cast<const void *>(viterbi_select_kernel<TL, true>), kWalkLds, done, "dag_viterbi_decode");
 }
 
 // What dagx_prepare_device does for the kernels of this file.
-template <typename TM, typename TL>
-static int prepare_backtracks() {
-    const int rc = prepare_backtrack<TM, TL, true>();
-    return rc ? rc : prepare_backtrack<TM, TL, false>();
-}
 template <typename TL>
 static int prepare_walks() {
     int rc = prepare_backtracks<float, TL>();
@@ -1090,9 +1147,10 @@ static int launch_decode(const void *links, const float *node_logp, const int64_
     if ((rc = check_launch("viterbi_table"))) return rc;
     DecodeArgs d{table, srcblk, links, out_len, node_tokens, penalty, T, L, translen, max_length, pad,
                  out_tokens, out_count, pred_length, nodes};
-    auto select = viterbi_select_kernel<TL>;
-    if ((rc = prepare_select<TL>())) return rc;
-    hipLaunchKernelGGL(select, dim3(B), dim3(kDecodeThreads), kWalkLds, st, d);
+    const bool staged = staged_decode(B);
+    auto select = staged ? viterbi_select_kernel<TL, true> : viterbi_select_kernel<TL, false>;
+    if (staged && (rc = prepare_select<TL>())) return rc;
+    hipLaunchKernelGGL(select, dim3(B), dim3(kDecodeThreads), staged ? kWalkLds : 0, st, d);
     return check_launch("viterbi_select");
 }
 

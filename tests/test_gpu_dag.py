@@ -304,6 +304,20 @@ def test_alignment_paths_that_dwell_and_jump(L, T, translen, hop, dtype):
     assert torch.equal(path.cpu(), _torch_path(match, links, ol, tl))
 
 
+@pytest.mark.parametrize("B,L,T", [(257, 70, 12), (257, 130, 16), (512, 129, 20), (513, 129, 20), (600, 65, 64), (2, 1024, 80)])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_alignment_on_both_sides_of_the_rule_for_the_walk(B, L, T, dtype):
+    """Batches beyond the number of CUs walk in memory or take turns; the last: long stays and a few far jumps, staged."""
+    match, links_sq, ol, tl = random_problem(B + L, B, L, T, dtype=torch.float32)
+    links = tn.extract_valid_links(links_sq, None)
+    links = (links * 2).round().masked_fill(torch.isinf(links), NEG_INF)
+    if B == 2:
+        links[:, :, 0] += 20.0
+    match, links = match.round().to(dtype), links.to(dtype)
+    path = dagx.dag_best_alignment(match.to(DEV), links.to(DEV), ol.to(DEV), tl.to(DEV))
+    assert torch.equal(path.cpu(), _torch_path(match, links, ol, tl))
+
+
 def test_alignment_calls_in_a_row_and_on_a_second_stream():
     """Calls of different shapes in a row on one stream (each clears its pipeline words itself, whatever the last call
     left in the reused workspace), then the same on a second stream and again on the first: all must give the

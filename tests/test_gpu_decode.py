@@ -62,6 +62,19 @@ def test_viterbi_walk_that_dwells_and_jumps(L, hop):
     _run_and_compare(links, u, tok, out_len, L - 1, 2.0, 1.0, True)
 
 
+@pytest.mark.parametrize("L,hop", [(63, 2), (150, 3), (150, 70)])
+def test_viterbi_decode_of_large_batches(L, hop):
+    """A batch of more samples than CUs walks in memory: the same as its slices, which stage where the path is long enough."""
+    links, u, tok, out_len = peaked_case(L, 260, L, hop=hop, min_len=L // 2)
+    shifted, u, tok, out_len = tn.extract_valid_links(links, L - 1).to(DEV), u.to(DEV), tok.to(DEV), out_len.to(DEV)
+    whole = dagx.dag_viterbi_decode(shifted, (u, tok), out_len, 2.0, 1.0, True, PAD)
+    for b in range(0, 260, 65):
+        cut = slice(b, b + 65)
+        part = dagx.dag_viterbi_decode(shifted[cut], (u[cut], tok[cut]), out_len[cut], 2.0, 1.0, True, PAD)
+        assert torch.equal(part.nodes, whole.nodes[cut]) and torch.equal(part.pred_length, whole.pred_length[cut])
+        assert torch.equal(part.output_tokens, whole.output_tokens[cut, :part.output_tokens.shape[1]])
+
+
 @pytest.mark.parametrize("joint", [False, True])
 def test_viterbi_decode_full_size(joint):
     """B=64, L=512 (64 source tokens upsampled 8 times), 128 steps."""
