@@ -133,7 +133,10 @@ __global__ __launch_bounds__(kLinkThreads) void links_fwd_kernel(
     const int sub = wave % WPR, head = head_of<H>(lane);
     // The last rows first, eight workgroups at a time (a row stays on the XCD that the backward takes it to): they are what
     // the producer of the scores wrote last, and the first rows, which the backward starts with, are the last that passed
-    // the memory-side cache.
+    // the memory-side cache.  Behind the copy that lays the scores out, that copy included, us, first rows first / last: B=64
+    // L=512 H=8 float32 280.6 / 272.6, float16 219.7 / 218.3, B=16 L=1024 H=8 float16 219.5 / 217.2; the products that make
+    // the scores and take the gradient, both copies, forward and backward together 1938 / 1935, 1135 / 1132, 1208 / 1206;
+    // tensors that fit the cache: the same.
     const unsigned octet = gridDim.x & ~7u, blk = blockIdx.x < octet ? (octet - 8 - (blockIdx.x & ~7u)) + (blockIdx.x & 7u) : blockIdx.x;
     const int64_t row = (int64_t)blk * (kLinkWaves / WPR) + wave / WPR;
     if (row >= rows) { if (WPR > 1) __syncthreads(); return; }   // the one barrier of the others

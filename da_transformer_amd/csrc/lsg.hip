@@ -127,8 +127,11 @@ __global__ __launch_bounds__(BLOCK) void lsg_fwd_kernel(
     constexpr int N = Pack<T>::N;
     // Last rows first, eight at a time (a row stays on the XCD that the backward takes it to): what the producer of the
     // logits, or a backward in the same storage, wrote last is still in the memory-side cache or on its way out of it, and
-    // so are the first rows when the backward begins with them.  [64,512,40000] float16, 64 ids: forward behind a backward
-    // 468.7 -> 444.3 us, backward 890.2 -> 883.1 us; [16,512,16000] 58.1 -> 55.6 us forward; smaller ones the same.
+    // so are the first rows when the backward begins with them.  Behind the matrix product that makes the logits (512 wide),
+    // the product included, us, first rows first / last: [64,512,40000] float16 2119 / 2038 (the forward alone 519 / 412),
+    // [16,1024,30522] float16 888 / 838, [16,512,16000] float32 1090 / 1076, float16 242.1 / 241.7; with the backward and
+    // the two products behind it 6184 / 6043, 2132 / 2100, 3072 / 3053, 639 / 640; smaller ones the same.  Behind a backward
+    // in the same storage, forward alone: 468.7 / 444.3 at [64,512,40000].
     const unsigned octet = gridDim.x & ~7u;
     const int64_t row = blockIdx.x < octet ? (octet - 8 - (blockIdx.x & ~7u)) + (blockIdx.x & 7u) : blockIdx.x;
     const int tid = threadIdx.x;

@@ -89,7 +89,7 @@ def dag_multihead_links(content, log_gates, valid_end, max_transition_length):
     the heads with log_gates (logsumexp); -inf where no transition is allowed.
 
     content [batch, prelen, prelen, heads] (the scaled query-key products), log_gates
-    [batch, prelen, heads], valid_end int64 [batch, prelen] (see valid_end_from_tokens /
+    [batch, prelen, heads] (log-probabilities as a rule; they are taken as they are, above 0 too), valid_end int64 [batch, prelen] (see valid_end_from_tokens /
     valid_end_from_bound).  As with dag_logsoftmax_gather_inplace, `content` must not be used
     afterwards when it requires grad: its storage is handed back as its gradient."""
     return DagMultiheadLinksFunc.apply(content, log_gates, valid_end, max_transition_length)

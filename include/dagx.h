@@ -103,7 +103,7 @@ int dagx_lsg_bwd(void *logits_inout, int dtype, int B, int L, int64_t V, int S,
  * log-probabilities, logsumexp over the heads -- in one pass (it has no counterpart among the
  * reference's native operators; the reference runs it as a chain of PyTorch calls).
  *   content   [B,L,L,H] contiguous, the dtype given; content[b,i,j,c] = score of i -> j for head c
- *   log_gates [B,L,H] float32;  valid_end [B,L] int64: transitions i -> j are allowed for
+ *   log_gates [B,L,H] float32, taken as they are (above 0 too);  valid_end [B,L] int64: transitions i -> j are allowed for
  *   i < j < valid_end[b,i] (the number of non-pad nodes, or bound_end + 1)
  *   links     [B,L,translen], same dtype: links[b,i,d] = log P(i -> i+d+1), -inf where not allowed
  *   lse       [B,L,H] float32 or NULL: per-head log normalisers, all the backward needs

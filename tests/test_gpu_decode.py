@@ -62,6 +62,18 @@ def test_viterbi_walk_that_dwells_and_jumps(L, hop):
     _run_and_compare(links, u, tok, out_len, L - 1, 2.0, 1.0, True)
 
 
+def test_viterbi_walk_that_stages_and_jumps():
+    """Enough steps a block for a staged walk, and one jump over four blocks in the middle of it."""
+    links, u, tok, out_len = peaked_case(9, 3, 500, hop=1, min_len=480)
+    links[:, 100, 101] = -20.0
+    links[:, 100, 400] = -0.01
+    _run_and_compare(links, u, tok, out_len, 499, 2.0, 1.0, True)
+    got = dagx.dag_viterbi_decode(tn.extract_valid_links(links, 499).to(DEV), (u.to(DEV), tok.to(DEV)), out_len.to(DEV), 2.0, 1.0, True, PAD)
+    nodes, n = got.nodes.cpu(), got.pred_length.cpu()
+    for b in range(3):
+        assert n[b] > 32 and (nodes[b, 1:n[b]] - nodes[b, :n[b] - 1]).max() >= 300
+
+
 @pytest.mark.parametrize("L,hop", [(63, 2), (150, 3), (150, 70)])
 def test_viterbi_decode_of_large_batches(L, hop):
     """A batch of more samples than CUs walks in memory: the same as its slices, which stage where the path is long enough."""
