@@ -810,9 +810,8 @@ static int launch_align(AlignArgs a, void *workspace, hipStream_t st) {
         const int B8 = (a.B + 7) & ~7;
         hipLaunchKernelGGL((dag_align_tiles_kernel<TM, TL>), dim3(B8 * C), dim3(kTileWaves * kWave), 0, st, ta);
         if ((rc = check_launch("dag_align_tiles"))) return rc;
-        // the backtrack, and the samples that the pipeline gave up on.  (float32, kernel time: with every step read from
-        // memory by one wave 38.7 us at B=64 L=512 T=64 and 174 us at B=16 L=1024 T=256, with the steps staged in LDS
-        // 24.1 and 65.0 us.)
+        // the backtrack, and the samples that the pipeline gave up on.  (float32, kernel time: walked in memory 39.5 us at
+        // B=64 L=512 T=64 and 172 us at B=16 L=1024 T=256, out of LDS 27.6 and 62.5 us.)
         const bool in_lds = trace_fits_lds(a.T, a.L);
         const size_t redo_lds = (size_t)a.L * 8 + (in_lds ? (size_t)a.T * a.L * 2 : (size_t)0);
         const bool staged = staged_alignment(a.B, a.L);
