@@ -1,0 +1,433 @@
+// The float32 sweep of dag_loss.hip in chunks of four steps: what a position block receives from the blocks below it is
+// a matrix product over the chunk's steps, on the matrix cores; only the 64 x 64 triangle on the diagonal is walked
+// step by step, by one wave.
+#pragma once
+
+#include "dag_tiles.h"
+
+namespace dagx {
+
+// Position block J works on chunk c (steps 4c+1 .. 4c+4) in stage 2J + c: everything it receives from the blocks
+// below it, which worked on that chunk at least two stages earlier, is multiplied out one stage ahead, by waves that
+// are not on the critical path, and one barrier a stage is the only synchronisation of a workgroup.
+//
+// Numbers are linear: a cell holds exp(value - kap ln 2) 2^kShift2 with one integer exponent kap per block and step,
+// chosen so that the block's largest cell lies in [2^(kShift2-1), 2^kShift2).  All scaling is by powers of two.
+constexpr int kChunk = 4;
+constexpr int kDeadExp = -(1 << 30);        // the exponent of a block without a live cell
+constexpr int kDeadBelow = -(1 << 29);      // any exponent below this is that of a dead block
+constexpr int kMatchExpMax = 1 << 17;       // match values beyond 2^+-this are rounded (down: to this or 0; up: the sample is done again)
+constexpr int kSpare = 62;                   // binades by which a step that does not scale its cells by their largest lowers them
+constexpr int kChunkBlocks = 8;             // a group owns at most this many blocks: one wave walks one block
+
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef int i32x4 __attribute__((ext_vector_type(4)));
+typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
+
+// Contiguous grouping of the position blocks [0, NBb) into at most C groups of at most kTileCap tiles (the diagonal
+// ones among them) and kChunkBlocks blocks, minimising the work of the busiest: walking and writing out a block costs
+// a workgroup about seven times what a tile costs it.  gstart[g] .. gstart[g+1]: blocks of group g (empty groups last).
+inline int partition_chunk_groups(int NBb, int W, int C, int *gstart) {
+    constexpr int kWalkCost = 7;
+    for (int cap = 1; ; ++cap) {
+        int groups = 1, tiles = 0, blocks = 0;
+        gstart[0] = 0;
+        const bool any = cap > kTileCap + kWalkCost * kChunkBlocks;   // (the work no longer bounds anything)
+        for (int Jb = 0; Jb < NBb; ++Jb) {
+            const int c = Jb - tile_ilo(Jb, W) + 1;
+            if (blocks > 0 && (tiles + c > kTileCap || blocks == kChunkBlocks || (!any && tiles + c + (blocks + 1) * (kWalkCost - 1) > cap))) {
+                if (groups < C) gstart[groups] = Jb;
+                ++groups; tiles = blocks = 0;
+            }
+            tiles += c; ++blocks;
+        }
+        if (groups <= C || any) {
+            for (int q = groups; q <= C; ++q) gstart[q] = NBb;
+            return groups;
+        }
+    }
+}
+
+// LDS of a group, in dwords.
+struct ChunkLds {
+    int depth;      // chunks of cells kept per block: read up to 2 (blocks of the group) stages after they are written
+    int eb;         // [nsrc][depth][256]  cells of four steps: (4 (i & 15) + (s & 3)) 4 + i / 16
+    int kap;        // [nsrc][depth][4]    their exponents
+    int part;       // [ntile + 1][2][256] products of a run of tiles, four steps per lane; behind them zeros
+    int part_scale; // [nblk][2][4]        the exponents they are relative to
+    int frows, foff;// [nfor][256], [nfor][64]  landing areas of table rows and offsets of blocks of lower groups
+    int total;
+};
+__device__ __host__ inline ChunkLds chunk_lds(int jb0, int nblk, int W) {
+    ChunkLds o;
+    const int flo = tile_ilo(jb0, W), nfor = jb0 - flo, nsrc = nfor + nblk;
+    int ntile = 0;
+    for (int q = 0; q < nblk; ++q) ntile += jb0 + q < W ? jb0 + q : W;
+    const int reach = nblk < W + 1 ? nblk : W + 1;
+    o.depth = 2 * reach < 3 ? 3 : 2 * reach;
+    int at = 0;
+    o.eb = at; at += nsrc * o.depth * 256;
+    o.part = at; at += (ntile + 1) * 2 * 256;
+    o.frows = at; at += nfor * 256;
+    o.foff = at; at += nfor * 64;
+    o.kap = at; at += nsrc * o.depth * 4;
+    o.part_scale = at; at += nblk * 2 * 4;
+    o.total = at;
+    return o;
+}
+constexpr int kForeign = 3;                  // foreign blocks a wave fetches at most
+constexpr int kChunkLdsBytes = 160 * 1024 - 512;
+
+// The tiles below the diagonal, block by block, dealt to the waves in runs: at most three to a wave that walks no block (a
+// helper), at most two to one that does (the triangle takes a third tile's registers).  What a wave does in a stage, in
+// hundreds of cycles (measured): walking 38, a tile 7, fetching a foreign block 4.  Helpers fetch, too; the walking waves take so many tiles that the busiest wave has least to do.
+struct TileDeal { unsigned char base_h, rem_h, base_o, rem_o; };    // tiles per helper and odd ones, tiles per walking wave and odd ones
+inline TileDeal deal_tiles(int ntile, int nblk, int nfor) {          // (on the host: its divisions cost the kernel 2 us)
+    const int helpers = kTileWaves - nblk;
+    int best = 0, best_cost = -1;
+    for (int x = 0; x <= 2 * nblk && x <= ntile; ++x) {              // tiles for the walking waves
+        const int rest = ntile - x;
+        if (rest > kTilesPerWave * helpers) continue;
+        const int own = 38 + 7 * ((x + nblk - 1) / nblk);
+        const int help = helpers > 0 ? (4 * nfor + 7 * rest + helpers - 1) / helpers : 0;
+        const int cost = own > help ? own : help;
+        if (best_cost < 0 || cost < best_cost) { best = x; best_cost = cost; }
+    }
+    const int rest = ntile - best;
+    return TileDeal{(unsigned char)(helpers > 0 ? rest / helpers : 0), (unsigned char)(helpers > 0 ? rest % helpers : 0),
+                    (unsigned char)(best / nblk), (unsigned char)(best % nblk)};
+}
+// first tile and number of tiles of a wave (the helpers' first, from the last wave down)
+__device__ __host__ __forceinline__ void wave_tiles(const TileDeal &d, int nblk, int wave, int &first, int &count) {
+    const bool walks = wave < nblk;
+    const int r = walks ? nblk - 1 - wave : kTileWaves - 1 - wave, base = walks ? d.base_o : d.base_h, rem = walks ? d.rem_o : d.rem_h;
+    first = (walks ? d.base_h * (kTileWaves - nblk) + d.rem_h : 0) + r * base + (r < rem ? r : rem);
+    count = base + (r < rem ? 1 : 0);
+}
+__device__ __host__ __forceinline__ int tiles_of_block(int J, int W) { return J < W ? J : W; }   // tiles below the diagonal
+
+// a = {a's lower half, b's lower half}, b = {a's upper half, b's upper half}.  (The results go through unsigned variables:
+// __builtin_bit_cast of an element of a vector yields element 0 with this compiler.)
+__device__ __forceinline__ void swap_halves(float &a, float &b) {
+    const u32x2 s = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(unsigned, a), __builtin_bit_cast(unsigned, b), false, false);
+    const unsigned x = s[0], y = s[1];
+    a = __builtin_bit_cast(float, x); b = __builtin_bit_cast(float, y);
+}
+
+// the largest of 64 numbers >= 0 as its bits, wave-uniform (a NaN is passed over)
+__device__ __forceinline__ unsigned wave64_max_positive(float x) {
+    unsigned v = __builtin_bit_cast(unsigned, x);
+    asm("s_nop 1\n\t"
+        "v_max_f32_dpp %0, %0, %0 quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"
+        "s_nop 1\n\t"
+        "v_max_f32_dpp %0, %0, %0 quad_perm:[2,3,0,1] row_mask:0xf bank_mask:0xf\n\t"
+        "s_nop 1\n\t"
+        "v_max_f32_dpp %0, %0, %0 row_half_mirror row_mask:0xf bank_mask:0xf\n\t"
+        "s_nop 1\n\t"
+        "v_max_f32_dpp %0, %0, %0 row_mirror row_mask:0xf bank_mask:0xf\n\t"
+        "s_nop 1\n\t"
+        "v_max_f32_dpp %0, %0, %0 row_bcast:15 row_mask:0xa bank_mask:0xf\n\t"
+        "s_nop 1\n\t"
+        "v_max_f32_dpp %0, %0, %0 row_bcast:31 row_mask:0xc bank_mask:0xf"
+        : "+v"(v));
+    return (unsigned)__builtin_amdgcn_readlane((int)v, 63);
+}
+// four maxima over the 64 lanes, each in lane 63 (side by side: no wait states between dependent steps)
+__device__ __forceinline__ void wave64_max4(float (&v)[4]) {
+    asm("s_nop 1\n\t"
+        "v_max_f32_dpp %0, %0, %0 quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"
+        "v_max_f32_dpp %1, %1, %1 quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"
+        "v_max_f32_dpp %2, %2, %2 quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"
+        "v_max_f32_dpp %3, %3, %3 quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"
+        "v_max_f32_dpp %0, %0, %0 quad_perm:[2,3,0,1] row_mask:0xf bank_mask:0xf\n\t"
+        "v_max_f32_dpp %1, %1, %1 quad_perm:[2,3,0,1] row_mask:0xf bank_mask:0xf\n\t"
+        "v_max_f32_dpp %2, %2, %2 quad_perm:[2,3,0,1] row_mask:0xf bank_mask:0xf\n\t"
+        "v_max_f32_dpp %3, %3, %3 quad_perm:[2,3,0,1] row_mask:0xf bank_mask:0xf\n\t"
+        "v_max_f32_dpp %0, %0, %0 row_half_mirror row_mask:0xf bank_mask:0xf\n\t"
+        "v_max_f32_dpp %1, %1, %1 row_half_mirror row_mask:0xf bank_mask:0xf\n\t"
+        "v_max_f32_dpp %2, %2, %2 row_half_mirror row_mask:0xf bank_mask:0xf\n\t"
+        "v_max_f32_dpp %3, %3, %3 row_half_mirror row_mask:0xf bank_mask:0xf\n\t"
+        "v_max_f32_dpp %0, %0, %0 row_mirror row_mask:0xf bank_mask:0xf\n\t"
+        "v_max_f32_dpp %1, %1, %1 row_mirror row_mask:0xf bank_mask:0xf\n\t"
+        "v_max_f32_dpp %2, %2, %2 row_mirror row_mask:0xf bank_mask:0xf\n\t"
+        "v_max_f32_dpp %3, %3, %3 row_mirror row_mask:0xf bank_mask:0xf\n\t"
+        "v_max_f32_dpp %0, %0, %0 row_bcast:15 row_mask:0xa bank_mask:0xf\n\t"
+        "v_max_f32_dpp %1, %1, %1 row_bcast:15 row_mask:0xa bank_mask:0xf\n\t"
+        "v_max_f32_dpp %2, %2, %2 row_bcast:15 row_mask:0xa bank_mask:0xf\n\t"
+        "v_max_f32_dpp %3, %3, %3 row_bcast:15 row_mask:0xa bank_mask:0xf\n\t"
+        "v_max_f32_dpp %0, %0, %0 row_bcast:31 row_mask:0xc bank_mask:0xf\n\t"
+        "v_max_f32_dpp %1, %1, %1 row_bcast:31 row_mask:0xc bank_mask:0xf\n\t"
+        "v_max_f32_dpp %2, %2, %2 row_bcast:31 row_mask:0xc bank_mask:0xf\n\t"
+        "v_max_f32_dpp %3, %3, %3 row_bcast:31 row_mask:0xc bank_mask:0xf"
+        : "+v"(v[0]), "+v"(v[1]), "+v"(v[2]), "+v"(v[3]));
+}
+// max over the lanes with the same lane & 3, in every lane
+__device__ __forceinline__ int by_step_max(int v) {
+    asm("s_nop 1\n\t"
+        "v_max_i32_dpp %0, %0, %0 row_ror:4 row_mask:0xf bank_mask:0xf\n\t"
+        "s_nop 1\n\t"
+        "v_max_i32_dpp %0, %0, %0 row_ror:8 row_mask:0xf bank_mask:0xf\n\t"
+        "s_nop 1"
+        : "+v"(v));
+    u32x2 p = __builtin_amdgcn_permlane16_swap((unsigned)v, (unsigned)v, false, false);
+    v = max((int)p[0], (int)p[1]);
+    p = __builtin_amdgcn_permlane32_swap((unsigned)v, (unsigned)v, false, false);
+    return max((int)p[0], (int)p[1]);
+}
+
+// g[t] (+)= f[lane t of the row] * a[t]: four steps, each with its own factor
+template <bool FIRST>
+__device__ __forceinline__ void scaled4(f32x4 &g, float f, f32x4 a) {
+    float g0 = g[0], g1 = g[1], g2 = g[2], g3 = g[3];
+    if constexpr (FIRST) {
+        asm("s_nop 1\n\t"
+            "v_mul_f32_dpp %0, %4, %5 row_newbcast:0 row_mask:0xf bank_mask:0xf\n\t"
+            "v_mul_f32_dpp %1, %4, %6 row_newbcast:1 row_mask:0xf bank_mask:0xf\n\t"
+            "v_mul_f32_dpp %2, %4, %7 row_newbcast:2 row_mask:0xf bank_mask:0xf\n\t"
+            "v_mul_f32_dpp %3, %4, %8 row_newbcast:3 row_mask:0xf bank_mask:0xf"
+            : "=&v"(g0), "=&v"(g1), "=&v"(g2), "=&v"(g3) : "v"(f), "v"(a[0]), "v"(a[1]), "v"(a[2]), "v"(a[3]));
+    } else {
+        asm("s_nop 1\n\t"
+            "v_fmac_f32_dpp %0, %4, %5 row_newbcast:0 row_mask:0xf bank_mask:0xf\n\t"
+            "v_fmac_f32_dpp %1, %4, %6 row_newbcast:1 row_mask:0xf bank_mask:0xf\n\t"
+            "v_fmac_f32_dpp %2, %4, %7 row_newbcast:2 row_mask:0xf bank_mask:0xf\n\t"
+            "v_fmac_f32_dpp %3, %4, %8 row_newbcast:3 row_mask:0xf bank_mask:0xf"
+            : "+v"(g0), "+v"(g1), "+v"(g2), "+v"(g3) : "v"(f), "v"(a[0]), "v"(a[1]), "v"(a[2]), "v"(a[3]));
+    }
+    g = f32x4{g0, g1, g2, g3};
+}
+
+// sum over the 64 rows of a tile for four steps: out[t] = sum_k e[k][t] P[k][lane].  e[q] holds rows 16q .. 16q+15,
+// lane 4 (k & 15) + t.  v_mfma_f32_4x4x1_16b multiplies, per 4-lane block, a 4 x 1 by a 1 x 4; with the first operand of
+// block abid broadcast to all sixteen (cbsz 4) that is four steps times 64 positions of one row.  Two chains of
+// accumulators: a dependent one issues every 12 cycles, two every 9.
+__device__ __forceinline__ f32x4 tile_product(const Tile &t, f32x4 e) {
+    f32x4 x = {0.f, 0.f, 0.f, 0.f}, y = {0.f, 0.f, 0.f, 0.f};
+#define DAGX_PAIR(q, k) \
+    x = __builtin_amdgcn_mfma_f32_4x4x1f32(e[q], t.p[16 * (q) + (k)], x, 4, (k), 0); \
+    y = __builtin_amdgcn_mfma_f32_4x4x1f32(e[q], t.p[16 * (q) + (k) + 1], y, 4, (k) + 1, 0);
+#define DAGX_ROWS(q) DAGX_PAIR(q, 0) DAGX_PAIR(q, 2) DAGX_PAIR(q, 4) DAGX_PAIR(q, 6) DAGX_PAIR(q, 8) DAGX_PAIR(q, 10) DAGX_PAIR(q, 12) DAGX_PAIR(q, 14)
+    DAGX_ROWS(0) DAGX_ROWS(1) DAGX_ROWS(2) DAGX_ROWS(3)
+#undef DAGX_ROWS
+#undef DAGX_PAIR
+    return x + y;
+}
+
+// The triangle on the diagonal (row i of a tile reaches lanes j > i only) in 48 registers instead of 64:
+//   p[0..31]:  lanes 0..31 rows 0..31, lanes 32..63 rows 32..63 -- the two 32 x 32 triangles side by side;
+//   p[32..47]: the square between them, lanes 32..63 rows 0..15, lanes 0..31 rows 16..31 of positions lane + 32.
+__device__ __forceinline__ void fold_triangle(Tile &t, int lane) {
+    const bool hi = lane >= 32;
+    float sq[16];
+#pragma unroll
+    for (int k = 0; k < 16; ++k) {
+        float x = t.p[16 + k], y = t.p[k];
+        swap_halves(x, y);       // y: lanes 0..31 have row 16 + k of lane + 32, lanes 32..63 row k
+        sq[k] = y;
+    }
+#pragma unroll
+    for (int r = 0; r < 32; ++r) t.p[r] = hi ? t.p[32 + r] : t.p[r];
+#pragma unroll
+    for (int k = 0; k < 16; ++k) t.p[32 + k] = sq[k];
+}
+// sum_i e[i] P[i][lane] over the folded triangle; upper_half: 0 in lanes 0..31, 1 in lanes 32..63.
+// v_permlane16_swap makes the rows {0,0,2,2} and {1,1,3,3} of e, v_permlane32_swap the rows {1,1,0,0} of those, another
+// one adds up the two halves' shares of the square.  A lane swap and a DPP operand want their source two wait states
+// old: the moves and swaps stand among the FMAs so that only the first needs an s_nop (one costs as much as two FMAs).
+__device__ __forceinline__ float triangle_dot(const Tile &t, float e, float upper_half) {
+    float a, b, b2, odd, crossed, rest;
+    asm("v_mov_b32 %2, %1\n\t"
+        "s_nop 1\n\t"
+        "v_permlane16_swap_b32 %1, %2\n\t"
+        "v_mov_b32 %3, %2\n\t"
+        "v_mov_b32 %4, %1\n\t"
+        "v_mul_f32_dpp %0, %1, %5 row_newbcast:0 row_mask:0xf bank_mask:0xf\n\t"
+        "v_fmac_f32_dpp %0, %1, %6 row_newbcast:1 row_mask:0xf bank_mask:0xf\n\t"
+        "v_permlane32_swap_b32 %3, %4\n\t"
+        "v_fmac_f32_dpp %0, %1, %7 row_newbcast:2 row_mask:0xf bank_mask:0xf\n\t"
+        "v_fmac_f32_dpp %0, %1, %8 row_newbcast:3 row_mask:0xf bank_mask:0xf\n\t"
+        "v_fmac_f32_dpp %0, %1, %9 row_newbcast:4 row_mask:0xf bank_mask:0xf\n\t"
+        "v_fmac_f32_dpp %0, %1, %10 row_newbcast:5 row_mask:0xf bank_mask:0xf\n\t"
+        "v_fmac_f32_dpp %0, %1, %11 row_newbcast:6 row_mask:0xf bank_mask:0xf\n\t"
+        "v_fmac_f32_dpp %0, %1, %12 row_newbcast:7 row_mask:0xf bank_mask:0xf\n\t"
+        "v_fmac_f32_dpp %0, %1, %13 row_newbcast:8 row_mask:0xf bank_mask:0xf\n\t"
+        "v_fmac_f32_dpp %0, %1, %14 row_newbcast:9 row_mask:0xf bank_mask:0xf\n\t"
+        "v_fmac_f32_dpp %0, %1, %15 row_newbcast:10 row_mask:0xf bank_mask:0xf\n\t"
+        "v_fmac_f32_dpp %0, %1, %16 row_newbcast:11 row_mask:0xf bank_mask:0xf\n\t"
+        "v_fmac_f32_dpp %0, %1, %17 row_newbcast:12 row_mask:0xf bank_mask:0xf\n\t"
+        "v_fmac_f32_dpp %0, %1, %18 row_newbcast:13 row_mask:0xf bank_mask:0xf\n\t"
+        "v_fmac_f32_dpp %0, %1, %19 row_newbcast:14 row_mask:0xf bank_mask:0xf\n\t"
+        "v_fmac_f32_dpp %0, %1, %20 row_newbcast:15 row_mask:0xf bank_mask:0xf"
+        : "=&v"(a), "+v"(e), "=&v"(odd), "=&v"(crossed), "=&v"(rest)
+        : "v"(t.p[0]), "v"(t.p[1]), "v"(t.p[2]), "v"(t.p[3]), "v"(t.p[4]), "v"(t.p[5]), "v"(t.p[6]), "v"(t.p[7]), "v"(t.p[8]), "v"(t.p[9]), "v"(t.p[10]), "v"(t.p[11]), "v"(t.p[12]), "v"(t.p[13]), "v"(t.p[14]), "v"(t.p[15]));
+    asm("v_mul_f32_dpp %0, %1, %2 row_newbcast:0 row_mask:0xf bank_mask:0xf\n\t"
+        "v_fmac_f32_dpp %0, %1, %3 row_newbcast:1 row_mask:0xf bank_mask:0xf\n\t"
+        "v_fmac_f32_dpp %0, %1, %4 row_newbcast:2 row_mask:0xf bank_mask:0xf\n\t"
+        "v_fmac_f32_dpp %0, %1, %5 row_newbcast:3 row_mask:0xf bank_mask:0xf\n\t"
+        "v_fmac_f32_dpp %0, %1, %6 row_newbcast:4 row_mask:0xf bank_mask:0xf\n\t"
+        "v_fmac_f32_dpp %0, %1, %7 row_newbcast:5 row_mask:0xf bank_mask:0xf\n\t"
+        "v_fmac_f32_dpp %0, %1, %8 row_newbcast:6 row_mask:0xf bank_mask:0xf\n\t"
+        "v_fmac_f32_dpp %0, %1, %9 row_newbcast:7 row_mask:0xf bank_mask:0xf\n\t"
+        "v_fmac_f32_dpp %0, %1, %10 row_newbcast:8 row_mask:0xf bank_mask:0xf\n\t"
+        "v_fmac_f32_dpp %0, %1, %11 row_newbcast:9 row_mask:0xf bank_mask:0xf\n\t"
+        "v_fmac_f32_dpp %0, %1, %12 row_newbcast:10 row_mask:0xf bank_mask:0xf\n\t"
+        "v_fmac_f32_dpp %0, %1, %13 row_newbcast:11 row_mask:0xf bank_mask:0xf\n\t"
+        "v_fmac_f32_dpp %0, %1, %14 row_newbcast:12 row_mask:0xf bank_mask:0xf\n\t"
+        "v_fmac_f32_dpp %0, %1, %15 row_newbcast:13 row_mask:0xf bank_mask:0xf\n\t"
+        "v_fmac_f32_dpp %0, %1, %16 row_newbcast:14 row_mask:0xf bank_mask:0xf\n\t"
+        "v_fmac_f32_dpp %0, %1, %17 row_newbcast:15 row_mask:0xf bank_mask:0xf"
+        : "=&v"(b) : "v"(crossed), "v"(t.p[32]), "v"(t.p[33]), "v"(t.p[34]), "v"(t.p[35]), "v"(t.p[36]), "v"(t.p[37]), "v"(t.p[38]), "v"(t.p[39]), "v"(t.p[40]), "v"(t.p[41]), "v"(t.p[42]), "v"(t.p[43]), "v"(t.p[44]), "v"(t.p[45]), "v"(t.p[46]), "v"(t.p[47]));
+    asm("v_mov_b32 %2, %1\n\t"
+        "v_fmac_f32_dpp %0, %3, %5 row_newbcast:0 row_mask:0xf bank_mask:0xf\n\t"
+        "v_fmac_f32_dpp %0, %3, %6 row_newbcast:1 row_mask:0xf bank_mask:0xf\n\t"
+        "v_permlane32_swap_b32 %1, %2\n\t"
+        "v_fmac_f32_dpp %0, %3, %7 row_newbcast:2 row_mask:0xf bank_mask:0xf\n\t"
+        "v_fmac_f32_dpp %0, %3, %8 row_newbcast:3 row_mask:0xf bank_mask:0xf\n\t"
+        "v_fmac_f32_dpp %0, %3, %9 row_newbcast:4 row_mask:0xf bank_mask:0xf\n\t"
+        "v_fmac_f32_dpp %0, %3, %10 row_newbcast:5 row_mask:0xf bank_mask:0xf\n\t"
+        "v_fmac_f32_dpp %0, %3, %11 row_newbcast:6 row_mask:0xf bank_mask:0xf\n\t"
+        "v_fmac_f32_dpp %0, %3, %12 row_newbcast:7 row_mask:0xf bank_mask:0xf\n\t"
+        "v_fmac_f32_dpp %0, %3, %13 row_newbcast:8 row_mask:0xf bank_mask:0xf\n\t"
+        "v_fmac_f32_dpp %0, %3, %14 row_newbcast:9 row_mask:0xf bank_mask:0xf\n\t"
+        "v_fmac_f32_dpp %0, %3, %15 row_newbcast:10 row_mask:0xf bank_mask:0xf\n\t"
+        "v_fmac_f32_dpp %0, %3, %16 row_newbcast:11 row_mask:0xf bank_mask:0xf\n\t"
+        "v_fmac_f32_dpp %0, %3, %17 row_newbcast:12 row_mask:0xf bank_mask:0xf\n\t"
+        "v_fmac_f32_dpp %0, %3, %18 row_newbcast:13 row_mask:0xf bank_mask:0xf\n\t"
+        "v_fmac_f32_dpp %0, %3, %19 row_newbcast:14 row_mask:0xf bank_mask:0xf\n\t"
+        "v_fmac_f32_dpp %0, %3, %20 row_newbcast:15 row_mask:0xf bank_mask:0xf\n\t"
+        "v_add_f32 %1, %1, %2\n\t"
+        "v_fmac_f32 %0, %1, %4"
+        : "+v"(a), "+v"(b), "=&v"(b2) : "v"(odd), "v"(upper_half), "v"(t.p[16]), "v"(t.p[17]), "v"(t.p[18]), "v"(t.p[19]), "v"(t.p[20]), "v"(t.p[21]), "v"(t.p[22]), "v"(t.p[23]), "v"(t.p[24]), "v"(t.p[25]), "v"(t.p[26]), "v"(t.p[27]), "v"(t.p[28]), "v"(t.p[29]), "v"(t.p[30]), "v"(t.p[31]));
+    return a;
+}
+
+// ---- staging -----------------------------------------------------------------------------------------------------
+// A tile's 64 x 64 transitions, loaded four neighbouring elements a lane (sixteen lanes a row), converted, and turned
+// through LDS into lane <-> output position.  What bounds staging is the number of vector-memory instructions: a CU
+// takes one per 26 cycles whatever its width, so 64 loads of one element each cost a tile of a full workgroup
+// 12 000 cycles, and the kernel 15 us at L = 512.
+//   alpha: row n of the patch is predecessor 64 I + n, memory runs along the output positions;
+//   beta:  row n is output position 64 J + n (node L_b - 1 - 64 J - n), memory runs against the predecessors.
+// The patch holds them as [row][column]: columns ascending with memory, so 63 - (position in block I) for beta.
+constexpr int kPatchPitch = kBlk + 4;      // (16-byte rows; 64 lanes a row apart meet every bank alike)
+typedef _Float16 h16x4 __attribute__((ext_vector_type(4)));
+typedef unsigned short u16x4 __attribute__((ext_vector_type(4)));
+template <typename TL> struct Quad;
+template <> struct Quad<float> { typedef f32x4 V; __device__ __forceinline__ static float get(V v, int k) { return v[k]; } };
+template <> struct Quad<__half> { typedef h16x4 V; __device__ __forceinline__ static float get(V v, int k) { return (float)v[k]; } };
+template <> struct Quad<bf16_t> { typedef u16x4 V; __device__ __forceinline__ static float get(V v, int k) { return __uint_as_float((unsigned)v[k] << 16); } };
+
+// one tile -> exp(E) 2^kShift2 in the wave's patch; `tiny` as in link_prob.  before / behind: how many elements the
+// tensor has in front of and behind the sample, where a load may reach (into places that are masked).
+template <typename TL>
+__device__ __forceinline__ void stage_tile(float *patch, const TL *links, int I, int J, int lane, int dir, int Lb, int translen, int last_index,
+                                           int before, int behind, float tiny) {
+    typedef typename Quad<TL>::V V;
+    const int dd = (J - I) * kBlk - 1, n0 = lane >> 4, c = 4 * (lane & 15);
+    const int index0 = dir == 0 ? (I * kBlk + n0) * translen + dd + c - n0 : (Lb - 1 - J * kBlk - n0) * translen + dd + n0 - c - 3;
+    const int step = 4 * (dir == 0 ? translen - 1 : 1 - translen);
+    const int lowest_i = min(index0, index0 + 15 * step), highest_i = max(index0, index0 + 15 * step) + 3;
+    float *const dst = patch + n0 * kPatchPitch + (dir == 0 ? c : kBlk - 4 - c);
+    // element k of group g (row n0 + 4 g): its distance is d0 + g dstep + k; it has a place in the sample for k < k_end(g)
+    const int d0 = dir == 0 ? dd + c - n0 : dd + n0 - c - 3, dstep = dir == 0 ? -4 : 4;
+    auto k_end = [&](const int g) { return dir == 0 ? Lb - J * kBlk - c : (J * kBlk + n0 + 4 * g < Lb ? 4 : 0); };
+    auto valid = [&](const int g, const int k, const int ke) { return (unsigned)(d0 + g * dstep + k) < (unsigned)translen && k < ke; };
+    const int back = kBlk * translen + 4 * kBlk;   // (an unsigned offset from a scalar base: one register a load)
+    const char *const base = reinterpret_cast<const char *>(links) - (int64_t)back * (int64_t)sizeof(TL);
+    auto load = [&](const int at) { V v; __builtin_memcpy(&v, base + (unsigned)(at + back) * (unsigned)sizeof(TL), sizeof(V)); return v; };
+    V raw[16];
+    if (__builtin_expect(__builtin_amdgcn_ballot_w64(lowest_i < -before || highest_i > last_index + behind) == 0, 1)) {
+#pragma unroll
+        for (int g = 0; g < 16; ++g) raw[g] = load(index0 + g * step);
+    } else {
+        // next to an end of the tensor (which has at least four elements): loads that would leave it are moved inside, and
+        // what they find there to where it belongs
+        const int most = last_index + behind - 3;
+#pragma unroll
+        for (int g = 0; g < 16; ++g) {
+            const int want = index0 + g * step;
+            raw[g] = load(want < -before ? -before : want > most ? most : want);
+        }
+#pragma unroll
+        for (int g = 0; g < 16; ++g) {
+            const int want = index0 + g * step, front = -before - want, over = want - most;
+#pragma unroll
+            for (int r = 1; r < 4; ++r) {
+                const V v = raw[g];
+                raw[g][0] = over >= r ? v[1] : v[0];
+                raw[g][1] = front >= r ? v[0] : over >= r ? v[2] : v[1];
+                raw[g][2] = front >= r ? v[1] : over >= r ? v[3] : v[2];
+                raw[g][3] = front >= r ? v[2] : v[3];
+            }
+        }
+    }
+    // every (row, column) of the tile is a transition of the sample
+    const bool interior = J > I && dd + kBlk - 1 < translen && J * kBlk + kBlk - 1 < Lb;
+    float lowest = 0.f;
+    if (interior) {
+#pragma unroll
+        for (int g = 0; g < 16; ++g)
+#pragma unroll
+            for (int k = 0; k < 4; ++k) lowest = fminf(lowest, Quad<TL>::get(raw[g], k));
+        if (__builtin_amdgcn_ballot_w64(lowest < -79.f) == 0) {
+#pragma unroll
+            for (int g = 0; g < 16; ++g) {
+                f32x4 w;
+#pragma unroll
+                for (int k = 0; k < 4; ++k) w[k] = __builtin_ldexpf(fast_exp2(Quad<TL>::get(raw[g], k) * kLog2e), kShift2);
+                *reinterpret_cast<f32x4 *>(dst + 4 * g * kPatchPitch) = w;
+            }
+            return;
+        }
+    } else {
+#pragma unroll
+        for (int g = 0; g < 16; ++g) {
+            const int ke = k_end(g);
+#pragma unroll
+            for (int k = 0; k < 4; ++k) lowest = fminf(lowest, valid(g, k, ke) ? Quad<TL>::get(raw[g], k) : 0.f);
+        }
+        if (__builtin_amdgcn_ballot_w64(lowest < -79.f) == 0) {
+#pragma unroll
+            for (int g = 0; g < 16; ++g) {
+                f32x4 w;
+                const int ke = k_end(g);
+#pragma unroll
+                for (int k = 0; k < 4; ++k) {
+                    const float v = __builtin_ldexpf(fast_exp2(Quad<TL>::get(raw[g], k) * kLog2e), kShift2);
+                    w[k] = valid(g, k, ke) ? v : 0.f;
+                }
+                *reinterpret_cast<f32x4 *>(dst + 4 * g * kPatchPitch) = w;
+            }
+            return;
+        }
+    }
+#pragma unroll
+    for (int g = 0; g < 16; ++g) {
+        f32x4 w;
+        const int ke = k_end(g);
+#pragma unroll
+        for (int k = 0; k < 4; ++k) w[k] = link_prob<true, kShift2>(Quad<TL>::get(raw[g], k), valid(g, k, ke), tiny);
+        *reinterpret_cast<f32x4 *>(dst + 4 * g * kPatchPitch) = w;
+    }
+}
+__device__ __forceinline__ void read_patch(Tile &t, const float *patch, int lane, int dir) {
+    asm volatile("" ::: "memory");
+    if (dir == 0) {
+#pragma unroll
+        for (int r = 0; r < kBlk; ++r) t.p[r] = patch[r * kPatchPitch + lane];
+    } else {
+#pragma unroll
+        for (int r = 0; r < kBlk; r += 4) {
+            const f32x4 v = *reinterpret_cast<const f32x4 *>(patch + lane * kPatchPitch + kBlk - 4 - r);
+            t.p[r] = v[3]; t.p[r + 1] = v[2]; t.p[r + 2] = v[1]; t.p[r + 3] = v[0];
+        }
+    }
+    asm volatile("" ::: "memory");
+}
+
+__device__ __forceinline__ float pow2_clamped(int x, int floor_exp) {   // 2^x for x <= 0; 2^floor_exp (or 0: floor -127) below
+    const int c = x > floor_exp ? x : floor_exp;
+    return __builtin_bit_cast(float, (unsigned)(c + 127) << 23);
+}
+
+}  // namespace dagx

@@ -13,18 +13,20 @@
 //   alpha[t][node] = off[t][p/64] + hat[t][node]          (hat indexed by node, off by position block)
 // so the residuals keep full fp32 resolution no matter how negative the log-likelihood is.
 //
-// Two sweep implementations write this format:
-//   * dag_sweep_tiles_kernel ("fast"): exp(E) is staged once into registers as 64x64 tiles
-//     (lane <-> output position, 64 predecessors per tile), each step is a block-scaled
-//     linear-domain mat-vec done with DPP row-broadcast FMAs; the tiles of one sweep are spread
-//     over a small pipeline of workgroups that hand the running vector on through global memory.
+// Three sweep implementations write this format:
+//   * sweep_chunks_group ("fast", float32): exp(E) is staged once into registers as 64x64 tiles (lane <-> output position,
+//     64 predecessors per tile).  Four steps at a time, what a block of positions receives from the blocks below it is
+//     a product on the matrix cores; the 64x64 triangle on its diagonal is walked step by step by one wave.  The tiles of
+//     one sweep are spread over a small pipeline of workgroups that hand the running vector on through global memory.
+//   * sweep_tiles_group ("wide", float64): the same tiles, every step a block-scaled linear-domain mat-vec done with DPP
+//     row-broadcast FMAs; re-does the samples whose float32 sweeps do not agree.
 //   * dag_sweep_exact_kernel: every term evaluated in the log domain, one workgroup per sweep.
-//     Handles any size and any dynamic range; it re-does the samples the fast kernel flags.
+//     Handles any size and any dynamic range; it re-does the samples the others leave.
 #include <atomic>
 #include <cstdint>
 #include <type_traits>
 
-#include "dag_tiles.h"
+#include "dag_chunks.h"
 
 namespace dagx {
 
@@ -53,6 +55,7 @@ struct SweepArgs {
     unsigned char rev[2], upper[2];
     int only_flagged;  // exact kernel: 0 = every sample; 1 = samples whose flag is set
     unsigned char gtab[kMaxBlocksFast + 1][12];  // fast path: gtab[NBb][g] = first block of group g (host-built)
+    TileDeal deal[kMaxBlocksFast + 1][12];       // and how its tiles are dealt to its waves (float32 sweeps)
     double *zfast;     // [2][B] the fast kernel's own read-outs (never rewritten by the exact kernel)
 };
 
@@ -242,20 +245,8 @@ __global__ __launch_bounds__(NT) void dag_sweep_exact_kernel(SweepArgs a) {
 }
 
 // ================================================================================================
-// Fast sweep: register-resident exp(E) tiles, DPP broadcast FMAs, pipelined workgroups
+// Tile sweeps: register-resident exp(E) tiles, pipelined workgroups
 // ================================================================================================
-
-// One step of one tile: sum_r e[r] * P[r][lane], e given 16-replicated in four registers
-__device__ __forceinline__ float tile_dot(const Tile &t, float e0, float e1, float e2, float e3) {
-    // one accumulator, started by a multiply: dependent DPP FMAs issue as fast as independent ones here, and
-    // every instruction saved is an issue slot of the SIMD
-    float a;
-    mul16_rowbcast(a, e0, t.p);
-    fma16_rowbcast(a, e1, t.p + 16);
-    fma16_rowbcast(a, e2, t.p + 32);
-    fma16_rowbcast(a, e3, t.p + 48);
-    return a;
-}
 
 // ---- the wide variant: the same sweep with float64 linear-domain numbers --------------------------------------
 // What the float32 sweep cannot hold is, almost always, a cell far under the maximum of its block or a block far
@@ -342,18 +333,8 @@ __device__ __forceinline__ void scaled_sum4(double &acc, double f, double v0, do
         : "+v"(acc) : "v"(f), "v"(v0), "v"(v1), "v"(v2), "v"(v3), "n"(U0), "n"(U0 + 1), "n"(U0 + 2), "n"(U0 + 3));
 }
 
-// The linear-domain number type of a sweep and what depends on it.
-template <bool WIDE> struct Lin;
-template <> struct Lin<false> {
-    using T = float;
-    static constexpr float kFacFloor = -126.f;                       // upper sweep: smallest exponent of a block factor
-    __device__ static __forceinline__ float tiny() { return kTinyStored; }
-    __device__ static __forceinline__ float flushed_sum() { return 2.4074124e-35f; }   // 2^-115, see own_block
-    __device__ static __forceinline__ float exp2s(float x) { return exp2_shifted(x); }          // 2^(x + shift)
-    __device__ static __forceinline__ float exp2u(float x) { return fast_exp2(x); }             // 2^x
-    __device__ static __forceinline__ float log2u(float y) { return log2_unshifted(y); }        // log2(y) - 2 * shift
-};
-template <> struct Lin<true> {
+// The float64 linear-domain numbers of the wide sweeps.
+struct Lin {
     using T = double;
     static constexpr float kFacFloor = -1022.f;
     __device__ static __forceinline__ double tiny() { return 2.2250738585072014e-308; }          // 2^-1022
@@ -383,12 +364,8 @@ template <> struct Lin<true> {
         return !(x <= -6000.0) ? r : 0.0;
     }
     __device__ static __forceinline__ double exp2s(float x) { return exp2_with(x, kShiftWide); }
-    __device__ static __forceinline__ double exp2u(float x) { return exp2_with(x, 0); }
-    // log2(y) minus the shift of a float64 number and that of a staged transition
-    __device__ static __forceinline__ float log2u(double y) {
-        return (float)(__builtin_amdgcn_frexp_exp(y) - (kShiftWide + kShiftLinksWide)) + fast_log2((float)__builtin_amdgcn_frexp_mant(y));
-    }
-    // the same as a float64 number: the exponent exactly, the logarithm of the fraction (in [-1, 0]) from v_log_f32
+    // log2(y) minus the shift of a float64 number and that of a staged transition: the exponent exactly, the logarithm of the
+    // fraction (in [-1, 0]) from v_log_f32
     __device__ static __forceinline__ double log2u_wide(double y) {
         return (double)(__builtin_amdgcn_frexp_exp(y) - (kShiftWide + kShiftLinksWide)) + (double)fast_log2((float)__builtin_amdgcn_frexp_mant(y));
     }
@@ -402,19 +379,19 @@ constexpr int kEvPart = kEvEbuf + 2 * kMaxBlocksFast * kBlk;            // [12][
 constexpr int kEvNowhere = kEvPart + kPartBlocks * kPartRows * kBlk;    // [64] where a wave's unused tile slots "write their partial sums"
 constexpr int kEvCount = kEvNowhere + kBlk;
 // then, in floats from the start of the dynamic segment:
-template <bool WIDE> struct StepLds {
-    static constexpr int kRelb = kEvCount * (WIDE ? 2 : 1);              // [2][16] block offsets rel. to the reference (float; double in the wide variant)
+struct StepLds {
+    static constexpr int kRelb = kEvCount * 2;              // [2][16] block offsets rel. to the reference (float; double in the wide variant)
     // landing areas of the asynchronous global -> LDS copies (one slot per consuming wave), double-buffered by step parity
-    static constexpr int kStageM = kRelb + 2 * kMaxBlocksFast * (WIDE ? 2 : 1);   // [2][8 waves][2][64] dwords: match rows of each wave's own blocks (raw elements)
+    static constexpr int kStageM = kRelb + 2 * kMaxBlocksFast * 2;   // [2][8 waves][2][64] dwords: match rows of each wave's own blocks (raw elements)
     static constexpr int kStageF = kStageM + 2 * kTileWaves * 2 * kBlk;  // [2][8 waves][2][64] floats: table residuals of the wave's foreign blocks
     static constexpr int kStageO = kStageF + 2 * kTileWaves * 2 * kBlk;  // [2][64] dwords: the table's offset row (16 doubles, padded)
     static constexpr int kStageP = kStageO + 2 * kBlk;                    // [2][64] dwords: snapshot of the progress word of the group below
     static constexpr int kLastV = kStageP + 2 * kBlk;                    // [8 waves][64] the values of the last step (for the read-out)
-    static constexpr int kLastC = kLastV + kTileWaves * kBlk * (WIDE ? 2 : 1);   // [8 waves] doubles: the reference they are relative to
+    static constexpr int kLastC = kLastV + kTileWaves * kBlk * 2;   // [8 waves] doubles: the reference they are relative to
     // (kLastV holds float64 values in the wide variant: twice the room)
     // the wide variant keeps the last rows of every wave's third tile here and reads them back in every step: the
     // registers they would occupy are what its float64 temporaries of phase B need
-    static constexpr int kTailRows = WIDE ? 12 : 0;
+    static constexpr int kTailRows = 12;
     static constexpr int kTail = kLastC + 2 * kTileWaves;                // [8 waves][kTailRows][64] floats
     static constexpr int kStepFloats = kTail + kTileWaves * kTailRows * kBlk;
 };
@@ -443,16 +420,16 @@ template <bool WIDE> struct StepLds {
 // addresses, table offsets, the tile's band limits -- is computed before the loop, the loop body is
 // instantiated for both parities of the double buffers (immediate LDS offsets), and the LDS reads
 // of a phase are issued together.
-template <typename TM, typename TL, bool WIDE>
+template <typename TM, typename TL>
 __device__ __forceinline__ void sweep_tiles_group(const SweepArgs &a, const int b, const int slot, const int g, float *lds_raw,
                                                   int *gstart, int *s_abort_p) {
-    using LN = Lin<WIDE>;
-    using EV = typename LN::T;          // exp(residual), tile sums, block factors: float, or double in the wide variant
+    using LN = Lin;
+    using EV = double;                  // exp(residual), tile sums, block factors
     // A cell's value relative to the step's reference: float, or double in the wide variant -- its samples are the
     // ones whose values lie hundreds of nats from their reference, where a float32 value is 3e-5 coarse, and the
     // two read-outs of a sample can only be held to 5e-5 of each other if they are finer than that.
-    using VT = typename LN::T;
-    using LD = StepLds<WIDE>;
+    using VT = double;
+    using LD = StepLds;
     constexpr int kLdsRelb = LD::kRelb, kLdsStageM = LD::kStageM, kLdsStageF = LD::kStageF, kLdsStageO = LD::kStageO,
                   kLdsStageP = LD::kStageP, kLdsLastV = LD::kLastV, kLdsLastC = LD::kLastC, kLdsStepFloats = LD::kStepFloats;
     // slot: which of the sample's two sweeps (its tables, pipeline words and read-out); dir: its direction;
@@ -545,7 +522,7 @@ __device__ __forceinline__ void sweep_tiles_group(const SweepArgs &a, const int 
     // What a finite transition below the staged range becomes: 0 in a lower sweep, the smallest number the staged
     // range holds in an upper sweep (exp(-126) under a certain transition in the float32 sweeps, exp(-175) in the
     // wide ones).
-    constexpr int kLinkShift = WIDE ? kShiftLinksWide : kShift2;
+    constexpr int kLinkShift = kShiftLinksWide;
     const float tiny = !upper ? 0.f : kTinyStored;   // (2^-126 as stored: at least any transition that is not staged, in either variant)
     if (my_ok[0]) load_tile<true, 16, TL, kLinkShift>(t0, links, my_I[0], my_J[0], lane, dir, Lb, translen, stage[wave], tiny);
     if (my_ok[1]) load_tile<true, 16, TL, kLinkShift>(t1, links, my_I[1], my_J[1], lane, dir, Lb, translen, stage[wave], tiny);
@@ -553,8 +530,7 @@ __device__ __forceinline__ void sweep_tiles_group(const SweepArgs &a, const int 
     __syncthreads();   // every wave is done with its transpose patch: the LDS now holds the step buffers
 
     EV *const ebuf = reinterpret_cast<EV *>(lds_raw) + kEvEbuf;   // [parity][block][64]
-    float *const relb = lds_raw + kLdsRelb;   // [parity][block]
-    double *const relb64 = reinterpret_cast<double *>(lds_raw + kLdsRelb);   // the same in the wide variant
+    double *const relb64 = reinterpret_cast<double *>(lds_raw + kLdsRelb);   // [parity][block]
     constexpr int kEbufPar = kMaxBlocksFast * kBlk;   // floats between the two parities of ebuf
 
     // ---- step 0 is known to every group: only position 0 is alive ----
@@ -566,14 +542,11 @@ __device__ __forceinline__ void sweep_tiles_group(const SweepArgs &a, const int 
     __syncthreads();
     constexpr int kTailRows = LD::kTailRows, kTailFirst = kBlk - kTailRows;
     float *const tail_lane = lds_raw + LD::kTail + wave * (kTailRows * kBlk) + lane;   // (read and written by this wave alone)
-    if constexpr (WIDE) {
 #pragma unroll
-        for (int u = 0; u < kTailRows; ++u) tail_lane[u * kBlk] = my_ok[2] ? t2.p[kTailFirst + u] : 0.f;
-    }
+    for (int u = 0; u < kTailRows; ++u) tail_lane[u * kBlk] = my_ok[2] ? t2.p[kTailFirst + u] : 0.f;
     if (tid == 0 && alive0) ebuf[0] = LN::exp2s(0.f);
     if (tid < 2 * kMaxBlocksFast) {
-        if constexpr (WIDE) relb64[tid] = (tid == 0 && alive0) ? 0.0 : (double)DAGX_NEG_INF;
-        else relb[tid] = (tid == 0 && alive0) ? 0.f : DAGX_NEG_INF;
+        relb64[tid] = (tid == 0 && alive0) ? 0.0 : (double)DAGX_NEG_INF;
     }
     for (int ob = wave; ob < nblk; ob += kTileWaves) {  // own blocks of the first row of the table
         const int Jb = jb0 + ob, p = Jb * kBlk + lane;
@@ -620,9 +593,8 @@ __device__ __forceinline__ void sweep_tiles_group(const SweepArgs &a, const int 
     // cell becomes, and what is added to every block sum for the products that may have been flushed.
     EV tiny_up = upper ? LN::tiny() : (EV)0, flush_up = upper ? LN::flushed_sum() : (EV)0;
     asm volatile("" : "+v"(tiny_up), "+v"(flush_up));
-    const float *const lds_l15 = lds_raw + (lane & 15);   // every 16-lane row addresses the same 16 values
     float *const lds_lane = lds_raw + lane;
-    const EV *const ev_l15 = reinterpret_cast<const EV *>(lds_raw) + (lane & 15);   // the same two for the linear-domain numbers
+    const EV *const ev_l15 = reinterpret_cast<const EV *>(lds_raw) + (lane & 15);   // every 16-lane row addresses the same 16 values
     EV *const ev_lane = reinterpret_cast<EV *>(lds_raw) + lane;
     // the block this wave owns in phase B (a second one, wave + 8, is handled without look-ahead)
     const bool owner = wave < nblk;
@@ -796,21 +768,19 @@ __device__ __forceinline__ void sweep_tiles_group(const SweepArgs &a, const int 
         if (__builtin_expect(fetcher, 0)) fetch_step(parity, s);   // step s + 1 uses the buffers that now hold step s - 1
         double rl64 = 0.0;
         float rl;
-        if constexpr (WIDE) { rl64 = relb64[CUR * kMaxBlocksFast + (lane & 15)]; rl = (float)rl64; }
-        else rl = lds_l15[kLdsRelb + CUR * kMaxBlocksFast];
+        rl64 = relb64[CUR * kMaxBlocksFast + (lane & 15)]; rl = (float)rl64;
         auto read_e = [&](const int sl, EV (&ev)[4]) __attribute__((always_inline)) {
             const EV *src = ev_l15 + opaque_uniform(e_off[sl]);
 #pragma unroll
             for (int q = 0; q < 4; ++q) ev[q] = src[CUR * kEbufPar + 16 * q];
         };
-        EV eva[4], evb[4];
+        EV eva[4];
         read_e(0, eva);
-        if constexpr (!WIDE) read_e(1, evb);
+        
         float tail[kTailRows > 0 ? kTailRows : 1];
-        if constexpr (WIDE) {   // (requested now, used behind the first two tiles)
+        // (requested now, used behind the first two tiles)
 #pragma unroll
-            for (int u = 0; u < kTailRows; ++u) tail[u] = tail_lane[u * kBlk];
-        }
+        for (int u = 0; u < kTailRows; ++u) tail[u] = tail_lane[u * kBlk];
         // Rvec: lane Jb holds the scale of position block Jb = max offset over its predecessor blocks
         const float rpre = row16_prefix_max(rl);
         const float dmax = lane_bcast(rpre, 15);
@@ -829,18 +799,13 @@ __device__ __forceinline__ void sweep_tiles_group(const SweepArgs &a, const int 
         // (here, with the reads of this step's vectors in flight: its one LDS read then costs no wait of its own)
         if (consumer) own_requests(parity, s);
         tile_step(0, t0, eva);
-        if constexpr (WIDE) {   // one set of float64 e values at a time: a second set does not fit the register file
-            read_e(1, eva);
-            tile_step(1, t1, eva);
-            read_e(2, eva);
-            EV acc = 0;
-            if (__builtin_expect(s >= s_lo[2] && s <= s_hi[2], 1)) acc = tile_dot_tail(t2, tail, eva[0], eva[1], eva[2], eva[3]);
-            ev_lane[opaque_uniform(part_off[2])] = acc;
-        } else {
-            read_e(2, eva);
-            tile_step(1, t1, evb);
-            tile_step(2, t2, eva);
-        }
+        // one set of float64 e values at a time: a second set does not fit the register file
+        read_e(1, eva);
+        tile_step(1, t1, eva);
+        read_e(2, eva);
+        EV acc = 0;
+        if (__builtin_expect(s >= s_lo[2] && s <= s_hi[2], 1)) acc = tile_dot_tail(t2, tail, eva[0], eva[1], eva[2], eva[3]);
+        ev_lane[opaque_uniform(part_off[2])] = acc;
         __syncthreads();
         // ---------------- phase B ----------------
         // Every earlier store of this wave is complete (those of step s-1 were issued a whole step ago, so
@@ -864,8 +829,7 @@ __device__ __forceinline__ void sweep_tiles_group(const SweepArgs &a, const int 
                 ev_lane[kEvEbuf + NXT * kEbufPar + I * kBlk] = I * kBlk + lane < Lb ? ef : (EV)0;
                 const double o = reinterpret_cast<const double *>(lds_raw + stage_o(NXT))[I];
                 if (lane == 0) {
-                    if constexpr (WIDE) relb64[NXT * kMaxBlocksFast + I] = o > (double)DAGX_NEG_INF ? o - cnext : (double)DAGX_NEG_INF;
-                    else relb[NXT * kMaxBlocksFast + I] = o > (double)DAGX_NEG_INF ? (float)(o - cnext) : DAGX_NEG_INF;
+                    relb64[NXT * kMaxBlocksFast + I] = o > (double)DAGX_NEG_INF ? o - cnext : (double)DAGX_NEG_INF;
                 }
             }
         }
@@ -884,7 +848,7 @@ __device__ __forceinline__ void sweep_tiles_group(const SweepArgs &a, const int 
             // for them (read four at a time, next to their use, they cost two, one behind the other)
             EV pr[8];
 #pragma unroll
-            for (int u = 0; u < (WIDE ? 4 : 8); ++u) pr[u] = prd[u * kBlk];   // (float64 sums: four at a time, for want of registers)
+            for (int u = 0; u < 4; ++u) pr[u] = prd[u * kBlk];   // (float64 sums: four at a time, for want of registers)
             asm volatile("" ::: "memory");
             float rlb = rl;
             asm volatile("" : "+v"(rlb));
@@ -894,39 +858,28 @@ __device__ __forceinline__ void sweep_tiles_group(const SweepArgs &a, const int 
             // finite - -inf (+inf) gives 0, factor 1, and -inf - -inf (NaN) the floor (the median of three with a NaN
             // among them is the smallest of the others), both in front of rows that hold 0.
             EV fac;
-            if constexpr (WIDE) {   // (the offsets' difference in float64: see Lin<true>::exp2_with)
-                double rlb64 = rl64;
-                asm volatile("" : "+v"(rlb64));
-                // (R is the float32 rounding of the largest offset, so the block that sets the scale may lie a rounding
-                //  error above it: capped at 2, not at 1, or it would lose that sliver of its mass in every step)
-                const double x = (rlb64 - (double)R) * (double)kLog2e;
-                fac = LN::exp2_with(__builtin_fmax(__builtin_fmin(x, 1.0), (double)fac_floor), 0);
-            } else {
-                fac = LN::exp2u(__builtin_amdgcn_fmed3f((rlb - R) * kLog2e, fac_floor, 0.f));
-            }
+            // (the offsets' difference in float64: see Lin::exp2_with)
+            double rlb64 = rl64;
+            asm volatile("" : "+v"(rlb64));
+            // (R is the float32 rounding of the largest offset, so the block that sets the scale may lie a rounding
+            //  error above it: capped at 2, not at 1, or it would lose that sliver of its mass in every step)
+            const double x = (rlb64 - (double)R) * (double)kLog2e;
+            fac = LN::exp2_with(__builtin_fmax(__builtin_fmin(x, 1.0), (double)fac_floor), 0);
             // partial row u belongs to predecessor block ilo + u (ilo = 0 when every lower block is a predecessor):
             // with the factors shifted down by ilo lanes, row u takes its factor from lane u by DPP broadcast
             EV facu = fac;
             if constexpr (!UNL) {
                 const int from = ((lane & 15) + tile_ilo(Jb, W)) << 2;
-                if constexpr (WIDE) {
-                    const long long bits = __builtin_bit_cast(long long, fac);
-                    const unsigned lo = (unsigned)__builtin_amdgcn_ds_bpermute(from, (int)(bits & 0xffffffffLL));
-                    const unsigned hi = (unsigned)__builtin_amdgcn_ds_bpermute(from, (int)(bits >> 32));
-                    facu = __builtin_bit_cast(double, ((long long)hi << 32) | (long long)lo);
-                } else {
-                    facu = __builtin_bit_cast(float, __builtin_amdgcn_ds_bpermute(from, __builtin_bit_cast(int, fac)));
-                }
+                const long long bits = __builtin_bit_cast(long long, fac);
+                const unsigned lo = (unsigned)__builtin_amdgcn_ds_bpermute(from, (int)(bits & 0xffffffffLL));
+                const unsigned hi = (unsigned)__builtin_amdgcn_ds_bpermute(from, (int)(bits >> 32));
+                facu = __builtin_bit_cast(double, ((long long)hi << 32) | (long long)lo);
             }
             EV tot;
             scaled_sum4<0>(tot, facu, pr[0], pr[1], pr[2], pr[3]);
-            if constexpr (WIDE) {
 #pragma unroll
-                for (int u = 0; u < 4; ++u) pr[u] = prd[(4 + u) * kBlk];
-                scaled_sum4<4>(tot, facu, pr[0], pr[1], pr[2], pr[3]);
-            } else {
-                scaled_sum4<4>(tot, facu, pr[4], pr[5], pr[6], pr[7]);
-            }
+            for (int u = 0; u < 4; ++u) pr[u] = prd[(4 + u) * kBlk];
+            scaled_sum4<4>(tot, facu, pr[0], pr[1], pr[2], pr[3]);
             if (__builtin_expect(nt > 8, 0)) {
                 scaled_sum4<8>(tot, facu, prd[8 * kBlk], prd[9 * kBlk], prd[10 * kBlk], prd[11 * kBlk]);
                 scaled_sum4<12>(tot, facu, prd[12 * kBlk], prd[13 * kBlk], prd[14 * kBlk], prd[15 * kBlk]);
@@ -941,31 +894,24 @@ __device__ __forceinline__ void sweep_tiles_group(const SweepArgs &a, const int 
             // are taken against -3e38 instead, which leaves them -inf and their exponentials 0.
             const bool inband = p >= s && p <= slack + s;
             VT vt;
-            if constexpr (WIDE) vt = inband ? ((double)R + LN::log2u_wide(tot) * 0.6931471805599453) + (double)mv : (double)DAGX_NEG_INF;
-            else vt = inband ? (R + LN::log2u(tot) * kLn2) + mv : DAGX_NEG_INF;
+            vt = inband ? ((double)R + LN::log2u_wide(tot) * 0.6931471805599453) + (double)mv : (double)DAGX_NEG_INF;
             const float v = (float)vt;
             const float vmax = wave64_max(v);
             const double offn = cref + (double)vmax;
             float fh;   // the residual against the block's maximum (formed from the float64 value in the wide variant)
-            if constexpr (WIDE) fh = (float)(vt - (double)fmaxf(vmax, -3.0e38f));
-            else fh = v - fmaxf(vmax, -3.0e38f);
+            fh = (float)(vt - (double)fmaxf(vmax, -3.0e38f));
             EV e;
-            if constexpr (WIDE) {
-                // exp(v - vmax) not from the rounded v but from the sum itself: tot * exp(R + match - vmax) in float64
-                // (the shift of the staged transitions taken out, that of the float64 numbers staying in), so that a
-                // cell hundreds of nats under its reference hands on what it received to float64 accuracy
-                const double x = ((((double)R - (double)vmax) + (double)mv) * (double)kLog2e) - (double)kShiftLinksWide;
-                // (a block without a live cell has vmax = -inf and exponentials 0 -- unless its sums are NaNs, which the
-                //  maximum skipped and which must stay NaNs)
-                e = !inband ? 0.0 : (vmax > -3.0e38f ? LN::times_exp2(tot, x) : (tot == tot ? 0.0 : tot));
-            } else {
-                e = LN::exp2s(fh * kLog2e);
-            }
+            // exp(v - vmax) not from the rounded v but from the sum itself: tot * exp(R + match - vmax) in float64
+            // (the shift of the staged transitions taken out, that of the float64 numbers staying in), so that a
+            // cell hundreds of nats under its reference hands on what it received to float64 accuracy
+            const double xe = ((((double)R - (double)vmax) + (double)mv) * (double)kLog2e) - (double)kShiftLinksWide;
+            // (a block without a live cell has vmax = -inf and exponentials 0 -- unless its sums are NaNs, which the
+            //  maximum skipped and which must stay NaNs)
+            e = !inband ? 0.0 : (vmax > -3.0e38f ? LN::times_exp2(tot, xe) : (tot == tot ? 0.0 : tot));
             e = (fh > -3.0e38f && e < tiny_up) ? tiny_up : e;   // upper sweep: a live cell never flushes (a NaN stays one)
             ev_lane[opaque_uniform(kEvEbuf + NXT * kEbufPar + Jb * kBlk)] = e;
             if (lane == 0) {
-                if constexpr (WIDE) relb64[NXT * kMaxBlocksFast + Jb] = (double)vmax - (double)d_s;
-                else relb[NXT * kMaxBlocksFast + Jb] = vmax - d_s;
+                relb64[NXT * kMaxBlocksFast + Jb] = (double)vmax - (double)d_s;
                 store_agent(off_at(t, Jb), offn);
             }
             if (p < Lb) store_agent(hat_at(t, node), fh);
@@ -1031,6 +977,511 @@ __device__ __forceinline__ void sweep_tiles_group(const SweepArgs &a, const int 
     }
 }
 
+// ---- the float32 sweeps, in chunks of four steps (geometry, tiles and products: dag_chunks.h) ------------------------
+// What a step-by-step sweep pays per step -- barriers, LDS round trips, scales, a few hundred instructions a wave around
+// the FMAs, 2.0 us at L = 512 -- is paid here once per four steps, and the tiles below the diagonal run on the matrix cores
+// at twice the rate of DPP FMAs.  What is left on the critical path is the walk of one block through four steps
+// (48 FMAs and 20 to 40 other instructions a step, 5.5 cycles each) and two stages per block of the graph.
+//   step by step -> chunks, forward: B = 64, L = 512, T = 64 134 -> 115 us; L = 64 (T = 64) 81 -> 46; L = 256 99 -> 70;
+//   B = 16, L = 1024, T = 256 572 -> 375; B = 64, L = 512, transitions of at most 32: 136 -> 99.
+// What bounds it: a SIMD gives its cycles either to matrix instructions or to vector instructions, never to both
+// (measured: a wave of DPP FMAs beside one of v_mfma_f32_4x4x1 advances only when that has ended, whatever their
+// priorities), so that products, walks and the rest of a stage add up: 6 600 cycles a stage at L = 512.
+// A walking wave loads and converts its own match rows and writes its own results (as duties of other waves, through
+// LDS, they cost those waves more than they save it).
+template <typename TM, typename TL>
+__device__ __forceinline__ void sweep_chunks_group(const SweepArgs &a, const int b, const int slot, const int g, float *lds_raw,
+                                                   int *gstart, int *s_abort_p) {
+    const int dir = a.rev[slot];
+    const bool upper = a.upper[slot] != 0;   // rounding side, see sweep_tiles_group
+    const int tid = threadIdx.x, lane = tid & (kWave - 1);
+    const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
+    const int C = a.C;
+    int *risk = a.sync + 16 + a.ndir * a.B * C + a.B + b;
+    // (through opaque_uniform: else the compiler reads them from the argument block again in every stage, a scalar-memory
+    //  round trip each)
+    const int L = opaque_uniform(a.L), T = a.T, translen = a.translen, NBK = opaque_uniform(a.NBK);
+    const int Lb = (int)a.out_len[b], Tb = (int)a.tgt_len[b];
+    if (!lengths_ok(Lb, Tb, L, T)) {
+        if (g == 0 && tid == 0) { a.logz[slot * a.B + b] = (double)DAGX_NEG_INF; if (slot == a.loss_dir) a.loss[b] = DAGX_NEG_INF; store_agent(a.zfast + slot * a.B + b, (double)DAGX_NEG_INF); }
+        return;
+    }
+    const TM *match = static_cast<const TM *>(a.match) + (int64_t)b * a.ms0;
+    const TL *links = static_cast<const TL *>(a.links) + (int64_t)b * L * translen;
+    float *hat = a.hat[slot] + (int64_t)b * T * L;
+    double *off = a.off[slot] + (int64_t)b * T * NBK;
+    int *prog = a.sync + 16 + (slot * a.B + b) * C;
+
+    const int t_first = dir ? Tb - 1 : 0, node_first = dir ? Lb - 1 : 0;
+    const float m0 = to_float(match[(int64_t)t_first * a.ms1 + (int64_t)node_first * a.ms2]);
+    const int slack = Lb - Tb;                    // band: s <= p <= slack + s
+    const int NBb = (Lb + kBlk - 1) / kBlk;
+    const int W = (translen + kBlk - 1) / kBlk;
+    if (tid <= C) gstart[tid] = a.gtab[NBb][tid];
+    __syncthreads();
+    const int jb0 = __builtin_amdgcn_readfirstlane(gstart[g]), jb1 = __builtin_amdgcn_readfirstlane(gstart[g + 1]);
+    int last_group = 0;
+    for (int q = 0; q < C; ++q) if (gstart[q + 1] > gstart[q]) last_group = q;
+    last_group = __builtin_amdgcn_readfirstlane(last_group);
+    if (jb0 >= jb1) return;                       // nothing to do for this group (short sample); nobody waits on it
+    const int nblk = jb1 - jb0;
+    const int flo = tile_ilo(jb0, W);             // lowest foreign block this group ever reads
+    const bool producer = g < last_group, consumer = flo < jb0;
+    const ChunkLds o = chunk_lds(jb0, nblk, W);
+    int ntile = 0;
+    for (int q = 0; q < nblk; ++q) ntile += tiles_of_block(jb0 + q, W);
+    if (nblk > kChunkBlocks || ntile > kTileCap - nblk || o.total * 4 > kChunkLdsBytes) {   // cannot happen with the host's partition
+        if (tid == 0) { store_agent(risk, 1); store_agent(prog + g, 1 << 30); }
+        return;
+    }
+    const bool owner = wave < nblk;               // this wave walks block jb0 + wave
+    const int helpers = kTileWaves - nblk;
+
+    // ---- my tiles below the diagonal.  A run is a wave's tiles that lead to one block; runs are numbered in the order of
+    //      the tiles.  Worked out with lane <-> block (f: its first tile) and lane <-> wave (w_first: its first tile). ----
+    const TileDeal deal = a.deal[NBb][g];
+    int my_first, my_count;
+    wave_tiles(deal, nblk, wave, my_first, my_count);
+    int f = 0, w_first, w_count;
+#pragma unroll
+    for (int q = 0; q < kChunkBlocks; ++q) f += q < lane && q < nblk ? tiles_of_block(jb0 + q, W) : 0;
+    wave_tiles(deal, nblk, lane & (kTileWaves - 1), w_first, w_count);
+    int f_of[kChunkBlocks + 1];
+    bool cuts = lane < kTileWaves && w_count > 0;   // this wave's first tile begins a run in the middle of a block
+#pragma unroll
+    for (int q = 0; q <= kChunkBlocks; ++q) {
+        f_of[q] = __builtin_amdgcn_readlane(f, q);
+        if (q < nblk) cuts = cuts && !(w_first == f_of[q] && tiles_of_block(jb0 + q, W) > 0);
+    }
+    const bool lone = jb0 == 0;                     // (block 0 has no tiles: the runs are counted from block 1)
+    // number of runs that begin at or before tile n of block q
+    auto runs_to = [&](const int q, const int n) { return q + (lone ? 0 : 1) + (int)__builtin_popcountll(__builtin_amdgcn_ballot_w64(cuts && w_first <= n)); };
+    int t_I[kTilesPerWave], t_q[kTilesPerWave], t_run[kTilesPerWave];   // source block, own block it leads to, run it belongs to
+    bool t_ok[kTilesPerWave], t_start[kTilesPerWave], t_end[kTilesPerWave], t_lead[kTilesPerWave];   // first / last tile of its run; run that states the scale
+#pragma unroll
+    for (int u = 0; u < kTilesPerWave; ++u) {
+        const int n = my_first + u;
+        t_ok[u] = u < my_count;
+        int q = 0;
+#pragma unroll
+        for (int x = 1; x < kChunkBlocks; ++x) q = x < nblk && n >= f_of[x] ? x : q;
+        const int lo = tile_ilo(jb0 + q, W), r = n - f_of[q];
+        t_q[u] = t_ok[u] ? q : 0;
+        t_I[u] = t_ok[u] ? lo + r : flo;
+        t_start[u] = u == 0 || r == 0;
+        t_end[u] = u == my_count - 1 || lo + r == jb0 + q - 1;
+        t_lead[u] = u >= r;                       // (the run reaches back to the block's first tile)
+        t_run[u] = runs_to(q, n) - 1;
+    }
+    // the runs that lead to the block this wave walks
+    int run_first = ntile, run_count = 1;         // (block 0 receives nothing: the zeros behind the products)
+    if (owner && tiles_of_block(jb0 + wave, W) > 0) {
+        const int n = __builtin_amdgcn_readlane(f, wave);
+        run_first = runs_to(wave, n) - 1;
+        run_count = runs_to(wave, n + tiles_of_block(jb0 + wave, W) - 1) - run_first;
+    }
+    // A consumer group has nothing to do for the first stages: it lets the first group of its sweep have the memory's
+    // bandwidth for its tiles.  (Progress words: 1 + chunks published, once the group's tiles are staged.)
+    if (consumer) {
+        if (wave == 0)
+            for (int spins = 0; spins < kSpinLimit && __builtin_amdgcn_readfirstlane(load_agent(prog)) < 1; ++spins) __builtin_amdgcn_s_sleep(8);
+        __syncthreads();
+    }
+    const unsigned lds_base = (unsigned)reinterpret_cast<uintptr_t>(lds_raw);
+    float *const patch = lds_raw + wave * (kBlk * kPatchPitch);
+    const int last_index = L * translen - 1;
+    const float tiny = !upper ? 0.f : kTinyStored;
+    if (owner) { t_I[kTilesPerWave - 1] = jb0 + wave; t_q[kTilesPerWave - 1] = wave; }   // the triangle
+    auto elements = [&](const int samples) { const int64_t n = (int64_t)samples * L * translen; return n < (1 << 28) ? (int)n : 1 << 28; };
+    const int before = elements(b), behind = elements(a.B - 1 - b);
+    auto stage = [&](const int u) __attribute__((always_inline)) {
+        stage_tile<TL>(patch, links, t_I[u], jb0 + t_q[u], lane, dir, Lb, translen, last_index, before, behind, tiny);
+    };
+    Tile t0, t1, t2;
+    if (t_ok[0]) { stage(0); read_patch(t0, patch, lane, dir); }
+    if (t_ok[1]) { stage(1); read_patch(t1, patch, lane, dir); }
+    if (t_ok[2] || owner) { stage(2); read_patch(t2, patch, lane, dir); }
+    if (owner) fold_triangle(t2, lane);
+    __syncthreads();   // every wave is done with its transpose patch: the LDS now holds the buffers of the stages
+    if (producer && g == 0 && tid == 0) store_agent(prog, 1);
+
+    int *const lds_i = reinterpret_cast<int *>(lds_raw);
+    const int D = o.depth;
+    // ---- step 0: only position 0 is alive ----
+    // exp(m): fraction in [1, 2) and exponent; what no such pair holds as in the constants above, +inf and NaN as NaN
+    auto split_exp = [&](const float m, float &frac, int &exp) __attribute__((always_inline)) {
+        const float hi = m * kLog2e;
+        const float fl = __builtin_floorf(hi);
+        // (the product's rounding error and log2(e)'s own: for a match of -60 they are worth 3e-6 of the cell)
+        const float lo = __builtin_fmaf(m, kLog2e, -hi) + m * 1.925963033500e-08f;
+        float f = fast_exp2((hi - fl) + lo);
+        int n = (int)__builtin_amdgcn_fmed3f(fl, -(float)kMatchExpMax, (float)kMatchExpMax);
+        if (!(hi >= -(float)kMatchExpMax)) f = upper ? 1.f : 0.f;
+        if (m == DAGX_NEG_INF) f = 0.f;
+        if (!(hi <= (float)kMatchExpMax)) { f = __builtin_nanf(""); n = 0; }
+        frac = f; exp = n;
+    };
+    float f0; int n0;
+    split_exp(m0, f0, n0);
+    n0 = __builtin_amdgcn_readfirstlane(n0);
+    const bool alive0 = !(f0 == 0.f);     // (a NaN is on its way)
+    const int cell_at = (lane & 15) * 16 + (lane >> 4);   // + 4 * (step & 3): this lane's cell in a chunk of cells
+    for (int q = wave; q < nblk; q += kTileWaves) {
+        const int Jb = jb0 + q, p = Jb * kBlk + lane;
+        const bool here = p == 0 && alive0;
+        lds_raw[o.eb + (jb0 - flo + q) * D * 256 + cell_at] = here ? __builtin_ldexpf(f0, kShift2 - 1) : 0.f;
+        if (lane == 0) lds_i[o.kap + (jb0 - flo + q) * D * 4] = here ? n0 + 1 : kDeadExp;
+        if (p < Lb) store_agent(hat + (int64_t)t_first * L + (dir ? Lb - 1 - p : p), here ? (fast_log2(f0) - 1.f) * kLn2 : DAGX_NEG_INF);
+        if (lane == 0) store_agent(off + (int64_t)t_first * NBK + Jb, Jb == 0 && alive0 ? (double)(n0 + 1) * 0.6931471805599453 : (double)DAGX_NEG_INF);
+    }
+    if (tid < 2 * 256) lds_raw[o.part + ntile * 2 * 256 + tid] = 0.f;
+    if (jb0 == 0 && tid < 2 * kChunk) lds_i[o.part_scale + tid] = kDeadExp;
+    if (Tb == 1 && tid == 0 && jb0 == 0) {
+        const double z = (Lb == 1 && alive0) ? (double)m0 : (double)DAGX_NEG_INF;
+        a.logz[slot * a.B + b] = z; if (slot == a.loss_dir) a.loss[b] = (float)z; store_agent(a.zfast + slot * a.B + b, z);
+    }
+    const char *hat_c = reinterpret_cast<const char *>(hat);
+    const char *off_c = reinterpret_cast<const char *>(off);
+    const char *match_c = reinterpret_cast<const char *>(match);
+    const unsigned long long hat_u = uniform_address(hat), off_u = uniform_address(off);
+    const int ms1 = opaque_uniform((int)a.ms1), ms2 = opaque_uniform((int)a.ms2);   // the host checked that match indices fit 32 bits
+    const int NC = (Tb - 1 + kChunk - 1) / kChunk;  // chunks of steps 1 .. T_b-1
+    const int floor_exp = upper ? -126 : -127;      // see pow2_clamped
+    const float tiny_up = upper ? kTinyStored : 0.f;
+    // more than everything that may have been flushed on the way to a block's sum: 64 products a tile under 2^-126
+    // each, 16 tiles, as many scaled sums
+    const float flush_up = upper ? 2.4074124e-35f : 0.f;
+    auto opaque_lane = [&] { int x = tid & (kWave - 1); asm volatile("" : "+v"(x)); return x; };
+    // a block's chunks with a live cell (4c+1 .. 4c+4 meets the block's band), and its chunks as a source (4c .. 4c+3)
+    auto dest_lo = [&](const int J) { return 16 * J - 1 - (slack >> 2); };
+    auto dest_hi = [&](const int J) { return 16 * J + 15; };
+    auto src_lo = [&](const int I) { return 16 * I - ((slack + 3) >> 2); };
+
+    // ---- the foreign blocks whose table rows this wave fetches: dealt to the helpers, or to all if there is none ----
+    int f_blk[kForeign];
+#pragma unroll
+    for (int u = 0; u < kForeign; ++u) {
+        const int fb = helpers == 0 ? flo + wave + kTileWaves * u : (owner ? jb0 : flo + (wave - nblk) + helpers * u);
+        f_blk[u] = fb < jb0 ? fb : -1;
+    }
+    // Table rows of steps 4c .. 4c+3 of a foreign block (complete: 64 positions): one copy of sixteen bytes a lane for the
+    // residuals (row lane / 16, in the order of the nodes), one for the offsets.
+    auto request_rows = [&](const int I, const int c, const int lane) __attribute__((always_inline)) {
+        auto row_of = [&](const int k) { const int s = kChunk * c + k, sc = s < Tb ? s : Tb - 1; return dir ? Tb - 1 - sc : sc; };
+        const int node = (dir ? Lb - kBlk - I * kBlk : I * kBlk) + 4 * (lane & 15);
+        dma_dwordx4_agent_u(lds_base + (unsigned)(o.frows + (I - flo) * 256) * 4u, hat_u, (unsigned)(row_of(lane >> 4) * L + node) * 4u);
+        dma_dword_agent_u(lds_base + (unsigned)(o.foff + (I - flo) * 64) * 4u, off_u,
+                          (unsigned)(row_of((lane >> 1) & 3) * NBK + I) * 8u + (unsigned)(lane & 1) * 4u);
+    };
+    // ... as cells: lane 4 (i & 15) + step has the four positions 16 q + (i & 15)
+    auto convert_rows = [&](const int I, const int sl, const int lane) __attribute__((always_inline)) {
+        const int at = I - flo;
+        const float *src = lds_raw + o.frows + at * 256 + (lane & 3) * kBlk + (dir ? kBlk - 1 - (lane >> 2) : lane >> 2);
+        const int pitch = dir ? -16 : 16;
+        float x[4];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) x[q] = src[q * pitch];
+        const double v = reinterpret_cast<const double *>(lds_raw + o.foff + at * 64)[lane & (kChunk - 1)];
+        f32x4 ev;
+#pragma unroll
+        for (int q = 0; q < 4; ++q) x[q] *= kLog2e;
+        if (__builtin_amdgcn_ballot_w64(!(fminf(fminf(x[0], x[1]), fminf(x[2], x[3])) >= -115.f)) == 0) {   // (as exp2_shifted above -115)
+#pragma unroll
+            for (int q = 0; q < 4; ++q) ev[q] = __builtin_ldexpf(fast_exp2(x[q]), kShift2);
+        } else {
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const float w = exp2_shifted(x[q]);
+                ev[q] = (x[q] > -3.0e38f && w < tiny_up) ? tiny_up : w;
+            }
+        }
+        *reinterpret_cast<f32x4 *>(lds_raw + o.eb + (at * D + sl) * 256 + lane * 4) = ev;
+        const int kp = v > (double)DAGX_NEG_INF ? (int)__builtin_rint(v * 1.4426950408889634) : kDeadExp;
+        if (lane < kChunk) lds_i[o.kap + (at * D + sl) * 4 + lane] = kp;
+    };
+
+    // ---- the stages ----
+    const int first_stage = consumer ? -2 : -1, end_stage = NC - 1 + 2 * (nblk - 1);
+    const int *below = prog + (g > 0 ? g - 1 : 0);
+    // stages in which a tile's block takes part, and those in which the tile's source has a live cell
+    int t_from[kTilesPerWave], t_to[kTilesPerWave], t_src_from[kTilesPerWave], t_src_to[kTilesPerWave];
+    int t_shift[kTilesPerWave], t_cells[kTilesPerWave], t_kaps[kTilesPerWave], t_scale_at[kTilesPerWave], t_scales[kTilesPerWave];
+#pragma unroll
+    for (int u = 0; u < kTilesPerWave; ++u) {
+        const int J = jb0 + t_q[u], at = 2 * t_q[u] - 1, lo = tile_ilo(J, W);   // chunk = stage - at
+        t_from[u] = at + (dest_lo(J) > 0 ? dest_lo(J) : 0);
+        t_to[u] = t_ok[u] ? at + (dest_hi(J) < NC - 1 ? dest_hi(J) : NC - 1) : -100;
+        t_src_from[u] = at + src_lo(t_I[u]); t_src_to[u] = at + dest_hi(t_I[u]);
+        t_shift[u] = (((-at) % D) + D) % D;
+        t_cells[u] = o.eb + (t_I[u] - flo) * D * 256; t_kaps[u] = o.kap + (t_I[u] - flo) * D * 4;
+        t_scale_at[u] = o.kap + (lo - flo) * D * 4; t_scales[u] = J - lo;
+    }
+    if (NC == 0) return;
+    __syncthreads();
+
+    // One barrier a stage; a loop for each kind of wave, so that the registers hold what that kind needs.
+    auto stages = [&](auto walks, auto fetches) __attribute__((always_inline)) {
+        constexpr bool WALKS = decltype(walks)::value, FETCHES = decltype(fetches)::value;
+        // ring slots: chunk c of a block's cells is in slot c mod D (ring: the stage mod D)
+        int slot_own = 0, slot_f = 0, seen = 0, requested = -1, ring = ((first_stage % D) + D) % D;
+        auto next_slot = [&](const int x) { return x + 1 == D ? 0 : x + 1; };
+        // the walking wave's state: the last step's cells and their exponent; the next chunk's match rows as loaded, then
+        // exp(match) relative to the rows' exponents N
+        const int J = jb0 + wave, first = J * kBlk, own_src = jb0 - flo + wave;
+        float e = 0.f;
+        int kap = kDeadExp, N[kChunk] = {0, 0, 0, 0};
+        float mt[kChunk] = {0.f, 0.f, 0.f, 0.f};
+        TM raw[kChunk];
+        if (WALKS && J == 0) {
+            if (lane == 0 && alive0) e = __builtin_ldexpf(f0, kShift2 - 1);
+            kap = alive0 ? n0 + 1 : kDeadExp;
+        }
+        auto load_match = [&](const int c, const int lane) __attribute__((always_inline)) {
+            const int p = first + lane, pc = p < Lb ? p : Lb - 1, s0 = kChunk * c + 1;
+            const unsigned lane_off = (unsigned)((dir ? Lb - 1 - pc : pc) * ms2) * (unsigned)sizeof(TM);
+            const char *row = match_c + (unsigned)((dir ? Tb - 1 - s0 : s0) * ms1) * (unsigned)sizeof(TM);
+            const int step = (dir ? -ms1 : ms1) * (int)sizeof(TM);
+#pragma unroll
+            for (int k = 0; k < kChunk; ++k) {
+                raw[k] = *reinterpret_cast<const TM *>(row + lane_off);
+                if (s0 + k + 1 < Tb) row += step;      // (rows past the last step: the last one again)
+            }
+        };
+        auto convert_match = [&](const int c, const int lane) __attribute__((always_inline)) {
+            const int s0 = kChunk * c + 1;
+            float m[kChunk], top[kChunk];
+#pragma unroll
+            for (int k = 0; k < kChunk; ++k) m[k] = to_float(raw[k]);
+            // in the band: s <= p <= slack + s (mostly the whole block, in all four steps)
+            if (!(first >= s0 + kChunk - 1 && first + kBlk - 1 <= slack + s0 && s0 + kChunk <= Tb)) {
+                const int d0 = first + lane - s0;
+#pragma unroll
+                for (int k = 0; k < kChunk; ++k)
+                    m[k] = (unsigned)(d0 - k) < (s0 + k < Tb ? (unsigned)slack + 1u : 0u) ? m[k] : DAGX_NEG_INF;
+            }
+#pragma unroll
+            for (int k = 0; k < kChunk; ++k) top[k] = m[k];
+            wave64_max4(top);
+            float log2e = kLog2e;
+            asm("" : "+v"(log2e));                    // (an instruction takes one scalar register: N)
+#pragma unroll
+            for (int k = 0; k < kChunk; ++k) {
+                // relative to the row's exponent: its largest cell becomes a number in (1/2, 1]
+                const float n = __builtin_amdgcn_fmed3f(__builtin_ceilf(top[k] * kLog2e), -(float)kMatchExpMax, (float)kMatchExpMax);
+                N[k] = __builtin_amdgcn_readlane((int)n, 63);
+                mt[k] = __builtin_fmaf(m[k], log2e, -lane_bcast(n, 63));
+            }
+            if (__builtin_amdgcn_ballot_w64(!(fminf(fminf(mt[0], mt[1]), fminf(mt[2], mt[3])) >= -126.f)) != 0 && upper) {
+#pragma unroll
+                for (int k = 0; k < kChunk; ++k) mt[k] = m[k] > DAGX_NEG_INF && mt[k] < -126.f ? -126.f : mt[k];
+            }
+#pragma unroll
+            for (int k = 0; k < kChunk; ++k) mt[k] = fast_exp2(mt[k]);
+        };
+        // the chunk just walked (cells v, exponents kk) into the tables
+        auto write_out = [&](const int c, const float (&v)[kChunk], const int (&kk)[kChunk], const int lane) __attribute__((always_inline)) {
+            const int s0 = kChunk * c + 1, row0 = dir ? Tb - 1 - s0 : s0;
+            float res[kChunk], lf[kChunk];
+            int ex[kChunk];
+#pragma unroll
+            for (int k = 0; k < kChunk; ++k) {   // (a dead cell: log of the fraction 0)
+                ex[k] = __builtin_amdgcn_frexp_expf(v[k]) - kShift2;
+                lf[k] = fast_log2(__builtin_amdgcn_frexp_mantf(v[k]));
+                res[k] = ((float)ex[k] + lf[k]) * kLn2;
+            }
+            const unsigned lane_off = (unsigned)(dir ? Lb - 1 - first - lane : first + lane) * 4u;
+            char *row = const_cast<char *>(hat_c) + (unsigned)(row0 * L) * 4u;
+            const int step = (dir ? -L : L) * 4;
+            auto put = [&](const int k) __attribute__((always_inline)) {
+                store_agent(reinterpret_cast<float *>(row + lane_off), res[k]);
+                row += step;
+            };
+            const int steps = Tb - s0 < kChunk ? Tb - s0 : kChunk;
+            if (__builtin_expect(steps == kChunk && first + kBlk <= Lb, 1)) { put(0); put(1); put(2); put(3); }
+            else if (first + lane < Lb) { put(0); if (steps > 1) put(1); if (steps > 2) put(2); if (steps > 3) put(3); }
+            const int k01 = lane & 1 ? kk[1] : kk[0], k23 = lane & 1 ? kk[3] : kk[2], kp = lane & 2 ? k23 : k01;
+            if (lane < steps)
+                store_agent(reinterpret_cast<double *>(const_cast<char *>(off_c) + (unsigned)((dir ? row0 - lane : row0 + lane) * NBK + J) * 8u),
+                            kp > kDeadBelow ? (double)kp * 0.6931471805599453 : (double)DAGX_NEG_INF);
+            if (__builtin_expect(c == NC - 1 && J == NBb - 1, 0)) {   // the read-out
+#pragma unroll
+                for (int k = 0; k < kChunk; ++k)
+                    if (k == steps - 1 && first + lane == Lb - 1) {
+                        const double z = kk[k] > kDeadBelow ? ((double)(ex[k] + kk[k]) + (double)lf[k]) * 0.6931471805599453 : (double)DAGX_NEG_INF;
+                        a.logz[slot * a.B + b] = z; if (slot == a.loss_dir) a.loss[b] = (float)z; store_agent(a.zfast + slot * a.B + b, z);
+                    }
+            }
+            return kp;
+        };
+        for (int tau = first_stage; tau <= end_stage; ++tau) {
+            const int par = tau & 1;
+            // (per-lane addresses are formed anew in every stage: held across the loop they would cost the tiles their registers)
+            const int lane = opaque_lane(), cell_at = (lane & 15) * 16 + (lane >> 4);
+            const int cf = tau + 2;                             // the foreign chunk this stage brings in
+            const bool bring = FETCHES && f_blk[0] >= 0 && cf < NC;
+            int published = 0;
+            if (bring) published = load_agent(below);
+            // ---------------- walk my block through chunk tau - 2 wave ----------------
+            if (WALKS) {
+                const int c = tau - 2 * wave;
+                const bool more = c >= -1 && c + 1 < NC;
+                if (more) load_match(c + 1, lane);
+                if (c >= 0 && c < NC) {
+                    float *const cells = lds_raw + o.eb + own_src * D * 256 + cell_at;
+                    float *const cells_next = cells + next_slot(slot_own) * 256;
+                    float *const cells_this = cells + slot_own * 256;
+                    int kk[kChunk];
+                    float v[kChunk];
+                    if (c >= dest_lo(J) && c <= dest_hi(J)) {
+                        __builtin_amdgcn_s_setprio(3);
+                        const i32x4 sc = *reinterpret_cast<const i32x4 *>(lds_i + o.part_scale + (wave * 2 + (par ^ 1)) * 4);
+                        const float *const parts = lds_raw + o.part + (run_first * 2 + (par ^ 1)) * 256 + lane * 4;
+                        const float upper_half = lane >= 32 ? 1.f : 0.f;
+                        f32x4 G = *reinterpret_cast<const f32x4 *>(parts);
+                        if (run_count > 1) {
+                            f32x4 G1 = *reinterpret_cast<const f32x4 *>(parts + 512);
+                            if (run_count > 2) {
+                                G += *reinterpret_cast<const f32x4 *>(parts + 1024);
+#pragma unroll 1
+                                for (int u = 3; u < run_count; ++u) G += *reinterpret_cast<const f32x4 *>(parts + u * 512);
+                            }
+                            G += G1;
+                        }
+                        int R[kChunk];
+#pragma unroll
+                        for (int k = 0; k < kChunk; ++k) R[k] = __builtin_amdgcn_readfirstlane(sc[k]);
+#pragma unroll
+                        for (int k = 0; k < kChunk; ++k) {
+                            // (kSpare: every other step does not scale its cells by their largest)
+                            const int ref = (kap > R[k] ? kap : R[k]) + (k & 1 ? 0 : kSpare);
+                            // (what ldexp flushes of either part is under flush_up, too)
+                            const float x = (__builtin_ldexpf(triangle_dot(t2, e, upper_half), kap - ref) + flush_up) + __builtin_ldexpf(G[k], R[k] - ref);
+                            // (upper sweep: a cell never flushes, live or not -- what a dead one gets is of the size of what is flushed)
+                            if (k & 1) {
+                                const float y = x * mt[k];
+                                // the exponent of the largest cell, at least that of 2^-72: its reciprocal has to be a float32 number
+                                const unsigned top = wave64_max_positive(y);
+                                const int tb = (int)(top >> 23) > 55 ? (int)(top >> 23) : 55;
+                                kap = top ? tb + ref + N[k] - (126 + 2 * kShift2) : kDeadExp;
+                                e = __builtin_fmaf(y, __builtin_bit_cast(float, (unsigned)(253 + kShift2 - tb) << 23), tiny_up);
+                            } else {   // at most 2^57, and mostly 15 to 45 binades lower
+                                kap = ref + N[k] - kShift2;
+                                e = __builtin_fmaf(x, mt[k], tiny_up);
+                            }
+                            kk[k] = kap;
+                            v[k] = e;
+                            if (k < kChunk - 1) cells_this[4 * (k + 1)] = e; else cells_next[0] = e;
+                        }
+                        __builtin_amdgcn_s_setprio(0);
+                    } else {
+                        e = 0.f; kap = kDeadExp;
+#pragma unroll
+                        for (int k = 0; k < kChunk; ++k) {
+                            kk[k] = kDeadExp;
+                            v[k] = 0.f;
+                            if (k < kChunk - 1) cells_this[4 * (k + 1)] = 0.f; else cells_next[0] = 0.f;
+                        }
+                    }
+                    if (more) convert_match(c + 1, lane);   // (in front of the stores: what it waits for is older than they)
+                    else wait_vmem_all();
+                    // Either wait covers what this wave stored in the last stage.  The other blocks are two chunks and more
+                    // ahead of the last one: when its wave has come here, every block's chunk c - 1 is in memory.
+                    if (producer && wave == nblk - 1 && c > 0 && lane == 0) store_agent(prog + g, 1 + c);
+                    const int kp = write_out(c, v, kk, lane);
+                    const int sl = (lane & 3) < kChunk - 1 ? slot_own * 4 + 1 + (lane & 3) : next_slot(slot_own) * 4;
+                    if (lane < kChunk) lds_i[o.kap + own_src * D * 4 + sl] = kp;
+                    slot_own = next_slot(slot_own);
+                }
+                else if (more) convert_match(c + 1, lane);
+            }
+            // ---------------- multiply out what chunk tau + 1 - 2 q of my tiles' blocks receives ----------------
+            if (my_count > 0) {
+                // (the LDS reads of two tiles are requested before the first is waited for, the third's behind the first)
+                f32x4 ev[2];
+                int kv[kTilesPerWave], rv[kTilesPerWave];
+                bool go[kTilesPerWave], src[kTilesPerWave];
+#pragma unroll
+                for (int u = 0; u < (WALKS ? kTilesPerWave - 1 : kTilesPerWave); ++u) {
+                    go[u] = tau >= t_from[u] && tau <= t_to[u];
+                    src[u] = tau >= t_src_from[u] && tau <= t_src_to[u];
+                    if (go[u]) {
+                        int sl = ring + t_shift[u]; sl -= sl >= D ? D : 0;
+                        if (u < 2) ev[u] = *reinterpret_cast<const f32x4 *>(lds_raw + t_cells[u] + sl * 256 + lane * 4);
+                        kv[u] = lds_i[t_kaps[u] + sl * 4 + (lane & 3)];
+                        if (t_start[u]) {
+                            const int n = (lane >> 2) < t_scales[u] ? lane >> 2 : 0;
+                            rv[u] = lds_i[t_scale_at[u] + sl * 4 + n * (D * 4) + (lane & 3)];
+                        }
+                    }
+                }
+                f32x4 G = {0.f, 0.f, 0.f, 0.f};
+                int R = kDeadExp;
+                auto product = [&](const int u, const Tile &t) __attribute__((always_inline)) {
+                    if (!go[u]) return;
+                    if (t_start[u]) {   // the scale: the largest exponent, step by step, among all blocks that lead here
+                        R = by_step_max(rv[u]);
+                        G = f32x4{0.f, 0.f, 0.f, 0.f};
+                    }
+                    if (src[u]) {
+                        const f32x4 v = tile_product(t, ev[u & 1]);
+                        scaled4<false>(G, pow2_clamped(kv[u] - R, floor_exp), v);
+                    }
+                    if (t_end[u]) {
+                        *reinterpret_cast<f32x4 *>(lds_raw + o.part + (t_run[u] * 2 + par) * 256 + lane * 4) = G;
+                        if (t_lead[u] && lane < 4) lds_i[o.part_scale + (t_q[u] * 2 + par) * 4 + lane] = R;
+                    }
+                };
+                product(0, t0);
+                if (!WALKS && go[2]) {
+                    int sl = ring + t_shift[2]; sl -= sl >= D ? D : 0;
+                    ev[0] = *reinterpret_cast<const f32x4 *>(lds_raw + t_cells[2] + sl * 256 + lane * 4);
+                }
+                product(1, t1);
+                if (!WALKS) product(2, t2);
+            }
+            // ---------------- table rows of foreign blocks: requested a stage ago if they were published by then ----------------
+            if (bring) {
+                published = __builtin_amdgcn_readfirstlane(published);
+                if (published > seen) seen = published;
+                auto request = [&](const int c) __attribute__((always_inline)) {
+#pragma unroll
+                    for (int u = 0; u < kForeign; ++u) { if (f_blk[u] < 0) break; request_rows(f_blk[u], c, lane); }
+                    requested = c;
+                };
+                if (requested < cf) {
+                    int spins = 0;
+                    while (seen <= cf + 1) {                    // (the word is 1 + chunks published)
+                        __builtin_amdgcn_s_sleep(1);
+                        seen = __builtin_amdgcn_readfirstlane(load_agent(below));
+                        if (++spins > kSpinLimit) { *s_abort_p = 1; break; }
+                    }
+                    if (seen > cf + 1) request(cf);
+                }
+                wait_vmem_all();
+#pragma unroll
+                for (int u = 0; u < kForeign; ++u) { if (f_blk[u] < 0) break; convert_rows(f_blk[u], slot_f, lane); }
+                slot_f = next_slot(slot_f);
+                if (cf + 1 < NC && seen > cf + 2) request(cf + 1);
+            }
+            ring = next_slot(ring);
+            __syncthreads();
+            if (consumer && __builtin_amdgcn_readfirstlane(*s_abort_p)) return;
+        }
+    };
+    if (owner && helpers == 0) stages(std::true_type{}, std::true_type{});
+    else if (owner) stages(std::true_type{}, std::false_type{});
+    else stages(std::false_type{}, std::true_type{});
+    if (producer) {
+        wait_vmem_all();
+        __syncthreads();
+        if (tid == 0) store_agent(prog + g, 1 + NC);
+    }
+    if (consumer && __builtin_amdgcn_readfirstlane(*s_abort_p)) {   // a producer never showed up: hand the sample on and let consumers go on
+        wait_vmem_all();
+        if (tid == 0) { store_agent(risk, 1); store_agent(prog + g, 1 << 30); }
+    }
+}
+
 // The two read-outs of a sample's tile sweeps bracket log Z: one sweep rounds everything the linear domain
 // cannot hold down to 0, the other up to the smallest number it holds.  Where they agree, what was flushed carried
 // no mass that matters and either read-out is log Z to the tolerance; where they do not (or one is not finite,
@@ -1048,7 +1499,7 @@ __device__ __forceinline__ void sweep_tiles_group(const SweepArgs &a, const int 
 // the path that carries the mass lies as deep.)
 __device__ __forceinline__ bool readouts_disagree(double za, double zb, bool wide) {
     if (!(za > (double)DAGX_NEG_INF) || !(zb > (double)DAGX_NEG_INF) || za != za || zb != zb) return true;
-    return fabs(za - zb) > (wide ? 1e-8 * fabs(zb) + 5e-5 : fmin(1e-7 * fabs(zb) + 5e-5, 1e-4));
+    return !(fabs(za - zb) <= (wide ? 1e-8 * fabs(zb) + 5e-5 : fmin(1e-7 * fabs(zb) + 5e-5, 1e-4)));
 }
 
 template <typename TM, typename TL, bool WIDE>
@@ -1078,7 +1529,10 @@ __global__ __launch_bounds__(kTileWaves * kWave) void dag_sweep_tiles_kernel(Swe
     // a launch for flagged samples only (the wide variant behind the float32 one): the workgroups of the others
     // leave at once, through the same bookkeeping
     const bool skip = has_sample && a.only_flagged && a.flags[b] != 1;
-    if (has_sample && !skip) sweep_tiles_group<TM, TL, WIDE>(a, b, slot, g, lds_raw, gstart, &s_abort);
+    if (has_sample && !skip) {
+        if constexpr (WIDE) sweep_tiles_group<TM, TL>(a, b, slot, g, lds_raw, gstart, &s_abort);
+        else sweep_chunks_group<TM, TL>(a, b, slot, g, lds_raw, gstart, &s_abort);
+    }
     // ---- leaving ----
     wait_vmem_all();   // this wave's stores (table rows, read-outs) are complete
     __syncthreads();
@@ -1711,7 +2165,7 @@ static size_t sweep_sync_ints(int B, int C) { return ((16 + (size_t)2 * B * C + 
 
 size_t loss_fwd_workspace_bytes(int B, int T, int L, int translen) {
     (void)T;
-    int C = groups_used(2 * ((B + 7) & ~7), L, translen, false);
+    int C = groups_used(2 * ((B + 7) & ~7), L, translen, false, kChunkBlocks);
     // ticket + progress words (rounded to 8 bytes), then the fast kernel's two read-outs per sample
     return C > 0 ? sweep_sync_ints(B, C) * sizeof(int) + (size_t)2 * B * sizeof(double) : 0;
 }
@@ -1723,7 +2177,8 @@ size_t loss_bwd_workspace_bytes(int B) { (void)B; return 0; }
 // dagx_prepare_device does it for every instantiation ahead of time).
 constexpr size_t kPatchBytes = (size_t)kTileWaves * kBlk * (kBlk + 1) * sizeof(float);
 template <bool WIDE> constexpr size_t tiles_lds_bytes() {
-    return kPatchBytes > (size_t)StepLds<WIDE>::kStepFloats * sizeof(float) ? kPatchBytes : (size_t)StepLds<WIDE>::kStepFloats * sizeof(float);
+    if (!WIDE) return kChunkLdsBytes;
+    return kPatchBytes > (size_t)StepLds::kStepFloats * sizeof(float) ? kPatchBytes : (size_t)StepLds::kStepFloats * sizeof(float);
 }
 template <typename TM, typename TL, bool WIDE>
 static int prepare_tiles_kernel() {
@@ -1751,10 +2206,11 @@ static int prepare_tiles_kernels_of() {
 
 template <typename TM, typename TL>
 static int launch_sweeps(SweepArgs a, hipStream_t st) {
-    int C = force_exact() ? 0 : groups_used(2 * ((a.B + 7) & ~7), a.L, a.translen, false);
+    int C = force_exact() ? 0 : groups_used(2 * ((a.B + 7) & ~7), a.L, a.translen, false, kChunkBlocks);
     // the tile kernel indexes match with 32-bit arithmetic
     const int64_t span = (int64_t)(a.T - 1) * (a.ms1 < 0 ? -a.ms1 : a.ms1) + (int64_t)(a.L - 1) * (a.ms2 < 0 ? -a.ms2 : a.ms2);
     if (span >= (1LL << 31) / (int64_t)sizeof(TM) || a.ms1 < 0 || a.ms2 < 0) C = 0;
+    if ((int64_t)a.B * a.L * a.translen < 4) C = 0;   // (the tiles are loaded four elements at a time)
     int rc;
     if (C == 0) {   // every sample goes to the log-domain kernel
         hipLaunchKernelGGL(dag_fill_int_kernel, dim3((a.B + 255) / 256), dim3(256), 0, st, a.flags, a.B, 1);
@@ -1770,12 +2226,25 @@ static int launch_sweeps(SweepArgs a, hipStream_t st) {
         a.rev[0] = 0; a.rev[1] = a.loss_dir ? 1 : 0;
         a.upper[0] = a.loss_dir ? 1 : 0; a.upper[1] = a.loss_dir ? 0 : 1;
         a.C = C;
-        {
+        {   // how the blocks of a sample are grouped and their tiles dealt, by its number of blocks; remembered for the next call
+            struct Grouping { int W = 0, C = 0, NB = 0; unsigned char gtab[kMaxBlocksFast + 1][12]; TileDeal deal[kMaxBlocksFast + 1][12]; };
+            static thread_local Grouping last;
             const int W = (a.translen + kBlk - 1) / kBlk;
-            int tmp[kTileCap + 2];
-            for (int nb = 0; nb <= kMaxBlocksFast; ++nb) {
-                partition_blocks(nb, W, C, tmp);
-                for (int q = 0; q <= C && q < 12; ++q) a.gtab[nb][q] = (unsigned char)tmp[q];
+            if (last.W != W || last.C != C || last.NB < a.NBK) {
+                int tmp[kTileCap + 2];
+                for (int nb = 0; nb <= a.NBK; ++nb) {
+                    partition_chunk_groups(nb, W, C, tmp);
+                    for (int q = 0; q <= C && q < 12; ++q) last.gtab[nb][q] = (unsigned char)tmp[q];
+                    for (int q = 0; q < C; ++q) {
+                        int ntile = 0;
+                        for (int Jb = tmp[q]; Jb < tmp[q + 1]; ++Jb) ntile += tiles_of_block(Jb, W);
+                        if (tmp[q] < tmp[q + 1]) last.deal[nb][q] = deal_tiles(ntile, tmp[q + 1] - tmp[q], tmp[q] - tile_ilo(tmp[q], W));
+                    }
+                }
+                last.W = W; last.C = C; last.NB = a.NBK;
+            }
+            for (int nb = 0; nb <= a.NBK; ++nb) {
+                for (int q = 0; q < 12; ++q) { a.gtab[nb][q] = last.gtab[nb][q]; a.deal[nb][q] = last.deal[nb][q]; }
             }
         }
         const int B8 = (a.B + 7) & ~7;

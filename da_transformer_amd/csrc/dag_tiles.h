@@ -9,7 +9,7 @@ namespace dagx {
 
 constexpr int kBlk = 64;            // positions per block
 constexpr int kMaxBlocksFast = 16;  // fast path: L <= 1024
-constexpr int kTileWaves = 8;       // waves per workgroup in the fast sweep
+constexpr int kTileWaves = 8;       // waves per workgroup in the tile sweeps
 constexpr int kTilesPerWave = 3;    // register-resident tiles per wave
 constexpr int kTileCap = kTileWaves * kTilesPerWave;
 // Linear-domain numbers of the fast sweep carry a constant factor 2^kShift2 each (transition probabilities
@@ -73,29 +73,6 @@ __device__ __forceinline__ void mul16_rowbcast(float &acc, float e, const float 
           "v"(p[8]), "v"(p[9]), "v"(p[10]), "v"(p[11]), "v"(p[12]), "v"(p[13]), "v"(p[14]), "v"(p[15]));
 }
 
-// acc (+)= sum_{u<4} f[lane U0+u of this lane's 16-lane row] * v[u]: four values per lane, each scaled by a factor
-// that sits in one lane of a 16-replicated vector.  U0 = 0 starts the sum with a multiply.  (Four at a time: with
-// eight operands per statement the register allocator had to evict tile registers around it.)
-template <int U0>
-__device__ __forceinline__ void scaled_sum4(float &acc, float f, float v0, float v1, float v2, float v3) {
-    static_assert(U0 % 4 == 0 && U0 >= 0 && U0 < 16, "");
-    if constexpr (U0 == 0) {
-        asm("s_nop 1\n\t"
-            "v_mul_f32_dpp %0, %1, %2 row_newbcast:0 row_mask:0xf bank_mask:0xf\n\t"
-            "v_fmac_f32_dpp %0, %1, %3 row_newbcast:1 row_mask:0xf bank_mask:0xf\n\t"
-            "v_fmac_f32_dpp %0, %1, %4 row_newbcast:2 row_mask:0xf bank_mask:0xf\n\t"
-            "v_fmac_f32_dpp %0, %1, %5 row_newbcast:3 row_mask:0xf bank_mask:0xf"
-            : "=&v"(acc) : "v"(f), "v"(v0), "v"(v1), "v"(v2), "v"(v3));
-    } else {
-        asm("s_nop 1\n\t"
-            "v_fmac_f32_dpp %0, %1, %2 row_newbcast:%c6 row_mask:0xf bank_mask:0xf\n\t"
-            "v_fmac_f32_dpp %0, %1, %3 row_newbcast:%c7 row_mask:0xf bank_mask:0xf\n\t"
-            "v_fmac_f32_dpp %0, %1, %4 row_newbcast:%c8 row_mask:0xf bank_mask:0xf\n\t"
-            "v_fmac_f32_dpp %0, %1, %5 row_newbcast:%c9 row_mask:0xf bank_mask:0xf"
-            : "+v"(acc) : "v"(f), "v"(v0), "v"(v1), "v"(v2), "v"(v3), "n"(U0), "n"(U0 + 1), "n"(U0 + 2), "n"(U0 + 3));
-    }
-}
-
 // Number of tiles of position block Jb: predecessor blocks I in [ilo, Jb]; W = blocks a transition can span.
 __device__ __host__ __forceinline__ int tile_ilo(int Jb, int W) { return Jb > W ? Jb - W : 0; }
 
@@ -126,29 +103,28 @@ __device__ __host__ inline int partition_blocks(int NBb, int W, int C, int *gsta
 }
 
 // Host: workgroups per sweep needed for graph size L (0 = the fast path does not apply).
-inline int groups_needed(int L, int translen) {
+inline int groups_needed(int L, int translen, int most = kMaxBlocksFast) {
     const int NB = (L + kBlk - 1) / kBlk;
     if (NB > kMaxBlocksFast) return 0;
     const int W = (translen + kBlk - 1) / kBlk;
-    int groups = 1, sum = 0;
+    int groups = 1, sum = 0, blocks = 0;
     for (int Jb = 0; Jb < NB; ++Jb) {
         int c = Jb - tile_ilo(Jb, W) + 1;
         if (c > kTileCap) return 0;
-        if (sum + c > kTileCap) { ++groups; sum = 0; }
-        sum += c;
+        if (sum + c > kTileCap || blocks == most) { ++groups; sum = blocks = 0; }
+        sum += c; ++blocks;
     }
     return groups <= 11 ? groups : 0;
 }
 
-// Host: workgroups per sweep actually launched.  More groups than needed mean fewer tiles per SIMD but a
-// hand-over between groups in every step and a deeper pipeline.  Measured on MI355X (B = 16..64, T = 64):
-// the loss sweeps (two per sample, a heavier owner phase) are fastest with the minimal number at every
-// graph size but 384 (there 6 % slower than with twice as many; at 128 and 256 nodes 20-26 % faster); the
+// Host: workgroups per sweep actually launched (`most`: blocks a group may own).  More groups than needed mean fewer
+// tiles per SIMD but a hand-over between groups in every step and a deeper pipeline.  Measured on MI355X (B = 16..64,
+// T = 64): the loss sweeps (two per sample) take the minimal number; the
 // alignment sweep gains 5-13 % from doubling the groups once when the graph has at least 4 blocks and the
 // device has room (one workgroup per CU), and loses from doubling twice; where twice the minimal number
 // exceeds the 11 the kernel supports (L > 704), 10 groups are used when they fit.
-inline int groups_used(int sweeps, int L, int translen, bool may_double) {
-    int C = groups_needed(L, translen);
+inline int groups_used(int sweeps, int L, int translen, bool may_double, int most = kMaxBlocksFast) {
+    int C = groups_needed(L, translen, most);
     if (C == 0) return 0;
     const int NB = (L + kBlk - 1) / kBlk;
     if (may_double) {
@@ -262,6 +238,10 @@ __device__ __forceinline__ void dma_dword_u(unsigned lds_byte, unsigned long lon
 __device__ __forceinline__ void dma_dword_agent_u(unsigned lds_byte, unsigned long long ubase, unsigned voff) {
     asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dword %0, %1 sc1" :: "v"(voff), "s"(ubase), "s"(lds_byte) : "memory", "m0");
 }
+// sixteen bytes a lane, to lds_byte + 16 * lane (the global address at least 4-byte aligned)
+__device__ __forceinline__ void dma_dwordx4_agent_u(unsigned lds_byte, unsigned long long ubase, unsigned voff) {
+    asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1 sc1" :: "v"(voff), "s"(ubase), "s"(lds_byte) : "memory", "m0");
+}
 __device__ __forceinline__ void dma_ushort_u(unsigned lds_byte, unsigned long long ubase, unsigned voff) {
     asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_ushort %0, %1" :: "v"(voff), "s"(ubase), "s"(lds_byte) : "memory", "m0");
 }
@@ -303,9 +283,8 @@ __device__ __forceinline__ void wait_vmem_but(int pending) {
 //    row apart.  The wave therefore reads row by row (lanes <-> r, coalesced) and transposes
 //    through a private LDS patch.
 // Loads are unconditional (clamped to element 0) so that all 64 of a tile can be in flight.
-// 2^(x + kShift2) and log2(y) - 2 * kShift2 with the rounding errors of the unshifted functions: the shift goes
-// through the exponent field (ldexp / frexp), not through the argument of v_exp_f32 or the result of
-// v_log_f32, where adding 56 would cost five bits of the fraction.
+// 2^(x + kShift2) with the rounding errors of the unshifted function: the shift goes through the exponent field
+// (ldexp), not through the argument of v_exp_f32, where adding 56 would cost five bits of the fraction.
 __device__ __forceinline__ float exp2_shifted(float x) {
     // (arguments below -115, results under 2^-59, take the shift inside the argument instead: v_exp_f32 alone
     //  would flush them, and their rounding no longer matters)
@@ -329,10 +308,6 @@ __device__ __forceinline__ float exp2_shifted_by(float x) {
     return __builtin_ldexpf(r, deep ? -24 : SHIFT);
 }
 template <int SHIFT> __device__ __forceinline__ constexpr float min_logp() { return SHIFT == kShift2 ? kMinLogP : kMinLogPWide; }
-__device__ __forceinline__ float log2_unshifted(float y) {   // y > 0
-    return (float)(__builtin_amdgcn_frexp_expf(y) - 2 * kShift2) + fast_log2(__builtin_amdgcn_frexp_mantf(y));
-}
-
 // `tiny`: what a finite transition too small for the linear domain becomes -- 0 in a sweep that must never
 // overstate (a lower bound of every sum), kTinyStored in one that must never understate (an upper bound).
 template <bool EXP, int SHIFT>
