@@ -174,7 +174,7 @@ __device__ __forceinline__ float tile_maxplus(const Tile &t, float a0, float a1,
 // bytes per row of the source-block table (rows padded to 16 bytes)
 __host__ __device__ static inline int srcblk_pitch(int L) { return (L + 15) & ~15; }
 
-static int align_groups(int B, int L, int translen) { return groups_used((B + 7) & ~7, L, translen, true); }
+static int align_groups(int B, int L, int translen) { return groups_used((B + 7) & ~7, L, translen); }
 
 struct AlignTileArgs {
     const void *match; int64_t ms0, ms1, ms2;

@@ -7,9 +7,10 @@
 
 namespace dagx {
 
-// Position block J works on chunk c (steps 4c+1 .. 4c+4) in stage 2J + c: everything it receives from the blocks
-// below it, which worked on that chunk at least two stages earlier, is multiplied out one stage ahead, by waves that
-// are not on the critical path, and one barrier a stage is the only synchronisation of a workgroup.
+// Position block J works on chunk c (steps 4c+1 .. 4c+4) in stage J + c, and one barrier a stage is the only synchronisation
+// of a workgroup.  What it receives from block J - 1, which worked on that chunk one stage earlier, the walking wave itself
+// multiplies out when the stage begins; what it receives from the blocks below that one is multiplied out one stage
+// ahead, by waves that are not on the critical path.
 //
 // Numbers are linear: a cell holds exp(value - kap ln 2) 2^kShift2 with one integer exponent kap per block and step,
 // chosen so that the block's largest cell lies in [2^(kShift2-1), 2^kShift2).  All scaling is by powers of two.
@@ -24,33 +25,12 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef int i32x4 __attribute__((ext_vector_type(4)));
 typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
 
-// Contiguous grouping of the position blocks [0, NBb) into at most C groups of at most kTileCap tiles (the diagonal
-// ones among them) and kChunkBlocks blocks, minimising the work of the busiest: walking and writing out a block costs
-// a workgroup about seven times what a tile costs it.  gstart[g] .. gstart[g+1]: blocks of group g (empty groups last).
-inline int partition_chunk_groups(int NBb, int W, int C, int *gstart) {
-    constexpr int kWalkCost = 7;
-    for (int cap = 1; ; ++cap) {
-        int groups = 1, tiles = 0, blocks = 0;
-        gstart[0] = 0;
-        const bool any = cap > kTileCap + kWalkCost * kChunkBlocks;   // (the work no longer bounds anything)
-        for (int Jb = 0; Jb < NBb; ++Jb) {
-            const int c = Jb - tile_ilo(Jb, W) + 1;
-            if (blocks > 0 && (tiles + c > kTileCap || blocks == kChunkBlocks || (!any && tiles + c + (blocks + 1) * (kWalkCost - 1) > cap))) {
-                if (groups < C) gstart[groups] = Jb;
-                ++groups; tiles = blocks = 0;
-            }
-            tiles += c; ++blocks;
-        }
-        if (groups <= C || any) {
-            for (int q = groups; q <= C; ++q) gstart[q] = NBb;
-            return groups;
-        }
-    }
-}
+// Tiles that are multiplied out a stage ahead: those below the diagonal but for the one next to it.
+__device__ __host__ __forceinline__ int tiles_of_block(int J, int W) { const int n = J < W ? J : W; return n > 1 ? n - 1 : 0; }
 
 // LDS of a group, in dwords.
 struct ChunkLds {
-    int depth;      // chunks of cells kept per block: read up to 2 (blocks of the group) stages after they are written
+    int depth;      // chunks of cells kept per block: read up to (blocks of the group) stages after they are written
     int eb;         // [nsrc][depth][256]  cells of four steps: (4 (i & 15) + (s & 3)) 4 + i / 16
     int kap;        // [nsrc][depth][4]    their exponents
     int part;       // [ntile + 1][2][256] products of a run of tiles, four steps per lane; behind them zeros
@@ -62,9 +42,9 @@ __device__ __host__ inline ChunkLds chunk_lds(int jb0, int nblk, int W) {
     ChunkLds o;
     const int flo = tile_ilo(jb0, W), nfor = jb0 - flo, nsrc = nfor + nblk;
     int ntile = 0;
-    for (int q = 0; q < nblk; ++q) ntile += jb0 + q < W ? jb0 + q : W;
-    const int reach = nblk < W + 1 ? nblk : W + 1;
-    o.depth = 2 * reach < 3 ? 3 : 2 * reach;
+    for (int q = 0; q < nblk; ++q) ntile += tiles_of_block(jb0 + q, W);
+    const int reach = nblk < W ? nblk : W;
+    o.depth = reach + 1 < 3 ? 3 : reach + 1;
     int at = 0;
     o.eb = at; at += nsrc * o.depth * 256;
     o.part = at; at += (ntile + 1) * 2 * 256;
@@ -78,33 +58,96 @@ __device__ __host__ inline ChunkLds chunk_lds(int jb0, int nblk, int W) {
 constexpr int kForeign = 3;                  // foreign blocks a wave fetches at most
 constexpr int kChunkLdsBytes = 160 * 1024 - 512;
 
-// The tiles below the diagonal, block by block, dealt to the waves in runs: at most three to a wave that walks no block (a
-// helper), at most two to one that does (the triangle takes a third tile's registers).  What a wave does in a stage, in
-// hundreds of cycles (measured): walking 38, a tile 7, fetching a foreign block 4.  Helpers fetch, too; the walking waves take so many tiles that the busiest wave has least to do.
-struct TileDeal { unsigned char base_h, rem_h, base_o, rem_o; };    // tiles per helper and odd ones, tiles per walking wave and odd ones
-inline TileDeal deal_tiles(int ntile, int nblk, int nfor) {          // (on the host: its divisions cost the kernel 2 us)
-    const int helpers = kTileWaves - nblk;
-    int best = 0, best_cost = -1;
-    for (int x = 0; x <= 2 * nblk && x <= ntile; ++x) {              // tiles for the walking waves
-        const int rest = ntile - x;
-        if (rest > kTilesPerWave * helpers) continue;
-        const int own = 38 + 7 * ((x + nblk - 1) / nblk);
-        const int help = helpers > 0 ? (4 * nfor + 7 * rest + helpers - 1) / helpers : 0;
-        const int cost = own > help ? own : help;
-        if (best_cost < 0 || cost < best_cost) { best = x; best_cost = cost; }
+// Those tiles, block by block, are dealt to the waves in runs: at most three to a wave that walks no block (a helper), at
+// most one to one that does (the triangle and the tile next to it take the registers of two), and the foreign blocks
+// to the helpers that fetch them.  What a wave does in a stage, in hundreds of cycles (measured): walking 45 with the
+// adjacent tile's product, a tile 7, fetching a foreign block 4.  Waves w and w + 4 share a SIMD, on which all of it
+// adds up: each tile goes where least is to be done.
+struct TileDeal { unsigned wave; };          // four bits a wave: tiles, foreign blocks << 2
+__device__ __host__ __forceinline__ int dealt_tiles(const TileDeal &d, int wave) { return (d.wave >> (4 * wave)) & 3; }
+__device__ __host__ __forceinline__ int dealt_foreign(const TileDeal &d, int wave) { return (d.wave >> (4 * wave + 2)) & 3; }
+// returns what the busiest SIMD has to do, -1 if there are more tiles than the waves have room for
+inline int deal_tiles(int jb0, int nblk, int W, TileDeal &deal) {    // (on the host: a plan made by the kernel costs it 2 us)
+    constexpr int kWalk = 45, kProduct = 7, kFetch = 4, kSimds = 4;
+    int load[kSimds] = {0, 0, 0, 0}, tiles[kTileWaves] = {0}, foreign[kTileWaves] = {0};
+    for (int w = 0; w < nblk; ++w) load[w % kSimds] += kWalk;
+    int ntile = 0;
+    const int nfor = jb0 - tile_ilo(jb0, W);
+    for (int q = 0; q < nblk; ++q) ntile += tiles_of_block(jb0 + q, W);
+    auto place = [&](int (&count)[kTileWaves], const bool fetch, const int cost) {
+        int best = -1;
+        for (int w = kTileWaves - 1; w >= 0; --w) {
+            const int most = fetch ? (w >= nblk || nblk == kTileWaves ? kForeign : 0) : (w >= nblk ? kTilesPerWave : 1);
+            if (count[w] >= most) continue;
+            if (best < 0 || load[w % kSimds] < load[best % kSimds] || (load[w % kSimds] == load[best % kSimds] && count[w] < count[best])) best = w;
+        }
+        if (best < 0) return false;
+        ++count[best];
+        load[best % kSimds] += cost;
+        return true;
+    };
+    for (int n = 0; n < ntile; ++n) if (!place(tiles, false, kProduct)) return -1;
+    for (int n = 0; n < nfor; ++n) if (!place(foreign, true, kFetch)) return -1;
+    deal.wave = 0;
+    int most = 0;
+    for (int w = 0; w < kTileWaves; ++w) deal.wave |= (unsigned)(tiles[w] | foreign[w] << 2) << (4 * w);
+    for (int x = 0; x < kSimds; ++x) most = load[x] > most ? load[x] : most;
+    return most;
+}
+// first tile, number of tiles, first foreign block and number of foreign blocks of a wave (the helpers' tiles first,
+// from the last wave down)
+__device__ __host__ __forceinline__ void wave_tiles(const TileDeal &d, int wave, int &first, int &count) {
+    first = 0; count = dealt_tiles(d, wave);
+    for (int w = 1; w < kTileWaves; ++w) first += w > wave ? dealt_tiles(d, w) : 0;
+}
+__device__ __host__ __forceinline__ void wave_foreign(const TileDeal &d, int wave, int &first, int &count) {
+    first = 0; count = dealt_foreign(d, wave);
+    for (int w = 1; w < kTileWaves; ++w) first += w > wave ? dealt_foreign(d, w) : 0;
+}
+
+// Host: the groupings of a graph's position blocks for every number of blocks up to NB, each into at most C contiguous
+// groups of at most kTileCap tiles (the diagonal ones among them) and kChunkBlocks blocks so that the busiest SIMD has
+// least to do.  gtab[nb][g] .. gtab[nb][g+1]: blocks of group g (empty groups last).
+struct ChunkPlan {
+    unsigned char gtab[kMaxBlocksFast + 1][12];
+    TileDeal deal[kMaxBlocksFast + 1][12];
+};
+inline void plan_chunks(int NB, int W, int C, ChunkPlan &plan) {
+    int cost[kMaxBlocksFast][kChunkBlocks + 1];
+    TileDeal deal[kMaxBlocksFast][kChunkBlocks + 1];
+    for (int j = 0; j < NB; ++j) {
+        int tiles = 0;
+        for (int n = 1; n <= kChunkBlocks; ++n) {
+            cost[j][n] = -1;
+            if (j + n > NB) continue;
+            tiles += j + n - tile_ilo(j + n - 1, W);
+            if (tiles <= kTileCap) cost[j][n] = deal_tiles(j, n, W, deal[j][n]);
+        }
     }
-    const int rest = ntile - best;
-    return TileDeal{(unsigned char)(helpers > 0 ? rest / helpers : 0), (unsigned char)(helpers > 0 ? rest % helpers : 0),
-                    (unsigned char)(best / nblk), (unsigned char)(best % nblk)};
+    for (int nb = 0; nb <= NB; ++nb) {
+        int low = 0, high = 1 << 12;                 // the least bound on a group's cost that C groups can keep
+        auto split = [&](const int most, unsigned char *g) {
+            int used = 0, j = 0;
+            g[0] = 0;
+            while (j < nb) {
+                int n = 0;
+                for (int x = 1; x <= kChunkBlocks && j + x <= nb; ++x) if (cost[j][x] >= 0 && cost[j][x] <= most) n = x;
+                if (n == 0 || used == C) return false;
+                j += n;
+                g[++used] = (unsigned char)j;
+            }
+            for (int q = used; q < C; ++q) g[q + 1] = (unsigned char)nb;
+            return true;
+        };
+        unsigned char g[16];
+        while (low < high) { const int mid = (low + high) / 2; if (split(mid, g)) high = mid; else low = mid + 1; }
+        split(high, g);
+        for (int q = 0; q < 12; ++q) {
+            plan.gtab[nb][q] = q <= C ? g[q] : (unsigned char)nb;
+            plan.deal[nb][q] = q < C && g[q + 1] > g[q] ? deal[g[q]][g[q + 1] - g[q]] : TileDeal{0};
+        }
+    }
 }
-// first tile and number of tiles of a wave (the helpers' first, from the last wave down)
-__device__ __host__ __forceinline__ void wave_tiles(const TileDeal &d, int nblk, int wave, int &first, int &count) {
-    const bool walks = wave < nblk;
-    const int r = walks ? nblk - 1 - wave : kTileWaves - 1 - wave, base = walks ? d.base_o : d.base_h, rem = walks ? d.rem_o : d.rem_h;
-    first = (walks ? d.base_h * (kTileWaves - nblk) + d.rem_h : 0) + r * base + (r < rem ? r : rem);
-    count = base + (r < rem ? 1 : 0);
-}
-__device__ __host__ __forceinline__ int tiles_of_block(int J, int W) { return J < W ? J : W; }   // tiles below the diagonal
 
 // a = {a's lower half, b's lower half}, b = {a's upper half, b's upper half}.  (The results go through unsigned variables:
 // __builtin_bit_cast of an element of a vector yields element 0 with this compiler.)

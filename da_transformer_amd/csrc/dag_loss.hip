@@ -54,8 +54,7 @@ struct SweepArgs {
     // domain holds, an upper bound).  With gradients {alpha/upper, beta/lower}, without {alpha/lower, alpha/upper}.
     unsigned char rev[2], upper[2];
     int only_flagged;  // exact kernel: 0 = every sample; 1 = samples whose flag is set
-    unsigned char gtab[kMaxBlocksFast + 1][12];  // fast path: gtab[NBb][g] = first block of group g (host-built)
-    TileDeal deal[kMaxBlocksFast + 1][12];       // and how its tiles are dealt to its waves (float32 sweeps)
+    ChunkPlan plan;    // fast path, host-built: gtab[NBb][g] = first block of group g, and how its tiles are dealt to its waves (float32 sweeps)
     double *zfast;     // [2][B] the fast kernel's own read-outs (never rewritten by the exact kernel)
 };
 
@@ -468,7 +467,7 @@ __device__ __forceinline__ void sweep_tiles_group(const SweepArgs &a, const int 
     const int slack = Lb - Tb;
     const int NBb = (Lb + kBlk - 1) / kBlk;
     const int W = (translen + kBlk - 1) / kBlk;
-    if (tid <= C) gstart[tid] = a.gtab[NBb][tid];
+    if (tid <= C) gstart[tid] = a.plan.gtab[NBb][tid];
     __syncthreads();
     const int jb0 = __builtin_amdgcn_readfirstlane(gstart[g]), jb1 = __builtin_amdgcn_readfirstlane(gstart[g + 1]);
     int last_group = 0;
@@ -981,12 +980,15 @@ __device__ __forceinline__ void sweep_tiles_group(const SweepArgs &a, const int 
 // What a step-by-step sweep pays per step -- barriers, LDS round trips, scales, a few hundred instructions a wave around
 // the FMAs, 2.0 us at L = 512 -- is paid here once per four steps, and the tiles below the diagonal run on the matrix cores
 // at twice the rate of DPP FMAs.  What is left on the critical path is the walk of one block through four steps
-// (48 FMAs and 20 to 40 other instructions a step, 5.5 cycles each) and two stages per block of the graph.
-//   step by step -> chunks, forward: B = 64, L = 512, T = 64 134 -> 115 us; L = 64 (T = 64) 81 -> 46; L = 256 99 -> 70;
-//   B = 16, L = 1024, T = 256 572 -> 375; B = 64, L = 512, transitions of at most 32: 136 -> 99.
+// (48 FMAs and 20 to 40 other instructions a step, 5.5 cycles each), the product of the tile next to the diagonal in
+// front of it, and one stage per block of the graph.  (With that product a stage ahead, too, the stages are 600 cycles
+// shorter but two per block: forward at B = 64, L = 512, T = 64 115 us instead of 107, L = 256 70 instead of 66,
+// L = 128 52 instead of 56.)
+//   step by step -> chunks, forward: B = 64, L = 512, T = 64 134 -> 107 us; L = 64 (T = 64) 81 -> 46; L = 256 99 -> 66;
+//   B = 16, L = 1024, T = 256 572 -> 357; B = 64, L = 512, transitions of at most 32: 136 -> 79.
 // What bounds it: a SIMD gives its cycles either to matrix instructions or to vector instructions, never to both
 // (measured: a wave of DPP FMAs beside one of v_mfma_f32_4x4x1 advances only when that has ended, whatever their
-// priorities), so that products, walks and the rest of a stage add up: 6 600 cycles a stage at L = 512.
+// priorities), so that products, walks and the rest of a stage add up.
 // A walking wave loads and converts its own match rows and writes its own results (as duties of other waves, through
 // LDS, they cost those waves more than they save it).
 template <typename TM, typename TL>
@@ -1017,7 +1019,7 @@ __device__ __forceinline__ void sweep_chunks_group(const SweepArgs &a, const int
     const int slack = Lb - Tb;                    // band: s <= p <= slack + s
     const int NBb = (Lb + kBlk - 1) / kBlk;
     const int W = (translen + kBlk - 1) / kBlk;
-    if (tid <= C) gstart[tid] = a.gtab[NBb][tid];
+    if (tid <= C) gstart[tid] = a.plan.gtab[NBb][tid];
     __syncthreads();
     const int jb0 = __builtin_amdgcn_readfirstlane(gstart[g]), jb1 = __builtin_amdgcn_readfirstlane(gstart[g + 1]);
     int last_group = 0;
@@ -1039,13 +1041,13 @@ __device__ __forceinline__ void sweep_chunks_group(const SweepArgs &a, const int
 
     // ---- my tiles below the diagonal.  A run is a wave's tiles that lead to one block; runs are numbered in the order of
     //      the tiles.  Worked out with lane <-> block (f: its first tile) and lane <-> wave (w_first: its first tile). ----
-    const TileDeal deal = a.deal[NBb][g];
+    const TileDeal deal = a.plan.deal[NBb][g];
     int my_first, my_count;
-    wave_tiles(deal, nblk, wave, my_first, my_count);
+    wave_tiles(deal, wave, my_first, my_count);
     int f = 0, w_first, w_count;
 #pragma unroll
     for (int q = 0; q < kChunkBlocks; ++q) f += q < lane && q < nblk ? tiles_of_block(jb0 + q, W) : 0;
-    wave_tiles(deal, nblk, lane & (kTileWaves - 1), w_first, w_count);
+    wave_tiles(deal, lane & (kTileWaves - 1), w_first, w_count);
     int f_of[kChunkBlocks + 1];
     bool cuts = lane < kTileWaves && w_count > 0;   // this wave's first tile begins a run in the middle of a block
 #pragma unroll
@@ -1053,28 +1055,28 @@ __device__ __forceinline__ void sweep_chunks_group(const SweepArgs &a, const int
         f_of[q] = __builtin_amdgcn_readlane(f, q);
         if (q < nblk) cuts = cuts && !(w_first == f_of[q] && tiles_of_block(jb0 + q, W) > 0);
     }
-    const bool lone = jb0 == 0;                     // (block 0 has no tiles: the runs are counted from block 1)
+    const int without = jb0 < 2 ? 2 - jb0 : 0;      // (blocks 0 and 1 have no such tiles)
     // number of runs that begin at or before tile n of block q
-    auto runs_to = [&](const int q, const int n) { return q + (lone ? 0 : 1) + (int)__builtin_popcountll(__builtin_amdgcn_ballot_w64(cuts && w_first <= n)); };
+    auto runs_to = [&](const int q, const int n) { return q + 1 - without + (int)__builtin_popcountll(__builtin_amdgcn_ballot_w64(cuts && w_first <= n)); };
     int t_I[kTilesPerWave], t_q[kTilesPerWave], t_run[kTilesPerWave];   // source block, own block it leads to, run it belongs to
     bool t_ok[kTilesPerWave], t_start[kTilesPerWave], t_end[kTilesPerWave], t_lead[kTilesPerWave];   // first / last tile of its run; run that states the scale
 #pragma unroll
     for (int u = 0; u < kTilesPerWave; ++u) {
-        const int n = my_first + u;
-        t_ok[u] = u < my_count;
+        const int r0 = owner ? u - 1 : u, n = my_first + r0;   // (a walking wave has the tile next to the diagonal in slot 0)
+        t_ok[u] = r0 >= 0 && r0 < my_count;
         int q = 0;
 #pragma unroll
         for (int x = 1; x < kChunkBlocks; ++x) q = x < nblk && n >= f_of[x] ? x : q;
         const int lo = tile_ilo(jb0 + q, W), r = n - f_of[q];
         t_q[u] = t_ok[u] ? q : 0;
         t_I[u] = t_ok[u] ? lo + r : flo;
-        t_start[u] = u == 0 || r == 0;
-        t_end[u] = u == my_count - 1 || lo + r == jb0 + q - 1;
-        t_lead[u] = u >= r;                       // (the run reaches back to the block's first tile)
+        t_start[u] = r0 == 0 || r == 0;
+        t_end[u] = r0 == my_count - 1 || lo + r == jb0 + q - 2;
+        t_lead[u] = r0 >= r;                      // (the run reaches back to the block's first tile)
         t_run[u] = runs_to(q, n) - 1;
     }
     // the runs that lead to the block this wave walks
-    int run_first = ntile, run_count = 1;         // (block 0 receives nothing: the zeros behind the products)
+    int run_first = ntile, run_count = 1;         // (a block without such tiles: the zeros behind the products)
     if (owner && tiles_of_block(jb0 + wave, W) > 0) {
         const int n = __builtin_amdgcn_readlane(f, wave);
         run_first = runs_to(wave, n) - 1;
@@ -1091,14 +1093,18 @@ __device__ __forceinline__ void sweep_chunks_group(const SweepArgs &a, const int
     float *const patch = lds_raw + wave * (kBlk * kPatchPitch);
     const int last_index = L * translen - 1;
     const float tiny = !upper ? 0.f : kTinyStored;
-    if (owner) { t_I[kTilesPerWave - 1] = jb0 + wave; t_q[kTilesPerWave - 1] = wave; }   // the triangle
+    const bool adjacent = owner && jb0 + wave > 0;
+    if (owner) {                                  // the triangle, and the tile next to it
+        t_I[kTilesPerWave - 1] = jb0 + wave; t_q[kTilesPerWave - 1] = wave;
+        t_I[0] = jb0 + wave - (adjacent ? 1 : 0); t_q[0] = wave;
+    }
     auto elements = [&](const int samples) { const int64_t n = (int64_t)samples * L * translen; return n < (1 << 28) ? (int)n : 1 << 28; };
     const int before = elements(b), behind = elements(a.B - 1 - b);
     auto stage = [&](const int u) __attribute__((always_inline)) {
         stage_tile<TL>(patch, links, t_I[u], jb0 + t_q[u], lane, dir, Lb, translen, last_index, before, behind, tiny);
     };
     Tile t0, t1, t2;
-    if (t_ok[0]) { stage(0); read_patch(t0, patch, lane, dir); }
+    if (t_ok[0] || adjacent) { stage(0); read_patch(t0, patch, lane, dir); }
     if (t_ok[1]) { stage(1); read_patch(t1, patch, lane, dir); }
     if (t_ok[2] || owner) { stage(2); read_patch(t2, patch, lane, dir); }
     if (owner) fold_triangle(t2, lane);
@@ -1135,7 +1141,7 @@ __device__ __forceinline__ void sweep_chunks_group(const SweepArgs &a, const int
         if (lane == 0) store_agent(off + (int64_t)t_first * NBK + Jb, Jb == 0 && alive0 ? (double)(n0 + 1) * 0.6931471805599453 : (double)DAGX_NEG_INF);
     }
     if (tid < 2 * 256) lds_raw[o.part + ntile * 2 * 256 + tid] = 0.f;
-    if (jb0 == 0 && tid < 2 * kChunk) lds_i[o.part_scale + tid] = kDeadExp;
+    if (tid < nblk * 2 * kChunk) lds_i[o.part_scale + tid] = kDeadExp;   // (stays with a block without such tiles)
     if (Tb == 1 && tid == 0 && jb0 == 0) {
         const double z = (Lb == 1 && alive0) ? (double)m0 : (double)DAGX_NEG_INF;
         a.logz[slot * a.B + b] = z; if (slot == a.loss_dir) a.loss[b] = (float)z; store_agent(a.zfast + slot * a.B + b, z);
@@ -1157,13 +1163,11 @@ __device__ __forceinline__ void sweep_chunks_group(const SweepArgs &a, const int
     auto dest_hi = [&](const int J) { return 16 * J + 15; };
     auto src_lo = [&](const int I) { return 16 * I - ((slack + 3) >> 2); };
 
-    // ---- the foreign blocks whose table rows this wave fetches: dealt to the helpers, or to all if there is none ----
-    int f_blk[kForeign];
+    // ---- the foreign blocks whose table rows this wave fetches ----
+    int f_blk[kForeign], f_first, f_count;
+    wave_foreign(deal, wave, f_first, f_count);
 #pragma unroll
-    for (int u = 0; u < kForeign; ++u) {
-        const int fb = helpers == 0 ? flo + wave + kTileWaves * u : (owner ? jb0 : flo + (wave - nblk) + helpers * u);
-        f_blk[u] = fb < jb0 ? fb : -1;
-    }
+    for (int u = 0; u < kForeign; ++u) f_blk[u] = u < f_count ? flo + f_first + u : -1;
     // Table rows of steps 4c .. 4c+3 of a foreign block (complete: 64 positions): one copy of sixteen bytes a lane for the
     // residuals (row lane / 16, in the order of the nodes), one for the offsets.
     auto request_rows = [&](const int I, const int c, const int lane) __attribute__((always_inline)) {
@@ -1201,20 +1205,20 @@ __device__ __forceinline__ void sweep_chunks_group(const SweepArgs &a, const int
     };
 
     // ---- the stages ----
-    const int first_stage = consumer ? -2 : -1, end_stage = NC - 1 + 2 * (nblk - 1);
+    const int first_stage = consumer ? -2 : -1, end_stage = NC - 1 + nblk - 1;
     const int *below = prog + (g > 0 ? g - 1 : 0);
     // stages in which a tile's block takes part, and those in which the tile's source has a live cell
     int t_from[kTilesPerWave], t_to[kTilesPerWave], t_src_from[kTilesPerWave], t_src_to[kTilesPerWave];
     int t_shift[kTilesPerWave], t_cells[kTilesPerWave], t_kaps[kTilesPerWave], t_scale_at[kTilesPerWave], t_scales[kTilesPerWave];
 #pragma unroll
     for (int u = 0; u < kTilesPerWave; ++u) {
-        const int J = jb0 + t_q[u], at = 2 * t_q[u] - 1, lo = tile_ilo(J, W);   // chunk = stage - at
+        const int J = jb0 + t_q[u], at = t_q[u] - 1, lo = tile_ilo(J, W);   // chunk = stage - at
         t_from[u] = at + (dest_lo(J) > 0 ? dest_lo(J) : 0);
         t_to[u] = t_ok[u] ? at + (dest_hi(J) < NC - 1 ? dest_hi(J) : NC - 1) : -100;
         t_src_from[u] = at + src_lo(t_I[u]); t_src_to[u] = at + dest_hi(t_I[u]);
         t_shift[u] = (((-at) % D) + D) % D;
         t_cells[u] = o.eb + (t_I[u] - flo) * D * 256; t_kaps[u] = o.kap + (t_I[u] - flo) * D * 4;
-        t_scale_at[u] = o.kap + (lo - flo) * D * 4; t_scales[u] = J - lo;
+        t_scale_at[u] = o.kap + (lo - flo) * D * 4; t_scales[u] = J - 1 - lo;
     }
     if (NC == 0) return;
     __syncthreads();
@@ -1321,9 +1325,9 @@ __device__ __forceinline__ void sweep_chunks_group(const SweepArgs &a, const int
             const bool bring = FETCHES && f_blk[0] >= 0 && cf < NC;
             int published = 0;
             if (bring) published = load_agent(below);
-            // ---------------- walk my block through chunk tau - 2 wave ----------------
+            // ---------------- walk my block through chunk tau - wave ----------------
             if (WALKS) {
-                const int c = tau - 2 * wave;
+                const int c = tau - wave;
                 const bool more = c >= -1 && c + 1 < NC;
                 if (more) load_match(c + 1, lane);
                 if (c >= 0 && c < NC) {
@@ -1334,7 +1338,21 @@ __device__ __forceinline__ void sweep_chunks_group(const SweepArgs &a, const int
                     float v[kChunk];
                     if (c >= dest_lo(J) && c <= dest_hi(J)) {
                         __builtin_amdgcn_s_setprio(3);
-                        const i32x4 sc = *reinterpret_cast<const i32x4 *>(lds_i + o.part_scale + (wave * 2 + (par ^ 1)) * 4);
+                        // what block J - 1 sends: its cells of this chunk, and (lane <-> step) their exponents, clamped as
+                        // a tile's under the largest of the blocks below
+                        const int rv = lds_i[o.part_scale + (wave * 2 + (par ^ 1)) * 4 + (lane & 3)];
+                        const bool lower = J > 0 && c >= src_lo(J - 1) && c <= dest_hi(J - 1);
+                        f32x4 Ga = {0.f, 0.f, 0.f, 0.f};
+                        int av = kDeadExp;
+                        if (lower) {
+                            const f32x4 ev = *reinterpret_cast<const f32x4 *>(lds_raw + o.eb + ((own_src - 1) * D + slot_own) * 256 + lane * 4);
+                            av = lds_i[o.kap + ((own_src - 1) * D + slot_own) * 4 + (lane & 3)];
+                            Ga = tile_product(t0, ev);
+                            if (av - rv < -126) av = upper ? rv - 126 : kDeadExp;
+                        }
+                        int A[kChunk], R[kChunk];
+#pragma unroll
+                        for (int k = 0; k < kChunk; ++k) { A[k] = __builtin_amdgcn_readlane(av, k); R[k] = __builtin_amdgcn_readlane(rv, k); }
                         const float *const parts = lds_raw + o.part + (run_first * 2 + (par ^ 1)) * 256 + lane * 4;
                         const float upper_half = lane >= 32 ? 1.f : 0.f;
                         f32x4 G = *reinterpret_cast<const f32x4 *>(parts);
@@ -1347,15 +1365,12 @@ __device__ __forceinline__ void sweep_chunks_group(const SweepArgs &a, const int
                             }
                             G += G1;
                         }
-                        int R[kChunk];
-#pragma unroll
-                        for (int k = 0; k < kChunk; ++k) R[k] = __builtin_amdgcn_readfirstlane(sc[k]);
 #pragma unroll
                         for (int k = 0; k < kChunk; ++k) {
                             // (kSpare: every other step does not scale its cells by their largest)
-                            const int ref = (kap > R[k] ? kap : R[k]) + (k & 1 ? 0 : kSpare);
+                            const int most = A[k] > R[k] ? A[k] : R[k], ref = (kap > most ? kap : most) + (k & 1 ? 0 : kSpare);
                             // (what ldexp flushes of either part is under flush_up, too)
-                            const float x = (__builtin_ldexpf(triangle_dot(t2, e, upper_half), kap - ref) + flush_up) + __builtin_ldexpf(G[k], R[k] - ref);
+                            const float x = (__builtin_ldexpf(triangle_dot(t2, e, upper_half), kap - ref) + flush_up) + (__builtin_ldexpf(G[k], R[k] - ref) + __builtin_ldexpf(Ga[k], A[k] - ref));
                             // (upper sweep: a cell never flushes, live or not -- what a dead one gets is of the size of what is flushed)
                             if (k & 1) {
                                 const float y = x * mt[k];
@@ -1384,7 +1399,7 @@ __device__ __forceinline__ void sweep_chunks_group(const SweepArgs &a, const int
                     }
                     if (more) convert_match(c + 1, lane);   // (in front of the stores: what it waits for is older than they)
                     else wait_vmem_all();
-                    // Either wait covers what this wave stored in the last stage.  The other blocks are two chunks and more
+                    // Either wait covers what this wave stored in the last stage.  The other blocks are a chunk and more
                     // ahead of the last one: when its wave has come here, every block's chunk c - 1 is in memory.
                     if (producer && wave == nblk - 1 && c > 0 && lane == 0) store_agent(prog + g, 1 + c);
                     const int kp = write_out(c, v, kk, lane);
@@ -1394,14 +1409,14 @@ __device__ __forceinline__ void sweep_chunks_group(const SweepArgs &a, const int
                 }
                 else if (more) convert_match(c + 1, lane);
             }
-            // ---------------- multiply out what chunk tau + 1 - 2 q of my tiles' blocks receives ----------------
+            // ---------------- multiply out what my tiles' blocks (q of the group) receive in chunk tau + 1 - q ----------------
             if (my_count > 0) {
                 // (the LDS reads of two tiles are requested before the first is waited for, the third's behind the first)
                 f32x4 ev[2];
                 int kv[kTilesPerWave], rv[kTilesPerWave];
                 bool go[kTilesPerWave], src[kTilesPerWave];
 #pragma unroll
-                for (int u = 0; u < (WALKS ? kTilesPerWave - 1 : kTilesPerWave); ++u) {
+                for (int u = WALKS ? 1 : 0; u < (WALKS ? 2 : kTilesPerWave); ++u) {
                     go[u] = tau >= t_from[u] && tau <= t_to[u];
                     src[u] = tau >= t_src_from[u] && tau <= t_src_to[u];
                     if (go[u]) {
@@ -1431,7 +1446,7 @@ __device__ __forceinline__ void sweep_chunks_group(const SweepArgs &a, const int
                         if (t_lead[u] && lane < 4) lds_i[o.part_scale + (t_q[u] * 2 + par) * 4 + lane] = R;
                     }
                 };
-                product(0, t0);
+                if (!WALKS) product(0, t0);
                 if (!WALKS && go[2]) {
                     int sl = ring + t_shift[2]; sl -= sl >= D ? D : 0;
                     ev[0] = *reinterpret_cast<const f32x4 *>(lds_raw + t_cells[2] + sl * 256 + lane * 4);
@@ -2163,9 +2178,19 @@ static bool force_exact() { return force_log_domain(); }
 // ticket + launch counter (16 ints), 2*B*C progress words, B "left" counters, B risk words; rounded to 8 bytes
 static size_t sweep_sync_ints(int B, int C) { return ((16 + (size_t)2 * B * C + (size_t)2 * B) + 1) & ~(size_t)1; }
 
+// Workgroups per sweep (two sweeps a sample): as few as hold the tiles, but with at most four blocks each, one walk to a
+// SIMD, where the device has a CU for every workgroup.  Forward with up to eight -> up to four blocks: B = 40, L = 328,
+// T = 41 67 -> 61 us; B = 16, L = 512, T = 64 102 -> 97.5; B = 64 and transitions of at most 32 88 -> 79; B = 16,
+// L = 1024 and transitions of at most 64 122 -> 104.  More groups than that gain nothing (L = 512 in four 96 us) or lose
+// (L = 256 in two 66 us for 64).
+static int sweep_groups(int B, int L, int translen) {
+    const int C = groups_needed(L, translen, 4), sweeps = 2 * ((B + 7) & ~7);
+    return (long long)sweeps * C <= 256 && C > 0 ? C : groups_needed(L, translen, kChunkBlocks);
+}
+
 size_t loss_fwd_workspace_bytes(int B, int T, int L, int translen) {
     (void)T;
-    int C = groups_used(2 * ((B + 7) & ~7), L, translen, false, kChunkBlocks);
+    int C = sweep_groups(B, L, translen);
     // ticket + progress words (rounded to 8 bytes), then the fast kernel's two read-outs per sample
     return C > 0 ? sweep_sync_ints(B, C) * sizeof(int) + (size_t)2 * B * sizeof(double) : 0;
 }
@@ -2206,7 +2231,7 @@ static int prepare_tiles_kernels_of() {
 
 template <typename TM, typename TL>
 static int launch_sweeps(SweepArgs a, hipStream_t st) {
-    int C = force_exact() ? 0 : groups_used(2 * ((a.B + 7) & ~7), a.L, a.translen, false, kChunkBlocks);
+    int C = force_exact() ? 0 : sweep_groups(a.B, a.L, a.translen);
     // the tile kernel indexes match with 32-bit arithmetic
     const int64_t span = (int64_t)(a.T - 1) * (a.ms1 < 0 ? -a.ms1 : a.ms1) + (int64_t)(a.L - 1) * (a.ms2 < 0 ? -a.ms2 : a.ms2);
     if (span >= (1LL << 31) / (int64_t)sizeof(TM) || a.ms1 < 0 || a.ms2 < 0) C = 0;
@@ -2227,25 +2252,14 @@ static int launch_sweeps(SweepArgs a, hipStream_t st) {
         a.upper[0] = a.loss_dir ? 1 : 0; a.upper[1] = a.loss_dir ? 0 : 1;
         a.C = C;
         {   // how the blocks of a sample are grouped and their tiles dealt, by its number of blocks; remembered for the next call
-            struct Grouping { int W = 0, C = 0, NB = 0; unsigned char gtab[kMaxBlocksFast + 1][12]; TileDeal deal[kMaxBlocksFast + 1][12]; };
+            struct Grouping { int W = 0, C = 0, NB = 0; ChunkPlan plan; };
             static thread_local Grouping last;
             const int W = (a.translen + kBlk - 1) / kBlk;
             if (last.W != W || last.C != C || last.NB < a.NBK) {
-                int tmp[kTileCap + 2];
-                for (int nb = 0; nb <= a.NBK; ++nb) {
-                    partition_chunk_groups(nb, W, C, tmp);
-                    for (int q = 0; q <= C && q < 12; ++q) last.gtab[nb][q] = (unsigned char)tmp[q];
-                    for (int q = 0; q < C; ++q) {
-                        int ntile = 0;
-                        for (int Jb = tmp[q]; Jb < tmp[q + 1]; ++Jb) ntile += tiles_of_block(Jb, W);
-                        if (tmp[q] < tmp[q + 1]) last.deal[nb][q] = deal_tiles(ntile, tmp[q + 1] - tmp[q], tmp[q] - tile_ilo(tmp[q], W));
-                    }
-                }
+                plan_chunks(a.NBK, W, C, last.plan);
                 last.W = W; last.C = C; last.NB = a.NBK;
             }
-            for (int nb = 0; nb <= a.NBK; ++nb) {
-                for (int q = 0; q < 12; ++q) { a.gtab[nb][q] = last.gtab[nb][q]; a.deal[nb][q] = last.deal[nb][q]; }
-            }
+            a.plan = last.plan;
         }
         const int B8 = (a.B + 7) & ~7;
         if ((rc = prepare_tiles_kernel<TM, TL, false>()) || (rc = prepare_tiles_kernel<TM, TL, true>())) return rc;

@@ -117,20 +117,17 @@ inline int groups_needed(int L, int translen, int most = kMaxBlocksFast) {
     return groups <= 11 ? groups : 0;
 }
 
-// Host: workgroups per sweep actually launched (`most`: blocks a group may own).  More groups than needed mean fewer
-// tiles per SIMD but a hand-over between groups in every step and a deeper pipeline.  Measured on MI355X (B = 16..64,
-// T = 64): the loss sweeps (two per sample) take the minimal number; the
+// Host: workgroups per sweep actually launched by the alignment.  More groups than needed mean fewer tiles per SIMD but a
+// hand-over between groups in every step and a deeper pipeline.  Measured on MI355X (B = 16..64, T = 64): the
 // alignment sweep gains 5-13 % from doubling the groups once when the graph has at least 4 blocks and the
 // device has room (one workgroup per CU), and loses from doubling twice; where twice the minimal number
 // exceeds the 11 the kernel supports (L > 704), 10 groups are used when they fit.
-inline int groups_used(int sweeps, int L, int translen, bool may_double, int most = kMaxBlocksFast) {
-    int C = groups_needed(L, translen, most);
+inline int groups_used(int sweeps, int L, int translen) {
+    int C = groups_needed(L, translen);
     if (C == 0) return 0;
     const int NB = (L + kBlk - 1) / kBlk;
-    if (may_double) {
-        if (NB >= 4 && 2 * C <= 11 && 2 * C <= NB && (long long)sweeps * 2 * C <= 256) C *= 2;
-        else if (C < 10 && NB >= 10 && (long long)sweeps * 10 <= 256) C = 10;   // L=1024, T=256, B=16: 0.93 -> 0.82 ms
-    }
+    if (NB >= 4 && 2 * C <= 11 && 2 * C <= NB && (long long)sweeps * 2 * C <= 256) C *= 2;
+    else if (C < 10 && NB >= 10 && (long long)sweeps * 10 <= 256) C = 10;   // L=1024, T=256, B=16: 0.93 -> 0.82 ms
     return C;
 }
 

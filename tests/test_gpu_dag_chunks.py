@@ -18,7 +18,8 @@ F32, F16, BF16 = torch.float32, torch.float16, torch.bfloat16
     (1, 63, 5, None, F32), (2, 64, 2, None, F16), (1, 65, 6, 63, F16), (3, 65, 9, 64, BF16), (2, 66, 10, 1, F32),
     (1, 127, 13, 65, F32), (2, 129, 17, 2, BF16), (1, 320, 8, None, F16), (2, 321, 9, 128, F32), (1, 385, 33, 63, F16),
     (2, 449, 30, 32, F32), (1, 511, 14, None, BF16), (2, 513, 7, 257, F32), (1, 705, 12, 130, F16), (2, 1024, 11, None, F32),
-    (1, 1023, 64, 200, F16)])
+    (1, 1023, 64, 200, F16),
+    (65, 320, 8, None, F16), (65, 1022, 20, 64, F16)])   # no room for groups of at most four blocks: five, eight
 def test_edges_of_blocks_chunks_and_windows(B, L, T, translen, dtype):
     match, links_sq, ol, tl = random_problem(L + T, B + 1, L, T, dtype=F32, ragged=False, translen=translen)
     if translen is not None:      # a path of T_b nodes spans at most (T_b - 1) translen transitions
