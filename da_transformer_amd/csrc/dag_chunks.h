@@ -12,14 +12,33 @@ namespace dagx {
 // multiplies out when the stage begins; what it receives from the blocks below that one is multiplied out one stage
 // ahead, by waves that are not on the critical path.
 //
-// Numbers are linear: a cell holds exp(value - kap ln 2) 2^kShift2 with one integer exponent kap per block and step,
-// chosen so that the block's largest cell lies in [2^(kShift2-1), 2^kShift2).  All scaling is by powers of two.
+// Numbers are linear: a cell holds exp(value - kap ln 2) 2^kShift with one integer exponent kap per block and step,
+// chosen so that the block's largest cell lies in [2^(kShift-1), 2^kShift).  All scaling is by powers of two.
+//
+// The wide variant keeps cells, products and sums in float64; the staged transitions stay float32 registers (the register
+// file holds no float64 tiles) and are converted as they are used.  What the float32 sweep cannot hold is, almost always,
+// a cell far under the maximum of its block or a block far under its neighbours (inputs whose best prefixes are not the
+// prefixes of the best paths); a float64 number has room for 1300 nats under its scale where a float32 number has 126.
 constexpr int kChunk = 4;
 constexpr int kDeadExp = -(1 << 30);        // the exponent of a block without a live cell
 constexpr int kDeadBelow = -(1 << 29);      // any exponent below this is that of a dead block
 constexpr int kMatchExpMax = 1 << 17;       // match values beyond 2^+-this are rounded (down: to this or 0; up: the sample is done again)
 constexpr int kSpare = 62;                   // binades by which a step that does not scale its cells by their largest lowers them
 constexpr int kChunkBlocks = 8;             // a group owns at most this many blocks: one wave walks one block
+
+template <bool WIDE> struct Chunks;
+template <> struct Chunks<false> {
+    typedef float Cell;
+    static constexpr int kShift = kShift2, kLinkShift = kShift2;   // powers of two that cells and staged transitions carry
+    static constexpr int kFloor = -126;                            // least exponent of a scale factor in the upper sweep (0 below it in the lower)
+    static constexpr int kStepPitch = 4;                           // distance of a cell's steps in a chunk of cells
+};
+template <> struct Chunks<true> {
+    typedef double Cell;
+    static constexpr int kShift = 850, kLinkShift = kShiftLinksWide;   // a sum of products: 2^(850 + 127 + 10) < 2^1024
+    static constexpr int kFloor = -1022;
+    static constexpr int kStepPitch = 2;
+};
 
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef int i32x4 __attribute__((ext_vector_type(4)));
@@ -31,29 +50,40 @@ __device__ __host__ __forceinline__ int tiles_of_block(int J, int W) { const int
 // LDS of a group, in dwords.
 struct ChunkLds {
     int depth;      // chunks of cells kept per block: read up to (blocks of the group) stages after they are written
-    int eb;         // [nsrc][depth][256]  cells of four steps: (4 (i & 15) + (s & 3)) 4 + i / 16
+    int runs;       // runs of tiles there can be
+    int eb;         // [nsrc][depth][256]  cells of four steps, in the order of the products' first operand (cell_place)
     int kap;        // [nsrc][depth][4]    their exponents
-    int part;       // [ntile + 1][2][256] products of a run of tiles, four steps per lane; behind them zeros
+    int part;       // [runs + 1][2][256]  products of a run of tiles (float32: four steps per lane; float64: [4][64]); behind them zeros
     int part_scale; // [nblk][2][4]        the exponents they are relative to
+    int turn;       // float64: [nblk][256] where a walking wave turns the adjacent tile's product
     int frows, foff;// [nfor][256], [nfor][64]  landing areas of table rows and offsets of blocks of lower groups
+    int both;       // [1]  counts the last two blocks' waves as they find their rows in memory
     int total;
 };
-__device__ __host__ inline ChunkLds chunk_lds(int jb0, int nblk, int W) {
+__device__ __host__ inline ChunkLds chunk_lds(int jb0, int nblk, int W, bool wide) {
     ChunkLds o;
-    const int flo = tile_ilo(jb0, W), nfor = jb0 - flo, nsrc = nfor + nblk;
+    const int flo = tile_ilo(jb0, W), nfor = jb0 - flo, nsrc = nfor + nblk, chunk = wide ? 512 : 256;
     int ntile = 0;
     for (int q = 0; q < nblk; ++q) ntile += tiles_of_block(jb0 + q, W);
     const int reach = nblk < W ? nblk : W;
     o.depth = reach + 1 < 3 ? 3 : reach + 1;
+    o.runs = ntile < kTileWaves + nblk - 1 ? ntile : kTileWaves + nblk - 1;
     int at = 0;
-    o.eb = at; at += nsrc * o.depth * 256;
-    o.part = at; at += (ntile + 1) * 2 * 256;
+    o.eb = at; at += nsrc * o.depth * chunk;
+    o.part = at; at += (o.runs + 1) * 2 * chunk;
+    o.turn = at; at += wide ? nblk * chunk : 0;
     o.frows = at; at += nfor * 256;
     o.foff = at; at += nfor * 64;
     o.kap = at; at += nsrc * o.depth * 4;
     o.part_scale = at; at += nblk * 2 * 4;
+    o.both = at; at += 4;
     o.total = at;
     return o;
+}
+// where a block's cell of step 4c + k, position `row`, stands in a chunk of cells: + kStepPitch k
+template <bool WIDE>
+__device__ __forceinline__ int cell_place(int row) {
+    return WIDE ? ((row >> 3) * 16 + (row & 3) * 4) * 2 + ((row >> 2) & 1) : (row & 15) * 16 + (row >> 4);
 }
 constexpr int kForeign = 3;                  // foreign blocks a wave fetches at most
 constexpr int kChunkLdsBytes = 160 * 1024 - 512;
@@ -61,14 +91,15 @@ constexpr int kChunkLdsBytes = 160 * 1024 - 512;
 // Those tiles, block by block, are dealt to the waves in runs: at most three to a wave that walks no block (a helper), at
 // most one to one that does (the triangle and the tile next to it take the registers of two), and the foreign blocks
 // to the helpers that fetch them.  What a wave does in a stage, in hundreds of cycles (measured): walking 45 with the
-// adjacent tile's product, a tile 7, fetching a foreign block 4.  Waves w and w + 4 share a SIMD, on which all of it
+// adjacent tile's product, a tile 7, fetching a foreign block 4; in float64 85, 17 and 11.  Waves w and w + 4 share a SIMD, on which all of it
 // adds up: each tile goes where least is to be done.
 struct TileDeal { unsigned wave; };          // four bits a wave: tiles, foreign blocks << 2
 __device__ __host__ __forceinline__ int dealt_tiles(const TileDeal &d, int wave) { return (d.wave >> (4 * wave)) & 3; }
 __device__ __host__ __forceinline__ int dealt_foreign(const TileDeal &d, int wave) { return (d.wave >> (4 * wave + 2)) & 3; }
 // returns what the busiest SIMD has to do, -1 if there are more tiles than the waves have room for
-inline int deal_tiles(int jb0, int nblk, int W, TileDeal &deal) {    // (on the host: a plan made by the kernel costs it 2 us)
-    constexpr int kWalk = 45, kProduct = 7, kFetch = 4, kSimds = 4;
+inline int deal_tiles(int jb0, int nblk, int W, bool wide, TileDeal &deal) {   // (on the host: a plan made by the kernel costs it 2 us)
+    const int kWalk = wide ? 85 : 45, kProduct = wide ? 17 : 7, kFetch = wide ? 11 : 4;
+    constexpr int kSimds = 4;
     int load[kSimds] = {0, 0, 0, 0}, tiles[kTileWaves] = {0}, foreign[kTileWaves] = {0};
     for (int w = 0; w < nblk; ++w) load[w % kSimds] += kWalk;
     int ntile = 0;
@@ -110,18 +141,18 @@ __device__ __host__ __forceinline__ void wave_foreign(const TileDeal &d, int wav
 // least to do.  gtab[nb][g] .. gtab[nb][g+1]: blocks of group g (empty groups last).
 struct ChunkPlan {
     unsigned char gtab[kMaxBlocksFast + 1][12];
-    TileDeal deal[kMaxBlocksFast + 1][12];
+    TileDeal deal[2][kMaxBlocksFast + 1][12];   // of the float32 and the float64 sweeps
 };
 inline void plan_chunks(int NB, int W, int C, ChunkPlan &plan) {
     int cost[kMaxBlocksFast][kChunkBlocks + 1];
-    TileDeal deal[kMaxBlocksFast][kChunkBlocks + 1];
+    TileDeal deal[2][kMaxBlocksFast][kChunkBlocks + 1];
     for (int j = 0; j < NB; ++j) {
         int tiles = 0;
         for (int n = 1; n <= kChunkBlocks; ++n) {
             cost[j][n] = -1;
             if (j + n > NB) continue;
             tiles += j + n - tile_ilo(j + n - 1, W);
-            if (tiles <= kTileCap) cost[j][n] = deal_tiles(j, n, W, deal[j][n]);
+            if (tiles <= kTileCap) { cost[j][n] = deal_tiles(j, n, W, false, deal[0][j][n]); deal_tiles(j, n, W, true, deal[1][j][n]); }
         }
     }
     for (int nb = 0; nb <= NB; ++nb) {
@@ -144,7 +175,7 @@ inline void plan_chunks(int NB, int W, int C, ChunkPlan &plan) {
         split(high, g);
         for (int q = 0; q < 12; ++q) {
             plan.gtab[nb][q] = q <= C ? g[q] : (unsigned char)nb;
-            plan.deal[nb][q] = q < C && g[q + 1] > g[q] ? deal[g[q]][g[q + 1] - g[q]] : TileDeal{0};
+            for (int w = 0; w < 2; ++w) plan.deal[w][nb][q] = q < C && g[q + 1] > g[q] ? deal[w][g[q]][g[q + 1] - g[q]] : TileDeal{0};
         }
     }
 }
@@ -172,6 +203,24 @@ __device__ __forceinline__ unsigned wave64_max_positive(float x) {
         "v_max_f32_dpp %0, %0, %0 row_bcast:15 row_mask:0xa bank_mask:0xf\n\t"
         "s_nop 1\n\t"
         "v_max_f32_dpp %0, %0, %0 row_bcast:31 row_mask:0xc bank_mask:0xf"
+        : "+v"(v));
+    return (unsigned)__builtin_amdgcn_readlane((int)v, 63);
+}
+// the same of the upper halves of 64 float64 numbers >= 0 (a NaN counts as the largest)
+__device__ __forceinline__ unsigned wave64_max_upper(double x) {
+    unsigned v = (unsigned)(__builtin_bit_cast(unsigned long long, x) >> 32);
+    asm("s_nop 1\n\t"
+        "v_max_u32_dpp %0, %0, %0 quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"
+        "s_nop 1\n\t"
+        "v_max_u32_dpp %0, %0, %0 quad_perm:[2,3,0,1] row_mask:0xf bank_mask:0xf\n\t"
+        "s_nop 1\n\t"
+        "v_max_u32_dpp %0, %0, %0 row_half_mirror row_mask:0xf bank_mask:0xf\n\t"
+        "s_nop 1\n\t"
+        "v_max_u32_dpp %0, %0, %0 row_mirror row_mask:0xf bank_mask:0xf\n\t"
+        "s_nop 1\n\t"
+        "v_max_u32_dpp %0, %0, %0 row_bcast:15 row_mask:0xa bank_mask:0xf\n\t"
+        "s_nop 1\n\t"
+        "v_max_u32_dpp %0, %0, %0 row_bcast:31 row_mask:0xc bank_mask:0xf"
         : "+v"(v));
     return (unsigned)__builtin_amdgcn_readlane((int)v, 63);
 }
@@ -218,6 +267,20 @@ __device__ __forceinline__ int by_step_max(int v) {
     return max((int)p[0], (int)p[1]);
 }
 
+// max over the sixteen lanes of a row, in every lane
+__device__ __forceinline__ int row16_max_int(int v) {
+    asm("s_nop 1\n\t"
+        "v_max_i32_dpp %0, %0, %0 quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"
+        "s_nop 1\n\t"
+        "v_max_i32_dpp %0, %0, %0 quad_perm:[2,3,0,1] row_mask:0xf bank_mask:0xf\n\t"
+        "s_nop 1\n\t"
+        "v_max_i32_dpp %0, %0, %0 row_half_mirror row_mask:0xf bank_mask:0xf\n\t"
+        "s_nop 1\n\t"
+        "v_max_i32_dpp %0, %0, %0 row_mirror row_mask:0xf bank_mask:0xf"
+        : "+v"(v));
+    return v;
+}
+
 // g[t] (+)= f[lane t of the row] * a[t]: four steps, each with its own factor
 template <bool FIRST>
 __device__ __forceinline__ void scaled4(f32x4 &g, float f, f32x4 a) {
@@ -254,6 +317,41 @@ __device__ __forceinline__ f32x4 tile_product(const Tile &t, f32x4 e) {
 #undef DAGX_ROWS
 #undef DAGX_PAIR
     return x + y;
+}
+
+// The same in float64, four steps times sixteen positions per accumulator: out[g], lane 16 m + o: step m, position 16 g + o.
+// v_mfma_f64_4x4x4_4b: first operand lane 4 b + m + 16 k = step m of row k (the same in all four blocks b), second lane
+// 4 b + n + 16 k = row k, position 4 b + n, result lane 4 b + 16 m + n.  Tile register 16 g + j: row 4 j + lane / 16,
+// position 16 g + lane mod 16.  (A float64 product takes 16.5 cycles, its operand's conversion 4 to 5.)
+__device__ __forceinline__ void tile_product(const Tile &t, const double *cells, int lane, double (&out)[4]) {
+    typedef double f64x2 __attribute__((ext_vector_type(2)));
+    const f64x2 *const e = reinterpret_cast<const f64x2 *>(cells) + (lane >> 4) * 4 + (lane & 3);
+#pragma unroll
+    for (int g = 0; g < 4; ++g) out[g] = 0.0;
+#pragma unroll
+    for (int jp = 0; jp < 8; ++jp) {
+        const f64x2 ev = e[16 * jp];
+        const double e0 = ev[0], e1 = ev[1];
+        // (by hand: the compiler would convert ahead of the loop over the stages, for which there are no registers.  A product
+        // reads its operands two wait states after a vector instruction has written them.)
+        double b[8];
+        asm volatile("v_cvt_f64_f32 %0, %8\n\t"
+                     "v_cvt_f64_f32 %1, %9\n\t"
+                     "v_cvt_f64_f32 %2, %10\n\t"
+                     "v_cvt_f64_f32 %3, %11\n\t"
+                     "v_cvt_f64_f32 %4, %12\n\t"
+                     "v_cvt_f64_f32 %5, %13\n\t"
+                     "v_cvt_f64_f32 %6, %14\n\t"
+                     "v_cvt_f64_f32 %7, %15\n\t"
+                     "s_nop 1"
+                     : "=&v"(b[0]), "=&v"(b[1]), "=&v"(b[2]), "=&v"(b[3]), "=&v"(b[4]), "=&v"(b[5]), "=&v"(b[6]), "=&v"(b[7])
+                     : "v"(t.p[2 * jp]), "v"(t.p[16 + 2 * jp]), "v"(t.p[32 + 2 * jp]), "v"(t.p[48 + 2 * jp]),
+                       "v"(t.p[2 * jp + 1]), "v"(t.p[16 + 2 * jp + 1]), "v"(t.p[32 + 2 * jp + 1]), "v"(t.p[48 + 2 * jp + 1]));
+#pragma unroll
+        for (int g = 0; g < 4; ++g) out[g] = __builtin_amdgcn_mfma_f64_4x4x4f64(e0, b[g], out[g], 0, 0, 0);
+#pragma unroll
+        for (int g = 0; g < 4; ++g) out[g] = __builtin_amdgcn_mfma_f64_4x4x4f64(e1, b[4 + g], out[g], 0, 0, 0);
+    }
 }
 
 // The triangle on the diagonal (row i of a tile reaches lanes j > i only) in 48 registers instead of 64:
@@ -344,6 +442,75 @@ __device__ __forceinline__ float triangle_dot(const Tile &t, float e, float uppe
     return a;
 }
 
+// the same in float64: each row is converted as it is used
+__device__ __forceinline__ void fma16_rowbcast(double &acc, double e, const float *p) {
+    double t0, t1;
+    asm("s_nop 1\n\t"
+        "v_cvt_f64_f32 %1, %4\n\t"
+        "v_cvt_f64_f32 %2, %5\n\t"
+        "v_fmac_f64_dpp %0, %3, %1 row_newbcast:0 row_mask:0xf bank_mask:0xf\n\t"
+        "v_cvt_f64_f32 %1, %6\n\t"
+        "v_fmac_f64_dpp %0, %3, %2 row_newbcast:1 row_mask:0xf bank_mask:0xf\n\t"
+        "v_cvt_f64_f32 %2, %7\n\t"
+        "v_fmac_f64_dpp %0, %3, %1 row_newbcast:2 row_mask:0xf bank_mask:0xf\n\t"
+        "v_cvt_f64_f32 %1, %8\n\t"
+        "v_fmac_f64_dpp %0, %3, %2 row_newbcast:3 row_mask:0xf bank_mask:0xf\n\t"
+        "v_cvt_f64_f32 %2, %9\n\t"
+        "v_fmac_f64_dpp %0, %3, %1 row_newbcast:4 row_mask:0xf bank_mask:0xf\n\t"
+        "v_cvt_f64_f32 %1, %10\n\t"
+        "v_fmac_f64_dpp %0, %3, %2 row_newbcast:5 row_mask:0xf bank_mask:0xf\n\t"
+        "v_cvt_f64_f32 %2, %11\n\t"
+        "v_fmac_f64_dpp %0, %3, %1 row_newbcast:6 row_mask:0xf bank_mask:0xf\n\t"
+        "v_cvt_f64_f32 %1, %12\n\t"
+        "v_fmac_f64_dpp %0, %3, %2 row_newbcast:7 row_mask:0xf bank_mask:0xf\n\t"
+        "v_cvt_f64_f32 %2, %13\n\t"
+        "v_fmac_f64_dpp %0, %3, %1 row_newbcast:8 row_mask:0xf bank_mask:0xf\n\t"
+        "v_cvt_f64_f32 %1, %14\n\t"
+        "v_fmac_f64_dpp %0, %3, %2 row_newbcast:9 row_mask:0xf bank_mask:0xf\n\t"
+        "v_cvt_f64_f32 %2, %15\n\t"
+        "v_fmac_f64_dpp %0, %3, %1 row_newbcast:10 row_mask:0xf bank_mask:0xf\n\t"
+        "v_cvt_f64_f32 %1, %16\n\t"
+        "v_fmac_f64_dpp %0, %3, %2 row_newbcast:11 row_mask:0xf bank_mask:0xf\n\t"
+        "v_cvt_f64_f32 %2, %17\n\t"
+        "v_fmac_f64_dpp %0, %3, %1 row_newbcast:12 row_mask:0xf bank_mask:0xf\n\t"
+        "v_cvt_f64_f32 %1, %18\n\t"
+        "v_fmac_f64_dpp %0, %3, %2 row_newbcast:13 row_mask:0xf bank_mask:0xf\n\t"
+        "v_cvt_f64_f32 %2, %19\n\t"
+        "v_fmac_f64_dpp %0, %3, %1 row_newbcast:14 row_mask:0xf bank_mask:0xf\n\t"
+        "s_nop 0\n\t"
+        "v_fmac_f64_dpp %0, %3, %2 row_newbcast:15 row_mask:0xf bank_mask:0xf"
+        : "+v"(acc), "=&v"(t0), "=&v"(t1)
+        : "v"(e), "v"(p[0]), "v"(p[1]), "v"(p[2]), "v"(p[3]), "v"(p[4]), "v"(p[5]), "v"(p[6]), "v"(p[7]),
+          "v"(p[8]), "v"(p[9]), "v"(p[10]), "v"(p[11]), "v"(p[12]), "v"(p[13]), "v"(p[14]), "v"(p[15]));
+}
+// {x, y} -> x: rows {x0 y0 x2 y2} / halves {x.lo, y.lo}; y: rows {x1 y1 x3 y3} / halves {x.hi, y.hi}
+template <int LANES>
+__device__ __forceinline__ void swap_lanes(double &x, double &y) {
+    const unsigned long long xb = __builtin_bit_cast(unsigned long long, x), yb = __builtin_bit_cast(unsigned long long, y);
+    unsigned word[2][2];
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+        const unsigned xw = (unsigned)(xb >> (32 * h)), yw = (unsigned)(yb >> (32 * h));
+        const u32x2 s = LANES == 16 ? __builtin_amdgcn_permlane16_swap(xw, yw, false, false) : __builtin_amdgcn_permlane32_swap(xw, yw, false, false);
+        word[0][h] = s[0]; word[1][h] = s[1];
+    }
+    x = __builtin_bit_cast(double, (unsigned long long)word[0][1] << 32 | word[0][0]);
+    y = __builtin_bit_cast(double, (unsigned long long)word[1][1] << 32 | word[1][0]);
+}
+__device__ __forceinline__ double triangle_dot(const Tile &t, double e, float upper_half) {
+    double even = e, odd = e;
+    swap_lanes<16>(even, odd);                 // rows {0,0,2,2} and {1,1,3,3} of e
+    double crossed = odd, rest = even;
+    swap_lanes<32>(crossed, rest);             // rows {1,1,0,0}
+    double a = 0.0, b = 0.0;
+    fma16_rowbcast(a, even, t.p);
+    fma16_rowbcast(b, crossed, t.p + 32);
+    fma16_rowbcast(a, odd, t.p + 16);
+    double other = b;
+    swap_lanes<32>(b, other);
+    return a + (b + other) * (double)upper_half;
+}
+
 // ---- staging -----------------------------------------------------------------------------------------------------
 // A tile's 64 x 64 transitions, loaded four neighbouring elements a lane (sixteen lanes a row), converted, and turned
 // through LDS into lane <-> output position.  What bounds staging is the number of vector-memory instructions: a CU
@@ -360,9 +527,9 @@ template <> struct Quad<float> { typedef f32x4 V; __device__ __forceinline__ sta
 template <> struct Quad<__half> { typedef h16x4 V; __device__ __forceinline__ static float get(V v, int k) { return (float)v[k]; } };
 template <> struct Quad<bf16_t> { typedef u16x4 V; __device__ __forceinline__ static float get(V v, int k) { return __uint_as_float((unsigned)v[k] << 16); } };
 
-// one tile -> exp(E) 2^kShift2 in the wave's patch; `tiny` as in link_prob.  before / behind: how many elements the
+// one tile -> exp(E) 2^SHIFT in the wave's patch; `tiny` as in link_prob.  before / behind: how many elements the
 // tensor has in front of and behind the sample, where a load may reach (into places that are masked).
-template <typename TL>
+template <typename TL, int SHIFT>
 __device__ __forceinline__ void stage_tile(float *patch, const TL *links, int I, int J, int lane, int dir, int Lb, int translen, int last_index,
                                            int before, int behind, float tiny) {
     typedef typename Quad<TL>::V V;
@@ -417,7 +584,7 @@ __device__ __forceinline__ void stage_tile(float *patch, const TL *links, int I,
             for (int g = 0; g < 16; ++g) {
                 f32x4 w;
 #pragma unroll
-                for (int k = 0; k < 4; ++k) w[k] = __builtin_ldexpf(fast_exp2(Quad<TL>::get(raw[g], k) * kLog2e), kShift2);
+                for (int k = 0; k < 4; ++k) w[k] = __builtin_ldexpf(fast_exp2(Quad<TL>::get(raw[g], k) * kLog2e), SHIFT);
                 *reinterpret_cast<f32x4 *>(dst + 4 * g * kPatchPitch) = w;
             }
             return;
@@ -436,7 +603,7 @@ __device__ __forceinline__ void stage_tile(float *patch, const TL *links, int I,
                 const int ke = k_end(g);
 #pragma unroll
                 for (int k = 0; k < 4; ++k) {
-                    const float v = __builtin_ldexpf(fast_exp2(Quad<TL>::get(raw[g], k) * kLog2e), kShift2);
+                    const float v = __builtin_ldexpf(fast_exp2(Quad<TL>::get(raw[g], k) * kLog2e), SHIFT);
                     w[k] = valid(g, k, ke) ? v : 0.f;
                 }
                 *reinterpret_cast<f32x4 *>(dst + 4 * g * kPatchPitch) = w;
@@ -449,7 +616,7 @@ __device__ __forceinline__ void stage_tile(float *patch, const TL *links, int I,
         f32x4 w;
         const int ke = k_end(g);
 #pragma unroll
-        for (int k = 0; k < 4; ++k) w[k] = link_prob<true, kShift2>(Quad<TL>::get(raw[g], k), valid(g, k, ke), tiny);
+        for (int k = 0; k < 4; ++k) w[k] = link_prob<true, SHIFT>(Quad<TL>::get(raw[g], k), valid(g, k, ke), tiny);
         *reinterpret_cast<f32x4 *>(dst + 4 * g * kPatchPitch) = w;
     }
 }
@@ -468,6 +635,29 @@ __device__ __forceinline__ void read_patch(Tile &t, const float *patch, int lane
     asm volatile("" ::: "memory");
 }
 
+// the patch as the float64 products want it: register 16 g + j, lane 16 k + o: row 4 j + k, position 16 g + o
+__device__ __forceinline__ void read_patch_wide(Tile &t, const float *patch, int lane, int dir) {
+    asm volatile("" ::: "memory");
+    const int o = lane & 15, k = lane >> 4;
+    const float *const src = dir == 0 ? patch + k * kPatchPitch + o : patch + o * kPatchPitch + kBlk - 1 - k;
+    if (dir == 0) {
+#pragma unroll
+        for (int g = 0; g < 4; ++g)
+#pragma unroll
+            for (int j = 0; j < 16; ++j) t.p[16 * g + j] = src[4 * j * kPatchPitch + 16 * g];
+    } else {
+#pragma unroll
+        for (int g = 0; g < 4; ++g)
+#pragma unroll
+            for (int j = 0; j < 16; ++j) t.p[16 * g + j] = src[16 * g * kPatchPitch - 4 * j];
+    }
+    asm volatile("" ::: "memory");
+}
+
+__device__ __forceinline__ double pow2_clamped_wide(int x, int floor_exp) {   // 2^x for x <= 0; 2^floor_exp (or 0: floor -1023) below
+    const int c = x > floor_exp ? x : floor_exp;
+    return __builtin_bit_cast(double, (unsigned long long)(unsigned)(c + 1023) << 52);
+}
 __device__ __forceinline__ float pow2_clamped(int x, int floor_exp) {   // 2^x for x <= 0; 2^floor_exp (or 0: floor -127) below
     const int c = x > floor_exp ? x : floor_exp;
     return __builtin_bit_cast(float, (unsigned)(c + 127) << 23);

@@ -13,13 +13,12 @@
 //   alpha[t][node] = off[t][p/64] + hat[t][node]          (hat indexed by node, off by position block)
 // so the residuals keep full fp32 resolution no matter how negative the log-likelihood is.
 //
-// Three sweep implementations write this format:
-//   * sweep_chunks_group ("fast", float32): exp(E) is staged once into registers as 64x64 tiles (lane <-> output position,
-//     64 predecessors per tile).  Four steps at a time, what a block of positions receives from the blocks below it is
-//     a product on the matrix cores; the 64x64 triangle on its diagonal is walked step by step by one wave.  The tiles of
-//     one sweep are spread over a small pipeline of workgroups that hand the running vector on through global memory.
-//   * sweep_tiles_group ("wide", float64): the same tiles, every step a block-scaled linear-domain mat-vec done with DPP
-//     row-broadcast FMAs; re-does the samples whose float32 sweeps do not agree.
+// Two sweep implementations write this format:
+//   * sweep_chunks_group ("fast"): exp(E) is staged once into registers as 64x64 tiles (lane <-> output position, 64
+//     predecessors per tile).  Four steps at a time, what a block of positions receives from the blocks below it is a
+//     product on the matrix cores; the 64x64 triangle on its diagonal is walked step by step by one wave.  The tiles of one
+//     sweep are spread over a small pipeline of workgroups that hand the running vector on through global memory.
+//     In float32 first; in float64 ("wide") for the samples whose float32 sweeps do not agree.
 //   * dag_sweep_exact_kernel: every term evaluated in the log domain, one workgroup per sweep.
 //     Handles any size and any dynamic range; it re-does the samples the others leave.
 #include <atomic>
@@ -48,7 +47,7 @@ struct SweepArgs {
     // words (a group of the sample gave up waiting for its producer)
     int *sync;
     int C;             // workgroups per sweep (fast path)
-    int ndir;          // sweeps per sample in the tile kernel: always two, which bracket the result (see sweep_tiles_group)
+    int ndir;          // sweeps per sample in the tile kernel: always two, which bracket the result (see sweep_chunks_group)
     // The two tile sweeps of a sample: direction (0: alpha, 1: beta) and rounding side (0: every number too small
     // for the linear domain becomes 0, a lower bound of the sum over paths; 1: it becomes the smallest number the
     // domain holds, an upper bound).  With gradients {alpha/upper, beta/lower}, without {alpha/lower, alpha/upper}.
@@ -247,755 +246,48 @@ __global__ __launch_bounds__(NT) void dag_sweep_exact_kernel(SweepArgs a) {
 // Tile sweeps: register-resident exp(E) tiles, pipelined workgroups
 // ================================================================================================
 
-// ---- the wide variant: the same sweep with float64 linear-domain numbers --------------------------------------
-// What the float32 sweep cannot hold is, almost always, a cell far under the maximum of its block or a block far
-// under its neighbours (inputs whose best prefixes are not the prefixes of the best paths); a float64 number has
-// room for 1300 nats under its scale where a float32 number has 126.  The wide variant keeps exp(residual), the
-// tile sums, the block factors and their sums in float64; the staged transitions stay float32 registers (the
-// register file holds no float64 tiles) and are converted as they are used: v_cvt_f64_f32 + v_fmac_f64 with the
-// same DPP row broadcast, two instructions per pair-update instead of one.  It runs, as a second launch, on the
-// samples whose float32 sweeps did not agree, and leaves to the log-domain kernel what it cannot settle either.
-constexpr int kShiftWide = 850;   // float64 numbers carry 2^850: 2^(850 + 127 + 10) < 2^1024 above, 2^-1022 below
-
-// acc += sum_{r<16} e[lane r of this lane's 16-lane row] * (double)p[r]
-__device__ __forceinline__ void fma16_rowbcast(double &acc, double e, const float *p) {
-    double t0, t1;
-    asm("s_nop 1\n\t"
-        "v_cvt_f64_f32 %1, %4\n\t"
-        "v_cvt_f64_f32 %2, %5\n\t"
-        "v_fmac_f64_dpp %0, %3, %1 row_newbcast:0 row_mask:0xf bank_mask:0xf\n\t"
-        "v_cvt_f64_f32 %1, %6\n\t"
-        "v_fmac_f64_dpp %0, %3, %2 row_newbcast:1 row_mask:0xf bank_mask:0xf\n\t"
-        "v_cvt_f64_f32 %2, %7\n\t"
-        "v_fmac_f64_dpp %0, %3, %1 row_newbcast:2 row_mask:0xf bank_mask:0xf\n\t"
-        "v_cvt_f64_f32 %1, %8\n\t"
-        "v_fmac_f64_dpp %0, %3, %2 row_newbcast:3 row_mask:0xf bank_mask:0xf\n\t"
-        "v_cvt_f64_f32 %2, %9\n\t"
-        "v_fmac_f64_dpp %0, %3, %1 row_newbcast:4 row_mask:0xf bank_mask:0xf\n\t"
-        "v_cvt_f64_f32 %1, %10\n\t"
-        "v_fmac_f64_dpp %0, %3, %2 row_newbcast:5 row_mask:0xf bank_mask:0xf\n\t"
-        "v_cvt_f64_f32 %2, %11\n\t"
-        "v_fmac_f64_dpp %0, %3, %1 row_newbcast:6 row_mask:0xf bank_mask:0xf\n\t"
-        "v_cvt_f64_f32 %1, %12\n\t"
-        "v_fmac_f64_dpp %0, %3, %2 row_newbcast:7 row_mask:0xf bank_mask:0xf\n\t"
-        "v_cvt_f64_f32 %2, %13\n\t"
-        "v_fmac_f64_dpp %0, %3, %1 row_newbcast:8 row_mask:0xf bank_mask:0xf\n\t"
-        "v_cvt_f64_f32 %1, %14\n\t"
-        "v_fmac_f64_dpp %0, %3, %2 row_newbcast:9 row_mask:0xf bank_mask:0xf\n\t"
-        "v_cvt_f64_f32 %2, %15\n\t"
-        "v_fmac_f64_dpp %0, %3, %1 row_newbcast:10 row_mask:0xf bank_mask:0xf\n\t"
-        "v_cvt_f64_f32 %1, %16\n\t"
-        "v_fmac_f64_dpp %0, %3, %2 row_newbcast:11 row_mask:0xf bank_mask:0xf\n\t"
-        "v_cvt_f64_f32 %2, %17\n\t"
-        "v_fmac_f64_dpp %0, %3, %1 row_newbcast:12 row_mask:0xf bank_mask:0xf\n\t"
-        "v_cvt_f64_f32 %1, %18\n\t"
-        "v_fmac_f64_dpp %0, %3, %2 row_newbcast:13 row_mask:0xf bank_mask:0xf\n\t"
-        "v_cvt_f64_f32 %2, %19\n\t"
-        "v_fmac_f64_dpp %0, %3, %1 row_newbcast:14 row_mask:0xf bank_mask:0xf\n\t"
-        "s_nop 0\n\t"
-        "v_fmac_f64_dpp %0, %3, %2 row_newbcast:15 row_mask:0xf bank_mask:0xf"
-        : "+v"(acc), "=&v"(t0), "=&v"(t1)
-        : "v"(e), "v"(p[0]), "v"(p[1]), "v"(p[2]), "v"(p[3]), "v"(p[4]), "v"(p[5]), "v"(p[6]), "v"(p[7]),
-          "v"(p[8]), "v"(p[9]), "v"(p[10]), "v"(p[11]), "v"(p[12]), "v"(p[13]), "v"(p[14]), "v"(p[15]));
-}
-__device__ __forceinline__ double tile_dot(const Tile &t, double e0, double e1, double e2, double e3) {
-    double a = 0.0;
-    fma16_rowbcast(a, e0, t.p);
-    fma16_rowbcast(a, e1, t.p + 16);
-    fma16_rowbcast(a, e2, t.p + 32);
-    fma16_rowbcast(a, e3, t.p + 48);
-    return a;
-}
-// the same with the tile's last NT rows held elsewhere
-template <int NT>
-__device__ __forceinline__ double tile_dot_tail(const Tile &t, const float (&tail)[NT], double e0, double e1, double e2, double e3) {
-    static_assert(NT > 0 && NT <= 16, "");
-    float last[16];
-#pragma unroll
-    for (int u = 0; u < 16; ++u) last[u] = u < 16 - NT ? t.p[48 + u] : tail[u - (16 - NT)];
-    double a = 0.0;
-    fma16_rowbcast(a, e0, t.p);
-    fma16_rowbcast(a, e1, t.p + 16);
-    fma16_rowbcast(a, e2, t.p + 32);
-    fma16_rowbcast(a, e3, last);
-    return a;
-}
-template <int U0>
-__device__ __forceinline__ void scaled_sum4(double &acc, double f, double v0, double v1, double v2, double v3) {
-    static_assert(U0 % 4 == 0 && U0 >= 0 && U0 < 16, "");
-    if constexpr (U0 == 0) acc = 0.0;
-    asm("s_nop 1\n\t"
-        "v_fmac_f64_dpp %0, %1, %2 row_newbcast:%c6 row_mask:0xf bank_mask:0xf\n\t"
-        "v_fmac_f64_dpp %0, %1, %3 row_newbcast:%c7 row_mask:0xf bank_mask:0xf\n\t"
-        "v_fmac_f64_dpp %0, %1, %4 row_newbcast:%c8 row_mask:0xf bank_mask:0xf\n\t"
-        "v_fmac_f64_dpp %0, %1, %5 row_newbcast:%c9 row_mask:0xf bank_mask:0xf"
-        : "+v"(acc) : "v"(f), "v"(v0), "v"(v1), "v"(v2), "v"(v3), "n"(U0), "n"(U0 + 1), "n"(U0 + 2), "n"(U0 + 3));
-}
-
-// The float64 linear-domain numbers of the wide sweeps.
-struct Lin {
-    using T = double;
-    static constexpr float kFacFloor = -1022.f;
-    __device__ static __forceinline__ double tiny() { return 2.2250738585072014e-308; }          // 2^-1022
-    __device__ static __forceinline__ double flushed_sum() { return 9.332636185032189e-302; }    // 2^-1000
-    // 2^(x + shift) for a float x (any value; -inf gives 0, a NaN stays one): the fraction through v_exp_f32, the
-    // integer part through the exponent field
-    __device__ static __forceinline__ double exp2_with(float x, int shift) {
-        const float n = __builtin_floorf(x);
-        const double m = (double)fast_exp2(x - n);
-        const double r = __builtin_ldexp(m, (int)__builtin_fmaxf(n, -4000.f) + shift);
-        return !(x <= -3000.f) ? r : 0.0;
-    }
-    // the same for a float64 argument (scale arithmetic of the wide sweeps: differences of offsets hundreds of nats
-    // apart, whose float32 rounding, repeated every step, would add up along a path)
-    __device__ static __forceinline__ double exp2_with(double x, int shift) {
-        const double n = __builtin_floor(x);
-        const double m = (double)fast_exp2((float)(x - n));
-        const double r = __builtin_ldexp(m, (int)(n > -4000.0 ? n : -4000.0) + shift);
-        return !(x <= -3000.0) ? r : 0.0;
-    }
-    // y * 2^x with the integer part of x going into y's exponent field (2^x by itself may lie outside the float64
-    // range where the product does not); x = -inf gives 0
-    __device__ static __forceinline__ double times_exp2(double y, double x) {
-        const double n = __builtin_floor(x);
-        const double m = (double)fast_exp2((float)(x - n));
-        const double r = __builtin_ldexp(y * m, (int)(n > -8000.0 ? n : -8000.0));
-        return !(x <= -6000.0) ? r : 0.0;
-    }
-    __device__ static __forceinline__ double exp2s(float x) { return exp2_with(x, kShiftWide); }
-    // log2(y) minus the shift of a float64 number and that of a staged transition: the exponent exactly, the logarithm of the
-    // fraction (in [-1, 0]) from v_log_f32
-    __device__ static __forceinline__ double log2u_wide(double y) {
-        return (double)(__builtin_amdgcn_frexp_exp(y) - (kShiftWide + kShiftLinksWide)) + (double)fast_log2((float)__builtin_amdgcn_frexp_mant(y));
-    }
-};
-
-constexpr int kPartBlocks = 12;   // a group never owns more blocks: every block but the first has >= 2 tiles
-constexpr int kPartRows = 16;     // partial-sum rows reserved per owned block (tiles per block <= 16)
-// LDS of the step loop.  First the linear-domain numbers, indexed in elements of the sweep's number type:
-constexpr int kEvEbuf = 0;                                              // [2][16][64] exp(residual), by position
-constexpr int kEvPart = kEvEbuf + 2 * kMaxBlocksFast * kBlk;            // [12][16][64] per-tile partial sums
-constexpr int kEvNowhere = kEvPart + kPartBlocks * kPartRows * kBlk;    // [64] where a wave's unused tile slots "write their partial sums"
-constexpr int kEvCount = kEvNowhere + kBlk;
-// then, in floats from the start of the dynamic segment:
-struct StepLds {
-    static constexpr int kRelb = kEvCount * 2;              // [2][16] block offsets rel. to the reference (float; double in the wide variant)
-    // landing areas of the asynchronous global -> LDS copies (one slot per consuming wave), double-buffered by step parity
-    static constexpr int kStageM = kRelb + 2 * kMaxBlocksFast * 2;   // [2][8 waves][2][64] dwords: match rows of each wave's own blocks (raw elements)
-    static constexpr int kStageF = kStageM + 2 * kTileWaves * 2 * kBlk;  // [2][8 waves][2][64] floats: table residuals of the wave's foreign blocks
-    static constexpr int kStageO = kStageF + 2 * kTileWaves * 2 * kBlk;  // [2][64] dwords: the table's offset row (16 doubles, padded)
-    static constexpr int kStageP = kStageO + 2 * kBlk;                    // [2][64] dwords: snapshot of the progress word of the group below
-    static constexpr int kLastV = kStageP + 2 * kBlk;                    // [8 waves][64] the values of the last step (for the read-out)
-    static constexpr int kLastC = kLastV + kTileWaves * kBlk * 2;   // [8 waves] doubles: the reference they are relative to
-    // (kLastV holds float64 values in the wide variant: twice the room)
-    // the wide variant keeps the last rows of every wave's third tile here and reads them back in every step: the
-    // registers they would occupy are what its float64 temporaries of phase B need
-    static constexpr int kTailRows = 12;
-    static constexpr int kTail = kLastC + 2 * kTileWaves;                // [8 waves][kTailRows][64] floats
-    static constexpr int kStepFloats = kTail + kTileWaves * kTailRows * kBlk;
-};
-
-// Memory traffic of the loop is asynchronous and off the critical path.  The last wave of the
-// workgroup is the fetcher (it holds no tiles whenever the group has at most 21): during phase A of
-// step s, while the other waves run their tiles, it requests (global -> LDS copies) what phase B of step
-// s + 1 needs -- the match rows of every owned block and, for consumer groups, the table rows of the
-// foreign blocks and a snapshot of the producer's progress word -- and only waits for what it requested
-// a whole step earlier.  Nobody waits for a load that was issued in the same step, unless a consumer
-// has caught up with its producer; then the fetcher polls the progress word (bounded).
-//
-// Inter-workgroup hand-over of the running vector (groups of one sweep form a one-way pipeline):
-//  * a producer writes its table rows (hat, off) with agent-scope write-through stores; a step
-//    later, when every wave has seen those stores complete, it raises its progress word;
-//  * a consumer's fetcher copies the rows of a step once a snapshot of that word covers the step.
-// Every wait is bounded: on expiry the sample is marked for the exact kernel and the group leaves.
-//
-// Leaving: every workgroup counts itself out of its sample and out of the launch.  The last one of a
-// sample compares the two read-outs of the tile sweeps, sets the sample's flag (1 = the log-domain kernel
-// must redo it) and clears the sample's pipeline words; the last one of the launch clears the ticket
-// counter -- so the words are all zero again when the launch is over and need no fill in front of it.
-//
-// The step loop is issue-bound (two waves per SIMD, a few hundred instructions per wave and step
-// around the 64 FMAs of each tile), so everything that does not change from step to step -- LDS
-// addresses, table offsets, the tile's band limits -- is computed before the loop, the loop body is
-// instantiated for both parities of the double buffers (immediate LDS offsets), and the LDS reads
-// of a phase are issued together.
-template <typename TM, typename TL>
-__device__ __forceinline__ void sweep_tiles_group(const SweepArgs &a, const int b, const int slot, const int g, float *lds_raw,
-                                                  int *gstart, int *s_abort_p) {
-    using LN = Lin;
-    using EV = double;                  // exp(residual), tile sums, block factors
-    // A cell's value relative to the step's reference: float, or double in the wide variant -- its samples are the
-    // ones whose values lie hundreds of nats from their reference, where a float32 value is 3e-5 coarse, and the
-    // two read-outs of a sample can only be held to 5e-5 of each other if they are finer than that.
-    using VT = double;
-    using LD = StepLds;
-    constexpr int kLdsRelb = LD::kRelb, kLdsStageM = LD::kStageM, kLdsStageF = LD::kStageF, kLdsStageO = LD::kStageO,
-                  kLdsStageP = LD::kStageP, kLdsLastV = LD::kLastV, kLdsLastC = LD::kLastC, kLdsStepFloats = LD::kStepFloats;
-    // slot: which of the sample's two sweeps (its tables, pipeline words and read-out); dir: its direction;
-    // upper: its rounding side.  The linear domain flushes what is more than 126 nats under its scale -- a
-    // transition, a cell under its block maximum, a block under the largest of its neighbours, a product of such
-    // numbers.  The lower sweep lets all of that become 0, so its read-out never exceeds log Z; the upper sweep
-    // puts the smallest normal number (or a constant that covers every flushed product) in its place, so its
-    // read-out never falls short of log Z.  The sample's result stands when the two read-outs agree; what was
-    // flushed then carried no mass that matters, wherever it was flushed.
-    const int dir = a.rev[slot];
-    const bool upper = a.upper[slot] != 0;
-    // Dynamic LDS, used twice: while the tiles are staged it holds one transpose patch per wave
-    // ([kTileWaves][kBlk][kBlk+1], beta tiles only); after the barrier that ends staging it holds the
-    // step buffers (kLds* above).
-    float (*stage)[kBlk][kBlk + 1] = reinterpret_cast<float (*)[kBlk][kBlk + 1]>(lds_raw);
-    int &s_abort = *s_abort_p;
-    const int tid = threadIdx.x, lane = tid & (kWave - 1);
-    const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
-    const int C = a.C;
-    int *risk = a.sync + 16 + a.ndir * a.B * C + a.B + b;
-
-    // (taken through opaque_uniform: otherwise the compiler re-reads them from the argument block inside the
-    //  step loop, a scalar-memory round trip on the critical path, instead of keeping them in registers)
-    const int L = opaque_uniform(a.L), T = a.T, translen = a.translen, NBK = opaque_uniform(a.NBK);
-    const int Lb = (int)a.out_len[b], Tb = (int)a.tgt_len[b];
-    if (!lengths_ok(Lb, Tb, L, T)) {
-        if (g == 0 && tid == 0) { a.logz[slot * a.B + b] = (double)DAGX_NEG_INF; if (slot == a.loss_dir) a.loss[b] = DAGX_NEG_INF; store_agent(a.zfast + slot * a.B + b, (double)DAGX_NEG_INF); }
-        return;
-    }
-    const TM *match = static_cast<const TM *>(a.match) + (int64_t)b * a.ms0;
-    const TL *links = static_cast<const TL *>(a.links) + (int64_t)b * L * translen;
-    float *hat = a.hat[slot] + (int64_t)b * T * L;
-    double *off = a.off[slot] + (int64_t)b * T * NBK;
-    int *prog = a.sync + 16 + (slot * a.B + b) * C;
-
-    const int slack = Lb - Tb;
-    const int NBb = (Lb + kBlk - 1) / kBlk;
-    const int W = (translen + kBlk - 1) / kBlk;
-    if (tid <= C) gstart[tid] = a.plan.gtab[NBb][tid];
-    __syncthreads();
-    const int jb0 = __builtin_amdgcn_readfirstlane(gstart[g]), jb1 = __builtin_amdgcn_readfirstlane(gstart[g + 1]);
-    int last_group = 0;
-    for (int q = 0; q < C; ++q) if (gstart[q + 1] > gstart[q]) last_group = q;
-    last_group = __builtin_amdgcn_readfirstlane(last_group);
-    if (jb0 >= jb1) return;  // nothing to do for this group (short sample); nobody waits on it
-    const int nblk = jb1 - jb0;
-    const int flo = tile_ilo(jb0, W);  // lowest foreign block this group ever reads
-    const bool producer = g < last_group;
-    const bool unlimited = W >= NBb - 1;   // every lower block is a predecessor block
-    if (nblk > kPartBlocks) {  // cannot happen with the host's partition; leave the sample to the exact kernel
-        if (tid == 0) { store_agent(risk, 1); store_agent(prog + g, 1 << 30); }
-        return;
-    }
-
-    // ---- my tiles: enumerated block by block; each wave takes a contiguous run of them ----
-    int ntile = 0;
-    for (int Jb = jb0; Jb < jb1; ++Jb) ntile += Jb - tile_ilo(Jb, W) + 1;
-    // The last wave fetches (see above) and takes tiles only when the others cannot hold them all.  The
-    // tiles are dealt out evenly; the odd ones go first to wave 3, whose SIMD it shares with the
-    // fetcher, then to waves 0, 1, 2, 4, ...
-    const int nwork = ntile <= kTilesPerWave * (kTileWaves - 1) ? kTileWaves - 1 : kTileWaves;
-    int my_first = 0, my_count = 0;
-    {
-        const int base = ntile / nwork, rem = ntile % nwork;
-        int first = 0;
-        for (int w = 0; w < kTileWaves; ++w) {
-            const int rank = nwork == kTileWaves ? w : (w == 3 ? 0 : (w < 3 ? w + 1 : w));
-            const int cnt = w < nwork ? base + (rank < rem ? 1 : 0) : 0;
-            if (w == wave) { my_first = first; my_count = cnt; }
-            first += cnt;
-        }
-    }
-    int my_I[kTilesPerWave], my_J[kTilesPerWave];
-    bool my_ok[kTilesPerWave];
-#pragma unroll
-    for (int sl = 0; sl < kTilesPerWave; ++sl) { my_I[sl] = 0; my_J[sl] = jb0; my_ok[sl] = false; }
-    {
-        int q = 0;
-        for (int Jb = jb0; Jb < jb1; ++Jb)
-            for (int I = tile_ilo(Jb, W); I <= Jb; ++I, ++q) {
-                const int sl = q - my_first;
-                if (sl >= 0 && sl < my_count) {
-#pragma unroll
-                    for (int u = 0; u < kTilesPerWave; ++u)
-                        if (u == sl) { my_I[u] = I; my_J[u] = Jb; my_ok[u] = true; }
-                }
-            }
-    }
-    Tile t0, t1, t2;
-    // What a finite transition below the staged range becomes: 0 in a lower sweep, the smallest number the staged
-    // range holds in an upper sweep (exp(-126) under a certain transition in the float32 sweeps, exp(-175) in the
-    // wide ones).
-    constexpr int kLinkShift = kShiftLinksWide;
-    const float tiny = !upper ? 0.f : kTinyStored;   // (2^-126 as stored: at least any transition that is not staged, in either variant)
-    if (my_ok[0]) load_tile<true, 16, TL, kLinkShift>(t0, links, my_I[0], my_J[0], lane, dir, Lb, translen, stage[wave], tiny);
-    if (my_ok[1]) load_tile<true, 16, TL, kLinkShift>(t1, links, my_I[1], my_J[1], lane, dir, Lb, translen, stage[wave], tiny);
-    if (my_ok[2]) load_tile<true, 16, TL, kLinkShift>(t2, links, my_I[2], my_J[2], lane, dir, Lb, translen, stage[wave], tiny);
-    __syncthreads();   // every wave is done with its transpose patch: the LDS now holds the step buffers
-
-    EV *const ebuf = reinterpret_cast<EV *>(lds_raw) + kEvEbuf;   // [parity][block][64]
-    double *const relb64 = reinterpret_cast<double *>(lds_raw + kLdsRelb);   // [parity][block]
-    constexpr int kEbufPar = kMaxBlocksFast * kBlk;   // floats between the two parities of ebuf
-
-    // ---- step 0 is known to every group: only position 0 is alive ----
-    const int t_first = dir ? Tb - 1 : 0, node_first = dir ? Lb - 1 : 0;
-    const float m0 = to_float(match[(int64_t)t_first * a.ms1 + (int64_t)node_first * a.ms2]);
-    const bool alive0 = m0 > DAGX_NEG_INF;
-    double cref = alive0 ? (double)m0 : 0.0;  // absolute value the relb / v numbers of this step are relative to
-    for (int q = tid; q < kLdsStepFloats; q += kTileWaves * kWave) lds_raw[q] = 0.f;   // ebuf, part (rows no tile writes stay 0)
-    __syncthreads();
-    constexpr int kTailRows = LD::kTailRows, kTailFirst = kBlk - kTailRows;
-    float *const tail_lane = lds_raw + LD::kTail + wave * (kTailRows * kBlk) + lane;   // (read and written by this wave alone)
-#pragma unroll
-    for (int u = 0; u < kTailRows; ++u) tail_lane[u * kBlk] = my_ok[2] ? t2.p[kTailFirst + u] : 0.f;
-    if (tid == 0 && alive0) ebuf[0] = LN::exp2s(0.f);
-    if (tid < 2 * kMaxBlocksFast) {
-        relb64[tid] = (tid == 0 && alive0) ? 0.0 : (double)DAGX_NEG_INF;
-    }
-    for (int ob = wave; ob < nblk; ob += kTileWaves) {  // own blocks of the first row of the table
-        const int Jb = jb0 + ob, p = Jb * kBlk + lane;
-        if (p < Lb) store_agent(hat + (int64_t)t_first * L + (dir ? Lb - 1 - p : p), (p == 0 && alive0) ? 0.f : DAGX_NEG_INF);
-        if (lane == 0) store_agent(off + (int64_t)t_first * NBK + Jb, (Jb == 0 && alive0) ? (double)m0 : (double)DAGX_NEG_INF);
-    }
-    if (Tb == 1 && tid == 0 && jb0 == 0) {
-        const double z = (Lb == 1 && alive0) ? (double)m0 : (double)DAGX_NEG_INF;
-        a.logz[slot * a.B + b] = z; if (slot == a.loss_dir) a.loss[b] = (float)z; store_agent(a.zfast + slot * a.B + b, z);
-    }
-
-    // Table rows are addressed as (uniform base) + 32-bit byte offset so that no 64-bit per-lane
-    // addresses stay live across the step loop (every register is needed for the tiles).
-    const char *hat_c = reinterpret_cast<const char *>(hat);
-    const char *off_c = reinterpret_cast<const char *>(off);
-    const char *match_c = reinterpret_cast<const char *>(match);
-    auto hat_at = [&](int trow, int node) -> float * {
-        return reinterpret_cast<float *>(const_cast<char *>(hat_c) + (unsigned)(trow * L + node) * 4u);
-    };
-    auto off_at = [&](int trow, int blk) -> double * {
-        return reinterpret_cast<double *>(const_cast<char *>(off_c) + (unsigned)(trow * NBK + blk) * 8u);
-    };
-    const int ms1 = (int)a.ms1, ms2 = (int)a.ms2;   // the host checked that match indices fit 32 bits
-
-    // ---- loop invariants of this wave ----
-    // Wave-uniform element offsets into the LDS (kept in scalar registers; per-lane addresses are
-    // formed from them inside the loop -- there is no vector register to spare for them):
-    // where a tile reads its e values and writes its partial sum, and the steps at which its output
-    // block lies inside the band (s_lo <= s <= s_hi).
-    int e_off[kTilesPerWave], part_off[kTilesPerWave], s_lo[kTilesPerWave], s_hi[kTilesPerWave];
-#pragma unroll
-    for (int sl = 0; sl < kTilesPerWave; ++sl) {
-        e_off[sl] = __builtin_amdgcn_readfirstlane(kEvEbuf + my_I[sl] * kBlk);
-        part_off[sl] = __builtin_amdgcn_readfirstlane(kEvPart + ((my_J[sl] - jb0) * kPartRows + (my_I[sl] - tile_ilo(my_J[sl], W))) * kBlk);
-        s_lo[sl] = __builtin_amdgcn_readfirstlane(my_J[sl] * kBlk - slack);
-        s_hi[sl] = __builtin_amdgcn_readfirstlane(my_J[sl] * kBlk + kBlk - 1);
-        // a slot without a tile is never "in the band" and stores its zero where nobody reads: no test of its own
-        // in the loop (every test there is an instruction slot, and its operands live in scarce scalar registers)
-        if (!my_ok[sl]) { part_off[sl] = kEvNowhere; s_lo[sl] = 0x7fffffff; s_hi[sl] = -1; }
-    }
-    const float fac_floor = upper ? LN::kFacFloor : DAGX_NEG_INF;
-    // The direction of rounding as numbers, not as a condition (a wave-uniform condition is a pair of scalar registers,
-    // and the loop has none to spare: it came back from a vector register's lanes at every use): what a flushed live
-    // cell becomes, and what is added to every block sum for the products that may have been flushed.
-    EV tiny_up = upper ? LN::tiny() : (EV)0, flush_up = upper ? LN::flushed_sum() : (EV)0;
-    asm volatile("" : "+v"(tiny_up), "+v"(flush_up));
-    float *const lds_lane = lds_raw + lane;
-    const EV *const ev_l15 = reinterpret_cast<const EV *>(lds_raw) + (lane & 15);   // every 16-lane row addresses the same 16 values
-    EV *const ev_lane = reinterpret_cast<EV *>(lds_raw) + lane;
-    // the block this wave owns in phase B (a second one, wave + 8, is handled without look-ahead)
-    const bool owner = wave < nblk;
-    const int Jown = jb0 + (owner ? wave : 0);
-    const int p_own = Jown * kBlk + lane;
-    const int node_own = dir ? Lb - 1 - p_own : p_own;
-    const int nt_own = Jown - tile_ilo(Jown, W) + 1;
-    const int own_part_off = __builtin_amdgcn_readfirstlane(kEvPart + (owner ? wave : 0) * kPartRows * kBlk);
-    // ---- staging slots: the match rows of own blocks wave and wave + 8, the table rows of two foreign blocks
-    //      (converted by this wave in phase B; dealt from the last wave down, so that the first waves, which own
-    //      blocks, rarely have a conversion in front of their own block's chain of dependent steps), one offset row ----
-    const unsigned lds_base = (unsigned)reinterpret_cast<uintptr_t>(lds_raw);   // LDS byte address of the dynamic segment
-    constexpr int kFetchSlots = 2;
-    const bool consumer = flo < jb0;
-    int f_blk[kFetchSlots];
-#pragma unroll
-    for (int u = 0; u < kFetchSlots; ++u) {
-        const int fb = flo + (kTileWaves - 1 - wave) + kTileWaves * u;
-        f_blk[u] = fb < jb0 ? fb : -1;
-    }
-    const int *below = prog + (g > 0 ? g - 1 : 0);
-    auto stage_m_of = [&](int par, int w, int u) -> int { return kLdsStageM + ((par * kTileWaves + w) * 2 + u) * kBlk; };
-    auto stage_f_of = [&](int par, int w, int u) -> int { return kLdsStageF + ((par * kTileWaves + w) * 2 + u) * kBlk; };
-    auto stage_m = [&](int par, int u) -> int { return stage_m_of(par, wave, u); };
-    auto stage_f = [&](int par, int u) -> int { return stage_f_of(par, wave, u); };
-    auto stage_o = [&](int par) -> int { return kLdsStageO + par * kBlk; };
-    auto stage_p = [&](int par) -> int { return kLdsStageP + par * kBlk; };
-    // ---- the fetcher (last wave): everything phase B reads from memory, requested one step ahead ----
-    const bool fetcher = wave == kTileWaves - 1;
-    int seen = 0;          // latest progress value of the group below known to the fetcher
-    int rows_issued = 0;   // the foreign table rows of steps <= rows_issued have been requested
-    int snapshot = 0;      // the producer's progress word as copied a step ago: what every wave of the group acts on
-    // A copy's address is (scalar base of the row and block) + (per-lane offset inside a block, the same for
-    // every block, recomputed each step from the lane number: no register is held across the loop for it);
-    // only the sample's last, partial block needs per-lane clamping (to its last node).  A wave issues about
-    // one instruction of any kind per five cycles, so what counts here is the number of instructions per copy:
-    // the forms used in the step loop (issue_*_unrolled) are straight-line code with the LDS destinations as
-    // constants and the block bases advanced by scalar adds.
-    const int nfull = min(nblk, Lb / kBlk - jb0);   // owned blocks that are complete (all but possibly the last)
-    const long long m_step = (long long)(dir ? -kBlk : kBlk) * ms2 * (long long)sizeof(TM);   // from one block's base to the next
-    const long long m_first = (long long)(dir ? Lb - kBlk - jb0 * kBlk : jb0 * kBlk) * ms2 * (long long)sizeof(TM);
-    const long long h_step = (long long)(dir ? -kBlk : kBlk) * 4;
-    const long long h_first = (long long)(dir ? Lb - kBlk - flo * kBlk : flo * kBlk) * 4;
-    const unsigned lds_base_u = opaque_uniform((int)lds_base);
-    auto match_partial = [&](const int par, const int ob, const unsigned long long mrow) __attribute__((always_inline)) {
-        const int pm = (jb0 + ob) * kBlk + lane, pmc = pm < Lb ? pm : Lb - 1;
-        dma_elem_u<TM>(lds_base_u + (unsigned)stage_m_of(par, ob & (kTileWaves - 1), ob / kTileWaves) * 4u, mrow,
-                       (unsigned)((dir ? Lb - 1 - pmc : pmc) * ms2) * (unsigned)sizeof(TM));
-    };
-    auto issue_match_unrolled = [&](auto parity, const int s2) __attribute__((always_inline)) {
-        constexpr int PAR = decltype(parity)::value;
-        const int row = dir ? Tb - 1 - s2 : s2;
-        const unsigned long long mrow = uniform_address(match_c + (unsigned)(row * ms1) * (unsigned)sizeof(TM));
-        const unsigned lane_off = (unsigned)((dir ? kBlk - 1 - lane : lane) * ms2) * (unsigned)sizeof(TM);
-        unsigned long long base = mrow + (unsigned long long)m_first;
-#pragma unroll
-        for (int ob = 0; ob < kPartBlocks; ++ob) {
-            if (ob >= nfull) break;
-            dma_elem_u<TM>(lds_base_u + (unsigned)stage_m_of(PAR, ob & (kTileWaves - 1), ob / kTileWaves) * 4u, base, lane_off);
-            base += (unsigned long long)m_step;
-        }
-        if (nfull < nblk) match_partial(PAR, nfull, mrow);
-    };
-    auto issue_rows = [&](const int s2) __attribute__((always_inline)) {    // table rows of the foreign blocks (all complete) for step s2
-        const int row = dir ? Tb - 1 - s2 : s2, par = s2 & 1;
-        unsigned long long base = uniform_address(hat_c + (unsigned)(row * L) * 4u) + (unsigned long long)h_first;
-        const unsigned lane_off = (unsigned)(dir ? kBlk - 1 - lane : lane) * 4u;
-        for (int q = 0; q < jb0 - flo; ++q, base += (unsigned long long)h_step)
-            dma_dword_agent_u(lds_base_u + (unsigned)stage_f_of(par, kTileWaves - 1 - (q & (kTileWaves - 1)), q / kTileWaves) * 4u, base, lane_off);
-        dma_dword_agent_u(lds_base_u + (unsigned)stage_o(par) * 4u, uniform_address(off_c + (unsigned)(row * NBK) * 8u),
-                          (unsigned)(lane < 2 * NBK ? lane : 2 * NBK - 1) * 4u);
-        rows_issued = s2;
-    };
-    // called in phase A of step s: make sure what phase B of step s reads has landed, request step s + 1
-    auto fetch_step = [&](auto parity_next, const int s) __attribute__((always_inline)) {
-        // parity_next: the buffers of step s + 1 (those of step s have the other parity)
-        constexpr int PN = decltype(parity_next)::value;
-        wait_vmem_all();   // everything requested a step ago
-        const bool need_rows = consumer && s < Tb - 1;
-        if (need_rows) {
-            snapshot = __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, lds_raw[stage_p(s & 1)]));   // requested a step ago
-            if (snapshot > seen) seen = snapshot;
-            if (rows_issued < s) {   // not requested yet: the producer is less than two steps ahead, poll its word
-                int spins = 0;
-                while (seen < s) {   // the rows of step s are published once the word reaches s
-                    seen = __builtin_amdgcn_readfirstlane(load_agent(below));
-                    if (seen >= s) break;
-                    __builtin_amdgcn_s_sleep(2);
-                    if (++spins > kSpinLimit) { s_abort = 1; break; }
-                }
-                if (seen >= s) { issue_rows(s); wait_vmem_all(); }
-            }
-        }
-        if (s + 1 < Tb) {
-            if (!consumer) issue_match_unrolled(parity_next, s + 1);   // (a consumer group's waves request their own rows)
-            if (consumer && s + 1 < Tb - 1) {
-                // The waves of a consumer group each request the table row of their own foreign block for step
-                // s + 1 (own_requests), all on the same evidence: the snapshot of the producer's progress word that
-                // was requested a step ago (every copy of a step has landed before the step's last barrier: the
-                // fetcher, too, waits for its requests at the top of phase B).  Here only what the waves share: the
-                // offsets of that row, and the next snapshot.
-                if (snapshot >= s + 1) {
-                    const int row = dir ? Tb - 2 - s : s + 1;
-                    dma_dword_agent_u(lds_base_u + (unsigned)stage_o(PN) * 4u, uniform_address(off_c + (unsigned)(row * NBK) * 8u),
-                                      (unsigned)(lane < 2 * NBK ? lane : 2 * NBK - 1) * 4u);
-                    rows_issued = s + 1;
-                }
-                dma_dword_agent(lds_base_u + (unsigned)stage_p(PN) * 4u, below, 0u);
-            }
-        }
-    };
-    // Every wave of a consumer group, in phase A of step s: request what its own phase B of step s + 1 reads -- the
-    // match row of the block(s) it owns and, once the fetcher's published progress covers step s + 1, the table
-    // row of its foreign block(s).  One or two copies per wave instead of all of them queued behind each other in
-    // the fetcher, whose arrival at the barrier was what the group's tile waves waited for.  A wave consumes only
-    // what it requested itself, after waits of its own (top of phase B; the fetcher at the top of its fetch).
-    auto own_requests = [&](auto parity_next, const int s) __attribute__((always_inline)) {
-        constexpr int PN = decltype(parity_next)::value;
-        if (s + 1 >= Tb) return;
-        const int row = dir ? Tb - 2 - s : s + 1;
-        if (owner) {
-            const unsigned long long mrow = uniform_address(match_c + (unsigned)(row * ms1) * (unsigned)sizeof(TM));
-#pragma unroll
-            for (int u = 0; u < 2; ++u) {
-                if (u == 1 && wave + kTileWaves >= nblk) break;
-                const int pm = p_own + u * kTileWaves * kBlk, pmc = pm < Lb ? pm : Lb - 1;
-                dma_elem_u<TM>(lds_base_u + (unsigned)stage_m(PN, u) * 4u, mrow,
-                               (unsigned)((dir ? Lb - 1 - pmc : pmc) * ms2) * (unsigned)sizeof(TM));
-            }
-        }
-        if (s + 1 < Tb - 1 && f_blk[0] >= 0) {
-            const int known = __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, lds_raw[stage_p(PN ^ 1)]));
-            if (known >= s + 1) {
-                const unsigned long long hrow = uniform_address(hat_c + (unsigned)(row * L) * 4u);
-                int ln = lane;   // (redone every step: ahead of the loop it would hold a register per slot)
-                asm volatile("" : "+v"(ln));
-#pragma unroll
-                for (int u = 0; u < kFetchSlots; ++u) {
-                    if (f_blk[u] < 0) break;
-                    const int pf = f_blk[u] * kBlk + ln;   // foreign blocks are complete
-                    dma_dword_agent_u(lds_base_u + (unsigned)stage_f(PN, u) * 4u, hrow, (unsigned)(dir ? Lb - 1 - pf : pf) * 4u);
-                }
-            }
-        }
-    };
-    auto uniform_double = [&](double v) -> double {
-        const long long bits = __builtin_bit_cast(long long, v);
-        const unsigned lo = (unsigned)__builtin_amdgcn_readfirstlane((int)(bits & 0xffffffffLL));
-        const unsigned hi = (unsigned)__builtin_amdgcn_readfirstlane((int)(bits >> 32));
-        return __builtin_bit_cast(double, ((long long)hi << 32) | (long long)lo);
-    };
-    if (fetcher && Tb > 1) {   // what phase B of step 1 needs
-        issue_match_unrolled(std::integral_constant<int, 1>{}, 1);
-        if (consumer && 1 < Tb - 1) dma_dword_agent(lds_base + (unsigned)stage_p(1) * 4u, below, 0u);
-    }
-    wait_vmem_all();
-    __syncthreads();
-
-    bool aborted = false;
-    // The read-out needs what the lane of position L_b-1 computed in the last step, and that step's reference.  The
-    // last step leaves them in LDS: as variables they would hold three registers across the whole loop.
-    VT *const last_v = reinterpret_cast<VT *>(lds_raw + kLdsLastV) + wave * kBlk + lane;
-    *last_v = (VT)DAGX_NEG_INF;
-    // One step; CUR = parity of the buffers that hold step s-1 (compile-time: immediate LDS offsets).
-    // UNL: every lower block is a predecessor block (compile-time: the hot path has no branch on it).
-    auto step = [&](auto parity, auto unl, const int s) __attribute__((always_inline)) {
-        constexpr int CUR = decltype(parity)::value, NXT = CUR ^ 1;
-        constexpr bool UNL = decltype(unl)::value;
-        const int t = dir ? Tb - 1 - s : s;
-        // ---------------- phase A: tile mat-vecs (LDS and registers only); the fetcher's copies ----------------
-        if (__builtin_expect(fetcher, 0)) fetch_step(parity, s);   // step s + 1 uses the buffers that now hold step s - 1
-        double rl64 = 0.0;
-        float rl;
-        rl64 = relb64[CUR * kMaxBlocksFast + (lane & 15)]; rl = (float)rl64;
-        auto read_e = [&](const int sl, EV (&ev)[4]) __attribute__((always_inline)) {
-            const EV *src = ev_l15 + opaque_uniform(e_off[sl]);
-#pragma unroll
-            for (int q = 0; q < 4; ++q) ev[q] = src[CUR * kEbufPar + 16 * q];
-        };
-        EV eva[4];
-        read_e(0, eva);
-        
-        float tail[kTailRows > 0 ? kTailRows : 1];
-        // (requested now, used behind the first two tiles)
-#pragma unroll
-        for (int u = 0; u < kTailRows; ++u) tail[u] = tail_lane[u * kBlk];
-        // Rvec: lane Jb holds the scale of position block Jb = max offset over its predecessor blocks
-        const float rpre = row16_prefix_max(rl);
-        const float dmax = lane_bcast(rpre, 15);
-        const float d_s = dmax > DAGX_NEG_INF ? dmax : 0.f;  // next step's reference = cref + d_s
-        auto block_scale = [&](int Jb) -> float {
-            if constexpr (UNL) return lane_bcast(rpre, Jb);
-            else return lane_bcast(row16_max(((lane & 15) >= tile_ilo(Jb, W) && (lane & 15) <= Jb) ? rl : DAGX_NEG_INF), 0);
-        };
-        auto tile_step = [&](const int sl, const Tile &tile, const EV (&ev)[4]) __attribute__((always_inline)) {
-            // the raw product (at most 64 * 2^112): the factor exp(off_I - R_J) that brings the tiles of one
-            // output block to a common scale is applied by the block's owner, for all its tiles at once
-            EV acc = 0;
-            if (__builtin_expect(s >= s_lo[sl] && s <= s_hi[sl], 1)) acc = tile_dot(tile, ev[0], ev[1], ev[2], ev[3]);
-            ev_lane[opaque_uniform(part_off[sl])] = acc;
-        };
-        // (here, with the reads of this step's vectors in flight: its one LDS read then costs no wait of its own)
-        if (consumer) own_requests(parity, s);
-        tile_step(0, t0, eva);
-        // one set of float64 e values at a time: a second set does not fit the register file
-        read_e(1, eva);
-        tile_step(1, t1, eva);
-        read_e(2, eva);
-        EV acc = 0;
-        if (__builtin_expect(s >= s_lo[2] && s <= s_hi[2], 1)) acc = tile_dot_tail(t2, tail, eva[0], eva[1], eva[2], eva[3]);
-        ev_lane[opaque_uniform(part_off[2])] = acc;
-        __syncthreads();
-        // ---------------- phase B ----------------
-        // Every earlier store of this wave is complete (those of step s-1 were issued a whole step ago, so
-        // this costs nothing), which lets the progress word below run one step behind instead of two.
-        // The copies this wave requested in phase A (for step s + 1) have landed, too -- they were issued one
-        // to two thousand cycles ago -- so that after the barrier that ends this step every wave may read any of
-        // them (the progress snapshot the whole group decides on).
-        wait_vmem_all();
-        // (set in phase A only, by the fetcher; requested here with the other LDS reads, looked at behind the barrier)
-        const int gave_up_v = consumer ? s_abort : 0;
-        const double cnext = cref + (double)d_s;
-        // (1) hand-over: rows of step s from the producer groups -> ebuf/relb of the next step
-        if (consumer && s < Tb - 1) {
-#pragma unroll
-            for (int u = 0; u < kFetchSlots; ++u) {
-                if (f_blk[u] < 0) continue;
-                const int I = f_blk[u];
-                const float fh = lds_lane[stage_f(NXT, u)];
-                EV ef = LN::exp2s(fh * kLog2e);
-                ef = (fh > -3.0e38f && ef < tiny_up) ? tiny_up : ef;   // (as in own_block)
-                ev_lane[kEvEbuf + NXT * kEbufPar + I * kBlk] = I * kBlk + lane < Lb ? ef : (EV)0;
-                const double o = reinterpret_cast<const double *>(lds_raw + stage_o(NXT))[I];
-                if (lane == 0) {
-                    relb64[NXT * kMaxBlocksFast + I] = o > (double)DAGX_NEG_INF ? o - cnext : (double)DAGX_NEG_INF;
-                }
-            }
-        }
-        // (2) sum the tiles of each owned block
-        auto own_block = [&](const int Jb, const int poff, const int nt, const int p, const int node,
-                             const float mv) __attribute__((always_inline)) -> VT {
-            // partial sums (rows past the last tile are never written and hold 0), each times the factor that
-            // brings its tile to the block's scale: lane I of every 16-lane row of `fac` holds exp(off_I - R) for
-            // predecessor block I, capped at 1 -- a predecessor's factor never exceeds it, and the lanes of blocks
-            // that are no predecessors (whose rows hold 0) must not turn into inf * 0 -- and 0 for a dead block
-            // whose successors are alive.
-            // (Computed here, behind the barrier, from a copy of the offsets the compiler cannot trace back into
-            //  phase A: hoisted in front of the tiles this arithmetic lengthened every wave's phase A.)
-            const EV *prd = ev_lane + opaque_uniform(poff);
-            // the first eight partial sums are requested before anything else, all at once: one LDS round trip
-            // for them (read four at a time, next to their use, they cost two, one behind the other)
-            EV pr[8];
-#pragma unroll
-            for (int u = 0; u < 4; ++u) pr[u] = prd[u * kBlk];   // (float64 sums: four at a time, for want of registers)
-            asm volatile("" ::: "memory");
-            float rlb = rl;
-            asm volatile("" : "+v"(rlb));
-            const float R = block_scale(Jb);
-            // exp2(clamp(x, floor, 0)), floor = -inf (lower sweep) or -126 (upper sweep: a live block's factor never
-            // flushes; a dead block's rows hold 0 whatever stands in front of them).  -inf - R gives the floor;
-            // finite - -inf (+inf) gives 0, factor 1, and -inf - -inf (NaN) the floor (the median of three with a NaN
-            // among them is the smallest of the others), both in front of rows that hold 0.
-            EV fac;
-            // (the offsets' difference in float64: see Lin::exp2_with)
-            double rlb64 = rl64;
-            asm volatile("" : "+v"(rlb64));
-            // (R is the float32 rounding of the largest offset, so the block that sets the scale may lie a rounding
-            //  error above it: capped at 2, not at 1, or it would lose that sliver of its mass in every step)
-            const double x = (rlb64 - (double)R) * (double)kLog2e;
-            fac = LN::exp2_with(__builtin_fmax(__builtin_fmin(x, 1.0), (double)fac_floor), 0);
-            // partial row u belongs to predecessor block ilo + u (ilo = 0 when every lower block is a predecessor):
-            // with the factors shifted down by ilo lanes, row u takes its factor from lane u by DPP broadcast
-            EV facu = fac;
-            if constexpr (!UNL) {
-                const int from = ((lane & 15) + tile_ilo(Jb, W)) << 2;
-                const long long bits = __builtin_bit_cast(long long, fac);
-                const unsigned lo = (unsigned)__builtin_amdgcn_ds_bpermute(from, (int)(bits & 0xffffffffLL));
-                const unsigned hi = (unsigned)__builtin_amdgcn_ds_bpermute(from, (int)(bits >> 32));
-                facu = __builtin_bit_cast(double, ((long long)hi << 32) | (long long)lo);
-            }
-            EV tot;
-            scaled_sum4<0>(tot, facu, pr[0], pr[1], pr[2], pr[3]);
-#pragma unroll
-            for (int u = 0; u < 4; ++u) pr[u] = prd[(4 + u) * kBlk];
-            scaled_sum4<4>(tot, facu, pr[0], pr[1], pr[2], pr[3]);
-            if (__builtin_expect(nt > 8, 0)) {
-                scaled_sum4<8>(tot, facu, prd[8 * kBlk], prd[9 * kBlk], prd[10 * kBlk], prd[11 * kBlk]);
-                scaled_sum4<12>(tot, facu, prd[12 * kBlk], prd[13 * kBlk], prd[14 * kBlk], prd[15 * kBlk]);
-            }
-            // upper sweep: more than every product that may have been flushed on the way to this sum (64 per tile
-            // under 2^-126 each, 16 tiles, 16 scaled partial sums under 2^-126)
-            tot += flush_up;
-            // Dead cells come out as -inf by arithmetic alone (every test here is an instruction of the busiest
-            // SIMD): no live predecessor gives tot = 0 and log2 = -inf (R is then finite or -inf, never +inf), a
-            // match of -inf adds -inf; only the band has to be imposed.  A block without any live cell has
-            // vmax = -inf: its offset (finite reference + -inf) and relative offset are -inf, and its residuals
-            // are taken against -3e38 instead, which leaves them -inf and their exponentials 0.
-            const bool inband = p >= s && p <= slack + s;
-            VT vt;
-            vt = inband ? ((double)R + LN::log2u_wide(tot) * 0.6931471805599453) + (double)mv : (double)DAGX_NEG_INF;
-            const float v = (float)vt;
-            const float vmax = wave64_max(v);
-            const double offn = cref + (double)vmax;
-            float fh;   // the residual against the block's maximum (formed from the float64 value in the wide variant)
-            fh = (float)(vt - (double)fmaxf(vmax, -3.0e38f));
-            EV e;
-            // exp(v - vmax) not from the rounded v but from the sum itself: tot * exp(R + match - vmax) in float64
-            // (the shift of the staged transitions taken out, that of the float64 numbers staying in), so that a
-            // cell hundreds of nats under its reference hands on what it received to float64 accuracy
-            const double xe = ((((double)R - (double)vmax) + (double)mv) * (double)kLog2e) - (double)kShiftLinksWide;
-            // (a block without a live cell has vmax = -inf and exponentials 0 -- unless its sums are NaNs, which the
-            //  maximum skipped and which must stay NaNs)
-            e = !inband ? 0.0 : (vmax > -3.0e38f ? LN::times_exp2(tot, xe) : (tot == tot ? 0.0 : tot));
-            e = (fh > -3.0e38f && e < tiny_up) ? tiny_up : e;   // upper sweep: a live cell never flushes (a NaN stays one)
-            ev_lane[opaque_uniform(kEvEbuf + NXT * kEbufPar + Jb * kBlk)] = e;
-            if (lane == 0) {
-                relb64[NXT * kMaxBlocksFast + Jb] = (double)vmax - (double)d_s;
-                store_agent(off_at(t, Jb), offn);
-            }
-            if (p < Lb) store_agent(hat_at(t, node), fh);
-            return vt;   // relative to cref; the last step's value at position L_b-1 is the read-out
-        };
-        const bool last_step = s == Tb - 1;
-        if (owner) {
-            const VT v1 = own_block(Jown, own_part_off, nt_own, p_own, node_own, dma_decode<TM>(__builtin_bit_cast(unsigned, lds_lane[stage_m(NXT, 0)])));
-            if (last_step) {
-                *last_v = v1;
-                if (lane == 0) reinterpret_cast<double *>(lds_raw + kLdsLastC)[wave] = cref;
-            }
-        }
-        if (wave + kTileWaves < nblk) {   // a second owned block (many narrow blocks)
-            const int Jb = Jown + kTileWaves, p = p_own + kTileWaves * kBlk, node = dir ? Lb - 1 - p : p;
-            const VT v2 = own_block(Jb, own_part_off + kTileWaves * kPartRows * kBlk, Jb - tile_ilo(Jb, W) + 1, p, node,
-                                       dma_decode<TM>(__builtin_bit_cast(unsigned, lds_lane[stage_m(NXT, 1)])));
-            if (last_step && p == Lb - 1) *last_v = v2;   // the lane of position L_b-1 keeps that block's value
-        }
-        __syncthreads();
-        if (__builtin_amdgcn_readfirstlane(gave_up_v)) {   // only a consumer's own spin can set the flag; dealt with behind the loop
-            aborted = true;
-            return;
-        }
-        // Every wave has seen its stores of step s-1 complete (the wait at the top of phase B).
-        if (__builtin_expect(tid == 0 && producer && s >= 1, 0)) store_agent(prog + g, s - 1);
-        cref = uniform_double(cnext);
-    };
-
-    auto sweep = [&](auto unl) __attribute__((always_inline)) {
-        for (int s = 1; s < Tb; s += 2) {
-            step(std::integral_constant<int, 0>{}, unl, s);
-            if (aborted) return;
-            if (s + 1 < Tb) {
-                step(std::integral_constant<int, 1>{}, unl, s + 1);
-                if (aborted) return;
-            }
-        }
-    };
-    if (unlimited) sweep(std::true_type{}); else sweep(std::false_type{});
-    if (aborted) {
-        // a producer never showed up: hand the sample to the exact kernel and let consumers go on
-        if (tid == 0) {
-            store_agent(risk, 1);
-            store_agent(prog + g, 1 << 30);
-        }
-        return;
-    }
-    // read-out: the value of position L_b-1 after the last step (T_b = 1 was written above)
-    if (Tb > 1) {
-        const int pl = Lb - 1, Jl = pl / kBlk;
-        if (Jl >= jb0 && Jl < jb1 && ((Jl - jb0) & (kTileWaves - 1)) == wave && (pl & (kBlk - 1)) == lane) {
-            const VT v_last = *last_v;   // (written by this very lane)
-            const double cref_last = reinterpret_cast<const double *>(lds_raw + kLdsLastC)[wave];   // (by lane 0 of this wave)
-            const double z = v_last > (VT)DAGX_NEG_INF ? cref_last + (double)v_last : (double)DAGX_NEG_INF;
-            a.logz[slot * a.B + b] = z; if (slot == a.loss_dir) a.loss[b] = (float)z; store_agent(a.zfast + slot * a.B + b, z);
-        }
-    }
-    if (producer) {
-        wait_vmem_all();
-        __syncthreads();
-        if (tid == 0) store_agent(prog + g, Tb - 1);
-    }
-}
-
-// ---- the float32 sweeps, in chunks of four steps (geometry, tiles and products: dag_chunks.h) ------------------------
+// ---- the sweeps in chunks of four steps (geometry, tiles and products: dag_chunks.h) ---------------------------------
 // What a step-by-step sweep pays per step -- barriers, LDS round trips, scales, a few hundred instructions a wave around
 // the FMAs, 2.0 us at L = 512 -- is paid here once per four steps, and the tiles below the diagonal run on the matrix cores
-// at twice the rate of DPP FMAs.  What is left on the critical path is the walk of one block through four steps
-// (48 FMAs and 20 to 40 other instructions a step, 5.5 cycles each), the product of the tile next to the diagonal in
-// front of it, and one stage per block of the graph.  (With that product a stage ahead, too, the stages are 600 cycles
-// shorter but two per block: forward at B = 64, L = 512, T = 64 115 us instead of 107, L = 256 70 instead of 66,
-// L = 128 52 instead of 56.)
-//   step by step -> chunks, forward: B = 64, L = 512, T = 64 134 -> 107 us; L = 64 (T = 64) 81 -> 46; L = 256 99 -> 66;
-//   B = 16, L = 1024, T = 256 572 -> 357; B = 64, L = 512, transitions of at most 32: 136 -> 79.
+// (float32: at twice the rate of DPP FMAs; float64: at their rate, but a transition is converted once per four steps).
+// What is left on the critical path is the walk of one block through four steps (48 FMAs and 20 to 40 other instructions
+// a step, 5.5 cycles each), the product of the tile next to the diagonal in front of it, and one stage per block of the
+// graph.  (With that product a stage ahead, too, the stages are 600 cycles shorter but two per block: forward at B = 64,
+// L = 512, T = 64 115 us instead of 107, L = 256 70 instead of 66, L = 128 52 instead of 56.)
+//   step by step -> chunks, forward: B = 64, L = 512, T = 64 134 -> 107 us; L = 64 (T = 64) 81 -> 47; L = 256 99 -> 66;
+//   B = 16, L = 1024, T = 256 572 -> 347; B = 64, L = 512, transitions of at most 32: 136 -> 78.
+//   In float64: B = 16, L = 1024, T = 256 833 -> 535 us; B = 64, L = 512, T = 64 216 -> 160.
 // What bounds it: a SIMD gives its cycles either to matrix instructions or to vector instructions, never to both
 // (measured: a wave of DPP FMAs beside one of v_mfma_f32_4x4x1 advances only when that has ended, whatever their
 // priorities), so that products, walks and the rest of a stage add up.
 // A walking wave loads and converts its own match rows and writes its own results (as duties of other waves, through
 // LDS, they cost those waves more than they save it).
-template <typename TM, typename TL>
+//
+// Inter-workgroup hand-over of the running vector (the groups of one sweep form a one-way pipeline): a producer writes its
+// table rows (hat, off) with agent-scope stores and raises its progress word when the waves of its last two blocks have
+// both seen theirs of the last stage complete, early in the next one; a consumer copies the rows of a chunk (global ->
+// LDS) when the word covers it: of the block right below it one stage before its first block walks that chunk, of the
+// others two.  (All of them two stages ahead, and the word raised half a stage later: four stages a hand-over instead of
+// one and a half, B = 16, L = 1024, T = 64 189 us instead of 159.)  Every wait is bounded: on expiry the sample is
+// marked for the log-domain kernel and the group leaves.
+//
+// Leaving: every workgroup counts itself out of its sample and out of the launch.  The last one of a sample compares the
+// two read-outs, sets the sample's flag (1 = still to be done) and clears the sample's pipeline words; the last one of
+// the launch clears the ticket counter -- so the words are all zero again when the launch is over and need no fill in
+// front of it.
+template <typename TM, typename TL, bool WIDE>
 __device__ __forceinline__ void sweep_chunks_group(const SweepArgs &a, const int b, const int slot, const int g, float *lds_raw,
                                                    int *gstart, int *s_abort_p) {
+    using CH = Chunks<WIDE>;
+    using Cell = typename CH::Cell;
+    // slot: which of the sample's two sweeps (its tables, pipeline words and read-out); dir: its direction;
+    // upper: its rounding side.  The linear domain flushes what is too far under its scale -- a transition, a cell under
+    // its block maximum, a block under the largest of its neighbours, a product of such numbers.  The lower sweep lets all
+    // of that become 0, so its read-out never exceeds log Z; the upper sweep puts the smallest normal number (or a constant
+    // that covers every flushed product) in its place, so its read-out never falls short of log Z.  The sample's result
+    // stands when the two read-outs agree; what was flushed then carried no mass that matters, wherever it was flushed.
     const int dir = a.rev[slot];
-    const bool upper = a.upper[slot] != 0;   // rounding side, see sweep_tiles_group
+    const bool upper = a.upper[slot] != 0;
     const int tid = threadIdx.x, lane = tid & (kWave - 1);
     const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
     const int C = a.C;
@@ -1029,7 +321,7 @@ __device__ __forceinline__ void sweep_chunks_group(const SweepArgs &a, const int
     const int nblk = jb1 - jb0;
     const int flo = tile_ilo(jb0, W);             // lowest foreign block this group ever reads
     const bool producer = g < last_group, consumer = flo < jb0;
-    const ChunkLds o = chunk_lds(jb0, nblk, W);
+    const ChunkLds o = chunk_lds(jb0, nblk, W, WIDE);
     int ntile = 0;
     for (int q = 0; q < nblk; ++q) ntile += tiles_of_block(jb0 + q, W);
     if (nblk > kChunkBlocks || ntile > kTileCap - nblk || o.total * 4 > kChunkLdsBytes) {   // cannot happen with the host's partition
@@ -1041,7 +333,7 @@ __device__ __forceinline__ void sweep_chunks_group(const SweepArgs &a, const int
 
     // ---- my tiles below the diagonal.  A run is a wave's tiles that lead to one block; runs are numbered in the order of
     //      the tiles.  Worked out with lane <-> block (f: its first tile) and lane <-> wave (w_first: its first tile). ----
-    const TileDeal deal = a.plan.deal[NBb][g];
+    const TileDeal deal = a.plan.deal[WIDE][NBb][g];
     int my_first, my_count;
     wave_tiles(deal, wave, my_first, my_count);
     int f = 0, w_first, w_count;
@@ -1076,14 +368,15 @@ __device__ __forceinline__ void sweep_chunks_group(const SweepArgs &a, const int
         t_run[u] = runs_to(q, n) - 1;
     }
     // the runs that lead to the block this wave walks
-    int run_first = ntile, run_count = 1;         // (a block without such tiles: the zeros behind the products)
+    int run_first = o.runs, run_count = 1;         // (a block without such tiles: the zeros behind the products)
     if (owner && tiles_of_block(jb0 + wave, W) > 0) {
         const int n = __builtin_amdgcn_readlane(f, wave);
         run_first = runs_to(wave, n) - 1;
         run_count = runs_to(wave, n + tiles_of_block(jb0 + wave, W) - 1) - run_first;
     }
     // A consumer group has nothing to do for the first stages: it lets the first group of its sweep have the memory's
-    // bandwidth for its tiles.  (Progress words: 1 + chunks published, once the group's tiles are staged.)
+    // bandwidth for its tiles.  (Progress words: 1 once the group's tiles are staged, then 2 + n when the rows of the first n
+    // chunks of its last block and n + 1 of the others are in memory -- and so, since it has read them, n of all blocks below.)
     if (consumer) {
         if (wave == 0)
             for (int spins = 0; spins < kSpinLimit && __builtin_amdgcn_readfirstlane(load_agent(prog)) < 1; ++spins) __builtin_amdgcn_s_sleep(8);
@@ -1101,17 +394,22 @@ __device__ __forceinline__ void sweep_chunks_group(const SweepArgs &a, const int
     auto elements = [&](const int samples) { const int64_t n = (int64_t)samples * L * translen; return n < (1 << 28) ? (int)n : 1 << 28; };
     const int before = elements(b), behind = elements(a.B - 1 - b);
     auto stage = [&](const int u) __attribute__((always_inline)) {
-        stage_tile<TL>(patch, links, t_I[u], jb0 + t_q[u], lane, dir, Lb, translen, last_index, before, behind, tiny);
+        stage_tile<TL, CH::kLinkShift>(patch, links, t_I[u], jb0 + t_q[u], lane, dir, Lb, translen, last_index, before, behind, tiny);
     };
     Tile t0, t1, t2;
-    if (t_ok[0] || adjacent) { stage(0); read_patch(t0, patch, lane, dir); }
-    if (t_ok[1]) { stage(1); read_patch(t1, patch, lane, dir); }
-    if (t_ok[2] || owner) { stage(2); read_patch(t2, patch, lane, dir); }
+    auto read = [&](Tile &t, const bool triangle) __attribute__((always_inline)) {
+        if (!WIDE || triangle) read_patch(t, patch, lane, dir); else read_patch_wide(t, patch, lane, dir);
+    };
+    if (t_ok[0] || adjacent) { stage(0); read(t0, false); }
+    if (t_ok[1]) { stage(1); read(t1, false); }
+    if (t_ok[2] || owner) { stage(2); read(t2, owner); }
     if (owner) fold_triangle(t2, lane);
     __syncthreads();   // every wave is done with its transpose patch: the LDS now holds the buffers of the stages
     if (producer && g == 0 && tid == 0) store_agent(prog, 1);
 
     int *const lds_i = reinterpret_cast<int *>(lds_raw);
+    int *const published_by = lds_i + o.both;
+    if (tid == 0) *published_by = 0;
     const int D = o.depth;
     // ---- step 0: only position 0 is alive ----
     // exp(m): fraction in [1, 2) and exponent; what no such pair holds as in the constants above, +inf and NaN as NaN
@@ -1131,16 +429,17 @@ __device__ __forceinline__ void sweep_chunks_group(const SweepArgs &a, const int
     split_exp(m0, f0, n0);
     n0 = __builtin_amdgcn_readfirstlane(n0);
     const bool alive0 = !(f0 == 0.f);     // (a NaN is on its way)
-    const int cell_at = (lane & 15) * 16 + (lane >> 4);   // + 4 * (step & 3): this lane's cell in a chunk of cells
+    Cell *const eb = reinterpret_cast<Cell *>(lds_raw + o.eb), *const part = reinterpret_cast<Cell *>(lds_raw + o.part);
+    auto pow2 = [](const Cell x, const int n) __attribute__((always_inline)) { if constexpr (WIDE) return __builtin_ldexp(x, n); else return __builtin_ldexpf(x, n); };
     for (int q = wave; q < nblk; q += kTileWaves) {
         const int Jb = jb0 + q, p = Jb * kBlk + lane;
         const bool here = p == 0 && alive0;
-        lds_raw[o.eb + (jb0 - flo + q) * D * 256 + cell_at] = here ? __builtin_ldexpf(f0, kShift2 - 1) : 0.f;
+        eb[(jb0 - flo + q) * D * 256 + cell_place<WIDE>(lane)] = here ? pow2((Cell)f0, CH::kShift - 1) : (Cell)0;
         if (lane == 0) lds_i[o.kap + (jb0 - flo + q) * D * 4] = here ? n0 + 1 : kDeadExp;
         if (p < Lb) store_agent(hat + (int64_t)t_first * L + (dir ? Lb - 1 - p : p), here ? (fast_log2(f0) - 1.f) * kLn2 : DAGX_NEG_INF);
         if (lane == 0) store_agent(off + (int64_t)t_first * NBK + Jb, Jb == 0 && alive0 ? (double)(n0 + 1) * 0.6931471805599453 : (double)DAGX_NEG_INF);
     }
-    if (tid < 2 * 256) lds_raw[o.part + ntile * 2 * 256 + tid] = 0.f;
+    if (tid < 2 * 256) part[o.runs * 2 * 256 + tid] = (Cell)0;
     if (tid < nblk * 2 * kChunk) lds_i[o.part_scale + tid] = kDeadExp;   // (stays with a block without such tiles)
     if (Tb == 1 && tid == 0 && jb0 == 0) {
         const double z = (Lb == 1 && alive0) ? (double)m0 : (double)DAGX_NEG_INF;
@@ -1152,11 +451,11 @@ __device__ __forceinline__ void sweep_chunks_group(const SweepArgs &a, const int
     const unsigned long long hat_u = uniform_address(hat), off_u = uniform_address(off);
     const int ms1 = opaque_uniform((int)a.ms1), ms2 = opaque_uniform((int)a.ms2);   // the host checked that match indices fit 32 bits
     const int NC = (Tb - 1 + kChunk - 1) / kChunk;  // chunks of steps 1 .. T_b-1
-    const int floor_exp = upper ? -126 : -127;      // see pow2_clamped
-    const float tiny_up = upper ? kTinyStored : 0.f;
-    // more than everything that may have been flushed on the way to a block's sum: 64 products a tile under 2^-126
+    const int floor_exp = upper ? CH::kFloor : CH::kFloor - 1;   // see pow2_clamped
+    const Cell tiny_up = upper ? (WIDE ? (Cell)2.2250738585072014e-308 : (Cell)kTinyStored) : (Cell)0;   // 2^kFloor
+    // more than everything that may have been flushed on the way to a block's sum: 64 products a tile under 2^kFloor
     // each, 16 tiles, as many scaled sums
-    const float flush_up = upper ? 2.4074124e-35f : 0.f;
+    const Cell flush_up = upper ? (WIDE ? (Cell)9.332636185032189e-302 : (Cell)2.4074124e-35f) : (Cell)0;
     auto opaque_lane = [&] { int x = tid & (kWave - 1); asm volatile("" : "+v"(x)); return x; };
     // a block's chunks with a live cell (4c+1 .. 4c+4 meets the block's band), and its chunks as a source (4c .. 4c+3)
     auto dest_lo = [&](const int J) { return 16 * J - 1 - (slack >> 2); };
@@ -1177,29 +476,50 @@ __device__ __forceinline__ void sweep_chunks_group(const SweepArgs &a, const int
         dma_dword_agent_u(lds_base + (unsigned)(o.foff + (I - flo) * 64) * 4u, off_u,
                           (unsigned)(row_of((lane >> 1) & 3) * NBK + I) * 8u + (unsigned)(lane & 1) * 4u);
     };
-    // ... as cells: lane 4 (i & 15) + step has the four positions 16 q + (i & 15)
+    // ... as cells, four positions of one step a lane
     auto convert_rows = [&](const int I, const int sl, const int lane) __attribute__((always_inline)) {
         const int at = I - flo;
-        const float *src = lds_raw + o.frows + at * 256 + (lane & 3) * kBlk + (dir ? kBlk - 1 - (lane >> 2) : lane >> 2);
-        const int pitch = dir ? -16 : 16;
-        float x[4];
-#pragma unroll
-        for (int q = 0; q < 4; ++q) x[q] = src[q * pitch];
+        const float *const row = lds_raw + o.frows + at * 256 + (lane & 3) * kBlk;
         const double v = reinterpret_cast<const double *>(lds_raw + o.foff + at * 64)[lane & (kChunk - 1)];
-        f32x4 ev;
-#pragma unroll
-        for (int q = 0; q < 4; ++q) x[q] *= kLog2e;
-        if (__builtin_amdgcn_ballot_w64(!(fminf(fminf(x[0], x[1]), fminf(x[2], x[3])) >= -115.f)) == 0) {   // (as exp2_shifted above -115)
-#pragma unroll
-            for (int q = 0; q < 4; ++q) ev[q] = __builtin_ldexpf(fast_exp2(x[q]), kShift2);
-        } else {
+        if constexpr (WIDE) {
+            // positions 8 (lane / 16) + (lane / 4 mod 4) + {0, 4, 32, 36}: two neighbours of a product's first operand each
+            typedef double f64x2 __attribute__((ext_vector_type(2)));
+            const int r = 8 * (lane >> 4) + ((lane >> 2) & 3);
+            const float *const src = row + (dir ? kBlk - 1 - r : r);
+            f64x2 *const dst = reinterpret_cast<f64x2 *>(eb + (at * D + sl) * 256) + lane;
+            const int pitch = dir ? -4 : 4;
+            double w[4];
 #pragma unroll
             for (int q = 0; q < 4; ++q) {
-                const float w = exp2_shifted(x[q]);
-                ev[q] = (x[q] > -3.0e38f && w < tiny_up) ? tiny_up : w;
+                const float x = src[pitch * (q < 2 ? q : q + 6)];
+                const float hi = x * kLog2e, n = __builtin_floorf(hi), lo = __builtin_fmaf(x, kLog2e, -hi) + x * 1.925963033500e-08f;
+                const double z = __builtin_ldexp((double)fast_exp2((hi - n) + lo), (int)__builtin_fmaxf(n, -4000.f) + CH::kShift);
+                w[q] = x == DAGX_NEG_INF ? 0.0 : z + tiny_up;
             }
+            dst[0] = f64x2{w[0], w[1]};
+            dst[64] = f64x2{w[2], w[3]};
+        } else {
+            // lane 4 (i & 15) + step has the positions 16 q + (i & 15)
+            const float *const src = row + (dir ? kBlk - 1 - (lane >> 2) : lane >> 2);
+            const int pitch = dir ? -16 : 16;
+            float x[4];
+#pragma unroll
+            for (int q = 0; q < 4; ++q) x[q] = src[q * pitch];
+            f32x4 ev;
+#pragma unroll
+            for (int q = 0; q < 4; ++q) x[q] *= kLog2e;
+            if (__builtin_amdgcn_ballot_w64(!(fminf(fminf(x[0], x[1]), fminf(x[2], x[3])) >= -115.f)) == 0) {   // (as exp2_shifted above -115)
+#pragma unroll
+                for (int q = 0; q < 4; ++q) ev[q] = __builtin_ldexpf(fast_exp2(x[q]), kShift2);
+            } else {
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {
+                    const float w = exp2_shifted(x[q]);
+                    ev[q] = (x[q] > -3.0e38f && w < (float)tiny_up) ? (float)tiny_up : w;
+                }
+            }
+            *reinterpret_cast<f32x4 *>(eb + (at * D + sl) * 256 + lane * 4) = ev;
         }
-        *reinterpret_cast<f32x4 *>(lds_raw + o.eb + (at * D + sl) * 256 + lane * 4) = ev;
         const int kp = v > (double)DAGX_NEG_INF ? (int)__builtin_rint(v * 1.4426950408889634) : kDeadExp;
         if (lane < kChunk) lds_i[o.kap + (at * D + sl) * 4 + lane] = kp;
     };
@@ -1217,7 +537,7 @@ __device__ __forceinline__ void sweep_chunks_group(const SweepArgs &a, const int
         t_to[u] = t_ok[u] ? at + (dest_hi(J) < NC - 1 ? dest_hi(J) : NC - 1) : -100;
         t_src_from[u] = at + src_lo(t_I[u]); t_src_to[u] = at + dest_hi(t_I[u]);
         t_shift[u] = (((-at) % D) + D) % D;
-        t_cells[u] = o.eb + (t_I[u] - flo) * D * 256; t_kaps[u] = o.kap + (t_I[u] - flo) * D * 4;
+        t_cells[u] = (t_I[u] - flo) * D * 256; t_kaps[u] = o.kap + (t_I[u] - flo) * D * 4;
         t_scale_at[u] = o.kap + (lo - flo) * D * 4; t_scales[u] = J - 1 - lo;
     }
     if (NC == 0) return;
@@ -1227,17 +547,18 @@ __device__ __forceinline__ void sweep_chunks_group(const SweepArgs &a, const int
     auto stages = [&](auto walks, auto fetches) __attribute__((always_inline)) {
         constexpr bool WALKS = decltype(walks)::value, FETCHES = decltype(fetches)::value;
         // ring slots: chunk c of a block's cells is in slot c mod D (ring: the stage mod D)
-        int slot_own = 0, slot_f = 0, seen = 0, requested = -1, ring = ((first_stage % D) + D) % D;
+        int slot_own = 0, seen = 0, requested = first_stage - 1, ring = ((first_stage % D) + D) % D;
         auto next_slot = [&](const int x) { return x + 1 == D ? 0 : x + 1; };
         // the walking wave's state: the last step's cells and their exponent; the next chunk's match rows as loaded, then
         // exp(match) relative to the rows' exponents N
         const int J = jb0 + wave, first = J * kBlk, own_src = jb0 - flo + wave;
-        float e = 0.f;
-        int kap = kDeadExp, N[kChunk] = {0, 0, 0, 0};
+        // (float64: a fraction and its exponent relative to N)
+        Cell e = 0;
+        int kap = kDeadExp, N[kChunk] = {0, 0, 0, 0}, mt_exp[kChunk] = {0, 0, 0, 0};
         float mt[kChunk] = {0.f, 0.f, 0.f, 0.f};
         TM raw[kChunk];
         if (WALKS && J == 0) {
-            if (lane == 0 && alive0) e = __builtin_ldexpf(f0, kShift2 - 1);
+            if (lane == 0 && alive0) e = pow2((Cell)f0, CH::kShift - 1);
             kap = alive0 ? n0 + 1 : kDeadExp;
         }
         auto load_match = [&](const int c, const int lane) __attribute__((always_inline)) {
@@ -1273,8 +594,12 @@ __device__ __forceinline__ void sweep_chunks_group(const SweepArgs &a, const int
                 // relative to the row's exponent: its largest cell becomes a number in (1/2, 1]
                 const float n = __builtin_amdgcn_fmed3f(__builtin_ceilf(top[k] * kLog2e), -(float)kMatchExpMax, (float)kMatchExpMax);
                 N[k] = __builtin_amdgcn_readlane((int)n, 63);
-                mt[k] = __builtin_fmaf(m[k], log2e, -lane_bcast(n, 63));
+                if constexpr (WIDE) {
+                    split_exp(m[k], mt[k], mt_exp[k]);
+                    mt_exp[k] -= N[k];
+                } else mt[k] = __builtin_fmaf(m[k], log2e, -lane_bcast(n, 63));
             }
+            if constexpr (WIDE) return;
             if (__builtin_amdgcn_ballot_w64(!(fminf(fminf(mt[0], mt[1]), fminf(mt[2], mt[3])) >= -126.f)) != 0 && upper) {
 #pragma unroll
                 for (int k = 0; k < kChunk; ++k) mt[k] = m[k] > DAGX_NEG_INF && mt[k] < -126.f ? -126.f : mt[k];
@@ -1283,15 +608,21 @@ __device__ __forceinline__ void sweep_chunks_group(const SweepArgs &a, const int
             for (int k = 0; k < kChunk; ++k) mt[k] = fast_exp2(mt[k]);
         };
         // the chunk just walked (cells v, exponents kk) into the tables
-        auto write_out = [&](const int c, const float (&v)[kChunk], const int (&kk)[kChunk], const int lane) __attribute__((always_inline)) {
+        auto write_out = [&](const int c, const Cell (&v)[kChunk], const int (&kk)[kChunk], const int lane) __attribute__((always_inline)) {
             const int s0 = kChunk * c + 1, row0 = dir ? Tb - 1 - s0 : s0;
             float res[kChunk], lf[kChunk];
             int ex[kChunk];
 #pragma unroll
             for (int k = 0; k < kChunk; ++k) {   // (a dead cell: log of the fraction 0)
-                ex[k] = __builtin_amdgcn_frexp_expf(v[k]) - kShift2;
-                lf[k] = fast_log2(__builtin_amdgcn_frexp_mantf(v[k]));
-                res[k] = ((float)ex[k] + lf[k]) * kLn2;
+                if constexpr (WIDE) {
+                    ex[k] = __builtin_amdgcn_frexp_exp(v[k]) - CH::kShift;
+                    lf[k] = fast_log2((float)__builtin_amdgcn_frexp_mant(v[k]));
+                    res[k] = (float)(((double)ex[k] + (double)lf[k]) * 0.6931471805599453);
+                } else {
+                    ex[k] = __builtin_amdgcn_frexp_expf(v[k]) - kShift2;
+                    lf[k] = fast_log2(__builtin_amdgcn_frexp_mantf(v[k]));
+                    res[k] = ((float)ex[k] + lf[k]) * kLn2;
+                }
             }
             const unsigned lane_off = (unsigned)(dir ? Lb - 1 - first - lane : first + lane) * 4u;
             char *row = const_cast<char *>(hat_c) + (unsigned)(row0 * L) * 4u;
@@ -1320,59 +651,108 @@ __device__ __forceinline__ void sweep_chunks_group(const SweepArgs &a, const int
         for (int tau = first_stage; tau <= end_stage; ++tau) {
             const int par = tau & 1;
             // (per-lane addresses are formed anew in every stage: held across the loop they would cost the tiles their registers)
-            const int lane = opaque_lane(), cell_at = (lane & 15) * 16 + (lane >> 4);
-            const int cf = tau + 2;                             // the foreign chunk this stage brings in
-            const bool bring = FETCHES && f_blk[0] >= 0 && cf < NC;
+            const int lane = opaque_lane();
+            // the foreign chunks this stage brings in: tau + 1 of the block below, which the walk of my first block wants, and
+            // tau + 2 of the others, which the products of the next stage want
+            const bool bring = FETCHES && f_blk[0] >= 0 && tau + 1 < NC;
             int published = 0;
             if (bring) published = load_agent(below);
             // ---------------- walk my block through chunk tau - wave ----------------
             if (WALKS) {
                 const int c = tau - wave;
-                const bool more = c >= -1 && c + 1 < NC;
+                const bool more = c >= -1 && c + 1 < NC, live = c >= 0 && c < NC && c >= dest_lo(J) && c <= dest_hi(J);
+                // what block J - 1 sends: its cells of this chunk
+                const bool lower = live && J > 0 && c >= src_lo(J - 1) && c <= dest_hi(J - 1);
+                Cell Ga[kChunk] = {0, 0, 0, 0};
+                if (lower) {
+                    __builtin_amdgcn_s_setprio(3);
+                    const Cell *const src_cells = eb + ((own_src - 1) * D + slot_own) * 256;
+                    if constexpr (WIDE) {
+                        double out[4];
+                        tile_product(t0, src_cells, lane, out);
+                        double *const turn = reinterpret_cast<double *>(lds_raw + o.turn) + wave * 256;
+#pragma unroll
+                        for (int q = 0; q < 4; ++q) turn[(lane >> 4) * kBlk + 16 * q + (lane & 15)] = out[q];
+#pragma unroll
+                        for (int k = 0; k < kChunk; ++k) Ga[k] = turn[k * kBlk + lane];
+                    } else {
+                        const f32x4 out = tile_product(t0, *reinterpret_cast<const f32x4 *>(src_cells + lane * 4));
+#pragma unroll
+                        for (int k = 0; k < kChunk; ++k) Ga[k] = out[k];
+                    }
+                }
+                // The last two blocks' rows of the last stage are in memory when both their waves have come here, the other
+                // blocks' of the stage before that (their waves have since waited for match rows requested behind them):
+                // the second of the two publishes.
+                if (producer && wave >= nblk - 2) {
+                    const int n = tau - (nblk - 1);                // chunks of the last block
+                    if (n >= 0 && n < NC) {
+                        wait_vmem_all();
+                        int both = 1;
+                        if (nblk > 1) {
+                            if (lane == 0) both = __hip_atomic_fetch_add(published_by, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) & 1;
+                        }
+                        if (lane == 0 && both) store_agent(prog + g, 2 + n);
+                    }
+                }
                 if (more) load_match(c + 1, lane);
                 if (c >= 0 && c < NC) {
-                    float *const cells = lds_raw + o.eb + own_src * D * 256 + cell_at;
-                    float *const cells_next = cells + next_slot(slot_own) * 256;
-                    float *const cells_this = cells + slot_own * 256;
+                    Cell *const cells = eb + own_src * D * 256 + cell_place<WIDE>(lane);
+                    Cell *const cells_next = cells + next_slot(slot_own) * 256;
+                    Cell *const cells_this = cells + slot_own * 256;
                     int kk[kChunk];
-                    float v[kChunk];
-                    if (c >= dest_lo(J) && c <= dest_hi(J)) {
+                    Cell v[kChunk];
+                    if (live) {
                         __builtin_amdgcn_s_setprio(3);
-                        // what block J - 1 sends: its cells of this chunk, and (lane <-> step) their exponents, clamped as
-                        // a tile's under the largest of the blocks below
+                        // (lane <-> step) the exponents of what is sent; block J - 1's clamped as a tile's under the largest of the
+                        // blocks below
                         const int rv = lds_i[o.part_scale + (wave * 2 + (par ^ 1)) * 4 + (lane & 3)];
-                        const bool lower = J > 0 && c >= src_lo(J - 1) && c <= dest_hi(J - 1);
-                        f32x4 Ga = {0.f, 0.f, 0.f, 0.f};
                         int av = kDeadExp;
                         if (lower) {
-                            const f32x4 ev = *reinterpret_cast<const f32x4 *>(lds_raw + o.eb + ((own_src - 1) * D + slot_own) * 256 + lane * 4);
                             av = lds_i[o.kap + ((own_src - 1) * D + slot_own) * 4 + (lane & 3)];
-                            Ga = tile_product(t0, ev);
-                            if (av - rv < -126) av = upper ? rv - 126 : kDeadExp;
+                            if (av - rv < CH::kFloor) av = upper ? rv + CH::kFloor : kDeadExp;
                         }
                         int A[kChunk], R[kChunk];
 #pragma unroll
                         for (int k = 0; k < kChunk; ++k) { A[k] = __builtin_amdgcn_readlane(av, k); R[k] = __builtin_amdgcn_readlane(rv, k); }
-                        const float *const parts = lds_raw + o.part + (run_first * 2 + (par ^ 1)) * 256 + lane * 4;
+                        const Cell *const parts = part + (run_first * 2 + (par ^ 1)) * 256 + lane * (WIDE ? 1 : 4);
                         const float upper_half = lane >= 32 ? 1.f : 0.f;
-                        f32x4 G = *reinterpret_cast<const f32x4 *>(parts);
-                        if (run_count > 1) {
-                            f32x4 G1 = *reinterpret_cast<const f32x4 *>(parts + 512);
-                            if (run_count > 2) {
-                                G += *reinterpret_cast<const f32x4 *>(parts + 1024);
+                        Cell G[kChunk];
+                        if constexpr (WIDE) {
+#pragma unroll
+                            for (int k = 0; k < kChunk; ++k) G[k] = parts[k * kBlk];
 #pragma unroll 1
-                                for (int u = 3; u < run_count; ++u) G += *reinterpret_cast<const f32x4 *>(parts + u * 512);
+                            for (int u = 1; u < run_count; ++u)
+#pragma unroll
+                                for (int k = 0; k < kChunk; ++k) G[k] += parts[u * 512 + k * kBlk];
+                        } else {
+                            f32x4 sum = *reinterpret_cast<const f32x4 *>(parts);
+                            if (run_count > 1) {
+                                f32x4 sum1 = *reinterpret_cast<const f32x4 *>(parts + 512);
+                                if (run_count > 2) {
+                                    sum += *reinterpret_cast<const f32x4 *>(parts + 1024);
+#pragma unroll 1
+                                    for (int u = 3; u < run_count; ++u) sum += *reinterpret_cast<const f32x4 *>(parts + u * 512);
+                                }
+                                sum += sum1;
                             }
-                            G += G1;
+#pragma unroll
+                            for (int k = 0; k < kChunk; ++k) G[k] = sum[k];
                         }
 #pragma unroll
                         for (int k = 0; k < kChunk; ++k) {
-                            // (kSpare: every other step does not scale its cells by their largest)
-                            const int most = A[k] > R[k] ? A[k] : R[k], ref = (kap > most ? kap : most) + (k & 1 ? 0 : kSpare);
+                            // (float32, kSpare: every other step does not scale its cells by their largest)
+                            const int most = A[k] > R[k] ? A[k] : R[k], ref = (kap > most ? kap : most) + (WIDE || (k & 1) ? 0 : kSpare);
                             // (what ldexp flushes of either part is under flush_up, too)
-                            const float x = (__builtin_ldexpf(triangle_dot(t2, e, upper_half), kap - ref) + flush_up) + (__builtin_ldexpf(G[k], R[k] - ref) + __builtin_ldexpf(Ga[k], A[k] - ref));
+                            const Cell x = (pow2(triangle_dot(t2, e, upper_half), kap - ref) + flush_up) + (pow2(G[k], R[k] - ref) + pow2(Ga[k], A[k] - ref));
                             // (upper sweep: a cell never flushes, live or not -- what a dead one gets is of the size of what is flushed)
-                            if (k & 1) {
+                            if constexpr (WIDE) {
+                                const double y = pow2(x * (double)mt[k], mt_exp[k]);
+                                const unsigned top = wave64_max_upper(y);
+                                const int tb = (int)(top >> 20) > 1 ? (int)(top >> 20) : 1;
+                                kap = top ? tb + ref + N[k] - (1022 + CH::kShift + CH::kLinkShift) : kDeadExp;
+                                e = pow2(y, 1022 + CH::kShift - tb) + tiny_up;
+                            } else if (k & 1) {
                                 const float y = x * mt[k];
                                 // the exponent of the largest cell, at least that of 2^-72: its reciprocal has to be a float32 number
                                 const unsigned top = wave64_max_positive(y);
@@ -1385,72 +765,89 @@ __device__ __forceinline__ void sweep_chunks_group(const SweepArgs &a, const int
                             }
                             kk[k] = kap;
                             v[k] = e;
-                            if (k < kChunk - 1) cells_this[4 * (k + 1)] = e; else cells_next[0] = e;
+                            if (k < kChunk - 1) cells_this[CH::kStepPitch * (k + 1)] = e; else cells_next[0] = e;
                         }
                         __builtin_amdgcn_s_setprio(0);
                     } else {
-                        e = 0.f; kap = kDeadExp;
+                        e = 0; kap = kDeadExp;
 #pragma unroll
                         for (int k = 0; k < kChunk; ++k) {
                             kk[k] = kDeadExp;
-                            v[k] = 0.f;
-                            if (k < kChunk - 1) cells_this[4 * (k + 1)] = 0.f; else cells_next[0] = 0.f;
+                            v[k] = 0;
+                            if (k < kChunk - 1) cells_this[CH::kStepPitch * (k + 1)] = 0; else cells_next[0] = 0;
                         }
                     }
                     if (more) convert_match(c + 1, lane);   // (in front of the stores: what it waits for is older than they)
                     else wait_vmem_all();
-                    // Either wait covers what this wave stored in the last stage.  The other blocks are a chunk and more
-                    // ahead of the last one: when its wave has come here, every block's chunk c - 1 is in memory.
-                    if (producer && wave == nblk - 1 && c > 0 && lane == 0) store_agent(prog + g, 1 + c);
                     const int kp = write_out(c, v, kk, lane);
                     const int sl = (lane & 3) < kChunk - 1 ? slot_own * 4 + 1 + (lane & 3) : next_slot(slot_own) * 4;
                     if (lane < kChunk) lds_i[o.kap + own_src * D * 4 + sl] = kp;
                     slot_own = next_slot(slot_own);
                 }
                 else if (more) convert_match(c + 1, lane);
+                else if (c == NC) wait_vmem_all();
             }
             // ---------------- multiply out what my tiles' blocks (q of the group) receive in chunk tau + 1 - q ----------------
             if (my_count > 0) {
-                // (the LDS reads of two tiles are requested before the first is waited for, the third's behind the first)
+                // (float32: the LDS reads of two tiles are requested before the first is waited for, the third's behind the first)
                 f32x4 ev[2];
-                int kv[kTilesPerWave], rv[kTilesPerWave];
+                int kv[kTilesPerWave], rv[kTilesPerWave], at[kTilesPerWave];
                 bool go[kTilesPerWave], src[kTilesPerWave];
+                const int step = WIDE ? lane >> 4 : lane & 3, other = WIDE ? lane & 15 : lane >> 2;   // (lane <-> step and block of what leads here)
+                auto cells_of = [&](const int u) __attribute__((always_inline)) { return *reinterpret_cast<const f32x4 *>(lds_raw + o.eb + at[u] + lane * 4); };
 #pragma unroll
                 for (int u = WALKS ? 1 : 0; u < (WALKS ? 2 : kTilesPerWave); ++u) {
                     go[u] = tau >= t_from[u] && tau <= t_to[u];
                     src[u] = tau >= t_src_from[u] && tau <= t_src_to[u];
                     if (go[u]) {
                         int sl = ring + t_shift[u]; sl -= sl >= D ? D : 0;
-                        if (u < 2) ev[u] = *reinterpret_cast<const f32x4 *>(lds_raw + t_cells[u] + sl * 256 + lane * 4);
-                        kv[u] = lds_i[t_kaps[u] + sl * 4 + (lane & 3)];
+                        at[u] = t_cells[u] + sl * 256;
+                        if (!WIDE && u < 2) ev[u] = cells_of(u);
+                        kv[u] = lds_i[t_kaps[u] + sl * 4 + step];
                         if (t_start[u]) {
-                            const int n = (lane >> 2) < t_scales[u] ? lane >> 2 : 0;
-                            rv[u] = lds_i[t_scale_at[u] + sl * 4 + n * (D * 4) + (lane & 3)];
+                            const int n = other < t_scales[u] ? other : 0;
+                            rv[u] = lds_i[t_scale_at[u] + sl * 4 + n * (D * 4) + step];
                         }
                     }
                 }
-                f32x4 G = {0.f, 0.f, 0.f, 0.f};
+                Cell G[4] = {0, 0, 0, 0};
                 int R = kDeadExp;
                 auto product = [&](const int u, const Tile &t) __attribute__((always_inline)) {
                     if (!go[u]) return;
                     if (t_start[u]) {   // the scale: the largest exponent, step by step, among all blocks that lead here
-                        R = by_step_max(rv[u]);
-                        G = f32x4{0.f, 0.f, 0.f, 0.f};
+                        if constexpr (WIDE) R = row16_max_int(rv[u]); else R = by_step_max(rv[u]);
+#pragma unroll
+                        for (int k = 0; k < 4; ++k) G[k] = 0;
                     }
                     if (src[u]) {
-                        const f32x4 v = tile_product(t, ev[u & 1]);
-                        scaled4<false>(G, pow2_clamped(kv[u] - R, floor_exp), v);
+                        if constexpr (WIDE) {
+                            double v[4];
+                            tile_product(t, eb + at[u], lane, v);
+                            const double f = pow2_clamped_wide(kv[u] - R, floor_exp);
+#pragma unroll
+                            for (int k = 0; k < 4; ++k) G[k] = __builtin_fma(v[k], f, G[k]);
+                        } else {
+                            const f32x4 v = tile_product(t, ev[u & 1]);
+                            f32x4 sum = {G[0], G[1], G[2], G[3]};
+                            scaled4<false>(sum, pow2_clamped(kv[u] - R, floor_exp), v);
+#pragma unroll
+                            for (int k = 0; k < 4; ++k) G[k] = sum[k];
+                        }
                     }
                     if (t_end[u]) {
-                        *reinterpret_cast<f32x4 *>(lds_raw + o.part + (t_run[u] * 2 + par) * 256 + lane * 4) = G;
-                        if (t_lead[u] && lane < 4) lds_i[o.part_scale + (t_q[u] * 2 + par) * 4 + lane] = R;
+                        Cell *const to = part + (t_run[u] * 2 + par) * 256;
+                        if constexpr (WIDE) {
+#pragma unroll
+                            for (int k = 0; k < 4; ++k) to[(lane >> 4) * kBlk + 16 * k + (lane & 15)] = G[k];
+                            if (t_lead[u] && (lane & 15) == 0) lds_i[o.part_scale + (t_q[u] * 2 + par) * 4 + step] = R;
+                        } else {
+                            *reinterpret_cast<f32x4 *>(to + lane * 4) = f32x4{G[0], G[1], G[2], G[3]};
+                            if (t_lead[u] && lane < 4) lds_i[o.part_scale + (t_q[u] * 2 + par) * 4 + lane] = R;
+                        }
                     }
                 };
                 if (!WALKS) product(0, t0);
-                if (!WALKS && go[2]) {
-                    int sl = ring + t_shift[2]; sl -= sl >= D ? D : 0;
-                    ev[0] = *reinterpret_cast<const f32x4 *>(lds_raw + t_cells[2] + sl * 256 + lane * 4);
-                }
+                if (!WIDE && !WALKS && go[2]) ev[0] = cells_of(2);
                 product(1, t1);
                 if (!WALKS) product(2, t2);
             }
@@ -1458,25 +855,34 @@ __device__ __forceinline__ void sweep_chunks_group(const SweepArgs &a, const int
             if (bring) {
                 published = __builtin_amdgcn_readfirstlane(published);
                 if (published > seen) seen = published;
-                auto request = [&](const int c) __attribute__((always_inline)) {
+                auto chunk_of = [&](const int u, const int t) { return t + (f_blk[u] == jb0 - 1 ? 1 : 2); };
+                auto request = [&](const int t) __attribute__((always_inline)) {   // what stage t brings in
 #pragma unroll
-                    for (int u = 0; u < kForeign; ++u) { if (f_blk[u] < 0) break; request_rows(f_blk[u], c, lane); }
-                    requested = c;
+                    for (int u = 0; u < kForeign; ++u) {
+                        if (f_blk[u] < 0) break;
+                        const int c = chunk_of(u, t);
+                        if (c >= 0 && c < NC) request_rows(f_blk[u], c, lane);
+                    }
+                    requested = t;
                 };
-                if (requested < cf) {
+                if (requested < tau) {
                     int spins = 0;
-                    while (seen <= cf + 1) {                    // (the word is 1 + chunks published)
+                    while (seen < tau + 4) {
                         __builtin_amdgcn_s_sleep(1);
                         seen = __builtin_amdgcn_readfirstlane(load_agent(below));
                         if (++spins > kSpinLimit) { *s_abort_p = 1; break; }
                     }
-                    if (seen > cf + 1) request(cf);
+                    if (seen >= tau + 4) request(tau);
                 }
                 wait_vmem_all();
 #pragma unroll
-                for (int u = 0; u < kForeign; ++u) { if (f_blk[u] < 0) break; convert_rows(f_blk[u], slot_f, lane); }
-                slot_f = next_slot(slot_f);
-                if (cf + 1 < NC && seen > cf + 2) request(cf + 1);
+                for (int u = 0; u < kForeign; ++u) {
+                    if (f_blk[u] < 0) break;
+                    const int c = chunk_of(u, tau);
+                    int sl = ring + c - tau; sl -= sl >= D ? D : 0;
+                    if (c >= 0 && c < NC) convert_rows(f_blk[u], sl, lane);
+                }
+                if (tau + 2 < NC && seen >= tau + 5) request(tau + 1);
             }
             ring = next_slot(ring);
             __syncthreads();
@@ -1489,7 +895,7 @@ __device__ __forceinline__ void sweep_chunks_group(const SweepArgs &a, const int
     if (producer) {
         wait_vmem_all();
         __syncthreads();
-        if (tid == 0) store_agent(prog + g, 1 + NC);
+        if (tid == 0) store_agent(prog + g, 2 + NC);
     }
     if (consumer && __builtin_amdgcn_readfirstlane(*s_abort_p)) {   // a producer never showed up: hand the sample on and let consumers go on
         wait_vmem_all();
@@ -1545,8 +951,7 @@ __global__ __launch_bounds__(kTileWaves * kWave) void dag_sweep_tiles_kernel(Swe
     // leave at once, through the same bookkeeping
     const bool skip = has_sample && a.only_flagged && a.flags[b] != 1;
     if (has_sample && !skip) {
-        if constexpr (WIDE) sweep_tiles_group<TM, TL>(a, b, slot, g, lds_raw, gstart, &s_abort);
-        else sweep_chunks_group<TM, TL>(a, b, slot, g, lds_raw, gstart, &s_abort);
+        sweep_chunks_group<TM, TL, WIDE>(a, b, slot, g, lds_raw, gstart, &s_abort);
     }
     // ---- leaving ----
     wait_vmem_all();   // this wave's stores (table rows, read-outs) are complete
@@ -2200,11 +1605,6 @@ size_t loss_bwd_workspace_bytes(int B) { (void)B; return 0; }
 // The tile kernel's dynamic LDS (transpose patches while the tiles are staged, step buffers afterwards) exceeds the
 // default limit: the limit is raised once per device and instantiation (not a call a graph capture may contain;
 // dagx_prepare_device does it for every instantiation ahead of time).
-constexpr size_t kPatchBytes = (size_t)kTileWaves * kBlk * (kBlk + 1) * sizeof(float);
-template <bool WIDE> constexpr size_t tiles_lds_bytes() {
-    if (!WIDE) return kChunkLdsBytes;
-    return kPatchBytes > (size_t)StepLds::kStepFloats * sizeof(float) ? kPatchBytes : (size_t)StepLds::kStepFloats * sizeof(float);
-}
 template <typename TM, typename TL, bool WIDE>
 static int prepare_tiles_kernel() {
     static std::atomic<unsigned long long> attr_set{0};   // per template instantiation: one bit per device
@@ -2212,8 +1612,8 @@ static int prepare_tiles_kernel() {
     (void)hipGetDevice(&device);
     const unsigned long long bit = 1ull << (device & 63);
     if (!(attr_set.load(std::memory_order_acquire) & bit)) {
-        hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(dag_sweep_tiles_kernel<TM, TL, WIDE>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)tiles_lds_bytes<WIDE>());
-        if (e != hipSuccess) { set_error("dag_loss_fwd: cannot reserve %zu bytes of LDS: %s", tiles_lds_bytes<WIDE>(), hipGetErrorString(e)); return DAGX_ERR_LAUNCH; }
+        hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(dag_sweep_tiles_kernel<TM, TL, WIDE>), hipFuncAttributeMaxDynamicSharedMemorySize, kChunkLdsBytes);
+        if (e != hipSuccess) { set_error("dag_loss_fwd: cannot reserve %d bytes of LDS: %s", kChunkLdsBytes, hipGetErrorString(e)); return DAGX_ERR_LAUNCH; }
         attr_set.fetch_or(bit, std::memory_order_release);
     }
     return DAGX_OK;
@@ -2265,7 +1665,7 @@ static int launch_sweeps(SweepArgs a, hipStream_t st) {
         if ((rc = prepare_tiles_kernel<TM, TL, false>()) || (rc = prepare_tiles_kernel<TM, TL, true>())) return rc;
         if (!float64_first()) {
             a.only_flagged = 0;
-            hipLaunchKernelGGL((dag_sweep_tiles_kernel<TM, TL, false>), dim3(a.ndir * B8 * C), dim3(kTileWaves * kWave), tiles_lds_bytes<false>(), st, a);
+            hipLaunchKernelGGL((dag_sweep_tiles_kernel<TM, TL, false>), dim3(a.ndir * B8 * C), dim3(kTileWaves * kWave), kChunkLdsBytes, st, a);
             if ((rc = check_launch("dag_sweep_tiles"))) return rc;
         } else {   // the caller knows its inputs for sharply peaked: no float32 pass whose result would not stand
             hipLaunchKernelGGL(dag_mark_all_kernel, dim3((a.B + 255) / 256), dim3(256), 0, st, a.flags, a.B, a.sync);
@@ -2274,7 +1674,7 @@ static int launch_sweeps(SweepArgs a, hipStream_t st) {
         // the samples whose two read-outs did not agree, once more with float64 linear-domain numbers (the pipeline
         // words are zero again, as the first launch found them)
         a.only_flagged = 1;
-        hipLaunchKernelGGL((dag_sweep_tiles_kernel<TM, TL, true>), dim3(a.ndir * B8 * C), dim3(kTileWaves * kWave), tiles_lds_bytes<true>(), st, a);
+        hipLaunchKernelGGL((dag_sweep_tiles_kernel<TM, TL, true>), dim3(a.ndir * B8 * C), dim3(kTileWaves * kWave), kChunkLdsBytes, st, a);
         if ((rc = check_launch("dag_sweep_tiles (wide)"))) return rc;
     }
     constexpr int NT = 1024;

@@ -1,9 +1,10 @@
-"""The chunked float32 sweeps of dag_loss at the sizes where they can go wrong: graphs one node short of, at and one
+"""The chunked sweeps of dag_loss, in float32 and float64, at the sizes where they can go wrong: graphs one node short of, at and one
 past a block of 64 and a group's last block, targets one step around a chunk of four, transition windows around a block,
 transitions that start at an odd element of their tensor or are its very first and last ones, one sample alone."""
 import pytest
 import torch
 
+from da_transformer_amd import _native as nat
 from da_transformer_amd.custom_ops.dag_loss import DagLossFunc
 from oracle import torch_native as tn
 from helpers import random_problem
@@ -13,6 +14,7 @@ pytestmark = pytest.mark.gpu
 F32, F16, BF16 = torch.float32, torch.float16, torch.bfloat16
 
 
+@pytest.mark.parametrize("wide", [False, True])
 @pytest.mark.parametrize("B,L,T,translen,dtype", [
     (1, 2, 2, 1, F32), (3, 2, 2, 1, F16), (2, 5, 5, 1, F32), (1, 20, 6, None, F16),
     (1, 63, 5, None, F32), (2, 64, 2, None, F16), (1, 65, 6, 63, F16), (3, 65, 9, 64, BF16), (2, 66, 10, 1, F32),
@@ -20,7 +22,7 @@ F32, F16, BF16 = torch.float32, torch.float16, torch.bfloat16
     (2, 449, 30, 32, F32), (1, 511, 14, None, BF16), (2, 513, 7, 257, F32), (1, 705, 12, 130, F16), (2, 1024, 11, None, F32),
     (1, 1023, 64, 200, F16),
     (65, 320, 8, None, F16), (65, 1022, 20, 64, F16)])   # no room for groups of at most four blocks: five, eight
-def test_edges_of_blocks_chunks_and_windows(B, L, T, translen, dtype):
+def test_edges_of_blocks_chunks_and_windows(B, L, T, translen, dtype, wide):
     match, links_sq, ol, tl = random_problem(L + T, B + 1, L, T, dtype=F32, ragged=False, translen=translen)
     if translen is not None:      # a path of T_b nodes spans at most (T_b - 1) translen transitions
         ol = torch.minimum(ol, (tl - 1) * translen + 1).clamp_(min=1)
@@ -32,9 +34,13 @@ def test_edges_of_blocks_chunks_and_windows(B, L, T, translen, dtype):
     g = torch.linspace(-1.0, 2.0, B)
     rloss, rgm, rgl = oracle_loss_and_grads(match[1:], links[1:], ol, tl, g)
     # views from the second sample on: contiguous, the first element anywhere in a four-byte word
-    loss, gm, gl = hip_loss_and_grads(match.to(DEV)[1:], links.to(DEV)[1:], ol, tl, g)
-    if B * L * links.shape[2] >= 4:       # the float32 sweeps' own result (but for a sample without a path)
-        assert (DagLossFunc.last_sample_flags.cpu()[torch.isfinite(rloss)] == 0).all()
+    before = nat.lib().dagx_loss_float64_first(int(wide))
+    try:
+        loss, gm, gl = hip_loss_and_grads(match.to(DEV)[1:], links.to(DEV)[1:], ol, tl, g)
+    finally:
+        nat.lib().dagx_loss_float64_first(before)
+    if B * L * links.shape[2] >= 4:       # the sweeps' own result (but for a sample without a path)
+        assert (DagLossFunc.last_sample_flags.cpu()[torch.isfinite(rloss)] == (2 if wide else 0)).all()
     # per step a chain of at most 64 products a tile, two exponentials and the partial sums: 6e-7 of the cell
     fin = torch.isfinite(rloss)
     assert torch.equal(torch.isfinite(loss), fin)
