@@ -4,7 +4,7 @@
 //   back[t][j] = the smallest i attaining the max; backtrack from (T_b-1, L_b-1).
 //
 // Two implementations:
-//  * dag_align_tiles_kernel + dag_backtrack_kernel (L <= 1024): the sweep keeps E as 64x64 register
+//  * dag_align_chunks_kernel or dag_align_steps_kernel + dag_backtrack_kernel (L <= 1024): the sweep keeps E as 64x64 register
 //    tiles and evaluates a step with one DPP-broadcast add and one max per (i, j) pair, spread over
 //    the same pipeline of workgroups as the loss sweeps; it stores only the score table.  The
 //    backtrack (a wave per sample walks, others may stage for it) then re-derives, for the T_b cells on the path only, the
@@ -15,7 +15,7 @@
 //    pipeline gave up on.
 // Both evaluate fl32(A + E) then + match, so their scores -- and therefore the paths -- are
 // bit-identical to the torch-native rule.
-#include "dag_tiles.h"
+#include "dag_chunks.h"
 
 #include <atomic>
 
@@ -121,6 +121,510 @@ __global__ __launch_bounds__(NT) void dag_align_kernel(AlignArgs a) {
 // Tile-resident max-plus sweep
 // ================================================================================================
 
+// b0 = max(b0, max_{r<8} (a0[lane R0 + r of this 16-lane row] + p[r])), b1 likewise with a1, R1 and q: per pair of rows two
+// sums and one three-way maximum (a maximum does not round: the result is that of one by one, bit for bit).  Two chains side
+// by side, because a wave waits 8 cycles for a result it needs at once: one alone takes 7.7 cycles an instruction.
+template <int R0, int R1>
+__device__ __forceinline__ void maxplus8x2(float &b0, float a0, const float *p, float &b1, float a1, const float *q) {
+    static_assert((R0 == 0 || R0 == 8) && (R1 == 0 || R1 == 8), "");
+    float t0, t1, t2, t3;
+#define DAGX_SUMS(X, Y, P0, P1, Q0, Q1, N0, N1) \
+        "v_add_f32_dpp %2, %6, " P0 " row_newbcast:" X " row_mask:0xf bank_mask:0xf\n\t" \
+        "v_add_f32_dpp %3, %6, " P1 " row_newbcast:" Y " row_mask:0xf bank_mask:0xf\n\t" \
+        "v_add_f32_dpp %4, %7, " Q0 " row_newbcast:" N0 " row_mask:0xf bank_mask:0xf\n\t" \
+        "v_add_f32_dpp %5, %7, " Q1 " row_newbcast:" N1 " row_mask:0xf bank_mask:0xf\n\t" \
+        "v_max3_f32 %0, %0, %2, %3\n\t" \
+        "v_max3_f32 %1, %1, %4, %5\n\t"
+#define DAGX_ROWS8(A0, A1, A2, A3, A4, A5, A6, A7, B0, B1, B2, B3, B4, B5, B6, B7) \
+    asm("s_nop 1\n\t" \
+        DAGX_SUMS(A0, A1, "%8", "%9", "%16", "%17", B0, B1) \
+        DAGX_SUMS(A2, A3, "%10", "%11", "%18", "%19", B2, B3) \
+        DAGX_SUMS(A4, A5, "%12", "%13", "%20", "%21", B4, B5) \
+        DAGX_SUMS(A6, A7, "%14", "%15", "%22", "%23", B6, B7) \
+        : "+v"(b0), "+v"(b1), "=&v"(t0), "=&v"(t1), "=&v"(t2), "=&v"(t3) \
+        : "v"(a0), "v"(a1), "v"(p[0]), "v"(p[1]), "v"(p[2]), "v"(p[3]), "v"(p[4]), "v"(p[5]), "v"(p[6]), "v"(p[7]), \
+          "v"(q[0]), "v"(q[1]), "v"(q[2]), "v"(q[3]), "v"(q[4]), "v"(q[5]), "v"(q[6]), "v"(q[7]))
+    if constexpr (R0 == 0 && R1 == 0) DAGX_ROWS8("0", "1", "2", "3", "4", "5", "6", "7", "0", "1", "2", "3", "4", "5", "6", "7");
+    else if constexpr (R0 == 8 && R1 == 8) DAGX_ROWS8("8", "9", "10", "11", "12", "13", "14", "15", "8", "9", "10", "11", "12", "13", "14", "15");
+    else if constexpr (R0 == 0) DAGX_ROWS8("0", "1", "2", "3", "4", "5", "6", "7", "8", "9", "10", "11", "12", "13", "14", "15");
+    else DAGX_ROWS8("8", "9", "10", "11", "12", "13", "14", "15", "0", "1", "2", "3", "4", "5", "6", "7");
+#undef DAGX_ROWS8
+#undef DAGX_SUMS
+}
+
+// out[k] = max_{r<64} (cells[k][r] + tile.p[r]) for two steps; `cells`: this lane's place lane & 15 in the first of them
+__device__ __forceinline__ void tile_maxplus2(const Tile &t, const float *cells, float &out0, float &out1) {
+    float b0 = DAGX_NEG_INF, b1 = DAGX_NEG_INF;
+    float a0[4], a1[4];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) { a0[q] = cells[16 * q]; a1[q] = cells[kBlk + 16 * q]; }
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+        maxplus8x2<0, 0>(b0, a0[q], t.p + 16 * q, b1, a1[q], t.p + 16 * q);
+        maxplus8x2<8, 8>(b0, a0[q], t.p + 16 * q + 8, b1, a1[q], t.p + 16 * q + 8);
+    }
+    out0 = b0; out1 = b1;
+}
+
+// {x, y} -> x: rows {x0 y0 x2 y2} of sixteen lanes, y: rows {x1 y1 x3 y3}
+__device__ __forceinline__ void swap_rows(float &x, float &y) {
+    const u32x2 s = __builtin_amdgcn_permlane16_swap(__builtin_bit_cast(unsigned, x), __builtin_bit_cast(unsigned, y), false, false);
+    const unsigned a = s[0], b = s[1];
+    x = __builtin_bit_cast(float, a); y = __builtin_bit_cast(float, b);
+}
+// max_i (a[i] + P[i][lane]) over a triangle as fold_triangle leaves it; `upper`: lanes 32..63
+__device__ __forceinline__ float triangle_maxplus(const Tile &t, float a, bool upper) {
+    float even = a, odd = a;
+    swap_rows(even, odd);                      // rows {0,0,2,2} and {1,1,3,3} of a
+    float crossed = odd, rest = even;
+    swap_halves(crossed, rest);                // rows {1,1,0,0}
+    float b0 = DAGX_NEG_INF, b1 = DAGX_NEG_INF, b2 = DAGX_NEG_INF;
+    maxplus8x2<0, 0>(b2, crossed, t.p + 32, b0, even, t.p);
+    maxplus8x2<8, 8>(b2, crossed, t.p + 40, b0, even, t.p + 8);
+    float other = b2;
+    swap_halves(b2, other);                    // (the square's two halves, for the upper lanes)
+    maxplus8x2<0, 8>(b0, odd, t.p + 16, b1, odd, t.p + 24);
+    b2 = fmaxf(b2, other);
+    return fmaxf(fmaxf(b0, b1), upper ? b2 : DAGX_NEG_INF);
+}
+
+// bytes per row of the source-block table (rows padded to 16 bytes)
+__host__ __device__ static inline int srcblk_pitch(int L) { return (L + 15) & ~15; }
+
+// Contiguous grouping of the position blocks [0, NBb) into at most C groups of at most kTileCap tiles,
+// minimising the largest group.  gstart[g] .. gstart[g+1] are the blocks of group g (empty groups last).
+__device__ __host__ inline int partition_blocks(int NBb, int W, int C, int *gstart) {
+    int best_cap = kTileCap;
+    for (int cap = 1; cap <= kTileCap; ++cap) {
+        int groups = 1, sum = 0; bool ok = true;
+        for (int Jb = 0; Jb < NBb; ++Jb) {
+            int c = Jb - tile_ilo(Jb, W) + 1;
+            if (c > cap) { ok = false; break; }
+            if (sum + c > cap) { ++groups; sum = 0; }
+            sum += c;
+        }
+        if (ok && groups <= C) { best_cap = cap; break; }
+    }
+    int g = 0, sum = 0;
+    gstart[0] = 0;
+    for (int Jb = 0; Jb < NBb; ++Jb) {
+        int c = Jb - tile_ilo(Jb, W) + 1;
+        if (sum + c > best_cap && sum > 0) { ++g; if (g < C) gstart[g] = Jb; sum = 0; }
+        sum += c;
+    }
+    int used = g + 1;
+    for (int q = used; q <= C; ++q) gstart[q] = NBb;
+    return used;
+}
+
+// Whether the sweep goes in chunks of four steps.  They cost T / 4 stages and one or two more for every block of nodes, single
+// steps T of a quarter of that: chunks win by 8 to 18 % at T = L / 8 and more on long graphs, tie there on short ones, and
+// lose by 5 to 20 % at T = L / 9 and less (alignment, chunks and steps: B = 64, L = 512, T = 64 129 and 140 us; B = 20, L = 1000,
+// T = 128 297 and 328; B = 48, L = 350, T = 40 81 and 76; B = 1, L = 140, T = 16 35 and 31).
+static bool align_in_chunks(int B, int T, int L, int translen) {
+    return 8 * (int64_t)T >= L && (int64_t)B * L * translen >= 4;   // (the chunked kernel's tiles are loaded four elements at a time)
+}
+
+// Workgroups per sweep.  In chunks: from four position blocks on as many as the device has room for (one per CU) up to one
+// for each block, at most ten.  (Fewer tiles a SIMD, against more hand-overs: as many as hold the tiles -> this, alignment of
+// B = 16, L = 1024, T = 256 484 -> 445 us; B = 4, L = 700, T = 100 211 -> 183; B = 64, L = 320, T = 48 83 -> 79; B = 64, L = 256,
+// T = 64 92 -> 80.)  Step by step: twice as many as hold the tiles where there is room and the graph has at least four
+// blocks (5 to 13 %; more lose); where that exceeds the 11 the kernel supports, ten when they fit.
+static int align_groups(int B, int T, int L, int translen) {
+    const int NB = (L + kBlk - 1) / kBlk, B8 = (B + 7) & ~7;
+    if (align_in_chunks(B, T, L, translen)) {
+        const int C = groups_needed(L, translen, kChunkBlocks);
+        if (C == 0 || NB < 4) return C;
+        const int room = 256 / B8, most = NB < 10 ? NB : 10, more = room < most ? room : most;
+        return more > C ? more : C;
+    }
+    const int C = groups_needed(L, translen, kMaxBlocksFast);
+    if (C == 0) return 0;
+    if (NB >= 4 && 2 * C <= 11 && 2 * C <= NB && (long long)B8 * 2 * C <= 256) return 2 * C;
+    return C < 10 && NB >= 10 && (long long)B8 * 10 <= 256 ? 10 : C;
+}
+
+struct AlignTileArgs {
+    const void *match; int64_t ms0, ms1, ms2;
+    const void *links;
+    const int64_t *out_len, *tgt_len;
+    int B, T, L, translen;
+    float *table;     // [B][T][L] best score of every cell, by node
+    unsigned char *srcblk;   // [B][T][pitch] block of 64 nodes that holds the best predecessor of every cell (the lowest such block); 16-byte aligned rows
+    int *sync;        // [0] ticket counter, [16 + b*C + group] progress
+    int *flags;       // [B] set when the pipeline gave up on a sample
+    int C;
+    int mcap;         // match row read at step s: min(s, mcap) (T-1 for the alignment: every step its own row)
+    int decode;       // Viterbi decoding: every sample runs all T steps (tgt_len is not read) and no cell is
+                      // pruned for being too far from the last node -- a path may end at any step
+    ChunkPlan<1> plan;   // gtab[NBb][g] = first block of group g, and how its tiles are dealt to its waves
+};
+
+// LDS of a group, in dwords: cells of four steps in the order of the table, results of a wave's tiles that lead to one block.
+struct AlignLds {
+    int depth, runs;    // chunks of cells kept per block; runs of tiles there can be
+    int eb;             // [nsrc][depth][4][64]
+    int both;           // [1] SPACING 1: counts the last two blocks' waves as they find their rows in memory
+    int part, from;     // [runs][2][64][4] best scores of four steps a lane; [runs][2][64] the blocks they come from, a byte each
+    int total;
+};
+__device__ __host__ inline AlignLds align_lds(int jb0, int nblk, int W, int spacing) {
+    AlignLds o;
+    const int nsrc = jb0 - tile_ilo(jb0, W) + nblk;
+    int ntile = 0;
+    for (int q = 0; q < nblk; ++q) ntile += spacing == 1 ? tiles_of_block<1>(jb0 + q, W) : tiles_of_block<2>(jb0 + q, W);
+    // (read up to SPACING (blocks of the group) stages after they are written; foreign rows are copied into place up to a
+    // stage before they are due)
+    o.depth = spacing * (nblk < W ? nblk : W) + 3 - spacing;
+    o.runs = ntile < kTileWaves + nblk - 1 ? ntile : kTileWaves + nblk - 1;
+    int at = 0;
+    o.eb = at; at += nsrc * o.depth * 256;
+    o.part = at; at += o.runs * 2 * 256;
+    o.from = at; at += o.runs * 2 * 64;
+    o.both = at; at += 4;
+    o.total = at;
+    return o;
+}
+
+// The pipeline of the loss sweeps (sweep_chunks_group: stages of four steps, tickets, one-way hand-over through the table
+// with agent-scope accesses, bounded waits), in the (max, +) semiring and without any rescaling: the table holds the plain
+// fp32 scores, and a foreign block's rows are copied straight to where the tiles read them.  A maximum does not round and
+// sums are formed as they are step by step, so that scores and source blocks do not depend on the order: of several
+// blocks with the best predecessor the lowest one counts (runs in the order of the blocks, then the block itself; a later
+// one replaces an earlier one only if it is larger).
+//
+// Step by step, with two barriers, LDS round trips and a hand-over in each, a step cost 1.8 us at L = 512 and 3.2 us at
+// L = 1024, of which the tiles' 96 instructions a step are a quarter.  What bounds the stages now is those instructions:
+// four steps of a tile take 2 700 cycles, 2 000 of a SIMD that two waves share, the walk of a block 3 500.
+//
+// SPACING (dag_chunks.h): a tile is nearly as much work as the walk here, so that where the walk bounds the stages and SIMDs
+// have time to spare -- small graphs, or hardly more than one block to a group -- two stages a block are shorter
+// (alignment with SPACING 1 and 2: B = 64, L = 256, T = 64 91 and 78 us; B = 64, L = 384, T = 48 91 and 86; B = 16, L = 400,
+// T = 50 99 and 93); where the tiles bound them every stage more costs (B = 64, L = 512, T = 64 128 and 137; B = 16, L = 1024,
+// T = 256 445 and 476).
+template <typename TM, typename TL, int SPACING>
+__global__ __launch_bounds__(kTileWaves * kWave) void dag_align_chunks_kernel(AlignTileArgs a) {
+    extern __shared__ float lds_raw[];
+    __shared__ int gstart[16];
+    __shared__ int s_ticket, s_abort;
+
+    const int tid = threadIdx.x, lane = tid & (kWave - 1);
+    const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
+    const int C = a.C;
+    if (tid == 0) { s_ticket = atomicAdd(a.sync, 1); s_abort = 0; }
+    __syncthreads();
+    const int ticket = __builtin_amdgcn_readfirstlane(s_ticket);
+    const int B8 = (a.B + 7) & ~7;
+    // first group 0 of every sample, then every group 1, ... (see the loss sweep kernel: producers hold smaller tickets,
+    // and what the dispatcher reaches last are consumers); the groups of a sample are a multiple of 8 tickets apart
+    const int g = ticket / B8;
+    const int b = ((ticket / 8) % (B8 / 8)) * 8 + (ticket % 8);
+    if (g >= C || b >= a.B) return;
+
+    const int L = opaque_uniform(a.L), T = a.T, translen = a.translen;
+    const int Lb = (int)a.out_len[b], Tb = a.decode ? T : (int)a.tgt_len[b];
+    if (!(Tb >= 1 && Lb >= 1 && Tb <= T && Lb <= L && (a.decode || Tb <= Lb))) return;   // the backtrack sees the lengths too
+    const TM *match = static_cast<const TM *>(a.match) + (int64_t)b * a.ms0;
+    const TL *links = static_cast<const TL *>(a.links) + (int64_t)b * L * translen;
+    float *table = a.table + (int64_t)b * T * L;
+    const int spitch = srcblk_pitch(L);
+    unsigned char *srcblk = a.srcblk + (int64_t)b * T * spitch;
+    int *prog = a.sync + 16 + b * C;
+
+    const int slack = a.decode ? L : Lb - Tb;
+    const int NBb = (Lb + kBlk - 1) / kBlk;
+    const int W = (translen + kBlk - 1) / kBlk;
+    if (tid <= C) gstart[tid] = a.plan.gtab[NBb][tid];
+    __syncthreads();
+    const int jb0 = __builtin_amdgcn_readfirstlane(gstart[g]), jb1 = __builtin_amdgcn_readfirstlane(gstart[g + 1]);
+    int last_group = 0;
+    for (int q = 0; q < C; ++q) if (gstart[q + 1] > gstart[q]) last_group = q;
+    last_group = __builtin_amdgcn_readfirstlane(last_group);
+    if (jb0 >= jb1) return;
+    const int nblk = jb1 - jb0;
+    const int flo = tile_ilo(jb0, W);
+    const bool producer = g < last_group, consumer = flo < jb0;
+    const AlignLds o = align_lds(jb0, nblk, W, SPACING);
+    if (nblk > kChunkBlocks || o.total * 4 > kChunkLdsBytes) {   // cannot happen with the host's partition
+        if (tid == 0) { a.flags[b] = 1; store_agent(prog + g, 1 << 30); }
+        return;
+    }
+    const bool owner = wave < nblk;               // this wave walks block jb0 + wave
+    const int helpers = kTileWaves - nblk;
+    const TileDeal deal = a.plan.deal[0][NBb][g];
+    const WaveTiles t = plan_wave<SPACING>(deal, jb0, nblk, W, 0, wave, lane);
+    // (Progress words as in the loss sweeps.)
+    if (consumer) {
+        if (wave == 0)
+            for (int spins = 0; spins < kSpinLimit && __builtin_amdgcn_readfirstlane(load_agent(prog)) < 1; ++spins) __builtin_amdgcn_s_sleep(8);
+        __syncthreads();
+    }
+    const unsigned lds_base = (unsigned)reinterpret_cast<uintptr_t>(lds_raw);
+    float *const patch = lds_raw + wave * (kBlk * kPatchPitch);
+    const int last_index = L * translen - 1;
+    auto elements = [&](const int samples) { const int64_t n = (int64_t)samples * L * translen; return n < (1 << 28) ? (int)n : 1 << 28; };
+    const int before = elements(b), behind = elements(a.B - 1 - b);
+    auto stage = [&](Tile &tile, const int u) __attribute__((always_inline)) {
+        stage_tile<TL, 0, false>(patch, links, t.I[u], jb0 + t.q[u], lane, 0, Lb, translen, last_index, before, behind, 0.f);
+        read_patch(tile, patch, lane, 0);
+    };
+    Tile t0, t1, t2;
+    if (t.ok[0] || t.adjacent) stage(t0, 0);
+    if (t.ok[1]) stage(t1, 1);
+    if (t.ok[2] || owner) stage(t2, 2);
+    if (owner) fold_triangle(t2, lane);
+    __syncthreads();   // every wave is done with its transpose patch: the LDS now holds the buffers of the stages
+    if (producer && g == 0 && tid == 0) store_agent(prog, 1);
+
+    int *const lds_i = reinterpret_cast<int *>(lds_raw);
+    int *const published_by = lds_i + o.both;
+    if (tid == 0) *published_by = 0;
+    const int D = o.depth;
+    const char *match_c = reinterpret_cast<const char *>(match);
+    const int ms1 = opaque_uniform((int)a.ms1), ms2 = opaque_uniform((int)a.ms2);   // the host checked that match indices fit 32 bits
+    // step 0: node 0 holds match[0][0] (even if that is -inf), everything else -inf
+    const float m0 = to_float(match[0]);
+    if (owner) {
+        const int p = (jb0 + wave) * kBlk + lane;
+        const float v = p == 0 ? m0 : DAGX_NEG_INF;
+        lds_raw[o.eb + (jb0 - flo + wave) * D * 256 + lane] = v;
+        if (p < Lb) store_agent(table + p, v);
+    }
+    const unsigned long long table_u = uniform_address(table);
+    char *const table_c = reinterpret_cast<char *>(table), *const srcblk_c = reinterpret_cast<char *>(srcblk);
+    const int NC = (Tb - 1 + kChunk - 1) / kChunk;  // chunks of steps 1 .. T_b-1
+    const int last_row = opaque_uniform(a.mcap < Tb - 1 ? a.mcap : Tb - 1);
+    auto opaque_lane = [&] { int x = tid & (kWave - 1); asm volatile("" : "+v"(x)); return x; };
+    // a block's chunks with a cell in the band (4c+1 .. 4c+4), and its chunks as a source (4c .. 4c+3)
+    auto dest_lo = [&](const int J) { return 16 * J - 1 - (slack >> 2); };
+    auto dest_hi = [&](const int J) { return 16 * J + 15; };
+    auto src_lo = [&](const int I) { return 16 * I - ((slack + 3) >> 2); };
+
+    // ---- the foreign blocks whose table rows this wave fetches ----
+    int f_blk[kForeign], f_first, f_count;
+    wave_foreign(deal, wave, f_first, f_count);
+#pragma unroll
+    for (int u = 0; u < kForeign; ++u) f_blk[u] = u < f_count ? flo + f_first + u : -1;
+    // table rows of steps 4c .. 4c+3 of a foreign block (complete: 64 nodes) to slot sl of its cells: sixteen bytes a lane
+    auto request_rows = [&](const int I, const int c, const int sl, const int lane) __attribute__((always_inline)) {
+        const int s = kChunk * c + (lane >> 4), row = s < Tb ? s : Tb - 1;
+        dma_dwordx4_agent_u(lds_base + (unsigned)(o.eb + ((I - flo) * D + sl) * 256) * 4u, table_u, (unsigned)(row * L + I * kBlk + 4 * (lane & 15)) * 4u);
+    };
+
+    // ---- the stages ----
+    const int first_stage = consumer ? -2 : -1, end_stage = NC - 1 + SPACING * (nblk - 1);
+    const int *below = prog + (g > 0 ? g - 1 : 0);
+    // stages in which a tile's block takes part, and those in which the tile's source has a cell in the band
+    int t_from[kTilesPerWave], t_to[kTilesPerWave], t_src_from[kTilesPerWave], t_src_to[kTilesPerWave], t_shift[kTilesPerWave], t_cells[kTilesPerWave];
+#pragma unroll
+    for (int u = 0; u < kTilesPerWave; ++u) {
+        const int J = jb0 + t.q[u], at = SPACING * t.q[u] - 1;               // chunk = stage - at
+        t_from[u] = at + (dest_lo(J) > 0 ? dest_lo(J) : 0);
+        t_to[u] = t.ok[u] ? at + (dest_hi(J) < NC - 1 ? dest_hi(J) : NC - 1) : -100;
+        t_src_from[u] = at + src_lo(t.I[u]); t_src_to[u] = at + dest_hi(t.I[u]);
+        t_shift[u] = (((-at) % D) + D) % D;
+        t_cells[u] = o.eb + (t.I[u] - flo) * D * 256;
+    }
+    if (NC == 0) return;
+    __syncthreads();
+
+    auto stages = [&](auto walks, auto fetches) __attribute__((always_inline)) {
+        constexpr bool WALKS = decltype(walks)::value, FETCHES = decltype(fetches)::value;
+        int slot_own = 0, seen = 0, requested = first_stage - 1, ring = ((first_stage % D) + D) % D;
+        auto next_slot = [&](const int x) { return x + 1 == D ? 0 : x + 1; };
+        const int J = jb0 + wave, first = J * kBlk, own_src = jb0 - flo + wave, ilo = tile_ilo(J, W);
+        float e = WALKS && J == 0 && lane == 0 ? m0 : DAGX_NEG_INF;          // the last step's scores
+        float mt[kChunk] = {0.f, 0.f, 0.f, 0.f};                             // the next chunk's match rows
+        TM raw[kChunk];
+        auto load_match = [&](const int c, const int lane) __attribute__((always_inline)) {
+            const int p = first + lane, pc = p < Lb ? p : Lb - 1, s0 = kChunk * c + 1;
+            const unsigned lane_off = (unsigned)(pc * ms2) * (unsigned)sizeof(TM);
+#pragma unroll
+            for (int k = 0; k < kChunk; ++k)
+                raw[k] = *reinterpret_cast<const TM *>(match_c + (unsigned)((s0 + k < last_row ? s0 + k : last_row) * ms1) * (unsigned)sizeof(TM) + lane_off);
+        };
+        auto convert_match = [&] {
+#pragma unroll
+            for (int k = 0; k < kChunk; ++k) mt[k] = to_float(raw[k]);
+        };
+        // a tile's best of four steps into the best so far (cells of four steps, 64 each)
+        auto take = [&](const Tile &tile, const float *cells, const int I, float (&best)[kChunk], int (&from)[kChunk]) __attribute__((always_inline)) {
+#pragma unroll
+            for (int k = 0; k < kChunk; k += 2) {
+                float x[2];
+                tile_maxplus2(tile, cells + k * kBlk, x[0], x[1]);
+#pragma unroll
+                for (int h = 0; h < 2; ++h) {
+                    const bool up = x[h] > best[k + h];
+                    best[k + h] = up ? x[h] : best[k + h]; from[k + h] = up ? I : from[k + h];
+                }
+            }
+        };
+        for (int tau = first_stage; tau <= end_stage; ++tau) {
+            const int par = tau & 1;
+            const int lane = opaque_lane(), r16 = lane & 15;
+            // (chunk tau + 2 of the foreign blocks, with SPACING 1 tau + 1 of the block below)
+            const bool bring = FETCHES && f_blk[0] >= 0 && tau + SPACING < NC;
+            int published = 0;
+            if (bring) published = load_agent(below);
+            // (as in the loss sweeps; with SPACING 2 the last block's wave alone: the other blocks are two stages ahead of it)
+            auto publish = [&]() __attribute__((always_inline)) {
+                const int n = tau - SPACING * (nblk - 1);      // chunks of the last block
+                if (!producer || wave < nblk - (SPACING == 1 ? 2 : 1) || n < 0 || n >= NC) return;
+                wait_vmem_all();
+                int both = 1;
+                if (SPACING == 1 && nblk > 1) {
+                    if (lane == 0) both = __hip_atomic_fetch_add(published_by, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) & 1;
+                }
+                if (lane == 0 && both) store_agent(prog + g, 2 + n);
+            };
+            // ---------------- walk my block through chunk tau - SPACING wave ----------------
+            if (WALKS) {
+                const int c = tau - SPACING * wave;
+                const bool more = c >= -1 && c + 1 < NC, live = c >= 0 && c < NC && c >= dest_lo(J) && c <= dest_hi(J);
+                float best[kChunk] = {DAGX_NEG_INF, DAGX_NEG_INF, DAGX_NEG_INF, DAGX_NEG_INF};
+                int from[kChunk] = {ilo, ilo, ilo, ilo};
+                if (live) {
+                    __builtin_amdgcn_s_setprio(3);
+                    if (J > (SPACING == 1 ? ilo + 1 : 0)) {
+#pragma unroll 1
+                        for (int u = 0; u < t.run_count; ++u) {
+                            const int at = (t.run_first + u) * 2 + (par ^ 1);
+                            const f32x4 x = *reinterpret_cast<const f32x4 *>(lds_raw + o.part + at * 256 + lane * 4);
+                            const int y = lds_i[o.from + at * 64 + lane];
+#pragma unroll
+                            for (int k = 0; k < kChunk; ++k) {
+                                const float xk = x[k];
+                                const bool up = xk > best[k];
+                                best[k] = up ? xk : best[k]; from[k] = up ? (y >> (8 * k)) & 255 : from[k];
+                            }
+                        }
+                    }
+                    if (SPACING == 1 && J > 0 && c >= src_lo(J - 1) && c <= dest_hi(J - 1))   // what block J - 1 sends
+                        take(t0, lds_raw + o.eb + ((own_src - 1) * D + slot_own) * 256 + r16, J - 1, best, from);
+                }
+                if (more) load_match(c + 1, lane);
+                if (c >= 0 && c < NC) {
+                    float *const cells = lds_raw + o.eb + own_src * D * 256 + lane;
+                    float *const cells_next = cells + next_slot(slot_own) * 256;
+                    float *const cells_this = cells + slot_own * 256;
+                    const int s0 = kChunk * c + 1;
+                    float v[kChunk];
+                    if (live) {
+                        const int d0 = first + lane - s0;
+#pragma unroll
+                        for (int k = 0; k < kChunk; ++k) {
+                            const float x = triangle_maxplus(t2, e, lane >= 32);
+                            const bool up = x > best[k];
+                            best[k] = up ? x : best[k]; from[k] = up ? J : from[k];
+                            // in the band: s <= p <= slack + s; the second (and last) rounding of the cell
+                            e = (unsigned)(d0 - k) <= (unsigned)slack ? best[k] + mt[k] : DAGX_NEG_INF;
+                            v[k] = e;
+                            if (k < kChunk - 1) cells_this[kBlk * (k + 1)] = e; else cells_next[0] = e;
+                            if (k == 0) publish();
+                        }
+                        __builtin_amdgcn_s_setprio(0);
+                    } else {
+                        publish();
+                        e = DAGX_NEG_INF;
+#pragma unroll
+                        for (int k = 0; k < kChunk; ++k) {
+                            v[k] = e;
+                            if (k < kChunk - 1) cells_this[kBlk * (k + 1)] = e; else cells_next[0] = e;
+                        }
+                    }
+                    if (more) convert_match();   // (in front of the stores: what it waits for is older than they)
+                    else wait_vmem_all();
+                    // into the tables
+                    const int steps = Tb - s0 < kChunk ? Tb - s0 : kChunk;
+                    if (first + lane < Lb) {
+                        char *row = table_c + (unsigned)(s0 * L) * 4u, *srow = srcblk_c + (unsigned)(s0 * spitch);
+                        const unsigned at = (unsigned)(first + lane);
+#pragma unroll
+                        for (int k = 0; k < kChunk; ++k) {
+                            if (k >= steps) break;
+                            store_agent(reinterpret_cast<float *>(row + at * 4u), v[k]);
+                            *reinterpret_cast<unsigned char *>(srow + at) = (unsigned char)from[k];
+                            row += L * 4; srow += spitch;
+                        }
+                    }
+                    slot_own = next_slot(slot_own);
+                }
+                else {
+                    publish();
+                    if (more) convert_match();
+                    else if (SPACING == 1 && c == NC) wait_vmem_all();
+                }
+            }
+            // ---------------- what my tiles' blocks (q of the group) receive in chunk tau + 1 - SPACING q ------
+            if (t.count > 0) {
+                float best[kChunk] = {DAGX_NEG_INF, DAGX_NEG_INF, DAGX_NEG_INF, DAGX_NEG_INF};
+                int from[kChunk] = {0, 0, 0, 0};
+                auto product = [&](const int u, const Tile &tile) __attribute__((always_inline)) {
+                    if (!(tau >= t_from[u] && tau <= t_to[u])) return;
+                    if (t.start[u]) {
+#pragma unroll
+                        for (int k = 0; k < kChunk; ++k) { best[k] = DAGX_NEG_INF; from[k] = 0; }
+                    }
+                    if (tau >= t_src_from[u] && tau <= t_src_to[u]) {
+                        int sl = ring + t_shift[u]; sl -= sl >= D ? D : 0;
+                        take(tile, lds_raw + t_cells[u] + sl * 256 + r16, t.I[u], best, from);
+                    }
+                    if (t.end[u]) {
+                        const int at = t.run[u] * 2 + par;
+                        *reinterpret_cast<f32x4 *>(lds_raw + o.part + at * 256 + lane * 4) = f32x4{best[0], best[1], best[2], best[3]};
+                        lds_i[o.from + at * 64 + lane] = from[0] | from[1] << 8 | from[2] << 16 | from[3] << 24;
+                    }
+                };
+                if (SPACING == 2 || !WALKS) product(0, t0);
+                product(1, t1);
+                if (!WALKS) product(2, t2);
+            }
+            // ---------------- table rows of foreign blocks: requested a stage ago if they were published by then ----------------
+            if (bring) {
+                published = __builtin_amdgcn_readfirstlane(published);
+                if (published > seen) seen = published;
+                auto request = [&](const int stage) __attribute__((always_inline)) {   // what a stage brings in
+#pragma unroll
+                    for (int u = 0; u < kForeign; ++u) {
+                        if (f_blk[u] < 0) break;
+                        const int c = stage + (SPACING == 1 && f_blk[u] == jb0 - 1 ? 1 : 2);
+                        int sl = ring + c - tau; sl -= sl >= D ? D : 0;
+                        if (SPACING == 2 || (c >= 0 && c < NC)) request_rows(f_blk[u], c, sl, lane);
+                    }
+                    requested = stage;
+                };
+                if (requested < tau) {
+                    int spins = 0;
+                    while (seen < tau + SPACING + 3) {
+                        __builtin_amdgcn_s_sleep(1);
+                        seen = __builtin_amdgcn_readfirstlane(load_agent(below));
+                        if (++spins > kSpinLimit) { s_abort = 1; break; }
+                    }
+                    if (seen >= tau + SPACING + 3) request(tau);
+                }
+                wait_vmem_all();
+                if (tau + 1 + SPACING < NC && seen >= tau + SPACING + 4) request(tau + 1);
+            }
+            ring = next_slot(ring);
+            __syncthreads();
+            if (consumer && __builtin_amdgcn_readfirstlane(s_abort)) return;
+        }
+    };
+    if (owner && helpers == 0) stages(std::true_type{}, std::true_type{});
+    else if (owner) stages(std::true_type{}, std::false_type{});
+    else stages(std::false_type{}, std::true_type{});
+    if (producer) {
+        wait_vmem_all();
+        __syncthreads();
+        if (tid == 0) store_agent(prog + g, 2 + NC);
+    }
+    if (consumer && __builtin_amdgcn_readfirstlane(s_abort)) {   // a producer never showed up: the sample is done again, and consumers go on
+        wait_vmem_all();
+        if (tid == 0) { a.flags[b] = 1; store_agent(prog + g, 1 << 30); }
+    }
+}
+
 // best = max(best, max_{r<16} (a[lane r of this 16-lane row] + e[r])): two sums, then one three-way maximum
 // (24 instructions for 16 rows instead of 32; a maximum does not round, so the result is the same bit for bit)
 __device__ __forceinline__ void maxplus16_rowbcast(float &best, float av, const float *e) {
@@ -171,32 +675,56 @@ __device__ __forceinline__ float tile_maxplus(const Tile &t, float a0, float a1,
     return fmaxf(b0, b1);
 }
 
-// bytes per row of the source-block table (rows padded to 16 bytes)
-__host__ __device__ static inline int srcblk_pitch(int L) { return (L + 15) & ~15; }
-
-static int align_groups(int B, int L, int translen) { return groups_used((B + 7) & ~7, L, translen); }
-
-struct AlignTileArgs {
-    const void *match; int64_t ms0, ms1, ms2;
-    const void *links;
-    const int64_t *out_len, *tgt_len;
-    int B, T, L, translen;
-    float *table;     // [B][T][L] best score of every cell, by node
-    unsigned char *srcblk;   // [B][T][pitch] block of 64 nodes that holds the best predecessor of every cell (the lowest such block); 16-byte aligned rows
-    int *sync;        // [0] ticket counter, [16 + b*C + group] progress
-    int *flags;       // [B] set when the pipeline gave up on a sample
-    int C;
-    int mcap;         // match row read at step s: min(s, mcap) (T-1 for the alignment: every step its own row)
-    int decode;       // Viterbi decoding: every sample runs all T steps (tgt_len is not read) and no cell is
-                      // pruned for being too far from the last node -- a path may end at any step
-    unsigned char gtab[kMaxBlocksFast + 1][12];
-};
-
-// Same workgroup pipeline as the loss sweeps (tickets, one-way hand-over through the table with
-// agent-scope accesses, bounded waits), in the (max, +) semiring and without any rescaling: the
-// table holds the plain fp32 scores.
+// The same sweep step by step, for few steps on many nodes (launch_align_sweep): the groups follow each other a few steps
+// apart instead of a few stages, and a step waits for nobody but the group below.
+//
+// One tile of scores: t.p[r] = E(node 64 I + r -> node 64 J + lane), -inf where there is no transition; sixteen loads in
+// flight (clamped to element 0).
+template <typename TL>
+__device__ __forceinline__ void load_scores(Tile &t, const TL *links, int I, int J, int lane, int Lb, int translen) {
+    const int dd = (J - I) * kBlk - 1;   // distance: dd + lane - r
+    const char *const lbase = reinterpret_cast<const char *>(links);
+    // every (row, lane) of the tile is a transition of the sample (wave-uniform)
+    const bool interior = J > I && dd + kBlk - 1 < translen && J * kBlk + kBlk - 1 < Lb;
+    constexpr int CH = 16;
+    const int p_out = J * kBlk + lane;
+    const int base = I * kBlk * translen + dd + lane;
+    const int step = translen - 1;
+    const bool col_ok = p_out < Lb;
+    TL raw[2][CH];
+    auto request = [&](const int c, TL (&dst)[CH]) __attribute__((always_inline)) {
+#pragma unroll
+        for (int r = 0; r < CH; ++r) {
+            const int d = dd + lane - (c + r);
+            const bool valid = col_ok && d >= 0 && d < translen;
+            dst[r] = *reinterpret_cast<const TL *>(lbase + (interior || valid ? (unsigned)(base + (c + r) * step) * (unsigned)sizeof(TL) : 0u));
+        }
+    };
+    request(0, raw[0]);
+#pragma unroll
+    for (int k = 0; k < kBlk / CH; ++k) {
+        const int c = k * CH;
+        if (k + 1 < kBlk / CH) request(c + CH, raw[(k + 1) & 1]);
+        __builtin_amdgcn_sched_barrier(0);
+        const TL (&e)[CH] = raw[k & 1];
+        if (interior) {
+#pragma unroll
+            for (int r = 0; r < CH; ++r) t.p[c + r] = to_float(e[r]);
+        } else {
+            bool valid[CH];
+#pragma unroll
+            for (int r = 0; r < CH; ++r) {
+                const int d = dd + lane - (c + r);
+                valid[r] = col_ok && d >= 0 && d < translen;
+            }
+#pragma unroll
+            for (int r = 0; r < CH; ++r) t.p[c + r] = valid[r] ? to_float(e[r]) : DAGX_NEG_INF;
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    }
+}
 template <typename TM, typename TL>
-__global__ __launch_bounds__(kTileWaves * kWave) void dag_align_tiles_kernel(AlignTileArgs a) {
+__global__ __launch_bounds__(kTileWaves * kWave) void dag_align_steps_kernel(AlignTileArgs a) {
     __shared__ float abuf[2][kMaxBlocksFast][kBlk];   // scores of the previous / next step, by node
     // tile results: the tiles of an owned block lie in consecutive rows that start at a multiple of eight, and the rows
     // behind them, up to the next multiple of eight, hold -inf for good: the owner reads whole eights without a test
@@ -236,7 +764,7 @@ __global__ __launch_bounds__(kTileWaves * kWave) void dag_align_tiles_kernel(Ali
     const int mcap = a.mcap;
     const int NBb = (Lb + kBlk - 1) / kBlk;
     const int W = (translen + kBlk - 1) / kBlk;
-    if (tid <= C) gstart[tid] = a.gtab[NBb][tid];
+    if (tid <= C) gstart[tid] = a.plan.gtab[NBb][tid];
     __syncthreads();
     const int jb0 = __builtin_amdgcn_readfirstlane(gstart[g]), jb1 = __builtin_amdgcn_readfirstlane(gstart[g + 1]);
     int last_group = 0;
@@ -250,7 +778,7 @@ __global__ __launch_bounds__(kTileWaves * kWave) void dag_align_tiles_kernel(Ali
 
     int ntile = 0;
     for (int Jb = jb0; Jb < jb1; ++Jb) ntile += Jb - tile_ilo(Jb, W) + 1;
-    // The last wave is the fetcher (see the loss sweep kernel) and takes tiles only when the others cannot
+    // The last wave is the fetcher (it works one step ahead of the others, see fetch_step) and takes tiles only when the others cannot
     // hold them all; the tiles are dealt out evenly, the odd ones first to wave 3 (the fetcher's SIMD).
     const int nwork = ntile <= kTilesPerWave * (kTileWaves - 1) ? kTileWaves - 1 : kTileWaves;
     int my_first = 0, my_count = 0;
@@ -282,9 +810,9 @@ __global__ __launch_bounds__(kTileWaves * kWave) void dag_align_tiles_kernel(Ali
         }
     }
     Tile t0, t1, t2;
-    if (my_q[0] >= 0) load_tile<false, 16>(t0, links, my_I[0], my_J[0], lane, 0, Lb, translen, nullptr, 0.f);
-    if (my_q[1] >= 0) load_tile<false, 16>(t1, links, my_I[1], my_J[1], lane, 0, Lb, translen, nullptr, 0.f);
-    if (my_q[2] >= 0) load_tile<false, 16>(t2, links, my_I[2], my_J[2], lane, 0, Lb, translen, nullptr, 0.f);
+    if (my_q[0] >= 0) load_scores(t0, links, my_I[0], my_J[0], lane, Lb, translen);
+    if (my_q[1] >= 0) load_scores(t1, links, my_I[1], my_J[1], lane, Lb, translen);
+    if (my_q[2] >= 0) load_scores(t2, links, my_I[2], my_J[2], lane, Lb, translen);
 
     const char *table_c = reinterpret_cast<const char *>(table);
     const char *match_c = reinterpret_cast<const char *>(match);
@@ -307,7 +835,7 @@ __global__ __launch_bounds__(kTileWaves * kWave) void dag_align_tiles_kernel(Ali
         const int p = (jb0 + ob) * kBlk + lane;
         if (p < Lb) store_agent(cell(0, p), p == 0 ? m0 : DAGX_NEG_INF);
     }
-    // ---- staging slots (see the loss sweep kernel): match rows of own blocks wave and wave + 8, table
+    // ---- staging slots: match rows of own blocks wave and wave + 8, table
     //      rows of foreign blocks flo + wave and flo + wave + 8, all filled by the fetcher ----
     constexpr int kFetchSlots = 2;
     int f_blk[kFetchSlots];
@@ -320,12 +848,11 @@ __global__ __launch_bounds__(kTileWaves * kWave) void dag_align_tiles_kernel(Ali
     auto lds_addr = [&](const void *p) -> unsigned { return (unsigned)reinterpret_cast<uintptr_t>(p); };
     const bool fetcher = wave == kTileWaves - 1;
     int seen = 0;   // last progress value of the group below that the fetcher has read
-    // The fetcher works one step ahead, as in the loss sweep: in phase A of step s it waits for what it requested
+    // The fetcher works one step ahead: in phase A of step s it waits for what it requested
     // a step ago (the rows phase B of step s reads), then requests the match rows of step s + 1, the foreign table
     // rows of step s + 1 if the snapshot of the producer's progress word (requested a step ago) shows them
     // published, and the next snapshot.  Only when the producer is less than two steps ahead does it poll the word
     // and fetch in the same step (one memory round trip inside phase A, which used to be every step's price).
-#define DAGX_STAMP(COND, SLOT)
     int rows_issued = 0;   // the foreign table rows of steps <= rows_issued have been requested
     auto issue_match = [&](const int s2, const int lane) __attribute__((always_inline)) {
         const int par = s2 & 1;
@@ -354,7 +881,6 @@ __global__ __launch_bounds__(kTileWaves * kWave) void dag_align_tiles_kernel(Ali
             if (snap > seen) seen = snap;
             if (rows_issued < s) {   // not requested yet: poll the producer's word
                 int spins = 0;
-                DAGX_STAMP(lane == 0, 5)   // (a step that had to poll)
                 while (seen < s) {   // the rows of step s are published once the word reaches s
                     seen = __builtin_amdgcn_readfirstlane(load_agent(below));
                     if (seen >= s) break;
@@ -415,10 +941,8 @@ __global__ __launch_bounds__(kTileWaves * kWave) void dag_align_tiles_kernel(Ali
     int cur = 0;
     for (int s = 1; s < Tb; ++s) {
         const int nxt = cur ^ 1;
-        DAGX_STAMP(tid == 0, 1)
         // ---- phase A: tile max-plus products; the fetcher's copies ----
         if (__builtin_expect(fetcher, 0)) fetch_step(s);
-        DAGX_STAMP(fetcher && lane == 0, 4)
         {
             // The scores for a tile are requested one tile ahead of its arithmetic.  A tile whose predecessor block
             // holds no finite score, or whose block lies outside the band, is skipped.
@@ -455,7 +979,6 @@ __global__ __launch_bounds__(kTileWaves * kWave) void dag_align_tiles_kernel(Ali
         // fetch; its requests for step s+1 stay in flight until the top of its next fetch.)
         if (!fetcher) wait_vmem_all();
         __syncthreads();
-        DAGX_STAMP(tid == 0, 2)
         // ---- phase B ----
         if (__builtin_expect(tid == 0 && producer, 0)) store_agent(prog + g, s - 1);
         const int par = s & 1;
@@ -501,7 +1024,6 @@ __global__ __launch_bounds__(kTileWaves * kWave) void dag_align_tiles_kernel(Ali
             }
         }
         __syncthreads();
-        DAGX_STAMP(tid == 0, 3)
         if (__builtin_amdgcn_readfirstlane(gave_up_v)) {
             if (tid == 0) { a.flags[b] = 1; store_agent(prog + g, 1 << 30); }
             return;
@@ -513,7 +1035,6 @@ __global__ __launch_bounds__(kTileWaves * kWave) void dag_align_tiles_kernel(Ali
         __syncthreads();
         if (tid == 0) store_agent(prog + g, Tb - 1);
     }
-#undef DAGX_STAMP
 }
 
 // Walking the path backwards through the score table.  The sweep has recorded, for every cell, the lowest block of 64
@@ -737,7 +1258,7 @@ static bool trace_fits_lds(int T, int L) {
 // workspace: [score table B*T*L f32 | sync 16 + B*C ints | flags B ints | source blocks B*T*L bytes] (tile path) then
 //            [trace B*T*L i32] when the back-pointers of the one-workgroup kernel do not fit LDS
 static size_t align_tile_words(int B, int T, int L, int translen) {
-    const int C = align_groups(B, L, translen);
+    const int C = align_groups(B, T, L, translen);
     // the last terms: one byte per cell in rows of srcblk_pitch(L) bytes, and room to start them on a 16-byte boundary
     return C > 0 ? (size_t)B * T * L + 16 + (size_t)B * C + (size_t)B + 4 + (size_t)B * T * srcblk_pitch(L) / 4 : 0;
 }
@@ -763,6 +1284,34 @@ static int raise_lds_limit(const void *kern, size_t bytes, std::atomic<unsigned 
     done.fetch_or(bit, std::memory_order_release);
     return DAGX_OK;
 }
+template <typename TM, typename TL, int SPACING>
+static int prepare_align_chunks() {
+    static std::atomic<unsigned long long> done{0};
+    return raise_lds_limit(reinterpret_cast<const void *>(dag_align_chunks_kernel<TM, TL, SPACING>), kChunkLdsBytes, done, "dag_best_alignment");
+}
+template <typename TM, typename TL, int SPACING>
+static int launch_align_chunks(AlignTileArgs &ta, const char *who, hipStream_t st) {
+    static const ChunkCosts costs[1] = {{SPACING == 1 ? 62 : 36, 27, 4, 75}};   // (measured)
+    ta.plan = chunk_plan<SPACING>(ta.translen, ta.C, costs);
+    if (int rc = prepare_align_chunks<TM, TL, SPACING>()) return rc;
+    hipLaunchKernelGGL((dag_align_chunks_kernel<TM, TL, SPACING>), dim3(((ta.B + 7) & ~7) * ta.C), dim3(kTileWaves * kWave), kChunkLdsBytes, st, ta);
+    return check_launch(who);
+}
+template <typename TM, typename TL>
+static int launch_align_sweep(AlignTileArgs &ta, const char *who, hipStream_t st) {
+    const int NB = (ta.L + kBlk - 1) / kBlk;
+    if (!align_in_chunks(ta.B, ta.T, ta.L, ta.translen)) {
+        const int W = (ta.translen + kBlk - 1) / kBlk;
+        int first[kTileCap + 2];
+        for (int nb = 0; nb <= kMaxBlocksFast; ++nb) {
+            partition_blocks(nb, W, ta.C, first);
+            for (int q = 0; q <= ta.C && q < 12; ++q) ta.plan.gtab[nb][q] = (unsigned char)first[q];
+        }
+        hipLaunchKernelGGL((dag_align_steps_kernel<TM, TL>), dim3(((ta.B + 7) & ~7) * ta.C), dim3(kTileWaves * kWave), 0, st, ta);
+        return check_launch(who);
+    }
+    return NB <= 5 || (NB <= 8 && 2 * NB <= 3 * ta.C) ? launch_align_chunks<TM, TL, 2>(ta, who, st) : launch_align_chunks<TM, TL, 1>(ta, who, st);
+}
 constexpr size_t kBacktrackMostLds = kAlignLdsBudget > kWalkLds ? kAlignLdsBudget : kWalkLds;   // (the redo alone asks for at most the former)
 template <typename TM, typename TL, bool TRACE_LDS, bool STAGED>
 static int prepare_backtrack() {
@@ -783,7 +1332,7 @@ static int launch_align(AlignArgs a, void *workspace, hipStream_t st) {
     constexpr int NT = 1024;
     const size_t tile_words = align_tile_words(a.B, a.T, a.L, a.translen);
     a.trace_ws = reinterpret_cast<int32_t *>(static_cast<float *>(workspace) + tile_words);
-    int C = align_groups(a.B, a.L, a.translen);
+    int C = align_groups(a.B, a.T, a.L, a.translen);
     const int64_t span = (int64_t)(a.T - 1) * (a.ms1 < 0 ? -a.ms1 : a.ms1) + (int64_t)(a.L - 1) * (a.ms2 < 0 ? -a.ms2 : a.ms2);
     if (span >= (1LL << 31) / (int64_t)sizeof(TM) || a.ms1 < 0 || a.ms2 < 0 || force_log_domain()) C = 0;
     if (C > 0) {
@@ -795,21 +1344,11 @@ static int launch_align(AlignArgs a, void *workspace, hipStream_t st) {
         ta.flags = ta.sync + 16 + a.B * C;
         ta.srcblk = reinterpret_cast<unsigned char *>((reinterpret_cast<uintptr_t>(ta.flags + a.B) + 15) & ~(uintptr_t)15);
         ta.C = C; ta.mcap = a.T - 1; ta.decode = 0;
-        {
-            const int W = (a.translen + kBlk - 1) / kBlk;
-            int tmp[kTileCap + 2];
-            for (int nb = 0; nb <= kMaxBlocksFast; ++nb) {
-                partition_blocks(nb, W, C, tmp);
-                for (int q = 0; q <= C && q < 12; ++q) ta.gtab[nb][q] = (unsigned char)tmp[q];
-            }
-        }
         const int nfill = 16 + a.B * C + a.B;
         hipLaunchKernelGGL(dag_align_fill_kernel, dim3((nfill + 255) / 256), dim3(256), 0, st, ta.sync, nfill, a.B, redo_every_sample() ? 1 : 0);
         int rc = check_launch("dag_align_fill");
         if (rc) return rc;
-        const int B8 = (a.B + 7) & ~7;
-        hipLaunchKernelGGL((dag_align_tiles_kernel<TM, TL>), dim3(B8 * C), dim3(kTileWaves * kWave), 0, st, ta);
-        if ((rc = check_launch("dag_align_tiles"))) return rc;
+        if ((rc = launch_align_sweep<TM, TL>(ta, "dag_align_sweep", st))) return rc;
         // the backtrack, and the samples that the pipeline gave up on.  (float32, kernel time: walked in memory 39.5 us at
         // B=64 L=512 T=64 and 172 us at B=16 L=1024 T=256, out of LDS 27.6 and 62.5 us.)
         const bool in_lds = trace_fits_lds(a.T, a.L);
@@ -1088,6 +1627,12 @@ static int prepare_walks() {
     int rc = prepare_backtracks<float, TL>();
     if (!rc) rc = prepare_backtracks<__half, TL>();
     if (!rc) rc = prepare_backtracks<bf16_t, TL>();
+    if (!rc) rc = prepare_align_chunks<float, TL, 1>();
+    if (!rc) rc = prepare_align_chunks<float, TL, 2>();
+    if (!rc) rc = prepare_align_chunks<__half, TL, 1>();
+    if (!rc) rc = prepare_align_chunks<__half, TL, 2>();
+    if (!rc) rc = prepare_align_chunks<bf16_t, TL, 1>();
+    if (!rc) rc = prepare_align_chunks<bf16_t, TL, 2>();
     return rc ? rc : prepare_select<TL>();
 }
 int prepare_align_kernels() {
@@ -1101,7 +1646,7 @@ static size_t decode_words(int B, int T, int L, int translen, int C) {
     return (size_t)B * T * L + 16 + (size_t)B * (C > 0 ? C : 1) + (size_t)B + 4 + (size_t)B * T * srcblk_pitch(L) / 4 + (size_t)B * 3 * L;
 }
 size_t decode_workspace_bytes(int B, int max_length, int L, int translen) {
-    return decode_words(B, max_length + 1, L, translen, align_groups(B, L, translen)) * 4;
+    return decode_words(B, max_length + 1, L, translen, align_groups(B, max_length + 1, L, translen)) * 4;
 }
 
 template <typename TL>
@@ -1110,7 +1655,7 @@ static int launch_decode(const void *links, const float *node_logp, const int64_
                          int64_t *out_tokens, int64_t *out_count, int64_t *pred_length, int64_t *nodes,
                          void *workspace, hipStream_t st) {
     const int T = max_length + 1;
-    int C = align_groups(B, L, translen);
+    int C = align_groups(B, T, L, translen);
     const int Cw = C > 0 ? C : 1;
     if (force_log_domain()) C = 0;
     float *table = static_cast<float *>(workspace);
@@ -1130,15 +1675,7 @@ static int launch_decode(const void *links, const float *node_logp, const int64_
         ta.out_len = out_len; ta.tgt_len = nullptr; ta.B = B; ta.T = T; ta.L = L; ta.translen = translen;
         ta.table = table; ta.sync = sync; ta.flags = flags; ta.srcblk = srcblk;
         ta.C = C; ta.mcap = 2; ta.decode = 1;
-        const int W = (translen + kBlk - 1) / kBlk;
-        int tmp[kTileCap + 2];
-        for (int nb = 0; nb <= kMaxBlocksFast; ++nb) {
-            partition_blocks(nb, W, C, tmp);
-            for (int q = 0; q <= C && q < 12; ++q) ta.gtab[nb][q] = (unsigned char)tmp[q];
-        }
-        const int B8 = (B + 7) & ~7;
-        hipLaunchKernelGGL((dag_align_tiles_kernel<float, TL>), dim3(B8 * C), dim3(kTileWaves * kWave), 0, st, ta);
-        if ((rc = check_launch("viterbi_tiles"))) return rc;
+        if ((rc = launch_align_sweep<float, TL>(ta, "viterbi_sweep", st))) return rc;
     }
     constexpr int NT = 1024;
     hipLaunchKernelGGL((viterbi_table_kernel<TL, NT>), dim3(B), dim3(NT), (size_t)L * 8, st, match3, static_cast<const TL *>(links),

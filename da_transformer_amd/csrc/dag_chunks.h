@@ -1,18 +1,19 @@
-// The float32 sweep of dag_loss.hip in chunks of four steps: what a position block receives from the blocks below it is
-// a matrix product over the chunk's steps, on the matrix cores; only the 64 x 64 triangle on the diagonal is walked
-// step by step, by one wave.
+// The sweeps of dag_loss.hip (log-semiring) and dag_align.hip (max-semiring) in chunks of four steps: what a position block
+// receives from the blocks below it is formed for four steps at once (in the loss on the matrix cores); only the 64 x 64
+// triangle on the diagonal is walked step by step, by one wave.
 #pragma once
 
 #include "dag_tiles.h"
 
 namespace dagx {
 
-// Position block J works on chunk c (steps 4c+1 .. 4c+4) in stage J + c, and one barrier a stage is the only synchronisation
-// of a workgroup.  What it receives from block J - 1, which worked on that chunk one stage earlier, the walking wave itself
-// multiplies out when the stage begins; what it receives from the blocks below that one is multiplied out one stage
-// ahead, by waves that are not on the critical path.
+// With SPACING 1 position block J works on chunk c (steps 4c+1 .. 4c+4) in stage J + c, with SPACING 2 in stage 2J + c; one
+// barrier a stage is the only synchronisation of a workgroup.  What a block receives from the blocks below it is formed one
+// stage ahead, by waves that are not on the critical path -- with SPACING 1 but for what it receives from block J - 1, which
+// worked on that chunk only one stage earlier: that the walking wave itself forms when the stage begins.  So SPACING 1
+// (the loss) has longer stages, by one tile, and one a block less: right where a tile is cheap beside a walk.
 //
-// Numbers are linear: a cell holds exp(value - kap ln 2) 2^kShift with one integer exponent kap per block and step,
+// In the loss numbers are linear: a cell holds exp(value - kap ln 2) 2^kShift with one integer exponent kap per block and step,
 // chosen so that the block's largest cell lies in [2^(kShift-1), 2^kShift).  All scaling is by powers of two.
 //
 // The wide variant keeps cells, products and sums in float64; the staged transitions stay float32 registers (the register
@@ -44,8 +45,9 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef int i32x4 __attribute__((ext_vector_type(4)));
 typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
 
-// Tiles that are multiplied out a stage ahead: those below the diagonal but for the one next to it.
-__device__ __host__ __forceinline__ int tiles_of_block(int J, int W) { const int n = J < W ? J : W; return n > 1 ? n - 1 : 0; }
+// Tiles that are multiplied out a stage ahead: those below the diagonal, with SPACING 1 but for the one next to it.
+template <int SPACING>
+__device__ __host__ __forceinline__ int tiles_of_block(int J, int W) { const int n = (J < W ? J : W) - (2 - SPACING); return n > 0 ? n : 0; }
 
 // LDS of a group, in dwords.
 struct ChunkLds {
@@ -64,7 +66,7 @@ __device__ __host__ inline ChunkLds chunk_lds(int jb0, int nblk, int W, bool wid
     ChunkLds o;
     const int flo = tile_ilo(jb0, W), nfor = jb0 - flo, nsrc = nfor + nblk, chunk = wide ? 512 : 256;
     int ntile = 0;
-    for (int q = 0; q < nblk; ++q) ntile += tiles_of_block(jb0 + q, W);
+    for (int q = 0; q < nblk; ++q) ntile += tiles_of_block<1>(jb0 + q, W);
     const int reach = nblk < W ? nblk : W;
     o.depth = reach + 1 < 3 ? 3 : reach + 1;
     o.runs = ntile < kTileWaves + nblk - 1 ? ntile : kTileWaves + nblk - 1;
@@ -89,40 +91,49 @@ constexpr int kForeign = 3;                  // foreign blocks a wave fetches at
 constexpr int kChunkLdsBytes = 160 * 1024 - 512;
 
 // Those tiles, block by block, are dealt to the waves in runs: at most three to a wave that walks no block (a helper), at
-// most one to one that does (the triangle and the tile next to it take the registers of two), and the foreign blocks
-// to the helpers that fetch them.  What a wave does in a stage, in hundreds of cycles (measured): walking 45 with the
-// adjacent tile's product, a tile 7, fetching a foreign block 4; in float64 85, 17 and 11.  Waves w and w + 4 share a SIMD, on which all of it
-// adds up: each tile goes where least is to be done.
+// most SPACING to one that does (the triangle, and with SPACING 1 the tile next to it, take registers), and the foreign blocks
+// to the helpers that fetch them: each to the wave that is done first with it.
 struct TileDeal { unsigned wave; };          // four bits a wave: tiles, foreign blocks << 2
 __device__ __host__ __forceinline__ int dealt_tiles(const TileDeal &d, int wave) { return (d.wave >> (4 * wave)) & 3; }
 __device__ __host__ __forceinline__ int dealt_foreign(const TileDeal &d, int wave) { return (d.wave >> (4 * wave + 2)) & 3; }
-// returns what the busiest SIMD has to do, -1 if there are more tiles than the waves have room for
-inline int deal_tiles(int jb0, int nblk, int W, bool wide, TileDeal &deal) {   // (on the host: a plan made by the kernel costs it 2 us)
-    const int kWalk = wide ? 85 : 45, kProduct = wide ? 17 : 7, kFetch = wide ? 11 : 4;
+// returns how long the busiest wave or SIMD takes, -1 if there are more tiles than the waves have room for
+// What a wave does in a stage, in hundreds of cycles, alone on its SIMD: walking a block (with SPACING 1 with the product
+// of the adjacent tile), a tile, fetching a foreign block; and how much of the sum of two waves' work a SIMD takes for both, in per cent
+// (waves w and w + 4 share one).
+struct ChunkCosts { int walk, product, fetch, shared; };
+template <int SPACING>
+inline int deal_tiles(int jb0, int nblk, int W, const ChunkCosts &cost, TileDeal &deal) {   // (on the host: a plan made by the kernel costs it 2 us)
     constexpr int kSimds = 4;
-    int load[kSimds] = {0, 0, 0, 0}, tiles[kTileWaves] = {0}, foreign[kTileWaves] = {0};
-    for (int w = 0; w < nblk; ++w) load[w % kSimds] += kWalk;
+    int load[kTileWaves] = {0}, tiles[kTileWaves] = {0}, foreign[kTileWaves] = {0};
+    for (int w = 0; w < nblk; ++w) load[w] = cost.walk - (SPACING == 1 && jb0 + w == 0 ? cost.product : 0);
     int ntile = 0;
     const int nfor = jb0 - tile_ilo(jb0, W);
-    for (int q = 0; q < nblk; ++q) ntile += tiles_of_block(jb0 + q, W);
-    auto place = [&](int (&count)[kTileWaves], const bool fetch, const int cost) {
+    for (int q = 0; q < nblk; ++q) ntile += tiles_of_block<SPACING>(jb0 + q, W);
+    auto busy = [&](const int w, const int more) {   // until when wave w (with `more` to do) keeps its SIMD or itself busy
+        const int both = (load[w] + load[(w + kSimds) % kTileWaves] + more) * cost.shared / 100;
+        return load[w] + more > both ? load[w] + more : both;
+    };
+    auto place = [&](int (&count)[kTileWaves], const bool fetch, const int work) {
         int best = -1;
         for (int w = kTileWaves - 1; w >= 0; --w) {
-            const int most = fetch ? (w >= nblk || nblk == kTileWaves ? kForeign : 0) : (w >= nblk ? kTilesPerWave : 1);
+            const int most = fetch ? (w >= nblk || nblk == kTileWaves ? kForeign : 0) : (w >= nblk ? kTilesPerWave : SPACING);
             if (count[w] >= most) continue;
-            if (best < 0 || load[w % kSimds] < load[best % kSimds] || (load[w % kSimds] == load[best % kSimds] && count[w] < count[best])) best = w;
+            const int now = best < 0 ? 0 : busy(w, work) - busy(best, work);
+            if (best < 0 || now < 0 || (now == 0 && count[w] < count[best])) best = w;
         }
         if (best < 0) return false;
         ++count[best];
-        load[best % kSimds] += cost;
+        load[best] += work;
         return true;
     };
-    for (int n = 0; n < ntile; ++n) if (!place(tiles, false, kProduct)) return -1;
-    for (int n = 0; n < nfor; ++n) if (!place(foreign, true, kFetch)) return -1;
+    for (int n = 0; n < ntile; ++n) if (!place(tiles, false, cost.product)) return -1;
+    for (int n = 0; n < nfor; ++n) if (!place(foreign, true, cost.fetch)) return -1;
     deal.wave = 0;
     int most = 0;
-    for (int w = 0; w < kTileWaves; ++w) deal.wave |= (unsigned)(tiles[w] | foreign[w] << 2) << (4 * w);
-    for (int x = 0; x < kSimds; ++x) most = load[x] > most ? load[x] : most;
+    for (int w = 0; w < kTileWaves; ++w) {
+        deal.wave |= (unsigned)(tiles[w] | foreign[w] << 2) << (4 * w);
+        most = busy(w, 0) > most ? busy(w, 0) : most;
+    }
     return most;
 }
 // first tile, number of tiles, first foreign block and number of foreign blocks of a wave (the helpers' tiles first,
@@ -139,27 +150,33 @@ __device__ __host__ __forceinline__ void wave_foreign(const TileDeal &d, int wav
 // Host: the groupings of a graph's position blocks for every number of blocks up to NB, each into at most C contiguous
 // groups of at most kTileCap tiles (the diagonal ones among them) and kChunkBlocks blocks so that the busiest SIMD has
 // least to do.  gtab[nb][g] .. gtab[nb][g+1]: blocks of group g (empty groups last).
+template <int N>
 struct ChunkPlan {
     unsigned char gtab[kMaxBlocksFast + 1][12];
-    TileDeal deal[2][kMaxBlocksFast + 1][12];   // of the float32 and the float64 sweeps
+    TileDeal deal[N][kMaxBlocksFast + 1][12];     // one for each set of costs; the first set decides on the groups
 };
-inline void plan_chunks(int NB, int W, int C, ChunkPlan &plan) {
-    int cost[kMaxBlocksFast][kChunkBlocks + 1];
-    TileDeal deal[2][kMaxBlocksFast][kChunkBlocks + 1];
+template <int SPACING, int N>
+inline void plan_chunks(int W, int C, const ChunkCosts (&costs)[N], ChunkPlan<N> &plan) {
+    constexpr int NB = kMaxBlocksFast;
+    int cost[NB][kChunkBlocks + 1];
+    TileDeal deal[N][NB][kChunkBlocks + 1];
     for (int j = 0; j < NB; ++j) {
         int tiles = 0;
         for (int n = 1; n <= kChunkBlocks; ++n) {
             cost[j][n] = -1;
             if (j + n > NB) continue;
             tiles += j + n - tile_ilo(j + n - 1, W);
-            if (tiles <= kTileCap) { cost[j][n] = deal_tiles(j, n, W, false, deal[0][j][n]); deal_tiles(j, n, W, true, deal[1][j][n]); }
+            if (tiles > kTileCap) continue;
+            for (int x = N - 1; x >= 0; --x) cost[j][n] = deal_tiles<SPACING>(j, n, W, costs[x], deal[x][j][n]);
         }
     }
     for (int nb = 0; nb <= NB; ++nb) {
         int low = 0, high = 1 << 12;                 // the least bound on a group's cost that C groups can keep
-        auto split = [&](const int most, unsigned char *g) {
+        unsigned char g[16];
+        auto split = [&](const int most) {
             int used = 0, j = 0;
             g[0] = 0;
+            for (int q = 1; q < 16; ++q) g[q] = (unsigned char)nb;
             while (j < nb) {
                 int n = 0;
                 for (int x = 1; x <= kChunkBlocks && j + x <= nb; ++x) if (cost[j][x] >= 0 && cost[j][x] <= most) n = x;
@@ -167,17 +184,88 @@ inline void plan_chunks(int NB, int W, int C, ChunkPlan &plan) {
                 j += n;
                 g[++used] = (unsigned char)j;
             }
-            for (int q = used; q < C; ++q) g[q + 1] = (unsigned char)nb;
             return true;
         };
-        unsigned char g[16];
-        while (low < high) { const int mid = (low + high) / 2; if (split(mid, g)) high = mid; else low = mid + 1; }
-        split(high, g);
+        while (low < high) { const int mid = (low + high) / 2; if (split(mid)) high = mid; else low = mid + 1; }
+        split(high);
         for (int q = 0; q < 12; ++q) {
-            plan.gtab[nb][q] = q <= C ? g[q] : (unsigned char)nb;
-            for (int w = 0; w < 2; ++w) plan.deal[w][nb][q] = q < C && g[q + 1] > g[q] ? deal[w][g[q]][g[q + 1] - g[q]] : TileDeal{0};
+            plan.gtab[nb][q] = g[q];
+            for (int x = 0; x < N; ++x) plan.deal[x][nb][q] = q < C && g[q + 1] > g[q] && g[q + 1] - g[q] <= kChunkBlocks ? deal[x][g[q]][g[q + 1] - g[q]] : TileDeal{0};
         }
     }
+}
+// the plan for a window of W blocks and C groups, remembered for the thread's next call (a plan takes 20 us to make; there are
+// at most kMaxBlocksFast windows, and C follows from the batch)
+template <int SPACING, int N>
+inline const ChunkPlan<N> &chunk_plan(int translen, int C, const ChunkCosts (&costs)[N]) {
+    struct Entry { int C = 0; ChunkPlan<N> plan; };
+    static thread_local Entry entries[kMaxBlocksFast];
+    const int w = (translen + kBlk - 1) / kBlk, W = w < kMaxBlocksFast ? w : kMaxBlocksFast;
+    Entry &e = entries[W - 1];
+    if (e.C != C) { plan_chunks<SPACING>(W, C, costs, e.plan); e.C = C; }
+    return e.plan;
+}
+
+// ---- what a wave has to do, worked out at the start of the kernel ----
+// A run is a wave's tiles that lead to one block; runs are numbered in the order of the tiles.
+struct WaveTiles {
+    int count;                                     // tiles to multiply out a stage ahead
+    int I[kTilesPerWave], q[kTilesPerWave];        // source block, own block it leads to (a walking wave: slot 2 the triangle, with
+                                                   // SPACING 1 slot 0 the tile next to it)
+    int run[kTilesPerWave];                        // run it belongs to
+    bool ok[kTilesPerWave], start[kTilesPerWave], end[kTilesPerWave], lead[kTilesPerWave];   // (slots to multiply out a stage ahead;) first / last tile of its run; run that begins with the block's first tile
+    bool adjacent;                                 // slot 0 holds a tile next to the diagonal
+    int run_first, run_count;                      // the runs that lead to the block this wave walks
+};
+template <int SPACING>
+__device__ __forceinline__ WaveTiles plan_wave(const TileDeal &deal, int jb0, int nblk, int W, int none, int wave, int lane) {
+    WaveTiles t;
+    const int flo = tile_ilo(jb0, W);
+    const bool owner = wave < nblk;
+    int my_first;
+    wave_tiles(deal, wave, my_first, t.count);
+    // lane <-> block (f: its first tile) and lane <-> wave (w_first: its first tile)
+    int f = 0, w_first, w_count;
+#pragma unroll
+    for (int q = 0; q < kChunkBlocks; ++q) f += q < lane && q < nblk ? tiles_of_block<SPACING>(jb0 + q, W) : 0;
+    wave_tiles(deal, lane & (kTileWaves - 1), w_first, w_count);
+    int f_of[kChunkBlocks + 1];
+    bool cuts = lane < kTileWaves && w_count > 0;   // this wave's first tile begins a run in the middle of a block
+#pragma unroll
+    for (int q = 0; q <= kChunkBlocks; ++q) {
+        f_of[q] = __builtin_amdgcn_readlane(f, q);
+        if (q < nblk) cuts = cuts && !(w_first == f_of[q] && tiles_of_block<SPACING>(jb0 + q, W) > 0);
+    }
+    const int without = jb0 < 3 - SPACING ? 3 - SPACING - jb0 : 0;   // (block 0, with SPACING 1 also block 1, has no such tiles)
+    // number of runs that begin at or before tile n of block q
+    auto runs_to = [&](const int q, const int n) { return q + 1 - without + (int)__builtin_popcountll(__builtin_amdgcn_ballot_w64(cuts && w_first <= n)); };
+#pragma unroll
+    for (int u = 0; u < kTilesPerWave; ++u) {
+        const int r0 = SPACING == 1 && owner ? u - 1 : u, n = my_first + r0;
+        t.ok[u] = r0 >= 0 && r0 < t.count;
+        int q = 0;
+#pragma unroll
+        for (int x = 1; x < kChunkBlocks; ++x) q = x < nblk && n >= f_of[x] ? x : q;
+        const int lo = tile_ilo(jb0 + q, W), r = n - f_of[q];
+        t.q[u] = t.ok[u] ? q : 0;
+        t.I[u] = t.ok[u] ? lo + r : flo;
+        t.start[u] = r0 == 0 || r == 0;
+        t.end[u] = r0 == t.count - 1 || lo + r == jb0 + q - (3 - SPACING);
+        t.lead[u] = r0 >= r;
+        t.run[u] = runs_to(q, n) - 1;
+    }
+    t.run_first = none; t.run_count = 1;           // (a block without such tiles)
+    if (owner && tiles_of_block<SPACING>(jb0 + wave, W) > 0) {
+        const int n = __builtin_amdgcn_readlane(f, wave);
+        t.run_first = runs_to(wave, n) - 1;
+        t.run_count = runs_to(wave, n + tiles_of_block<SPACING>(jb0 + wave, W) - 1) - t.run_first;
+    }
+    t.adjacent = SPACING == 1 && owner && jb0 + wave > 0;
+    if (owner) {
+        t.I[kTilesPerWave - 1] = jb0 + wave; t.q[kTilesPerWave - 1] = wave;
+        if (SPACING == 1) { t.I[0] = jb0 + wave - (t.adjacent ? 1 : 0); t.q[0] = wave; }
+    }
+    return t;
 }
 
 // a = {a's lower half, b's lower half}, b = {a's upper half, b's upper half}.  (The results go through unsigned variables:
@@ -527,9 +615,9 @@ template <> struct Quad<float> { typedef f32x4 V; __device__ __forceinline__ sta
 template <> struct Quad<__half> { typedef h16x4 V; __device__ __forceinline__ static float get(V v, int k) { return (float)v[k]; } };
 template <> struct Quad<bf16_t> { typedef u16x4 V; __device__ __forceinline__ static float get(V v, int k) { return __uint_as_float((unsigned)v[k] << 16); } };
 
-// one tile -> exp(E) 2^SHIFT in the wave's patch; `tiny` as in link_prob.  before / behind: how many elements the
+// one tile -> exp(E) 2^SHIFT (or E itself: !EXP) in the wave's patch; `tiny` as in link_prob.  before / behind: how many elements the
 // tensor has in front of and behind the sample, where a load may reach (into places that are masked).
-template <typename TL, int SHIFT>
+template <typename TL, int SHIFT, bool EXP = true, int BATCH = 16>
 __device__ __forceinline__ void stage_tile(float *patch, const TL *links, int I, int J, int lane, int dir, int Lb, int translen, int last_index,
                                            int before, int behind, float tiny) {
     typedef typename Quad<TL>::V V;
@@ -538,86 +626,103 @@ __device__ __forceinline__ void stage_tile(float *patch, const TL *links, int I,
     const int step = 4 * (dir == 0 ? translen - 1 : 1 - translen);
     const int lowest_i = min(index0, index0 + 15 * step), highest_i = max(index0, index0 + 15 * step) + 3;
     float *const dst = patch + n0 * kPatchPitch + (dir == 0 ? c : kBlk - 4 - c);
-    // element k of group g (row n0 + 4 g): its distance is d0 + g dstep + k; it has a place in the sample for k < k_end(g)
+    // element k of group g (row n0 + 4 g): its distance is d0 + g dstep + k; it has a place in the sample for k < k_end(g0 + g)
     const int d0 = dir == 0 ? dd + c - n0 : dd + n0 - c - 3, dstep = dir == 0 ? -4 : 4;
     auto k_end = [&](const int g) { return dir == 0 ? Lb - J * kBlk - c : (J * kBlk + n0 + 4 * g < Lb ? 4 : 0); };
     auto valid = [&](const int g, const int k, const int ke) { return (unsigned)(d0 + g * dstep + k) < (unsigned)translen && k < ke; };
     const int back = kBlk * translen + 4 * kBlk;   // (an unsigned offset from a scalar base: one register a load)
     const char *const base = reinterpret_cast<const char *>(links) - (int64_t)back * (int64_t)sizeof(TL);
     auto load = [&](const int at) { V v; __builtin_memcpy(&v, base + (unsigned)(at + back) * (unsigned)sizeof(TL), sizeof(V)); return v; };
-    V raw[16];
-    if (__builtin_expect(__builtin_amdgcn_ballot_w64(lowest_i < -before || highest_i > last_index + behind) == 0, 1)) {
-#pragma unroll
-        for (int g = 0; g < 16; ++g) raw[g] = load(index0 + g * step);
-    } else {
-        // next to an end of the tensor (which has at least four elements): loads that would leave it are moved inside, and
-        // what they find there to where it belongs
-        const int most = last_index + behind - 3;
-#pragma unroll
-        for (int g = 0; g < 16; ++g) {
-            const int want = index0 + g * step;
-            raw[g] = load(want < -before ? -before : want > most ? most : want);
-        }
-#pragma unroll
-        for (int g = 0; g < 16; ++g) {
-            const int want = index0 + g * step, front = -before - want, over = want - most;
-#pragma unroll
-            for (int r = 1; r < 4; ++r) {
-                const V v = raw[g];
-                raw[g][0] = over >= r ? v[1] : v[0];
-                raw[g][1] = front >= r ? v[0] : over >= r ? v[2] : v[1];
-                raw[g][2] = front >= r ? v[1] : over >= r ? v[3] : v[2];
-                raw[g][3] = front >= r ? v[2] : v[3];
-            }
-        }
-    }
     // every (row, column) of the tile is a transition of the sample
     const bool interior = J > I && dd + kBlk - 1 < translen && J * kBlk + kBlk - 1 < Lb;
-    float lowest = 0.f;
-    if (interior) {
+    const bool inside = __builtin_amdgcn_ballot_w64(lowest_i < -before || highest_i > last_index + behind) == 0;
+    // (BATCH loads in flight: sixteen, fewer where the registers would not do)
 #pragma unroll
-        for (int g = 0; g < 16; ++g)
+    for (int g0 = 0; g0 < 16; g0 += BATCH) {
+        if (BATCH < 16) __builtin_amdgcn_sched_barrier(0);
+        V raw[BATCH];
+        if (__builtin_expect(inside, 1)) {
 #pragma unroll
-            for (int k = 0; k < 4; ++k) lowest = fminf(lowest, Quad<TL>::get(raw[g], k));
-        if (__builtin_amdgcn_ballot_w64(lowest < -79.f) == 0) {
+            for (int g = 0; g < BATCH; ++g) raw[g] = load(index0 + (g0 + g) * step);
+        } else {
+            // next to an end of the tensor (which has at least four elements): loads that would leave it are moved inside, and
+            // what they find there to where it belongs
+            const int most = last_index + behind - 3;
 #pragma unroll
-            for (int g = 0; g < 16; ++g) {
-                f32x4 w;
-#pragma unroll
-                for (int k = 0; k < 4; ++k) w[k] = __builtin_ldexpf(fast_exp2(Quad<TL>::get(raw[g], k) * kLog2e), SHIFT);
-                *reinterpret_cast<f32x4 *>(dst + 4 * g * kPatchPitch) = w;
+            for (int g = 0; g < BATCH; ++g) {
+                const int want = index0 + (g0 + g) * step;
+                raw[g] = load(want < -before ? -before : want > most ? most : want);
             }
-            return;
-        }
-    } else {
 #pragma unroll
-        for (int g = 0; g < 16; ++g) {
-            const int ke = k_end(g);
+            for (int g = 0; g < BATCH; ++g) {
+                const int want = index0 + (g0 + g) * step, front = -before - want, over = want - most;
 #pragma unroll
-            for (int k = 0; k < 4; ++k) lowest = fminf(lowest, valid(g, k, ke) ? Quad<TL>::get(raw[g], k) : 0.f);
-        }
-        if (__builtin_amdgcn_ballot_w64(lowest < -79.f) == 0) {
-#pragma unroll
-            for (int g = 0; g < 16; ++g) {
-                f32x4 w;
-                const int ke = k_end(g);
-#pragma unroll
-                for (int k = 0; k < 4; ++k) {
-                    const float v = __builtin_ldexpf(fast_exp2(Quad<TL>::get(raw[g], k) * kLog2e), SHIFT);
-                    w[k] = valid(g, k, ke) ? v : 0.f;
+                for (int r = 1; r < 4; ++r) {
+                    const V v = raw[g];
+                    raw[g][0] = over >= r ? v[1] : v[0];
+                    raw[g][1] = front >= r ? v[0] : over >= r ? v[2] : v[1];
+                    raw[g][2] = front >= r ? v[1] : over >= r ? v[3] : v[2];
+                    raw[g][3] = front >= r ? v[2] : v[3];
                 }
-                *reinterpret_cast<f32x4 *>(dst + 4 * g * kPatchPitch) = w;
             }
-            return;
         }
-    }
+        if constexpr (!EXP) {                    // the scores themselves, -inf where there is no transition
 #pragma unroll
-    for (int g = 0; g < 16; ++g) {
-        f32x4 w;
-        const int ke = k_end(g);
+            for (int g = 0; g < BATCH; ++g) {
+                f32x4 w;
+                const int ke = k_end(g0 + g);
 #pragma unroll
-        for (int k = 0; k < 4; ++k) w[k] = link_prob<true, SHIFT>(Quad<TL>::get(raw[g], k), valid(g, k, ke), tiny);
-        *reinterpret_cast<f32x4 *>(dst + 4 * g * kPatchPitch) = w;
+                for (int k = 0; k < 4; ++k) w[k] = interior || valid(g0 + g, k, ke) ? Quad<TL>::get(raw[g], k) : DAGX_NEG_INF;
+                *reinterpret_cast<f32x4 *>(dst + 4 * (g0 + g) * kPatchPitch) = w;
+            }
+            continue;
+        }
+        float lowest = 0.f;
+        if (interior) {
+#pragma unroll
+            for (int g = 0; g < BATCH; ++g)
+#pragma unroll
+                for (int k = 0; k < 4; ++k) lowest = fminf(lowest, Quad<TL>::get(raw[g], k));
+            if (__builtin_amdgcn_ballot_w64(lowest < -79.f) == 0) {
+#pragma unroll
+                for (int g = 0; g < BATCH; ++g) {
+                    f32x4 w;
+#pragma unroll
+                    for (int k = 0; k < 4; ++k) w[k] = __builtin_ldexpf(fast_exp2(Quad<TL>::get(raw[g], k) * kLog2e), SHIFT);
+                    *reinterpret_cast<f32x4 *>(dst + 4 * (g0 + g) * kPatchPitch) = w;
+                }
+                continue;
+            }
+        } else {
+#pragma unroll
+            for (int g = 0; g < BATCH; ++g) {
+                const int ke = k_end(g0 + g);
+#pragma unroll
+                for (int k = 0; k < 4; ++k) lowest = fminf(lowest, valid(g0 + g, k, ke) ? Quad<TL>::get(raw[g], k) : 0.f);
+            }
+            if (__builtin_amdgcn_ballot_w64(lowest < -79.f) == 0) {
+#pragma unroll
+                for (int g = 0; g < BATCH; ++g) {
+                    f32x4 w;
+                    const int ke = k_end(g0 + g);
+#pragma unroll
+                    for (int k = 0; k < 4; ++k) {
+                        const float v = __builtin_ldexpf(fast_exp2(Quad<TL>::get(raw[g], k) * kLog2e), SHIFT);
+                        w[k] = valid(g0 + g, k, ke) ? v : 0.f;
+                    }
+                    *reinterpret_cast<f32x4 *>(dst + 4 * (g0 + g) * kPatchPitch) = w;
+                }
+                continue;
+            }
+        }
+#pragma unroll
+        for (int g = 0; g < BATCH; ++g) {
+            f32x4 w;
+            const int ke = k_end(g0 + g);
+#pragma unroll
+            for (int k = 0; k < 4; ++k) w[k] = link_prob<SHIFT>(Quad<TL>::get(raw[g], k), valid(g0 + g, k, ke), tiny);
+            *reinterpret_cast<f32x4 *>(dst + 4 * (g0 + g) * kPatchPitch) = w;
+        }
     }
 }
 __device__ __forceinline__ void read_patch(Tile &t, const float *patch, int lane, int dir) {

@@ -53,7 +53,8 @@ struct SweepArgs {
     // domain holds, an upper bound).  With gradients {alpha/upper, beta/lower}, without {alpha/lower, alpha/upper}.
     unsigned char rev[2], upper[2];
     int only_flagged;  // exact kernel: 0 = every sample; 1 = samples whose flag is set
-    ChunkPlan plan;    // fast path, host-built: gtab[NBb][g] = first block of group g, and how its tiles are dealt to its waves (float32 sweeps)
+    ChunkPlan<2> plan; // fast path, host-built: gtab[NBb][g] = first block of group g, and how its tiles are dealt to its waves
+                       // (deal[0]: float32 sweeps, deal[1]: float64)
     double *zfast;     // [2][B] the fast kernel's own read-outs (never rewritten by the exact kernel)
 };
 
@@ -323,7 +324,7 @@ __device__ __forceinline__ void sweep_chunks_group(const SweepArgs &a, const int
     const bool producer = g < last_group, consumer = flo < jb0;
     const ChunkLds o = chunk_lds(jb0, nblk, W, WIDE);
     int ntile = 0;
-    for (int q = 0; q < nblk; ++q) ntile += tiles_of_block(jb0 + q, W);
+    for (int q = 0; q < nblk; ++q) ntile += tiles_of_block<1>(jb0 + q, W);
     if (nblk > kChunkBlocks || ntile > kTileCap - nblk || o.total * 4 > kChunkLdsBytes) {   // cannot happen with the host's partition
         if (tid == 0) { store_agent(risk, 1); store_agent(prog + g, 1 << 30); }
         return;
@@ -331,49 +332,8 @@ __device__ __forceinline__ void sweep_chunks_group(const SweepArgs &a, const int
     const bool owner = wave < nblk;               // this wave walks block jb0 + wave
     const int helpers = kTileWaves - nblk;
 
-    // ---- my tiles below the diagonal.  A run is a wave's tiles that lead to one block; runs are numbered in the order of
-    //      the tiles.  Worked out with lane <-> block (f: its first tile) and lane <-> wave (w_first: its first tile). ----
     const TileDeal deal = a.plan.deal[WIDE][NBb][g];
-    int my_first, my_count;
-    wave_tiles(deal, wave, my_first, my_count);
-    int f = 0, w_first, w_count;
-#pragma unroll
-    for (int q = 0; q < kChunkBlocks; ++q) f += q < lane && q < nblk ? tiles_of_block(jb0 + q, W) : 0;
-    wave_tiles(deal, lane & (kTileWaves - 1), w_first, w_count);
-    int f_of[kChunkBlocks + 1];
-    bool cuts = lane < kTileWaves && w_count > 0;   // this wave's first tile begins a run in the middle of a block
-#pragma unroll
-    for (int q = 0; q <= kChunkBlocks; ++q) {
-        f_of[q] = __builtin_amdgcn_readlane(f, q);
-        if (q < nblk) cuts = cuts && !(w_first == f_of[q] && tiles_of_block(jb0 + q, W) > 0);
-    }
-    const int without = jb0 < 2 ? 2 - jb0 : 0;      // (blocks 0 and 1 have no such tiles)
-    // number of runs that begin at or before tile n of block q
-    auto runs_to = [&](const int q, const int n) { return q + 1 - without + (int)__builtin_popcountll(__builtin_amdgcn_ballot_w64(cuts && w_first <= n)); };
-    int t_I[kTilesPerWave], t_q[kTilesPerWave], t_run[kTilesPerWave];   // source block, own block it leads to, run it belongs to
-    bool t_ok[kTilesPerWave], t_start[kTilesPerWave], t_end[kTilesPerWave], t_lead[kTilesPerWave];   // first / last tile of its run; run that states the scale
-#pragma unroll
-    for (int u = 0; u < kTilesPerWave; ++u) {
-        const int r0 = owner ? u - 1 : u, n = my_first + r0;   // (a walking wave has the tile next to the diagonal in slot 0)
-        t_ok[u] = r0 >= 0 && r0 < my_count;
-        int q = 0;
-#pragma unroll
-        for (int x = 1; x < kChunkBlocks; ++x) q = x < nblk && n >= f_of[x] ? x : q;
-        const int lo = tile_ilo(jb0 + q, W), r = n - f_of[q];
-        t_q[u] = t_ok[u] ? q : 0;
-        t_I[u] = t_ok[u] ? lo + r : flo;
-        t_start[u] = r0 == 0 || r == 0;
-        t_end[u] = r0 == my_count - 1 || lo + r == jb0 + q - 2;
-        t_lead[u] = r0 >= r;                      // (the run reaches back to the block's first tile)
-        t_run[u] = runs_to(q, n) - 1;
-    }
-    // the runs that lead to the block this wave walks
-    int run_first = o.runs, run_count = 1;         // (a block without such tiles: the zeros behind the products)
-    if (owner && tiles_of_block(jb0 + wave, W) > 0) {
-        const int n = __builtin_amdgcn_readlane(f, wave);
-        run_first = runs_to(wave, n) - 1;
-        run_count = runs_to(wave, n + tiles_of_block(jb0 + wave, W) - 1) - run_first;
-    }
+    const WaveTiles t = plan_wave<1>(deal, jb0, nblk, W, o.runs, wave, lane);
     // A consumer group has nothing to do for the first stages: it lets the first group of its sweep have the memory's
     // bandwidth for its tiles.  (Progress words: 1 once the group's tiles are staged, then 2 + n when the rows of the first n
     // chunks of its last block and n + 1 of the others are in memory -- and so, since it has read them, n of all blocks below.)
@@ -386,23 +346,18 @@ __device__ __forceinline__ void sweep_chunks_group(const SweepArgs &a, const int
     float *const patch = lds_raw + wave * (kBlk * kPatchPitch);
     const int last_index = L * translen - 1;
     const float tiny = !upper ? 0.f : kTinyStored;
-    const bool adjacent = owner && jb0 + wave > 0;
-    if (owner) {                                  // the triangle, and the tile next to it
-        t_I[kTilesPerWave - 1] = jb0 + wave; t_q[kTilesPerWave - 1] = wave;
-        t_I[0] = jb0 + wave - (adjacent ? 1 : 0); t_q[0] = wave;
-    }
     auto elements = [&](const int samples) { const int64_t n = (int64_t)samples * L * translen; return n < (1 << 28) ? (int)n : 1 << 28; };
     const int before = elements(b), behind = elements(a.B - 1 - b);
     auto stage = [&](const int u) __attribute__((always_inline)) {
-        stage_tile<TL, CH::kLinkShift>(patch, links, t_I[u], jb0 + t_q[u], lane, dir, Lb, translen, last_index, before, behind, tiny);
+        stage_tile<TL, CH::kLinkShift, true, 8>(patch, links, t.I[u], jb0 + t.q[u], lane, dir, Lb, translen, last_index, before, behind, tiny);
     };
     Tile t0, t1, t2;
-    auto read = [&](Tile &t, const bool triangle) __attribute__((always_inline)) {
-        if (!WIDE || triangle) read_patch(t, patch, lane, dir); else read_patch_wide(t, patch, lane, dir);
+    auto read = [&](Tile &tile, const bool triangle) __attribute__((always_inline)) {
+        if (!WIDE || triangle) read_patch(tile, patch, lane, dir); else read_patch_wide(tile, patch, lane, dir);
     };
-    if (t_ok[0] || adjacent) { stage(0); read(t0, false); }
-    if (t_ok[1]) { stage(1); read(t1, false); }
-    if (t_ok[2] || owner) { stage(2); read(t2, owner); }
+    if (t.ok[0] || t.adjacent) { stage(0); read(t0, false); }
+    if (t.ok[1]) { stage(1); read(t1, false); }
+    if (t.ok[2] || owner) { stage(2); read(t2, owner); }
     if (owner) fold_triangle(t2, lane);
     __syncthreads();   // every wave is done with its transpose patch: the LDS now holds the buffers of the stages
     if (producer && g == 0 && tid == 0) store_agent(prog, 1);
@@ -532,12 +487,12 @@ __device__ __forceinline__ void sweep_chunks_group(const SweepArgs &a, const int
     int t_shift[kTilesPerWave], t_cells[kTilesPerWave], t_kaps[kTilesPerWave], t_scale_at[kTilesPerWave], t_scales[kTilesPerWave];
 #pragma unroll
     for (int u = 0; u < kTilesPerWave; ++u) {
-        const int J = jb0 + t_q[u], at = t_q[u] - 1, lo = tile_ilo(J, W);   // chunk = stage - at
+        const int J = jb0 + t.q[u], at = t.q[u] - 1, lo = tile_ilo(J, W);   // chunk = stage - at
         t_from[u] = at + (dest_lo(J) > 0 ? dest_lo(J) : 0);
-        t_to[u] = t_ok[u] ? at + (dest_hi(J) < NC - 1 ? dest_hi(J) : NC - 1) : -100;
-        t_src_from[u] = at + src_lo(t_I[u]); t_src_to[u] = at + dest_hi(t_I[u]);
+        t_to[u] = t.ok[u] ? at + (dest_hi(J) < NC - 1 ? dest_hi(J) : NC - 1) : -100;
+        t_src_from[u] = at + src_lo(t.I[u]); t_src_to[u] = at + dest_hi(t.I[u]);
         t_shift[u] = (((-at) % D) + D) % D;
-        t_cells[u] = (t_I[u] - flo) * D * 256; t_kaps[u] = o.kap + (t_I[u] - flo) * D * 4;
+        t_cells[u] = (t.I[u] - flo) * D * 256; t_kaps[u] = o.kap + (t.I[u] - flo) * D * 4;
         t_scale_at[u] = o.kap + (lo - flo) * D * 4; t_scales[u] = J - 1 - lo;
     }
     if (NC == 0) return;
@@ -657,6 +612,20 @@ __device__ __forceinline__ void sweep_chunks_group(const SweepArgs &a, const int
             const bool bring = FETCHES && f_blk[0] >= 0 && tau + 1 < NC;
             int published = 0;
             if (bring) published = load_agent(below);
+            // The last two blocks' rows of the last stage are in memory when both their waves have come here, the other
+            // blocks' of the stage before that (their waves have since waited for match rows requested behind them): the
+            // second of the two publishes.  (In front of the walk, although it waits there: half way through it, where the rows are
+            // there without a wait, B = 16, L = 1024, T = 64 takes 166 us instead of 158.)
+            auto publish = [&]() __attribute__((always_inline)) {
+                const int n = tau - (nblk - 1);                // chunks of the last block
+                if (!producer || wave < nblk - 2 || n < 0 || n >= NC) return;
+                wait_vmem_all();
+                int both = 1;
+                if (nblk > 1) {
+                    if (lane == 0) both = __hip_atomic_fetch_add(published_by, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) & 1;
+                }
+                if (lane == 0 && both) store_agent(prog + g, 2 + n);
+            };
             // ---------------- walk my block through chunk tau - wave ----------------
             if (WALKS) {
                 const int c = tau - wave;
@@ -681,20 +650,7 @@ __device__ __forceinline__ void sweep_chunks_group(const SweepArgs &a, const int
                         for (int k = 0; k < kChunk; ++k) Ga[k] = out[k];
                     }
                 }
-                // The last two blocks' rows of the last stage are in memory when both their waves have come here, the other
-                // blocks' of the stage before that (their waves have since waited for match rows requested behind them):
-                // the second of the two publishes.
-                if (producer && wave >= nblk - 2) {
-                    const int n = tau - (nblk - 1);                // chunks of the last block
-                    if (n >= 0 && n < NC) {
-                        wait_vmem_all();
-                        int both = 1;
-                        if (nblk > 1) {
-                            if (lane == 0) both = __hip_atomic_fetch_add(published_by, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) & 1;
-                        }
-                        if (lane == 0 && both) store_agent(prog + g, 2 + n);
-                    }
-                }
+                publish();
                 if (more) load_match(c + 1, lane);
                 if (c >= 0 && c < NC) {
                     Cell *const cells = eb + own_src * D * 256 + cell_place<WIDE>(lane);
@@ -715,24 +671,24 @@ __device__ __forceinline__ void sweep_chunks_group(const SweepArgs &a, const int
                         int A[kChunk], R[kChunk];
 #pragma unroll
                         for (int k = 0; k < kChunk; ++k) { A[k] = __builtin_amdgcn_readlane(av, k); R[k] = __builtin_amdgcn_readlane(rv, k); }
-                        const Cell *const parts = part + (run_first * 2 + (par ^ 1)) * 256 + lane * (WIDE ? 1 : 4);
+                        const Cell *const parts = part + (t.run_first * 2 + (par ^ 1)) * 256 + lane * (WIDE ? 1 : 4);
                         const float upper_half = lane >= 32 ? 1.f : 0.f;
                         Cell G[kChunk];
                         if constexpr (WIDE) {
 #pragma unroll
                             for (int k = 0; k < kChunk; ++k) G[k] = parts[k * kBlk];
 #pragma unroll 1
-                            for (int u = 1; u < run_count; ++u)
+                            for (int u = 1; u < t.run_count; ++u)
 #pragma unroll
                                 for (int k = 0; k < kChunk; ++k) G[k] += parts[u * 512 + k * kBlk];
                         } else {
                             f32x4 sum = *reinterpret_cast<const f32x4 *>(parts);
-                            if (run_count > 1) {
+                            if (t.run_count > 1) {
                                 f32x4 sum1 = *reinterpret_cast<const f32x4 *>(parts + 512);
-                                if (run_count > 2) {
+                                if (t.run_count > 2) {
                                     sum += *reinterpret_cast<const f32x4 *>(parts + 1024);
 #pragma unroll 1
-                                    for (int u = 3; u < run_count; ++u) sum += *reinterpret_cast<const f32x4 *>(parts + u * 512);
+                                    for (int u = 3; u < t.run_count; ++u) sum += *reinterpret_cast<const f32x4 *>(parts + u * 512);
                                 }
                                 sum += sum1;
                             }
@@ -788,7 +744,7 @@ __device__ __forceinline__ void sweep_chunks_group(const SweepArgs &a, const int
                 else if (c == NC) wait_vmem_all();
             }
             // ---------------- multiply out what my tiles' blocks (q of the group) receive in chunk tau + 1 - q ----------------
-            if (my_count > 0) {
+            if (t.count > 0) {
                 // (float32: the LDS reads of two tiles are requested before the first is waited for, the third's behind the first)
                 f32x4 ev[2];
                 int kv[kTilesPerWave], rv[kTilesPerWave], at[kTilesPerWave];
@@ -804,7 +760,7 @@ __device__ __forceinline__ void sweep_chunks_group(const SweepArgs &a, const int
                         at[u] = t_cells[u] + sl * 256;
                         if (!WIDE && u < 2) ev[u] = cells_of(u);
                         kv[u] = lds_i[t_kaps[u] + sl * 4 + step];
-                        if (t_start[u]) {
+                        if (t.start[u]) {
                             const int n = other < t_scales[u] ? other : 0;
                             rv[u] = lds_i[t_scale_at[u] + sl * 4 + n * (D * 4) + step];
                         }
@@ -812,9 +768,9 @@ __device__ __forceinline__ void sweep_chunks_group(const SweepArgs &a, const int
                 }
                 Cell G[4] = {0, 0, 0, 0};
                 int R = kDeadExp;
-                auto product = [&](const int u, const Tile &t) __attribute__((always_inline)) {
+                auto product = [&](const int u, const Tile &tile) __attribute__((always_inline)) {
                     if (!go[u]) return;
-                    if (t_start[u]) {   // the scale: the largest exponent, step by step, among all blocks that lead here
+                    if (t.start[u]) {   // the scale: the largest exponent, step by step, among all blocks that lead here
                         if constexpr (WIDE) R = row16_max_int(rv[u]); else R = by_step_max(rv[u]);
 #pragma unroll
                         for (int k = 0; k < 4; ++k) G[k] = 0;
@@ -822,27 +778,27 @@ __device__ __forceinline__ void sweep_chunks_group(const SweepArgs &a, const int
                     if (src[u]) {
                         if constexpr (WIDE) {
                             double v[4];
-                            tile_product(t, eb + at[u], lane, v);
+                            tile_product(tile, eb + at[u], lane, v);
                             const double f = pow2_clamped_wide(kv[u] - R, floor_exp);
 #pragma unroll
                             for (int k = 0; k < 4; ++k) G[k] = __builtin_fma(v[k], f, G[k]);
                         } else {
-                            const f32x4 v = tile_product(t, ev[u & 1]);
+                            const f32x4 v = tile_product(tile, ev[u & 1]);
                             f32x4 sum = {G[0], G[1], G[2], G[3]};
                             scaled4<false>(sum, pow2_clamped(kv[u] - R, floor_exp), v);
 #pragma unroll
                             for (int k = 0; k < 4; ++k) G[k] = sum[k];
                         }
                     }
-                    if (t_end[u]) {
-                        Cell *const to = part + (t_run[u] * 2 + par) * 256;
+                    if (t.end[u]) {
+                        Cell *const to = part + (t.run[u] * 2 + par) * 256;
                         if constexpr (WIDE) {
 #pragma unroll
                             for (int k = 0; k < 4; ++k) to[(lane >> 4) * kBlk + 16 * k + (lane & 15)] = G[k];
-                            if (t_lead[u] && (lane & 15) == 0) lds_i[o.part_scale + (t_q[u] * 2 + par) * 4 + step] = R;
+                            if (t.lead[u] && (lane & 15) == 0) lds_i[o.part_scale + (t.q[u] * 2 + par) * 4 + step] = R;
                         } else {
                             *reinterpret_cast<f32x4 *>(to + lane * 4) = f32x4{G[0], G[1], G[2], G[3]};
-                            if (t_lead[u] && lane < 4) lds_i[o.part_scale + (t_q[u] * 2 + par) * 4 + lane] = R;
+                            if (t.lead[u] && lane < 4) lds_i[o.part_scale + (t.q[u] * 2 + par) * 4 + lane] = R;
                         }
                     }
                 };
@@ -855,15 +811,15 @@ __device__ __forceinline__ void sweep_chunks_group(const SweepArgs &a, const int
             if (bring) {
                 published = __builtin_amdgcn_readfirstlane(published);
                 if (published > seen) seen = published;
-                auto chunk_of = [&](const int u, const int t) { return t + (f_blk[u] == jb0 - 1 ? 1 : 2); };
-                auto request = [&](const int t) __attribute__((always_inline)) {   // what stage t brings in
+                auto chunk_of = [&](const int u, const int stage) { return stage + (f_blk[u] == jb0 - 1 ? 1 : 2); };
+                auto request = [&](const int stage) __attribute__((always_inline)) {   // what a stage brings in
 #pragma unroll
                     for (int u = 0; u < kForeign; ++u) {
                         if (f_blk[u] < 0) break;
-                        const int c = chunk_of(u, t);
+                        const int c = chunk_of(u, stage);
                         if (c >= 0 && c < NC) request_rows(f_blk[u], c, lane);
                     }
-                    requested = t;
+                    requested = stage;
                 };
                 if (requested < tau) {
                     int spins = 0;
@@ -1651,16 +1607,8 @@ static int launch_sweeps(SweepArgs a, hipStream_t st) {
         a.rev[0] = 0; a.rev[1] = a.loss_dir ? 1 : 0;
         a.upper[0] = a.loss_dir ? 1 : 0; a.upper[1] = a.loss_dir ? 0 : 1;
         a.C = C;
-        {   // how the blocks of a sample are grouped and their tiles dealt, by its number of blocks; remembered for the next call
-            struct Grouping { int W = 0, C = 0, NB = 0; ChunkPlan plan; };
-            static thread_local Grouping last;
-            const int W = (a.translen + kBlk - 1) / kBlk;
-            if (last.W != W || last.C != C || last.NB < a.NBK) {
-                plan_chunks(a.NBK, W, C, last.plan);
-                last.W = W; last.C = C; last.NB = a.NBK;
-            }
-            a.plan = last.plan;
-        }
+        static const ChunkCosts kCosts[2] = {{45, 7, 4, 100}, {85, 17, 11, 100}};   // (measured)
+        a.plan = chunk_plan<1>(a.translen, C, kCosts);
         const int B8 = (a.B + 7) & ~7;
         if ((rc = prepare_tiles_kernel<TM, TL, false>()) || (rc = prepare_tiles_kernel<TM, TL, true>())) return rc;
         if (!float64_first()) {

@@ -1,9 +1,11 @@
-"""The chunked sweeps of dag_loss, in float32 and float64, at the sizes where they can go wrong: graphs one node short of, at and one
+"""The chunked sweeps of dag_loss, in float32 and float64, and of dag_best_alignment at the sizes where they can go
+wrong: graphs one node short of, at and one
 past a block of 64 and a group's last block, targets one step around a chunk of four, transition windows around a block,
 transitions that start at an odd element of their tensor or are its very first and last ones, one sample alone."""
 import pytest
 import torch
 
+import da_transformer_amd as dagx
 from da_transformer_amd import _native as nat
 from da_transformer_amd.custom_ops.dag_loss import DagLossFunc
 from oracle import torch_native as tn
@@ -47,3 +49,29 @@ def test_edges_of_blocks_chunks_and_windows(B, L, T, translen, dtype, wide):
     assert ((loss.double() - rloss)[fin].abs() <= 6e-7 * T + 2e-7 * rloss[fin].abs()).all(), (loss, rloss)
     assert_close(gm.float(), rgm, RTOL[dtype], "grad_match")
     assert_close(gl.float(), rgl, RTOL[dtype], "grad_links")
+
+
+@pytest.mark.parametrize("B,L,T,translen,dtype", [
+    (1, 2, 2, 1, F32), (3, 2, 2, 1, F16), (2, 5, 5, 1, F32), (1, 63, 5, None, F16), (2, 64, 2, None, F32), (1, 65, 6, 63, BF16),
+    (3, 65, 9, 64, F32), (2, 129, 17, 2, F16), (1, 257, 8, None, F32), (2, 320, 9, 128, F16), (1, 321, 33, 63, F32),
+    (2, 449, 30, 32, BF16), (1, 511, 14, None, F32), (2, 513, 7, 257, F16), (1, 705, 12, 130, F32), (2, 1024, 11, None, F16),
+    (1, 1023, 64, 200, F32),
+    # T at and under L / 8: in chunks and step by step
+    (2, 128, 16, None, F32), (2, 129, 16, None, F32), (2, 448, 56, None, F16), (2, 449, 56, 100, F32),
+    # few workgroups a sample: groups of several blocks (of eight in the last), one and two stages a block
+    (65, 250, 33, None, F32), (65, 512, 66, None, F16), (129, 1022, 130, 64, F16)])
+def test_alignment_at_edges_of_blocks_chunks_and_windows(B, L, T, translen, dtype):
+    match, links_sq, ol, tl = random_problem(L + T, B + 1, L, T, dtype=F32, ragged=False, translen=translen)
+    if translen is not None:      # a path of T_b nodes spans at most (T_b - 1) translen transitions
+        ol = torch.minimum(ol, (tl - 1) * translen + 1).clamp_(min=1)
+    if B > 1:
+        tl[1] = max(1, T - 1)
+        ol[1] = max(int(tl[1]), int(ol[1]) - 3) if translen is None else int(tl[1])
+    match, links = match.to(dtype), tn.extract_valid_links(links_sq, translen).to(dtype)
+    ol, tl = ol[:B], tl[:B]
+    # coarse scores: many ties, which the lowest predecessor has to win
+    match, links = (match * 4).round() / 4, (links * 4).round() / 4
+    got = dagx.dag_best_alignment(match.to(DEV)[1:], links.to(DEV)[1:], ol.to(DEV), tl.to(DEV)).cpu()
+    some = sorted({0, min(1, B - 1), B // 2, B - 1})
+    want = tn.torch_dag_best_alignment(match[1:][some].float(), tn.restore_valid_links(links[1:][some].float()), ol[some], tl[some])
+    assert torch.equal(got[some], want)
