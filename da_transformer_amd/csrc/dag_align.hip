@@ -218,11 +218,11 @@ __device__ __host__ inline int partition_blocks(int NBb, int W, int C, int *gsta
 }
 
 // Whether the sweep goes in chunks of four steps.  They cost T / 4 stages and one or two more for every block of nodes, single
-// steps T of a quarter of that: chunks win by 8 to 18 % at T = L / 8 and more on long graphs, tie there on short ones, and
-// lose by 5 to 20 % at T = L / 9 and less (alignment, chunks and steps: B = 64, L = 512, T = 64 129 and 140 us; B = 20, L = 1000,
-// T = 128 297 and 328; B = 48, L = 350, T = 40 81 and 76; B = 1, L = 140, T = 16 35 and 31).
+// steps T of two fifths of that: even at about six steps for every block of nodes and eight more (alignment, chunks and
+// steps: B = 64, L = 512, T = 64 129 and 140 us; B = 28, L = 450, T = 50 108 and 103; B = 20, L = 1000, T = 128 297 and 328; B = 1,
+// L = 900, T = 70 196 and 179; B = 48, L = 350, T = 40 81 and 76; B = 8, L = 128, T = 32 38 and 44; B = 1, L = 115, T = 15 29 and 27).
 static bool align_in_chunks(int B, int T, int L, int translen) {
-    return 8 * (int64_t)T >= L && (int64_t)B * L * translen >= 4;   // (the chunked kernel's tiles are loaded four elements at a time)
+    return T >= 6 * ((L + kBlk - 1) / kBlk) + 8 && (int64_t)B * L * translen >= 4;   // (the chunked kernel's tiles are loaded four elements at a time)
 }
 
 // Workgroups per sweep.  In chunks: from four position blocks on as many as the device has room for (one per CU) up to one

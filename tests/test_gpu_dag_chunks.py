@@ -56,8 +56,9 @@ def test_edges_of_blocks_chunks_and_windows(B, L, T, translen, dtype, wide):
     (3, 65, 9, 64, F32), (2, 129, 17, 2, F16), (1, 257, 8, None, F32), (2, 320, 9, 128, F16), (1, 321, 33, 63, F32),
     (2, 449, 30, 32, BF16), (1, 511, 14, None, F32), (2, 513, 7, 257, F16), (1, 705, 12, 130, F32), (2, 1024, 11, None, F16),
     (1, 1023, 64, 200, F32),
-    # T at and under L / 8: in chunks and step by step
-    (2, 128, 16, None, F32), (2, 129, 16, None, F32), (2, 448, 56, None, F16), (2, 449, 56, 100, F32),
+    # in chunks where T is at least 6 ceil(L / 64) + 8, else step by step
+    (1, 64, 13, None, F32), (2, 128, 20, None, F32), (2, 129, 25, None, F32), (1, 129, 26, None, F16),
+    (2, 448, 50, None, F16), (2, 449, 56, 100, F32), (1, 513, 62, 257, F16), (1, 705, 80, 130, F32), (2, 1024, 104, None, F16),
     # few workgroups a sample: groups of several blocks (of eight in the last), one and two stages a block
     (65, 250, 33, None, F32), (65, 512, 66, None, F16), (129, 1022, 130, 64, F16)])
 def test_alignment_at_edges_of_blocks_chunks_and_windows(B, L, T, translen, dtype):
