@@ -1549,11 +1549,13 @@ static int sweep_groups(int B, int L, int translen) {
     return (long long)sweeps * C <= 256 && C > 0 ? C : groups_needed(L, translen, kChunkBlocks);
 }
 
+// ticket + progress words (rounded to 8 bytes), then the fast kernel's two read-outs per sample
+static size_t sweep_bytes(int B, int C) { return sweep_sync_ints(B, C) * sizeof(int) + (size_t)2 * B * sizeof(double); }
+
 size_t loss_fwd_workspace_bytes(int B, int T, int L, int translen) {
     (void)T;
-    int C = sweep_groups(B, L, translen);
-    // ticket + progress words (rounded to 8 bytes), then the fast kernel's two read-outs per sample
-    return C > 0 ? sweep_sync_ints(B, C) * sizeof(int) + (size_t)2 * B * sizeof(double) : 0;
+    const int C = sweep_groups(B, L, translen);
+    return C > 0 ? sweep_bytes(B, C) : 0;
 }
 
 size_t loss_bwd_workspace_bytes(int B) { (void)B; return 0; }
@@ -1756,7 +1758,10 @@ extern "C" int dagx_loss_fwd(const void *match, int match_dtype, const int64_t m
 // device array owned by the library: every GPU the library runs on holds its own copy until the process
 // ends.  Zero when the code object is loaded; the sweep kernel leaves every word it used zero again.
 constexpr size_t kScratchBytes = 128 * 1024;
-static __device__ __align__(256) unsigned char scratch[kScratchBytes];
+// (What fits is decided as for groups of any number of blocks; groups of at most eight can be one more, 40 bytes a sample
+//  instead of 32.)
+constexpr size_t kScratchHeld = kScratchBytes / 4 * 5 + 256;
+static __device__ __align__(256) unsigned char scratch[kScratchHeld];
 
 constexpr int kMaxDevices = 64;
 static std::atomic<void *> g_scratch_ptr[kMaxDevices];
@@ -1812,9 +1817,11 @@ extern "C" int dagx_loss_fwd_noalloc(const void *match, int match_dtype, const i
                                      void *stream) {
     if (B < 0 || T < 1 || L < 1 || translen < 1) { set_error("dag_loss_fwd_noalloc: bad sizes B=%d T=%d L=%d translen=%d", B, T, L, translen); return DAGX_ERR_ARGUMENT; }
     const size_t need = loss_fwd_workspace_bytes(B, T, L, translen);
-    if (need > kScratchBytes) {
+    const int C = groups_needed(L, translen, kMaxBlocksFast);
+    const size_t asked = C > 0 ? sweep_bytes(B, C) : 0;
+    if (asked > kScratchBytes || need > kScratchHeld) {
         set_error("dag_loss_fwd_noalloc: B=%d, L=%d needs %zu bytes of pipeline words, the built-in scratch holds %zu "
-                  "(use dagx_loss_fwd with a caller workspace)", B, L, need, kScratchBytes);
+                  "(use dagx_loss_fwd with a caller workspace)", B, L, asked, kScratchBytes);
         return DAGX_ERR_UNSUPPORTED;
     }
     void *ptr = nullptr;
@@ -1824,7 +1831,7 @@ extern "C" int dagx_loss_fwd_noalloc(const void *match, int match_dtype, const i
     }
     return loss_fwd_impl(match, match_dtype, match_strides, links, links_dtype, out_len, tgt_len, B, T, L, translen,
                          alpha_hat, beta_hat, alpha_off, beta_off, logz, loss, sample_flags, require_gradient,
-                         ptr, need > 0 ? kScratchBytes : 0, stream);
+                         ptr, need > 0 ? kScratchHeld : 0, stream);
 }
 
 extern "C" int dagx_loss_bwd(const float *grad_out, int64_t grad_out_stride,

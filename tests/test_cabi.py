@@ -159,3 +159,15 @@ def test_header_is_valid_c_and_cpp_and_a_c_program_links_against_the_library(tmp
                     "-Wl,-rpath," + libdir], check=True)
     out = subprocess.run([str(exe)], check=True, capture_output=True, text=True).stdout
     assert "gfx950" in out and f"{len(names)} entry points" in out
+
+
+@pytest.mark.parametrize("B,accepted", [(3276, True), (4090, True), (4098, False)])
+def test_what_the_built_in_scratch_takes_does_not_depend_on_the_grouping(B, accepted):
+    """Twelve blocks of nodes with short transitions fit one workgroup's tiles but are swept by two: 40 bytes of pipeline
+    words a sample, and still as many samples as 32 bytes each allow.  (Null pointers: nothing is launched.)"""
+    lib = _native.lib()
+    s3 = (ctypes.c_int64 * 3)(14 * 768, 768, 1)
+    rc = lib.dagx_loss_fwd_noalloc(None, 0, s3, None, 0, None, None, B, 14, 768, 64, None, None, None, None, None, None, None, 1, None)
+    assert (rc == 2) == (not accepted), lib.dagx_last_error()
+    if not accepted:
+        assert b"scratch" in lib.dagx_last_error()
