@@ -717,7 +717,14 @@ __device__ __forceinline__ void sweep_chunks_group(const SweepArgs &a, const int
                                 e = __builtin_fmaf(y, __builtin_bit_cast(float, (unsigned)(253 + kShift2 - tb) << 23), tiny_up);
                             } else {   // at most 2^57, and mostly 15 to 45 binades lower
                                 kap = ref + N[k] - kShift2;
-                                e = __builtin_fmaf(x, mt[k], tiny_up);
+                                const float y = x * mt[k];
+                                if (__builtin_expect(__builtin_amdgcn_ballot_w64(y >= kScaleBelow) != 0, 1)) e = y + tiny_up;
+                                else {   // (so far below that it would cost the cells under it their range)
+                                    const unsigned top = wave64_max_positive(y);
+                                    const int tb = (int)(top >> 23) > 55 ? (int)(top >> 23) : 55;
+                                    kap = top ? kap + tb - (126 + kShift2) : kDeadExp;
+                                    e = __builtin_fmaf(y, __builtin_bit_cast(float, (unsigned)(253 + kShift2 - tb) << 23), tiny_up);
+                                }
                             }
                             kk[k] = kap;
                             v[k] = e;
