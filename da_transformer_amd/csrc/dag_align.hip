@@ -293,8 +293,8 @@ __device__ __host__ inline AlignLds align_lds(int jb0, int nblk, int W, int spac
 // blocks with the best predecessor the lowest one counts (runs in the order of the blocks, then the block itself; a later
 // one replaces an earlier one only if it is larger).
 //
-// Step by step, with two barriers, LDS round trips and a hand-over in each, a step cost 1.8 us at L = 512 and 3.2 us at
-// L = 1024, of which the tiles' 96 instructions a step are a quarter.  What bounds the stages now is those instructions:
+// Step by step, with two barriers, LDS round trips and a hand-over in each, a step costs 1.6 us at L = 512 and 1.8 us at
+// L = 1024, of which the tiles' 96 instructions a step are a third.  What bounds the stages now is those instructions:
 // four steps of a tile take 2 700 cycles, 2 000 of a SIMD that two waves share, the walk of a block 3 500.
 //
 // SPACING (dag_chunks.h): a tile is nearly as much work as the walk here, so that where the walk bounds the stages and SIMDs

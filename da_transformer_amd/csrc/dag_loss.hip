@@ -255,9 +255,9 @@ __global__ __launch_bounds__(NT) void dag_sweep_exact_kernel(SweepArgs a) {
 // a step, 5.5 cycles each), the product of the tile next to the diagonal in front of it, and one stage per block of the
 // graph.  (With that product a stage ahead, too, the stages are 600 cycles shorter but two per block: forward at B = 64,
 // L = 512, T = 64 115 us instead of 107, L = 256 70 instead of 66, L = 128 52 instead of 56.)
-//   step by step -> chunks, forward: B = 64, L = 512, T = 64 134 -> 107 us; L = 64 (T = 64) 81 -> 47; L = 256 99 -> 66;
-//   B = 16, L = 1024, T = 256 572 -> 347; B = 64, L = 512, transitions of at most 32: 136 -> 78.
-//   In float64: B = 16, L = 1024, T = 256 833 -> 535 us; B = 64, L = 512, T = 64 216 -> 160.
+//   step by step -> chunks, forward: B = 64, L = 512, T = 64 134 -> 106 us; L = 64 (T = 64) 81 -> 47; L = 256 99 -> 65;
+//   B = 16, L = 1024, T = 256 572 -> 341; B = 64, L = 512, transitions of at most 32: 136 -> 77.
+//   In float64: B = 16, L = 1024, T = 256 833 -> 512 us; B = 64, L = 512, T = 64 216 -> 150.
 // What bounds it: a SIMD gives its cycles either to matrix instructions or to vector instructions, never to both
 // (measured: a wave of DPP FMAs beside one of v_mfma_f32_4x4x1 advances only when that has ended, whatever their
 // priorities), so that products, walks and the rest of a stage add up.
