@@ -299,23 +299,22 @@ __device__ __forceinline__ unsigned wave64_max_positive(float x) {
         : "+v"(v));
     return (unsigned)__builtin_amdgcn_readlane((int)v, 63);
 }
-// the same of the upper halves of 64 float64 numbers >= 0 (a NaN counts as the largest)
-__device__ __forceinline__ unsigned wave64_max_upper(double x) {
-    unsigned v = (unsigned)(__builtin_bit_cast(unsigned long long, x) >> 32);
+// the largest of 64 integers, wave-uniform
+__device__ __forceinline__ int wave64_max_int(int v) {
     asm("s_nop 1\n\t"
-        "v_max_u32_dpp %0, %0, %0 quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"
+        "v_max_i32_dpp %0, %0, %0 quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"
         "s_nop 1\n\t"
-        "v_max_u32_dpp %0, %0, %0 quad_perm:[2,3,0,1] row_mask:0xf bank_mask:0xf\n\t"
+        "v_max_i32_dpp %0, %0, %0 quad_perm:[2,3,0,1] row_mask:0xf bank_mask:0xf\n\t"
         "s_nop 1\n\t"
-        "v_max_u32_dpp %0, %0, %0 row_half_mirror row_mask:0xf bank_mask:0xf\n\t"
+        "v_max_i32_dpp %0, %0, %0 row_half_mirror row_mask:0xf bank_mask:0xf\n\t"
         "s_nop 1\n\t"
-        "v_max_u32_dpp %0, %0, %0 row_mirror row_mask:0xf bank_mask:0xf\n\t"
+        "v_max_i32_dpp %0, %0, %0 row_mirror row_mask:0xf bank_mask:0xf\n\t"
         "s_nop 1\n\t"
-        "v_max_u32_dpp %0, %0, %0 row_bcast:15 row_mask:0xa bank_mask:0xf\n\t"
+        "v_max_i32_dpp %0, %0, %0 row_bcast:15 row_mask:0xa bank_mask:0xf\n\t"
         "s_nop 1\n\t"
-        "v_max_u32_dpp %0, %0, %0 row_bcast:31 row_mask:0xc bank_mask:0xf"
+        "v_max_i32_dpp %0, %0, %0 row_bcast:31 row_mask:0xc bank_mask:0xf"
         : "+v"(v));
-    return (unsigned)__builtin_amdgcn_readlane((int)v, 63);
+    return __builtin_amdgcn_readlane(v, 63);
 }
 // four maxima over the 64 lanes, each in lane 63 (side by side: no wait states between dependent steps)
 __device__ __forceinline__ void wave64_max4(float (&v)[4]) {

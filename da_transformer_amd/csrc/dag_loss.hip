@@ -701,29 +701,31 @@ __device__ __forceinline__ void sweep_chunks_group(const SweepArgs &a, const int
                             const int most = A[k] > R[k] ? A[k] : R[k], ref = (kap > most ? kap : most) + (WIDE || (k & 1) ? 0 : kSpare);
                             // (what ldexp flushes of either part is under flush_up, too)
                             const Cell x = (pow2(triangle_dot(t2, e, upper_half), kap - ref) + flush_up) + (pow2(G[k], R[k] - ref) + pow2(Ga[k], A[k] - ref));
-                            // (upper sweep: a cell never flushes, live or not -- what a dead one gets is of the size of what is flushed)
+                            // (upper sweep: a cell never flushes, live or not -- what a dead one gets is of the size of what is flushed.
+                            //  So the scale must not be applied to the finished product x exp(match), which may have flushed: it is
+                            //  split between the factors, or, in float64, joined with the match exponent.)
                             if constexpr (WIDE) {
-                                const double y = pow2(x * (double)mt[k], mt_exp[k]);
-                                const unsigned top = wave64_max_upper(y);
-                                const int tb = (int)(top >> 20) > 1 ? (int)(top >> 20) : 1;
-                                kap = top ? tb + ref + N[k] - (1022 + CH::kShift + CH::kLinkShift) : kDeadExp;
-                                e = pow2(y, 1022 + CH::kShift - tb) + tiny_up;
-                            } else if (k & 1) {
+                                const double y = x * (double)mt[k];
+                                // exponent of y 2^mt_exp; a cell of 0 has the least (exp(match) is 0) or no weight (lower sweep)
+                                const int tb = wave64_max_int((int)((unsigned)(__builtin_bit_cast(unsigned long long, y) >> 52)) + mt_exp[k]);
+                                kap = __builtin_amdgcn_ballot_w64(y != 0.0) != 0 ? tb + ref + N[k] - (1022 + CH::kShift + CH::kLinkShift) : kDeadExp;
+                                e = pow2(y, mt_exp[k] + (1022 + CH::kShift) - tb) + tiny_up;
+                            } else {
                                 const float y = x * mt[k];
-                                // the exponent of the largest cell, at least that of 2^-72: its reciprocal has to be a float32 number
-                                const unsigned top = wave64_max_positive(y);
-                                const int tb = (int)(top >> 23) > 55 ? (int)(top >> 23) : 55;
-                                kap = top ? tb + ref + N[k] - (126 + 2 * kShift2) : kDeadExp;
-                                e = __builtin_fmaf(y, __builtin_bit_cast(float, (unsigned)(253 + kShift2 - tb) << 23), tiny_up);
-                            } else {   // at most 2^57, and mostly 15 to 45 binades lower
-                                kap = ref + N[k] - kShift2;
-                                const float y = x * mt[k];
-                                if (__builtin_expect(__builtin_amdgcn_ballot_w64(y >= kScaleBelow) != 0, 1)) e = y + tiny_up;
-                                else {   // (so far below that it would cost the cells under it their range)
+                                auto scaled = [&](const int base) __attribute__((always_inline)) {
+                                    // the exponent of the largest cell, at least that of 2^-72: its reciprocal has to be a float32 number
                                     const unsigned top = wave64_max_positive(y);
-                                    const int tb = (int)(top >> 23) > 55 ? (int)(top >> 23) : 55;
-                                    kap = top ? kap + tb - (126 + kShift2) : kDeadExp;
-                                    e = __builtin_fmaf(y, __builtin_bit_cast(float, (unsigned)(253 + kShift2 - tb) << 23), tiny_up);
+                                    const int tb = (int)(top >> 23) > 55 ? (int)(top >> 23) : 55, up = 253 + kShift2 - tb;
+                                    kap = top ? base + tb : kDeadExp;
+                                    // (a factor below 1 goes to x, one above 1 to exp(match), which is 0 or at least 2^-126)
+                                    e = __builtin_fmaf(x * __builtin_bit_cast(float, (unsigned)(up < 127 ? up : 127) << 23),
+                                                       mt[k] * __builtin_bit_cast(float, (unsigned)(up > 127 ? up : 127) << 23), tiny_up);
+                                };
+                                if (k & 1) scaled(ref + N[k] - (126 + 2 * kShift2));
+                                else {   // at most 2^60, and mostly 15 to 45 binades lower
+                                    kap = ref + N[k] - kShift2;
+                                    if (__builtin_expect(__builtin_amdgcn_ballot_w64(y >= kScaleBelow) != 0, 1)) e = y + tiny_up;
+                                    else scaled(kap - (126 + kShift2));   // (so far below that it would cost the cells under it their range)
                                 }
                             }
                             kk[k] = kap;

@@ -206,3 +206,66 @@ def test_float64_sweeps_first_gives_the_same_results(with_grad):
     loss, gm, gl, flags = run()
     assert flags == [0] + [ROUTE[case.__name__] for case in CASES] + [0] * (B - 1 - len(CASES)), flags
     assert_close(loss, rloss, 1e-4, "loss (switched off again)")
+
+
+U = math.log(2.0)
+# Graphs of one block in which a step's cells are scaled up by more than a factor below them had room for: the cell that
+# carries the mass is lost by the product with exp(match) unless that product and the scale are taken together.  Values in
+# units of ln 2; the reference value of log Z (same units) after the name.
+SCALED_UP = {
+    # the first step is scaled up by 2^70 and the cell that matters lies 52 binades under the largest
+    "odd_and_even_step": (-203.0, 6, 4, {(0, 0): 0, (1, 1): 0, (1, 2): -102, (2, 3): -50, (2, 4): 0, (3, 5): 0},
+                          {(0, 1): -70, (0, 2): -100, (1, 3): -100, (2, 4): -1, (3, 5): 0, (4, 5): 0}),
+    # both directions lose the same cell: a loss 28 nats off, with gradients and without
+    "both_directions_short": (-280.0, 9, 3, {(0, 0): 0, (1, 2): -200, (1, 7): -70, (2, 8): 0},
+                              {(0, 2): -80, (0, 7): -120, (2, 8): 0, (7, 8): -130}),
+    "both_directions": (-220.0, 6, 5, {(0, 0): 0, (1, 1): 0, (2, 2): 0, (3, 3): 0, (3, 4): -140, (4, 5): 0},
+                        {(0, 1): 0, (1, 2): 0, (2, 3): -120, (2, 4): -80, (3, 5): -160, (4, 5): 0}),
+    # the same in the float64 sweeps
+    "float64": (-2080.0, 9, 5, {(0, 0): 0, (1, 2): -2030, (1, 3): 0, (1, 4): -1270, (2, 4): 0, (2, 6): -1320, (3, 7): 0, (4, 8): 0},
+                {(0, 2): -50, (0, 4): 0, (2, 4): 0, (4, 6): 0, (4, 7): 0, (6, 7): 0, (7, 8): 0}),
+}
+
+
+@pytest.mark.parametrize("with_grad", [False, True])
+@pytest.mark.parametrize("name", SCALED_UP)
+def test_a_cell_lost_before_its_step_is_scaled_up_is_never_lost_silently(name, with_grad):
+    z, L, T, cells, edges = SCALED_UP[name]
+    match, links, ol, tl = sparse_case(L, T, {k: v * U for k, v in cells.items()}, {k: v * U for k, v in edges.items()})
+    rloss, rgm, rgl = oracle_loss_and_grads(match, links, ol, tl)
+    assert abs(rloss.item() - z * U) < 1e-3 * abs(z)      # the case is what its description says
+    if with_grad:
+        loss, gm, gl = hip_loss_and_grads(match, links, ol, tl)
+        assert_close(gm, rgm, 1e-4, "grad_match")
+        assert_close(gl, rgl, 1e-4, "grad_links")
+    else:
+        with torch.no_grad():
+            loss = dagx.dag_loss(match.to(DEV), links.to(DEV), ol.to(DEV), tl.to(DEV)).cpu()
+    assert_close(loss, rloss, 1e-4, "loss")
+
+
+@pytest.mark.parametrize("with_grad", [False, True])
+@pytest.mark.parametrize("scale", [100.0, 200.0, 1500.0])
+def test_random_sparse_peaked_graphs(scale, with_grad):
+    """Two thousand small graphs with scores spread over the whole range of the sweeps' numbers and beyond: whichever
+    kernel's result stands, it is the oracle's.  (Cells lost in front of a scale made one in five hundred wrong.)"""
+    B, L, T = 2000, 12, 7
+    gen = torch.Generator().manual_seed(int(scale))
+    spread = lambda *shape: -torch.where(torch.rand(shape, generator=gen) < 0.4, 0.0, torch.rand(shape, generator=gen))
+    match = torch.where(torch.rand(B, T, L, generator=gen) < 0.7, spread(B, T, L) * scale, NEG_INF)
+    sq = torch.where(torch.rand(B, L, L, generator=gen) < 0.7, spread(B, L, L) * min(scale, 170.0), NEG_INF)
+    sq = sq.masked_fill(torch.arange(L).view(1, L) <= torch.arange(L).view(L, 1), NEG_INF)
+    tl = torch.randint(3, T + 1, (B,), generator=gen)
+    ol = torch.minimum(tl + torch.randint(0, 7, (B,), generator=gen), torch.tensor(L))
+    rows = torch.arange(B)
+    match[rows, 0, 0] = 0.0
+    match[rows, tl - 1, ol - 1] = 0.0
+    links = tn.extract_valid_links(sq)
+    with torch.no_grad():
+        rloss = tn.torch_dag_loss(match.double(), tn.restore_valid_links(links.double()), ol, tl)
+    leaf = match.to(DEV).requires_grad_(with_grad)
+    loss = dagx.dag_loss(leaf, links.to(DEV), ol.to(DEV), tl.to(DEV)).detach().cpu().double()
+    fin = torch.isfinite(rloss)
+    assert int(fin.sum()) > B // 4 and torch.equal(torch.isfinite(loss), fin)
+    # what two sweeps may differ by and still stand (1e-4), on top of float32 rounding of the result
+    assert ((loss - rloss)[fin].abs() <= 1e-4 + 2e-7 * rloss[fin].abs()).all(), (loss - rloss)[fin].abs().max()
