@@ -304,7 +304,7 @@ __device__ __host__ inline AlignLds align_lds(int jb0, int nblk, int W, int spac
 // T = 256 445 and 476).
 template <typename TM, typename TL, int SPACING>
 __global__ __launch_bounds__(kTileWaves * kWave) void dag_align_chunks_kernel(AlignTileArgs a) {
-    extern __shared__ float lds_raw[];
+    extern __shared__ __align__(16) float lds_raw[];
     __shared__ int gstart[16];
     __shared__ int s_ticket, s_abort;
 

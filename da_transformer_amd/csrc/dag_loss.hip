@@ -890,7 +890,7 @@ __device__ __forceinline__ bool readouts_disagree(double za, double zb, bool wid
 
 template <typename TM, typename TL, bool WIDE>
 __global__ __launch_bounds__(kTileWaves * kWave) void dag_sweep_tiles_kernel(SweepArgs a) {
-    extern __shared__ float lds_raw[];
+    extern __shared__ __align__(16) float lds_raw[];
     __shared__ int gstart[kTileCap + 2];
     __shared__ int s_ticket, s_abort;
     const int tid = threadIdx.x;
