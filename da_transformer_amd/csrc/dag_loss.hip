@@ -527,7 +527,8 @@ __device__ __forceinline__ void sweep_chunks_group(const SweepArgs &a, const int
                 if (s0 + k + 1 < Tb) row += step;      // (rows past the last step: the last one again)
             }
         };
-        auto convert_match = [&](const int c, const int lane) __attribute__((always_inline)) {
+        // (with_pair: the walked chunk's fold_two is reduced along with the match rows)
+        auto convert_match = [&](const int c, const int lane, auto with_pair, float &pair) __attribute__((always_inline)) {
             const int s0 = kChunk * c + 1;
             float m[kChunk], top[kChunk];
 #pragma unroll
@@ -541,7 +542,7 @@ __device__ __forceinline__ void sweep_chunks_group(const SweepArgs &a, const int
             }
 #pragma unroll
             for (int k = 0; k < kChunk; ++k) top[k] = m[k];
-            wave64_max4(top);
+            wave64_max4<decltype(with_pair)::value>(top, pair);
             float log2e = kLog2e;
             asm("" : "+v"(log2e));                    // (an instruction takes one scalar register: N)
 #pragma unroll
@@ -562,11 +563,22 @@ __device__ __forceinline__ void sweep_chunks_group(const SweepArgs &a, const int
 #pragma unroll
             for (int k = 0; k < kChunk; ++k) mt[k] = fast_exp2(mt[k]);
         };
-        // the chunk just walked (cells v, exponents kk) into the tables
-        auto write_out = [&](const int c, const Cell (&v)[kChunk], const int (&kk)[kChunk], const int lane) __attribute__((always_inline)) {
+        // the chunk just walked (cells v, exponents kk; kept: the largest of its steps 0 and 2) into the tables
+        auto write_out = [&](const int c, const Cell (&v)[kChunk], const int (&kk)[kChunk], const float kept, const int lane) __attribute__((always_inline)) {
             const int s0 = kChunk * c + 1, row0 = dir ? Tb - 1 - s0 : s0;
             float res[kChunk], lf[kChunk];
             int ex[kChunk];
+            // In the table the offset is that of the block's largest cell, to a binade, in every step, and no residual is above 0
+            // (the gradients' rule on what their products hold counts on both): a step that kept its scale is moved by as many
+            // binades as its largest cell lies beside the scale.  (What the blocks of this group read in LDS stays as it is.  With the
+            // offsets as the walk has them, up to 44 binades above the largest cell, the backward at B = 16, L = 1024, T = 256 and
+            // transition logits of standard deviation 3 and 5 sent steps to its direct form for nothing: 78.9 -> 68.2 and
+            // 103.6 -> 93.6 us; the maxima cost the forward 0.7 us of 105 at L = 512, 1.1 of 57 in scoring.)
+            int moved[kChunk] = {0, 0, 0, 0};
+            if constexpr (!WIDE) {
+                moved[0] = (__builtin_amdgcn_readlane(__builtin_bit_cast(int, kept), 31) >> 23) - (126 + kShift2);
+                moved[2] = (__builtin_amdgcn_readlane(__builtin_bit_cast(int, kept), 63) >> 23) - (126 + kShift2);
+            }
 #pragma unroll
             for (int k = 0; k < kChunk; ++k) {   // (a dead cell: log of the fraction 0)
                 if constexpr (WIDE) {
@@ -576,7 +588,7 @@ __device__ __forceinline__ void sweep_chunks_group(const SweepArgs &a, const int
                 } else {
                     ex[k] = __builtin_amdgcn_frexp_expf(v[k]) - kShift2;
                     lf[k] = fast_log2(__builtin_amdgcn_frexp_mantf(v[k]));
-                    res[k] = ((float)ex[k] + lf[k]) * kLn2;
+                    res[k] = ((float)(ex[k] - moved[k]) + lf[k]) * kLn2;
                 }
             }
             const unsigned lane_off = (unsigned)(dir ? Lb - 1 - first - lane : first + lane) * 4u;
@@ -590,9 +602,10 @@ __device__ __forceinline__ void sweep_chunks_group(const SweepArgs &a, const int
             if (__builtin_expect(steps == kChunk && first + kBlk <= Lb, 1)) { put(0); put(1); put(2); put(3); }
             else if (first + lane < Lb) { put(0); if (steps > 1) put(1); if (steps > 2) put(2); if (steps > 3) put(3); }
             const int k01 = lane & 1 ? kk[1] : kk[0], k23 = lane & 1 ? kk[3] : kk[2], kp = lane & 2 ? k23 : k01;
+            const int kt = kp + (WIDE || (lane & 1) ? 0 : lane & 2 ? moved[2] : moved[0]);
             if (lane < steps)
                 store_agent(reinterpret_cast<double *>(const_cast<char *>(off_c) + (unsigned)((dir ? row0 - lane : row0 + lane) * NBK + J) * 8u),
-                            kp > kDeadBelow ? (double)kp * 0.6931471805599453 : (double)DAGX_NEG_INF);
+                            kt > kDeadBelow ? (double)kt * 0.6931471805599453 : (double)DAGX_NEG_INF);
             if (__builtin_expect(c == NC - 1 && J == NBb - 1, 0)) {   // the read-out
 #pragma unroll
                 for (int k = 0; k < kChunk; ++k)
@@ -742,14 +755,19 @@ __device__ __forceinline__ void sweep_chunks_group(const SweepArgs &a, const int
                             if (k < kChunk - 1) cells_this[CH::kStepPitch * (k + 1)] = 0; else cells_next[0] = 0;
                         }
                     }
-                    if (more) convert_match(c + 1, lane);   // (in front of the stores: what it waits for is older than they)
-                    else wait_vmem_all();
-                    const int kp = write_out(c, v, kk, lane);
+                    float kept = 0.f;
+                    if constexpr (!WIDE) kept = fold_two(v[0], v[2]);
+                    if (more) convert_match(c + 1, lane, std::bool_constant<!WIDE>{}, kept);   // (in front of the stores: what it waits for is older than they)
+                    else {
+                        if constexpr (!WIDE) half_max(kept);
+                        wait_vmem_all();
+                    }
+                    const int kp = write_out(c, v, kk, kept, lane);
                     const int sl = (lane & 3) < kChunk - 1 ? slot_own * 4 + 1 + (lane & 3) : next_slot(slot_own) * 4;
                     if (lane < kChunk) lds_i[o.kap + own_src * D * 4 + sl] = kp;
                     slot_own = next_slot(slot_own);
                 }
-                else if (more) convert_match(c + 1, lane);
+                else if (more) { float none = 0.f; convert_match(c + 1, lane, std::false_type{}, none); }
                 else if (c == NC) wait_vmem_all();
             }
             // ---------------- multiply out what my tiles' blocks (q of the group) receive in chunk tau + 1 - q ----------------

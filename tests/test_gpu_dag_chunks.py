@@ -1,13 +1,14 @@
-"""The chunked sweeps of dag_loss, in float32 and float64, and of dag_best_alignment at the sizes where they can go
-wrong: graphs one node short of, at and one
-past a block of 64 and a group's last block, targets one step around a chunk of four, transition windows around a block,
+"""The chunked sweeps of dag_loss, in float32 and float64, and of dag_best_alignment at the sizes where they can go wrong:
+graphs one node short of, at and one past a block of 64 and a group's last block, targets one step around a chunk of four, transition windows around a block,
 transitions that start at an odd element of their tensor or are its very first and last ones, one sample alone."""
+import math
+
 import pytest
 import torch
 
 import da_transformer_amd as dagx
 from da_transformer_amd import _native as nat
-from da_transformer_amd.custom_ops.dag_loss import DagLossFunc
+from da_transformer_amd.custom_ops.dag_loss import DagLossFunc, _sweep_offsets
 from oracle import torch_native as tn
 from helpers import random_problem
 from test_gpu_dag import DEV, hip_loss_and_grads, oracle_loss_and_grads, assert_close, RTOL
@@ -76,3 +77,40 @@ def test_alignment_at_edges_of_blocks_chunks_and_windows(B, L, T, translen, dtyp
     some = sorted({0, min(1, B - 1), B // 2, B - 1})
     want = tn.torch_dag_best_alignment(match[1:][some].float(), tn.restore_valid_links(links[1:][some].float()), ol[some], tl[some])
     assert torch.equal(got[some], want)
+
+
+@pytest.mark.parametrize("wide", [False, True])
+@pytest.mark.parametrize("B,L,T,translen,score", [
+    (2, 640, 41, 639, 0.0),        # hundreds of predecessors with transitions of 1 feed every cell: sums of up to 2^9 cells
+    (2, 1024, 102, 1023, -0.01), (3, 200, 22, 64, 0.0),
+    (2, 130, 9, 129, None), (3, 512, 64, 511, None), (65, 321, 30, 320, None)])
+def test_tables_are_relative_to_the_largest_cell_of_their_block(B, L, T, translen, score, wide):
+    """What the gradients rely on, in every step and not only in those that scale their cells: a residual is never above 0, and
+    the largest one of a block with a live cell lies within a binade below it."""
+    match, links_sq, ol, tl = random_problem(L + T, B, L, T, dtype=F32, ragged=False, translen=translen)
+    if score is not None:
+        links_sq = torch.where(torch.isfinite(links_sq), torch.tensor(score), links_sq)
+        match = torch.where(torch.isfinite(match), torch.tensor(score), match)
+    ol = torch.minimum(ol, (tl - 1) * translen + 1)
+    ol[B - 1] = max(T, L - 37)
+    links = tn.extract_valid_links(links_sq, translen)
+    before = nat.lib().dagx_loss_float64_first(int(wide))
+    try:
+        loss = DagLossFunc.apply(match.to(DEV).requires_grad_(), links.to(DEV), ol.to(DEV), tl.to(DEV))
+    finally:
+        nat.lib().dagx_loss_float64_first(before)
+    assert (DagLossFunc.last_sample_flags.cpu() == (2 if wide else 0)).all()
+    hats, offs = (x.cpu() for x in loss.grad_fn.saved_tensors[:2])
+    NBK = (L + 63) // 64
+    nhat, noff = _sweep_offsets(B, T, L)
+    for direction in range(2):
+        hat = hats[direction * nhat:(direction + 1) * nhat].view(B, T, L)
+        off = offs[direction * noff:(direction + 1) * noff].view(B, T, NBK)
+        for b in range(B):
+            n, steps = int(ol[b]), int(tl[b])
+            cells = hat[b, :steps, :n].flip(1) if direction else hat[b, :steps, :n]      # by position
+            cells = torch.nn.functional.pad(cells, (0, -n % 64), value=float("-inf")).view(steps, -1, 64)
+            top, alive = cells.amax(2), torch.isfinite(off[b, :steps, :cells.shape[1]])
+            assert (top[alive] <= 0).all(), (direction, b, top[alive].max())
+            # (a logarithm of a fraction in [1/2, 1), two float32 roundings)
+            assert (top[alive] >= -math.log(2.0) - 1e-6).all(), (direction, b, top[alive].min())
