@@ -229,7 +229,7 @@ static bool align_in_chunks(int B, int T, int L, int translen) {
 // for each block, at most ten.  (Fewer tiles a SIMD, against more hand-overs: as many as hold the tiles -> this, alignment of
 // B = 16, L = 1024, T = 256 484 -> 445 us; B = 4, L = 700, T = 100 211 -> 183; B = 64, L = 320, T = 48 83 -> 79; B = 64, L = 256,
 // T = 64 92 -> 80.)  Step by step: twice as many as hold the tiles where there is room and the graph has at least four
-// blocks (5 to 13 %; more lose); where that exceeds the 11 the kernel supports, ten when they fit.
+// blocks (5 to 13 %; more lose); where that exceeds what the kernel supports, ten when they fit.
 static int align_groups(int B, int T, int L, int translen) {
     const int NB = (L + kBlk - 1) / kBlk, B8 = (B + 7) & ~7;
     if (align_in_chunks(B, T, L, translen)) {
@@ -240,7 +240,7 @@ static int align_groups(int B, int T, int L, int translen) {
     }
     const int C = groups_needed(L, translen, kMaxBlocksFast);
     if (C == 0) return 0;
-    if (NB >= 4 && 2 * C <= 11 && 2 * C <= NB && (long long)B8 * 2 * C <= 256) return 2 * C;
+    if (NB >= 4 && 2 * C <= kMaxGroups && 2 * C <= NB && (long long)B8 * 2 * C <= 256) return 2 * C;
     return C < 10 && NB >= 10 && (long long)B8 * 10 <= 256 ? 10 : C;
 }
 

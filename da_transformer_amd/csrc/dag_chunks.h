@@ -3,6 +3,8 @@
 // triangle on the diagonal is walked step by step, by one wave.
 #pragma once
 
+#include <memory>
+
 #include "dag_tiles.h"
 
 namespace dagx {
@@ -200,16 +202,19 @@ inline void plan_chunks(int W, int C, const ChunkCosts (&costs)[N], ChunkPlan<N>
         }
     }
 }
-// the plan for a window of W blocks and C groups, remembered for the thread's next call (a plan takes 20 us to make; there are
-// at most kMaxBlocksFast windows, and C follows from the batch)
+// The plan for a window and a number of groups, remembered for the thread's later calls: a plan takes 10 to 25 us to make, and
+// C follows from the batch size, so that batches of changing size ask for several in turn.  There are at most
+// kMaxBlocksFast * kMaxGroups of them, 1 to 2 KB each, given back when the thread ends.
 template <int SPACING, int N>
 inline const ChunkPlan<N> &chunk_plan(int translen, int C, const ChunkCosts (&costs)[N]) {
-    struct Entry { int C = 0; ChunkPlan<N> plan; };
-    static thread_local Entry entries[kMaxBlocksFast];
+    static thread_local std::unique_ptr<ChunkPlan<N>> plans[kMaxBlocksFast][kMaxGroups];
     const int w = (translen + kBlk - 1) / kBlk, W = w < kMaxBlocksFast ? w : kMaxBlocksFast;
-    Entry &e = entries[W - 1];
-    if (e.C != C) { plan_chunks<SPACING>(W, C, costs, e.plan); e.C = C; }
-    return e.plan;
+    std::unique_ptr<ChunkPlan<N>> &plan = plans[W - 1][C - 1];
+    if (!plan) {
+        plan.reset(new ChunkPlan<N>);
+        plan_chunks<SPACING>(W, C, costs, *plan);
+    }
+    return *plan;
 }
 
 // ---- what a wave has to do, worked out at the start of the kernel ----

@@ -9,6 +9,7 @@ namespace dagx {
 
 constexpr int kBlk = 64;            // positions per block
 constexpr int kMaxBlocksFast = 16;  // fast path: L <= 1024
+constexpr int kMaxGroups = 11;      // workgroups of one sweep
 constexpr int kTileWaves = 8;       // waves per workgroup in the tile sweeps
 constexpr int kTilesPerWave = 3;    // register-resident tiles per wave
 constexpr int kTileCap = kTileWaves * kTilesPerWave;
@@ -39,7 +40,7 @@ inline int groups_needed(int L, int translen, int most) {
         if (sum + c > kTileCap || blocks == most) { ++groups; sum = blocks = 0; }
         sum += c; ++blocks;
     }
-    return groups <= 11 ? groups : 0;
+    return groups <= kMaxGroups ? groups : 0;
 }
 
 // ---- DPP lane reductions (no LDS traffic) ----------------------------------------------------
