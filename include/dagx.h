@@ -175,11 +175,13 @@ int dagx_prepare_device(void);
 /*
  * dagx_loss_fwd for callers that cannot allocate device memory (code under HIP graph capture, tight serving
  * loops, harnesses that forbid hipMalloc).  It has no counterpart in the reference.  Same arguments and
- * results as dagx_loss_fwd but for the workspace: the pipeline words live in a device array of
- * dagx_loss_fwd_noalloc_max_bytes() = 128 KiB that the library owns (one copy per GPU, held until the process
- * ends), so the call allocates nothing, frees nothing and calls no allocating routine.  Shapes whose
- * dagx_workspace_bytes(DAGX_OP_LOSS_FWD, ...) exceed that size are refused with DAGX_ERR_UNSUPPORTED (with
- * B <= 64 every graph size fits; L <= 512 fits up to B = 1024).  All calls on one GPU share the array: calls
+ * results as dagx_loss_fwd but for the workspace: the pipeline words live in a device array of 160 KiB that the
+ * library owns (one copy per GPU, held until the process ends), so the call allocates nothing, frees nothing and calls
+ * no allocating routine.  A shape whose dagx_workspace_bytes(DAGX_OP_LOSS_FWD, ...) are at most
+ * dagx_loss_fwd_noalloc_max_bytes() = 128 KiB is taken, one with more than 160 KiB refused with DAGX_ERR_UNSUPPORTED.
+ * In between it is taken if it would need at most 128 KiB in groups of as many blocks of nodes as hold its tiles (graphs
+ * of more than 512 nodes with short transitions are swept by more groups than that); ask by calling, a refusal
+ * launches nothing.  (With B <= 64 every graph size fits, L <= 512 up to B = 1024.)  All calls on one GPU share the array: calls
  * that overlap in time on one GPU (different streams, or different host threads) race and must be
  * serialised by the caller; consecutive calls on one stream are fine (the kernels leave the array zero, which
  * is the state they need on entry).  Under stream capture: call dagx_prepare_device() once on the device before

@@ -171,3 +171,19 @@ def test_what_the_built_in_scratch_takes_does_not_depend_on_the_grouping(B, acce
     assert (rc == 2) == (not accepted), lib.dagx_last_error()
     if not accepted:
         assert b"scratch" in lib.dagx_last_error()
+
+
+@pytest.mark.parametrize("L,translen", [(64, 63), (512, 511), (513, 64), (640, 100), (768, 64), (768, 767), (1024, 32), (1024, 1023)])
+def test_the_built_in_scratch_takes_what_its_header_says(L, translen):
+    """Up to dagx_loss_fwd_noalloc_max_bytes() of workspace a shape is taken, beyond 160 KiB it is refused."""
+    lib = _native.lib()
+    s3 = (ctypes.c_int64 * 3)(14 * L, L, 1)
+    most = lib.dagx_loss_fwd_noalloc_max_bytes()
+    assert most == 128 * 1024
+    for B in [*range(1, 8192, 61), 4090, 4094, 4095, 5118, 5119]:
+        need = lib.dagx_workspace_bytes(_native.OP_LOSS_FWD, B, 14, L, translen)
+        rc = lib.dagx_loss_fwd_noalloc(None, 0, s3, None, 0, None, None, B, 14, L, translen, None, None, None, None, None, None, None, 1, None)
+        if need <= most:
+            assert rc != 2, (B, need)        # (but for the null pointers; nothing is launched)
+        elif need > 160 * 1024:
+            assert rc == 2, (B, need)
