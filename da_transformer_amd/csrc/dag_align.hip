@@ -5,8 +5,9 @@
 //
 // Two implementations:
 //  * dag_align_chunks_kernel or dag_align_steps_kernel + dag_backtrack_kernel (L <= 1024): the sweep keeps E as 64x64 register
-//    tiles and evaluates a step with one DPP-broadcast add and one max per (i, j) pair, spread over
-//    the same pipeline of workgroups as the loss sweeps; it stores only the score table.  The
+//    tiles, spread over the same pipeline of workgroups as the loss sweeps, and forms two DPP-broadcast sums and one
+//    three-way maximum per two (i, j) pairs -- four steps a stage, or, for few steps on many nodes, step by step
+//    (align_in_chunks).  It stores the score table and the block of 64 nodes each cell's best predecessor lies in.  The
 //    backtrack (a wave per sample walks, others may stage for it) then re-derives, for the T_b cells on the path only, the
 //    lowest predecessor index attaining the stored maximum.
 //  * dag_align_kernel: one workgroup per sample, thread <-> node j scanning its predecessors in

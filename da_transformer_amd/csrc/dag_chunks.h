@@ -50,7 +50,6 @@ template <> struct Chunks<true> {
 };
 
 typedef float f32x4 __attribute__((ext_vector_type(4)));
-typedef int i32x4 __attribute__((ext_vector_type(4)));
 typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
 
 // Tiles that are multiplied out a stage ahead: those below the diagonal, with SPACING 1 but for the one next to it.
@@ -104,11 +103,11 @@ constexpr int kChunkLdsBytes = 160 * 1024 - 512;
 struct TileDeal { unsigned wave; };          // four bits a wave: tiles, foreign blocks << 2
 __device__ __host__ __forceinline__ int dealt_tiles(const TileDeal &d, int wave) { return (d.wave >> (4 * wave)) & 3; }
 __device__ __host__ __forceinline__ int dealt_foreign(const TileDeal &d, int wave) { return (d.wave >> (4 * wave + 2)) & 3; }
-// returns how long the busiest wave or SIMD takes, -1 if there are more tiles than the waves have room for
 // What a wave does in a stage, in hundreds of cycles, alone on its SIMD: walking a block (with SPACING 1 with the product
 // of the adjacent tile), a tile, fetching a foreign block; and how much of the sum of two waves' work a SIMD takes for both, in per cent
 // (waves w and w + 4 share one).
 struct ChunkCosts { int walk, product, fetch, shared; };
+// Returns how long the busiest wave or SIMD takes, -1 if there are more tiles than the waves have room for.
 template <int SPACING>
 inline int deal_tiles(int jb0, int nblk, int W, const ChunkCosts &cost, TileDeal &deal) {   // (on the host: a plan made by the kernel costs it 2 us)
     constexpr int kSimds = 4;
@@ -430,25 +429,15 @@ __device__ __forceinline__ int row16_max_int(int v) {
     return v;
 }
 
-// g[t] (+)= f[lane t of the row] * a[t]: four steps, each with its own factor
-template <bool FIRST>
+// g[t] += f[lane t of the row] * a[t]: four steps, each with its own factor
 __device__ __forceinline__ void scaled4(f32x4 &g, float f, f32x4 a) {
     float g0 = g[0], g1 = g[1], g2 = g[2], g3 = g[3];
-    if constexpr (FIRST) {
-        asm("s_nop 1\n\t"
-            "v_mul_f32_dpp %0, %4, %5 row_newbcast:0 row_mask:0xf bank_mask:0xf\n\t"
-            "v_mul_f32_dpp %1, %4, %6 row_newbcast:1 row_mask:0xf bank_mask:0xf\n\t"
-            "v_mul_f32_dpp %2, %4, %7 row_newbcast:2 row_mask:0xf bank_mask:0xf\n\t"
-            "v_mul_f32_dpp %3, %4, %8 row_newbcast:3 row_mask:0xf bank_mask:0xf"
-            : "=&v"(g0), "=&v"(g1), "=&v"(g2), "=&v"(g3) : "v"(f), "v"(a[0]), "v"(a[1]), "v"(a[2]), "v"(a[3]));
-    } else {
-        asm("s_nop 1\n\t"
-            "v_fmac_f32_dpp %0, %4, %5 row_newbcast:0 row_mask:0xf bank_mask:0xf\n\t"
-            "v_fmac_f32_dpp %1, %4, %6 row_newbcast:1 row_mask:0xf bank_mask:0xf\n\t"
-            "v_fmac_f32_dpp %2, %4, %7 row_newbcast:2 row_mask:0xf bank_mask:0xf\n\t"
-            "v_fmac_f32_dpp %3, %4, %8 row_newbcast:3 row_mask:0xf bank_mask:0xf"
-            : "+v"(g0), "+v"(g1), "+v"(g2), "+v"(g3) : "v"(f), "v"(a[0]), "v"(a[1]), "v"(a[2]), "v"(a[3]));
-    }
+    asm("s_nop 1\n\t"
+        "v_fmac_f32_dpp %0, %4, %5 row_newbcast:0 row_mask:0xf bank_mask:0xf\n\t"
+        "v_fmac_f32_dpp %1, %4, %6 row_newbcast:1 row_mask:0xf bank_mask:0xf\n\t"
+        "v_fmac_f32_dpp %2, %4, %7 row_newbcast:2 row_mask:0xf bank_mask:0xf\n\t"
+        "v_fmac_f32_dpp %3, %4, %8 row_newbcast:3 row_mask:0xf bank_mask:0xf"
+        : "+v"(g0), "+v"(g1), "+v"(g2), "+v"(g3) : "v"(f), "v"(a[0]), "v"(a[1]), "v"(a[2]), "v"(a[3]));
     g = f32x4{g0, g1, g2, g3};
 }
 

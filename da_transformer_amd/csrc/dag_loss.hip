@@ -812,7 +812,7 @@ __device__ __forceinline__ void sweep_chunks_group(const SweepArgs &a, const int
                         } else {
                             const f32x4 v = tile_product(tile, ev[u & 1]);
                             f32x4 sum = {G[0], G[1], G[2], G[3]};
-                            scaled4<false>(sum, pow2_clamped(kv[u] - R, floor_exp), v);
+                            scaled4(sum, pow2_clamped(kv[u] - R, floor_exp), v);
 #pragma unroll
                             for (int k = 0; k < 4; ++k) G[k] = sum[k];
                         }

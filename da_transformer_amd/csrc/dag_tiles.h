@@ -44,11 +44,6 @@ inline int groups_needed(int L, int translen, int most) {
 }
 
 // ---- DPP lane reductions (no LDS traffic) ----------------------------------------------------
-template <int CTRL>
-__device__ __forceinline__ float dpp_mov(float v) {
-    return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(__builtin_bit_cast(int, v), __builtin_bit_cast(int, v),
-                                                                 CTRL, 0xf, 0xf, false));
-}
 // max over each 16-lane row, result in every lane of the row (butterfly; each DPP op needs its
 // source written two wait states earlier)
 __device__ __forceinline__ float row16_max(float v) {
@@ -63,19 +58,6 @@ __device__ __forceinline__ float row16_max(float v) {
         "v_max_f32_dpp %0, %0, %0 row_mirror row_mask:0xf bank_mask:0xf"
         : "=&v"(r) : "v"(v));
     return r;
-}
-// inclusive prefix max within each 16-lane row: lane k gets max over lanes 0..k of the row
-__device__ __forceinline__ float row16_prefix_max(float v) {
-    asm("s_nop 1\n\t"
-        "v_max_f32_dpp %0, %0, %0 row_shr:1 row_mask:0xf bank_mask:0xf\n\t"
-        "s_nop 1\n\t"
-        "v_max_f32_dpp %0, %0, %0 row_shr:2 row_mask:0xf bank_mask:0xf\n\t"
-        "s_nop 1\n\t"
-        "v_max_f32_dpp %0, %0, %0 row_shr:4 row_mask:0xf bank_mask:0xf\n\t"
-        "s_nop 1\n\t"
-        "v_max_f32_dpp %0, %0, %0 row_shr:8 row_mask:0xf bank_mask:0xf"
-        : "+v"(v));
-    return v;
 }
 __device__ __forceinline__ float lane_bcast(float v, int lane) {
     return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), lane));
