@@ -9,7 +9,8 @@ fp32 accumulation), inputs resident in HBM: `value` = samples/s over the timed s
 run also times, with HIP events on the launch stream, the individual operators through the C ABI:
 
   roofline         the tile sweeps of the forward (the headline's dominant kernel) against the
-                   vector-ALU roof, HBM bytes per launch read from the committed traffic profile
+                   roof of their mix of vector and matrix instructions (a SIMD issues one or the
+                   other), HBM bytes per launch read from the committed traffic profile
   roofline_dp      sweeps + gradient kernels against the same roof (frac: the two timed one by one;
                    frac_over_timed_steps: the same work over the timed steps of `value`)
   roofline_gather  log-softmax + gather backward (and forward) at [64,512,40000] fp16 against 8 TB/s
@@ -33,6 +34,7 @@ sys.path.insert(0, os.path.join(ROOT, "tests"))
 
 HBM_PEAK_GBS = 8000.0            # MI355X HBM3E, published
 VALU_PEAK_LANEOPS = 256 * 64 * 2.4e9   # 256 CUs x 64 fp32 lanes x 2.4 GHz (single issue)
+MFMA_F32_PEAK_PAIRS = 2 * VALU_PEAK_LANEOPS   # the same per pair-update on v_mfma_f32 (157.3 TFLOP/s, published)
 CALIBRATION_COPY_BYTES = 1 << 30       # the --leg dag run ends with three plain device copies of this size
 
 
@@ -640,6 +642,11 @@ def main():
     # ---- roofline of the headline's dominant kernel: the tile sweeps (one launch = both sweeps = 2U pair-updates;
     #      the timed forward also contains the check launch behind it, which finds nothing to redo) ----
     fwd_s = k16["fwd_ms"] * 1e-3
+    # pair-updates inside a block of 64 positions are vector FMAs, the others float32 matrix products at twice their rate; a
+    # SIMD gives its cycles to one or the other
+    on_diagonal = (L // 64) * (64 * 63 // 2) / (L * (L - 1) // 2)
+    sweep_peak = 1.0 / (on_diagonal / VALU_PEAK_LANEOPS + (1 - on_diagonal) / MFMA_F32_PEAK_PAIRS)
+    dp_peak = 3.0 / (2 / sweep_peak + 1 / MFMA_F32_PEAK_PAIRS)      # two sweeps, and the gradient on the matrix cores
     sweep_traffic = traffic_bytes("dag_loss_B64_L512_T64_hbm_traffic.md", "dagx::dag_sweep_tiles_kernel<__half, __half, false>", 3, 4)
     # LDS and vector-ALU utilisation of the same kernel from the committed counter summary (profiles/): busy fractions
     # of the LDS pipeline (128 bytes per clock and CU) and of the SIMDs, and the source revision they were taken at
@@ -657,26 +664,27 @@ def main():
     roofline = {"kernel": "dag_sweep_tiles_kernel<half,half,float32 numbers> (dagx_loss_fwd: the sweeps of alpha and beta)",
                 "valu_busy_frac": cell_frac(lds_row, 4), "lds_frac": cell_frac(lds_row, 8), "lds_bank_conflict_frac": cell_frac(lds_row, 9),
                 "counters_from": profile_source_revision("dag_loss_B64_L512_T64_sq_counters.md"),
-                "bound": "valu", "achieved": 2 * U / fwd_s, "peak": VALU_PEAK_LANEOPS, "unit": "pair-updates/s",
-                "frac": 2 * U / fwd_s / VALU_PEAK_LANEOPS, "traffic": sweep_traffic,
+                "bound": "valu+mfma", "achieved": 2 * U / fwd_s, "peak": sweep_peak, "unit": "pair-updates/s",
+                "frac": 2 * U / fwd_s / sweep_peak, "frac_of_valu_peak": 2 * U / fwd_s / VALU_PEAK_LANEOPS, "traffic": sweep_traffic,
                 "algorithmic_pair_updates": 2 * U, "kernel_ms": k16["fwd_ms"],
                 # kernel_ms is one dagx_loss_fwd between HIP events: the float32 tile sweeps and, behind them, the float64 and
                 # log-domain launches, idle here (4.6 us each in a kernel trace, about 1 us each back to back); the
                 # committed kernel trace has the tile kernel by itself
                 "kernel_ms_covers": "float32 tile sweeps + the idle float64 and log-domain launches of the same call",
                 "kernel_alone_avg_us_in_profile": trace_avg_us,
-                "frac_kernel_alone_from_profile": (2 * U / (trace_avg_us * 1e-6) / VALU_PEAK_LANEOPS) if trace_avg_us else None,
+                "frac_kernel_alone_from_profile": (2 * U / (trace_avg_us * 1e-6) / sweep_peak) if trace_avg_us else None,
                 "achieved_TFLOPs": 2 * 2 * U / fwd_s / 1e12,
                 "frac_of_published_fp32_vector_peak": 2 * 2 * U / fwd_s / 157.3e12,
-                "note": "peak = 256 CUs x 64 fp32 lanes x 2.4 GHz, one FMA per pair-update (the published 157.3 TFLOP/s "
-                        "counts packed FMAs, which this build does not use); traffic = HBM bytes per launch (not the bound)"}
+                "note": "peak = 256 CUs x 64 fp32 lanes x 2.4 GHz, one FMA per pair-update, for the blocks on the diagonal (the "
+                        "published 157.3 TFLOP/s counts packed FMAs, which this build does not use), twice that for the "
+                        "tiles below it; traffic = HBM bytes per launch (not the bound)"}
     dp_time_s = (k16["fwd_ms"] + k16["bwd_ms"]) * 1e-3
-    roofline_dp = {"bound": "valu", "achieved": 3 * U / dp_time_s, "peak": VALU_PEAK_LANEOPS,
-                   "unit": "pair-updates/s", "frac": 3 * U / dp_time_s / VALU_PEAK_LANEOPS,
+    roofline_dp = {"bound": "valu+mfma", "achieved": 3 * U / dp_time_s, "peak": dp_peak,
+                   "unit": "pair-updates/s", "frac": 3 * U / dp_time_s / dp_peak,
                    "pair_updates_per_step": 3 * U, "kernel_ms": dp_time_s * 1e3,
                    # the same work against the timed steps themselves (forward and backward alternate there, so a
                    # launch is set up while its predecessor drains; the legs above time each on its own)
-                   "timed_step_ms": ms_per_step, "frac_over_timed_steps": 3 * U / (ms_per_step * 1e-3) / VALU_PEAK_LANEOPS}
+                   "timed_step_ms": ms_per_step, "frac_over_timed_steps": 3 * U / (ms_per_step * 1e-3) / dp_peak}
 
     # ---- other DAG-loss workloads (kernel times through the C ABI) ----
     def other_dag_legs():
