@@ -335,7 +335,7 @@ __global__ __launch_bounds__(kTileWaves * kWave) void dag_align_chunks_kernel(Al
     const int slack = a.decode ? L : Lb - Tb;
     const int NBb = (Lb + kBlk - 1) / kBlk;
     const int W = (translen + kBlk - 1) / kBlk;
-    if (tid <= C) gstart[tid] = a.plan.gtab[NBb][tid];
+    if (tid <= C) gstart[tid] = a.plan.gtab[0][NBb][tid];
     __syncthreads();
     const int jb0 = __builtin_amdgcn_readfirstlane(gstart[g]), jb1 = __builtin_amdgcn_readfirstlane(gstart[g + 1]);
     int last_group = 0;
@@ -765,7 +765,7 @@ __global__ __launch_bounds__(kTileWaves * kWave) void dag_align_steps_kernel(Ali
     const int mcap = a.mcap;
     const int NBb = (Lb + kBlk - 1) / kBlk;
     const int W = (translen + kBlk - 1) / kBlk;
-    if (tid <= C) gstart[tid] = a.plan.gtab[NBb][tid];
+    if (tid <= C) gstart[tid] = a.plan.gtab[0][NBb][tid];
     __syncthreads();
     const int jb0 = __builtin_amdgcn_readfirstlane(gstart[g]), jb1 = __builtin_amdgcn_readfirstlane(gstart[g + 1]);
     int last_group = 0;
@@ -1306,7 +1306,7 @@ static int launch_align_sweep(AlignTileArgs &ta, const char *who, hipStream_t st
         int first[kTileCap + 2];
         for (int nb = 0; nb <= kMaxBlocksFast; ++nb) {
             partition_blocks(nb, W, ta.C, first);
-            for (int q = 0; q <= ta.C && q < 12; ++q) ta.plan.gtab[nb][q] = (unsigned char)first[q];
+            for (int q = 0; q <= ta.C && q < 12; ++q) ta.plan.gtab[0][nb][q] = (unsigned char)first[q];
         }
         hipLaunchKernelGGL((dag_align_steps_kernel<TM, TL>), dim3(((ta.B + 7) & ~7) * ta.C), dim3(kTileWaves * kWave), 0, st, ta);
         return check_launch(who);

@@ -103,9 +103,9 @@ constexpr int kChunkLdsBytes = 160 * 1024 - 512;
 struct TileDeal { unsigned wave; };          // four bits a wave: tiles, foreign blocks << 2
 __device__ __host__ __forceinline__ int dealt_tiles(const TileDeal &d, int wave) { return (d.wave >> (4 * wave)) & 3; }
 __device__ __host__ __forceinline__ int dealt_foreign(const TileDeal &d, int wave) { return (d.wave >> (4 * wave + 2)) & 3; }
-// What a wave does in a stage, in hundreds of cycles, alone on its SIMD: walking a block (with SPACING 1 with the product
-// of the adjacent tile), a tile, fetching a foreign block; and how much of the sum of two waves' work a SIMD takes for both, in per cent
-// (waves w and w + 4 share one).
+// How long a wave takes for its pieces of a stage, in about hundreds of cycles: walking a block (with SPACING 1 with the product
+// of the adjacent tile), a tile, fetching a foreign block (most of it waits); and how much of the sum of two waves' times a SIMD takes for
+// both, in per cent (waves w and w + 4 share one).
 struct ChunkCosts { int walk, product, fetch, shared; };
 // Returns how long the busiest wave or SIMD takes, -1 if there are more tiles than the waves have room for.
 template <int SPACING>
@@ -159,45 +159,50 @@ __device__ __host__ __forceinline__ void wave_foreign(const TileDeal &d, int wav
 // least to do.  gtab[nb][g] .. gtab[nb][g+1]: blocks of group g (empty groups last).
 template <int N>
 struct ChunkPlan {
-    unsigned char gtab[kMaxBlocksFast + 1][12];
-    TileDeal deal[N][kMaxBlocksFast + 1][12];     // one for each set of costs; the first set decides on the groups
+    // one of each for each set of costs
+    unsigned char gtab[N][kMaxBlocksFast + 1][12];
+    TileDeal deal[N][kMaxBlocksFast + 1][12];
+    short busiest[N][kMaxBlocksFast + 1];         // how long the busiest SIMD of the graph's groups takes; kNoPlan: C groups do not hold it
 };
+constexpr int kNoPlan = 1 << 12;
 template <int SPACING, int N>
 inline void plan_chunks(int W, int C, const ChunkCosts (&costs)[N], ChunkPlan<N> &plan) {
     constexpr int NB = kMaxBlocksFast;
-    int cost[NB][kChunkBlocks + 1];
-    TileDeal deal[N][NB][kChunkBlocks + 1];
-    for (int j = 0; j < NB; ++j) {
-        int tiles = 0;
-        for (int n = 1; n <= kChunkBlocks; ++n) {
-            cost[j][n] = -1;
-            if (j + n > NB) continue;
-            tiles += j + n - tile_ilo(j + n - 1, W);
-            if (tiles > kTileCap) continue;
-            for (int x = N - 1; x >= 0; --x) cost[j][n] = deal_tiles<SPACING>(j, n, W, costs[x], deal[x][j][n]);
-        }
-    }
-    for (int nb = 0; nb <= NB; ++nb) {
-        int low = 0, high = 1 << 12;                 // the least bound on a group's cost that C groups can keep
-        unsigned char g[16];
-        auto split = [&](const int most) {
-            int used = 0, j = 0;
-            g[0] = 0;
-            for (int q = 1; q < 16; ++q) g[q] = (unsigned char)nb;
-            while (j < nb) {
-                int n = 0;
-                for (int x = 1; x <= kChunkBlocks && j + x <= nb; ++x) if (cost[j][x] >= 0 && cost[j][x] <= most) n = x;
-                if (n == 0 || used == C) return false;
-                j += n;
-                g[++used] = (unsigned char)j;
+    for (int x = 0; x < N; ++x) {
+        int cost[NB][kChunkBlocks + 1];
+        TileDeal deal[NB][kChunkBlocks + 1];
+        for (int j = 0; j < NB; ++j) {
+            int tiles = 0;
+            for (int n = 1; n <= kChunkBlocks; ++n) {
+                cost[j][n] = -1;
+                if (j + n > NB) continue;
+                tiles += j + n - tile_ilo(j + n - 1, W);
+                if (tiles <= kTileCap) cost[j][n] = deal_tiles<SPACING>(j, n, W, costs[x], deal[j][n]);
             }
-            return true;
-        };
-        while (low < high) { const int mid = (low + high) / 2; if (split(mid)) high = mid; else low = mid + 1; }
-        split(high);
-        for (int q = 0; q < 12; ++q) {
-            plan.gtab[nb][q] = g[q];
-            for (int x = 0; x < N; ++x) plan.deal[x][nb][q] = q < C && g[q + 1] > g[q] && g[q + 1] - g[q] <= kChunkBlocks ? deal[x][g[q]][g[q + 1] - g[q]] : TileDeal{0};
+        }
+        for (int nb = 0; nb <= NB; ++nb) {
+            int low = 0, high = kNoPlan;                 // the least bound on a group's cost that C groups can keep
+            unsigned char g[16];
+            auto split = [&](const int most) {
+                int used = 0, j = 0;
+                g[0] = 0;
+                for (int q = 1; q < 16; ++q) g[q] = (unsigned char)nb;
+                while (j < nb) {
+                    int n = 0;
+                    for (int y = 1; y <= kChunkBlocks && j + y <= nb; ++y) if (cost[j][y] >= 0 && cost[j][y] <= most) n = y;
+                    if (n == 0 || used == C) return false;
+                    j += n;
+                    g[++used] = (unsigned char)j;
+                }
+                return true;
+            };
+            while (low < high) { const int mid = (low + high) / 2; if (split(mid)) high = mid; else low = mid + 1; }
+            split(high);
+            plan.busiest[x][nb] = (short)high;
+            for (int q = 0; q < 12; ++q) {
+                plan.gtab[x][nb][q] = g[q];
+                plan.deal[x][nb][q] = q < C && g[q + 1] > g[q] && g[q + 1] - g[q] <= kChunkBlocks ? deal[g[q]][g[q + 1] - g[q]] : TileDeal{0};
+            }
         }
     }
 }
@@ -214,6 +219,71 @@ inline const ChunkPlan<N> &chunk_plan(int translen, int C, const ChunkCosts (&co
         plan_chunks<SPACING>(W, C, costs, *plan);
     }
     return *plan;
+}
+
+// ---- how many groups a sample gets (the loss) ----
+// Table 0 has `least` groups for every sample, the others more for the longest samples and as many for shorter ones as it takes
+// to keep the bound that the longest can keep: the time of a batch is that of its longest samples.  A launch takes the last
+// table whose workgroups all find a CU; only the kernel knows the lengths, so it decides.  (B = 16, L = 1024, lengths from three
+// quarters on: nine groups for samples of 16 blocks, six for 13, against eight for all: sweep, T = 256 330 -> 303 us, T = 128
+// 213 -> 203; B = 14, L = 1000, T = 200 281 -> 257; B = 28, L = 640, T = 128 156 -> 147.)
+struct GroupTable {
+    unsigned char gtab[kMaxBlocksFast + 1][12];
+    TileDeal deal[kMaxBlocksFast + 1][12];
+};
+constexpr int kMostTables = 3;
+constexpr int kSweepCus = 256;          // workgroups of the sweeps that run side by side, one a CU
+constexpr int kMostForTables = kWave;   // batches of at most this many samples choose: a lane looks at a sample's length
+struct TableChoice {
+    unsigned long long ngroups[kMostTables];   // (tables 1 ..) four bits for each number of blocks from 1 on: a sample's groups
+    int ntable, least, most;                   // most: the most groups of any sample in any table
+};
+// A table is offered where the longest sample's stages (one a chunk, one a block, one and a half a hand-over) take at most 97 %
+// of what they take in `least` groups (L = 512, T = 170 in four groups, 97 to 99 % depending on T, 156 to 160 us for 156), and
+// where two sweeps of samples of seven eighths of L would all find a CU.
+template <int SPACING, int N>
+inline void make_tables(GroupTable (&tables)[kMostTables], TableChoice &o, int B, int T, int L, int translen, int least, const ChunkCosts (&costs)[N], int which) {
+    auto plan_of = [&](const int c) -> const ChunkPlan<N> & { return chunk_plan<SPACING>(translen, c, costs); };
+    auto copy_row = [&](GroupTable &table, const int nb, const ChunkPlan<N> &plan) {
+        for (int q = 0; q < 12; ++q) { table.gtab[nb][q] = plan.gtab[which][nb][q]; table.deal[nb][q] = plan.deal[which][nb][q]; }
+    };
+    o.ntable = 1;
+    o.least = o.most = least;
+    const int NB = (L + kBlk - 1) / kBlk, NC = (T - 1 + kChunk - 1) / kChunk;
+    for (int nb = 0; nb <= kMaxBlocksFast; ++nb) copy_row(tables[0], nb, plan_of(least));
+    if (B > kMostForTables || NB <= 4) return;
+    auto stages2 = [&](const int c) { return 2 * (NC + NB) + 3 * (c - 1); };
+    int best = plan_of(least).busiest[which][NB];
+    const long long now = (long long)best * stages2(least);
+    for (int c = least + 1; c <= kMaxGroups && o.ntable < kMostTables; ++c) {
+        const int bound = plan_of(c).busiest[which][NB];
+        if (bound >= best || 100 * (long long)bound * stages2(c) > 97 * now) continue;
+        GroupTable &table = tables[o.ntable];
+        unsigned long long ngroups = 0;
+        int most = 1;
+        for (int nb = 0; nb <= kMaxBlocksFast; ++nb) {
+            int u = nb >= 1 && nb <= NB ? 1 : c, n = 0;
+            while (u < c && plan_of(u).busiest[which][nb] > bound) ++u;
+            const ChunkPlan<N> &plan = plan_of(u);
+            copy_row(table, nb, plan);
+            if (nb < 1 || nb > NB) continue;
+            while (n < u && plan.gtab[which][nb][n + 1] > plan.gtab[which][nb][n]) ++n;
+            ngroups |= (unsigned long long)n << (4 * (nb - 1));
+            most = n > most ? n : most;
+        }
+        const int typical = (int)(ngroups >> (4 * ((7 * L / 8 + kBlk - 1) / kBlk - 1))) & 15;
+        if (2 * B * typical > kSweepCus) break;
+        o.ngroups[o.ntable++] = ngroups;
+        o.most = most > o.most ? most : o.most;
+        best = bound;
+    }
+}
+// Ticket r among those of the n samples that have a certain group -> which of the samples, which of its sweeps: a sample's
+// two sweeps eight tickets apart while there are eight samples more (so they mostly share an XCD).
+__device__ __host__ __forceinline__ void place_of_ticket(int r, int n, int ndir, int &rank, int &slot) {
+    const int full = n & ~7, rest = n - full > 0 ? n - full : 1;
+    if (r < ndir * full) { rank = (r / (8 * ndir)) * 8 + r % 8; slot = (r / 8) % ndir; }
+    else { r -= ndir * full; rank = full + r % rest; slot = r / rest; }
 }
 
 // ---- what a wave has to do, worked out at the start of the kernel ----

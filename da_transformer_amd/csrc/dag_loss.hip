@@ -46,16 +46,19 @@ struct SweepArgs {
     // [16 + (dir*B + b)*C + group] progress words, then [B] workgroups of the sample that have left, then [B] "risk"
     // words (a group of the sample gave up waiting for its producer)
     int *sync;
-    int C;             // workgroups per sweep (fast path)
+    int C;             // workgroups per sweep (fast path): the most of any table
+    TableChoice choice; // (here, not behind the tables: what a kernel reads first lies in as few lines of the argument block as possible)
     int ndir;          // sweeps per sample in the tile kernel: always two, which bracket the result (see sweep_chunks_group)
     // The two tile sweeps of a sample: direction (0: alpha, 1: beta) and rounding side (0: every number too small
     // for the linear domain becomes 0, a lower bound of the sum over paths; 1: it becomes the smallest number the
     // domain holds, an upper bound).  With gradients {alpha/upper, beta/lower}, without {alpha/lower, alpha/upper}.
     unsigned char rev[2], upper[2];
     int only_flagged;  // exact kernel: 0 = every sample; 1 = samples whose flag is set
-    ChunkPlan<2> plan; // fast path, host-built: gtab[NBb][g] = first block of group g, and how its tiles are dealt to its waves
-                       // (deal[0]: float32 sweeps, deal[1]: float64)
     double *zfast;     // [2][B] the fast kernel's own read-outs (never rewritten by the exact kernel)
+};
+
+struct TileSweepArgs : SweepArgs {
+    GroupTable table[kMostTables];   // fast path, host-built
 };
 
 __device__ __forceinline__ bool lengths_ok(int Lb, int Tb, int L, int T) {
@@ -277,8 +280,8 @@ __global__ __launch_bounds__(NT) void dag_sweep_exact_kernel(SweepArgs a) {
 // the launch clears the ticket counter -- so the words are all zero again when the launch is over and need no fill in
 // front of it.
 template <typename TM, typename TL, bool WIDE>
-__device__ __forceinline__ void sweep_chunks_group(const SweepArgs &a, const int b, const int slot, const int g, float *lds_raw,
-                                                   int *gstart, int *s_abort_p) {
+__device__ __forceinline__ void sweep_chunks_group(const TileSweepArgs &a, const GroupTable &plan, const int b, const int slot, const int g,
+                                                   float *lds_raw, int *gstart, int *s_abort_p) {
     using CH = Chunks<WIDE>;
     using Cell = typename CH::Cell;
     // slot: which of the sample's two sweeps (its tables, pipeline words and read-out); dir: its direction;
@@ -312,7 +315,7 @@ __device__ __forceinline__ void sweep_chunks_group(const SweepArgs &a, const int
     const int slack = Lb - Tb;                    // band: s <= p <= slack + s
     const int NBb = (Lb + kBlk - 1) / kBlk;
     const int W = (translen + kBlk - 1) / kBlk;
-    if (tid <= C) gstart[tid] = a.plan.gtab[NBb][tid];
+    if (tid <= C) gstart[tid] = plan.gtab[NBb][tid];
     __syncthreads();
     const int jb0 = __builtin_amdgcn_readfirstlane(gstart[g]), jb1 = __builtin_amdgcn_readfirstlane(gstart[g + 1]);
     int last_group = 0;
@@ -332,7 +335,7 @@ __device__ __forceinline__ void sweep_chunks_group(const SweepArgs &a, const int
     const bool owner = wave < nblk;               // this wave walks block jb0 + wave
     const int helpers = kTileWaves - nblk;
 
-    const TileDeal deal = a.plan.deal[WIDE][NBb][g];
+    const TileDeal deal = plan.deal[NBb][g];
     const WaveTiles t = plan_wave<1>(deal, jb0, nblk, W, o.runs, wave, lane);
     // A consumer group has nothing to do for the first stages: it lets the first group of its sweep have the memory's
     // bandwidth for its tiles.  (Progress words: 1 once the group's tiles are staged, then 2 + n when the rows of the first n
@@ -907,7 +910,7 @@ __device__ __forceinline__ bool readouts_disagree(double za, double zb, bool wid
 }
 
 template <typename TM, typename TL, bool WIDE>
-__global__ __launch_bounds__(kTileWaves * kWave) void dag_sweep_tiles_kernel(SweepArgs a) {
+__global__ __launch_bounds__(kTileWaves * kWave) void dag_sweep_tiles_kernel(TileSweepArgs a) {
     extern __shared__ __align__(16) float lds_raw[];
     __shared__ int gstart[kTileCap + 2];
     __shared__ int s_ticket, s_abort;
@@ -916,25 +919,68 @@ __global__ __launch_bounds__(kTileWaves * kWave) void dag_sweep_tiles_kernel(Swe
     // The wide launch behind a float32 launch that flagged nothing (the usual case) ends here, after one load: the
     // float32 launch counts the samples it flags in word 2 of the pipeline words, the wide launch clears it.
     if constexpr (WIDE) { if (a.sync[2] == 0) return; }
+    const int B8 = (a.B + 7) & ~7;
+    // Which table, and with it how many workgroups take part: all of them come to the same answer from the lengths alone.  The
+    // others leave at once; they are the last of the grid, so they cost a CU that has become free a look at the lengths.
+    int mine = 0, used = 0, workgroups = a.ndir * B8 * a.choice.least;   // (lane <-> sample) groups of a sample, table
+    if (a.choice.ntable > 1) {
+        const int lane = tid & (kWave - 1);
+        const int64_t len = a.out_len[lane < a.B ? lane : 0];
+        const int nb = len >= 1 && len <= a.L ? ((int)len + kBlk - 1) / kBlk : 1;
+        for (int x = a.choice.ntable - 1; x > 0 && used == 0; --x) {
+            const int n = lane < a.B ? (int)(a.choice.ngroups[x] >> (4 * (nb - 1))) & 15 : 0;
+            int all = n;
+#pragma unroll
+            for (int d = 32; d > 0; d >>= 1) all += __shfl_xor(all, d, kWave);
+            all = __builtin_amdgcn_readfirstlane(all) * a.ndir;
+            if (all <= kSweepCus) { mine = n; used = x; workgroups = all; }
+        }
+        used = __builtin_amdgcn_readfirstlane(used);
+        workgroups = __builtin_amdgcn_readfirstlane(workgroups);
+        if ((int)blockIdx.x >= workgroups) return;
+    }
     if (tid == 0) { s_ticket = atomicAdd(a.sync, 1); s_abort = 0; }
     __syncthreads();
     // ticket -> (group, sweep, sample): first group 0 of every sweep of every sample, then every group 1, and so on.
     // Every group waits only on groups with a smaller ticket, so a waiting workgroup's producers have already
     // started; and the workgroups that the dispatcher reaches last (it needs several microseconds for the grid)
     // are consumers, which could not start any sooner than their producers' first rows anyway.  The two sweeps of a
-    // sample are 8 tickets apart, the workgroups of a sample a multiple of 8: they share an XCD and its L2.
+    // sample are 8 tickets apart, the workgroups of a sample a multiple of 8 (table 0): they share an XCD and its L2.
     const int k = __builtin_amdgcn_readfirstlane(s_ticket);
-    const int B8 = (a.B + 7) & ~7;
-    const int runs = a.ndir * (B8 / 8);   // runs of eight (sweep, sample) pairs
-    const int g = k / (8 * runs), run = (k / 8) % runs;
-    const int b_k = (run / a.ndir) * 8 + (k % 8);
-    const bool has_sample = g < C && b_k < a.B;
-    const int b = has_sample ? b_k : 0, slot = has_sample ? run % a.ndir : 0;
+    int g, b_k, slot_k, groups = a.choice.least;
+    bool has_sample;
+    if (used == 0) {
+        const int runs = a.ndir * (B8 / 8);   // runs of eight (sweep, sample) pairs
+        const int run = (k / 8) % runs;
+        g = k / (8 * runs); slot_k = run % a.ndir;
+        b_k = (run / a.ndir) * 8 + (k % 8);
+        has_sample = g < a.choice.least && b_k < a.B;
+    } else {   // samples without a group g are passed over; k < workgroups, so there is a (group, sweep, sample) for it
+        int r = k, n = 0;
+        unsigned long long have = 0;
+        for (g = 0; g < C; ++g) {
+            have = __builtin_amdgcn_ballot_w64(mine > g);
+            n = __builtin_popcountll(have);
+            if (r < a.ndir * n) break;
+            r -= a.ndir * n;
+        }
+        int rank;
+        place_of_ticket(r, n, a.ndir, rank, slot_k);
+        const int lane = tid & (kWave - 1);
+        const int before = __builtin_popcountll(have & ((1ull << lane) - 1));
+        const unsigned long long at = __builtin_amdgcn_ballot_w64((have >> lane & 1) != 0 && before == rank);
+        has_sample = g < C && at != 0;
+        b_k = has_sample ? (int)__builtin_ctzll(at) : 0;
+        groups = __builtin_amdgcn_readlane(mine, b_k);
+    }
+    has_sample = __builtin_amdgcn_readfirstlane(has_sample) != 0;
+    g = __builtin_amdgcn_readfirstlane(g);
+    const int b = __builtin_amdgcn_readfirstlane(has_sample ? b_k : 0), slot = __builtin_amdgcn_readfirstlane(has_sample ? slot_k : 0);
     // a launch for flagged samples only (the wide variant behind the float32 one): the workgroups of the others
     // leave at once, through the same bookkeeping
     const bool skip = has_sample && a.only_flagged && a.flags[b] != 1;
     if (has_sample && !skip) {
-        sweep_chunks_group<TM, TL, WIDE>(a, b, slot, g, lds_raw, gstart, &s_abort);
+        sweep_chunks_group<TM, TL, WIDE>(a, a.table[used], b, slot, g, lds_raw, gstart, &s_abort);
     }
     // ---- leaving ----
     wait_vmem_all();   // this wave's stores (table rows, read-outs) are complete
@@ -943,7 +989,7 @@ __global__ __launch_bounds__(kTileWaves * kWave) void dag_sweep_tiles_kernel(Swe
         if (has_sample) {
             int *left = a.sync + 16 + a.ndir * a.B * C + b, *risk = left + a.B;
             const int n = __hip_atomic_fetch_add(left, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1;
-            if (n == a.ndir * C) {   // every workgroup of the sample has left
+            if (n == a.ndir * groups) {   // every workgroup of the sample has left
                 bool bad = load_agent(risk) != 0;
                 const int Lb = (int)a.out_len[b], Tb = (int)a.tgt_len[b];
                 if (!bad && lengths_ok(Lb, Tb, a.L, a.T)) {
@@ -959,7 +1005,7 @@ __global__ __launch_bounds__(kTileWaves * kWave) void dag_sweep_tiles_kernel(Swe
             }
         }
         const int n_all = __hip_atomic_fetch_add(a.sync + 1, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1;
-        if (n_all == (int)gridDim.x) { store_agent(a.sync, 0); store_agent(a.sync + 1, 0); if (WIDE) store_agent(a.sync + 2, 0); }
+        if (n_all == workgroups) { store_agent(a.sync, 0); store_agent(a.sync + 1, 0); if (WIDE) store_agent(a.sync + 2, 0); }
     }
 }
 
@@ -1569,11 +1615,15 @@ static size_t sweep_sync_ints(int B, int C) { return ((16 + (size_t)2 * B * C + 
 // Workgroups per sweep (two sweeps a sample): as few as hold the tiles, but with at most four blocks each, one walk to a
 // SIMD, where the device has a CU for every workgroup.  Forward with up to eight -> up to four blocks: B = 40, L = 328,
 // T = 41 67 -> 61 us; B = 16, L = 512, T = 64 102 -> 97.5; B = 64 and transitions of at most 32 88 -> 79; B = 16,
-// L = 1024 and transitions of at most 64 122 -> 104.  More groups than that gain nothing (L = 512 in four 96 us) or lose
-// (L = 256 in two 66 us for 64).
+// L = 1024 and transitions of at most 64 122 -> 104.  More groups than that: see make_tables.
 static int sweep_groups(int B, int L, int translen) {
     const int C = groups_needed(L, translen, 4), sweeps = 2 * ((B + 7) & ~7);
-    return (long long)sweeps * C <= 256 && C > 0 ? C : groups_needed(L, translen, kChunkBlocks);
+    return (long long)sweeps * C <= kSweepCus && C > 0 ? C : groups_needed(L, translen, kChunkBlocks);
+}
+// The most groups a launch may have (the workspace is laid out for them, whatever T).
+static int most_groups(int B, int L, int translen) {
+    const int C = sweep_groups(B, L, translen);
+    return C > 0 && B <= kMostForTables ? kMaxGroups : C;
 }
 
 // ticket + progress words (rounded to 8 bytes), then the fast kernel's two read-outs per sample
@@ -1581,7 +1631,7 @@ static size_t sweep_bytes(int B, int C) { return sweep_sync_ints(B, C) * sizeof(
 
 size_t loss_fwd_workspace_bytes(int B, int T, int L, int translen) {
     (void)T;
-    const int C = sweep_groups(B, L, translen);
+    const int C = most_groups(B, L, translen);
     return C > 0 ? sweep_bytes(B, C) : 0;
 }
 
@@ -1614,8 +1664,17 @@ static int prepare_tiles_kernels_of() {
     return rc;
 }
 
+// float32, float64.  Found by timing the sweeps themselves under some forty sets (us; first the costs of each piece timed alone,
+// with a SIMD taking the sum of its two waves' work, {45, 7, 4, 100} and {85, 17, 11, 100}; then these): float32 B = 64, L = 512, T = 64
+// 107 -> 95; B = 16, L = 1024, T = 256 347 -> 329; B = 16, L = 512, T = 128 134 -> 127; B = 8, L = 1024, T = 256 334 -> 302; float64 at the
+// first of them 151 -> 141.  A fetched block waits for the rows of its producer and for LDS twice, so it keeps its wave for longer than
+// its instructions take; and while a wave waits, the other wave of its SIMD works.
+static const ChunkCosts kSweepCosts[2] = {{45, 9, 12, 70}, {85, 25, 16, 80}};
+
 template <typename TM, typename TL>
-static int launch_sweeps(SweepArgs a, hipStream_t st) {
+static int launch_sweeps(SweepArgs base, hipStream_t st) {
+    TileSweepArgs a{};
+    static_cast<SweepArgs &>(a) = base;
     int C = force_exact() ? 0 : sweep_groups(a.B, a.L, a.translen);
     // the tile kernel indexes match with 32-bit arithmetic
     const int64_t span = (int64_t)(a.T - 1) * (a.ms1 < 0 ? -a.ms1 : a.ms1) + (int64_t)(a.L - 1) * (a.ms2 < 0 ? -a.ms2 : a.ms2);
@@ -1627,7 +1686,6 @@ static int launch_sweeps(SweepArgs a, hipStream_t st) {
         if ((rc = check_launch("dag_fill"))) return rc;
     }
     if (C > 0) {
-        a.zfast = reinterpret_cast<double *>(a.sync + sweep_sync_ints(a.B, C));
         // Two sweeps per sample whose read-outs bracket log Z.  With gradients they are the alpha sweep (rounding
         // up) and the beta sweep (rounding down; its read-out is the loss, as in fs_plugins/custom_ops/dag_loss.py:106-109).
         // Without, the reference runs the alpha sweep alone (dag_loss.cu:346-371); here a second alpha sweep that
@@ -1635,14 +1693,17 @@ static int launch_sweeps(SweepArgs a, hipStream_t st) {
         a.ndir = 2;
         a.rev[0] = 0; a.rev[1] = a.loss_dir ? 1 : 0;
         a.upper[0] = a.loss_dir ? 1 : 0; a.upper[1] = a.loss_dir ? 0 : 1;
-        a.C = C;
-        static const ChunkCosts kCosts[2] = {{45, 7, 4, 100}, {85, 17, 11, 100}};   // (measured)
-        a.plan = chunk_plan<1>(a.translen, C, kCosts);
         const int B8 = (a.B + 7) & ~7;
+        auto plan_for = [&](const bool wide) {
+            make_tables<1>(a.table, a.choice, a.B, a.T, a.L, a.translen, C, kSweepCosts, wide);
+            a.C = a.choice.most;
+            a.zfast = reinterpret_cast<double *>(a.sync + sweep_sync_ints(a.B, a.C));   // (zero again behind every launch, as the words in front)
+        };
+        plan_for(float64_first());
         if ((rc = prepare_tiles_kernel<TM, TL, false>()) || (rc = prepare_tiles_kernel<TM, TL, true>())) return rc;
         if (!float64_first()) {
             a.only_flagged = 0;
-            hipLaunchKernelGGL((dag_sweep_tiles_kernel<TM, TL, false>), dim3(a.ndir * B8 * C), dim3(kTileWaves * kWave), kChunkLdsBytes, st, a);
+            hipLaunchKernelGGL((dag_sweep_tiles_kernel<TM, TL, false>), dim3(a.ndir * B8 * a.C), dim3(kTileWaves * kWave), kChunkLdsBytes, st, a);
             if ((rc = check_launch("dag_sweep_tiles"))) return rc;
         } else {   // the caller knows its inputs for sharply peaked: no float32 pass whose result would not stand
             hipLaunchKernelGGL(dag_mark_all_kernel, dim3((a.B + 255) / 256), dim3(256), 0, st, a.flags, a.B, a.sync);
@@ -1651,18 +1712,20 @@ static int launch_sweeps(SweepArgs a, hipStream_t st) {
         // the samples whose two read-outs did not agree, once more with float64 linear-domain numbers (the pipeline
         // words are zero again, as the first launch found them)
         a.only_flagged = 1;
-        hipLaunchKernelGGL((dag_sweep_tiles_kernel<TM, TL, true>), dim3(a.ndir * B8 * C), dim3(kTileWaves * kWave), kChunkLdsBytes, st, a);
+        if (!float64_first()) plan_for(true);
+        hipLaunchKernelGGL((dag_sweep_tiles_kernel<TM, TL, true>), dim3(a.ndir * B8 * a.C), dim3(kTileWaves * kWave), kChunkLdsBytes, st, a);
         if ((rc = check_launch("dag_sweep_tiles (wide)"))) return rc;
     }
     constexpr int NT = 1024;
-    a.only_flagged = 1;
+    base = a;
+    base.only_flagged = 1;
     const size_t lds = (size_t)a.L * 2 * sizeof(double);
     auto exact_kernel = dag_sweep_exact_kernel<TM, TL, NT>;
     if (lds > 48 * 1024) {
         hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(exact_kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
         if (e != hipSuccess) { set_error("dag_loss_fwd: cannot reserve %zu bytes of LDS: %s", lds, hipGetErrorString(e)); return DAGX_ERR_LAUNCH; }
     }
-    hipLaunchKernelGGL(exact_kernel, dim3(a.B, a.loss_dir ? 2 : 1), dim3(NT), lds, st, a);
+    hipLaunchKernelGGL(exact_kernel, dim3(a.B, a.loss_dir ? 2 : 1), dim3(NT), lds, st, base);
     return check_launch("dag_sweep_exact");
 }
 

@@ -52,6 +52,39 @@ def test_edges_of_blocks_chunks_and_windows(B, L, T, translen, dtype, wide):
     assert_close(gl.float(), rgl, RTOL[dtype], "grad_links")
 
 
+@pytest.mark.parametrize("wide", [False, True])
+@pytest.mark.parametrize("B,L,T,shortest,dtype", [
+    # samples of some lengths get more workgroups than those of others; full lengths find no room (20, 24) or do (3, 16)
+    (3, 650, 24, 1, F32), (16, 760, 24, 570, F32), (16, 768, 21, 768, F16), (20, 760, 24, 760, F32), (20, 765, 24, 400, BF16),
+    (24, 768, 24, 768, F32), (5, 1024, 98, 700, F32), (64, 390, 12, 1, F16)])
+def test_batches_whose_samples_get_different_numbers_of_workgroups(B, L, T, shortest, dtype, wide):
+    match, links_sq, ol, tl = random_problem(L + B, B, L, T, dtype=F32, ragged=False)
+    ol = torch.randint(shortest, L + 1, (B,), generator=torch.Generator().manual_seed(B))
+    ol[0] = L
+    tl = torch.minimum(tl, ol)
+    if B > 4:
+        ol[2], tl[3] = 0, T + 1          # samples without a length, among the others
+    cols = torch.arange(L).view(1, 1, L) < ol.view(B, 1, 1)
+    links_sq = torch.log_softmax(links_sq.masked_fill(~cols, -1e30), -1).masked_fill(~cols | ~torch.isfinite(links_sq), float("-inf"))
+    match, links = match.to(dtype), tn.extract_valid_links(links_sq).to(dtype)
+    good = (ol >= 1) & (tl <= T) & (tl <= ol)
+    g = torch.linspace(0.5, 2.0, B)
+    rloss, rgm, rgl = oracle_loss_and_grads(match[good], links[good], ol[good], tl[good], g[good])
+    before = nat.lib().dagx_loss_float64_first(int(wide))
+    try:
+        for _ in range(2):               # the pipeline words are left as they were found
+            loss, gm, gl = hip_loss_and_grads(match.to(DEV), links.to(DEV), ol, tl, g)
+    finally:
+        nat.lib().dagx_loss_float64_first(before)
+    fin = torch.isfinite(rloss)
+    assert (DagLossFunc.last_sample_flags.cpu()[good][fin] == (2 if wide else 0)).all()
+    assert torch.isneginf(loss[~good]).all() and torch.equal(torch.isfinite(loss[good]), fin)
+    # as above: 6e-7 of a cell and step
+    assert ((loss[good].double() - rloss)[fin].abs() <= 6e-7 * T + 2e-7 * rloss[fin].abs()).all()
+    assert_close(gm.float()[good], rgm, RTOL[dtype], "grad_match")
+    assert_close(gl.float()[good], rgl, RTOL[dtype], "grad_links")
+
+
 @pytest.mark.parametrize("B,L,T,translen,dtype", [
     (1, 2, 2, 1, F32), (3, 2, 2, 1, F16), (2, 5, 5, 1, F32), (1, 63, 5, None, F16), (2, 64, 2, None, F32), (1, 65, 6, 63, BF16),
     (3, 65, 9, 64, F32), (2, 129, 17, 2, F16), (1, 257, 8, None, F32), (2, 320, 9, 128, F16), (1, 321, 33, 63, F32),
