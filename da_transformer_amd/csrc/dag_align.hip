@@ -1052,49 +1052,68 @@ __global__ __launch_bounds__(kTileWaves * kWave) void dag_align_steps_kernel(Ali
 // over a block stages again in front of the next step.  Measured: see launch_align; when it does not pay: see walk_back.
 constexpr int kWalkRows = 48;             // two buffers and the decoder's own 25 KB fit the 160 KB of a CU
 constexpr int kWalkPitch = kBlk + 1;      // the lanes read a column of the transitions: no two in one bank
-struct WalkStage {
+struct alignas(16) WalkStage {
     float e[2 * kBlk * kWalkPitch];       // E[(J-1)*64 + r][J*64 + c] at r * kWalkPitch + c, -inf where there is none
     float a[kWalkRows * 2 * kBlk];        // row r: A[hi - 1 - r] of blocks J - 1 and J
     unsigned src[kWalkRows * kBlk / 4];   // row r: source blocks of (hi - r, block J), a byte each
 };
 constexpr size_t kWalkLds = 2 * sizeof(WalkStage);
 
+// Four neighbouring elements a lane: a CU takes one vector-memory instruction per 26 cycles whatever its width, and with one element
+// a lane a block was 255 of them; now it is 75.  (Backtrack at B=64 L=512 T=64 24 -> 22.4 us, with the walker's priority; at
+// B=16 L=1024 T=256, where a block of nodes is sixteen steps, the steps bound it: 65 us before and after.)
 template <typename TL, int NT>
 __device__ __forceinline__ void stage_walk(WalkStage &w, const float *A, const unsigned char *srcblk, int spitch, const TL *links,
                                            int L, int translen, int J, int hi) {
-    constexpr int kHelpers = NT - kWave;
+    constexpr int kHelpers = NT - kWave, kQuads = kBlk / 4;
     const int q = (int)threadIdx.x - kWave;
-    constexpr int kE = (2 * kBlk * kBlk + kHelpers - 1) / kHelpers, kA = (kWalkRows * 2 * kBlk + kHelpers - 1) / kHelpers;
-    constexpr int kS = (kWalkRows * kBlk / 4 + kHelpers - 1) / kHelpers;
-    TL ve[kE];
-    float va[kA];
-    unsigned vs[kS];
-    bool in[kE];
+    typedef typename Quad<TL>::V V;
+    typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
+    constexpr int kEQuads = 2 * kBlk * kQuads, kAQuads = kWalkRows * 2 * kQuads, kSQuads = kWalkRows * kBlk / 16;
+    constexpr int kE = (kEQuads + kHelpers - 1) / kHelpers, kA = (kAQuads + kHelpers - 1) / kHelpers;
+    static_assert(kSQuads <= kHelpers, "one load of source blocks a thread");
+    V ve[kE];
+    f32x4 va[kA];
+    u32x4 vs;
+    const int64_t most = (int64_t)L * translen - 4;   // (walk_back: at least 0)
+    // element k of quad u is at place at_e[u] + k of the sample's links, its distance is d_e[u] + k; it is one for k < end_e[u]
+    int64_t at_e[kE];
+    int d_e[kE], end_e[kE];
 #pragma unroll
     for (int u = 0; u < kE; ++u) {   // everything is requested before anything is stored
-        const int x = q + u * kHelpers, i = (J - 1) * kBlk + x / kBlk, j = J * kBlk + x % kBlk, d = j - i - 1;
-        in[u] = x < 2 * kBlk * kBlk && i >= 0 && j < L && d >= 0 && d < translen;
-        ve[u] = links[in[u] ? (int64_t)i * translen + d : 0];
+        const int x = q + u * kHelpers, i = (J - 1) * kBlk + x / kQuads, j = J * kBlk + 4 * (x % kQuads);
+        d_e[u] = j - i - 1;
+        at_e[u] = (int64_t)i * translen + d_e[u];
+        end_e[u] = i >= 0 && x < kEQuads ? min(L - j, translen - d_e[u]) : 0;
+        // (a load that would leave the sample is moved inside; its elements, at an end of the sample, are read one by one below)
+        const int64_t at = at_e[u] < 0 ? 0 : at_e[u] > most ? most : at_e[u];
+        __builtin_memcpy(&ve[u], links + at, sizeof(V));
     }
 #pragma unroll
-    for (int u = 0; u < kA; ++u) {
-        const int x = q + u * kHelpers, row = hi - 1 - x / (2 * kBlk), i = (J - 1) * kBlk + x % (2 * kBlk);
-        va[u] = A[row >= 0 && i >= 0 && i < L && x < kWalkRows * 2 * kBlk ? (int64_t)row * L + i : 0];
+    for (int u = 0; u < kA; ++u) {   // (up to three elements past a row's end: row + 1 <= hi is a row of the table)
+        const int x = q + u * kHelpers, row = hi - 1 - x / (2 * kQuads), i = (J - 1) * kBlk + 4 * (x % (2 * kQuads));
+        __builtin_memcpy(&va[u], A + (row >= 0 && i >= 0 && i < L && x < kAQuads ? (int64_t)row * L + i : 0), sizeof(f32x4));
     }
-#pragma unroll
-    for (int u = 0; u < kS; ++u) {
-        const int x = q + u * kHelpers, row = hi - x / (kBlk / 4), at = J * kBlk + (x % (kBlk / 4)) * 4;
-        vs[u] = *reinterpret_cast<const unsigned *>(srcblk + (row >= 1 && at < spitch && x < kWalkRows * kBlk / 4 ? (int64_t)row * spitch + at : 0));
+    {
+        const int row = hi - q / (kBlk / 16), at = J * kBlk + 16 * (q % (kBlk / 16));   // (rows are padded to 16 bytes)
+        vs = *reinterpret_cast<const u32x4 *>(srcblk + (q < kSQuads && row >= 1 && at < spitch ? (int64_t)row * spitch + at : 0));
     }
 #pragma unroll
     for (int u = 0; u < kE; ++u) {
         const int x = q + u * kHelpers;
-        if (x < 2 * kBlk * kBlk) w.e[(x / kBlk) * kWalkPitch + x % kBlk] = in[u] ? to_float(ve[u]) : DAGX_NEG_INF;
+        if (x >= kEQuads) continue;
+        float *const to = &w.e[(x / kQuads) * kWalkPitch + 4 * (x % kQuads)];
+        if (__builtin_expect(at_e[u] >= 0 && at_e[u] <= most, 1)) {
+#pragma unroll
+            for (int k = 0; k < 4; ++k) to[k] = d_e[u] + k >= 0 && k < end_e[u] ? Quad<TL>::get(ve[u], k) : DAGX_NEG_INF;
+        } else {
+#pragma unroll
+            for (int k = 0; k < 4; ++k) to[k] = d_e[u] + k >= 0 && k < end_e[u] ? to_float(links[at_e[u] + k]) : DAGX_NEG_INF;
+        }
     }
 #pragma unroll
-    for (int u = 0; u < kA; ++u) { const int x = q + u * kHelpers; if (x < kWalkRows * 2 * kBlk) w.a[x] = va[u]; }
-#pragma unroll
-    for (int u = 0; u < kS; ++u) { const int x = q + u * kHelpers; if (x < kWalkRows * kBlk / 4) w.src[x] = vs[u]; }
+    for (int u = 0; u < kA; ++u) { const int x = q + u * kHelpers; if (x < kAQuads) *reinterpret_cast<f32x4 *>(&w.a[4 * x]) = va[u]; }
+    if (q < kSQuads) *reinterpret_cast<u32x4 *>(&w.src[4 * q]) = vs;
 }
 
 // The walk with every step read from memory, by one wave, without LDS: the row of source blocks of the next step is fetched
@@ -1152,6 +1171,7 @@ __device__ __forceinline__ void walk_back_staged(const float *A, const unsigned 
         if (!walker) {
             if (J > 0 && next_hi > stop) stage_walk<TL, NT>(lds[cur ^ 1], A, srcblk, spitch, links, L, translen, J - 1, next_hi);
         } else {
+            __builtin_amdgcn_s_setprio(3);   // (three of the other waves share its SIMD)
             const WalkStage &w = lds[cur];
             const unsigned char *src = reinterpret_cast<const unsigned char *>(w.src) + (hi - s) * kBlk;
             const float *arow = w.a + (hi - s) * 2 * kBlk + lane, *ecol = w.e + lane * kWalkPitch;
@@ -1209,7 +1229,7 @@ constexpr int kWalkStepsPerBlock = 4;
 template <typename TL, int NT, bool ZERO_FOR_DEAD, bool STAGED, typename PUT>
 __device__ __forceinline__ void walk_back(const float *A, const unsigned char *srcblk, int spitch, const TL *links, int L,
                                           int translen, int s, int j, int stop, WalkStage *lds, PUT put) {
-    if (STAGED && s - stop >= kWalkStepsPerBlock * (j / kBlk + 1))
+    if (STAGED && L >= 4 && s - stop >= kWalkStepsPerBlock * (j / kBlk + 1))   // (four elements a load)
         walk_back_staged<TL, NT, ZERO_FOR_DEAD>(A, srcblk, spitch, links, L, translen, s, j, stop, lds, put);
     else if (threadIdx.x < kWave)
         walk_back_in_memory<TL, ZERO_FOR_DEAD>(A, srcblk, spitch, links, L, translen, s, j, stop, put);
@@ -1221,7 +1241,7 @@ constexpr int kOneGroupThreads = 1024;
 template <typename TM, typename TL, bool TRACE_LDS, bool STAGED>
 __global__ __launch_bounds__(kOneGroupThreads) void dag_backtrack_kernel(
     const float *__restrict__ table, const unsigned char *__restrict__ srcblk_all, const int *__restrict__ flags, AlignArgs a) {
-    extern __shared__ float lds_a[];
+    extern __shared__ __align__(16) float lds_a[];
     const int b = blockIdx.x;
     if (flags[b]) {
         align_one_sample<TM, TL, kOneGroupThreads, TRACE_LDS>(a, b, lds_a);
@@ -1507,7 +1527,7 @@ struct DecodeArgs {
 // One workgroup per sample: the best node of every step, the best length, the walk back (walk_back) and the tokens.
 template <typename TL, bool STAGED>
 __global__ __launch_bounds__(kDecodeThreads) void viterbi_select_kernel(DecodeArgs a) {
-    extern __shared__ float lds_walk[];
+    extern __shared__ __align__(16) float lds_walk[];
     __shared__ int s_star;
     __shared__ float sbest[kDecodeMaxSteps];
     __shared__ int sidx[kDecodeMaxSteps];
