@@ -96,8 +96,13 @@ def dag_viterbi_decode(links, output_logits_normalized, output_length, decode_up
     links = links.contiguous()
     output_length = output_length.contiguous()
     # the reference's penalty tensor, computed the same way on the host
-    penalty = ((torch.arange(max_length) + 1) ** decode_viterbibeta).to(torch.float32).to(links.device)
+    penalty = ((torch.arange(max_length) + 1) ** decode_viterbibeta).to(torch.float32)
     with nat.on_device(links.device):
+        # (out of pinned memory: from pageable memory the host waits for the copy, which stands behind what the stream still
+        #  has to do, and enqueues the sweep only then)
+        if penalty.device.type == "cpu":
+            penalty = penalty.pin_memory()
+        penalty = penalty.to(links.device, non_blocking=True)
         both, nodes, out_tokens, out_count = _outputs(bsz, max_length, links.device)
         pred_length = torch.empty(bsz, dtype=torch.int64, device=links.device)
         nbytes = nat.workspace_bytes(nat.OP_VITERBI_DECODE, bsz, max_length, prelen, translen)
