@@ -1312,7 +1312,10 @@ static int prepare_align_chunks() {
 }
 template <typename TM, typename TL, int SPACING>
 static int launch_align_chunks(AlignTileArgs &ta, const char *who, hipStream_t st) {
-    static const ChunkCosts costs[1] = {{SPACING == 1 ? 62 : 36, 27, 4, 75}};   // (measured)
+    // Found by timing calls under some twenty sets, from the pieces' own times {62 or 36, 27, 4, 75} on (us): B = 64, L = 512, T = 64
+    // 120.3 -> 116.6, B = 16, L = 768, T = 192 276.5 -> 268, B = 4, L = 700, T = 110 187 -> 179, B = 64, L = 256, T = 64
+    // (SPACING 2) 79.0 -> 76.1, B = 40, L = 400, T = 60 (SPACING 2) 99.5 -> 95.2; the others the same.
+    static const ChunkCosts costs[1] = {SPACING == 1 ? ChunkCosts{62, 27, 2, 65} : ChunkCosts{36, 27, 4, 55}};
     ta.plan = chunk_plan<SPACING>(ta.translen, ta.C, costs);
     if (int rc = prepare_align_chunks<TM, TL, SPACING>()) return rc;
     hipLaunchKernelGGL((dag_align_chunks_kernel<TM, TL, SPACING>), dim3(((ta.B + 7) & ~7) * ta.C), dim3(kTileWaves * kWave), kChunkLdsBytes, st, ta);
