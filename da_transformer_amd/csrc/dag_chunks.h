@@ -238,6 +238,32 @@ struct TableChoice {
     unsigned long long ngroups[kMostTables];   // (tables 1 ..) four bits for each number of blocks from 1 on: a sample's groups
     int ntable, least, most;                   // most: the most groups of any sample in any table
 };
+// Groups of a sample of nb blocks that keeps `bound` with as few as can be, at most c: the plan they are from and their number.
+template <int SPACING, int N>
+inline const ChunkPlan<N> &plan_for_bound(int translen, int c, int nb, int bound, const ChunkCosts (&costs)[N], int which, int &n) {
+    int u = 1;
+    while (u < c && chunk_plan<SPACING>(translen, u, costs).busiest[which][nb] > bound) ++u;
+    const ChunkPlan<N> &plan = chunk_plan<SPACING>(translen, u, costs);
+    for (n = 0; n < u && plan.gtab[which][nb][n + 1] > plan.gtab[which][nb][n];) ++n;
+    return plan;
+}
+// Whether two sweeps of samples of seven eighths of L, with the bound that the longest keeps with c groups, would all find a CU.
+template <int SPACING, int N>
+inline bool typical_fits(int B, int L, int translen, int c, const ChunkCosts (&costs)[N], int which) {
+    int n;
+    plan_for_bound<SPACING>(translen, c, (7 * L / 8 + kBlk - 1) / kBlk, chunk_plan<SPACING>(translen, c, costs).busiest[which][(L + kBlk - 1) / kBlk], costs, which, n);
+    return 2 * B * n <= kSweepCus;
+}
+inline bool may_choose(int B, int L) { return B <= kMostForTables && L > 4 * kBlk; }
+// The most groups that any table for this batch can have, whatever T and the costs: what a workspace is laid out for.
+template <int SPACING, int N>
+inline int most_groups(int B, int L, int translen, int least, const ChunkCosts (&costs)[N]) {
+    int most = least;
+    if (least > 0 && may_choose(B, L))
+        for (int which = 0; which < N; ++which)
+            for (int c = most + 1; c <= kMaxGroups; ++c) if (typical_fits<SPACING>(B, L, translen, c, costs, which)) most = c;
+    return most;
+}
 // A table is offered where the longest sample's stages (one a chunk, one a block, one and a half a hand-over) take at most 97 %
 // of what they take in `least` groups (L = 512, T = 170 in four groups, 97 to 99 % depending on T, 156 to 160 us for 156), and
 // where two sweeps of samples of seven eighths of L would all find a CU.
@@ -251,7 +277,7 @@ inline void make_tables(GroupTable (&tables)[kMostTables], TableChoice &o, int B
     o.least = o.most = least;
     const int NB = (L + kBlk - 1) / kBlk, NC = (T - 1 + kChunk - 1) / kChunk;
     for (int nb = 0; nb <= kMaxBlocksFast; ++nb) copy_row(tables[0], nb, plan_of(least));
-    if (B > kMostForTables || NB <= 4) return;
+    if (!may_choose(B, L)) return;
     auto stages2 = [&](const int c) { return 2 * (NC + NB) + 3 * (c - 1); };
     int best = plan_of(least).busiest[which][NB];
     const long long now = (long long)best * stages2(least);
@@ -261,18 +287,14 @@ inline void make_tables(GroupTable (&tables)[kMostTables], TableChoice &o, int B
         GroupTable &table = tables[o.ntable];
         unsigned long long ngroups = 0;
         int most = 1;
+        if (!typical_fits<SPACING>(B, L, translen, c, costs, which)) continue;
         for (int nb = 0; nb <= kMaxBlocksFast; ++nb) {
-            int u = nb >= 1 && nb <= NB ? 1 : c, n = 0;
-            while (u < c && plan_of(u).busiest[which][nb] > bound) ++u;
-            const ChunkPlan<N> &plan = plan_of(u);
-            copy_row(table, nb, plan);
-            if (nb < 1 || nb > NB) continue;
-            while (n < u && plan.gtab[which][nb][n + 1] > plan.gtab[which][nb][n]) ++n;
+            if (nb < 1 || nb > NB) { copy_row(table, nb, plan_of(c)); continue; }
+            int n;
+            copy_row(table, nb, plan_for_bound<SPACING>(translen, c, nb, bound, costs, which, n));
             ngroups |= (unsigned long long)n << (4 * (nb - 1));
             most = n > most ? n : most;
         }
-        const int typical = (int)(ngroups >> (4 * ((7 * L / 8 + kBlk - 1) / kBlk - 1))) & 15;
-        if (2 * B * typical > kSweepCus) break;
         o.ngroups[o.ntable++] = ngroups;
         o.most = most > o.most ? most : o.most;
         best = bound;

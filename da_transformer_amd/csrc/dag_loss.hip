@@ -919,27 +919,32 @@ __global__ __launch_bounds__(kTileWaves * kWave) void dag_sweep_tiles_kernel(Til
     // The wide launch behind a float32 launch that flagged nothing (the usual case) ends here, after one load: the
     // float32 launch counts the samples it flags in word 2 of the pipeline words, the wide launch clears it.
     if constexpr (WIDE) { if (a.sync[2] == 0) return; }
-    const int B8 = (a.B + 7) & ~7;
+    // (all that the ticket waits for in one round trip to the argument block)
+    int *sync = a.sync;
+    int ntable = a.choice.ntable, least = a.choice.least, B = a.B, ndir = a.ndir;
+    asm volatile("" : "+s"(sync), "+s"(ntable), "+s"(least), "+s"(B), "+s"(ndir));
+    const int B8 = (B + 7) & ~7;
     // Which table, and with it how many workgroups take part: all of them come to the same answer from the lengths alone.  The
     // others leave at once; they are the last of the grid, so they cost a CU that has become free a look at the lengths.
-    int mine = 0, used = 0, workgroups = a.ndir * B8 * a.choice.least;   // (lane <-> sample) groups of a sample, table
-    if (a.choice.ntable > 1) {
+    int mine = 0, used = 0, workgroups = ndir * B8 * least;   // (lane <-> sample) groups of a sample, table
+    if (__builtin_expect(ntable > 1, 0)) {   // (unlikely: out of the way of batches without a choice, which else wait for these instructions:
+                                             //  scoring at B = 40, L = 328 58.6 us for 57.5)
         const int lane = tid & (kWave - 1);
-        const int64_t len = a.out_len[lane < a.B ? lane : 0];
+        const int64_t len = a.out_len[lane < B ? lane : 0];
         const int nb = len >= 1 && len <= a.L ? ((int)len + kBlk - 1) / kBlk : 1;
-        for (int x = a.choice.ntable - 1; x > 0 && used == 0; --x) {
-            const int n = lane < a.B ? (int)(a.choice.ngroups[x] >> (4 * (nb - 1))) & 15 : 0;
+        for (int x = ntable - 1; x > 0 && used == 0; --x) {
+            const int n = lane < B ? (int)(a.choice.ngroups[x] >> (4 * (nb - 1))) & 15 : 0;
             int all = n;
 #pragma unroll
             for (int d = 32; d > 0; d >>= 1) all += __shfl_xor(all, d, kWave);
-            all = __builtin_amdgcn_readfirstlane(all) * a.ndir;
+            all = __builtin_amdgcn_readfirstlane(all) * ndir;
             if (all <= kSweepCus) { mine = n; used = x; workgroups = all; }
         }
         used = __builtin_amdgcn_readfirstlane(used);
         workgroups = __builtin_amdgcn_readfirstlane(workgroups);
         if ((int)blockIdx.x >= workgroups) return;
     }
-    if (tid == 0) { s_ticket = atomicAdd(a.sync, 1); s_abort = 0; }
+    if (tid == 0) { s_ticket = atomicAdd(sync, 1); s_abort = 0; }
     __syncthreads();
     // ticket -> (group, sweep, sample): first group 0 of every sweep of every sample, then every group 1, and so on.
     // Every group waits only on groups with a smaller ticket, so a waiting workgroup's producers have already
@@ -947,25 +952,26 @@ __global__ __launch_bounds__(kTileWaves * kWave) void dag_sweep_tiles_kernel(Til
     // are consumers, which could not start any sooner than their producers' first rows anyway.  The two sweeps of a
     // sample are 8 tickets apart, the workgroups of a sample a multiple of 8 (table 0): they share an XCD and its L2.
     const int k = __builtin_amdgcn_readfirstlane(s_ticket);
-    int g, b_k, slot_k, groups = a.choice.least;
+    int g, b_k, slot_k, groups = least;
     bool has_sample;
-    if (used == 0) {
-        const int runs = a.ndir * (B8 / 8);   // runs of eight (sweep, sample) pairs
+    if (__builtin_expect(used == 0, 1)) {
+        const int runs = ndir * (B8 / 8);   // runs of eight (sweep, sample) pairs
         const int run = (k / 8) % runs;
-        g = k / (8 * runs); slot_k = run % a.ndir;
-        b_k = (run / a.ndir) * 8 + (k % 8);
-        has_sample = g < a.choice.least && b_k < a.B;
+        g = k / (8 * runs); slot_k = run % ndir;
+        b_k = (run / ndir) * 8 + (k % 8);
+        has_sample = g < least && b_k < B;
     } else {   // samples without a group g are passed over; k < workgroups, so there is a (group, sweep, sample) for it
         int r = k, n = 0;
         unsigned long long have = 0;
+#pragma unroll 1
         for (g = 0; g < C; ++g) {
             have = __builtin_amdgcn_ballot_w64(mine > g);
             n = __builtin_popcountll(have);
-            if (r < a.ndir * n) break;
-            r -= a.ndir * n;
+            if (r < ndir * n) break;
+            r -= ndir * n;
         }
         int rank;
-        place_of_ticket(r, n, a.ndir, rank, slot_k);
+        place_of_ticket(r, n, ndir, rank, slot_k);
         const int lane = tid & (kWave - 1);
         const int before = __builtin_popcountll(have & ((1ull << lane) - 1));
         const unsigned long long at = __builtin_amdgcn_ballot_w64((have >> lane & 1) != 0 && before == rank);
@@ -1620,18 +1626,19 @@ static int sweep_groups(int B, int L, int translen) {
     const int C = groups_needed(L, translen, 4), sweeps = 2 * ((B + 7) & ~7);
     return (long long)sweeps * C <= kSweepCus && C > 0 ? C : groups_needed(L, translen, kChunkBlocks);
 }
-// The most groups a launch may have (the workspace is laid out for them, whatever T).
-static int most_groups(int B, int L, int translen) {
-    const int C = sweep_groups(B, L, translen);
-    return C > 0 && B <= kMostForTables ? kMaxGroups : C;
-}
+// float32, float64.  Found by timing the sweeps themselves under some forty sets (us; first the costs of each piece timed alone,
+// with a SIMD taking the sum of its two waves' work, {45, 7, 4, 100} and {85, 17, 11, 100}; then these): float32 B = 64, L = 512, T = 64
+// 107 -> 95; B = 16, L = 1024, T = 256 347 -> 329; B = 16, L = 512, T = 128 134 -> 127; B = 8, L = 1024, T = 256 334 -> 302; float64 at the
+// first of them 151 -> 141.  A fetched block waits for the rows of its producer and for LDS twice, so it keeps its wave for longer than
+// its instructions take; and while a wave waits, the other wave of its SIMD works.
+static const ChunkCosts kSweepCosts[2] = {{45, 9, 12, 70}, {85, 25, 16, 80}};
 
 // ticket + progress words (rounded to 8 bytes), then the fast kernel's two read-outs per sample
 static size_t sweep_bytes(int B, int C) { return sweep_sync_ints(B, C) * sizeof(int) + (size_t)2 * B * sizeof(double); }
 
 size_t loss_fwd_workspace_bytes(int B, int T, int L, int translen) {
     (void)T;
-    const int C = most_groups(B, L, translen);
+    const int C = most_groups<1>(B, L, translen, sweep_groups(B, L, translen), kSweepCosts);
     return C > 0 ? sweep_bytes(B, C) : 0;
 }
 
@@ -1663,13 +1670,6 @@ static int prepare_tiles_kernels_of() {
     if (!rc) rc = prepare_tiles_kernel<TM, bf16_t, true>();
     return rc;
 }
-
-// float32, float64.  Found by timing the sweeps themselves under some forty sets (us; first the costs of each piece timed alone,
-// with a SIMD taking the sum of its two waves' work, {45, 7, 4, 100} and {85, 17, 11, 100}; then these): float32 B = 64, L = 512, T = 64
-// 107 -> 95; B = 16, L = 1024, T = 256 347 -> 329; B = 16, L = 512, T = 128 134 -> 127; B = 8, L = 1024, T = 256 334 -> 302; float64 at the
-// first of them 151 -> 141.  A fetched block waits for the rows of its producer and for LDS twice, so it keeps its wave for longer than
-// its instructions take; and while a wave waits, the other wave of its SIMD works.
-static const ChunkCosts kSweepCosts[2] = {{45, 9, 12, 70}, {85, 25, 16, 80}};
 
 template <typename TM, typename TL>
 static int launch_sweeps(SweepArgs base, hipStream_t st) {
