@@ -1223,7 +1223,7 @@ __device__ __forceinline__ void walk_back_staged(const float *A, const unsigned 
 }
 
 // STAGED: lds holds kWalkLds bytes.  A path with few steps a block, as Viterbi decoding finds where no transition stands out,
-// walks in memory all the same: a block staged costs as much as about four steps from memory (2.3 and 0.6 us; Viterbi decoding
+// walks in memory all the same: a block staged cost as much as about four steps from memory (2.3 and 0.6 us, with one element a load; Viterbi decoding
 // at B=64, paths of 13 nodes: L=512 staged 229 us, in memory 221; L=1024 982 and 967).
 constexpr int kWalkStepsPerBlock = 4;
 template <typename TL, int NT, bool ZERO_FOR_DEAD, bool STAGED, typename PUT>
@@ -1374,7 +1374,7 @@ static int launch_align(AlignArgs a, void *workspace, hipStream_t st) {
         if (rc) return rc;
         if ((rc = launch_align_sweep<TM, TL>(ta, "dag_align_sweep", st))) return rc;
         // the backtrack, and the samples that the pipeline gave up on.  (float32, kernel time: walked in memory 39.5 us at
-        // B=64 L=512 T=64 and 172 us at B=16 L=1024 T=256, out of LDS 27.6 and 62.5 us.)
+        // B=64 L=512 T=64 and 172 us at B=16 L=1024 T=256, out of LDS 22.4 and 65 us.)
         const bool in_lds = trace_fits_lds(a.T, a.L);
         const size_t redo_lds = (size_t)a.L * 8 + (in_lds ? (size_t)a.T * a.L * 2 : (size_t)0);
         const bool staged = staged_alignment(a.B, a.L);
