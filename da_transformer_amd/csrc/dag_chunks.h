@@ -255,20 +255,13 @@ inline bool typical_fits(int B, int L, int translen, int c, const ChunkCosts (&c
     return 2 * B * n <= kSweepCus;
 }
 inline bool may_choose(int B, int L) { return B <= kMostForTables && L > 4 * kBlk; }
-// The most groups that any table for this batch can have, whatever T and the costs: what a workspace is laid out for.
-template <int SPACING, int N>
-inline int most_groups(int B, int L, int translen, int least, const ChunkCosts (&costs)[N]) {
-    int most = least;
-    if (least > 0 && may_choose(B, L))
-        for (int which = 0; which < N; ++which)
-            for (int c = most + 1; c <= kMaxGroups; ++c) if (typical_fits<SPACING>(B, L, translen, c, costs, which)) most = c;
-    return most;
-}
 // A table is offered where the longest sample's stages (one a chunk, one a block, one and a half a hand-over) take at most 97 %
 // of what they take in `least` groups (L = 512, T = 170 in four groups, 97 to 99 % depending on T, 156 to 160 us for 156), and
-// where two sweeps of samples of seven eighths of L would all find a CU.
+// where two sweeps of samples of seven eighths of L would all find a CU.  room: the most groups a sweep that the caller's workspace has
+// pipeline words for; with `least` there is only table 0.
 template <int SPACING, int N>
-inline void make_tables(GroupTable (&tables)[kMostTables], TableChoice &o, int B, int T, int L, int translen, int least, const ChunkCosts (&costs)[N], int which) {
+inline void make_tables(GroupTable (&tables)[kMostTables], TableChoice &o, int B, int T, int L, int translen, int least, int room,
+                        const ChunkCosts (&costs)[N], int which) {
     auto plan_of = [&](const int c) -> const ChunkPlan<N> & { return chunk_plan<SPACING>(translen, c, costs); };
     auto copy_row = [&](GroupTable &table, const int nb, const ChunkPlan<N> &plan) {
         for (int q = 0; q < 12; ++q) { table.gtab[nb][q] = plan.gtab[which][nb][q]; table.deal[nb][q] = plan.deal[which][nb][q]; }
@@ -277,7 +270,7 @@ inline void make_tables(GroupTable (&tables)[kMostTables], TableChoice &o, int B
     o.least = o.most = least;
     const int NB = (L + kBlk - 1) / kBlk, NC = (T - 1 + kChunk - 1) / kChunk;
     for (int nb = 0; nb <= kMaxBlocksFast; ++nb) copy_row(tables[0], nb, plan_of(least));
-    if (!may_choose(B, L)) return;
+    if (!may_choose(B, L) || room <= least) return;
     auto stages2 = [&](const int c) { return 2 * (NC + NB) + 3 * (c - 1); };
     int best = plan_of(least).busiest[which][NB];
     const long long now = (long long)best * stages2(least);
@@ -295,6 +288,7 @@ inline void make_tables(GroupTable (&tables)[kMostTables], TableChoice &o, int B
             ngroups |= (unsigned long long)n << (4 * (nb - 1));
             most = n > most ? n : most;
         }
+        if (most > room) continue;
         o.ngroups[o.ntable++] = ngroups;
         o.most = most > o.most ? most : o.most;
         best = bound;

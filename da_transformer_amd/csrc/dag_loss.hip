@@ -1636,10 +1636,17 @@ static const ChunkCosts kSweepCosts[2] = {{45, 9, 12, 70}, {85, 25, 16, 80}};
 // ticket + progress words (rounded to 8 bytes), then the fast kernel's two read-outs per sample
 static size_t sweep_bytes(int B, int C) { return sweep_sync_ints(B, C) * sizeof(int) + (size_t)2 * B * sizeof(double); }
 
+// For table 0.  Tables with more groups are used where the caller's workspace has room for them: a buffer that is large enough for the
+// largest graph must stay large enough for smaller ones, whose tables may have more groups.
 size_t loss_fwd_workspace_bytes(int B, int T, int L, int translen) {
     (void)T;
-    const int C = most_groups<1>(B, L, translen, sweep_groups(B, L, translen), kSweepCosts);
+    const int C = sweep_groups(B, L, translen);
     return C > 0 ? sweep_bytes(B, C) : 0;
+}
+static int groups_that_fit(int B, size_t workspace_bytes) {
+    int C = kMaxGroups;
+    while (C > 0 && sweep_bytes(B, C) > workspace_bytes) --C;
+    return C;
 }
 
 size_t loss_bwd_workspace_bytes(int B) { (void)B; return 0; }
@@ -1672,7 +1679,7 @@ static int prepare_tiles_kernels_of() {
 }
 
 template <typename TM, typename TL>
-static int launch_sweeps(SweepArgs base, hipStream_t st) {
+static int launch_sweeps(SweepArgs base, size_t workspace_bytes, hipStream_t st) {
     TileSweepArgs a{};
     static_cast<SweepArgs &>(a) = base;
     int C = force_exact() ? 0 : sweep_groups(a.B, a.L, a.translen);
@@ -1693,9 +1700,9 @@ static int launch_sweeps(SweepArgs base, hipStream_t st) {
         a.ndir = 2;
         a.rev[0] = 0; a.rev[1] = a.loss_dir ? 1 : 0;
         a.upper[0] = a.loss_dir ? 1 : 0; a.upper[1] = a.loss_dir ? 0 : 1;
-        const int B8 = (a.B + 7) & ~7;
+        const int B8 = (a.B + 7) & ~7, room = groups_that_fit(a.B, workspace_bytes);
         auto plan_for = [&](const bool wide) {
-            make_tables<1>(a.table, a.choice, a.B, a.T, a.L, a.translen, C, kSweepCosts, wide);
+            make_tables<1>(a.table, a.choice, a.B, a.T, a.L, a.translen, C, room, kSweepCosts, wide);
             a.C = a.choice.most;
             a.zfast = reinterpret_cast<double *>(a.sync + sweep_sync_ints(a.B, a.C));   // (zero again behind every launch, as the words in front)
         };
@@ -1730,11 +1737,11 @@ static int launch_sweeps(SweepArgs base, hipStream_t st) {
 }
 
 template <typename TM>
-static int dispatch_links(int ldt, const SweepArgs &a, hipStream_t st) {
+static int dispatch_links(int ldt, const SweepArgs &a, size_t workspace_bytes, hipStream_t st) {
     switch (ldt) {
-        case DAGX_F32: return launch_sweeps<TM, float>(a, st);
-        case DAGX_F16: return launch_sweeps<TM, __half>(a, st);
-        default: return launch_sweeps<TM, bf16_t>(a, st);
+        case DAGX_F32: return launch_sweeps<TM, float>(a, workspace_bytes, st);
+        case DAGX_F16: return launch_sweeps<TM, __half>(a, workspace_bytes, st);
+        default: return launch_sweeps<TM, bf16_t>(a, workspace_bytes, st);
     }
 }
 
@@ -1825,9 +1832,9 @@ static int loss_fwd_impl(const void *match, int match_dtype, const int64_t match
     a.logz = logz; a.loss = loss; a.loss_dir = require_gradient ? 1 : 0; a.flags = sample_flags; a.sync = static_cast<int *>(workspace);
     hipStream_t st = static_cast<hipStream_t>(stream);
     switch (match_dtype) {
-        case DAGX_F32: return dispatch_links<float>(links_dtype, a, st);
-        case DAGX_F16: return dispatch_links<__half>(links_dtype, a, st);
-        default: return dispatch_links<bf16_t>(links_dtype, a, st);
+        case DAGX_F32: return dispatch_links<float>(links_dtype, a, workspace_bytes, st);
+        case DAGX_F16: return dispatch_links<__half>(links_dtype, a, workspace_bytes, st);
+        default: return dispatch_links<bf16_t>(links_dtype, a, workspace_bytes, st);
     }
 }
 

@@ -37,6 +37,9 @@ def get_dag_kernel():
 
 
 _clean_workspaces = {}
+# Enough for every batch of up to 64 samples with as many workgroups as the sweeps may choose, and for larger batches of short
+# graphs: a buffer is not replaced (a captured graph may point at it) because a batch of smaller graphs has more workgroups.
+_SMALLEST_WORKSPACE = 8192
 
 
 def _clean_workspace(dev, nbytes):
@@ -45,7 +48,7 @@ def _clean_workspace(dev, nbytes):
     key = (dev.index, nat.raw_stream(dev.index))
     ws = _clean_workspaces.get(key)
     if ws is None or ws.numel() < nbytes:
-        ws = torch.zeros(max(nbytes, 8), dtype=torch.uint8, device=dev)
+        ws = torch.zeros(max(nbytes, _SMALLEST_WORKSPACE), dtype=torch.uint8, device=dev)
         _clean_workspaces[key] = ws
     return ws
 
@@ -117,7 +120,7 @@ class DagLossFunc(Function):
                     nat.ptr(match_all), nat.dtype_code(match_all), nat.strides3(match_all),
                     nat.ptr(links), nat.dtype_code(links), nat.ptr(output_length), nat.ptr(target_length),
                     bsz, tarlen, prelen, translen, hat, hat + 4 * nhat, off, off + 8 * noff,
-                    off + 16 * noff, nat.ptr(loss), nat.ptr(flags), int(need_grad), nat.ptr(ws), nbytes, nat.stream_of(match_all)))
+                    off + 16 * noff, nat.ptr(loss), nat.ptr(flags), int(need_grad), nat.ptr(ws), ws.numel(), nat.stream_of(match_all)))
             except RuntimeError:
                 _forget_workspace(dev)
                 raise

@@ -135,7 +135,9 @@ int dagx_links_bwd(void *content_inout, int dtype, const float *log_gates, const
  * sweeps', 1 the log-domain kernel's (a diagnostic; the tables have one format and the backward does not look).
  *
  * DAG loss forward.
- * workspace: dagx_workspace_bytes(DAGX_OP_LOSS_FWD, ...) bytes, 8-byte aligned.  It MUST BE ZERO-FILLED when it
+ * workspace: workspace_bytes, at least dagx_workspace_bytes(DAGX_OP_LOSS_FWD, ...), 8-byte aligned.  With B <= 64 and more than
+ * 256 nodes a sweep may be divided among more workgroups than that many bytes have words for, which changes the order of sums
+ * and is up to 1.3 times as fast; it is where workspace_bytes are enough, which 8192 always are.  All of it MUST BE ZERO-FILLED when it
  * is first handed to this function (dagx_loss_fwd_init_workspace does that; with garbage in it the result is
  * undefined and nothing detects it); every call leaves it zero-filled again (its kernels clear the words they
  * used), so one buffer, cleared once, serves any number of consecutive calls of any shape.  Calls that overlap
@@ -175,7 +177,7 @@ int dagx_prepare_device(void);
 /*
  * dagx_loss_fwd for callers that cannot allocate device memory (code under HIP graph capture, tight serving
  * loops, harnesses that forbid hipMalloc).  It has no counterpart in the reference.  Same arguments and
- * results as dagx_loss_fwd but for the workspace: the pipeline words live in a device array of 160 KiB that the
+ * results as dagx_loss_fwd with a workspace of at least 8192 bytes, but for the workspace: the pipeline words live in a device array of 160 KiB that the
  * library owns (one copy per GPU, held until the process ends), so the call allocates nothing, frees nothing and calls
  * no allocating routine.  A shape whose dagx_workspace_bytes(DAGX_OP_LOSS_FWD, ...) are at most
  * dagx_loss_fwd_noalloc_max_bytes() = 128 KiB is taken, one with more than 160 KiB refused with DAGX_ERR_UNSUPPORTED.

@@ -28,9 +28,10 @@ int main() {
         const int four = groups_needed(L, W, 4), least = 2 * ((B + 7) & ~7) * four <= 256 && four > 0 ? four : groups_needed(L, W, kChunkBlocks);
         if (least == 0) continue;
         const int which = round & 1, NB = (L + kBlk - 1) / kBlk, blocks = (W + kBlk - 1) / kBlk;
-        make_tables<1>(tables, t, B, T, L, W, least, costs, which);
+        const int room = draw(0, 2) ? kMaxGroups : draw(least, kMaxGroups);   // groups a sweep that the workspace has words for
+        make_tables<1>(tables, t, B, T, L, W, least, room, costs, which);
         if (t.ntable < 1 || t.ntable > kMostTables || t.most < least || t.most > kMaxGroups || t.least != least) return fail("sizes", B, T, L, W, 0);
-        if (t.most > most_groups<1>(B, L, W, least, costs)) return fail("more groups than the workspace has", B, T, L, W, 0);
+        if (t.most > room) return fail("more groups than the workspace has", B, T, L, W, 0);
         offered += t.ntable > 1;
         for (int x = 0; x < t.ntable; ++x)
             for (int nb = 1; nb <= NB; ++nb) {
