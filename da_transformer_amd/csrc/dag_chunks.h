@@ -121,12 +121,12 @@ inline int deal_tiles(int jb0, int nblk, int W, const ChunkCosts &cost, TileDeal
         return load[w] + more > both ? load[w] + more : both;
     };
     auto place = [&](int (&count)[kTileWaves], const bool fetch, const int work) {
-        int best = -1;
+        int best = -1, until = 0;
         for (int w = kTileWaves - 1; w >= 0; --w) {
             const int most = fetch ? (w >= nblk || nblk == kTileWaves ? kForeign : 0) : (w >= nblk ? kTilesPerWave : SPACING);
             if (count[w] >= most) continue;
-            const int now = best < 0 ? 0 : busy(w, work) - busy(best, work);
-            if (best < 0 || now < 0 || (now == 0 && count[w] < count[best])) best = w;
+            const int now = busy(w, work);
+            if (best < 0 || now < until || (now == until && count[w] < count[best])) { best = w; until = now; }
         }
         if (best < 0) return false;
         ++count[best];
@@ -165,31 +165,44 @@ struct ChunkPlan {
     short busiest[N][kMaxBlocksFast + 1];         // how long the busiest SIMD of the graph's groups takes; kNoPlan: C groups do not hold it
 };
 constexpr int kNoPlan = 1 << 12;
+// Every group there can be with a window, whatever the number of groups: group of blocks j .. j + n - 1.
+template <int N>
+struct GroupDeals {
+    short cost[N][kMaxBlocksFast][kChunkBlocks + 1];   // -1: more tiles than a workgroup has room for
+    TileDeal deal[N][kMaxBlocksFast][kChunkBlocks + 1];
+    short most[N];                                     // the greatest of the costs
+};
 template <int SPACING, int N>
-inline void plan_chunks(int W, int C, const ChunkCosts (&costs)[N], ChunkPlan<N> &plan) {
-    constexpr int NB = kMaxBlocksFast;
+inline void deal_groups(int W, const ChunkCosts (&costs)[N], GroupDeals<N> &o) {
     for (int x = 0; x < N; ++x) {
-        int cost[NB][kChunkBlocks + 1];
-        TileDeal deal[NB][kChunkBlocks + 1];
-        for (int j = 0; j < NB; ++j) {
+        o.most[x] = 0;
+        for (int j = 0; j < kMaxBlocksFast; ++j) {
             int tiles = 0;
             for (int n = 1; n <= kChunkBlocks; ++n) {
-                cost[j][n] = -1;
-                if (j + n > NB) continue;
+                o.cost[x][j][n] = -1;
+                o.deal[x][j][n] = TileDeal{0};
+                if (j + n > kMaxBlocksFast) continue;
                 tiles += j + n - tile_ilo(j + n - 1, W);
-                if (tiles <= kTileCap) cost[j][n] = deal_tiles<SPACING>(j, n, W, costs[x], deal[j][n]);
+                if (tiles <= kTileCap) o.cost[x][j][n] = (short)deal_tiles<SPACING>(j, n, W, costs[x], o.deal[x][j][n]);
+                o.most[x] = o.cost[x][j][n] > o.most[x] ? o.cost[x][j][n] : o.most[x];
             }
         }
-        for (int nb = 0; nb <= NB; ++nb) {
-            int low = 0, high = kNoPlan;                 // the least bound on a group's cost that C groups can keep
+    }
+}
+template <int N>
+inline void plan_chunks(const GroupDeals<N> &groups, int C, ChunkPlan<N> &plan) {
+    for (int x = 0; x < N; ++x) {
+        const auto &cost = groups.cost[x];
+        for (int nb = 0; nb <= kMaxBlocksFast; ++nb) {
+            int low = 0, high = groups.most[x] + 1;      // the least bound on a group's cost that C groups can keep
             unsigned char g[16];
             auto split = [&](const int most) {
                 int used = 0, j = 0;
                 g[0] = 0;
                 for (int q = 1; q < 16; ++q) g[q] = (unsigned char)nb;
                 while (j < nb) {
-                    int n = 0;
-                    for (int y = 1; y <= kChunkBlocks && j + y <= nb; ++y) if (cost[j][y] >= 0 && cost[j][y] <= most) n = y;
+                    int n = nb - j < kChunkBlocks ? nb - j : kChunkBlocks;
+                    while (n > 0 && (cost[j][n] < 0 || cost[j][n] > most)) --n;
                     if (n == 0 || used == C) return false;
                     j += n;
                     g[++used] = (unsigned char)j;
@@ -197,26 +210,38 @@ inline void plan_chunks(int W, int C, const ChunkCosts (&costs)[N], ChunkPlan<N>
                 return true;
             };
             while (low < high) { const int mid = (low + high) / 2; if (split(mid)) high = mid; else low = mid + 1; }
-            split(high);
-            plan.busiest[x][nb] = (short)high;
+            plan.busiest[x][nb] = (short)(split(high) ? high : kNoPlan);
             for (int q = 0; q < 12; ++q) {
                 plan.gtab[x][nb][q] = g[q];
-                plan.deal[x][nb][q] = q < C && g[q + 1] > g[q] && g[q + 1] - g[q] <= kChunkBlocks ? deal[g[q]][g[q + 1] - g[q]] : TileDeal{0};
+                plan.deal[x][nb][q] = q < C && g[q + 1] > g[q] && g[q + 1] - g[q] <= kChunkBlocks ? groups.deal[x][g[q]][g[q + 1] - g[q]] : TileDeal{0};
             }
         }
     }
 }
-// The plan for a window and a number of groups, remembered for the thread's later calls: a plan takes 10 to 25 us to make, and
-// C follows from the batch size, so that batches of changing size ask for several in turn.  There are at most
-// kMaxBlocksFast * kMaxGroups of them, 1 to 2 KB each, given back when the thread ends.
+template <int SPACING, int N>
+inline void plan_chunks(int W, int C, const ChunkCosts (&costs)[N], ChunkPlan<N> &plan) {
+    GroupDeals<N> groups;
+    deal_groups<SPACING>(W, costs, groups);
+    plan_chunks(groups, C, plan);
+}
+// The plan for a window and a number of groups, remembered for the thread's later calls: C follows from the batch size, so that
+// batches of changing size ask for several in turn, and the loss weighs the plans of several C in one call.  What they share, the
+// deals of all groups, takes 10 to 20 us a window, a plan 2 to 5 (a plan with deals of its own 15 to 50, the first loss call of a
+// window 450 for 110).  At most kMaxBlocksFast windows of 1 to 2 KB and kMaxBlocksFast * kMaxGroups plans of as much, given back when
+// the thread ends.
 template <int SPACING, int N>
 inline const ChunkPlan<N> &chunk_plan(int translen, int C, const ChunkCosts (&costs)[N]) {
+    static thread_local std::unique_ptr<GroupDeals<N>> deals[kMaxBlocksFast];
     static thread_local std::unique_ptr<ChunkPlan<N>> plans[kMaxBlocksFast][kMaxGroups];
     const int w = (translen + kBlk - 1) / kBlk, W = w < kMaxBlocksFast ? w : kMaxBlocksFast;
     std::unique_ptr<ChunkPlan<N>> &plan = plans[W - 1][C - 1];
     if (!plan) {
+        if (!deals[W - 1]) {
+            deals[W - 1].reset(new GroupDeals<N>);
+            deal_groups<SPACING>(W, costs, *deals[W - 1]);
+        }
         plan.reset(new ChunkPlan<N>);
-        plan_chunks<SPACING>(W, C, costs, *plan);
+        plan_chunks(*deals[W - 1], C, *plan);
     }
     return *plan;
 }
@@ -274,7 +299,7 @@ inline void make_tables(GroupTable (&tables)[kMostTables], TableChoice &o, int B
     auto stages2 = [&](const int c) { return 2 * (NC + NB) + 3 * (c - 1); };
     int best = plan_of(least).busiest[which][NB];
     const long long now = (long long)best * stages2(least);
-    for (int c = least + 1; c <= kMaxGroups && o.ntable < kMostTables; ++c) {
+    for (int c = least + 1; c <= kMaxGroups && c <= NB && o.ntable < kMostTables; ++c) {
         const int bound = plan_of(c).busiest[which][NB];
         if (bound >= best || 100 * (long long)bound * stages2(c) > 97 * now) continue;
         GroupTable &table = tables[o.ntable];
