@@ -107,9 +107,10 @@ __device__ __host__ __forceinline__ int dealt_foreign(const TileDeal &d, int wav
 // of the adjacent tile), a tile, fetching a foreign block (most of it waits); and how much of the sum of two waves' times a SIMD takes for
 // both, in per cent (waves w and w + 4 share one).
 struct ChunkCosts { int walk, product, fetch, shared; };
-// Returns how long the busiest wave or SIMD takes, -1 if there are more tiles than the waves have room for.
+// Returns how long the busiest wave or SIMD takes, -1 if there are more tiles than the waves have room for; alone: how long the busiest
+// SIMD takes if it does nothing for one wave while it does something for the other.
 template <int SPACING>
-inline int deal_tiles(int jb0, int nblk, int W, const ChunkCosts &cost, TileDeal &deal) {   // (on the host: a plan made by the kernel costs it 2 us)
+inline int deal_tiles(int jb0, int nblk, int W, const ChunkCosts &cost, TileDeal &deal, int &alone) {   // (on the host: a plan made by the kernel costs it 2 us)
     constexpr int kSimds = 4;
     int load[kTileWaves] = {0}, tiles[kTileWaves] = {0}, foreign[kTileWaves] = {0};
     for (int w = 0; w < nblk; ++w) load[w] = cost.walk - (SPACING == 1 && jb0 + w == 0 ? cost.product : 0);
@@ -137,9 +138,12 @@ inline int deal_tiles(int jb0, int nblk, int W, const ChunkCosts &cost, TileDeal
     for (int n = 0; n < nfor; ++n) if (!place(foreign, true, cost.fetch)) return -1;
     deal.wave = 0;
     int most = 0;
+    alone = 0;
     for (int w = 0; w < kTileWaves; ++w) {
         deal.wave |= (unsigned)(tiles[w] | foreign[w] << 2) << (4 * w);
         most = busy(w, 0) > most ? busy(w, 0) : most;
+        const int both = load[w] + load[(w + kSimds) % kTileWaves];
+        alone = both > alone ? both : alone;
     }
     return most;
 }
@@ -156,7 +160,14 @@ __device__ __host__ __forceinline__ void wave_foreign(const TileDeal &d, int wav
 
 // Host: the groupings of a graph's position blocks for every number of blocks up to NB, each into at most C contiguous
 // groups of at most kTileCap tiles (the diagonal ones among them) and kChunkBlocks blocks so that the busiest SIMD has
-// least to do.  gtab[nb][g] .. gtab[nb][g+1]: blocks of group g (empty groups last).
+// least to do: as few groups as can be, or more even ones.  In a SIMD with a walk and little else the costs hide the other wave's work
+// behind the walk; measured, a stage is longer by about a sixth of that, and by no more than the same share of the groups' mean.  So of
+// the groupings with that bound the one whose busiest such SIMD has least is taken where that gains more than the further hand-overs
+// take (one and a half stages each, of as many as a target of a fifth of the graph has).  us, as few as can be -> as measured with the
+// groups here: alignment B = 1, L = 456, T = 182, transitions of at most 11 (two groups of four blocks -> four of two) 173.5 -> 159.5; B = 3,
+// L = 811, T = 162, at most 166 (4 3 3 3 -> 3 2 2 2 2 2) 229 -> 216; B = 29, L = 240, T = 96, at most 27 94.6 -> 89.3; loss B = 58, L = 271,
+// T = 54 (4 1 -> 3 2) 74.8 -> 69; and where as few as can be are kept: B = 12, L = 540, T = 67 120 against 124 with 3 2 1 1 1 1 for 4 2 1 1 1, B = 32,
+// L = 452, T = 56, at most 92 89 against 93.  gtab[nb][g] .. gtab[nb][g+1]: blocks of group g (empty groups last).
 template <int N>
 struct ChunkPlan {
     // one of each for each set of costs
@@ -170,12 +181,15 @@ template <int N>
 struct GroupDeals {
     short cost[N][kMaxBlocksFast][kChunkBlocks + 1];   // -1: more tiles than a workgroup has room for
     TileDeal deal[N][kMaxBlocksFast][kChunkBlocks + 1];
-    short most[N];                                     // the greatest of the costs
+    short alone[N][kMaxBlocksFast][kChunkBlocks + 1];
+    short most[N], most_alone[N];                      // the greatest of them
+    int spacing;
 };
 template <int SPACING, int N>
 inline void deal_groups(int W, const ChunkCosts (&costs)[N], GroupDeals<N> &o) {
+    o.spacing = SPACING;
     for (int x = 0; x < N; ++x) {
-        o.most[x] = 0;
+        o.most[x] = o.most_alone[x] = 0;
         for (int j = 0; j < kMaxBlocksFast; ++j) {
             int tiles = 0;
             for (int n = 1; n <= kChunkBlocks; ++n) {
@@ -183,8 +197,11 @@ inline void deal_groups(int W, const ChunkCosts (&costs)[N], GroupDeals<N> &o) {
                 o.deal[x][j][n] = TileDeal{0};
                 if (j + n > kMaxBlocksFast) continue;
                 tiles += j + n - tile_ilo(j + n - 1, W);
-                if (tiles <= kTileCap) o.cost[x][j][n] = (short)deal_tiles<SPACING>(j, n, W, costs[x], o.deal[x][j][n]);
+                int alone = 0;
+                if (tiles <= kTileCap) o.cost[x][j][n] = (short)deal_tiles<SPACING>(j, n, W, costs[x], o.deal[x][j][n], alone);
+                o.alone[x][j][n] = (short)alone;
                 o.most[x] = o.cost[x][j][n] > o.most[x] ? o.cost[x][j][n] : o.most[x];
+                o.most_alone[x] = o.alone[x][j][n] > o.most_alone[x] ? o.alone[x][j][n] : o.most_alone[x];
             }
         }
     }
@@ -192,25 +209,47 @@ inline void deal_groups(int W, const ChunkCosts (&costs)[N], GroupDeals<N> &o) {
 template <int N>
 inline void plan_chunks(const GroupDeals<N> &groups, int C, ChunkPlan<N> &plan) {
     for (int x = 0; x < N; ++x) {
-        const auto &cost = groups.cost[x];
+        const auto &cost = groups.cost[x], &alone = groups.alone[x];
         for (int nb = 0; nb <= kMaxBlocksFast; ++nb) {
             int low = 0, high = groups.most[x] + 1;      // the least bound on a group's cost that C groups can keep
             unsigned char g[16];
-            auto split = [&](const int most) {
+            auto split = [&](const int most, const int most_alone) {   // (the second holds for groups that take `most`)
                 int used = 0, j = 0;
                 g[0] = 0;
                 for (int q = 1; q < 16; ++q) g[q] = (unsigned char)nb;
                 while (j < nb) {
                     int n = nb - j < kChunkBlocks ? nb - j : kChunkBlocks;
-                    while (n > 0 && (cost[j][n] < 0 || cost[j][n] > most)) --n;
+                    while (n > 0 && (cost[j][n] < 0 || cost[j][n] > most || (cost[j][n] == most && alone[j][n] > most_alone))) --n;
                     if (n == 0 || used == C) return false;
                     j += n;
                     g[++used] = (unsigned char)j;
                 }
                 return true;
             };
-            while (low < high) { const int mid = (low + high) / 2; if (split(mid)) high = mid; else low = mid + 1; }
-            plan.busiest[x][nb] = (short)(split(high) ? high : kNoPlan);
+            // groups, how much longer than `high` the busiest SIMD of any takes if its waves' work does not overlap, and the sum over all
+            auto over = [&](int &n, int &most, int &sum) {
+                n = most = sum = 0;
+                for (; n < C && g[n + 1] > g[n]; ++n) {
+                    const int more = alone[g[n]][g[n + 1] - g[n]] - high;
+                    most = more > most ? more : most;
+                    sum += more > 0 ? more : 0;
+                }
+            };
+            const int any = groups.most_alone[x];
+            while (low < high) { const int mid = (low + high) / 2; if (split(mid, any)) high = mid; else low = mid + 1; }
+            const bool ok = split(high, any);
+            int n, most, sum;
+            over(n, most, sum);
+            if (ok && most > 0) {
+                int n2, most2, sum2, low_alone = high, high_alone = high + most;
+                while (low_alone < high_alone) { const int mid = (low_alone + high_alone) / 2; if (split(high, mid)) high_alone = mid; else low_alone = mid + 1; }
+                split(high, high_alone);
+                over(n2, most2, sum2);
+                const long long stages = (16 + 5 * groups.spacing) * nb, cost = 90 * high * (n2 - n);   // (stages: five times)
+                const bool pays = 2 * (most - most2) * stages > cost && 2 * (sum * n2 - sum2 * n) * stages > cost * n * n2;
+                if (!pays) split(high, any);
+            }
+            plan.busiest[x][nb] = (short)(ok ? high : kNoPlan);
             for (int q = 0; q < 12; ++q) {
                 plan.gtab[x][nb][q] = g[q];
                 plan.deal[x][nb][q] = q < C && g[q + 1] > g[q] && g[q + 1] - g[q] <= kChunkBlocks ? groups.deal[x][g[q]][g[q + 1] - g[q]] : TileDeal{0};
@@ -226,8 +265,7 @@ inline void plan_chunks(int W, int C, const ChunkCosts (&costs)[N], ChunkPlan<N>
 }
 // The plan for a window and a number of groups, remembered for the thread's later calls: C follows from the batch size, so that
 // batches of changing size ask for several in turn, and the loss weighs the plans of several C in one call.  What they share, the
-// deals of all groups, takes 10 to 20 us a window, a plan 2 to 5 (a plan with deals of its own 15 to 50, the first loss call of a
-// window 450 for 110).  At most kMaxBlocksFast windows of 1 to 2 KB and kMaxBlocksFast * kMaxGroups plans of as much, given back when
+// deals of all groups, takes 10 to 20 us a window, a plan 3 to 10 (eleven plans of a window with deals of their own 450 us, so 150).  At most kMaxBlocksFast windows of 1 to 2 KB and kMaxBlocksFast * kMaxGroups plans of as much, given back when
 // the thread ends.
 template <int SPACING, int N>
 inline const ChunkPlan<N> &chunk_plan(int translen, int C, const ChunkCosts (&costs)[N]) {

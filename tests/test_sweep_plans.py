@@ -39,6 +39,20 @@ static int check(const ChunkCosts (&costs)[N]) {
     // a window longer than any graph the sweeps take is that of the longest
     return &chunk_plan<SPACING>(8192, 4, costs) != &chunk_plan<SPACING>(64 * kMaxBlocksFast, 4, costs);
 }
+// blocks of the groups of a graph of nb blocks
+template <int SPACING>
+static bool groups_are(const ChunkCosts &cost, int W, int C, int nb, std::vector<int> want) {
+    const ChunkCosts costs[1] = {cost};
+    ChunkPlan<1> plan;
+    plan_chunks<SPACING>(W, C, costs, plan);
+    std::vector<int> got;
+    for (int q = 0; q < C && plan.gtab[0][nb][q + 1] > plan.gtab[0][nb][q]; ++q) got.push_back(plan.gtab[0][nb][q + 1] - plan.gtab[0][nb][q]);
+    if (got == want) return true;
+    std::printf("W=%d C=%d nb=%d:", W, C, nb);
+    for (const int n : got) std::printf(" %d", n);
+    std::printf("\n");
+    return false;
+}
 // us to make the plans of a window for C = 1 .. most, on a thread that has made none: the median of 41
 static double first(const ChunkCosts (&costs)[2], int translen, int most) {
     std::vector<double> us;
@@ -53,6 +67,10 @@ static double first(const ChunkCosts (&costs)[2], int translen, int most) {
 }
 int main() {
     static const ChunkCosts loss[2] = {{45, 7, 4, 100}, {85, 17, 11, 100}}, one[1] = {{62, 27, 4, 75}}, two[1] = {{36, 27, 4, 75}};
+    // groupings as good as each other for the busiest SIMD: more even ones, where they gain more than their hand-overs take
+    if (!groups_are<2>({36, 27, 4, 55}, 1, 8, 8, {2, 2, 2, 2}) || !groups_are<1>({62, 27, 2, 65}, 3, 10, 13, {3, 2, 2, 2, 2, 2}) ||
+        !groups_are<1>({45, 9, 12, 70}, 5, 2, 5, {3, 2}) || !groups_are<1>({62, 27, 2, 65}, 9, 9, 9, {4, 2, 1, 1, 1}) ||
+        !groups_are<2>({36, 27, 4, 55}, 2, 8, 8, {3, 2, 2, 1})) return 1;
     // eleven plans, as the first loss call of a window may weigh: each for itself they took eleven times as long as one
     for (const int translen : {300, 511, 1023})
         if (first(loss, translen, 11) > 7 * first(loss, translen, 1)) { std::printf("translen %d: %.0f us, one plan %.0f us\n", translen, first(loss, translen, 11), first(loss, translen, 1)); return 1; }
