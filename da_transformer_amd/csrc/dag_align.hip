@@ -218,33 +218,6 @@ __device__ __host__ inline int partition_blocks(int NBb, int W, int C, int *gsta
     return used;
 }
 
-// Whether the sweep goes in chunks of four steps.  They cost T / 4 stages and one or two more for every block of nodes, single
-// steps T of two fifths of that: even at about six steps for every block of nodes and eight more (alignment, chunks and
-// steps: B = 64, L = 512, T = 64 129 and 140 us; B = 28, L = 450, T = 50 108 and 103; B = 20, L = 1000, T = 128 297 and 328; B = 1,
-// L = 900, T = 70 196 and 179; B = 48, L = 350, T = 40 81 and 76; B = 8, L = 128, T = 32 38 and 44; B = 1, L = 115, T = 15 29 and 27).
-static bool align_in_chunks(int B, int T, int L, int translen) {
-    return T >= 6 * ((L + kBlk - 1) / kBlk) + 8 && (int64_t)B * L * translen >= 4;   // (the chunked kernel's tiles are loaded four elements at a time)
-}
-
-// Workgroups per sweep.  In chunks: from four position blocks on as many as the device has room for (one per CU) up to one
-// for each block, at most ten.  (Fewer tiles a SIMD, against more hand-overs: as many as hold the tiles -> this, alignment of
-// B = 16, L = 1024, T = 256 484 -> 445 us; B = 4, L = 700, T = 100 211 -> 183; B = 64, L = 320, T = 48 83 -> 79; B = 64, L = 256,
-// T = 64 92 -> 80.)  Step by step: twice as many as hold the tiles where there is room and the graph has at least four
-// blocks (5 to 13 %; more lose); where that exceeds what the kernel supports, ten when they fit.
-static int align_groups(int B, int T, int L, int translen) {
-    const int NB = (L + kBlk - 1) / kBlk, B8 = (B + 7) & ~7;
-    if (align_in_chunks(B, T, L, translen)) {
-        const int C = groups_needed(L, translen, kChunkBlocks);
-        if (C == 0 || NB < 4) return C;
-        const int room = 256 / B8, most = NB < 10 ? NB : 10, more = room < most ? room : most;
-        return more > C ? more : C;
-    }
-    const int C = groups_needed(L, translen, kMaxBlocksFast);
-    if (C == 0) return 0;
-    if (NB >= 4 && 2 * C <= kMaxGroups && 2 * C <= NB && (long long)B8 * 2 * C <= 256) return 2 * C;
-    return C < 10 && NB >= 10 && (long long)B8 * 10 <= 256 ? 10 : C;
-}
-
 struct AlignTileArgs {
     const void *match; int64_t ms0, ms1, ms2;
     const void *links;
@@ -260,32 +233,6 @@ struct AlignTileArgs {
                       // pruned for being too far from the last node -- a path may end at any step
     ChunkPlan<1> plan;   // gtab[NBb][g] = first block of group g, and how its tiles are dealt to its waves
 };
-
-// LDS of a group, in dwords: cells of four steps in the order of the table, results of a wave's tiles that lead to one block.
-struct AlignLds {
-    int depth, runs;    // chunks of cells kept per block; runs of tiles there can be
-    int eb;             // [nsrc][depth][4][64]
-    int both;           // [1] SPACING 1: counts the last two blocks' waves as they find their rows in memory
-    int part, from;     // [runs][2][64][4] best scores of four steps a lane; [runs][2][64] the blocks they come from, a byte each
-    int total;
-};
-__device__ __host__ inline AlignLds align_lds(int jb0, int nblk, int W, int spacing) {
-    AlignLds o;
-    const int nsrc = jb0 - tile_ilo(jb0, W) + nblk;
-    int ntile = 0;
-    for (int q = 0; q < nblk; ++q) ntile += spacing == 1 ? tiles_of_block<1>(jb0 + q, W) : tiles_of_block<2>(jb0 + q, W);
-    // (read up to SPACING (blocks of the group) stages after they are written; foreign rows are copied into place up to a
-    // stage before they are due)
-    o.depth = spacing * (nblk < W ? nblk : W) + 3 - spacing;
-    o.runs = ntile < kTileWaves + nblk - 1 ? ntile : kTileWaves + nblk - 1;
-    int at = 0;
-    o.eb = at; at += nsrc * o.depth * 256;
-    o.part = at; at += o.runs * 2 * 256;
-    o.from = at; at += o.runs * 2 * 64;
-    o.both = at; at += 4;
-    o.total = at;
-    return o;
-}
 
 // The pipeline of the loss sweeps (sweep_chunks_group: stages of four steps, tickets, one-way hand-over through the table
 // with agent-scope accesses, bounded waits), in the (max, +) semiring and without any rescaling: the table holds the plain
@@ -1312,11 +1259,7 @@ static int prepare_align_chunks() {
 }
 template <typename TM, typename TL, int SPACING>
 static int launch_align_chunks(AlignTileArgs &ta, const char *who, hipStream_t st) {
-    // Found by timing calls under some twenty sets, from the pieces' own times {62 or 36, 27, 4, 75} on (us): B = 64, L = 512, T = 64
-    // 120.3 -> 116.6, B = 16, L = 768, T = 192 276.5 -> 268, B = 4, L = 700, T = 110 187 -> 179, B = 64, L = 256, T = 64
-    // (SPACING 2) 79.0 -> 76.1, B = 40, L = 400, T = 60 (SPACING 2) 99.5 -> 95.2; the others the same.
-    static const ChunkCosts costs[1] = {SPACING == 1 ? ChunkCosts{62, 27, 2, 65} : ChunkCosts{36, 27, 4, 55}};
-    ta.plan = chunk_plan<SPACING>(ta.translen, ta.C, costs);
+    ta.plan = chunk_plan<SPACING>(ta.translen, ta.C, kAlignCosts<SPACING>);
     if (int rc = prepare_align_chunks<TM, TL, SPACING>()) return rc;
     hipLaunchKernelGGL((dag_align_chunks_kernel<TM, TL, SPACING>), dim3(((ta.B + 7) & ~7) * ta.C), dim3(kTileWaves * kWave), kChunkLdsBytes, st, ta);
     return check_launch(who);
@@ -1334,7 +1277,7 @@ static int launch_align_sweep(AlignTileArgs &ta, const char *who, hipStream_t st
         hipLaunchKernelGGL((dag_align_steps_kernel<TM, TL>), dim3(((ta.B + 7) & ~7) * ta.C), dim3(kTileWaves * kWave), 0, st, ta);
         return check_launch(who);
     }
-    return NB <= 5 || (NB <= 8 && 2 * NB <= 3 * ta.C) ? launch_align_chunks<TM, TL, 2>(ta, who, st) : launch_align_chunks<TM, TL, 1>(ta, who, st);
+    return align_spacing(NB, ta.C) == 2 ? launch_align_chunks<TM, TL, 2>(ta, who, st) : launch_align_chunks<TM, TL, 1>(ta, who, st);
 }
 constexpr size_t kBacktrackMostLds = kAlignLdsBudget > kWalkLds ? kAlignLdsBudget : kWalkLds;   // (the redo alone asks for at most the former)
 template <typename TM, typename TL, bool TRACE_LDS, bool STAGED>

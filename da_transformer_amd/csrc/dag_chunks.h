@@ -263,23 +263,29 @@ inline void plan_chunks(int W, int C, const ChunkCosts (&costs)[N], ChunkPlan<N>
     deal_groups<SPACING>(W, costs, groups);
     plan_chunks(groups, C, plan);
 }
-// The plan for a window and a number of groups, remembered for the thread's later calls: C follows from the batch size, so that
-// batches of changing size ask for several in turn, and the loss weighs the plans of several C in one call.  What they share, the
-// deals of all groups, takes 10 to 20 us a window, a plan 3 to 10 (eleven plans of a window with deals of their own 450 us, so 150).  At most kMaxBlocksFast windows of 1 to 2 KB and kMaxBlocksFast * kMaxGroups plans of as much, given back when
-// the thread ends.
+// The deals and the plans for a window, remembered for the thread's later calls: C follows from the batch size, so that batches of
+// changing size ask for several plans in turn, and the loss weighs the plans of several C in one call.  What these share, the deals of
+// all groups, takes 10 to 20 us, a plan 3 to 10 (eleven plans with deals of their own 450 us, so 150).  At most kMaxBlocksFast windows'
+// deals and kMaxBlocksFast * kMaxGroups plans, 1 to 2 KB each, given back when the thread ends.
+inline int window_blocks(int translen) { const int w = (translen + kBlk - 1) / kBlk; return w < kMaxBlocksFast ? w : kMaxBlocksFast; }
+template <int SPACING, int N>
+inline const GroupDeals<N> &group_deals(int translen, const ChunkCosts (&costs)[N]) {
+    static thread_local std::unique_ptr<GroupDeals<N>> deals[kMaxBlocksFast];
+    const int W = window_blocks(translen);
+    std::unique_ptr<GroupDeals<N>> &of = deals[W - 1];
+    if (!of) {
+        of.reset(new GroupDeals<N>);
+        deal_groups<SPACING>(W, costs, *of);
+    }
+    return *of;
+}
 template <int SPACING, int N>
 inline const ChunkPlan<N> &chunk_plan(int translen, int C, const ChunkCosts (&costs)[N]) {
-    static thread_local std::unique_ptr<GroupDeals<N>> deals[kMaxBlocksFast];
     static thread_local std::unique_ptr<ChunkPlan<N>> plans[kMaxBlocksFast][kMaxGroups];
-    const int w = (translen + kBlk - 1) / kBlk, W = w < kMaxBlocksFast ? w : kMaxBlocksFast;
-    std::unique_ptr<ChunkPlan<N>> &plan = plans[W - 1][C - 1];
+    std::unique_ptr<ChunkPlan<N>> &plan = plans[window_blocks(translen) - 1][C - 1];
     if (!plan) {
-        if (!deals[W - 1]) {
-            deals[W - 1].reset(new GroupDeals<N>);
-            deal_groups<SPACING>(W, costs, *deals[W - 1]);
-        }
         plan.reset(new ChunkPlan<N>);
-        plan_chunks(*deals[W - 1], C, *plan);
+        plan_chunks(group_deals<SPACING>(translen, costs), C, *plan);
     }
     return *plan;
 }
@@ -363,6 +369,82 @@ __device__ __host__ __forceinline__ void place_of_ticket(int r, int n, int ndir,
     const int full = n & ~7, rest = n - full > 0 ? n - full : 1;
     if (r < ndir * full) { rank = (r / (8 * ndir)) * 8 + r % 8; slot = (r / 8) % ndir; }
     else { r -= ndir * full; rank = full + r % rest; slot = r / rest; }
+}
+
+// Workgroups per sweep (two sweeps a sample): as few as hold the tiles, but with at most four blocks each, one walk to a
+// SIMD, where the device has a CU for every workgroup.  Forward with up to eight -> up to four blocks: B = 40, L = 328,
+// T = 41 67 -> 61 us; B = 16, L = 512, T = 64 102 -> 97.5; B = 64 and transitions of at most 32 88 -> 79; B = 16,
+// L = 1024 and transitions of at most 64 122 -> 104.  More groups than that: see make_tables.
+inline int sweep_groups(int B, int L, int translen) {
+    const int C = groups_needed(L, translen, 4), sweeps = 2 * ((B + 7) & ~7);
+    return (long long)sweeps * C <= kSweepCus && C > 0 ? C : groups_needed(L, translen, kChunkBlocks);
+}
+// float32, float64.  Found by timing the sweeps themselves under some forty sets (us; first the costs of each piece timed alone,
+// with a SIMD taking the sum of its two waves' work, {45, 7, 4, 100} and {85, 17, 11, 100}; then these): float32 B = 64, L = 512, T = 64
+// 107 -> 95; B = 16, L = 1024, T = 256 347 -> 329; B = 16, L = 512, T = 128 134 -> 127; B = 8, L = 1024, T = 256 334 -> 302; float64 at the
+// first of them 151 -> 141.  A fetched block waits for the rows of its producer and for LDS twice, so it keeps its wave for longer than
+// its instructions take; and while a wave waits, the other wave of its SIMD works.
+constexpr ChunkCosts kSweepCosts[2] = {{45, 9, 12, 70}, {85, 25, 16, 80}};
+
+// ---- the alignment's rules ----
+// Whether the sweep goes in chunks of four steps.  They cost T / 4 stages and one or two more for every block of nodes, single
+// steps T of two fifths of that: even at about six steps for every block of nodes and eight more (alignment, chunks and
+// steps: B = 64, L = 512, T = 64 129 and 140 us; B = 28, L = 450, T = 50 108 and 103; B = 20, L = 1000, T = 128 297 and 328; B = 1,
+// L = 900, T = 70 196 and 179; B = 48, L = 350, T = 40 81 and 76; B = 8, L = 128, T = 32 38 and 44; B = 1, L = 115, T = 15 29 and 27).
+inline bool align_in_chunks(int B, int T, int L, int translen) {
+    return T >= 6 * ((L + kBlk - 1) / kBlk) + 8 && (int64_t)B * L * translen >= 4;   // (the chunked kernel's tiles are loaded four elements at a time)
+}
+
+// Workgroups per sweep.  In chunks: from four position blocks on as many as the device has room for (one per CU) up to one
+// for each block, at most ten.  (Fewer tiles a SIMD, against more hand-overs: as many as hold the tiles -> this, alignment of
+// B = 16, L = 1024, T = 256 484 -> 445 us; B = 4, L = 700, T = 100 211 -> 183; B = 64, L = 320, T = 48 83 -> 79; B = 64, L = 256,
+// T = 64 92 -> 80.)  Step by step: twice as many as hold the tiles where there is room and the graph has at least four
+// blocks (5 to 13 %; more lose); where that exceeds what the kernel supports, ten when they fit.
+inline int align_groups(int B, int T, int L, int translen) {
+    const int NB = (L + kBlk - 1) / kBlk, B8 = (B + 7) & ~7;
+    if (align_in_chunks(B, T, L, translen)) {
+        const int C = groups_needed(L, translen, kChunkBlocks);
+        if (C == 0 || NB < 4) return C;
+        const int room = 256 / B8, most = NB < 10 ? NB : 10, more = room < most ? room : most;
+        return more > C ? more : C;
+    }
+    const int C = groups_needed(L, translen, kMaxBlocksFast);
+    if (C == 0) return 0;
+    if (NB >= 4 && 2 * C <= kMaxGroups && 2 * C <= NB && (long long)B8 * 2 * C <= 256) return 2 * C;
+    return C < 10 && NB >= 10 && (long long)B8 * 10 <= 256 ? 10 : C;
+}
+// Stages from a block's walk of a chunk to the next block's: see dag_align_chunks_kernel.
+inline int align_spacing(int NB, int C) { return NB <= 5 || (NB <= 8 && 2 * NB <= 3 * C) ? 2 : 1; }
+// Found by timing calls under some twenty sets, from the pieces' own times {62 or 36, 27, 4, 75} on (us): B = 64, L = 512, T = 64
+// 120.3 -> 116.6, B = 16, L = 768, T = 192 276.5 -> 268, B = 4, L = 700, T = 110 187 -> 179, B = 64, L = 256, T = 64
+// (SPACING 2) 79.0 -> 76.1, B = 40, L = 400, T = 60 (SPACING 2) 99.5 -> 95.2; the others the same.
+template <int SPACING>
+constexpr ChunkCosts kAlignCosts[1] = {SPACING == 1 ? ChunkCosts{62, 27, 2, 65} : ChunkCosts{36, 27, 4, 55}};
+
+// LDS of a group, in dwords: cells of four steps in the order of the table, results of a wave's tiles that lead to one block.
+struct AlignLds {
+    int depth, runs;    // chunks of cells kept per block; runs of tiles there can be
+    int eb;             // [nsrc][depth][4][64]
+    int both;           // [1] SPACING 1: counts the last two blocks' waves as they find their rows in memory
+    int part, from;     // [runs][2][64][4] best scores of four steps a lane; [runs][2][64] the blocks they come from, a byte each
+    int total;
+};
+__device__ __host__ inline AlignLds align_lds(int jb0, int nblk, int W, int spacing) {
+    AlignLds o;
+    const int nsrc = jb0 - tile_ilo(jb0, W) + nblk;
+    int ntile = 0;
+    for (int q = 0; q < nblk; ++q) ntile += spacing == 1 ? tiles_of_block<1>(jb0 + q, W) : tiles_of_block<2>(jb0 + q, W);
+    // (read up to SPACING (blocks of the group) stages after they are written; foreign rows are copied into place up to a
+    // stage before they are due)
+    o.depth = spacing * (nblk < W ? nblk : W) + 3 - spacing;
+    o.runs = ntile < kTileWaves + nblk - 1 ? ntile : kTileWaves + nblk - 1;
+    int at = 0;
+    o.eb = at; at += nsrc * o.depth * 256;
+    o.part = at; at += o.runs * 2 * 256;
+    o.from = at; at += o.runs * 2 * 64;
+    o.both = at; at += 4;
+    o.total = at;
+    return o;
 }
 
 // ---- what a wave has to do, worked out at the start of the kernel ----

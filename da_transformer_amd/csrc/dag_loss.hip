@@ -1618,21 +1618,6 @@ static bool force_exact() { return force_log_domain(); }
 // ticket + launch counter (16 ints), 2*B*C progress words, B "left" counters, B risk words; rounded to 8 bytes
 static size_t sweep_sync_ints(int B, int C) { return ((16 + (size_t)2 * B * C + (size_t)2 * B) + 1) & ~(size_t)1; }
 
-// Workgroups per sweep (two sweeps a sample): as few as hold the tiles, but with at most four blocks each, one walk to a
-// SIMD, where the device has a CU for every workgroup.  Forward with up to eight -> up to four blocks: B = 40, L = 328,
-// T = 41 67 -> 61 us; B = 16, L = 512, T = 64 102 -> 97.5; B = 64 and transitions of at most 32 88 -> 79; B = 16,
-// L = 1024 and transitions of at most 64 122 -> 104.  More groups than that: see make_tables.
-static int sweep_groups(int B, int L, int translen) {
-    const int C = groups_needed(L, translen, 4), sweeps = 2 * ((B + 7) & ~7);
-    return (long long)sweeps * C <= kSweepCus && C > 0 ? C : groups_needed(L, translen, kChunkBlocks);
-}
-// float32, float64.  Found by timing the sweeps themselves under some forty sets (us; first the costs of each piece timed alone,
-// with a SIMD taking the sum of its two waves' work, {45, 7, 4, 100} and {85, 17, 11, 100}; then these): float32 B = 64, L = 512, T = 64
-// 107 -> 95; B = 16, L = 1024, T = 256 347 -> 329; B = 16, L = 512, T = 128 134 -> 127; B = 8, L = 1024, T = 256 334 -> 302; float64 at the
-// first of them 151 -> 141.  A fetched block waits for the rows of its producer and for LDS twice, so it keeps its wave for longer than
-// its instructions take; and while a wave waits, the other wave of its SIMD works.
-static const ChunkCosts kSweepCosts[2] = {{45, 9, 12, 70}, {85, 25, 16, 80}};
-
 // ticket + progress words (rounded to 8 bytes), then the fast kernel's two read-outs per sample
 static size_t sweep_bytes(int B, int C) { return sweep_sync_ints(B, C) * sizeof(int) + (size_t)2 * B * sizeof(double); }
 

@@ -9,12 +9,9 @@ import pytest
 from conftest import ROOT
 
 PROGRAM = r"""
-#include <algorithm>
-#include <chrono>
 #include <cstdio>
 #include <cstring>
 #include <memory>
-#include <thread>
 #include <vector>
 #include "dag_chunks.h"
 using namespace dagx;
@@ -28,11 +25,13 @@ static int check(const ChunkCosts (&costs)[N]) {
             for (int C = 1; C <= 11; ++C) {
                 auto fresh = std::make_unique<ChunkPlan<N>>();
                 plan_chunks<SPACING>(W, C, costs, *fresh);
-                if (std::memcmp(fresh->gtab, kept[C]->gtab, sizeof fresh->gtab) || std::memcmp(fresh->deal, kept[C]->deal, sizeof fresh->deal)) {
+                if (std::memcmp(fresh->gtab, kept[C]->gtab, sizeof fresh->gtab) || std::memcmp(fresh->deal, kept[C]->deal, sizeof fresh->deal) ||
+                    std::memcmp(fresh->busiest, kept[C]->busiest, sizeof fresh->busiest)) {
                     std::printf("W=%d C=%d: another plan in its place\n", W, C);
                     return 1;
                 }
             }
+            if (&group_deals<SPACING>(64 * W - 1, costs) != &group_deals<SPACING>(64 * W, costs)) { std::printf("W=%d: deals made again\n", W); return 1; }
             for (int C = 1; C <= 11; ++C)
                 if (kept[C] != &chunk_plan<SPACING>(64 * W, C, costs)) { std::printf("W=%d C=%d: made again\n", W, C); return 1; }
         }
@@ -53,28 +52,55 @@ static bool groups_are(const ChunkCosts &cost, int W, int C, int nb, std::vector
     std::printf("\n");
     return false;
 }
-// us to make the plans of a window for C = 1 .. most, on a thread that has made none: the median of 41
-static double first(const ChunkCosts (&costs)[2], int translen, int most) {
-    std::vector<double> us;
-    for (int round = 0; round < 41; ++round)
-        std::thread([&] {
-            const auto start = std::chrono::steady_clock::now();
-            for (int C = 1; C <= most; ++C) chunk_plan<1>(translen, C, costs);
-            us.push_back(std::chrono::duration<double, std::micro>(std::chrono::steady_clock::now() - start).count());
-        }).join();
-    std::sort(us.begin(), us.end());
-    return us[20];
+// Every group of an alignment's plan has its tiles and foreign blocks dealt to waves that have room for them, and fits a CU's LDS: one that
+// does not sends its samples to the one-workgroup redo.
+template <int SPACING>
+static bool alignment_fits(int B, int T, int L, int translen, int C) {
+    const ChunkPlan<1> &plan = chunk_plan<SPACING>(translen, C, kAlignCosts<SPACING>);
+    const int W = (translen + kBlk - 1) / kBlk;
+    for (int nb = 1; nb <= (L + kBlk - 1) / kBlk; ++nb) {
+        const unsigned char *g = plan.gtab[0][nb];
+        int n = 0;
+        bool ok = plan.busiest[0][nb] < kNoPlan;
+        for (int q = 0; q < C; ++q) {
+            if (g[q + 1] == g[q]) continue;
+            const int size = g[q + 1] - g[q];
+            int tiles = 0, foreign = 0, want = 0;
+            ok = ok && q == n++ && size > 0 && size <= kChunkBlocks;
+            for (int w = 0; ok && w < kTileWaves; ++w) {
+                const int mine = dealt_tiles(plan.deal[0][nb][q], w), fetch = dealt_foreign(plan.deal[0][nb][q], w);
+                ok = w >= size || (mine <= SPACING && (fetch == 0 || size == kTileWaves));
+                tiles += mine; foreign += fetch;
+            }
+            for (int J = g[q]; J < g[q + 1]; ++J) want += tiles_of_block<SPACING>(J, W);
+            ok = ok && tiles == want && foreign == g[q] - tile_ilo(g[q], W) && align_lds(g[q], size, W, SPACING).total * 4 <= kChunkLdsBytes;
+        }
+        if (ok && g[0] == 0 && g[n] == nb) continue;
+        std::printf("alignment B=%d T=%d L=%d translen=%d: C=%d nb=%d\n", B, T, L, translen, C, nb);
+        return false;
+    }
+    return true;
+}
+static int alignment() {
+    int seen = 0;
+    for (int B = 1; B <= 128; B += B < 70 ? 3 : 29)
+        for (int L = 2; L <= 1024; L += 31)
+            for (int translen = 1; translen < L; translen = translen < 64 ? 64 : translen + 64) {
+                const int T = L;
+                if (!align_in_chunks(B, T, L, translen)) continue;
+                const int C = align_groups(B, T, L, translen);
+                if (C == 0) continue;
+                ++seen;
+                if (align_spacing((L + kBlk - 1) / kBlk, C) == 2 ? !alignment_fits<2>(B, T, L, translen, C) : !alignment_fits<1>(B, T, L, translen, C)) return 1;
+            }
+    return seen < 3000;
 }
 int main() {
-    static const ChunkCosts loss[2] = {{45, 7, 4, 100}, {85, 17, 11, 100}}, one[1] = {{62, 27, 4, 75}}, two[1] = {{36, 27, 4, 75}};
     // groupings as good as each other for the busiest SIMD: more even ones, where they gain more than their hand-overs take
-    if (!groups_are<2>({36, 27, 4, 55}, 1, 8, 8, {2, 2, 2, 2}) || !groups_are<1>({62, 27, 2, 65}, 3, 10, 13, {3, 2, 2, 2, 2, 2}) ||
-        !groups_are<1>({45, 9, 12, 70}, 5, 2, 5, {3, 2}) || !groups_are<1>({62, 27, 2, 65}, 9, 9, 9, {4, 2, 1, 1, 1}) ||
-        !groups_are<2>({36, 27, 4, 55}, 2, 8, 8, {3, 2, 2, 1})) return 1;
-    // eleven plans, as the first loss call of a window may weigh: each for itself they took eleven times as long as one
-    for (const int translen : {300, 511, 1023})
-        if (first(loss, translen, 11) > 7 * first(loss, translen, 1)) { std::printf("translen %d: %.0f us, one plan %.0f us\n", translen, first(loss, translen, 11), first(loss, translen, 1)); return 1; }
-    return check<1>(loss) || check<1>(one) || check<2>(two);
+    if (!groups_are<2>(kAlignCosts<2>[0], 1, 8, 8, {2, 2, 2, 2}) || !groups_are<1>(kAlignCosts<1>[0], 3, 10, 13, {3, 2, 2, 2, 2, 2}) ||
+        !groups_are<1>(kSweepCosts[0], 5, 2, 5, {3, 2}) || !groups_are<1>(kAlignCosts<1>[0], 9, 9, 9, {4, 2, 1, 1, 1}) ||
+        !groups_are<2>(kAlignCosts<2>[0], 2, 8, 8, {3, 2, 2, 1})) return 1;
+    return check<1>(kSweepCosts) || check<1>(kAlignCosts<1>) || check<2>(kAlignCosts<2>) || alignment();
 }
 """
 
@@ -84,7 +110,7 @@ def test_a_plan_outlives_calls_with_other_numbers_of_workgroups(tmp_path):
     src, exe = tmp_path / "plans.hip", tmp_path / "plans"
     src.write_text(PROGRAM)
     subprocess.run(["/opt/rocm/bin/hipcc", "--offload-arch=gfx950", "--cuda-host-only", "-O1", "-std=c++17", "-Wno-unused-function",
-                    "-pthread", "-I", os.path.join(ROOT, "include"), "-I", os.path.join(ROOT, "da_transformer_amd", "csrc"), str(src), "-o", str(exe)],
+                    "-I", os.path.join(ROOT, "include"), "-I", os.path.join(ROOT, "da_transformer_amd", "csrc"), str(src), "-o", str(exe)],
                    check=True, capture_output=True)
     run = subprocess.run([str(exe)], capture_output=True, text=True)
     assert run.returncode == 0, run.stdout

@@ -15,7 +15,6 @@ PROGRAM = r"""
 #include <tuple>
 #include "dag_chunks.h"
 using namespace dagx;
-static const ChunkCosts costs[2] = {{45, 9, 12, 70}, {85, 25, 16, 80}};
 static int fail(const char *what, int B, int T, int L, int W, int x) { std::printf("%s: B=%d T=%d L=%d translen=%d table %d\n", what, B, T, L, W, x); return 1; }
 int main() {
     std::mt19937 rng(5);
@@ -25,11 +24,11 @@ int main() {
     TableChoice t;
     for (int round = 0; round < 3000; ++round) {
         const int B = draw(1, 70), L = draw(1, 1024), T = draw(1, L < 300 ? L : 300), W = draw(0, 1) ? L : draw(1, L);
-        const int four = groups_needed(L, W, 4), least = 2 * ((B + 7) & ~7) * four <= 256 && four > 0 ? four : groups_needed(L, W, kChunkBlocks);
+        const int least = sweep_groups(B, L, W);
         if (least == 0) continue;
         const int which = round & 1, NB = (L + kBlk - 1) / kBlk, blocks = (W + kBlk - 1) / kBlk;
         const int room = draw(0, 2) ? kMaxGroups : draw(least, kMaxGroups);   // groups a sweep that the workspace has words for
-        make_tables<1>(tables, t, B, T, L, W, least, room, costs, which);
+        make_tables<1>(tables, t, B, T, L, W, least, room, kSweepCosts, which);
         if (t.ntable < 1 || t.ntable > kMostTables || t.most < least || t.most > kMaxGroups || t.least != least) return fail("sizes", B, T, L, W, 0);
         if (t.most > room) return fail("more groups than the workspace has", B, T, L, W, 0);
         offered += t.ntable > 1;
