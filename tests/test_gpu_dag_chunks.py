@@ -8,7 +8,7 @@ import torch
 
 import da_transformer_amd as dagx
 from da_transformer_amd import _native as nat
-from da_transformer_amd.custom_ops.dag_loss import DagLossFunc, _sweep_offsets
+from da_transformer_amd.custom_ops.dag_loss import DagLossFunc, _clean_workspaces, _sweep_offsets
 from oracle import torch_native as tn
 from helpers import random_problem
 from test_gpu_dag import DEV, hip_loss_and_grads, oracle_loss_and_grads, assert_close, RTOL
@@ -52,18 +52,31 @@ def test_edges_of_blocks_chunks_and_windows(B, L, T, translen, dtype, wide):
     assert_close(gl.float(), rgl, RTOL[dtype], "grad_links")
 
 
-@pytest.mark.parametrize("wide", [False, True])
-@pytest.mark.parametrize("B,L,T,shortest,dtype", [
-    # samples of some lengths get more workgroups than those of others; full lengths find no room (20, 24) or do (3, 16)
-    (3, 650, 24, 1, F32), (16, 760, 24, 570, F32), (16, 768, 21, 768, F16), (20, 760, 24, 760, F32), (20, 765, 24, 400, BF16),
-    (24, 768, 24, 768, F32), (5, 1024, 98, 700, F32), (64, 390, 12, 1, F16)])
-def test_batches_whose_samples_get_different_numbers_of_workgroups(B, L, T, shortest, dtype, wide):
-    match, links_sq, ol, tl = random_problem(L + B, B, L, T, dtype=F32, ragged=False)
+# Batches in which samples of some lengths get more workgroups than those of others, with the table of groups that the float32 and the
+# float64 sweeps of a call take, 0: as many for every sample (test_sweep_tables.py works it out from the same lengths).
+TABLE_BATCHES = [
+    # B, L, T, shortest, dtype, tables
+    (3, 650, 24, 1, F32, (2, 2)), (16, 760, 24, 570, F32, (2, 2)), (16, 768, 21, 768, F16, (2, 2)), (20, 760, 24, 760, F32, (1, 1)),
+    (20, 765, 24, 400, BF16, (2, 2)), (24, 768, 24, 768, F32, (0, 0)), (5, 1024, 98, 700, F32, (0, 0)), (64, 390, 12, 1, F16, (0, 1)),
+    (16, 1024, 128, 768, F32, (1, 1)), (16, 1000, 131, 750, F16, (1, 2)), (14, 1010, 130, 760, BF16, (1, 2)), (16, 1024, 130, 1024, F32, (0, 0)),
+    (1, 800, 60, 800, F32, (2, 2)), (2, 523, 104, 400, F32, (2, 2))]
+
+
+def table_lengths(B, L, T, shortest):
     ol = torch.randint(shortest, L + 1, (B,), generator=torch.Generator().manual_seed(B))
+    tl = torch.full((B,), T)
     ol[0] = L
     tl = torch.minimum(tl, ol)
     if B > 4:
         ol[2], tl[3] = 0, T + 1          # samples without a length, among the others
+    return ol, tl
+
+
+@pytest.mark.parametrize("wide", [False, True])
+@pytest.mark.parametrize("B,L,T,shortest,dtype", [batch[:5] for batch in TABLE_BATCHES])
+def test_batches_whose_samples_get_different_numbers_of_workgroups(B, L, T, shortest, dtype, wide):
+    match, links_sq, _, _ = random_problem(L + B, B, L, T, dtype=F32, ragged=False)
+    ol, tl = table_lengths(B, L, T, shortest)
     cols = torch.arange(L).view(1, 1, L) < ol.view(B, 1, 1)
     links_sq = torch.log_softmax(links_sq.masked_fill(~cols, -1e30), -1).masked_fill(~cols | ~torch.isfinite(links_sq), float("-inf"))
     match, links = match.to(dtype), tn.extract_valid_links(links_sq).to(dtype)
@@ -83,6 +96,46 @@ def test_batches_whose_samples_get_different_numbers_of_workgroups(B, L, T, shor
     assert ((loss[good].double() - rloss)[fin].abs() <= 6e-7 * T + 2e-7 * rloss[fin].abs()).all()
     assert_close(gm.float()[good], rgm, RTOL[dtype], "grad_match")
     assert_close(gl.float()[good], rgl, RTOL[dtype], "grad_links")
+
+
+def mixed_lengths():
+    T, L = 130, 1024
+    ol = torch.randint(768, L + 1, (16,), generator=torch.Generator().manual_seed(3))
+    ol[0] = L
+    return T, L, ol
+
+
+@pytest.mark.parametrize("with_grad", [True, False])
+def test_some_samples_of_a_batch_with_tables_go_on_to_the_float64_sweeps(with_grad):
+    """The float32 and the float64 launch of a call have groups, and so a layout of the workspace, of their own; the float64 launch
+    passes over the samples that the float32 launch settled."""
+    T, L, ol = mixed_lengths()
+    B = len(ol)
+    peaked = torch.arange(B) % 3 == 1
+    cols = torch.arange(L).view(1, 1, L) < ol.view(B, 1, 1)
+    gen = torch.Generator().manual_seed(11)
+    sq = torch.randn(B, L, L, generator=gen) * torch.where(peaked, 20.0, 1.0).view(B, 1, 1)
+    sq = tn.restore_valid_links(tn.extract_valid_links(sq))
+    dead = ~(torch.isfinite(sq) & cols)
+    links = tn.extract_valid_links(torch.log_softmax(sq.masked_fill(dead, -1e30), -1).masked_fill(dead, float("-inf")))
+    match = torch.randn(B, T, L, generator=gen) - 2.0
+    tl = torch.full((B,), T)
+    g = torch.linspace(0.5, 2.0, B)
+    rloss, rgm, rgl = oracle_loss_and_grads(match, links, ol, tl, g)
+    assert torch.isfinite(rloss).all()
+    for _ in range(2):
+        if with_grad:
+            loss, gm, gl = hip_loss_and_grads(match, links, ol, tl, g)
+            assert_close(gm, rgm, RTOL[F32], "grad_match")
+            assert_close(gl, rgl, RTOL[F32], "grad_links")
+        else:
+            with torch.no_grad():
+                loss = dagx.dag_loss(match.to(DEV), links.to(DEV), ol.to(DEV), tl.to(DEV)).cpu()
+        flags = DagLossFunc.last_sample_flags.cpu()
+        assert (flags[~peaked] == 0).all() and (flags[peaked] == 2).any(), flags
+        # the float32 sweeps' bound as above; the float64 ones' read-outs agree to 1e-8 of the value and 5e-5
+        assert ((loss.double() - rloss).abs() <= 6e-7 * T + 2e-7 * rloss.abs()).all(), (loss, rloss)
+        assert all(int(ws.count_nonzero()) == 0 for ws in _clean_workspaces.values())
 
 
 @pytest.mark.parametrize("B,L,T,translen,dtype", [

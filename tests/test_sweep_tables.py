@@ -7,6 +7,7 @@ import subprocess
 import pytest
 
 from conftest import ROOT
+from test_gpu_dag_chunks import TABLE_BATCHES, mixed_lengths, table_lengths
 
 PROGRAM = r"""
 #include <cstdio>
@@ -94,12 +95,57 @@ int main() {
 """
 
 
-@pytest.mark.skipif(not os.path.exists("/opt/rocm/bin/hipcc"), reason="no hipcc")
-def test_every_group_has_one_workgroup_whatever_table_is_chosen(tmp_path):
+# What a launch takes, from the lengths alone: its table in float32 and in float64, and the groups of its longest sample.
+CHOICE = r"""
+#include <cstdio>
+#include <vector>
+#include "dag_chunks.h"
+using namespace dagx;
+int main() {
+    static GroupTable tables[kMostTables];
+    int B, T, L;
+    while (std::scanf("%d %d %d", &B, &T, &L) == 3) {
+        std::vector<int> len(B);
+        for (int &n : len) if (std::scanf("%d", &n) != 1) return 1;
+        for (int which = 0; which < 2; ++which) {
+            TableChoice t;
+            make_tables<1>(tables, t, B, T, L, L - 1, sweep_groups(B, L, L - 1), kMaxGroups, kSweepCosts, which);
+            int used = 0;
+            for (int x = t.ntable - 1; x > 0 && used == 0; --x) {
+                int all = 0;
+                for (const int n : len) all += 2 * (int)(t.ngroups[x] >> (4 * ((n >= 1 && n <= L ? (n + kBlk - 1) / kBlk : 1) - 1)) & 15);
+                if (all <= kSweepCus) used = x;
+            }
+            std::printf("%d %d ", used, t.most);
+        }
+        std::printf("\n");
+    }
+}
+"""
+
+
+def _run(program, tmp_path, given=""):
     src, exe = tmp_path / "tables.hip", tmp_path / "tables"
-    src.write_text(PROGRAM)
+    src.write_text(program)
     subprocess.run(["/opt/rocm/bin/hipcc", "--offload-arch=gfx950", "--cuda-host-only", "-O1", "-std=c++17", "-Wno-unused-function",
                     "-I", os.path.join(ROOT, "include"), "-I", os.path.join(ROOT, "da_transformer_amd", "csrc"), str(src), "-o", str(exe)],
                    check=True, capture_output=True)
-    run = subprocess.run([str(exe)], capture_output=True, text=True)
+    run = subprocess.run([str(exe)], capture_output=True, text=True, input=given)
     assert run.returncode == 0, run.stdout
+    return run.stdout
+
+
+@pytest.mark.skipif(not os.path.exists("/opt/rocm/bin/hipcc"), reason="no hipcc")
+def test_every_group_has_one_workgroup_whatever_table_is_chosen(tmp_path):
+    _run(PROGRAM, tmp_path)
+
+
+@pytest.mark.skipif(not os.path.exists("/opt/rocm/bin/hipcc"), reason="no hipcc")
+def test_the_batches_of_the_gpu_tests_take_the_tables_they_are_there_for(tmp_path):
+    batches = [(B, T, L, table_lengths(B, L, T, shortest)[0].tolist()) for B, L, T, shortest, _, _ in TABLE_BATCHES]
+    batches += [(len(ol), T, L, ol.tolist()) for T, L, ol in [mixed_lengths()]]
+    given = "\n".join(" ".join(map(str, [B, T, L] + lengths)) for B, T, L, lengths in batches)
+    got = [[int(n) for n in line.split()] for line in _run(CHOICE, tmp_path, given).splitlines()]
+    assert [(x[0], x[2]) for x in got[:-1]] == [batch[5] for batch in TABLE_BATCHES]
+    table32, most32, table64, most64 = got[-1]
+    assert table32 > 0 and table64 > 0 and most32 != most64    # the two launches of a call lay the workspace out differently
