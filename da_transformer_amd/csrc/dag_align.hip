@@ -113,7 +113,7 @@ __device__ __forceinline__ void align_one_sample(const AlignArgs &a, const int b
 
 template <typename TM, typename TL, int NT, bool TRACE_LDS>
 __global__ __launch_bounds__(NT) void dag_align_kernel(AlignArgs a) {
-    extern __shared__ float lds_a[];
+    extern __shared__ __align__(16) float lds_a[];
     align_one_sample<TM, TL, NT, TRACE_LDS>(a, blockIdx.x, lds_a);
 }
 
