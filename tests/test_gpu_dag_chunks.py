@@ -165,6 +165,29 @@ def test_alignment_at_edges_of_blocks_chunks_and_windows(B, L, T, translen, dtyp
     assert torch.equal(got[some], want)
 
 
+@pytest.mark.parametrize("B,L,T,translen,dtype,first", [
+    (1, 4, 4, 1, F32, 0), (2, 4, 4, 3, F16, 1), (3, 5, 5, 1, F16, 3), (2, 6, 6, 2, F32, 2), (2, 63, 32, 2, F16, 1), (3, 64, 64, 1, F32, 1),
+    (2, 65, 40, 3, BF16, 3), (1, 66, 66, 1, F16, 0), (3, 127, 64, 3, F32, 3), (2, 129, 129, 1, BF16, 1), (2, 130, 70, 2, F32, 2),
+    (2, 195, 100, 2, F16, 3), (1, 321, 200, 3, F32, 1)])
+def test_staged_walks_at_the_ends_of_a_sample_and_with_windows_of_one_to_three(B, L, T, translen, dtype, first):
+    """The walk stages transitions four neighbouring elements a load.  Loads that would leave the sample are moved inside; what stands
+    in front of the tensor, behind it and in the samples beside it, here better than any transition, is nobody's successor."""
+    gen = torch.Generator().manual_seed(L + T)
+    links = (torch.randn(B, L, translen, generator=gen) * 4).round() / 4 - 2.0
+    node = torch.arange(L).view(1, L, 1)
+    links = links.masked_fill(node + torch.arange(1, translen + 1) >= L, 40.0 if translen > 1 else float("-inf"))
+    match = (torch.randn(B, T, L, generator=gen) * 4).round() / 4
+    ol = torch.full((B,), min(L, (T - 1) * translen + 1))
+    tl = torch.full((B,), T)
+    links, match = links.to(dtype), match.to(dtype)
+    room = torch.full((first + links.numel() + 8,), 40.0, dtype=dtype, device=DEV)
+    room[first:first + links.numel()] = links.to(DEV).reshape(-1)
+    got = dagx.dag_best_alignment(match.to(DEV), room[first:first + links.numel()].view(links.shape), ol.to(DEV), tl.to(DEV)).cpu()
+    inside = links.float().masked_fill(node + torch.arange(1, translen + 1) >= ol.view(B, 1, 1), float("-inf"))
+    want = tn.torch_dag_best_alignment(match.float(), tn.restore_valid_links(inside), ol, tl)
+    assert torch.equal(got, want)
+
+
 @pytest.mark.parametrize("wide", [False, True])
 @pytest.mark.parametrize("B,L,T,translen,score", [
     (2, 640, 41, 639, 0.0),        # hundreds of predecessors with transitions of 1 feed every cell: sums of up to 2^9 cells
