@@ -316,7 +316,9 @@ inline const ChunkPlan<N> &plan_for_bound(int translen, int c, int nb, int bound
     for (n = 0; n < u && plan.gtab[which][nb][n + 1] > plan.gtab[which][nb][n];) ++n;
     return plan;
 }
-// Whether two sweeps of samples of seven eighths of L, with the bound that the longest keeps with c groups, would all find a CU.
+// Whether two sweeps of samples of seven eighths of L, with the bound that the longest keeps with c groups, would all find a CU.  (Where
+// they would, most batches of ragged samples do; where all lengths are L and do not, the look at the lengths costs a few us: B = 20, L = 900,
+// T = 180 332 -> 336, B = 17, L = 897 325 -> 328; of lengths from three quarters on 283 -> 230, from a third on 249 -> 227.)
 template <int SPACING, int N>
 inline bool typical_fits(int B, int L, int translen, int c, const ChunkCosts (&costs)[N], int which) {
     int n;
@@ -325,7 +327,8 @@ inline bool typical_fits(int B, int L, int translen, int c, const ChunkCosts (&c
 }
 inline bool may_choose(int B, int L) { return B <= kMostForTables && L > 4 * kBlk; }
 // A table is offered where the longest sample's stages (one a chunk, one a block, one and a half a hand-over) take at most 97 %
-// of what they take in `least` groups (L = 512, T = 170 in four groups, 97 to 99 % depending on T, 156 to 160 us for 156), and
+// of what they take in `least` groups and are shorter by a twelfth of a walk (with a bound of 48 already, groups for one of 45, a
+// walk alone, lose: B = 32, L = 512, T = 256 216 -> 227 us, T = 170 158 -> 165; B = 13, L = 458, T = 157 143.5 -> 149), and
 // where two sweeps of samples of seven eighths of L would all find a CU.  room: the most groups a sweep that the caller's workspace has
 // pipeline words for; with `least` there is only table 0.
 template <int SPACING, int N>
@@ -341,11 +344,12 @@ inline void make_tables(GroupTable (&tables)[kMostTables], TableChoice &o, int B
     for (int nb = 0; nb <= kMaxBlocksFast; ++nb) copy_row(tables[0], nb, plan_of(least));
     if (!may_choose(B, L) || room <= least) return;
     auto stages2 = [&](const int c) { return 2 * (NC + NB) + 3 * (c - 1); };
-    int best = plan_of(least).busiest[which][NB];
-    const long long now = (long long)best * stages2(least);
+    const int first = plan_of(least).busiest[which][NB];
+    int best = first;
+    const long long now = (long long)first * stages2(least);
     for (int c = least + 1; c <= kMaxGroups && c <= NB && o.ntable < kMostTables; ++c) {
         const int bound = plan_of(c).busiest[which][NB];
-        if (bound >= best || 100 * (long long)bound * stages2(c) > 97 * now) continue;
+        if (bound >= best || 12 * (first - bound) < costs[which].walk || 100 * (long long)bound * stages2(c) > 97 * now) continue;
         GroupTable &table = tables[o.ntable];
         unsigned long long ngroups = 0;
         int most = 1;

@@ -21,6 +21,14 @@ int main() {
     std::mt19937 rng(5);
     auto draw = [&](int lo, int hi) { return lo + (int)(rng() % (unsigned)(hi - lo + 1)); };
     int offered = 0, chosen = 0;
+    const auto tables_of = [](const int B, const int T, const int L, const int which) {
+        static GroupTable some[kMostTables];
+        TableChoice choice;
+        make_tables<1>(some, choice, B, T, L, L - 1, sweep_groups(B, L, L - 1), kMaxGroups, kSweepCosts, which);
+        return choice.ntable;
+    };
+    // a bound that is hardly above a walk's own length is left alone
+    if (tables_of(32, 256, 512, 0) != 1 || tables_of(13, 157, 458, 0) != 1 || tables_of(16, 256, 1024, 0) == 1 || tables_of(32, 162, 554, 0) == 1) return fail("offers", 32, 256, 512, 511, 0);
     static GroupTable tables[kMostTables];
     TableChoice t;
     for (int round = 0; round < 3000; ++round) {
