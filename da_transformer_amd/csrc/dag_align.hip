@@ -247,9 +247,8 @@ struct AlignTileArgs {
 //
 // SPACING (dag_chunks.h): a tile is nearly as much work as the walk here, so that where the walk bounds the stages and SIMDs
 // have time to spare -- small graphs, or hardly more than one block to a group -- two stages a block are shorter
-// (alignment with SPACING 1 and 2: B = 64, L = 256, T = 64 91 and 78 us; B = 64, L = 384, T = 48 91 and 86; B = 16, L = 400,
-// T = 50 99 and 93); where the tiles bound them every stage more costs (B = 64, L = 512, T = 64 128 and 137; B = 16, L = 1024,
-// T = 256 445 and 476).
+// (alignment with SPACING 1 and 2: B = 64, L = 256, T = 64 83 and 75 us; B = 40, L = 400, T = 60 99 and 96; B = 16, L = 512,
+// T = 128 167.5 and 156); where the tiles bound them every stage more costs (B = 64, L = 512, T = 64 116 and 125).
 template <typename TM, typename TL, int SPACING>
 __global__ __launch_bounds__(kTileWaves * kWave) void dag_align_chunks_kernel(AlignTileArgs a) {
     extern __shared__ __align__(16) float lds_raw[];
@@ -1007,7 +1006,7 @@ struct alignas(16) WalkStage {
 constexpr size_t kWalkLds = 2 * sizeof(WalkStage);
 
 // Four neighbouring elements a lane: a CU takes one vector-memory instruction per 26 cycles whatever its width, and with one element
-// a lane a block was 255 of them; now it is 75.  (Backtrack at B=64 L=512 T=64 24 -> 22.4 us, with the walker's priority; at
+// a lane a block was 255 of them; now it is 90.  (Backtrack at B=64 L=512 T=64 24 -> 22.4 us, with the walker's priority; at
 // B=16 L=1024 T=256, where a block of nodes is sixteen steps, the steps bound it: 65 us before and after.)
 template <typename TL, int NT>
 __device__ __forceinline__ void stage_walk(WalkStage &w, const float *A, const unsigned char *srcblk, int spitch, const TL *links,

@@ -375,10 +375,11 @@ __device__ __host__ __forceinline__ void place_of_ticket(int r, int n, int ndir,
     else { r -= ndir * full; rank = full + r % rest; slot = r / rest; }
 }
 
-// Workgroups per sweep (two sweeps a sample): as few as hold the tiles, but with at most four blocks each, one walk to a
-// SIMD, where the device has a CU for every workgroup.  Forward with up to eight -> up to four blocks: B = 40, L = 328,
-// T = 41 67 -> 61 us; B = 16, L = 512, T = 64 102 -> 97.5; B = 64 and transitions of at most 32 88 -> 79; B = 16,
-// L = 1024 and transitions of at most 64 122 -> 104.  More groups than that: see make_tables.
+// Workgroups per sweep (two sweeps a sample) in table 0: as few as hold the tiles, but with at most four blocks each, one walk to a
+// SIMD, where the device has a CU for every workgroup (with the plans before there were tables, forward, up to eight -> up to four
+// blocks: B = 40, L = 328, T = 41 67 -> 61 us; B = 16, L = 512, T = 64 102 -> 97.5; B = 64 and transitions of at most 32 88 -> 79; B = 16,
+// L = 1024 and transitions of at most 64 122 -> 104).  Where a table may have more groups the two come out the same now (62.6 and 62.1;
+// 89.6 and 90.2; 82.7 and 82.2; T = 128 144.8 and 144.4): the line decides for workspaces that have room for table 0 alone.
 inline int sweep_groups(int B, int L, int translen) {
     const int C = groups_needed(L, translen, 4), sweeps = 2 * ((B + 7) & ~7);
     return (long long)sweeps * C <= kSweepCus && C > 0 ? C : groups_needed(L, translen, kChunkBlocks);
@@ -393,16 +394,17 @@ constexpr ChunkCosts kSweepCosts[2] = {{45, 9, 12, 70}, {85, 25, 16, 80}};
 // ---- the alignment's rules ----
 // Whether the sweep goes in chunks of four steps.  They cost T / 4 stages and one or two more for every block of nodes, single
 // steps T of two fifths of that: even at about six steps for every block of nodes and eight more (alignment, chunks and
-// steps: B = 64, L = 512, T = 64 129 and 140 us; B = 28, L = 450, T = 50 108 and 103; B = 20, L = 1000, T = 128 297 and 328; B = 1,
-// L = 900, T = 70 196 and 179; B = 48, L = 350, T = 40 81 and 76; B = 8, L = 128, T = 32 38 and 44; B = 1, L = 115, T = 15 29 and 27).
+// steps: B = 64, L = 512, T = 64 114 and 131 us; B = 28, L = 450, T = 50 99.4 and 98.0, T = 56 103 and 106; B = 20, L = 1000, T = 128 277 and
+// 312; B = 1, L = 900, T = 70 190 and 178, T = 98 222 and 223; B = 48, L = 350, T = 40 73.2 and 73.5; B = 8, L = 128, T = 32 39 and 44;
+// B = 1, L = 115, T = 15 30 and 27).
 inline bool align_in_chunks(int B, int T, int L, int translen) {
     return T >= 6 * ((L + kBlk - 1) / kBlk) + 8 && (int64_t)B * L * translen >= 4;   // (the chunked kernel's tiles are loaded four elements at a time)
 }
 
 // Workgroups per sweep.  In chunks: from four position blocks on as many as the device has room for (one per CU) up to one
 // for each block, at most ten.  (Fewer tiles a SIMD, against more hand-overs: as many as hold the tiles -> this, alignment of
-// B = 16, L = 1024, T = 256 484 -> 445 us; B = 4, L = 700, T = 100 211 -> 183; B = 64, L = 320, T = 48 83 -> 79; B = 64, L = 256,
-// T = 64 92 -> 80.)  Step by step: twice as many as hold the tiles where there is room and the graph has at least four
+// B = 16, L = 1024, T = 256 504 -> 423 us; B = 16, L = 768, T = 192 365 -> 267; B = 4, L = 700, T = 110 250 -> 178; B = 64, L = 320,
+// T = 48 90 -> 72; B = 64, L = 256, T = 64 91 -> 75.)  Step by step: twice as many as hold the tiles where there is room and the graph has at least four
 // blocks (5 to 13 %; more lose); where that exceeds what the kernel supports, ten when they fit.
 inline int align_groups(int B, int T, int L, int translen) {
     const int NB = (L + kBlk - 1) / kBlk, B8 = (B + 7) & ~7;
@@ -419,9 +421,9 @@ inline int align_groups(int B, int T, int L, int translen) {
 }
 // Stages from a block's walk of a chunk to the next block's: see dag_align_chunks_kernel.
 inline int align_spacing(int NB, int C) { return NB <= 5 || (NB <= 8 && 2 * NB <= 3 * C) ? 2 : 1; }
-// Found by timing calls under some twenty sets, from the pieces' own times {62 or 36, 27, 4, 75} on (us): B = 64, L = 512, T = 64
+// The alignment's costs, found by timing calls under some twenty sets, from the pieces' own times {62 or 36, 27, 4, 75} on (us): B = 64, L = 512, T = 64
 // 120.3 -> 116.6, B = 16, L = 768, T = 192 276.5 -> 268, B = 4, L = 700, T = 110 187 -> 179, B = 64, L = 256, T = 64
-// (SPACING 2) 79.0 -> 76.1, B = 40, L = 400, T = 60 (SPACING 2) 99.5 -> 95.2; the others the same.
+// (SPACING 2) 79.0 -> 76.1, B = 40, L = 400, T = 60 (SPACING 2) 99.5 -> 95.2.  (Windows of one to three blocks: see ChunkPlan.)
 template <int SPACING>
 constexpr ChunkCosts kAlignCosts[1] = {SPACING == 1 ? ChunkCosts{62, 27, 2, 65} : ChunkCosts{36, 27, 4, 55}};
 
