@@ -99,7 +99,7 @@ int main() {
     // groupings as good as each other for the busiest SIMD: more even ones, where they gain more than their hand-overs take
     if (!groups_are<2>(kAlignCosts<2>[0], 1, 8, 8, {2, 2, 2, 2}) || !groups_are<1>(kAlignCosts<1>[0], 3, 10, 13, {3, 2, 2, 2, 2, 2}) ||
         !groups_are<1>(kSweepCosts[0], 5, 2, 5, {3, 2}) || !groups_are<1>(kAlignCosts<1>[0], 9, 9, 9, {4, 2, 1, 1, 1}) ||
-        !groups_are<2>(kAlignCosts<2>[0], 2, 8, 8, {3, 2, 2, 1})) return 1;
+        !groups_are<2>(kAlignCosts<2>[0], 2, 8, 8, {3, 2, 2, 1}) || !groups_are<1>(kAlignCosts<1>[0], 2, 2, 14, {8, 6})) return 1;
     return check<1>(kSweepCosts) || check<1>(kAlignCosts<1>) || check<2>(kAlignCosts<2>) || alignment();
 }
 """
