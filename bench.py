@@ -550,8 +550,8 @@ def main():
         flags = torch.empty(B, dtype=torch.int32, device=dev)
         ms3 = nat.strides3(match)
         mdt, ldt = nat.dtype_code(match), nat.dtype_code(links)
-        nb_f = nat.workspace_bytes(nat.OP_LOSS_FWD, B, T, L, translen)
-        ws = torch.zeros(max(nb_f, 4), dtype=torch.uint8, device=dev)   # the forward wants it zero and leaves it zero
+        nb_f = max(8192, nat.workspace_bytes(nat.OP_LOSS_FWD, B, T, L, translen))   # (8192: see include/dagx.h)
+        ws = torch.zeros(nb_f, dtype=torch.uint8, device=dev)   # the forward wants it zero and leaves it zero
 
         def fwd(need_grad=1):
             nat.check(lib.dagx_loss_fwd(match.data_ptr(), mdt, ms3, links.data_ptr(), ldt, ol.data_ptr(), tl.data_ptr(),
