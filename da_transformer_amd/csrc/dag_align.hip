@@ -1258,7 +1258,7 @@ static int prepare_align_chunks() {
 }
 template <typename TM, typename TL, int SPACING>
 static int launch_align_chunks(AlignTileArgs &ta, const char *who, hipStream_t st) {
-    ta.plan = chunk_plan<SPACING>(ta.translen, ta.C, kAlignCosts<SPACING>);
+    ta.plan = chunk_plan<SPACING>(ta.translen, ta.C, align_costs<SPACING>(ta.translen));
     if (int rc = prepare_align_chunks<TM, TL, SPACING>()) return rc;
     hipLaunchKernelGGL((dag_align_chunks_kernel<TM, TL, SPACING>), dim3(((ta.B + 7) & ~7) * ta.C), dim3(kTileWaves * kWave), kChunkLdsBytes, st, ta);
     return check_launch(who);

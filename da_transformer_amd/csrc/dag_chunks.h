@@ -422,12 +422,17 @@ inline int align_groups(int B, int T, int L, int translen) {
 // Stages from a block's walk of a chunk to the next block's: see dag_align_chunks_kernel.
 inline int align_spacing(int NB, int C) { return NB <= 5 || (NB <= 8 && 2 * NB <= 3 * C) ? 2 : 1; }
 // The alignment's costs, found by timing calls under some twenty sets, from the pieces' own times {62 or 36, 27, 4, 75} on (us): B = 64,
-// L = 512, T = 64 119.8 -> 115.5, B = 16, L = 768, T = 192 278 -> 268, B = 4, L = 700, T = 110 187 -> 177, B = 64, L = 256, T = 64
-// (SPACING 2) 79.0 -> 76.1, B = 40, L = 400, T = 60 (SPACING 2) 99.5 -> 95.2.  A fetched block at 2 instead of 4 changes groupings alone,
-// and mostly for the worse: B = 91, L = 896, T = 358, transitions of at most 65 608 us for 560; B = 74, L = 468, T = 58, at most 139 106 for
-// 101; B = 14, L = 955, T = 238, at most 113 303 for 289; but B = 2, L = 846, T = 338 430 for 440, B = 67, L = 718, T = 89 221 for 229.
+// L = 512, T = 64 119.8 -> 115.2, B = 16, L = 768, T = 192 278 -> 268, B = 4, L = 700, T = 110 187 -> 177, B = 64, L = 256, T = 64
+// (SPACING 2) 79.0 -> 76.1, B = 40, L = 400, T = 60 (SPACING 2) 99.5 -> 95.2.  With SPACING 1 a fetched block weighs 2 where windows
+// span more than three blocks, so that a group fetches many and their waits overlap, else its own time, 4.  With 4 for all: B = 42, L = 880,
+// T = 176 444 us for 423, B = 9, L = 876, T = 175 293 for 285, B = 2, L = 846, T = 338 440 for 429 (but B = 41, L = 944, T = 283 525 for 539);
+// with 2 for all: B = 91, L = 896, T = 358, transitions of at most 65 607 for 559, B = 74, L = 468, T = 58, at most 139 106 for 101.5,
+// B = 14, L = 955, T = 238, at most 113 302 for 289.
 template <int SPACING>
-constexpr ChunkCosts kAlignCosts[1] = {SPACING == 1 ? ChunkCosts{62, 27, 4, 65} : ChunkCosts{36, 27, 4, 55}};
+constexpr ChunkCosts kAlignCosts[2][1] = {{SPACING == 1 ? ChunkCosts{62, 27, 2, 65} : ChunkCosts{36, 27, 4, 55}},
+                                          {SPACING == 1 ? ChunkCosts{62, 27, 4, 65} : ChunkCosts{36, 27, 4, 55}}};
+template <int SPACING>
+inline const ChunkCosts (&align_costs(int translen))[1] { return kAlignCosts<SPACING>[window_blocks(translen) <= 3]; }
 
 // LDS of a group, in dwords: cells of four steps in the order of the table, results of a wave's tiles that lead to one block.
 struct AlignLds {

@@ -15,11 +15,12 @@ PROGRAM = r"""
 #include <vector>
 #include "dag_chunks.h"
 using namespace dagx;
-template <int SPACING, int N>
-static int check(const ChunkCosts (&costs)[N]) {
+template <int SPACING, int N, typename COSTS>
+static int check(COSTS costs_of) {
     // batches of changing size: every number of workgroups in turn, windows of every number of blocks
     for (int round = 0; round < 2; ++round)
         for (int W = 1; W <= kMaxBlocksFast; ++W) {
+            const ChunkCosts (&costs)[N] = costs_of(64 * W);
             const ChunkPlan<N> *kept[12] = {};
             for (int C = 1; C <= 11; ++C) kept[C] = &chunk_plan<SPACING>(64 * W - 1, C, costs);
             for (int C = 1; C <= 11; ++C) {
@@ -36,7 +37,7 @@ static int check(const ChunkCosts (&costs)[N]) {
                 if (kept[C] != &chunk_plan<SPACING>(64 * W, C, costs)) { std::printf("W=%d C=%d: made again\n", W, C); return 1; }
         }
     // a window longer than any graph the sweeps take is that of the longest
-    return &chunk_plan<SPACING>(8192, 4, costs) != &chunk_plan<SPACING>(64 * kMaxBlocksFast, 4, costs);
+    return &chunk_plan<SPACING>(8192, 4, costs_of(8192)) != &chunk_plan<SPACING>(64 * kMaxBlocksFast, 4, costs_of(8192));
 }
 // blocks of the groups of a graph of nb blocks
 template <int SPACING>
@@ -56,7 +57,7 @@ static bool groups_are(const ChunkCosts &cost, int W, int C, int nb, std::vector
 // does not sends its samples to the one-workgroup redo.
 template <int SPACING>
 static bool alignment_fits(int B, int T, int L, int translen, int C) {
-    const ChunkPlan<1> &plan = chunk_plan<SPACING>(translen, C, kAlignCosts<SPACING>);
+    const ChunkPlan<1> &plan = chunk_plan<SPACING>(translen, C, align_costs<SPACING>(translen));
     const int W = (translen + kBlk - 1) / kBlk;
     for (int nb = 1; nb <= (L + kBlk - 1) / kBlk; ++nb) {
         const unsigned char *g = plan.gtab[0][nb];
@@ -97,10 +98,11 @@ static int alignment() {
 }
 int main() {
     // groupings as good as each other for the busiest SIMD: more even ones, where they gain more than their hand-overs take
-    if (!groups_are<2>(kAlignCosts<2>[0], 1, 8, 8, {2, 2, 2, 2}) || !groups_are<1>(kAlignCosts<1>[0], 3, 10, 13, {3, 2, 2, 2, 2, 2}) ||
-        !groups_are<1>(kSweepCosts[0], 5, 2, 5, {3, 2}) || !groups_are<1>(kAlignCosts<1>[0], 9, 9, 9, {4, 2, 1, 1, 1}) ||
-        !groups_are<2>(kAlignCosts<2>[0], 2, 8, 8, {3, 2, 2, 1}) || !groups_are<1>(kAlignCosts<1>[0], 2, 2, 14, {8, 6})) return 1;
-    return check<1>(kSweepCosts) || check<1>(kAlignCosts<1>) || check<2>(kAlignCosts<2>) || alignment();
+    if (!groups_are<2>(align_costs<2>(64)[0], 1, 8, 8, {2, 2, 2, 2}) || !groups_are<1>(align_costs<1>(192)[0], 3, 10, 13, {3, 2, 2, 2, 2, 2}) ||
+        !groups_are<1>(kSweepCosts[0], 5, 2, 5, {3, 2}) || !groups_are<1>(align_costs<1>(576)[0], 9, 9, 9, {4, 2, 1, 1, 1}) ||
+        !groups_are<2>(align_costs<2>(128)[0], 2, 8, 8, {3, 2, 2, 1}) || !groups_are<1>(align_costs<1>(128)[0], 2, 2, 14, {8, 6}) ||
+        !groups_are<1>(align_costs<1>(896)[0], 14, 10, 14, {4, 2, 1, 1, 1, 1, 1, 1, 1, 1})) return 1;
+    return check<1, 2>([](int) -> const ChunkCosts (&)[2] { return kSweepCosts; }) || check<1, 1>(align_costs<1>) || check<2, 1>(align_costs<2>) || alignment();
 }
 """
 
