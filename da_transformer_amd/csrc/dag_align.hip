@@ -122,49 +122,43 @@ __global__ __launch_bounds__(NT) void dag_align_kernel(AlignArgs a) {
 // Tile-resident max-plus sweep
 // ================================================================================================
 
-// b0 = max(b0, max_{r<8} (a0[lane R0 + r of this 16-lane row] + p[r])), b1 likewise with a1, R1 and q: per pair of rows two
-// sums and one three-way maximum (a maximum does not round: the result is that of one by one, bit for bit).  Two chains side
-// by side, because a wave waits 8 cycles for a result it needs at once: one alone takes 7.7 cycles an instruction.
-template <int R0, int R1>
-__device__ __forceinline__ void maxplus8x2(float &b0, float a0, const float *p, float &b1, float a1, const float *q) {
-    static_assert((R0 == 0 || R0 == 8) && (R1 == 0 || R1 == 8), "");
-    float t0, t1, t2, t3;
-#define DAGX_SUMS(X, Y, P0, P1, Q0, Q1, N0, N1) \
-        "v_add_f32_dpp %2, %6, " P0 " row_newbcast:" X " row_mask:0xf bank_mask:0xf\n\t" \
-        "v_add_f32_dpp %3, %6, " P1 " row_newbcast:" Y " row_mask:0xf bank_mask:0xf\n\t" \
-        "v_add_f32_dpp %4, %7, " Q0 " row_newbcast:" N0 " row_mask:0xf bank_mask:0xf\n\t" \
-        "v_add_f32_dpp %5, %7, " Q1 " row_newbcast:" N1 " row_mask:0xf bank_mask:0xf\n\t" \
-        "v_max3_f32 %0, %0, %2, %3\n\t" \
-        "v_max3_f32 %1, %1, %4, %5\n\t"
-#define DAGX_ROWS8(A0, A1, A2, A3, A4, A5, A6, A7, B0, B1, B2, B3, B4, B5, B6, B7) \
-    asm("s_nop 1\n\t" \
-        DAGX_SUMS(A0, A1, "%8", "%9", "%16", "%17", B0, B1) \
-        DAGX_SUMS(A2, A3, "%10", "%11", "%18", "%19", B2, B3) \
-        DAGX_SUMS(A4, A5, "%12", "%13", "%20", "%21", B4, B5) \
-        DAGX_SUMS(A6, A7, "%14", "%15", "%22", "%23", B6, B7) \
-        : "+v"(b0), "+v"(b1), "=&v"(t0), "=&v"(t1), "=&v"(t2), "=&v"(t3) \
-        : "v"(a0), "v"(a1), "v"(p[0]), "v"(p[1]), "v"(p[2]), "v"(p[3]), "v"(p[4]), "v"(p[5]), "v"(p[6]), "v"(p[7]), \
-          "v"(q[0]), "v"(q[1]), "v"(q[2]), "v"(q[3]), "v"(q[4]), "v"(q[5]), "v"(q[6]), "v"(q[7]))
-    if constexpr (R0 == 0 && R1 == 0) DAGX_ROWS8("0", "1", "2", "3", "4", "5", "6", "7", "0", "1", "2", "3", "4", "5", "6", "7");
-    else if constexpr (R0 == 8 && R1 == 8) DAGX_ROWS8("8", "9", "10", "11", "12", "13", "14", "15", "8", "9", "10", "11", "12", "13", "14", "15");
-    else if constexpr (R0 == 0) DAGX_ROWS8("0", "1", "2", "3", "4", "5", "6", "7", "8", "9", "10", "11", "12", "13", "14", "15");
-    else DAGX_ROWS8("8", "9", "10", "11", "12", "13", "14", "15", "0", "1", "2", "3", "4", "5", "6", "7");
-#undef DAGX_ROWS8
-#undef DAGX_SUMS
+// The sums of max-plus on the matrix cores: v_mfma_f32_4x4x1_16b with a second operand of ones and the tile's registers as the
+// third is cells[row] + P[row][lane] for four rows, one rounding each (1 * x is exact: the bits of v_add_f32, subnormals
+// and infinities among them).  256 sums take 8.2 cycles of a SIMD and four v_add_f32_dpp 18; the maxima, a three-way one for two
+// sums at 4.5 cycles, are all that vector instructions have left to do.  A change between matrix and vector instructions costs
+// a SIMD about 6.5 cycles, hence four of the former and eight of the latter at a time, sixteen registers of sums (one at a time 655, eight
+// at a time 487, with sixteen registers more).  Four steps of a tile, ns, on a wave alone and on one of two that share a SIMD:
+// 540 and 518, in two DPP sums and a maximum for every two rows 942 and 766.
+//
+// d = cells[4 ABID + i] + t.p[ROW + i] for i < 4; CBSZ 4: the cells of all 64 lanes are candidates, 3: those of a lane's own half
+template <int CBSZ, int ABID, int ROW>
+__device__ __forceinline__ f32x4 four_sums(const Tile &t, float cells) {
+    return __builtin_amdgcn_mfma_f32_4x4x1f32(cells, 1.f, f32x4{t.p[ROW], t.p[ROW + 1], t.p[ROW + 2], t.p[ROW + 3]}, CBSZ, ABID, 0);
 }
+// (a maximum does not round: neither three-way ones nor the order change anything)
+__device__ __forceinline__ void raise(float &b0, float &b1, f32x4 d) {
+    b0 = fmaxf(fmaxf(d[0], d[1]), b0);
+    b1 = fmaxf(fmaxf(d[2], d[3]), b1);
+}
+// (batches stay as they are written)
+__device__ __forceinline__ void batch_end() { __builtin_amdgcn_sched_barrier(0); }
 
-// out[k] = max_{r<64} (cells[k][r] + tile.p[r]) for two steps; `cells`: this lane's place lane & 15 in the first of them
-__device__ __forceinline__ void tile_maxplus2(const Tile &t, const float *cells, float &out0, float &out1) {
-    float b0 = DAGX_NEG_INF, b1 = DAGX_NEG_INF;
-    float a0[4], a1[4];
-#pragma unroll
-    for (int q = 0; q < 4; ++q) { a0[q] = cells[16 * q]; a1[q] = cells[kBlk + 16 * q]; }
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-        maxplus8x2<0, 0>(b0, a0[q], t.p + 16 * q, b1, a1[q], t.p + 16 * q);
-        maxplus8x2<8, 8>(b0, a0[q], t.p + 16 * q + 8, b1, a1[q], t.p + 16 * q + 8);
-    }
-    out0 = b0; out1 = b1;
+// max_{r<64} (cells[r] + tile.p[r]) for two steps; lane r holds cells[r]
+__device__ __forceinline__ void tile_maxplus2(const Tile &t, float x, float y, float &out0, float &out1) {
+    float b0 = DAGX_NEG_INF, b1 = DAGX_NEG_INF, c0 = DAGX_NEG_INF, c1 = DAGX_NEG_INF;
+    auto rows8 = [&](auto at) __attribute__((always_inline)) {
+        constexpr int K = decltype(at)::value;
+        const f32x4 d0 = four_sums<4, K, 4 * K>(t, x), d1 = four_sums<4, K, 4 * K>(t, y);
+        const f32x4 d2 = four_sums<4, K + 1, 4 * K + 4>(t, x), d3 = four_sums<4, K + 1, 4 * K + 4>(t, y);
+        batch_end();
+        raise(b0, b1, d0); raise(c0, c1, d1); raise(b0, b1, d2); raise(c0, c1, d3);
+        batch_end();
+    };
+    rows8(std::integral_constant<int, 0>{}); rows8(std::integral_constant<int, 2>{});
+    rows8(std::integral_constant<int, 4>{}); rows8(std::integral_constant<int, 6>{});
+    rows8(std::integral_constant<int, 8>{}); rows8(std::integral_constant<int, 10>{});
+    rows8(std::integral_constant<int, 12>{}); rows8(std::integral_constant<int, 14>{});
+    out0 = fmaxf(b0, b1); out1 = fmaxf(c0, c1);
 }
 
 // {x, y} -> x: rows {x0 y0 x2 y2} of sixteen lanes, y: rows {x1 y1 x3 y3}
@@ -173,20 +167,28 @@ __device__ __forceinline__ void swap_rows(float &x, float &y) {
     const unsigned a = s[0], b = s[1];
     x = __builtin_bit_cast(float, a); y = __builtin_bit_cast(float, b);
 }
+// b0, b1 raised by sixteen rows of one step
+template <int CBSZ, int ABID, int ROW>
+__device__ __forceinline__ void rows16(const Tile &t, float cells, float &b0, float &b1) {
+    const f32x4 d0 = four_sums<CBSZ, ABID, ROW>(t, cells), d1 = four_sums<CBSZ, ABID + 1, ROW + 4>(t, cells);
+    const f32x4 d2 = four_sums<CBSZ, ABID + 2, ROW + 8>(t, cells), d3 = four_sums<CBSZ, ABID + 3, ROW + 12>(t, cells);
+    batch_end();
+    raise(b0, b1, d0); raise(b0, b1, d1); raise(b0, b1, d2); raise(b0, b1, d3);
+    batch_end();
+}
 // max_i (a[i] + P[i][lane]) over a triangle as fold_triangle leaves it; `upper`: lanes 32..63
 __device__ __forceinline__ float triangle_maxplus(const Tile &t, float a, bool upper) {
-    float even = a, odd = a;
-    swap_rows(even, odd);                      // rows {0,0,2,2} and {1,1,3,3} of a
-    float crossed = odd, rest = even;
-    swap_halves(crossed, rest);                // rows {1,1,0,0}
-    float b0 = DAGX_NEG_INF, b1 = DAGX_NEG_INF, b2 = DAGX_NEG_INF;
-    maxplus8x2<0, 0>(b2, crossed, t.p + 32, b0, even, t.p);
-    maxplus8x2<8, 8>(b2, crossed, t.p + 40, b0, even, t.p + 8);
-    float other = b2;
-    swap_halves(b2, other);                    // (the square's two halves, for the upper lanes)
-    maxplus8x2<0, 8>(b0, odd, t.p + 16, b1, odd, t.p + 24);
-    b2 = fmaxf(b2, other);
-    return fmaxf(fmaxf(b0, b1), upper ? b2 : DAGX_NEG_INF);
+    float even = a, crossed = a;
+    swap_rows(even, crossed);                  // rows {0,0,2,2} and {1,1,3,3} of a
+    float b0 = DAGX_NEG_INF, b1 = DAGX_NEG_INF, c0 = DAGX_NEG_INF, c1 = DAGX_NEG_INF;
+    swap_halves(crossed, even);                // rows {1,1,0,0}
+    rows16<3, 0, 32>(t, crossed, c0, c1);
+    float other = fmaxf(c0, c1), square = other;
+    rows16<3, 0, 0>(t, a, b0, b1);
+    swap_halves(square, other);                // (the square's two halves, for the upper lanes)
+    rows16<3, 4, 16>(t, a, b0, b1);
+    square = fmaxf(square, other);
+    return fmaxf(fmaxf(b0, b1), upper ? square : DAGX_NEG_INF);
 }
 
 // bytes per row of the source-block table (rows padded to 16 bytes)
@@ -394,12 +396,15 @@ __global__ __launch_bounds__(kTileWaves * kWave) void dag_align_chunks_kernel(Al
 #pragma unroll
             for (int k = 0; k < kChunk; ++k) mt[k] = to_float(raw[k]);
         };
-        // a tile's best of four steps into the best so far (cells of four steps, 64 each)
+        // a tile's best of four steps into the best so far (this lane's place in the cells of four steps, 64 each)
         auto take = [&](const Tile &tile, const float *cells, const int I, float (&best)[kChunk], int (&from)[kChunk]) __attribute__((always_inline)) {
+            float cell[kChunk];
+#pragma unroll
+            for (int k = 0; k < kChunk; ++k) cell[k] = cells[k * kBlk];
 #pragma unroll
             for (int k = 0; k < kChunk; k += 2) {
                 float x[2];
-                tile_maxplus2(tile, cells + k * kBlk, x[0], x[1]);
+                tile_maxplus2(tile, cell[k], cell[k + 1], x[0], x[1]);
 #pragma unroll
                 for (int h = 0; h < 2; ++h) {
                     const bool up = x[h] > best[k + h];
@@ -409,7 +414,7 @@ __global__ __launch_bounds__(kTileWaves * kWave) void dag_align_chunks_kernel(Al
         };
         for (int tau = first_stage; tau <= end_stage; ++tau) {
             const int par = tau & 1;
-            const int lane = opaque_lane(), r16 = lane & 15;
+            const int lane = opaque_lane();
             // (chunk tau + 2 of the foreign blocks, with SPACING 1 tau + 1 of the block below)
             const bool bring = FETCHES && f_blk[0] >= 0 && tau + SPACING < NC;
             int published = 0;
@@ -448,7 +453,7 @@ __global__ __launch_bounds__(kTileWaves * kWave) void dag_align_chunks_kernel(Al
                         }
                     }
                     if (SPACING == 1 && J > 0 && c >= src_lo(J - 1) && c <= dest_hi(J - 1))   // what block J - 1 sends
-                        take(t0, lds_raw + o.eb + ((own_src - 1) * D + slot_own) * 256 + r16, J - 1, best, from);
+                        take(t0, lds_raw + o.eb + ((own_src - 1) * D + slot_own) * 256 + lane, J - 1, best, from);
                 }
                 if (more) load_match(c + 1, lane);
                 if (c >= 0 && c < NC) {
@@ -515,7 +520,7 @@ __global__ __launch_bounds__(kTileWaves * kWave) void dag_align_chunks_kernel(Al
                     }
                     if (tau >= t_src_from[u] && tau <= t_src_to[u]) {
                         int sl = ring + t_shift[u]; sl -= sl >= D ? D : 0;
-                        take(tile, lds_raw + t_cells[u] + sl * 256 + r16, t.I[u], best, from);
+                        take(tile, lds_raw + t_cells[u] + sl * 256 + lane, t.I[u], best, from);
                     }
                     if (t.end[u]) {
                         const int at = t.run[u] * 2 + par;
@@ -572,53 +577,19 @@ __global__ __launch_bounds__(kTileWaves * kWave) void dag_align_chunks_kernel(Al
     }
 }
 
-// best = max(best, max_{r<16} (a[lane r of this 16-lane row] + e[r])): two sums, then one three-way maximum
-// (24 instructions for 16 rows instead of 32; a maximum does not round, so the result is the same bit for bit)
-__device__ __forceinline__ void maxplus16_rowbcast(float &best, float av, const float *e) {
-    float t1, t2;
-    asm("s_nop 1\n\t"
-        "v_add_f32_dpp %1, %3, %4 row_newbcast:0 row_mask:0xf bank_mask:0xf\n\t"
-        "v_add_f32_dpp %2, %3, %5 row_newbcast:1 row_mask:0xf bank_mask:0xf\n\t"
-        "v_max3_f32 %0, %0, %1, %2\n\t"
-        "v_add_f32_dpp %1, %3, %6 row_newbcast:2 row_mask:0xf bank_mask:0xf\n\t"
-        "v_add_f32_dpp %2, %3, %7 row_newbcast:3 row_mask:0xf bank_mask:0xf\n\t"
-        "v_max3_f32 %0, %0, %1, %2\n\t"
-        "v_add_f32_dpp %1, %3, %8 row_newbcast:4 row_mask:0xf bank_mask:0xf\n\t"
-        "v_add_f32_dpp %2, %3, %9 row_newbcast:5 row_mask:0xf bank_mask:0xf\n\t"
-        "v_max3_f32 %0, %0, %1, %2\n\t"
-        "v_add_f32_dpp %1, %3, %10 row_newbcast:6 row_mask:0xf bank_mask:0xf\n\t"
-        "v_add_f32_dpp %2, %3, %11 row_newbcast:7 row_mask:0xf bank_mask:0xf\n\t"
-        "v_max3_f32 %0, %0, %1, %2\n\t"
-        "v_add_f32_dpp %1, %3, %12 row_newbcast:8 row_mask:0xf bank_mask:0xf\n\t"
-        "v_add_f32_dpp %2, %3, %13 row_newbcast:9 row_mask:0xf bank_mask:0xf\n\t"
-        "v_max3_f32 %0, %0, %1, %2\n\t"
-        "v_add_f32_dpp %1, %3, %14 row_newbcast:10 row_mask:0xf bank_mask:0xf\n\t"
-        "v_add_f32_dpp %2, %3, %15 row_newbcast:11 row_mask:0xf bank_mask:0xf\n\t"
-        "v_max3_f32 %0, %0, %1, %2\n\t"
-        "v_add_f32_dpp %1, %3, %16 row_newbcast:12 row_mask:0xf bank_mask:0xf\n\t"
-        "v_add_f32_dpp %2, %3, %17 row_newbcast:13 row_mask:0xf bank_mask:0xf\n\t"
-        "v_max3_f32 %0, %0, %1, %2\n\t"
-        "v_add_f32_dpp %1, %3, %18 row_newbcast:14 row_mask:0xf bank_mask:0xf\n\t"
-        "v_add_f32_dpp %2, %3, %19 row_newbcast:15 row_mask:0xf bank_mask:0xf\n\t"
-        "v_max3_f32 %0, %0, %1, %2"
-        : "+v"(best), "=&v"(t1), "=&v"(t2)
-        : "v"(av), "v"(e[0]), "v"(e[1]), "v"(e[2]), "v"(e[3]), "v"(e[4]), "v"(e[5]), "v"(e[6]), "v"(e[7]),
-          "v"(e[8]), "v"(e[9]), "v"(e[10]), "v"(e[11]), "v"(e[12]), "v"(e[13]), "v"(e[14]), "v"(e[15]));
-}
-
 __device__ __forceinline__ float max3(float a, float b, float c) {
     float d;
     asm("v_max3_f32 %0, %1, %2, %3" : "=v"(d) : "v"(a), "v"(b), "v"(c));
     return d;
 }
 
-// max_{r<64} (a[r] + tile.p[r]); lane l holds a[l & 15], a[16 + (l & 15)], a[32 + (l & 15)], a[48 + (l & 15)]
-__device__ __forceinline__ float tile_maxplus(const Tile &t, float a0, float a1, float a2, float a3) {
+// max_{r<64} (a[r] + tile.p[r]); lane r holds a[r]
+__device__ __forceinline__ float tile_maxplus(const Tile &t, float a) {
     float b0 = DAGX_NEG_INF, b1 = DAGX_NEG_INF;
-    maxplus16_rowbcast(b0, a0, t.p);
-    maxplus16_rowbcast(b1, a1, t.p + 16);
-    maxplus16_rowbcast(b0, a2, t.p + 32);
-    maxplus16_rowbcast(b1, a3, t.p + 48);
+    rows16<4, 0, 0>(t, a, b0, b1);
+    rows16<4, 4, 16>(t, a, b0, b1);
+    rows16<4, 8, 32>(t, a, b0, b1);
+    rows16<4, 12, 48>(t, a, b0, b1);
     return fmaxf(b0, b1);
 }
 
@@ -862,7 +833,6 @@ __global__ __launch_bounds__(kTileWaves * kWave) void dag_align_steps_kernel(Ali
         return row0;
     };
     const float *part_own = &part[own0 ? part_row0(own_J) : 0][lane];
-    const int r16 = lane & 15;
 
     // the cell values of one owned block: maximum over its tiles (the first tile that attains it is remembered), plus
     // the match score; written to LDS for the next step and to the table
@@ -893,22 +863,16 @@ __global__ __launch_bounds__(kTileWaves * kWave) void dag_align_steps_kernel(Ali
         {
             // The scores for a tile are requested one tile ahead of its arithmetic.  A tile whose predecessor block
             // holds no finite score, or whose block lies outside the band, is skipped.
-            float av[kTilesPerWave][4];
+            float av[kTilesPerWave];
             bool geo[kTilesPerWave];
 #define DAGX_ALIGN_READ(SL)                                                                        \
             geo[SL] = my_q[SL] >= 0 && my_J[SL] * kBlk <= slack + s && my_J[SL] * kBlk + kBlk - 1 >= s; \
-            if (geo[SL]) {                                                                         \
-                const float *ab = &abuf[cur][my_I[SL]][r16];                                       \
-                av[SL][0] = ab[0]; av[SL][1] = ab[16]; av[SL][2] = ab[32]; av[SL][3] = ab[48];     \
-            }
+            if (geo[SL]) av[SL] = abuf[cur][my_I[SL]][lane];
 #define DAGX_ALIGN_TILE(SL, TILE)                                                                  \
             if (my_q[SL] >= 0) {                                                                   \
                 float best = DAGX_NEG_INF;                                                         \
-                if (geo[SL]) {                                                                     \
-                    const float top = fmaxf(fmaxf(av[SL][0], av[SL][1]), fmaxf(av[SL][2], av[SL][3])); \
-                    if (__builtin_amdgcn_ballot_w64(top > DAGX_NEG_INF) != 0)                     \
-                        best = tile_maxplus(TILE, av[SL][0], av[SL][1], av[SL][2], av[SL][3]);     \
-                }                                                                                  \
+                if (geo[SL] && __builtin_amdgcn_ballot_w64(av[SL] > DAGX_NEG_INF) != 0)           \
+                    best = tile_maxplus(TILE, av[SL]);                                             \
                 part[my_q[SL]][lane] = best;                                                       \
             }
             DAGX_ALIGN_READ(0)
