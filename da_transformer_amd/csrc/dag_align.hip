@@ -1063,8 +1063,12 @@ __device__ __forceinline__ void walk_back_in_memory(const float *A, const unsign
 // predecessors found.  Where no candidate has a finite score the walk ends, or with ZERO_FOR_DEAD goes on from node 0.
 // lds: kWalkLds bytes.  s, j are uniform over the workgroup.
 // A step is a chain of dependent instructions of one wave, so its length is what counts: the byte that names the block and
-// the scores and transitions of both blocks are read in one LDS round trip, and the nodes found are kept in a register, one
-// a lane, and put 64 rows at a time.
+// the scores and transitions of both blocks are read in one LDS round trip, in whose shade what is not part of the chain is
+// done, and the nodes found are kept in a register, one a lane, and put 64 rows at a time.  While the path stays in the block
+// a step has one jump, whose condition also covers what ends the run of steps (another block, a cell without a finite score):
+// a step into a block further away has then been taken from the two at hand, and is taken again from memory.  Kernel, us, against
+// a step with a jump for each of these and the keeping at its end: alignment B = 64, L = 512, T = 64 22.3 -> 18.7, B = 16, L = 1024,
+// T = 256 64.1 -> 54.1 (0.21 us a step).
 template <typename TL, int NT, bool ZERO_FOR_DEAD, typename PUT>
 __device__ __forceinline__ void walk_back_staged(const float *A, const unsigned char *srcblk, int spitch, const TL *links, int L,
                                           int translen, int s, int j, int stop, WalkStage *lds, PUT put) {
@@ -1085,29 +1089,46 @@ __device__ __forceinline__ void walk_back_staged(const float *A, const unsigned 
             const WalkStage &w = lds[cur];
             const unsigned char *src = reinterpret_cast<const unsigned char *>(w.src) + (hi - s) * kBlk;
             const float *arow = w.a + (hi - s) * 2 * kBlk + lane, *ecol = w.e + lane * kWalkPitch;
-            for (int left = min(s - stop, kWalkRows - (hi - s)); left > 0 && j >> 6 == J; --left) {   // (-1: no block)
-                const int c = j & (kBlk - 1);
-                int byte = src[c];
-                float e0 = ecol[c], e1 = ecol[kBlk * kWalkPitch + c], a0 = arow[0], a1 = arow[kBlk];
-                asm volatile("" : "+v"(byte), "+v"(e0), "+v"(e1), "+v"(a0), "+v"(a1));   // (else read one after the other)
+            while (s > stop && hi - s < kWalkRows && j >> 6 == J) {   // (-1: no block)
+                // as far as rows are staged and nodes found can be kept, while the path stays in the block
+                const int until = max(max(stop, hi - kWalkRows), (s - 1) & ~(kWave - 1));
+                int c = j & (kBlk - 1), from, byte, last = -1;     // last: where a step's node is to be kept, behind the next one's reads
+                float x, top;
+                unsigned long long stays;
+                do {
+                    from = c;
+                    byte = src[c];
+                    float e0 = ecol[c], e1 = ecol[kBlk * kWalkPitch + c], a0 = arow[0], a1 = arow[kBlk];
+                    __builtin_amdgcn_sched_barrier(0);
+                    mine = lane == last ? J * kBlk + c : mine;
+                    --s;
+                    last = s & (kWave - 1);
+                    src += kBlk; arow += 2 * kBlk;
+                    const bool more = s > until;
+                    __builtin_amdgcn_sched_barrier(0);
+                    asm volatile("" : "+v"(byte), "+v"(e0), "+v"(e1), "+v"(a0), "+v"(a1));   // (else read one after the other)
+                    x = byte == J ? a1 + e1 : a0 + e0;
+                    stays = __builtin_amdgcn_ballot_w64(byte == J);
+                    top = wave64_max(x);
+                    // lowest lane among those that hold the maximum
+                    const unsigned long long at_top = __builtin_amdgcn_ballot_w64(x == top);
+                    c = (int)__builtin_ctzll(at_top);
+                    stays &= at_top & __builtin_amdgcn_ballot_w64(top > DAGX_NEG_INF);   // (no lane: a NaN)
+                    if (!more) break;
+                } while (stays != 0);
                 const int I = __builtin_amdgcn_readfirstlane(byte);
-                float x = I == J ? a1 + e1 : a0 + e0;
                 if (__builtin_expect((unsigned)(J - I) > 1u, 0)) {
-                    const int i = I * kBlk + lane, d = j - i - 1;
+                    const int i = I * kBlk + lane, d = J * kBlk + from - i - 1;
                     const bool valid = d >= 0 && d < translen && i < L;
                     const float e = to_float(links[valid ? (int64_t)i * translen + d : 0]);
-                    const float av = A[(int64_t)(s - 1) * L + (i < L ? i : L - 1)];
+                    const float av = A[(int64_t)s * L + (i < L ? i : L - 1)];
                     x = valid ? av + e : DAGX_NEG_INF;
+                    top = wave64_max(x);
+                    c = (int)__builtin_ctzll(__builtin_amdgcn_ballot_w64(x == top));
                 }
-                const float top = wave64_max(x);
-                // lowest lane among those that hold the maximum
-                j = I * kBlk + (int)__builtin_ctzll(__builtin_amdgcn_ballot_w64(x == top));
-                if (__builtin_expect(!(top > DAGX_NEG_INF), 0)) j = ZERO_FOR_DEAD ? 0 : -1;
-                --s;
-                src += kBlk; arow += 2 * kBlk;
-                const int slot = s & (kWave - 1);
-                mine = lane == slot ? j : mine;
-                if (slot == 0) {
+                j = __builtin_amdgcn_readfirstlane(top > DAGX_NEG_INF ? I * kBlk + c : ZERO_FOR_DEAD ? 0 : -1);
+                mine = lane == last ? j : mine;
+                if (last == 0) {
                     if (mine >= 0) put(s + lane, mine);
                     mine = -1;
                 }
@@ -1280,7 +1301,7 @@ static int launch_align(AlignArgs a, void *workspace, hipStream_t st) {
         if (rc) return rc;
         if ((rc = launch_align_sweep<TM, TL>(ta, "dag_align_sweep", st))) return rc;
         // the backtrack, and the samples that the pipeline gave up on.  (float32, kernel time: walked in memory 39.5 us at
-        // B=64 L=512 T=64 and 172 us at B=16 L=1024 T=256, out of LDS 22.4 and 65 us.)
+        // B=64 L=512 T=64 and 172 us at B=16 L=1024 T=256, out of LDS 18.7 and 54 us.)
         const bool in_lds = trace_fits_lds(a.T, a.L);
         const size_t redo_lds = (size_t)a.L * 8 + (in_lds ? (size_t)a.T * a.L * 2 : (size_t)0);
         const bool staged = staged_alignment(a.B, a.L);

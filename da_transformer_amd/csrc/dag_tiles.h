@@ -66,13 +66,21 @@ __device__ __forceinline__ float lane_bcast(float v, int lane) {
 // results are folded across rows with the two wave-level DPP broadcasts (row 0 -> 1, row 2 -> 3 via
 // row_bcast:15; rows 0-1 -> rows 2-3 via row_bcast:31) and lane 63 holds the maximum.
 __device__ __forceinline__ float wave64_max(float v) {
-    v = row16_max(v);
+    float r;
     asm("s_nop 1\n\t"
+        "v_max_f32_dpp %0, %1, %1 quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"
+        "s_nop 1\n\t"
+        "v_max_f32_dpp %0, %0, %0 quad_perm:[2,3,0,1] row_mask:0xf bank_mask:0xf\n\t"
+        "s_nop 1\n\t"
+        "v_max_f32_dpp %0, %0, %0 row_half_mirror row_mask:0xf bank_mask:0xf\n\t"
+        "s_nop 1\n\t"
+        "v_max_f32_dpp %0, %0, %0 row_mirror row_mask:0xf bank_mask:0xf\n\t"
+        "s_nop 1\n\t"
         "v_max_f32_dpp %0, %0, %0 row_bcast:15 row_mask:0xa bank_mask:0xf\n\t"
         "s_nop 1\n\t"
         "v_max_f32_dpp %0, %0, %0 row_bcast:31 row_mask:0xc bank_mask:0xf"
-        : "+v"(v));
-    return lane_bcast(v, 63);
+        : "=&v"(r) : "v"(v));
+    return lane_bcast(r, 63);
 }
 
 // A wave-uniform value the compiler must take as new at this point: address arithmetic built on it
