@@ -165,6 +165,19 @@ def test_alignment_at_edges_of_blocks_chunks_and_windows(B, L, T, translen, dtyp
     assert torch.equal(got[some], want)
 
 
+@pytest.mark.parametrize("B,L,T", [(2, 64, 13), (2, 129, 25), (65, 250, 33), (65, 512, 66), (1, 1000, 110)])   # steps, chunks of both spacings
+def test_alignment_of_subnormal_scores(B, L, T):
+    """The sums of scores are formed by matrix instructions, which keep every bit of subnormal ones: whole multiples of the smallest."""
+    match, links_sq, ol, tl = random_problem(L, B, L, T, dtype=F32)
+    links = tn.extract_valid_links(links_sq, None)
+    match, links = (match * 8).round() * 2.0 ** -149, (links * 8).round() * 2.0 ** -149
+    assert 0 < match.abs().max() < 2.0 ** -126
+    got = dagx.dag_best_alignment(match.to(DEV), links.to(DEV), ol.to(DEV), tl.to(DEV)).cpu()
+    some = sorted({0, B // 2, B - 1})
+    want = tn.torch_dag_best_alignment(match[some], tn.restore_valid_links(links[some]), ol[some], tl[some])
+    assert torch.equal(got[some], want)
+
+
 @pytest.mark.parametrize("B,L,T,translen,dtype,first", [
     (1, 4, 4, 1, F32, 0), (2, 4, 4, 3, F16, 1), (3, 5, 5, 1, F16, 3), (2, 6, 6, 2, F32, 2), (2, 63, 32, 2, F16, 1), (3, 64, 64, 1, F32, 1),
     (2, 65, 40, 3, BF16, 3), (1, 66, 66, 1, F16, 0), (3, 127, 64, 3, F32, 3), (2, 129, 129, 1, BF16, 1), (2, 130, 70, 2, F32, 2),
