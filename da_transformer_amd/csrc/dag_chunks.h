@@ -393,12 +393,15 @@ constexpr ChunkCosts kSweepCosts[2] = {{45, 9, 12, 70}, {85, 25, 16, 80}};
 
 // ---- the alignment's rules ----
 // Whether the sweep goes in chunks of four steps.  They cost T / 4 stages and one or two more for every block of nodes, single
-// steps T of two fifths of that: even at about six steps for every block of nodes and eight more (alignment, chunks and
-// steps: B = 64, L = 512, T = 64 114 and 131 us; B = 28, L = 450, T = 50 99.4 and 98.0, T = 56 103 and 106; B = 20, L = 1000, T = 128 277 and
-// 312; B = 1, L = 900, T = 70 190 and 178, T = 98 222 and 223; B = 48, L = 350, T = 40 73.2 and 73.5; B = 8, L = 128, T = 32 39 and 44;
-// B = 1, L = 115, T = 15 30 and 27).
+// steps T of two fifths of that, and a stage of four steps is hardly longer where the sums are formed by matrix instructions: even
+// at two steps for every block and 22 more, where windows are short and a step has few tiles at four and 14 (alignment, steps
+// and chunks, us: B = 64, L = 512, T = 40 101.1 and 88.5, T = 32 93.6 and 85.7, but B = 16 of them 81.5 and 85.4; B = 16, L = 768, T = 64 163 and 135,
+// T = 36 120 and 111; B = 20, L = 1000, T = 96 259 and 212; B = 1, L = 900, T = 70 187 and 168; B = 64, L = 256, T = 25 48.6 and 45.7, but B = 200
+// and T = 20 48.2 and 53.0; B = 32, L = 768, transitions of at most 100, T = 48 109 and 108, T = 60 120 and 118; B = 4, L = 992, of at
+// most 136, T = 70 141 and 146).  Up to three blocks the line is where it was for both, six for every block and 8 more.
 inline bool align_in_chunks(int B, int T, int L, int translen) {
-    return T >= 6 * ((L + kBlk - 1) / kBlk) + 8 && (int64_t)B * L * translen >= 4;   // (the chunked kernel's tiles are loaded four elements at a time)
+    const int NB = (L + kBlk - 1) / kBlk, line = window_blocks(translen) <= 3 ? 4 * NB + 14 : 2 * NB + 22, most = 6 * NB + 8;
+    return T >= (line < most ? line : most) && (int64_t)B * L * translen >= 4;   // (the chunked kernel's tiles are loaded four elements at a time)
 }
 
 // Workgroups per sweep.  In chunks: from four position blocks on as many as the device has room for (one per CU) up to one
