@@ -5,7 +5,7 @@
 //
 // Two implementations:
 //  * dag_align_chunks_kernel or dag_align_steps_kernel + dag_backtrack_kernel (L <= 1024): the sweep keeps E as 64x64 register
-//    tiles, spread over the same pipeline of workgroups as the loss sweeps, and forms two DPP-broadcast sums and one
+//    tiles, spread over the same pipeline of workgroups as the loss sweeps, and forms the sums by matrix instructions and one
 //    three-way maximum per two (i, j) pairs -- four steps a stage, or, for few steps on many nodes, step by step
 //    (align_in_chunks).  It stores the score table and the block of 64 nodes each cell's best predecessor lies in.  The
 //    backtrack (a wave per sample walks, others may stage for it) then re-derives, for the T_b cells on the path only, the
@@ -243,14 +243,13 @@ struct AlignTileArgs {
 // blocks with the best predecessor the lowest one counts (runs in the order of the blocks, then the block itself; a later
 // one replaces an earlier one only if it is larger).
 //
-// Step by step, with two barriers, LDS round trips and a hand-over in each, a step costs 1.6 us at L = 512 and 1.8 us at
-// L = 1024, of which the tiles' 96 instructions a step are a third.  What bounds the stages now is those instructions:
-// four steps of a tile take 2 700 cycles, 2 000 of a SIMD that two waves share, the walk of a block 3 500.
+// What bounds the stages is the tiles' sums and maxima, 1 300 cycles of a SIMD for four steps of a tile (a SIMD gives its cycles
+// to matrix or to vector instructions, so that two waves that share one gain hardly anything), and the walks.
 //
 // SPACING (dag_chunks.h): a tile is nearly as much work as the walk here, so that where the walk bounds the stages and SIMDs
 // have time to spare -- small graphs, or hardly more than one block to a group -- two stages a block are shorter
-// (alignment with SPACING 1 and 2: B = 64, L = 256, T = 64 83 and 75 us; B = 40, L = 400, T = 60 99 and 96; B = 16, L = 512,
-// T = 128 167.5 and 156); where the tiles bound them every stage more costs (B = 64, L = 512, T = 64 116 and 125).
+// (alignment with SPACING 1 and 2: B = 64, L = 256, T = 64 77.0 and 70.5 us; B = 64, L = 320, T = 48 69.9 and 66.9; B = 40, L = 400, T = 60 91.2
+// and 90.8); where the tiles bound them every stage more costs (B = 64, L = 512, T = 64 109.4 and 112.6).
 template <typename TM, typename TL, int SPACING>
 __global__ __launch_bounds__(kTileWaves * kWave) void dag_align_chunks_kernel(AlignTileArgs a) {
     extern __shared__ __align__(16) float lds_raw[];
