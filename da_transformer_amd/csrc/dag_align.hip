@@ -815,6 +815,13 @@ __global__ __launch_bounds__(kTileWaves * kWave) void dag_align_steps_kernel(Ali
             }
         }
     };
+    // The fetcher's instructions are what a step waits for where windows are long, and the wave that shares its SIMD multiplies tiles
+    // meanwhile: without priority matrix instructions make it later than vector ones did, by up to 0.2 us a step.  Alignment, us, DPP sums /
+    // matrix sums / those and the fetcher first: B = 1, L = 1024, T = 53 159.1 / 168.1 / 157.0, T = 14 74.1 / 77.2 / 72.8; B = 24, L = 960, T = 14
+    // 78.2 / 82.5 / 78.3; B = 1, L = 640, T = 41 89.4 / 95.2 / 89.2; B = 64, L = 1024, T = 30 165.1 / 165.2 / 156.2; B = 64, L = 512, T = 29
+    // 80.4 / 81.5 / 79.5; B = 1, L = 256, transitions of at most 64, T = 29 44.3 / 45.8 / 43.3; B = 130, L = 400, of at most 180, T = 41
+    // 103.2 / 90.4 / 90.2.  (Priority only while it fetches: B = 24, L = 960, T = 14 80.5; B = 1, L = 1024, T = 20 89.1 for 86.3.)
+    if (fetcher) __builtin_amdgcn_s_setprio(3);
     if (fetcher && Tb > 1) {   // what phase B of step 1 needs
         issue_match(1, lane);
         if (consumer && 1 < Tb - 1) dma_dword_agent(lds_addr(&stage_p[1][0]), below, 0u);

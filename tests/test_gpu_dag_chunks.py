@@ -150,7 +150,10 @@ def test_some_samples_of_a_batch_with_tables_go_on_to_the_float64_sweeps(with_gr
     (65, 250, 33, None, F32), (65, 512, 66, None, F16), (129, 1022, 130, 64, F16),
     # in chunks from 2 ceil(L / 64) + 22 on, where transitions span at most three blocks from 4 ceil(L / 64) + 14 on
     (2, 256, 29, None, F32), (2, 256, 30, None, F16), (1, 300, 31, None, F32), (3, 300, 32, 200, F32), (65, 500, 37, None, F16), (65, 500, 38, None, F32),
-    (2, 1024, 53, None, F16), (2, 1024, 54, None, F32), (1, 700, 57, 192, F32), (2, 700, 58, 192, F16), (2, 1000, 78, 100, F32), (1, 700, 44, 193, F16)])
+    (2, 1024, 53, None, F16), (2, 1024, 54, None, F32), (1, 700, 57, 192, F32), (2, 700, 58, 192, F16), (2, 1000, 78, 100, F32), (1, 700, 44, 193, F16),
+    # step by step, one workgroup a sample: twelve and eleven blocks in eight waves, and as many tiles as make the fetching wave take some; a
+    # single block more than waves
+    (129, 768, 40, 64, F32), (129, 700, 57, 64, F16), (129, 576, 30, 64, BF16)])
 def test_alignment_at_edges_of_blocks_chunks_and_windows(B, L, T, translen, dtype):
     match, links_sq, ol, tl = random_problem(L + T, B + 1, L, T, dtype=F32, ragged=False, translen=translen)
     if translen is not None:      # a path of T_b nodes spans at most (T_b - 1) translen transitions
