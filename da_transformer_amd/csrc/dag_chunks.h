@@ -394,13 +394,17 @@ constexpr ChunkCosts kSweepCosts[2] = {{45, 9, 12, 70}, {85, 25, 16, 80}};
 // ---- the alignment's rules ----
 // Whether the sweep goes in chunks of four steps.  They cost T / 4 stages and one or two more for every block of nodes, single
 // steps T of two fifths of that, and a stage of four steps is hardly longer where the sums are formed by matrix instructions: even
-// at two steps for every block and 22 more, where windows are short and a step has few tiles at four and 14 (alignment, steps
-// and chunks, us: B = 64, L = 512, T = 40 101.1 and 88.5, T = 32 93.6 and 85.7, but B = 16 of them 81.5 and 85.4; B = 16, L = 768, T = 64 163 and 135,
-// T = 36 120 and 111; B = 20, L = 1000, T = 96 259 and 212; B = 1, L = 900, T = 70 187 and 168; B = 64, L = 256, T = 25 48.6 and 45.7, but B = 200
-// and T = 20 48.2 and 53.0; B = 32, L = 768, transitions of at most 100, T = 48 109 and 108, T = 60 120 and 118; B = 4, L = 992, of at
-// most 136, T = 70 141 and 146).  Up to three blocks the line is where it was for both, six for every block and 8 more.
+// at about two steps for every block and 22 more, where windows are short and a step has few tiles at four and 14 (alignment, steps
+// and chunks, us: B = 64, L = 512, T = 28 76.9 and 75.2, T = 40 98.4 and 87.3; B = 16, L = 768, T = 36 110 and 108, T = 48 135 and 124; B = 64, L = 640,
+// T = 40 112 and 109; B = 1, L = 900, T = 52 150 and 152, T = 60 165 and 162; B = 40, L = 1024, T = 56 227 and 187; B = 64, L = 320, T = 32
+// 55.7 and 55.6; B = 200, L = 256, T = 30 54.6 and 55.9; transitions of at most 100: B = 16, L = 768, T = 60 108 and 110; B = 1, L = 900, T = 75 135 and 128).
+// Eight blocks of a workgroup each, with two stages a block, take longest to fill: 43 (L = 512: B = 1, T = 40 76.7 and 79.7; B = 16, T = 40 83.2 and
+// 86.3, T = 48 87.9 and 87.7; B = 32, T = 38 83.5 and 87.5, T = 44 89.1 and 88.4).  Up to three blocks the line is at six for every block and 8 more.
+// (A few steps earlier would do for four blocks, and for those of most sizes with B > 32, but not for all: B = 64, L = 256, T = 26 44.7 and 44.5,
+// B = 200 50.5 and 53.5; B = 40, L = 1024, T = 32 155 and 148, B = 1 114 and 133.)
 inline bool align_in_chunks(int B, int T, int L, int translen) {
-    const int NB = (L + kBlk - 1) / kBlk, line = window_blocks(translen) <= 3 ? 4 * NB + 14 : 2 * NB + 22, most = 6 * NB + 8;
+    const int NB = (L + kBlk - 1) / kBlk, most = 6 * NB + 8;
+    const int line = window_blocks(translen) <= 3 ? 4 * NB + 14 : NB == 8 && ((B + 7) & ~7) * NB <= 256 ? 43 : 2 * NB + 22;
     return T >= (line < most ? line : most) && (int64_t)B * L * translen >= 4;   // (the chunked kernel's tiles are loaded four elements at a time)
 }
 

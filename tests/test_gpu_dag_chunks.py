@@ -143,13 +143,16 @@ def test_some_samples_of_a_batch_with_tables_go_on_to_the_float64_sweeps(with_gr
     (3, 65, 9, 64, F32), (2, 129, 17, 2, F16), (1, 257, 8, None, F32), (2, 320, 9, 128, F16), (1, 321, 33, 63, F32),
     (2, 449, 30, 32, BF16), (1, 511, 14, None, F32), (2, 513, 7, 257, F16), (1, 705, 12, 130, F32), (2, 1024, 11, None, F16),
     (1, 1023, 64, 200, F32),
-    # in chunks where T is at least 6 ceil(L / 64) + 8 (from four blocks of 64 nodes on a smaller line holds: the last ones), else step by step
+    # up to three blocks of 64 nodes in chunks where T is at least 6 ceil(L / 64) + 8, else step by step
     (1, 64, 13, None, F32), (2, 128, 20, None, F32), (2, 129, 25, None, F32), (1, 129, 26, None, F16),
+    # in chunks, of more than three blocks
     (2, 448, 50, None, F16), (2, 449, 56, 100, F32), (1, 513, 62, 257, F16), (1, 705, 80, 130, F32), (2, 1024, 104, None, F16),
     # few workgroups a sample: groups of several blocks (of eight in the last), one and two stages a block
     (65, 250, 33, None, F32), (65, 512, 66, None, F16), (129, 1022, 130, 64, F16),
-    # in chunks from 2 ceil(L / 64) + 22 on, where transitions span at most three blocks from 4 ceil(L / 64) + 14 on
+    # of more than three blocks in chunks from 2 ceil(L / 64) + 22 on, where transitions span at most three blocks from 4 ceil(L / 64) + 14 on,
+    # of eight blocks with a workgroup each from 43 on
     (2, 256, 29, None, F32), (2, 256, 30, None, F16), (1, 300, 31, None, F32), (3, 300, 32, 200, F32), (65, 500, 37, None, F16), (65, 500, 38, None, F32),
+    (3, 500, 42, None, F32), (3, 500, 43, None, F16),
     (2, 1024, 53, None, F16), (2, 1024, 54, None, F32), (1, 700, 57, 192, F32), (2, 700, 58, 192, F16), (2, 1000, 78, 100, F32), (1, 700, 44, 193, F16),
     # step by step, one workgroup a sample: twelve and eleven blocks in eight waves, and as many tiles as make the fetching wave take some; a
     # single block more than waves

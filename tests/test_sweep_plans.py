@@ -96,7 +96,16 @@ static int alignment() {
             }
     return seen < 3000;
 }
+// where the alignment's sweep goes in chunks: the step at which it begins to
+static bool chunks_from(int B, int L, int translen, int T) {
+    if (!align_in_chunks(B, T - 1, L, translen) && align_in_chunks(B, T, L, translen)) return true;
+    std::printf("alignment B=%d L=%d translen=%d: not in chunks from T=%d on\n", B, L, translen, T);
+    return false;
+}
 int main() {
+    // (eight blocks with a workgroup each, and with less room; other graphs; windows of at most three blocks)
+    if (!chunks_from(1, 449, 448, 43) || !chunks_from(32, 512, 193, 43) || !chunks_from(33, 512, 511, 38) || !chunks_from(32, 448, 447, 36) ||
+        !chunks_from(32, 513, 512, 40) || !chunks_from(32, 512, 192, 46) || !chunks_from(1, 1024, 1023, 54) || !chunks_from(64, 192, 191, 26)) return 1;
     // groupings as good as each other for the busiest SIMD: more even ones, where they gain more than their hand-overs take
     if (!groups_are<2>(align_costs<2>(64)[0], 1, 8, 8, {2, 2, 2, 2}) || !groups_are<1>(align_costs<1>(192)[0], 3, 10, 13, {3, 2, 2, 2, 2, 2}) ||
         !groups_are<1>(kSweepCosts[0], 5, 2, 5, {3, 2}) || !groups_are<1>(align_costs<1>(576)[0], 9, 9, 9, {4, 2, 1, 1, 1}) ||
