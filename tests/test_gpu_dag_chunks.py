@@ -187,6 +187,82 @@ def test_alignment_of_subnormal_scores(B, L, T):
     assert torch.equal(got[some], want)
 
 
+def alignment_by_the_rule(match, square, out_len, tgt_len):
+    """One sample in float32: the first largest candidate wins, a sum that is no number is no candidate, and an end without a finite or
+    infinite score above -inf has no path."""
+    neg = float("-inf")
+    cells = torch.full((square.shape[0],), neg)
+    cells[0] = match[0, 0]
+    came_from = []
+    for t in range(1, tgt_len):
+        sums = cells.unsqueeze(1) + square
+        best, first = sums.masked_fill(sums.isnan(), neg).max(0)
+        came_from.append(first)
+        cells = best + match[t]
+    path = torch.full((square.shape[0],), -1)
+    node = out_len - 1
+    if not cells[node] > neg:
+        return path
+    path[node] = tgt_len - 1
+    for t in range(tgt_len - 1, 0, -1):
+        node = int(came_from[t - 1][node])
+        path[node] = t - 1
+    return path
+
+
+def with_extremes(kind, x, gen):
+    """Some of the scores replaced: 'lowest' what masks stand for -inf with, whose sums overflow to it; 'huge' sums that overflow on either
+    side; 'special' infinities and NaN."""
+    pick = torch.rand(x.shape, generator=gen)
+    if kind == "lowest":
+        return x.masked_fill((pick < 0.5) & torch.isfinite(x), torch.finfo(x.dtype).min)
+    if kind == "huge":
+        return torch.where(pick < 0.3, x * 3e37, x)
+    x = x.masked_fill(pick < 2e-3, float("inf"))
+    return x.masked_fill(pick > 0.98, float("nan"))
+
+
+@pytest.mark.parametrize("kind,dtype", [("lowest", F32), ("lowest", BF16), ("huge", F32), ("special", F32), ("special", F16)])
+@pytest.mark.parametrize("B,L,T", [(3, 64, 20), (3, 200, 18), (65, 250, 33), (260, 130, 12), (65, 512, 66), (2, 1000, 24)])
+def test_alignment_of_lowest_overflowing_infinite_and_undefined_scores(B, L, T, kind, dtype):
+    gen = torch.Generator().manual_seed(L + T)
+    match, links_sq, ol, tl = random_problem(L, B, L, T, dtype=F32)
+    links = with_extremes(kind, tn.extract_valid_links(links_sq, None).to(dtype), gen)
+    match = with_extremes(kind, match.to(dtype), gen)
+    match[:, 0, 0] = -1.0
+    some = sorted({0, 1, B // 2, B - 1})
+    want = torch.stack([alignment_by_the_rule(match[b].float(), tn.restore_valid_links(links[b:b + 1].float())[0], int(ol[b]), int(tl[b])) for b in some])
+    assert (want >= 0).any(1).all()
+    for mode in (0, 1, 2):      # the sweeps; one workgroup a sample; the sweeps, and every sample done again
+        before = nat.lib().dagx_force_log_domain(mode)
+        try:
+            got = dagx.dag_best_alignment(match.to(DEV), links.to(DEV), ol.to(DEV), tl.to(DEV)).cpu()
+        finally:
+            nat.lib().dagx_force_log_domain(before)
+        assert torch.equal(got[some], want), mode
+
+
+@pytest.mark.parametrize("kind", ["lowest", "huge", "special"])
+@pytest.mark.parametrize("B,L,steps", [(3, 64, 10), (3, 64, 20), (3, 250, 12), (65, 512, 64), (2, 1000, 24), (260, 100, 30)])
+def test_viterbi_decoding_of_lowest_overflowing_infinite_and_undefined_scores(B, L, steps, kind):
+    """The sweeps against the table by one workgroup a sample."""
+    gen = torch.Generator().manual_seed(L + steps)
+    _, links_sq, ol, _ = random_problem(L, B, L, 4, dtype=F32)
+    links = with_extremes(kind, tn.extract_valid_links(links_sq, None), gen).to(DEV)
+    scores = with_extremes(kind, torch.randn(B, L, generator=gen) - 2.0, gen).to(DEV)
+    tokens = torch.randint(4, 50, (B, L), generator=gen).to(DEV)
+    out = []
+    for mode in (0, 1):
+        before = nat.lib().dagx_force_log_domain(mode)
+        try:
+            out.append(dagx.dag_viterbi_decode(links, (scores, tokens), ol.to(DEV), 2 * L / steps, 1.0, True, 1))
+        finally:
+            nat.lib().dagx_force_log_domain(before)
+    assert out[0].nodes.shape[1] == steps
+    for name in ("output_tokens", "pred_length", "nodes"):
+        assert torch.equal(getattr(out[0], name), getattr(out[1], name)), name
+
+
 @pytest.mark.parametrize("B,L,T,translen,dtype,first", [
     (1, 4, 4, 1, F32, 0), (2, 4, 4, 3, F16, 1), (3, 5, 5, 1, F16, 3), (2, 6, 6, 2, F32, 2), (2, 63, 32, 2, F16, 1), (3, 64, 64, 1, F32, 1),
     (2, 65, 40, 3, BF16, 3), (1, 66, 66, 1, F16, 0), (3, 127, 64, 3, F32, 3), (2, 129, 129, 1, BF16, 1), (2, 130, 70, 2, F32, 2),
