@@ -1,6 +1,6 @@
 // Building blocks shared by the tile-resident sweep kernels (log-semiring loss, max-semiring
-// alignment): tile geometry, the grouping of position blocks into a pipeline of workgroups, DPP
-// broadcast arithmetic and lane reductions, agent-scope loads/stores for the hand-over.
+// alignment): tile geometry, the grouping of position blocks into a pipeline of workgroups, the maximum
+// over a wave, agent-scope loads/stores and copies to LDS for the hand-over, exponentials with a shift.
 #pragma once
 
 #include "dagx_common.h"
@@ -44,26 +44,11 @@ inline int groups_needed(int L, int translen, int most) {
 }
 
 // ---- DPP lane reductions (no LDS traffic) ----------------------------------------------------
-// max over each 16-lane row, result in every lane of the row (butterfly; each DPP op needs its
-// source written two wait states earlier)
-__device__ __forceinline__ float row16_max(float v) {
-    float r;
-    asm("s_nop 1\n\t"
-        "v_max_f32_dpp %0, %1, %1 quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"
-        "s_nop 1\n\t"
-        "v_max_f32_dpp %0, %0, %0 quad_perm:[2,3,0,1] row_mask:0xf bank_mask:0xf\n\t"
-        "s_nop 1\n\t"
-        "v_max_f32_dpp %0, %0, %0 row_half_mirror row_mask:0xf bank_mask:0xf\n\t"
-        "s_nop 1\n\t"
-        "v_max_f32_dpp %0, %0, %0 row_mirror row_mask:0xf bank_mask:0xf"
-        : "=&v"(r) : "v"(v));
-    return r;
-}
 __device__ __forceinline__ float lane_bcast(float v, int lane) {
     return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), lane));
 }
-// max over the 64 lanes, wave-uniform result: butterfly inside the 16-lane rows, then the row
-// results are folded across rows with the two wave-level DPP broadcasts (row 0 -> 1, row 2 -> 3 via
+// max over the 64 lanes, wave-uniform result: butterfly inside the 16-lane rows (each DPP op needs its source written two wait
+// states earlier), then the row results are folded across rows with the two wave-level DPP broadcasts (row 0 -> 1, row 2 -> 3 via
 // row_bcast:15; rows 0-1 -> rows 2-3 via row_bcast:31) and lane 63 holds the maximum.
 __device__ __forceinline__ float wave64_max(float v) {
     float r;
