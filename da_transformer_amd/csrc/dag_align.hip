@@ -126,9 +126,9 @@ __global__ __launch_bounds__(NT) void dag_align_kernel(AlignArgs a) {
 // third is cells[row] + P[row][lane] for four rows, one rounding each (1 * x is exact: the bits of v_add_f32, subnormals
 // and infinities among them).  256 sums take 8.2 cycles of a SIMD and four v_add_f32_dpp 18; the maxima, a three-way one for two
 // sums at 4.5 cycles, are all that vector instructions have left to do.  A change between matrix and vector instructions costs
-// a SIMD about 6.5 cycles, hence four of the former and eight of the latter at a time, sixteen registers of sums (one at a time 655, eight
-// at a time 487, with sixteen registers more).  Four steps of a tile, ns, on a wave alone and on one of two that share a SIMD:
-// 540 and 518, in two DPP sums and a maximum for every two rows 942 and 766.
+// a SIMD about 6.5 cycles, hence four of the former and eight of the latter at a time, sixteen registers of sums.  Four steps of a
+// tile, ns, on a wave alone and for each of two that share a SIMD, all in one run: four at a time 585 and 546, one at a time 824 and 690, eight
+// at a time, with sixteen registers more, 560 and 517; in two DPP sums and a maximum for every two rows 980 and 782.
 //
 // d = cells[4 ABID + i] + t.p[ROW + i] for i < 4; CBSZ 4: the cells of all 64 lanes are candidates, 3: those of a lane's own half
 template <int CBSZ, int ABID, int ROW>

@@ -103,9 +103,9 @@ constexpr int kChunkLdsBytes = 160 * 1024 - 512;
 struct TileDeal { unsigned wave; };          // four bits a wave: tiles, foreign blocks << 2
 __device__ __host__ __forceinline__ int dealt_tiles(const TileDeal &d, int wave) { return (d.wave >> (4 * wave)) & 3; }
 __device__ __host__ __forceinline__ int dealt_foreign(const TileDeal &d, int wave) { return (d.wave >> (4 * wave + 2)) & 3; }
-// How long a wave takes for its pieces of a stage, in about hundreds of cycles: walking a block (with SPACING 1 with the product
-// of the adjacent tile), a tile, fetching a foreign block (most of it waits); and how much of the sum of two waves' times a SIMD takes for
-// both, in per cent (waves w and w + 4 share one).
+// What a wave's pieces of a stage weigh in a plan: walking a block (with SPACING 1 with the product of the adjacent tile), a tile,
+// fetching a foreign block (most of it waits); and how much of the sum of two waves' weights a SIMD takes for both, in per cent (waves w
+// and w + 4 share one).  Set by timing calls, from the pieces' own times in hundreds of cycles on.
 struct ChunkCosts { int walk, product, fetch, shared; };
 // Returns how long the busiest wave or SIMD takes, -1 if there are more tiles than the waves have room for; alone: how long the busiest
 // SIMD takes if it does nothing for one wave while it does something for the other.
@@ -428,13 +428,14 @@ inline int align_groups(int B, int T, int L, int translen) {
 }
 // Stages from a block's walk of a chunk to the next block's: see dag_align_chunks_kernel.
 inline int align_spacing(int NB, int C) { return NB <= 5 || (NB <= 8 && 2 * NB <= 3 * C) ? 2 : 1; }
-// The alignment's costs, found by timing calls under some twenty sets, from the pieces' own times {62 or 36, 27, 4, 75} on (us): B = 64,
-// L = 512, T = 64 119.8 -> 115.2, B = 16, L = 768, T = 192 278 -> 268, B = 4, L = 700, T = 110 187 -> 177, B = 64, L = 256, T = 64
-// (SPACING 2) 79.0 -> 76.1, B = 40, L = 400, T = 60 (SPACING 2) 99.5 -> 95.2.  With SPACING 1 a fetched block weighs 2 where windows
-// span more than three blocks, so that a group fetches many and their waits overlap, else its own time, 4.  With 4 for all: B = 42, L = 880,
-// T = 176 444 us for 423, B = 9, L = 876, T = 175 293 for 285, B = 2, L = 846, T = 338 440 for 429 (but B = 41, L = 944, T = 283 525 for 539);
-// with 2 for all: B = 91, L = 896, T = 358, transitions of at most 65 607 for 559, B = 74, L = 468, T = 58, at most 139 106 for 101.5,
-// B = 14, L = 955, T = 238, at most 113 302 for 289.
+// The alignment's weights: those that timing calls under some twenty sets found when its sums were formed by vector instructions.  A tile
+// takes half as long now and two waves of a SIMD hardly less than one after the other, but some ten sets timed again found none better, and
+// weights by the pieces' times of today, {45 or 30, 13, 4, 100}, are worse: alignment, us, these and those, B = 64, L = 512, T = 64 101.6 and 104,
+// B = 16, L = 768, T = 192 230 and 238, B = 4, L = 700, T = 110 151 and 159, B = 64, L = 256, T = 64 (SPACING 2) 65.0 and 68.4, B = 40, L = 400,
+// T = 60 (SPACING 2) 88.5 and 93.2.  With SPACING 1 a fetched block weighs 2 where windows span more than three blocks, so that a group
+// fetches many and their waits overlap, else 4.  With 4 for all: B = 9, L = 876, T = 175 254 us for 250, B = 2, L = 846, T = 338 369 for 364
+// (but B = 41, L = 944, T = 283 418 for 429); with 2 for all: B = 91, L = 896, T = 358, transitions of at most 65 481 for 467, B = 74, L = 468, T = 58,
+// at most 139 92.0 for 88.6, B = 14, L = 955, T = 238, at most 113 269 for 246.
 template <int SPACING>
 constexpr ChunkCosts kAlignCosts[2][1] = {{SPACING == 1 ? ChunkCosts{62, 27, 2, 65} : ChunkCosts{36, 27, 4, 55}},
                                           {SPACING == 1 ? ChunkCosts{62, 27, 4, 65} : ChunkCosts{36, 27, 4, 55}}};
