@@ -400,8 +400,8 @@ constexpr ChunkCosts kSweepCosts[2] = {{45, 9, 12, 70}, {85, 25, 16, 80}};
 // 55.7 and 55.6; B = 200, L = 256, T = 30 54.6 and 55.9; transitions of at most 100: B = 16, L = 768, T = 60 108 and 110; B = 1, L = 900, T = 75 135 and 128).
 // Eight blocks of a workgroup each, with two stages a block, take longest to fill: 43 (L = 512: B = 1, T = 40 76.7 and 79.7; B = 16, T = 40 83.2 and
 // 86.3, T = 48 87.9 and 87.7; B = 32, T = 38 83.5 and 87.5, T = 44 89.1 and 88.4).  Up to three blocks the line is at six for every block and 8 more.
-// (A few steps earlier would do for four blocks, and for those of most sizes with B > 32, but not for all: B = 64, L = 256, T = 26 44.7 and 44.5,
-// B = 200 50.5 and 53.5; B = 40, L = 1024, T = 32 155 and 148, B = 1 114 and 133.)
+// (The line is that of few samples.  With more it could be lower for most sizes, but not for all: B = 64, L = 256, T = 26 44.7 and 44.5, B = 200
+// 50.5 and 53.5; L = 1024, T = 32 B = 40 155 and 148, B = 1 114 and 133.)
 inline bool align_in_chunks(int B, int T, int L, int translen) {
     const int NB = (L + kBlk - 1) / kBlk, most = 6 * NB + 8;
     const int line = window_blocks(translen) <= 3 ? 4 * NB + 14 : NB == 8 && ((B + 7) & ~7) * NB <= 256 ? 43 : 2 * NB + 22;
